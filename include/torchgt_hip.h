@@ -579,6 +579,79 @@ int tgt_gen_edge_input(const int32_t* d_path, const void* d_edge_feat, int feat_
 int tgt_floyd_warshall(const uint8_t* d_adj, const int32_t* d_n_nodes, int num_graphs, int n_max, int32_t* d_dist,
                        int32_t* d_path, void* stream);
 
+/* ---- the node-local part of an encoder layer in one pass ---------------------------------------------------------
+ * Everything between two attention launches of the Graphormer layers (models/graphormer_dist_node_level.py:246-314,
+ * models/graphormer_graph_level.py:267-306), hidden and feed-forward width 64, dtype TGT_DTYPE_F32 or TGT_DTYPE_BF16:
+ *     s1 = s + a Wo^T + bo;   s' = s1 + W2 gelu(W1 LN(s1) + b1) + b2;   q, k, v = LN'(s') W^T + b
+ * The kernels read packed parameters.  tgt_node_pack: `mats` are n_mats weights [rows[i] <= 64, 64] with row stride ld[i]
+ * elements (rows behind rows[i] count as zero), `vecs` n_vecs vectors of lens[i] <= 64 elements; d_frags takes
+ * tgt_node_frag_bytes(n_mats, dtype) bytes: weight i for products with the weight at i * unit, for products with its
+ * transpose at (n_mats + i) * unit, unit = tgt_node_frag_bytes(1, dtype) / 2; d_vecs takes n_vecs * 64 floats. */
+int64_t tgt_node_frag_bytes(int n_mats, int dtype);
+int tgt_node_pack(const void* const* mats, const int* ld, const int* rows, int n_mats, const void* const* vecs, const int* lens,
+                  int n_vecs, int dtype, void* d_frags, float* d_vecs, void* stream);
+/* Forward.  attn: the attention's rows [rows, 64], or NULL for the part in front of the first layer (then s' = s_in, whose
+ * first `tokens` rows are taken from `token` and written to s_out; s_in and s_out are the same array).  w_post: packed Wo,
+ * W1, W2; v_post: bo, gamma, beta, b1, b2.  q, k, v: rows for the next attention (w_next: packed Wq, Wk, Wv; v_next: gamma,
+ * beta, bq, bk, bv), or NULL.  logp: [rows - tokens, classes] log_softmax(LN(s') Wh^T + bh) without the token rows (w_next:
+ * packed Wh; v_next: gamma, beta, bh), or NULL. */
+typedef struct {
+    int64_t rows;
+    int32_t dtype, tokens, classes;
+    float eps_post, eps_next;
+    const void *attn, *s_in, *token;
+    void* s_out;
+    const void *w_post, *w_next;
+    const float *v_post, *v_next;
+    void *q, *k, *v, *logp;
+} tgt_node_fwd_args;
+int tgt_node_fwd(const tgt_node_fwd_args* args, void* stream);
+/* Backward of the part in front of an attention: g_out = g_in + d LN'(...) for dq, dk, dv (w_back: the transposed packed Wq,
+ * Wk, Wv; s: the rows LN' normalised), or of the classes (dlogp, logp; no g_in, dq, dk, dv; w_back: transposed packed Wh).
+ * d_token: the first `tokens` rows of g_out once more (the gradient of the global tokens behind the first layer), or NULL.
+ * partial: tgt_node_bwd_workers(rows) partial sums of the gradients of (Wq, Wk, Wv, bq, bk, bv, gamma, beta) or of
+ * (Wh, bh, gamma, beta), each mats * 4096 + (mats + 2) * 64 floats: see tgt_node_sums. */
+typedef struct {
+    int64_t rows;
+    int32_t dtype, tokens, classes;
+    float eps;
+    const void *dq, *dk, *dv, *g_in, *s, *dlogp, *logp;
+    const void* w_back;
+    const float* v_next;
+    void *g_out, *d_token;
+    float* partial;
+} tgt_node_bwd_pre_args;
+int tgt_node_bwd_workers(int64_t rows);
+int tgt_node_bwd_pre(const tgt_node_bwd_pre_args* args, void* stream);
+/* Backward of the part behind an attention: from g_in = ds' to g_out = ds (residual path) and d_attn = da; s and attn as the
+ * forward read them.  nd: per node and head (1 / (Z + 1e-6), da . a), what the sparse attention's backward begins with
+ * (tgt_sparse_attn_bwd_from_nd), or NULL.  partial: sums for (Wo, W1, W2, bo, b1, b2, gamma, beta). */
+typedef struct {
+    int64_t rows;
+    int32_t dtype, heads;
+    float eps;
+    const void *g_in, *s, *attn;
+    const void *w_post, *w_back;
+    const float* v_post;
+    const float* Z;
+    void *g_out, *d_attn;
+    float *nd, *partial;
+} tgt_node_bwd_post_args;
+int tgt_node_bwd_post(const tgt_node_bwd_post_args* args, void* stream);
+/* Fixed-order sums of such partials, all of a backward in one launch.  out: mats weights [rows, 64], mats biases [rows],
+ * gamma, beta [64] (NULL: not wanted). */
+typedef struct {
+    const float* partial;
+    int32_t workers, mats, rows;
+    void* out[8];
+} tgt_node_sum;
+int tgt_node_sums(const tgt_node_sum* sums, int count, int dtype, void* stream);
+/* tgt_sparse_attn_bwd for a caller that has already written the per-node side to the head of the workspace
+ * (tgt_node_bwd_post with nd = d_workspace): no bias, and out and Z are not read. */
+int tgt_sparse_attn_bwd_from_nd(const tgt_plan_t* plan, const void* d_q, const void* d_k, const void* d_v, int H, int d, int dtype,
+                                const void* d_dout, void* d_dq, void* d_dk, void* d_dv, void* d_workspace, int64_t workspace_bytes,
+                                void* stream);
+
 /* ---- per-kernel timing --------------------------------------------------
  * The reference times this path with torch.profiler around whole iterations
  * (attn_module.py:415-438).  When enabled, every kernel the library launches is

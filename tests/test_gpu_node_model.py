@@ -1,0 +1,78 @@
+"""The whole-model operators against the same models run layer by layer (whose kernels are compared with the oracle in
+test_gpu_encoder.py): output and every parameter gradient, at the sizes where the fused kernels can go wrong - row counts around
+a wave's 32 rows and a workgroup's 128 and 256, class counts around the halves of a row, odd feature widths, all head shapes.
+
+Bars: float32 1e-5 of the largest value of the tensor, bf16 6e-2 (the layer-by-layer path rounds every intermediate tensor)."""
+import pytest
+import torch
+
+from torchgt_amd import Graphormer, GraphPlan
+from torchgt_amd.graph_prep import fix_edge_index
+
+pytestmark = pytest.mark.gpu
+TOL = {torch.float32: 1e-5, torch.bfloat16: 6e-2}
+
+
+def random_edges(n, tokens, seed, device):
+    g = torch.Generator().manual_seed(seed)
+    e = torch.cat([torch.randint(0, n, (2, 5 * n), generator=g), torch.arange(n).repeat(2, 1)], 1).to(device)
+    return fix_edge_index(e, n) if tokens else e
+
+
+def scaled(model, seed, dtype, device):
+    g = torch.Generator().manual_seed(seed)
+    with torch.no_grad():
+        for p in model.parameters():
+            if p.dim() == 1:
+                p.add_(torch.randn(p.shape, generator=g) * 0.1)
+            else:
+                p.copy_(torch.randn(p.shape, generator=g) / p.shape[-1] ** 0.5)
+    return model.to(device, dtype)
+
+
+def compare(cls, model, x, plan, seed):
+    """(output, input gradient, parameter gradients) of both paths"""
+    w = torch.randn(x.shape[0], 64, generator=torch.Generator().manual_seed(seed)).to(x.device)
+    got = []
+    for fused in (True, False):
+        cls.one_operator = fused
+        try:
+            model.zero_grad(set_to_none=True)
+            xr = x.clone().requires_grad_(True)
+            out = model(xr, None, plan, attn_type="sparse")
+            (out.float() * w[:, :out.shape[1]]).sum().backward()
+            grads = {k: p.grad for k, p in model.named_parameters() if p.grad is not None}
+            got.append((out.detach(), xr.grad, grads))
+            with torch.no_grad():
+                assert torch.equal(model(x, None, plan, attn_type="sparse"), out)
+        finally:
+            cls.one_operator = True
+    tol = TOL[x.dtype]
+    worst = max(float(g.float().abs().max()) for g in got[1][2].values())
+    (o1, x1, g1), (o0, x0, g0) = got
+
+    def close(name, a, b, floor=0.0):
+        scale = max(float(b.float().abs().max()), floor)
+        err = float((a.float() - b.float()).abs().max()) / (scale or 1.0)
+        assert a.shape == b.shape and err <= tol, f"{name}: {err}"
+
+    close("output", o1, o0)
+    close("input gradient", x1, x0)
+    assert g1.keys() == g0.keys()
+    for k in g0:
+        # (a key bias moves all scores of a query alike: its gradient is rounding noise and is held to the largest gradient)
+        close(k, g1[k], g0[k], floor=worst * (1.0 if k.endswith("linear_k.bias") else 1e-2))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,features,classes,heads,layers", [(1, 32, 1, 8, 1), (30, 40, 5, 4, 2), (31, 100, 33, 8, 1), (32, 64, 32, 2, 2), (126, 72, 47, 8, 1),
+                                                             (127, 128, 64, 8, 2), (128, 65, 31, 4, 1), (256, 128, 40, 8, 3), (1000, 500, 47, 8, 2),
+                                                             (33333, 128, 40, 8, 2)])
+def test_node_graphormer_as_one_operator(cuda, dtype, n, features, classes, heads, layers):
+    print(f"node_graphormer case: n={n} features={features} classes={classes} heads={heads} layers={layers} {dtype}", flush=True)
+    torch.manual_seed(n)
+    model = scaled(Graphormer(layers, heads, features, 64, classes, 1, 0.0, 0.0, 0.0, 64, 1), n + 1, dtype, cuda)
+    x = torch.randn(n, features).to(cuda, dtype)
+    plan = GraphPlan(random_edges(n, 1, n + 2, cuda), n + 1)
+    assert model._one_operator(x, None, plan, None, "sparse")
+    compare(Graphormer, model, x, plan, n + 3)

@@ -108,6 +108,14 @@ SIGNATURES = {
     "tgt_embedding_sum_bwd_workspace_bytes": (_i64, [_i32, _i32]),
     "tgt_embedding_sum_bwd": (_i32, [_vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _i64, _vp]),
     "tgt_gen_edge_input": (_i32, [_vp, _vp, _i32, _i32, _vp, _i32, _i32, _i32, _vp, _vp]),
+    "tgt_node_frag_bytes": (_i64, [_i32, _i32]),
+    "tgt_node_pack": (_i32, [_vp, _vp, _vp, _i32, _vp, _vp, _i32, _i32, _vp, _vp, _vp]),
+    "tgt_node_fwd": (_i32, [_vp, _vp]),
+    "tgt_node_bwd_workers": (_i32, [_i64]),
+    "tgt_node_bwd_pre": (_i32, [_vp, _vp]),
+    "tgt_node_bwd_post": (_i32, [_vp, _vp]),
+    "tgt_node_sums": (_i32, [_vp, _i32, _i32, _vp]),
+    "tgt_sparse_attn_bwd_from_nd": (_i32, [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),
     "tgt_timing_enable": (_i32, [_i32]),
     "tgt_timing_reset": (_i32, []),
     "tgt_timing_slots": (_i32, []),

@@ -14,7 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(CSRC, "build")
 LIB_PATH = os.path.join(HERE, "libtorchgt_hip.so")
-EXT_SRC = os.path.join(CSRC, "torch_binding.cpp")
+EXT_SRCS = [os.path.join(CSRC, f) for f in ("torch_binding.cpp", "torch_models.cpp")]
 EXT_PATH = os.path.join(HERE, "_torchgt_ext.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -90,18 +90,24 @@ def build_extension(verbose=True):
     import torch
     from torch.utils import cpp_extension
     tlib = os.path.join(os.path.dirname(torch.__file__), "lib")
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
-    cmd += [f"-I{p}" for p in cpp_extension.include_paths()] + ["-I/opt/rocm/include", EXT_SRC, "-o", EXT_PATH + ".tmp",
-            f"-L{tlib}", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_hip", f"-L{HERE}", "-ltorchgt_hip",
-            "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{tlib}"]
+    cxx = os.environ.get("CXX", "g++")
+    flags = ["-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    flags += [f"-I{p}" for p in cpp_extension.include_paths()] + ["-I/opt/rocm/include"]
+    objs = [os.path.join(OBJ_DIR, os.path.basename(src) + ".ext") for src in EXT_SRCS]
+    cmds = [[cxx] + flags + ["-c", src, "-o", obj] for src, obj in zip(EXT_SRCS, objs)]
     t0 = time.time()
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    if r.returncode != 0:
-        raise RuntimeError("building the torch extension failed:\n" + r.stdout + r.stderr)
+    with ThreadPoolExecutor(max_workers=len(cmds)) as ex:
+        results = list(ex.map(lambda cmd: subprocess.run(cmd, capture_output=True, text=True), cmds))
+    results.append(subprocess.run([cxx, "-shared", "-o", EXT_PATH + ".tmp"] + objs +
+                                  [f"-L{tlib}", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_hip", f"-L{HERE}", "-ltorchgt_hip",
+                                   "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{tlib}"], capture_output=True, text=True))
+    for r in results:
+        if r.returncode != 0:
+            raise RuntimeError("building the torch extension failed:\n" + r.stdout + r.stderr)
     os.replace(EXT_PATH + ".tmp", EXT_PATH)
     if verbose:
-        print(f"[torchgt_amd.build] torch_binding.cpp: {time.time() - t0:.1f}s -> {EXT_PATH}")
+        print(f"[torchgt_amd.build] torch extension: {time.time() - t0:.1f}s -> {EXT_PATH}")
     return EXT_PATH
 
 

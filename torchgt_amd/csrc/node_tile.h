@@ -1,0 +1,400 @@
+// Building blocks of the fused per-node kernels (node_layer.hip): everything between two attention launches of an
+// encoder layer works on node rows of 64 features, so a wave takes 32 rows and keeps them in registers from the first
+// load to the last store.
+//
+// Register layout.  v_mfma_f32_32x32x16_bf16 leaves D[8 j + 4 h + t][c] in lane c + 32 h (register 4 j + t) and takes
+// operand B[k][c] in lane c + 32 h (eight k per lane).  With node rows as columns (c = node) and the rows of the
+// weights handed over in a permuted order, lane (node n, half h) of a product holds the output features 32 h .. 32 h + 31
+// of its node in register order, and these registers are the B operand of the next product as they stand: a chain of
+// linears, residual adds, LayerNorms and activations never leaves the registers.  LayerNorm sums are 32 adds in a lane
+// and one exchange between the halves.
+//
+// Number formats.  float32 rows go through the matrix unit as three bf16 planes (see linear.hip: hi + mid + lo is exact,
+// six products per pair of planes give the float32 product to a few 2^-23); bf16 rows as one.  P = number of planes.
+#pragma once
+#include "common.h"
+
+namespace tgt {
+namespace {
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float float16_t __attribute__((ext_vector_type(16)));
+typedef short short4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t vec16 __attribute__((ext_vector_type(4)));      // 16 bytes in registers
+struct nbf16 { uint16_t x; };
+
+template <typename T> struct Num;
+template <> struct Num<float> { static constexpr int P = 3; };
+template <> struct Num<nbf16> { static constexpr int P = 1; };
+
+// Lane (n = lane % 32, h = lane / 32) holds features 32 h .. 32 h + 31 of node n: at(i) is feature 32 h + i.
+struct Tile {
+    float v[32];
+    __device__ __forceinline__ float get(int i) const { return v[i]; }
+    __device__ __forceinline__ void set(int i, float x) { v[i] = x; }
+};
+#define TGT_EACH(i) _Pragma("unroll") for (int i = 0; i < 32; ++i)
+
+__device__ __forceinline__ void zero(Tile& t) { TGT_EACH(i) t.set(i, 0.f); }
+
+// the three parts of a float as float words whose lower half is zero (hi, mid) or unused (lo)
+__device__ __forceinline__ void cut3(float x, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+    hi = __float_as_uint(x) & 0xffff0000u;
+    const float r1 = x - __uint_as_float(hi);
+    mid = __float_as_uint(r1) & 0xffff0000u;
+    lo = __float_as_uint(r1 - __uint_as_float(mid));
+}
+__device__ __forceinline__ bf16x8_t upper8(const uint32_t (&w)[8]) {
+    vec16 u;
+    u.x = __builtin_amdgcn_perm(w[1], w[0], 0x07060302u);
+    u.y = __builtin_amdgcn_perm(w[3], w[2], 0x07060302u);
+    u.z = __builtin_amdgcn_perm(w[5], w[4], 0x07060302u);
+    u.w = __builtin_amdgcn_perm(w[7], w[6], 0x07060302u);
+    return __builtin_bit_cast(bf16x8_t, u);
+}
+__device__ __forceinline__ void to_planes(const float (&v)[8], bf16x8_t (&p)[3]) {
+    uint32_t a[8], b[8], c[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) cut3(v[i], a[i], b[i], c[i]);
+    p[0] = upper8(a); p[1] = upper8(b); p[2] = upper8(c);
+}
+__device__ __forceinline__ void to_planes(const float (&v)[8], bf16x8_t (&p)[1]) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) p[0][i] = static_cast<__bf16>(v[i]);
+}
+// the eight contraction indices of step s as matrix operands
+template <int P> __device__ __forceinline__ void step_planes(const Tile& t, int s, bf16x8_t (&p)[P]) {
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = t.get(8 * s + i);
+    to_planes(v, p);
+}
+
+__device__ __forceinline__ float16_t mma(bf16x8_t a, bf16x8_t b, float16_t c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+// c += a b for one contraction step in P planes each, small terms first
+__device__ __forceinline__ float16_t mma_planes(const bf16x8_t (&a)[3], const bf16x8_t (&b)[3], float16_t c) {
+    c = mma(a[2], b[0], c);
+    c = mma(a[0], b[2], c);
+    c = mma(a[1], b[1], c);
+    c = mma(a[1], b[0], c);
+    c = mma(a[0], b[1], c);
+    return mma(a[0], b[0], c);
+}
+__device__ __forceinline__ float16_t mma_planes(const bf16x8_t (&a)[1], const bf16x8_t (&b)[1], float16_t c) { return mma(a[0], b[0], c); }
+
+// A packed 64 x 64 weight: operand A of step s and row block m, plane p, at ((2 s + m) P + p) * 64 + lane (16 bytes per
+// lane): row block m, row 8 j + 4 hh + t is output feature 32 hh + 16 m + 4 j + t; a lane's eight contraction indices are
+// the input features 32 (lane / 32) + 8 s ... + 7.
+template <int P> constexpr int kFragVecs = 8 * P * 64;
+
+// Nothing is moved across: left alone, the scheduler asks for every operand of a product before its first instruction, and
+// the registers for that are not there
+__device__ __forceinline__ void fence_schedule() { __builtin_amdgcn_sched_barrier(0); }
+
+// B operands of a whole tile
+template <int P> struct Frags { bf16x8_t p[4][P]; };
+template <int P> __device__ __forceinline__ void make_frags(Frags<P>& f, const Tile& t) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) step_planes<P>(t, s, f.p[s]);
+}
+
+// acc += W b: w = packed weight in LDS, b = node rows (a tile, cut into planes one contraction step at a time, or planes);
+// the weight operands of the next step are asked for before the products of this one
+template <int P> struct StepWeights { bf16x8_t a[2][P]; };
+template <int P> __device__ __forceinline__ void step_weights(StepWeights<P>& f, const vec16* w, int s, int lane) {
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int p = 0; p < P; ++p) f.a[m][p] = __builtin_bit_cast(bf16x8_t, w[((2 * s + m) * P + p) * 64 + lane]);
+}
+template <int P> __device__ __forceinline__ void step_operand(bf16x8_t (&x)[P], const Tile& b, int s) { step_planes<P>(b, s, x); }
+template <int P> __device__ __forceinline__ void step_operand(bf16x8_t (&x)[P], const Frags<P>& b, int s) {
+#pragma unroll
+    for (int p = 0; p < P; ++p) x[p] = b.p[s][p];
+}
+template <int P, typename B> __device__ __forceinline__ void gemm(Tile& acc, const B& b, const vec16* w, int lane) {
+    StepWeights<P> f[2];
+    step_weights<P>(f[0], w, 0, lane);
+    float16_t c[2];
+    TGT_EACH(i) c[i >> 4][i & 15] = acc.get(i);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        if (s < 3) step_weights<P>(f[(s + 1) & 1], w, s + 1, lane);
+        bf16x8_t x[P];
+        step_operand<P>(x, b, s);
+#pragma unroll
+        for (int m = 0; m < 2; ++m) c[m] = mma_planes(f[s & 1].a[m], x, c[m]);
+        fence_schedule();
+    }
+    TGT_EACH(i) acc.set(i, c[i >> 4][i & 15]);
+}
+
+// LDS exchanges between lanes of one wave: the hardware runs a wave's LDS accesses in order, this keeps the compiler to it
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The 32 rows of a wave: first row and how many of them exist (wave-uniform, so the addresses have scalar bases)
+struct Rows {
+    int64_t first;
+    int left;       // <= 0: none
+    __device__ __forceinline__ Rows(int64_t tile, int64_t N) {
+        const int64_t r = N - tile * 32;
+        left = r > 32 ? 32 : (int)r;
+        first = left > 0 ? tile * 32 : 0;
+    }
+};
+
+// 32 node rows on their way between global memory (coalesced: consecutive lanes, consecutive 16-byte pieces) and the
+// register layout, through a wave-private LDS image of the rows.  Piece q of row r sits in slot q ^ (r mod pieces): both
+// the row-wise and the node-wise accesses spread over all banks, and the slots of a lane differ from its first one by an
+// exclusive or, which is formed at each access (kept in registers, the addresses of all accesses would crowd out the tiles).
+template <typename T> struct RowShape {
+    static constexpr int kPieces = 64 * (int)sizeof(T) / 16;      // 16-byte pieces of a row: 16 or 8
+    static constexpr int kPer = 64 / kPieces;                     // rows per access of the wave
+    static constexpr int kAcc = 32 / kPer;                        // accesses per tile
+    static constexpr int kVecs = 32 * kPieces;                    // 16-byte vectors of the image
+};
+template <typename T> struct Raw { vec16 v[RowShape<T>::kAcc]; };
+
+__device__ __forceinline__ int forgotten(int v) { asm volatile("" : "+v"(v)); return v; }
+// slot of access i of the row-wise walk: rows i * kPer ..., consecutive lanes along a row
+template <typename T> __device__ __forceinline__ int row_slot(int base, int i) {
+    constexpr int PP = RowShape<T>::kPieces, PER = RowShape<T>::kPer;
+    return (base ^ ((i * PER) & (PP - 1))) + i * PER * PP;
+}
+template <typename T> __device__ __forceinline__ int row_base(int lane) {
+    constexpr int PP = RowShape<T>::kPieces;
+    const int r = lane / PP;
+    return forgotten(r * PP + ((lane % PP) ^ r));
+}
+// slot of piece i of the lane's half of its node's row
+template <typename T> __device__ __forceinline__ int node_base(int lane) {
+    constexpr int PP = RowShape<T>::kPieces;
+    const int n = lane & 31, h = lane >> 5;
+    return forgotten(n * PP + ((h * (PP / 2)) ^ (n & (PP - 1))));
+}
+
+template <typename T> __device__ __forceinline__ void fetch(Raw<T>& raw, const T* __restrict__ src, const Rows& rows, int lane) {
+    constexpr int PP = RowShape<T>::kPieces, PER = RowShape<T>::kPer;
+    const vec16* p = reinterpret_cast<const vec16*>(src) + rows.first * PP;
+    const int last = rows.left > 0 ? rows.left - 1 : 0, r0 = forgotten(lane / PP), q = lane % PP;
+#pragma unroll
+    for (int i = 0; i < RowShape<T>::kAcc; ++i) {
+        const int r = r0 + i * PER;
+        raw.v[i] = p[(uint32_t)((r < last ? r : last) * PP + q)];
+    }
+}
+__device__ __forceinline__ void unpack16(const vec16& u, float (&f)[4], const float*) {
+    f[0] = __uint_as_float(u.x); f[1] = __uint_as_float(u.y); f[2] = __uint_as_float(u.z); f[3] = __uint_as_float(u.w);
+}
+__device__ __forceinline__ void unpack16(const vec16& u, float (&f)[8], const nbf16*) {
+    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        f[2 * i] = __uint_as_float(w[i] << 16);
+        f[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    }
+}
+__device__ __forceinline__ vec16 pack16(const float (&f)[4], const float*) {
+    return vec16{__float_as_uint(f[0]), __float_as_uint(f[1]), __float_as_uint(f[2]), __float_as_uint(f[3])};
+}
+__device__ __forceinline__ vec16 pack16(const float (&f)[8], const nbf16*) {
+    bf16x8_t b;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) b[i] = static_cast<__bf16>(f[i]);
+    return __builtin_bit_cast(vec16, b);
+}
+// ZERO: rows past the end read as zero (they enter sums over nodes); otherwise they repeat the last row
+template <typename T, bool ZERO> __device__ __forceinline__ void settle(Tile& t, Raw<T>& raw, vec16* stage, const Rows& rows, int lane) {
+    constexpr int PP = RowShape<T>::kPieces, PER = RowShape<T>::kPer, VE = 16 / (int)sizeof(T);
+    if (ZERO && rows.left < 32) {
+#pragma unroll
+        for (int i = 0; i < RowShape<T>::kAcc; ++i)
+            if (i * PER + lane / PP >= rows.left) raw.v[i] = vec16{0u, 0u, 0u, 0u};
+    }
+    wave_sync();
+    const int rb = row_base<T>(lane);
+#pragma unroll
+    for (int i = 0; i < RowShape<T>::kAcc; ++i) stage[row_slot<T>(rb, i)] = raw.v[i];
+    wave_sync();
+    const int nb = node_base<T>(lane);
+#pragma unroll
+    for (int i = 0; i < PP / 2; ++i) {
+        float f[VE];
+        unpack16(stage[nb ^ i], f, (const T*)nullptr);
+#pragma unroll
+        for (int e = 0; e < VE; ++e) t.set(i * VE + e, f[e]);
+    }
+}
+template <typename T> __device__ __forceinline__ void put_rows(T* __restrict__ dst, const Tile& t, vec16* stage, const Rows& rows, int lane) {
+    constexpr int PP = RowShape<T>::kPieces, PER = RowShape<T>::kPer, VE = 16 / (int)sizeof(T);
+    wave_sync();
+    const int nb = node_base<T>(lane);
+#pragma unroll
+    for (int i = 0; i < PP / 2; ++i) {
+        float f[VE];
+#pragma unroll
+        for (int e = 0; e < VE; ++e) f[e] = t.get(i * VE + e);
+        stage[nb ^ i] = pack16(f, (const T*)nullptr);
+    }
+    wave_sync();
+    vec16* p = reinterpret_cast<vec16*>(dst) + rows.first * PP;
+    const int rb = row_base<T>(lane), r0 = forgotten(lane / PP), q = lane % PP;
+    vec16 v[RowShape<T>::kAcc];
+#pragma unroll
+    for (int i = 0; i < RowShape<T>::kAcc; ++i) v[i] = stage[row_slot<T>(rb, i)];
+    if (rows.left >= 32) {
+#pragma unroll
+        for (int i = 0; i < RowShape<T>::kAcc; ++i) p[(uint32_t)((r0 + i * PER) * PP + q)] = v[i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < RowShape<T>::kAcc; ++i)
+            if (r0 + i * PER < rows.left) p[(uint32_t)((r0 + i * PER) * PP + q)] = v[i];
+    }
+}
+// the value as it will be read back from a T row
+__device__ __forceinline__ float stored(float v, const float*) { return v; }
+__device__ __forceinline__ float stored(float v, const nbf16*) { return static_cast<float>(static_cast<__bf16>(v)); }
+
+// v of this lane plus v of the lane that holds the other half of the node
+__device__ __forceinline__ float both_halves(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// vec: 64 floats in LDS
+__device__ __forceinline__ void load_vec(Tile& t, const float* vec, int h) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float4 f = *reinterpret_cast<const float4*>(vec + 32 * h + 4 * i);
+        t.set(4 * i, f.x); t.set(4 * i + 1, f.y); t.set(4 * i + 2, f.z); t.set(4 * i + 3, f.w);
+    }
+}
+// x -> (x - mean) * rstd over the 64 features; returns rstd
+__device__ __forceinline__ float normalise(Tile& x, float eps) {
+    float s = 0.f;
+    TGT_EACH(i) s += x.get(i);
+    const float mean = both_halves(s) * (1.f / 64);
+    float v = 0.f;
+    TGT_EACH(i) { const float d = x.get(i) - mean; v += d * d; }
+    const float rstd = rsqrtf(both_halves(v) * (1.f / 64) + eps);
+    TGT_EACH(i) x.set(i, (x.get(i) - mean) * rstd);
+    return rstd;
+}
+// xhat * gamma + beta, vectors in LDS
+__device__ __forceinline__ void affine(Tile& y, const Tile& xhat, const float* gamma, const float* beta, int h) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float4 g = *reinterpret_cast<const float4*>(gamma + 32 * h + 4 * i);
+        const float4 b = *reinterpret_cast<const float4*>(beta + 32 * h + 4 * i);
+        y.set(4 * i, xhat.get(4 * i) * g.x + b.x);
+        y.set(4 * i + 1, xhat.get(4 * i + 1) * g.y + b.y);
+        y.set(4 * i + 2, xhat.get(4 * i + 2) * g.z + b.z);
+        y.set(4 * i + 3, xhat.get(4 * i + 3) * g.w + b.w);
+    }
+}
+// g += LayerNorm backward of dy (gamma in LDS)
+__device__ __forceinline__ void ln_back(Tile& g, const Tile& dy, const Tile& xhat, float rstd, const float* gamma, int h) {
+    Tile d;
+    load_vec(d, gamma, h);
+    float c1 = 0.f, c2 = 0.f;
+    TGT_EACH(i) {
+        const float v = d.get(i) * dy.get(i);
+        d.set(i, v);
+        c1 += v;
+        c2 += v * xhat.get(i);
+    }
+    c1 = both_halves(c1) * (1.f / 64);
+    c2 = both_halves(c2) * (1.f / 64);
+    TGT_EACH(i) g.set(i, g.get(i) + rstd * (d.get(i) - c1 - xhat.get(i) * c2));
+}
+
+// Sum over the 32 nodes of every feature: lane l returns the sum of feature l.  A reduce-scatter over the lanes of a
+// half: at each of the five steps a lane hands half of its values to a partner and keeps the other half.  All exchanges are
+// operands of vector instructions (row swap, mirrors within 16 and 8 lanes, quad permutes), none goes through the LDS.
+template <int CTRL> __device__ __forceinline__ float lane_permuted(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <int BIT, int CTRL, int NV> __device__ __forceinline__ void scatter_step(float (&v)[NV], int lane) {
+    const bool up = (lane & BIT) != 0;
+#pragma unroll
+    for (int i = 0; i < BIT; ++i) {
+        const float keep = up ? v[i + BIT] : v[i], send = up ? v[i] : v[i + BIT];
+        v[i] = keep + lane_permuted<CTRL>(send);
+    }
+}
+__device__ __forceinline__ float column_sums(const Tile& t, int lane) {
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {      // rows of 16 lanes: the first keeps value i, the second value i + 16
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(t.get(i)), __float_as_uint(t.get(i + 16)), false, false);
+        v[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    scatter_step<8, 0x140>(v, lane);      // row_mirror
+    scatter_step<4, 0x141>(v, lane);      // row_half_mirror
+    scatter_step<2, 0x4e>(v, lane);       // quad_perm 2 3 0 1
+    scatter_step<1, 0xb1>(v, lane);       // quad_perm 1 0 3 2
+    return v[0];
+}
+
+// Makes the compiler forget what it knows about the values: without it, the planes of a tile that two products use (some
+// forty instructions' worth each) are computed once and kept in registers that are not there
+__device__ __forceinline__ void forget(Tile& t) {
+    TGT_EACH(i) asm volatile("" : "+v"(t.v[i]));
+}
+
+// ---- weight gradients: contraction over nodes ---------------------------------------------------------------------------
+// 128 node rows of an operand in LDS, P bf16 planes of 128 rows x 128 bytes; a wave writes its 32 rows as they sit in its
+// registers and the products read them back transposed (ds_read_b64_tr_b16: within 16 lanes, lane i hands over the address
+// of four consecutive elements of row i / 4 and receives column i of the four rows).  16-byte chunk c of row r sits in slot
+// c ^ (r mod 8): eight lanes of a write and sixteen of a transposed read touch different banks.
+constexpr int kPlaneBytes = 128 * 128;
+
+template <int P> __device__ __forceinline__ void put_planes(unsigned char* planes, int row, int h, const Frags<P>& f) {
+    const int base = forgotten(row * 128 + (((4 * h) ^ (row & 7)) << 4));
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int p = 0; p < P; ++p) *reinterpret_cast<bf16x8_t*>(planes + p * kPlaneBytes + (base ^ (s << 4))) = f.p[s][p];
+}
+// Address of a lane's first piece of the operand that has features 32 block .. + 31 as rows: nodes 8 (lane / 32) ... + 3
+__device__ __forceinline__ int operand_base(int block, int lane) {
+    const int i = lane & 15, chunk = 4 * block + 2 * ((lane >> 4) & 1) + ((i & 3) >> 1);
+    return (8 * (lane >> 5) + (i >> 2)) * 128 + ((chunk ^ (i >> 2)) << 4) + 8 * (i & 1);
+}
+template <int P> __device__ __forceinline__ void node_operand(bf16x8_t (&out)[P], const unsigned char* planes, int base, int node0) {
+    typedef __attribute__((address_space(3))) short4_t lds_short4;
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const unsigned char* q = planes + p * kPlaneBytes + node0 * 128;
+        const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(q + base));
+        const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(q + (base ^ 64) + 512));     // rows + 4
+        const uint2 a = __builtin_bit_cast(uint2, lo), b = __builtin_bit_cast(uint2, hi);
+        out[p] = __builtin_bit_cast(bf16x8_t, vec16{a.x, a.y, b.x, b.y});
+    }
+}
+// acc += dy^T x over the 128 nodes, one 32 x 32 block (bases of its rows and columns from operand_base); the operands of
+// the next sixteen nodes are asked for before the products of these
+template <int P> __device__ __forceinline__ void node_product(float16_t& acc, const unsigned char* dy, const unsigned char* x, int base_dy, int base_x) {
+    bf16x8_t a[2][P], b[2][P];
+    node_operand<P>(a[0], dy, base_dy, 0);
+    node_operand<P>(b[0], x, base_x, 0);
+#pragma unroll
+    for (int k = 0; k < 128; k += 16) {
+        const int now = (k >> 4) & 1;
+        if (k + 16 < 128) {
+            node_operand<P>(a[now ^ 1], dy, base_dy, k + 16);
+            node_operand<P>(b[now ^ 1], x, base_x, k + 16);
+        }
+        acc = mma_planes(a[now], b[now], acc);
+        fence_schedule();
+    }
+}
+
+}  // namespace
+}  // namespace tgt

@@ -1410,5 +1410,14 @@ int tgt_sparse_attn_bwd(const tgt_plan_t* plan, const void* d_q, const void* d_k
                                      d_dk, d_dv, d_dbias, d_workspace, workspace_bytes, stream, nullptr, false);
 }
 
+int tgt_sparse_attn_bwd_from_nd(const tgt_plan_t* plan, const void* d_q, const void* d_k, const void* d_v, int H, int d, int dtype,
+                                const void* d_dout, void* d_dq, void* d_dk, void* d_dv, void* d_workspace, int64_t workspace_bytes,
+                                void* stream) {
+    if (int rc = refuse_remaining(plan)) return rc;
+    // out and Z only feed the per-node side, which is there already: any non-null pointers will do
+    return tgt::sparse_attn_bwd_impl(plan, d_q, d_k, d_v, nullptr, TGT_BIAS_NONE, H, d, dtype, d_dout, static_cast<const float*>(d_dout),
+                                     d_dout, d_dq, d_dk, d_dv, nullptr, d_workspace, workspace_bytes, stream, nullptr, true);
+}
+
 }  // extern "C"
 #endif  // part 0: C entry points

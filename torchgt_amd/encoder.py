@@ -89,6 +89,21 @@ class EncoderLayer(nn.Module):
         return all(w % ve == 0 for w in widths) and att.num_heads * att.att_size == x.shape[-1] and all(
             lin.bias is not None for lin in (att.linear_q, att.linear_k, att.linear_v, att.output_layer, self.ffn.layer1, self.ffn.layer2))
 
+    def fits_one_operator(self, training):
+        """Whether a whole-model operator can take this layer: no dropout at work, 64 wide throughout, every bias there."""
+        att, ffn = self.self_attention, self.ffn
+        if not self.one_operator or not att.one_operator or (training and (self.self_attention_dropout.p > 0 or self.ffn_dropout.p > 0)):
+            return False
+        if att.output_layer is None or ffn.layer1.out_features != 64 or self.self_attention_norm.weight is None:
+            return False
+        return all(lin.bias is not None for lin in (att.linear_q, att.linear_k, att.linear_v, att.output_layer, ffn.layer1, ffn.layer2))
+
+    def parameters_in_order(self):
+        att, n1, n2, l1, l2 = self.self_attention, self.self_attention_norm, self.ffn_norm, self.ffn.layer1, self.ffn.layer2
+        q, k, v, o = att.linear_q, att.linear_k, att.linear_v, att.output_layer
+        return [n1.weight, n1.bias, q.weight, q.bias, k.weight, k.bias, v.weight, v.bias, o.weight, o.bias, n2.weight, n2.bias,
+                l1.weight, l1.bias, l2.weight, l2.bias]
+
     def forward(self, x, attn_bias=None, edge_index=None, attn_type=None, residual=None, defer_residual=False):
         """``residual``: a tensor still to be added to x (the previous layer's FFN output when it was
         called with ``defer_residual=True``); the add rides on this layer's first LayerNorm.
@@ -138,7 +153,44 @@ class Graphormer(nn.Module):
         self.graph_token_virtual_distance = nn.Embedding(self.num_global_node, attn_bias_dim)
         self.apply(lambda module: init_params(module, n_layers=n_layers))
 
+    one_operator = True      # False: always run the model layer by layer
+
+    def _one_operator(self, x, attn_bias, edge_index, perturb, attn_type):
+        """Whether ``torch.ops.torchgt.node_graphormer`` covers this call: sparse attention without a bias, hidden and
+        feed-forward width 64, at most 64 classes, no dropout at work, every linear with its bias, one dtype."""
+        if not self.one_operator or attn_type != "sparse" or attn_bias is not None or perturb is not None or edge_index is None:
+            return False
+        if self.hidden_dim != 64 or self.num_heads not in (2, 4, 8) or x.dim() != 2 or not x.is_cuda or x.dtype not in _DT:
+            return False
+        head = self.downstream_out_proj
+        if head.out_features > 64 or head.bias is None or self.node_encoder.bias is None or self.final_ln.weight is None:
+            return False
+        if self.training and self.input_dropout.p > 0:
+            return False
+        if x.dtype != head.weight.dtype or len(self.layers) == 0:
+            return False
+        return all(layer.fits_one_operator(self.training) for layer in self.layers)
+
+    def _parameters_in_order(self):
+        P = [self.node_encoder.weight, self.node_encoder.bias, self.graph_token.weight]
+        for layer in self.layers:
+            P += layer.parameters_in_order()
+        return P + [self.final_ln.weight, self.final_ln.bias, self.downstream_out_proj.weight, self.downstream_out_proj.bias]
+
     def forward(self, x, attn_bias, edge_index, perturb=None, attn_type=None):
+        if self._one_operator(x, attn_bias, edge_index, perturb, attn_type):
+            # the whole model as one operator and one autograd node over kernels that take a layer's node-local part
+            # in one pass each way
+            plan = edge_index if isinstance(edge_index, GraphPlan) else get_plan(edge_index, x.shape[0] + self.num_global_node)
+            plan.handle      # raises if the plan was closed
+            P = self._parameters_in_order()
+            pad = (-x.shape[1]) % (4 if x.dtype == torch.float32 else 8)
+            if pad:
+                x = F.pad(x, (0, pad))
+                P[0] = F.pad(P[0], (0, pad))
+            eps = [e for layer in self.layers for e in (layer.self_attention_norm.eps, layer.ffn_norm.eps)] + [self.final_ln.eps]
+            return _ext.ops().node_graphormer(x.contiguous(), P, plan.holder, plan.workspace(self.num_heads, 64 // self.num_heads),
+                                              self.num_heads, self.num_global_node, eps)
         x = x.unsqueeze(0)
         n_graph = x.shape[0]
         (node_feature,) = fused_linear(x, self.node_encoder)
