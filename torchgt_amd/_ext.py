@@ -23,3 +23,16 @@ def ops():
         torch.ops.load_library(EXT_PATH)
         _loaded = True
     return torch.ops.torchgt
+
+
+_entries = {}
+
+
+def op(name):
+    """The operator ``torch.ops.torchgt.<name>`` itself, bound once.  ``torch.ops`` looks through every argument of an
+    operator that takes a script object (a plan's holder) for traced stand-ins, which for a list of seventy parameters
+    costs more host time than the launches; nothing here is traced."""
+    entry = _entries.get(name)
+    if entry is None:
+        entry = _entries[name] = getattr(ops(), name).default._op
+    return entry

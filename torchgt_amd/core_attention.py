@@ -65,7 +65,7 @@ class SparseAttentionFunction:
                 else:
                     plan.edge_order()                  # makes sure the plan holds the map for this mode
         plan.handle      # raises if the plan was closed
-        return _ext.ops().sparse_attention(q, k, v, edge_bias, plan.holder, mode, plan.workspace(H, d))
+        return _ext.op("sparse_attention")(q, k, v, edge_bias, plan.holder, mode, plan.workspace(H, d))
 
 
 class DenseAttentionFunction:
@@ -77,7 +77,7 @@ class DenseAttentionFunction:
 
     @staticmethod
     def apply(q, k, v, bias, p_drop=0.0, seed=0, bf16_products=False):
-        return _ext.ops().dense_attention(q, k, v, bias, float(p_drop), int(seed), bool(bf16_products))
+        return _ext.op("dense_attention")(q, k, v, bias, float(p_drop), int(seed), bool(bf16_products))
 
 
 def dense_dropout_mask(b, S, H, p_drop, seed, device):
@@ -124,7 +124,7 @@ def dense_attention(q, k, v, attn_bias=None, p_drop=0.0, seed=None, bf16_product
         if ids.fits and (q.dtype == torch.bfloat16 or bf16_products):
             ab = None if ids.attn_bias is None else ids.attn_bias.to(q.dtype)
             try:
-                return _ext.ops().dense_attention_ids(q, k, v, ab, ids.sp16, ids.et16, ids.spatial_table.to(q.dtype),
+                return _ext.op("dense_attention_ids")(q, k, v, ab, ids.sp16, ids.et16, ids.spatial_table.to(q.dtype),
                                                       ids.edge_table.to(q.dtype), ids.virtual_dist.to(q.dtype), float(p_drop),
                                                       int(seed or 0), bool(bf16_products))
             except RuntimeError as exc:

@@ -17,6 +17,7 @@
 // operands into LDS, four waves (128 nodes) at a time, and every wave adds one 32 x 32 block over its share of the nodes.
 #include "node_tile.h"
 #include <algorithm>
+#include <atomic>
 
 namespace tgt {
 namespace {
@@ -114,7 +115,61 @@ template <typename T, bool POST, int NEXT> constexpr int fwd_lds() {
     return fwd_resident_mats<T, POST, NEXT>() * kFragVecs<Num<T>::P> * 16 + 10 * kVec * 4 + fwd_waves<T>() * RowShape<T>::kVecs * 16;
 }
 
-// rows of class values: a wave's 32 rows are 32 C consecutive elements of the [N - tokens, C] array
+// Rows of class values.  A wave's 32 rows are 32 C consecutive elements of the [N - tokens, C] array and travel through its
+// row image, in words: for bf16 the image starts one element late where the rows begin in the middle of a word.
+template <typename T> struct ClassRows {
+    static constexpr int kPerWord = 4 / (int)sizeof(T);
+    T* img;
+    int C, lo, hi;            // elements of the wave's rows that exist: [lo, hi)
+    int64_t first, total;     // element of the array the rows start at (negative: token rows), elements of the array
+    int shift;
+    __device__ __forceinline__ ClassRows(vec16* stage, int64_t row0, int64_t N, int tokens, int classes) {
+        C = classes;
+        const int64_t r = row0 - tokens, left = N - row0;
+        first = r * C; total = (N - tokens) * C;
+        lo = r < 0 ? (int)(-r < 32 ? -r : 32) * C : 0;
+        hi = (int)(left < 0 ? 0 : (left < 32 ? left : 32)) * C;
+        shift = kPerWord == 2 ? (int)(first & 1) : 0;
+        img = reinterpret_cast<T*>(stage) + shift;
+    }
+    __device__ __forceinline__ int words() const { return (hi + shift + kPerWord - 1) / kPerWord; }
+    // array -> image; every load is issued before the first is waited for
+    __device__ __forceinline__ void load(const T* __restrict__ src, int lane) {
+        const int n = words();
+        const int64_t w0 = (first - shift) / kPerWord, last = total / kPerWord - 1;
+        const uint32_t* p = reinterpret_cast<const uint32_t*>(src);
+        uint32_t v[32];
+#pragma unroll
+        for (int i = 0; i < 32; ++i)
+            if (i * 64 < n && last >= 0) {
+                int64_t w = w0 + i * 64 + lane;
+                w = w < 0 ? 0 : (w > last ? last : w);
+                v[i] = p[w];
+            }
+        wave_sync();
+        uint32_t* d = reinterpret_cast<uint32_t*>(img - shift);
+#pragma unroll
+        for (int i = 0; i < 32; ++i)
+            if (i * 64 < n && last >= 0 && i * 64 + lane < n) d[i * 64 + lane] = v[i];
+        wave_sync();
+        if (kPerWord == 2 && (total & 1) && first + hi == total && hi > lo && lane == 0) img[hi - 1] = src[total - 1];      // half a word at the end
+        wave_sync();
+    }
+    __device__ __forceinline__ void store(T* __restrict__ dst, int lane) const {
+        const uint32_t* d = reinterpret_cast<const uint32_t*>(img - shift);
+        T* out = dst + first;
+        const int n = words();
+        for (int w = lane; w < n; w += 64) {
+            const int e = w * kPerWord - shift;
+            if (e >= lo && e + kPerWord <= hi) *reinterpret_cast<uint32_t*>(out + e) = d[w];
+            else {
+#pragma unroll
+                for (int k = 0; k < kPerWord; ++k)
+                    if (e + k >= lo && e + k < hi) out[e + k] = img[e + k];
+            }
+        }
+    }
+};
 template <typename T> __device__ __forceinline__ T to_elem(float v);
 template <> __device__ __forceinline__ float to_elem<float>(float v) { return v; }
 template <> __device__ __forceinline__ nbf16 to_elem<nbf16>(float v) { return nbf16{__builtin_bit_cast(uint16_t, static_cast<__bf16>(v))}; }
@@ -179,8 +234,10 @@ __global__ __launch_bounds__(fwd_waves<T>() * 64) void k_node_fwd(const tgt_node
                 load_vec(y, vec + 3 * kVec, h);
                 gemm<P>(y, x, w + FV, lane);                      // u
                 TGT_EACH(i) {
-                    y.set(i, act_value<false>(y.get(i)));
-                    if (i % 4 == 3) fence_schedule();
+                    float cdf, bell;
+                    normal_cdf(y.get(i), cdf, bell);
+                    y.set(i, y.get(i) * cdf);
+                    if (i % 8 == 7) fence_schedule();
                 }
                 load_vec(x, vec + 4 * kVec, h);
                 TGT_EACH(i) s.set(i, s.get(i) + x.get(i));
@@ -217,15 +274,11 @@ __global__ __launch_bounds__(fwd_waves<T>() * 64) void k_node_fwd(const tgt_node
                 top = fmaxf(top, __shfl_xor(top, 32, 64));
                 TGT_EACH(i) if (32 * h + i < C) sum += expf(y.get(i) - top);
                 const float lse = top + logf(both_halves(sum));
-                T* img = reinterpret_cast<T*>(stage);
+                const ClassRows<T> out(stage, row0, N, a.tokens, C);
                 wave_sync();
-                TGT_EACH(i) if (32 * h + i < C) img[(lane & 31) * C + 32 * h + i] = to_elem<T>(y.get(i) - lse);
+                TGT_EACH(i) if (32 * h + i < C) out.img[(lane & 31) * C + 32 * h + i] = to_elem<T>(y.get(i) - lse);
                 wave_sync();
-                const int64_t first = row0 - a.tokens;
-                const int lo = first < 0 ? (int)(-first) * C : 0, hi = (int)(N - row0 < 32 ? N - row0 : 32) * C;
-                T* out = reinterpret_cast<T*>(a.logp) + first * C;
-                for (int e = lane; e < hi; e += 64)
-                    if (e >= lo) out[e] = img[e];
+                out.store(reinterpret_cast<T*>(a.logp), lane);
             }
         }
     }
@@ -267,27 +320,19 @@ template <int NM, int NV> __device__ __forceinline__ void write_partial(float* _
 // Class gradients of a wave's 32 rows: d logits = d logp - softmax * sum(d logp); zero for tokens and past the end.
 template <typename T> __device__ __forceinline__ void class_grads(Tile& d, const T* __restrict__ dlogp, const T* __restrict__ logp, int C, int tokens, int64_t row0, int64_t N,
                                                                   vec16* stage, int lane) {
-    T* img = reinterpret_cast<T*>(stage);
     const int n = lane & 31, h = lane >> 5;
-    const int64_t first = row0 - tokens, left = N - row0;
-    const int lo = first < 0 ? (int)(-first) * C : 0, hi = (int)(left < 32 ? left : 32) * C;
-    const bool in = row0 + n >= tokens && row0 + n < N;
-    float p[32], sum = 0.f;
-#pragma unroll
-    for (int pass = 0; pass < 2; ++pass) {
-        const T* src = (pass ? dlogp : logp) + first * C;
-        wave_sync();
-        for (int e = lane; e < hi; e += 64)
-            if (e >= lo) img[e] = src[e];
-        wave_sync();
-        TGT_EACH(i) {
-            const float v = in && 32 * h + i < C ? as_float(img[n * C + 32 * h + i]) : 0.f;
-            if (pass == 0) p[i] = in && 32 * h + i < C ? expf(v) : 0.f;
-            else { d.set(i, v); sum += v; }
-        }
+    ClassRows<T> rows(stage, row0, N, tokens, C);
+    const bool in = n * C >= rows.lo && n * C < rows.hi;
+    const T* mine = rows.img + (in ? n * C + 32 * h : 0);
+    rows.load(dlogp, lane);
+    float sum = 0.f;
+    TGT_EACH(i) {
+        d.set(i, in && 32 * h + i < C ? as_float(mine[i]) : 0.f);
+        sum += d.get(i);
     }
     sum = both_halves(sum);
-    TGT_EACH(i) d.set(i, d.get(i) - p[i] * sum);
+    rows.load(logp, lane);
+    TGT_EACH(i) if (in && 32 * h + i < C) d.set(i, d.get(i) - expf(as_float(mine[i])) * sum);
 }
 
 // ---- backward of the part in front of an attention (or of the classes) ------------------------------------------------------
@@ -448,10 +493,12 @@ __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_post(const tgt_node_bw
             gemm<P>(t, f, w, lane);                                 // u
             __syncthreads();                                        // W1 has been used
             TGT_EACH(i) {
-                const float u = t.get(i), cdf = 0.5f * (1.f + erff(u * 0.70710678118654752f));
+                const float u = t.get(i);
+                float cdf, bell;
+                normal_cdf(u, cdf, bell);
                 t.set(i, u * cdf);
-                slope.set(i, cdf + u * __expf(-0.5f * u * u) * 0.39894228040143268f);
-                if (i % 4 == 3) fence_schedule();
+                slope.set(i, cdf + u * bell * 0.39894228040143268f);
+                if (i % 8 == 7) fence_schedule();
             }
             make_frags(f, t);
             put_planes<P>(p_x, row, h, f);
@@ -595,36 +642,39 @@ int num_cus() {
 // a workgroup of `waves` waves per CU (LDS), fewer when there is less work
 int grid_for(int64_t rows, int waves) { return (int)std::max<int64_t>(1, std::min<int64_t>(num_cus(), ((rows + 31) / 32 + waves - 1) / waves)); }
 
-template <typename K> int allow_lds(K kernel, int bytes) {
-    if (bytes > 65536) TGT_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+// Raises the dynamic LDS limit of a kernel, once per kernel and device (`done`: one bit per device, kept by the caller)
+int allow_lds(const void* kernel, int bytes, std::atomic<uint64_t>& done) {
+    int dev = 0;
+    TGT_HIP_CHECK(hipGetDevice(&dev));
+    const uint64_t bit = 1ull << (dev & 63);
+    if (done.load(std::memory_order_relaxed) & bit) return TGT_OK;
+    TGT_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+    done.fetch_or(bit, std::memory_order_relaxed);
+    return TGT_OK;
+}
+template <typename... Args> int launch(void (*kernel)(Args...), std::atomic<uint64_t>& done, int grid, int threads, int lds, hipStream_t st, Args... args) {
+    if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), lds, done)) return rc;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds, st, args...);
+    TGT_HIP_CHECK(hipGetLastError());
     return TGT_OK;
 }
 
 template <typename T, bool POST, int NEXT> int launch_fwd(const tgt_node_fwd_args& a, hipStream_t st) {
-    constexpr int lds = fwd_lds<T, POST, NEXT>();
-    if (int rc = allow_lds(&k_node_fwd<T, POST, NEXT>, lds)) return rc;
-    hipLaunchKernelGGL((k_node_fwd<T, POST, NEXT>), dim3(grid_for(a.rows, fwd_waves<T>())), dim3(fwd_waves<T>() * 64), lds, st, a);
-    TGT_HIP_CHECK(hipGetLastError());
-    return TGT_OK;
+    static std::atomic<uint64_t> done{0};
+    return launch(&k_node_fwd<T, POST, NEXT>, done, grid_for(a.rows, fwd_waves<T>()), fwd_waves<T>() * 64, fwd_lds<T, POST, NEXT>(), st, a);
 }
 template <typename T> int dispatch_fwd(const tgt_node_fwd_args& a, hipStream_t st) {
     if (a.attn) return a.logp ? launch_fwd<T, true, NEXT_CLASSES>(a, st) : (a.q ? launch_fwd<T, true, NEXT_QKV>(a, st) : launch_fwd<T, true, NEXT_NONE>(a, st));
     return launch_fwd<T, false, NEXT_QKV>(a, st);
 }
 template <typename T> int dispatch_bwd_pre(const tgt_node_bwd_pre_args& a, int workers, hipStream_t st) {
-    constexpr int lds = BwdLds<T>::kBytes;
-    if (int rc = a.dlogp ? allow_lds(&k_node_bwd_pre<T, true>, lds) : allow_lds(&k_node_bwd_pre<T, false>, lds)) return rc;
-    if (a.dlogp) hipLaunchKernelGGL((k_node_bwd_pre<T, true>), dim3(workers), dim3(kBwdThreads), lds, st, a);
-    else hipLaunchKernelGGL((k_node_bwd_pre<T, false>), dim3(workers), dim3(kBwdThreads), lds, st, a);
-    TGT_HIP_CHECK(hipGetLastError());
-    return TGT_OK;
+    static std::atomic<uint64_t> done[2];
+    return a.dlogp ? launch(&k_node_bwd_pre<T, true>, done[1], workers, kBwdThreads, BwdLds<T>::kBytes, st, a)
+                   : launch(&k_node_bwd_pre<T, false>, done[0], workers, kBwdThreads, BwdLds<T>::kBytes, st, a);
 }
 template <typename T> int dispatch_bwd_post(const tgt_node_bwd_post_args& a, int workers, hipStream_t st) {
-    constexpr int lds = BwdLds<T>::kBytes;
-    if (int rc = allow_lds(&k_node_bwd_post<T>, lds)) return rc;
-    hipLaunchKernelGGL((k_node_bwd_post<T>), dim3(workers), dim3(kBwdThreads), lds, st, a);
-    TGT_HIP_CHECK(hipGetLastError());
-    return TGT_OK;
+    static std::atomic<uint64_t> done{0};
+    return launch(&k_node_bwd_post<T>, done, workers, kBwdThreads, BwdLds<T>::kBytes, st, a);
 }
 bool dtype_ok(int dtype) { return dtype == TGT_DTYPE_F32 || dtype == TGT_DTYPE_BF16; }
 

@@ -314,6 +314,25 @@ __device__ __forceinline__ void ln_back(Tile& g, const Tile& dy, const Tile& xha
     TGT_EACH(i) g.set(i, g.get(i) + rstd * (d.get(i) - c1 - xhat.get(i) * c2));
 }
 
+// Standard normal distribution function and exp(-u^2 / 2), what GELU and its derivative are made of.  For z = |u| the upper
+// tail is exp(-z^2 / 2) R(1 / (1 + 0.325 z)) with a polynomial R of degree 7 without constant term (weighted least squares
+// fit of the scaled complementary error function, made for this kernel: 2.2e-9 from the exact tail everywhere); with the
+// roundings of float32 u * cdf is within 3.9e-7 of the exact product on [-8, 8], where 0.5 (1 + erff(u / sqrt 2)) is within
+// 4.5e-7.  About twenty instructions without a branch, the exponential shared by value and derivative, instead of fifty.
+__device__ __forceinline__ void normal_cdf(float u, float& cdf, float& bell) {
+    const float t = __builtin_amdgcn_rcpf(fmaf(fabsf(u), 0.325f, 1.f));
+    bell = __builtin_amdgcn_exp2f(u * u * -0.72134752044448170f);
+    float r = 0.044371370618908994f;
+    r = fmaf(r, t, -0.2242534139094417f);
+    r = fmaf(r, t, 0.3557655723199327f);
+    r = fmaf(r, t, -0.11197278379825516f);
+    r = fmaf(r, t, 0.1901310032946691f);
+    r = fmaf(r, t, 0.11514759226601201f);
+    r = fmaf(r, t, 0.1308106570246585f);
+    const float tail = r * t * bell;
+    cdf = u > 0.f ? 1.f - tail : tail;
+}
+
 // Sum over the 32 nodes of every feature: lane l returns the sum of feature l.  A reduce-scatter over the lanes of a
 // half: at each of the five steps a lane hands half of its values to a partner and keeps the other half.  All exchanges are
 // operands of vector instructions (row swap, mirrors within 16 and 8 lanes, quad permutes), none goes through the LDS.

@@ -13,6 +13,7 @@ supports); with a positive rate in training mode torch's dropout is applied at
 the reference's places, with torch's random stream.
 """
 import math
+import weakref
 
 import torch
 import torch.nn as nn
@@ -30,7 +31,7 @@ def nll_loss(log_probs, target, ignore_index=-100):
     single workgroup, ~95 + 60 us forward + backward for 64 K rows against ~5 + 3 here).  A target outside
     [0, C) other than ``ignore_index`` counts as ignored - torch raises there: check labels that may be corrupt
     before they reach the loss."""
-    return _ext.ops().nll_loss(log_probs, target, int(ignore_index))
+    return _ext.op("nll_loss")(log_probs, target, int(ignore_index))
 
 
 def init_params(module, n_layers):
@@ -41,6 +42,72 @@ def init_params(module, n_layers):
             module.bias.data.zero_()
     if isinstance(module, nn.Embedding):
         module.weight.data.normal_(mean=0.0, std=0.02)
+
+
+# a layer's parameters in the order of the whole-model operators
+LAYER_PARAMETERS = [f"{m}.{k}" for m in ("self_attention_norm", "self_attention.linear_q", "self_attention.linear_k", "self_attention.linear_v",
+                                         "self_attention.output_layer", "ffn_norm", "ffn.layer1", "ffn.layer2") for k in ("weight", "bias")]
+
+
+class ModuleTree:
+    """Where a model's parameters are: for the whole-model operators, whose host time is counted in microseconds, the
+    attribute look-ups of seventy parameters through ``nn.Module`` would be a third of it.  Remembers the dictionaries of the
+    modules, not the parameters, and notices when a module of the tree was exchanged (``current``)."""
+
+    def __init__(self, root, names, dropouts, square=64):
+        self.links, self.slots, self.square = [], [], square
+        seen = set()
+
+        def step(module, name):
+            child = module._modules.get(name)
+            if (id(module), name) not in seen:
+                seen.add((id(module), name))
+                self.links.append((module._modules, name, child))
+            return child
+
+        self.missing = False
+        for full in names:
+            *path, leaf = full.split(".")
+            m = root
+            for part in path:
+                m = step(m, part) if m is not None else None
+            if m is None:
+                self.missing = True
+                return
+            self.slots.append((m._parameters, leaf))
+        self.count = len(root.layers)
+        self.layers = root.layers._modules
+        self.dropouts = [m for n, m in root.named_modules() if n.rsplit(".", 1)[-1] in dropouts]
+        self.shapes = None
+
+    def current(self):
+        if self.missing or len(self.layers) != self.count:
+            return False
+        for d, name, child in self.links:
+            if d.get(name) is not child:
+                return False
+        return True
+
+    def parameters(self, dtype, training):
+        """The parameters in order, or None: one is absent, has another dtype, a layer is not square, or dropout is at work."""
+        if self.missing or self.count == 0:
+            return None
+        if training:
+            for m in self.dropouts:
+                if m.p > 0:
+                    return None
+        P = [d.get(name) for d, name in self.slots]
+        for p in P:
+            if p is None or p.dtype is not dtype:
+                return None
+        # the layers' parameters (everything but the first three and the last four): 64 wide throughout
+        for p in P[3:-4]:
+            if p.shape[0] != self.square or p.shape[-1] != self.square:
+                return None
+        return P
+
+
+_TREES = weakref.WeakKeyDictionary()      # model -> ModuleTree (which holds the model's modules, not the model)
 
 
 class FeedForwardNetwork(nn.Module):
@@ -55,9 +122,9 @@ class FeedForwardNetwork(nn.Module):
         ve = 4 if x.dtype == torch.float32 else 8
         if x.is_cuda and l1.bias is not None and l2.bias is not None and not (l1.in_features % ve or l1.out_features % ve or l2.out_features % ve):
             # one operator: GELU in the epilogue of layer1 (64 -> 64) and in the input gradient of layer2
-            return _ext.ops().ffn(x, l1.weight, l1.bias, l2.weight, l2.bias)
+            return _ext.op("ffn")(x, l1.weight, l1.bias, l2.weight, l2.bias)
         (u,) = fused_linear(x, l1)
-        h = _ext.ops().gelu(u)
+        h = _ext.op("gelu")(u)
         (y,) = fused_linear(h, l2)
         return y
 
@@ -89,21 +156,6 @@ class EncoderLayer(nn.Module):
         return all(w % ve == 0 for w in widths) and att.num_heads * att.att_size == x.shape[-1] and all(
             lin.bias is not None for lin in (att.linear_q, att.linear_k, att.linear_v, att.output_layer, self.ffn.layer1, self.ffn.layer2))
 
-    def fits_one_operator(self, training):
-        """Whether a whole-model operator can take this layer: no dropout at work, 64 wide throughout, every bias there."""
-        att, ffn = self.self_attention, self.ffn
-        if not self.one_operator or not att.one_operator or (training and (self.self_attention_dropout.p > 0 or self.ffn_dropout.p > 0)):
-            return False
-        if att.output_layer is None or ffn.layer1.out_features != 64 or self.self_attention_norm.weight is None:
-            return False
-        return all(lin.bias is not None for lin in (att.linear_q, att.linear_k, att.linear_v, att.output_layer, ffn.layer1, ffn.layer2))
-
-    def parameters_in_order(self):
-        att, n1, n2, l1, l2 = self.self_attention, self.self_attention_norm, self.ffn_norm, self.ffn.layer1, self.ffn.layer2
-        q, k, v, o = att.linear_q, att.linear_k, att.linear_v, att.output_layer
-        return [n1.weight, n1.bias, q.weight, q.bias, k.weight, k.bias, v.weight, v.bias, o.weight, o.bias, n2.weight, n2.bias,
-                l1.weight, l1.bias, l2.weight, l2.bias]
-
     def forward(self, x, attn_bias=None, edge_index=None, attn_type=None, residual=None, defer_residual=False):
         """``residual``: a tensor still to be added to x (the previous layer's FFN output when it was
         called with ``defer_residual=True``); the add rides on this layer's first LayerNorm.
@@ -118,18 +170,18 @@ class EncoderLayer(nn.Module):
                       att.linear_v.weight, att.linear_v.bias, att.output_layer.weight, att.output_layer.bias, n2.weight, n2.bias,
                       self.ffn.layer1.weight, self.ffn.layer1.bias, self.ffn.layer2.weight, self.ffn.layer2.bias]
             plan.handle      # raises if the plan was closed
-            x, y = _ext.ops().encoder_layer(x, residual, params, plan.holder, plan.workspace(att.num_heads, att.att_size),
+            x, y = _ext.op("encoder_layer")(x, residual, params, plan.holder, plan.workspace(att.num_heads, att.att_size),
                                             att.num_heads, n1.eps, n2.eps)
-            return (x, y) if defer_residual else _ext.ops().add(x, y)
-        x, y = _ext.ops().add_layer_norm(x, residual, n1.weight, n1.bias, float(n1.eps))
+            return (x, y) if defer_residual else _ext.op("add")(x, y)
+        x, y = _ext.op("add_layer_norm")(x, residual, n1.weight, n1.bias, float(n1.eps))
         y = self.self_attention(y, attn_bias, edge_index, attn_type=attn_type)
         y = self.self_attention_dropout(y)
-        x, y = _ext.ops().add_layer_norm(x, y, n2.weight, n2.bias, float(n2.eps))
+        x, y = _ext.op("add_layer_norm")(x, y, n2.weight, n2.bias, float(n2.eps))
         y = self.ffn(y)
         y = self.ffn_dropout(y)
         if defer_residual:
             return x, y
-        return _ext.ops().add(x, y)
+        return _ext.op("add")(x, y)
 
 
 class Graphormer(nn.Module):
@@ -156,40 +208,37 @@ class Graphormer(nn.Module):
     one_operator = True      # False: always run the model layer by layer
 
     def _one_operator(self, x, attn_bias, edge_index, perturb, attn_type):
-        """Whether ``torch.ops.torchgt.node_graphormer`` covers this call: sparse attention without a bias, hidden and
-        feed-forward width 64, at most 64 classes, no dropout at work, every linear with its bias, one dtype."""
+        """The model's parameters in the operator's order when ``torch.ops.torchgt.node_graphormer`` covers this call - sparse
+        attention without a bias, hidden and feed-forward width 64, at most 64 classes, no dropout at work, every linear with
+        its bias, one dtype - else None."""
         if not self.one_operator or attn_type != "sparse" or attn_bias is not None or perturb is not None or edge_index is None:
-            return False
+            return None
         if self.hidden_dim != 64 or self.num_heads not in (2, 4, 8) or x.dim() != 2 or not x.is_cuda or x.dtype not in _DT:
-            return False
-        head = self.downstream_out_proj
-        if head.out_features > 64 or head.bias is None or self.node_encoder.bias is None or self.final_ln.weight is None:
-            return False
-        if self.training and self.input_dropout.p > 0:
-            return False
-        if x.dtype != head.weight.dtype or len(self.layers) == 0:
-            return False
-        return all(layer.fits_one_operator(self.training) for layer in self.layers)
+            return None
+        tree = _TREES.get(self)
+        if tree is None or not tree.current():
+            tree = _TREES[self] = ModuleTree(self, self._parameter_names(), ["self_attention_dropout", "ffn_dropout", "input_dropout"])
+        return tree.parameters(x.dtype, self.training)
 
-    def _parameters_in_order(self):
-        P = [self.node_encoder.weight, self.node_encoder.bias, self.graph_token.weight]
-        for layer in self.layers:
-            P += layer.parameters_in_order()
-        return P + [self.final_ln.weight, self.final_ln.bias, self.downstream_out_proj.weight, self.downstream_out_proj.bias]
+    def _parameter_names(self):
+        names = ["node_encoder.weight", "node_encoder.bias", "graph_token.weight"]
+        for i in range(len(self.layers)):
+            names += [f"layers.{i}.{k}" for k in LAYER_PARAMETERS]
+        return names + ["final_ln.weight", "final_ln.bias", "downstream_out_proj.weight", "downstream_out_proj.bias"]
 
     def forward(self, x, attn_bias, edge_index, perturb=None, attn_type=None):
-        if self._one_operator(x, attn_bias, edge_index, perturb, attn_type):
+        P = self._one_operator(x, attn_bias, edge_index, perturb, attn_type)
+        if P is not None and P[-1].shape[0] <= 64 and all(layer.one_operator and layer.self_attention.one_operator for layer in self.layers):
             # the whole model as one operator and one autograd node over kernels that take a layer's node-local part
             # in one pass each way
             plan = edge_index if isinstance(edge_index, GraphPlan) else get_plan(edge_index, x.shape[0] + self.num_global_node)
             plan.handle      # raises if the plan was closed
-            P = self._parameters_in_order()
             pad = (-x.shape[1]) % (4 if x.dtype == torch.float32 else 8)
             if pad:
                 x = F.pad(x, (0, pad))
                 P[0] = F.pad(P[0], (0, pad))
             eps = [e for layer in self.layers for e in (layer.self_attention_norm.eps, layer.ffn_norm.eps)] + [self.final_ln.eps]
-            return _ext.ops().node_graphormer(x.contiguous(), P, plan.holder, plan.workspace(self.num_heads, 64 // self.num_heads),
+            return _ext.op("node_graphormer")(x.contiguous(), P, plan.holder, plan.workspace(self.num_heads, 64 // self.num_heads),
                                               self.num_heads, self.num_global_node, eps)
         x = x.unsqueeze(0)
         n_graph = x.shape[0]
@@ -215,7 +264,7 @@ class Graphormer(nn.Module):
             output, pending = enc_layer(output, attn_bias=graph_attn_bias, edge_index=edge_index, attn_type=attn_type,
                                         residual=pending, defer_residual=True)
         fl = self.final_ln
-        _, output = _ext.ops().add_layer_norm(output, pending, fl.weight, fl.bias, float(fl.eps))
+        _, output = _ext.op("add_layer_norm")(output, pending, fl.weight, fl.bias, float(fl.eps))
         # rows 1.. of graph 0 (:391 `output[0, 1:, :]`); through a view, so that autograd pads the gradient once, not twice
         (output,) = fused_linear(output.reshape(-1, self.hidden_dim)[1:output.shape[1]], self.downstream_out_proj)
         return F.log_softmax(output, dim=1)

@@ -138,7 +138,7 @@ class GraphAttnBias(nn.Module):
             sp_w, e_w, vd_w = self.spatial_pos_encoder.weight, self.edge_encoder.weight, self.graph_token_virtual_distance.weight
             if not batched_data.attn_bias.is_cuda:
                 raise RuntimeError("GraphAttnBias runs on the GPU only (no CPU fallback)")
-            sp16, et16 = _ext.ops().dense_ids_pack(batched_data.spatial_pos, batched_data.attn_edge_type, sp_w.shape[0], e_w.shape[0])
+            sp16, et16 = _ext.op("dense_ids_pack")(batched_data.spatial_pos, batched_data.attn_edge_type, sp_w.shape[0], e_w.shape[0])
             build = lambda: GraphAttnBiasFunction.apply(batched_data.attn_bias, batched_data.spatial_pos,
                                                         batched_data.attn_edge_type, sp_w, e_w, vd_w)
             return GraphBiasIds(batched_data.attn_bias, sp16, et16, sp_w, e_w, vd_w, build)

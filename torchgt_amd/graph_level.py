@@ -142,22 +142,22 @@ class EncoderLayer(nn.Module):
                       att.linear_v.weight, att.linear_v.bias, att.output_layer.weight, att.output_layer.bias, n2.weight, n2.bias,
                       self.ffn.layer1.weight, self.ffn.layer1.bias, self.ffn.layer2.weight, self.ffn.layer2.bias]
             try:
-                x2, y = _ext.ops().dense_encoder_layer(x, residual, params, extra, ab, sp16, et16, att.num_heads, n1.eps, n2.eps, p,
+                x2, y = _ext.op("dense_encoder_layer")(x, residual, params, extra, ab, sp16, et16, att.num_heads, n1.eps, n2.eps, p,
                                                        seed, bool(core.dense_bf16_products))
-                return (x2, y) if defer_residual else _ext.ops().add(x2, y)
+                return (x2, y) if defer_residual else _ext.op("add")(x2, y)
             except RuntimeError as exc:
                 if sp16 is None or "bytes of LDS" not in str(exc):
                     raise
                 attn_bias.fits = False       # this shape needs the bias tensor: the attention below builds it once
-        x, y = _ext.ops().add_layer_norm(x, residual, n1.weight, n1.bias, float(n1.eps))
+        x, y = _ext.op("add_layer_norm")(x, residual, n1.weight, n1.bias, float(n1.eps))
         y = self.self_attention(y, attn_bias, None, attn_type="full")
         y = self.self_attention_dropout(y)
-        x, y = _ext.ops().add_layer_norm(x, y, n2.weight, n2.bias, float(n2.eps))
+        x, y = _ext.op("add_layer_norm")(x, y, n2.weight, n2.bias, float(n2.eps))
         y = self.ffn(y)
         y = self.ffn_dropout(y)
         if defer_residual:
             return x, y
-        return _ext.ops().add(x, y)
+        return _ext.op("add")(x, y)
 
 
 class Graphormer(nn.Module):
@@ -200,7 +200,7 @@ class Graphormer(nn.Module):
         for enc_layer in self.layers:
             output, pending = enc_layer(output, attn_bias, mask=None, residual=pending, defer_residual=True)
         fl = self.final_ln
-        _, output = _ext.ops().add_layer_norm(output, pending, fl.weight, fl.bias, float(fl.eps))
+        _, output = _ext.op("add_layer_norm")(output, pending, fl.weight, fl.bias, float(fl.eps))
         head = self.out_proj if hasattr(self, "out_proj") else self.downstream_out_proj
         (output,) = fused_linear(output[:, 0, :].contiguous(), head)      # the virtual node's row (:387)
         return output

@@ -25,7 +25,7 @@ class ReluFunction:
 
     @staticmethod
     def apply(u):
-        return _ext.ops().relu(u)
+        return _ext.op("relu")(u)
 
 
 class EncoderLayer(nn.Module):
@@ -49,12 +49,12 @@ class EncoderLayer(nn.Module):
         y = self.self_attention(x, attn_bias, edge_index=edge_index, attn_type=attn_type)      # :244
         y = self.self_attention_dropout(y)
         (y,) = fused_linear(y, self.O)                                                         # :246
-        _, x = _ext.ops().add_layer_norm(x, y, n1.weight, n1.bias, float(n1.eps))                    # :247-248
+        _, x = _ext.op("add_layer_norm")(x, y, n1.weight, n1.bias, float(n1.eps))                    # :247-248
         (y,) = fused_linear(y, self.FFN_layer1)                                                # :254
         y = ReluFunction.apply(y)
         y = self.self_attention_dropout(y)
         (y,) = fused_linear(y, self.FFN_layer2)
-        _, x = _ext.ops().add_layer_norm(x, y, n2.weight, n2.bias, float(n2.eps))                    # :258-259
+        _, x = _ext.op("add_layer_norm")(x, y, n2.weight, n2.bias, float(n2.eps))                    # :258-259
         return x
 
 

@@ -36,7 +36,7 @@ class LinearFunction:
         Ws, bs = list(wb[0::2]), list(wb[1::2])
         if not 1 <= len(Ws) <= 3 or len(bs) != len(Ws):
             raise ValueError("LinearFunction takes 1 to 3 (weight, bias) pairs")
-        return tuple(_ext.ops().linear(x, Ws, bs))
+        return tuple(_ext.op("linear")(x, Ws, bs))
 
 
 def fused_linear(x, *layers):
@@ -117,7 +117,7 @@ class MultiHeadAttention(nn.Module):
             if self.output_layer is not None:
                 params += [self.output_layer.weight, self.output_layer.bias]
             plan.handle      # raises if the plan was closed
-            return _ext.ops().multi_head_attention(x, params, plan.holder, plan.workspace(self.num_heads, self.att_size), self.num_heads)
+            return _ext.op("multi_head_attention")(x, params, plan.holder, plan.workspace(self.num_heads, self.att_size), self.num_heads)
         batch_size = x.size(0)
         q, k, v = fused_linear(x, self.linear_q, self.linear_k, self.linear_v)
         q = q.view(batch_size, -1, self.num_heads, self.att_size)
