@@ -506,6 +506,13 @@ int tgt_graph_attn_bias_bwd(const void* d_dout, const int64_t* d_spatial_pos, co
                             int num_spatial, int num_edges, int b, int s, int H, int dtype, void* d_dspatial_table,
                             void* d_dedge_table, void* d_dvirtual_dist, void* d_workspace, int64_t workspace_bytes,
                             void* stream);
+/* The same for the sum of n_douts (1 to 4) gradients of one bias, which is what the layers of a model that share it leave: a HOST
+ * array of device pointers, read side by side and added in float32.  More than one: at most 8 heads and one edge feature
+ * (TGT_ERR_UNSUPPORTED otherwise). */
+int tgt_graph_attn_bias_bwd_sum(const void* const* d_douts, int n_douts, const int64_t* d_spatial_pos, const int64_t* d_edge_type, int F,
+                                int num_spatial, int num_edges, int b, int s, int H, int dtype, void* d_dspatial_table,
+                                void* d_dedge_table, void* d_dvirtual_dist, void* d_workspace, int64_t workspace_bytes,
+                                void* stream);
 /* GraphNodeFeature.forward (models/graphormer_graph_level.py:18-60): the input rows of the
  * graph-level model, virtual node first:
  *   out[g, 0, :]     = graph_token
@@ -646,6 +653,13 @@ typedef struct {
     void* out[8];
 } tgt_node_sum;
 int tgt_node_sums(const tgt_node_sum* sums, int count, int dtype, void* stream);
+/* The head of the graph-level models (models/graphormer_graph_level.py:383-388: final LayerNorm, the virtual node's row, output
+ * projection): y[g] = LN(s[g, 0]) W^T + bias for s [b, S, 64], W [outputs, 64], 1 to 64 outputs.  Backward: g_out [b, S, 64] =
+ * gradient of s (zero but for the virtual nodes' rows), dW, dbias, dgamma, dbeta (added in a fixed order). */
+int tgt_graph_head_fwd(const void* d_s, const void* d_gamma, const void* d_beta, float eps, const void* d_W, const void* d_bias, int b, int S,
+                       int outputs, int dtype, void* d_y, void* stream);
+int tgt_graph_head_bwd(const void* d_s, const void* d_gamma, const void* d_beta, float eps, const void* d_W, const void* d_dy, int b, int S,
+                       int outputs, int dtype, void* d_g_out, void* d_dW, void* d_dbias, void* d_dgamma, void* d_dbeta, void* stream);
 /* tgt_sparse_attn_bwd for a caller that has already written the per-node side to the head of the workspace
  * (tgt_node_bwd_post with nd = d_workspace): no bias, and out and Z are not read. */
 int tgt_sparse_attn_bwd_from_nd(const tgt_plan_t* plan, const void* d_q, const void* d_k, const void* d_v, int H, int d, int dtype,

@@ -3,10 +3,12 @@ test_gpu_encoder.py): output and every parameter gradient, at the sizes where th
 a wave's 32 rows and a workgroup's 128 and 256, class counts around the halves of a row, odd feature widths, all head shapes.
 
 Bars: float32 1e-5 of the largest value of the tensor, bf16 6e-2 (the layer-by-layer path rounds every intermediate tensor)."""
+import types
+
 import pytest
 import torch
 
-from torchgt_amd import Graphormer, GraphPlan
+from torchgt_amd import GraphLevelGraphormer, Graphormer, GraphPlan
 from torchgt_amd.graph_prep import fix_edge_index
 
 pytestmark = pytest.mark.gpu
@@ -76,3 +78,42 @@ def test_node_graphormer_as_one_operator(cuda, dtype, n, features, classes, head
     plan = GraphPlan(random_edges(n, 1, n + 2, cuda), n + 1)
     assert model._one_operator(x, None, plan, None, "sparse") is not None
     compare(Graphormer, model, x, plan, n + 3)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("b,s,outputs,heads,layers,edge_type,features,p_drop", [(1, 1, 1, 8, 1, "single_hop", 1, 0.0), (3, 31, 17, 8, 4, "single_hop", 1, 0.0),
+                                                                              (17, 40, 64, 4, 5, "single_hop", 1, 0.3), (5, 70, 2, 2, 2, "single_hop", 3, 0.0),
+                                                                              (33, 24, 1, 8, 3, "multi_hop", 1, 0.1)])
+def test_graph_graphormer_as_one_operator(cuda, dtype, b, s, outputs, heads, layers, edge_type, features, p_drop):
+    """The whole graph-level model against its layers one by one: one to five layers share the bias (up to four gradients of it
+    are folded into the tables side by side, one edge feature or several), outputs around the sixteen of a pass."""
+    print(f"graph_graphormer case: b={b} s={s} outputs={outputs} heads={heads} layers={layers} {edge_type} {dtype}", flush=True)
+    torch.manual_seed(b)
+    model = GraphLevelGraphormer(layers, heads, 64, 0.0, 0.0, 64, "ZINC", edge_type, 5, p_drop, outputs)
+    model = scaled(model, b + 1, dtype, cuda)
+    with torch.no_grad():      # queries of a size whose products mean something in bf16 (the layer multiplies them by sqrt(d))
+        for layer in model.layers:
+            layer.self_attention.linear_q.weight.mul_(0.2)
+    g = torch.Generator().manual_seed(b + 2)
+    ids = lambda hi, *shape: torch.randint(0, hi, shape, generator=g).to(cuda)
+    batch = types.SimpleNamespace(x=ids(64, b, s, 1), in_degree=ids(64, b, s), out_degree=ids(64, b, s), attn_bias=torch.zeros(b, s + 1, s + 1, device=cuda, dtype=dtype),
+                                  spatial_pos=ids(40, b, s, s), attn_edge_type=ids(64, b, s, s, features), edge_input=ids(64, b, s, s, 5, features))
+    w = torch.randn(b, outputs, generator=g).to(cuda)
+    got = []
+    for fused in (True, False):
+        model.one_operator = fused
+        assert (model._one_operator(batch) is not None) == fused
+        model.zero_grad(set_to_none=True)
+        torch.manual_seed(7)
+        out = model(batch)
+        (out.float() * w).sum().backward()
+        got.append((out.detach(), {k: p.grad for k, p in model.named_parameters() if p.grad is not None}))
+    (o1, g1), (o0, g0) = got
+    tol = (3 if dtype == torch.float32 else 2) * TOL[dtype]      # float32: the tables are summed with atomics; bf16: up to five layers of rounding on both sides
+    assert float((o1.float() - o0.float()).abs().max()) <= tol * float(o0.float().abs().max())
+    assert g1.keys() == g0.keys()
+    worst = max(float(v.float().abs().max()) for v in g0.values())
+    for k in g0:
+        floor = worst * (1.0 if k.endswith("linear_k.bias") else 1e-2)
+        err = float((g1[k].float() - g0[k].float()).abs().max()) / max(float(g0[k].float().abs().max()), floor)
+        assert err <= tol, f"{k}: {err}"

@@ -203,15 +203,17 @@ constexpr int kBiasHot = 5;       // spatial ids 1..5 (self, one to four hops) a
 
 // What one lane reads for one position and one pass (up to kBiasFeat edge features, eight heads), kept
 // as loaded: converting or clamping a value where it is fetched would make the wave wait for it there.
-template <typename T, int FC>
+// NS gradients of one and the same bias (the layers of a model share it) are read side by side and added in float.
+template <typename T> struct BiasGrads { const T* p[4]; };
+template <typename T, int FC, int NS>
 struct BiasFetch {
     int64_t spr, er[FC];
-    T raw[8];
+    T raw[NS][8];
     bool valid, inner;
 };
-template <typename T, int FC>
-__device__ __forceinline__ void bias_fetch(const BiasArgs& a, const T* __restrict__ dout, const BiasPos& p, bool valid, int f0,
-                                           int h0, BiasFetch<T, FC>& x) {
+template <typename T, int FC, int NS>
+__device__ __forceinline__ void bias_fetch(const BiasArgs& a, const BiasGrads<T>& dout, const BiasPos& p, bool valid, int f0,
+                                           int h0, BiasFetch<T, FC, NS>& x) {
     const int S1 = a.s + 1;
     const int64_t plane = (int64_t)S1 * S1;
     x.valid = valid;
@@ -227,13 +229,16 @@ __device__ __forceinline__ void bias_fetch(const BiasArgs& a, const T* __restric
 #pragma unroll
         for (int u = 0; u < FC; ++u) x.er[u] = a.edge_type[pos * a.F + min(f0 + u, a.F - 1)];
     }
-    const T* __restrict__ dg = dout + g * a.H * plane + ij;          // head h of this position: dg[h * plane]
 #pragma unroll
-    for (int u = 0; u < 8; ++u) x.raw[u] = dg[(int64_t)min(h0 + u, a.H - 1) * plane];
+    for (int k = 0; k < NS; ++k) {
+        const T* __restrict__ dg = dout.p[k] + g * a.H * plane + ij;          // head h of this position: dg[h * plane]
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x.raw[k][u] = dg[(int64_t)min(h0 + u, a.H - 1) * plane];
+    }
 }
 
-template <typename T, int NHOT, int FC>
-__device__ __forceinline__ void bias_consume(const BiasArgs& a, const BiasFetch<T, FC>& x, int f0, int h0, float* acc_sp, float* acc_e,
+template <typename T, int NHOT, int FC, int NS>
+__device__ __forceinline__ void bias_consume(const BiasArgs& a, const BiasFetch<T, FC, NS>& x, int f0, int h0, float* acc_sp, float* acc_e,
                                              float* acc_v, float (&hot)[NHOT > 0 ? NHOT : 1][8]) {
     const int H = a.H;
     const int sp = x.inner && f0 == 0 ? clamp_id(x.spr, a.num_spatial) : 0;
@@ -244,7 +249,11 @@ __device__ __forceinline__ void bias_consume(const BiasArgs& a, const BiasFetch<
     const bool cold = sp > NHOT;
     float v[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = ldf(&x.raw[u]);
+    for (int u = 0; u < 8; ++u) {
+        v[u] = ldf(&x.raw[0][u]);
+#pragma unroll
+        for (int k = 1; k < NS; ++k) v[u] += ldf(&x.raw[k][u]);
+    }
     if (NHOT > 0) {
 #pragma unroll
         for (int r = 0; r < NHOT; ++r) {
@@ -268,8 +277,8 @@ __device__ __forceinline__ void bias_consume(const BiasArgs& a, const BiasFetch<
 
 // ONEPASS: H <= 8 and F <= FC, one fetch per position; the fetch of the next position is issued
 // before the current one is consumed.
-template <typename T, int NHOT, bool ONEPASS, int FC>
-__global__ __launch_bounds__(256) void k_graph_bias_bwd(BiasArgs a, const T* __restrict__ dout, float* __restrict__ partial,
+template <typename T, int NHOT, bool ONEPASS, int FC, int NS>
+__global__ __launch_bounds__(256) void k_graph_bias_bwd(BiasArgs a, BiasGrads<T> dout, float* __restrict__ partial,
                                                         int copies) {
     extern __shared__ float acc_all[];
     const int n_acc = (a.num_spatial + a.num_edges + 1) * a.H;
@@ -289,7 +298,7 @@ __global__ __launch_bounds__(256) void k_graph_bias_bwd(BiasArgs a, const T* __r
 #pragma unroll
         for (int u = 0; u < 8; ++u) hot[r][u] = 0.f;
     if (ONEPASS) {
-        BiasFetch<T, FC> cur, nxt;
+        BiasFetch<T, FC, NS> cur, nxt;
         int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
         const BiasStep step = bias_step(stride, a.s + 1);
         BiasPos p = bias_pos(t, a.s + 1);
@@ -297,17 +306,17 @@ __global__ __launch_bounds__(256) void k_graph_bias_bwd(BiasArgs a, const T* __r
         for (; t - threadIdx.x < total; t += stride) {
             bias_advance(p, step, a.s + 1);
             bias_fetch(a, dout, p, t + stride < total, 0, 0, nxt);
-            bias_consume<T, NHOT, FC>(a, cur, 0, 0, acc_sp, acc_e, acc_v, hot);
+            bias_consume<T, NHOT, FC, NS>(a, cur, 0, 0, acc_sp, acc_e, acc_v, hot);
             cur = nxt;
         }
     } else {
         for (int64_t t0 = (int64_t)blockIdx.x * 256; t0 < total; t0 += stride)
             for (int f0 = 0; f0 < F; f0 += FC)
                 for (int h0 = 0; h0 < H; h0 += 8) {
-                    BiasFetch<T, FC> x;
+                    BiasFetch<T, FC, NS> x;
                     bias_fetch(a, dout, bias_pos(t0 + threadIdx.x, a.s + 1), t0 + threadIdx.x < total, f0, h0, x);
                     // the spatial id counts once per head pass, in the first feature pass
-                    bias_consume<T, NHOT, FC>(a, x, f0, h0, acc_sp, acc_e, acc_v, hot);
+                    bias_consume<T, NHOT, FC, NS>(a, x, f0, h0, acc_sp, acc_e, acc_v, hot);
                 }
     }
     if (NHOT > 0) {
@@ -467,7 +476,7 @@ int64_t tgt_graph_attn_bias_bwd_workspace_bytes(int num_spatial, int num_edges, 
     return (int64_t)sizeof(float) * tgt::kBiasWorkers * (num_spatial + num_edges + 1) * H;
 }
 
-int tgt_graph_attn_bias_bwd(const void* d_dout, const int64_t* d_spatial_pos, const int64_t* d_edge_type, int F,
+int tgt_graph_attn_bias_bwd_sum(const void* const* d_douts, int n_douts, const int64_t* d_spatial_pos, const int64_t* d_edge_type, int F,
                             int num_spatial, int num_edges, int b, int s, int H, int dtype, void* d_dspatial_table,
                             void* d_dedge_table, void* d_dvirtual_dist, void* d_workspace, int64_t workspace_bytes,
                             void* stream) {
@@ -475,10 +484,15 @@ int tgt_graph_attn_bias_bwd(const void* d_dout, const int64_t* d_spatial_pos, co
     const int rc = bias_check(b, s, H, F, num_spatial, num_edges, dtype, "tgt_graph_attn_bias_bwd");
     if (rc != TGT_OK) return rc;
     if (!d_dspatial_table || !d_dedge_table || !d_dvirtual_dist ||
-        (b > 0 && (!d_dout || (s > 0 && (!d_spatial_pos || !d_edge_type))))) {
-        set_error("tgt_graph_attn_bias_bwd: null pointer");
+        !d_douts || n_douts < 1 || n_douts > 4 || (b > 0 && ((s > 0 && (!d_spatial_pos || !d_edge_type))))) {
+        set_error("tgt_graph_attn_bias_bwd: null pointer, or not 1 to 4 gradients");
         return TGT_ERR_INVALID_ARG;
     }
+    for (int k = 0; k < n_douts; ++k)
+        if (b > 0 && !d_douts[k]) {
+            set_error("tgt_graph_attn_bias_bwd: null pointer");
+            return TGT_ERR_INVALID_ARG;
+        }
     const int n_acc = (num_spatial + num_edges + 1) * H;
     if ((size_t)n_acc * sizeof(float) > 128 * 1024) {
         set_error("tgt_graph_attn_bias_bwd: (num_spatial + num_edges + 1) * H = %d table entries exceed the %d kept on chip",
@@ -500,7 +514,7 @@ int tgt_graph_attn_bias_bwd(const void* d_dout, const int64_t* d_spatial_pos, co
     while (copies > 1 && (size_t)n_acc * copies * sizeof(float) > 16 * 1024) copies /= 2;      // more workgroups per CU beat more copies
     const size_t lds = (size_t)n_acc * copies * sizeof(float);
     const unsigned rgrid = (unsigned)((n_acc + 3) / 4);
-    auto launch = [&](auto kernel, auto reduce, auto* dout, auto* dsp, auto* de, auto* dv) -> int {
+    auto launch = [&](auto kernel, auto reduce, auto dout, auto* dsp, auto* de, auto* dv) -> int {
         if (lds > 48 * 1024)
             TGT_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                               128 * 1024));
@@ -511,27 +525,37 @@ int tgt_graph_attn_bias_bwd(const void* d_dout, const int64_t* d_spatial_pos, co
     };
     // registers for the frequent ids need one pass over the heads; the prefetching loop one pass over the features too
     const int variant = H > 8 ? 0 : (F > kBiasFeat ? 1 : (F > 1 ? 2 : 3));
-    int lrc;
-    if (dtype == TGT_DTYPE_F32) {
-        auto* red = &k_graph_bias_reduce<float>;
-        const float* dout = (const float*)d_dout;
-        float *dsp = (float*)d_dspatial_table, *de = (float*)d_dedge_table, *dv = (float*)d_dvirtual_dist;
-        lrc = variant == 3   ? launch(&k_graph_bias_bwd<float, kBiasHot, true, 1>, red, dout, dsp, de, dv)
-              : variant == 2 ? launch(&k_graph_bias_bwd<float, kBiasHot, true, kBiasFeat>, red, dout, dsp, de, dv)
-              : variant == 1 ? launch(&k_graph_bias_bwd<float, kBiasHot, false, kBiasFeat>, red, dout, dsp, de, dv)
-                             : launch(&k_graph_bias_bwd<float, 0, false, kBiasFeat>, red, dout, dsp, de, dv);
-    } else {
-        auto* red = &k_graph_bias_reduce<gbf16>;
-        const gbf16* dout = (const gbf16*)d_dout;
-        gbf16 *dsp = (gbf16*)d_dspatial_table, *de = (gbf16*)d_dedge_table, *dv = (gbf16*)d_dvirtual_dist;
-        lrc = variant == 3   ? launch(&k_graph_bias_bwd<gbf16, kBiasHot, true, 1>, red, dout, dsp, de, dv)
-              : variant == 2 ? launch(&k_graph_bias_bwd<gbf16, kBiasHot, true, kBiasFeat>, red, dout, dsp, de, dv)
-              : variant == 1 ? launch(&k_graph_bias_bwd<gbf16, kBiasHot, false, kBiasFeat>, red, dout, dsp, de, dv)
-                             : launch(&k_graph_bias_bwd<gbf16, 0, false, kBiasFeat>, red, dout, dsp, de, dv);
+    if (n_douts > 1 && variant != 3) {
+        set_error("tgt_graph_attn_bias_bwd_sum: several gradients with at most 8 heads and one edge feature only");
+        return TGT_ERR_UNSUPPORTED;
     }
+    int lrc;
+    auto run = [&](auto tag) -> int {
+        using T = decltype(tag);
+        auto* red = &k_graph_bias_reduce<T>;
+        BiasGrads<T> dout;
+        for (int k = 0; k < 4; ++k) dout.p[k] = (const T*)d_douts[k < n_douts ? k : 0];
+        T *dsp = (T*)d_dspatial_table, *de = (T*)d_dedge_table, *dv = (T*)d_dvirtual_dist;
+        if (n_douts == 4) return launch(&k_graph_bias_bwd<T, kBiasHot, true, 1, 4>, red, dout, dsp, de, dv);
+        if (n_douts == 3) return launch(&k_graph_bias_bwd<T, kBiasHot, true, 1, 3>, red, dout, dsp, de, dv);
+        if (n_douts == 2) return launch(&k_graph_bias_bwd<T, kBiasHot, true, 1, 2>, red, dout, dsp, de, dv);
+        return variant == 3   ? launch(&k_graph_bias_bwd<T, kBiasHot, true, 1, 1>, red, dout, dsp, de, dv)
+               : variant == 2 ? launch(&k_graph_bias_bwd<T, kBiasHot, true, kBiasFeat, 1>, red, dout, dsp, de, dv)
+               : variant == 1 ? launch(&k_graph_bias_bwd<T, kBiasHot, false, kBiasFeat, 1>, red, dout, dsp, de, dv)
+                              : launch(&k_graph_bias_bwd<T, 0, false, kBiasFeat, 1>, red, dout, dsp, de, dv);
+    };
+    lrc = dtype == TGT_DTYPE_F32 ? run(float()) : run(gbf16());
     if (lrc != TGT_OK) return lrc;
     TGT_HIP_CHECK(hipGetLastError());
     return TGT_OK;
+}
+
+int tgt_graph_attn_bias_bwd(const void* d_dout, const int64_t* d_spatial_pos, const int64_t* d_edge_type, int F,
+                            int num_spatial, int num_edges, int b, int s, int H, int dtype, void* d_dspatial_table,
+                            void* d_dedge_table, void* d_dvirtual_dist, void* d_workspace, int64_t workspace_bytes,
+                            void* stream) {
+    return tgt_graph_attn_bias_bwd_sum(&d_dout, 1, d_spatial_pos, d_edge_type, F, num_spatial, num_edges, b, s, H, dtype, d_dspatial_table,
+                                       d_dedge_table, d_dvirtual_dist, d_workspace, workspace_bytes, stream);
 }
 
 int tgt_floyd_warshall(const uint8_t* d_adj, const int32_t* d_n_nodes, int num_graphs, int n_max, int32_t* d_dist,

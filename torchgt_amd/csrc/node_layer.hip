@@ -634,6 +634,84 @@ template <typename T> __global__ __launch_bounds__(1024) void k_node_sums(const 
     }
 }
 
+// ---- head of the graph-level models ---------------------------------------------------------------------------------------
+// One row per graph (the virtual node's): a few microseconds of latency whatever the shape.  Lane = feature.
+__device__ __forceinline__ float wave_sum(float v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+template <typename T> __device__ __forceinline__ float head_row(const T* __restrict__ s, int64_t row, float eps, int lane, float& rstd) {
+    const float v = as_float(s[row * 64 + lane]), mean = wave_sum(v) * (1.f / 64), d = v - mean;
+    rstd = rsqrtf(wave_sum(d * d) * (1.f / 64) + eps);
+    return d * rstd;
+}
+template <typename T>
+__global__ __launch_bounds__(256) void k_graph_head_fwd(const T* __restrict__ s, const T* __restrict__ gamma, const T* __restrict__ beta, float eps, const T* __restrict__ W,
+                                                         const T* __restrict__ bias, int b, int S, int O, T* __restrict__ y) {
+    const int lane = threadIdx.x & 63, g = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (g >= b) return;
+    float rstd;
+    const float xhat = head_row(s, (int64_t)g * S, eps, lane, rstd);
+    const float v = stored(xhat * as_float(gamma[lane]) + as_float(beta[lane]), (const T*)nullptr);
+    for (int o = 0; o < O; ++o) {
+        const float t = wave_sum(v * as_float(W[o * 64 + lane]));
+        if (lane == 0) y[(int64_t)g * O + o] = to_elem<T>(t + as_float(bias[o]));
+    }
+}
+// Workgroup 0: the virtual nodes' rows and all parameter gradients, sixteen graphs at a time (wave = graph for the rows; wave =
+// slice of the outputs for the sums over graphs).  The others write the zero rows.
+template <typename T>
+__global__ __launch_bounds__(1024) void k_graph_head_bwd(const T* __restrict__ s, const T* __restrict__ gamma, const T* __restrict__ beta, float eps, const T* __restrict__ W,
+                                                          const T* __restrict__ dy, int b, int S, int O, T* __restrict__ g_out, T* __restrict__ dW, T* __restrict__ db,
+                                                          T* __restrict__ dgamma, T* __restrict__ dbeta) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (blockIdx.x > 0) {
+        constexpr int PP = RowShape<T>::kPieces;
+        const int64_t n = (int64_t)b * S * PP;
+        for (int64_t i = (int64_t)(blockIdx.x - 1) * 1024 + threadIdx.x; i < n; i += (int64_t)(gridDim.x - 1) * 1024)
+            if ((i / PP) % S != 0) reinterpret_cast<vec16*>(g_out)[i] = vec16{0u, 0u, 0u, 0u};
+        return;
+    }
+    __shared__ float sy[16][64], sd[16][64], sx[16][64], sdy[16][64];
+    float aw[4] = {0.f, 0.f, 0.f, 0.f}, ab[4] = {0.f, 0.f, 0.f, 0.f}, ag = 0.f, abt = 0.f;
+    const float gm = as_float(gamma[lane]), bt = as_float(beta[lane]);
+    for (int g0 = 0; g0 < b; g0 += 16) {
+        const int g = g0 + wave;
+        float d = 0.f, xhat = 0.f, rstd = 0.f, v = 0.f;
+        if (g < b) {
+            xhat = head_row(s, (int64_t)g * S, eps, lane, rstd);
+            v = stored(xhat * gm + bt, (const T*)nullptr);
+            for (int o = 0; o < O; ++o) d += as_float(dy[(int64_t)g * O + o]) * as_float(W[o * 64 + lane]);
+            const float t = d * gm, c1 = wave_sum(t) * (1.f / 64), c2 = wave_sum(t * xhat) * (1.f / 64);
+            g_out[(int64_t)g * S * 64 + lane] = to_elem<T>(rstd * (t - c1 - xhat * c2));
+        }
+        sy[wave][lane] = v; sd[wave][lane] = d; sx[wave][lane] = d * xhat;
+        sdy[wave][lane] = g < b && lane < O ? as_float(dy[(int64_t)g * O + lane]) : 0.f;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int o = wave + 16 * k;
+            if (o < O)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) { aw[k] += sdy[i][o] * sy[i][lane]; ab[k] += sdy[i][o]; }
+        }
+        if (wave == 0)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) { abt += sd[i][lane]; ag += sx[i][lane]; }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int o = wave + 16 * k;
+        if (o < O) {
+            dW[o * 64 + lane] = to_elem<T>(aw[k]);
+            if (lane == 0) db[o] = to_elem<T>(ab[k]);
+        }
+    }
+    if (wave == 0) { dgamma[lane] = to_elem<T>(ag); dbeta[lane] = to_elem<T>(abt); }
+}
+
 int bad(const char* who, const char* what) { set_error("%s: %s", who, what); return TGT_ERR_INVALID_ARG; }
 int num_cus() {
     static const int n = [] { int dev = 0, v = 256; if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev); return v > 0 ? v : 256; }();
@@ -745,6 +823,39 @@ int tgt_node_bwd_post(const tgt_node_bwd_post_args* a, void* stream) {
     KernelTimer t(KS_LINEAR_DX, (hipStream_t)stream);
     const int workers = grid_for(a->rows, 4);
     return a->dtype == TGT_DTYPE_F32 ? dispatch_bwd_post<float>(*a, workers, (hipStream_t)stream) : dispatch_bwd_post<nbf16>(*a, workers, (hipStream_t)stream);
+}
+
+int tgt_graph_head_fwd(const void* d_s, const void* d_gamma, const void* d_beta, float eps, const void* d_W, const void* d_bias, int b, int S,
+                       int outputs, int dtype, void* d_y, void* stream) {
+    using namespace tgt;
+    if (!d_s || !d_gamma || !d_beta || !d_W || !d_bias || !d_y || b < 0 || S < 1 || outputs < 1 || outputs > 64 || !dtype_ok(dtype)) return bad("tgt_graph_head_fwd", "null or bad argument");
+    if (b == 0) return TGT_OK;
+    KernelTimer t(KS_LINEAR_FWD, (hipStream_t)stream);
+    const auto run = [&](auto tag) {
+        using T = decltype(tag);
+        hipLaunchKernelGGL((k_graph_head_fwd<T>), dim3((b + 3) / 4), dim3(256), 0, (hipStream_t)stream, (const T*)d_s, (const T*)d_gamma, (const T*)d_beta, eps, (const T*)d_W,
+                           (const T*)d_bias, b, S, outputs, (T*)d_y);
+    };
+    if (dtype == TGT_DTYPE_F32) run(float()); else run(nbf16());
+    TGT_HIP_CHECK(hipGetLastError());
+    return TGT_OK;
+}
+
+int tgt_graph_head_bwd(const void* d_s, const void* d_gamma, const void* d_beta, float eps, const void* d_W, const void* d_dy, int b, int S,
+                       int outputs, int dtype, void* d_g_out, void* d_dW, void* d_dbias, void* d_dgamma, void* d_dbeta, void* stream) {
+    using namespace tgt;
+    if (!d_s || !d_gamma || !d_beta || !d_W || !d_dy || !d_g_out || !d_dW || !d_dbias || !d_dgamma || !d_dbeta || b < 1 || S < 1 || outputs < 1 || outputs > 64 || !dtype_ok(dtype))
+        return bad("tgt_graph_head_bwd", "null or bad argument");
+    KernelTimer t(KS_LINEAR_DX, (hipStream_t)stream);
+    const int zeros = (int)std::min<int64_t>(num_cus(), ((int64_t)b * S * 16 + 1023) / 1024);
+    const auto run = [&](auto tag) {
+        using T = decltype(tag);
+        hipLaunchKernelGGL((k_graph_head_bwd<T>), dim3(1 + zeros), dim3(1024), 0, (hipStream_t)stream, (const T*)d_s, (const T*)d_gamma, (const T*)d_beta, eps, (const T*)d_W,
+                           (const T*)d_dy, b, S, outputs, (T*)d_g_out, (T*)d_dW, (T*)d_dbias, (T*)d_dgamma, (T*)d_dbeta);
+    };
+    if (dtype == TGT_DTYPE_F32) run(float()); else run(nbf16());
+    TGT_HIP_CHECK(hipGetLastError());
+    return TGT_OK;
 }
 
 int tgt_node_sums(const tgt_node_sum* sums, int count, int dtype, void* stream) {

@@ -2,6 +2,8 @@
 // attention: between Python and the kernels of a step there is one call forward and one backward.
 //
 //   torchgt::node_graphormer(x, params[7 + 16 L], plan holder, workspace, heads, tokens, eps[2 L + 1]) -> log-probabilities
+//   torchgt::graph_graphormer(x, in_degree, out_degree, attn_bias, spatial_pos, edge_ids, params[11 (12) + 16 L], multi_hop, max_dist,
+//                             heads, eps[2 L + 1], p_drop, seeds[L], bf16_products) -> predictions
 //
 // A step's intermediate rows live in one allocation, its parameter gradients in another: with some seventy parameters the
 // host's time for tensors of their own would be longer than the kernels of a small graph take.
@@ -289,10 +291,255 @@ Tensor node_graphormer(const Tensor& x, at::TensorList P, const c10::intrusive_p
     return st.logp;
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// graph-level Graphormer (models/graphormer_graph_level.py:309-389): node features, attention bias, layers around the dense
+// attention, head; attention dropout inside the kernels, no other dropout at work
+// ---------------------------------------------------------------------------------------------------------------
+// params: atom, in-degree, out-degree tables, graph token; spatial table, edge table, virtual distance (, hop matrices);
+// 16 per layer; gamma, beta (final norm), Wh, bh
+struct GraphCall {
+    bool multi_hop = false, bf16_products = false;
+    int64_t max_dist = 0, H = 0;
+    double p_drop = 0;
+    std::vector<double> eps;
+    std::vector<int64_t> seeds;
+};
+
+struct GraphBatch { Tensor x, in_degree, out_degree, spatial, edges; };      // int64, contiguous
+
+struct GraphGraphormerFn : public torch::autograd::Function<GraphGraphormerFn> {
+    static constexpr int kFixed = 7;
+    // dlse etc. of the layers live next to the rows: s_0 .. s_L, then q, k, v, a of every layer
+    static Tensor compute(const GraphBatch& in, const Tensor& attn_bias, const std::vector<Tensor>& p, const GraphCall& c, bool keep, Tensor& rows, Tensor& lse, Tensor& bias,
+                          Packed& packed) {
+        const int code = dtype_code(p[0]), H = (int)c.H, tables = kFixed + (c.multi_hop ? 1 : 0);
+        const int dense = code == TGT_DTYPE_F32 && c.bf16_products ? TGT_DTYPE_F32_BF16_PRODUCTS : code;
+        const int64_t L = (int64_t)(p.size() - tables - 4) / 16, b = in.x.size(0), s = in.x.size(1), S = s + 1, N = b * S;
+        const auto opt = p[0].options();
+        void* stream = stream_of(p[0]);
+        const int64_t ns = keep ? L + 1 : 1, na = keep ? 4 * L : 4;
+        rows = at::empty({(ns + na) * N, kWidth}, opt);
+        lse = at::empty({keep ? L * b * H * S : b * H * S}, opt.dtype(at::kFloat));
+        bias = at::empty({b, H, S, S}, opt);
+        packed = Packed(p.data() + tables, L, nullptr, code, opt, stream);
+        auto s_row = [&](int64_t l) { return at_row(rows, keep ? l * N : 0); };
+        auto a_row = [&](int64_t l, int i) { return at_row(rows, (ns + (keep ? 4 * l : 0) + i) * N); };
+        check(tgt_graph_node_feature_fwd(in.x.data_ptr<int64_t>(), in.in_degree.data_ptr<int64_t>(), in.out_degree.data_ptr<int64_t>(), (int)in.x.size(2), p[0].data_ptr(),
+                                         (int)p[0].size(0), p[1].data_ptr(), (int)p[1].size(0), p[2].data_ptr(), (int)p[2].size(0), p[3].data_ptr(), (int)b, (int)s,
+                                         (int)kWidth, code, s_row(0), stream),
+              "tgt_graph_node_feature_fwd");
+        if (c.multi_hop)
+            check(tgt_graph_attn_bias_multi_hop_fwd(attn_bias.data_ptr(), in.spatial.data_ptr<int64_t>(), in.edges.data_ptr<int64_t>(), (int)in.edges.size(3),
+                                                    (int)in.edges.size(4), p[4].data_ptr(), (int)p[4].size(0), p[5].data_ptr(), (int)p[5].size(0), p[7].data_ptr(),
+                                                    (int)(p[7].numel() / (H * H)), p[6].data_ptr(), (int)c.max_dist, (int)b, (int)s, H, code, bias.data_ptr(), stream),
+                  "tgt_graph_attn_bias_multi_hop_fwd");
+        else
+            check(tgt_graph_attn_bias_fwd(attn_bias.data_ptr(), in.spatial.data_ptr<int64_t>(), in.edges.data_ptr<int64_t>(), (int)in.edges.size(3), p[4].data_ptr(),
+                                          (int)p[4].size(0), p[5].data_ptr(), (int)p[5].size(0), p[6].data_ptr(), (int)b, (int)s, H, code, bias.data_ptr(), stream),
+                  "tgt_graph_attn_bias_fwd");
+        for (int64_t l = 0; l <= L; ++l) {
+            tgt_node_fwd_args a{};
+            a.rows = N; a.dtype = code;
+            a.s_in = s_row(l ? l - 1 : 0); a.s_out = s_row(l);
+            if (l > 0) {
+                a.attn = a_row(l - 1, 3);
+                a.w_post = packed.weight(6 * (l - 1)); a.v_post = packed.vec(10 * (l - 1)); a.eps_post = (float)c.eps[2 * (l - 1) + 1];
+            }
+            if (l < L) {
+                a.q = a_row(l, 0); a.k = a_row(l, 1); a.v = a_row(l, 2);
+                a.w_next = packed.weight(6 * l + 3); a.v_next = packed.vec(10 * l + 5); a.eps_next = (float)c.eps[2 * l];
+            }
+            check(tgt_node_fwd(&a, stream), "tgt_node_fwd");
+            if (l < L)
+                check(tgt_dense_attn_dropout_fwd(a.q, a.k, a.v, bias.data_ptr(), (int)b, (int)S, H, (int)(kWidth / H), dense, (float)c.p_drop, (uint64_t)c.seeds[l], a_row(l, 3),
+                                                 lse.data_ptr<float>() + (keep ? l * b * H * S : 0), stream),
+                      "tgt_dense_attn_dropout_fwd");
+        }
+        const Tensor* head = p.data() + tables + 16 * L;
+        Tensor y = at::empty({b, head[2].size(0)}, opt);
+        check(tgt_graph_head_fwd(s_row(L), head[0].data_ptr(), head[1].data_ptr(), (float)c.eps[2 * L], head[2].data_ptr(), head[3].data_ptr(), (int)b, (int)S,
+                                 (int)head[2].size(0), code, y.data_ptr(), stream),
+              "tgt_graph_head_fwd");
+        return y;
+    }
+    static Tensor forward(AutogradContext* ctx, at::TensorList P, Tensor x, Tensor in_degree, Tensor out_degree, Tensor attn_bias, Tensor spatial, Tensor edges, GraphCall c) {
+        std::vector<Tensor> p;
+        p.reserve(P.size());
+        for (const Tensor& t : P) p.push_back(t.contiguous());
+        c10::DeviceGuard guard(p[0].device());
+        Tensor rows, lse, bias;
+        Packed packed;
+        Tensor y = compute(GraphBatch{x, in_degree, out_degree, spatial, edges}, attn_bias, p, c, true, rows, lse, bias, packed);
+        const size_t head = p.size() - 4;
+        ctx->save_for_backward({x, in_degree, out_degree, spatial, edges, rows, lse, bias, packed.frags, p[0], p[1], p[2], p[4], p[5], c.multi_hop ? p[7] : Tensor(), p[head],
+                                p[head + 1], p[head + 2], p[3], p[6]});
+        ctx->saved_data["multi_hop"] = c.multi_hop;
+        ctx->saved_data["dense"] = c.bf16_products;
+        ctx->saved_data["ints"] = std::vector<int64_t>{c.max_dist, c.H, (int64_t)p.size()};
+        ctx->saved_data["p"] = c.p_drop;
+        ctx->saved_data["eps"] = c.eps;
+        ctx->saved_data["seeds"] = c.seeds;
+        return y;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        auto sv = ctx->get_saved_variables();
+        const Tensor &x = sv[0], &ind = sv[1], &outd = sv[2], &spatial = sv[3], &edges = sv[4], &rows = sv[5], &lse = sv[6], &bias = sv[7], &atom = sv[9], &tin = sv[10],
+                     &tout = sv[11], &sp = sv[12], &et = sv[13], &hops = sv[14], &gamma = sv[15], &beta = sv[16], &Wh = sv[17], &token = sv[18], &vd = sv[19];
+        const bool multi_hop = ctx->saved_data["multi_hop"].toBool();
+        const auto ints = ctx->saved_data["ints"].toIntVector();
+        const auto eps = ctx->saved_data["eps"].toDoubleVector();
+        const auto seeds = ctx->saved_data["seeds"].toIntVector();
+        const double p_drop = ctx->saved_data["p"].toDouble();
+        const int tables = kFixed + (multi_hop ? 1 : 0), H = (int)ints[1];
+        const int64_t L = (ints[2] - tables - 4) / 16, b = x.size(0), s = x.size(1), S = s + 1, N = b * S, O = Wh.size(0);
+        const int code = dtype_code(atom), dense = code == TGT_DTYPE_F32 && ctx->saved_data["dense"].toBool() ? TGT_DTYPE_F32_BF16_PRODUCTS : code;
+        c10::DeviceGuard guard(atom.device());
+        void* stream = stream_of(atom);
+        const auto opt = atom.options(), bytes_opt = opt.dtype(at::kByte);
+        const Packed packed(sv[8], (int)(6 * L), code);
+        std::vector<std::vector<int64_t>> shapes;
+        for (const Tensor* t : {&atom, &tin, &tout, &token, &sp, &et, &vd}) shapes.push_back(t->sizes().vec());
+        if (multi_hop) shapes.push_back(hops.sizes().vec());
+        for (int64_t l = 0; l < L; ++l)
+            for (int i = 0; i < 16; ++i) shapes.push_back(i >= 2 && i % 2 == 0 && i != 10 ? std::vector<int64_t>{kWidth, kWidth} : std::vector<int64_t>{kWidth});
+        shapes.push_back({kWidth});
+        shapes.push_back({kWidth});
+        shapes.push_back({O, kWidth});
+        shapes.push_back({O});
+        FlatGrads G(shapes, opt);
+        const Tensor dy = grads[0].contiguous();
+        const int workers = tgt_node_bwd_workers(N);
+        Tensor work = at::empty({6 * N, kWidth}, opt);
+        Tensor partial = at::empty({workers * 2 * L * kLayerPartial}, opt.dtype(at::kFloat));
+        char *g[2] = {at_row(work, 0), at_row(work, N)}, *da = at_row(work, 2 * N), *dq = at_row(work, 3 * N), *dk = at_row(work, 4 * N), *dv = at_row(work, 5 * N);
+        float* next_partial = partial.data_ptr<float>();
+        std::vector<tgt_node_sum> sums;
+        auto new_sum = [&]() -> tgt_node_sum& {
+            sums.push_back(tgt_node_sum{});
+            sums.back().partial = next_partial; sums.back().workers = workers; sums.back().mats = 3; sums.back().rows = (int)kWidth;
+            next_partial += workers * kLayerPartial;
+            return sums.back();
+        };
+        const Tensor* head = G.t.data() + tables + 16 * L;
+        check(tgt_graph_head_bwd(at_row(rows, L * N), gamma.data_ptr(), beta.data_ptr(), (float)eps[2 * L], Wh.data_ptr(), dy.data_ptr(), (int)b, (int)S, (int)O, code, g[0],
+                                 head[2].data_ptr(), head[3].data_ptr(), head[0].data_ptr(), head[1].data_ptr(), stream),
+              "tgt_graph_head_bwd");
+        // the layers share one bias: their gradients of it are added where they are folded into the tables, four at a time
+        const bool side_by_side = !multi_hop && H <= 8 && edges.size(3) == 1;
+        std::vector<Tensor> dbias;
+        for (int64_t l = L - 1; l >= 0; --l) {
+            const Tensor* w = G.t.data() + tables + 16 * l;
+            const int64_t unit = N * kWidth * rows.element_size();
+            const char *q = at_row(rows, (L + 1 + 4 * l) * N), *k = q + unit, *v = k + unit, *at = v + unit;
+            tgt_node_bwd_post_args post{};
+            post.rows = N; post.dtype = code; post.heads = H; post.eps = (float)eps[2 * l + 1];
+            post.g_in = g[0]; post.s = at_row(rows, l * N); post.attn = at; post.w_post = packed.weight(6 * l); post.w_back = packed.transposed(6 * l);
+            post.v_post = packed.vec(10 * l); post.g_out = g[1]; post.d_attn = da; post.partial = next_partial;
+            static const int to_post[8] = {8, 12, 14, 9, 13, 15, 10, 11}, to_pre[8] = {2, 4, 6, 3, 5, 7, 0, 1};
+            tgt_node_sum& s1 = new_sum();
+            for (int i = 0; i < 8; ++i) s1.out[i] = w[to_post[i]].data_ptr();
+            check(tgt_node_bwd_post(&post, stream), "tgt_node_bwd_post");
+            Tensor db = at::empty_like(bias);
+            check(tgt_dense_attn_dropout_bwd(q, k, v, bias.data_ptr(), (int)b, (int)S, H, (int)(kWidth / H), dense, (float)p_drop, (uint64_t)seeds[l], at,
+                                             lse.data_ptr<float>() + l * b * H * S, da, dq, dk, dv, db.data_ptr(), stream),
+                  "tgt_dense_attn_dropout_bwd");
+            if (dbias.empty() || (side_by_side && dbias.size() < 4)) dbias.push_back(db);
+            else dbias.back().add_(db);
+            tgt_node_bwd_pre_args pre{};
+            pre.rows = N; pre.dtype = code; pre.eps = (float)eps[2 * l];
+            pre.dq = dq; pre.dk = dk; pre.dv = dv; pre.g_in = g[1]; pre.s = at_row(rows, l * N);
+            pre.w_back = packed.transposed(6 * l + 3); pre.v_next = packed.vec(10 * l + 5); pre.g_out = g[0]; pre.partial = next_partial;
+            tgt_node_sum& s2 = new_sum();
+            for (int i = 0; i < 8; ++i) s2.out[i] = w[to_pre[i]].data_ptr();
+            check(tgt_node_bwd_pre(&pre, stream), "tgt_node_bwd_pre");
+        }
+        check(tgt_node_sums(sums.data(), (int)sums.size(), code, stream), "tgt_node_sums");
+        if (multi_hop) {
+            const int D0 = (int)edges.size(3), md = (int)ints[0], D = md > 0 && md < D0 ? md : D0;
+            const int64_t bytes = tgt_graph_attn_bias_multi_hop_bwd_workspace_bytes((int)sp.size(0), (int)et.size(0), H, D);
+            Tensor ws = at::empty({bytes}, bytes_opt);
+            check(tgt_graph_attn_bias_multi_hop_bwd(dbias[0].data_ptr(), spatial.data_ptr<int64_t>(), edges.data_ptr<int64_t>(), D0, (int)edges.size(4), et.data_ptr(),
+                                                    (int)sp.size(0), (int)et.size(0), hops.data_ptr(), (int)(hops.numel() / (H * H)), md, (int)b, (int)s, H, code,
+                                                    G.t[4].data_ptr(), G.t[5].data_ptr(), G.t[7].data_ptr(), G.t[6].data_ptr(), ws.data_ptr(), bytes, stream),
+                  "tgt_graph_attn_bias_multi_hop_bwd");
+        } else {
+            const void* d[4] = {nullptr, nullptr, nullptr, nullptr};
+            for (size_t i = 0; i < dbias.size(); ++i) d[i] = dbias[i].data_ptr();
+            const int64_t bytes = tgt_graph_attn_bias_bwd_workspace_bytes((int)sp.size(0), (int)et.size(0), H);
+            Tensor ws = at::empty({bytes}, bytes_opt);
+            check(tgt_graph_attn_bias_bwd_sum(d, (int)dbias.size(), spatial.data_ptr<int64_t>(), edges.data_ptr<int64_t>(), (int)edges.size(3), (int)sp.size(0), (int)et.size(0),
+                                              (int)b, (int)s, H, code, G.t[4].data_ptr(), G.t[5].data_ptr(), G.t[6].data_ptr(), ws.data_ptr(), bytes, stream),
+                  "tgt_graph_attn_bias_bwd_sum");
+        }
+        {
+            const int64_t bytes = tgt_graph_node_feature_bwd_workspace_bytes((int)atom.size(0), (int)tin.size(0), (int)tout.size(0), (int)kWidth);
+            Tensor ws = at::empty({bytes}, bytes_opt);
+            check(tgt_graph_node_feature_bwd(g[0], x.data_ptr<int64_t>(), ind.data_ptr<int64_t>(), outd.data_ptr<int64_t>(), (int)x.size(2), (int)atom.size(0), (int)tin.size(0),
+                                             (int)tout.size(0), (int)b, (int)s, (int)kWidth, code, G.t[0].data_ptr(), G.t[1].data_ptr(), G.t[2].data_ptr(), G.t[3].data_ptr(),
+                                             ws.data_ptr(), bytes, stream),
+                  "tgt_graph_node_feature_bwd");
+        }
+        variable_list out;
+        out.reserve(G.t.size() + 7);
+        for (Tensor& t : G.t) out.push_back(std::move(t));
+        for (int i = 0; i < 7; ++i) out.push_back(Tensor());
+        return out;
+    }
+};
+
+Tensor graph_graphormer(const Tensor& x, const Tensor& in_degree, const Tensor& out_degree, const Tensor& attn_bias, const Tensor& spatial_pos, const Tensor& edge_ids,
+                        at::TensorList P, bool multi_hop, int64_t max_dist, int64_t H, at::ArrayRef<double> eps, double p_drop, at::IntArrayRef seeds, bool bf16_products) {
+    on_gpu(attn_bias, "graph_graphormer");
+    const int64_t tables = GraphGraphormerFn::kFixed + (multi_hop ? 1 : 0);
+    TORCH_CHECK((int64_t)P.size() >= tables + 4 && (P.size() - tables - 4) % 16 == 0, "graph_graphormer takes ", tables + 4, " + 16 L parameter tensors");
+    const int64_t L = (int64_t)(P.size() - tables - 4) / 16;
+    TORCH_CHECK((int64_t)eps.size() == 2 * L + 1 && (int64_t)seeds.size() == L, "graph_graphormer: 2 L + 1 values of eps, L seeds");
+    TORCH_CHECK(H == 8 || H == 4 || H == 2, "graph_graphormer: 8, 4 or 2 heads");
+    bool train = false;
+    for (const Tensor& t : P) {
+        TORCH_CHECK(t.defined() && t.is_cuda() && t.scalar_type() == P[0].scalar_type(), "graph_graphormer: parameters must be GPU tensors of one dtype");
+        train = train || t.requires_grad();
+    }
+    for (int i : {0, 1, 2, 3}) TORCH_CHECK(P[i].dim() == 2 && P[i].size(1) == kWidth, "graph_graphormer: feature tables are [rows, 64]");
+    for (int i : {4, 5, 6}) TORCH_CHECK(P[i].dim() == 2 && P[i].size(1) == H, "graph_graphormer: bias tables are [rows, heads]");
+    TORCH_CHECK(!multi_hop || P[7].numel() % (H * H) == 0, "graph_graphormer: hop matrices");
+    const Tensor* q = P.data() + tables;
+    for (int64_t i = 0; i < 16 * L; ++i) {
+        const int64_t k = i % 16;
+        TORCH_CHECK(q[i].numel() == (k >= 2 && k % 2 == 0 && k != 10 ? kWidth * kWidth : kWidth), "graph_graphormer: layers are 64 wide");
+    }
+    q += 16 * L;
+    TORCH_CHECK(q[0].numel() == kWidth && q[1].numel() == kWidth && q[2].dim() == 2 && q[2].size(1) == kWidth && q[2].size(0) >= 1 && q[2].size(0) <= 64 && q[3].numel() == q[2].size(0),
+                "graph_graphormer: 1 to 64 outputs on 64 features");
+    const int64_t b = x.size(0), s = x.size(1);
+    TORCH_CHECK(x.dim() == 3 && in_degree.numel() == b * s && out_degree.numel() == b * s && attn_bias.dim() == 3 && attn_bias.size(0) == b && attn_bias.size(1) == s + 1 &&
+                    attn_bias.size(2) == s + 1 && spatial_pos.dim() == 3 && spatial_pos.size(0) == b && spatial_pos.size(1) == s && spatial_pos.size(2) == s &&
+                    edge_ids.dim() == (multi_hop ? 5 : 4) && edge_ids.size(0) == b && edge_ids.size(1) == s && edge_ids.size(2) == s,
+                "graph_graphormer: x [b, s, F], degrees [b, s], attn_bias [b, s + 1, s + 1], spatial_pos [b, s, s], edge ids [b, s, s, ...]");
+    GraphCall c;
+    c.multi_hop = multi_hop; c.bf16_products = bf16_products; c.max_dist = max_dist; c.H = H; c.p_drop = p_drop;
+    c.eps.assign(eps.begin(), eps.end());
+    c.seeds.assign(seeds.begin(), seeds.end());
+    const auto ids = [](const Tensor& t) { return t.to(at::kLong).contiguous(); };
+    c10::DeviceGuard guard(P[0].device());
+    const Tensor ab = attn_bias.to(P[0].scalar_type()).contiguous();
+    if (at::GradMode::is_enabled() && train) return GraphGraphormerFn::apply(P, ids(x), ids(in_degree), ids(out_degree), ab, ids(spatial_pos), ids(edge_ids), c);
+    std::vector<Tensor> p;
+    for (const Tensor& t : P) p.push_back(t.contiguous());
+    Tensor rows, lse, bias;
+    Packed packed;
+    return GraphGraphormerFn::compute(GraphBatch{ids(x), ids(in_degree), ids(out_degree), ids(spatial_pos), ids(edge_ids)}, ab, p, c, false, rows, lse, bias, packed);
+}
+
 }  // namespace
 
 TORCH_LIBRARY_FRAGMENT(torchgt, m) {
     m.def("node_graphormer(Tensor x, Tensor[] params, __torch__.torch.classes.torchgt.PlanHolder plan, Tensor workspace, int heads, int tokens, "
           "float[] eps) -> Tensor");
+    m.def("graph_graphormer(Tensor x, Tensor in_degree, Tensor out_degree, Tensor attn_bias, Tensor spatial_pos, Tensor edge_ids, Tensor[] params, "
+          "bool multi_hop, int max_dist, int heads, float[] eps, float p_drop, int[] seeds, bool bf16_products) -> Tensor");
 }
-TORCH_LIBRARY_IMPL(torchgt, CompositeImplicitAutograd, m) { m.impl("node_graphormer", node_graphormer); }
+TORCH_LIBRARY_IMPL(torchgt, CompositeImplicitAutograd, m) {
+    m.impl("node_graphormer", node_graphormer);
+    m.impl("graph_graphormer", graph_graphormer);
+}

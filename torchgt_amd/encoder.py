@@ -54,8 +54,8 @@ class ModuleTree:
     attribute look-ups of seventy parameters through ``nn.Module`` would be a third of it.  Remembers the dictionaries of the
     modules, not the parameters, and notices when a module of the tree was exchanged (``current``)."""
 
-    def __init__(self, root, names, dropouts, square=64):
-        self.links, self.slots, self.square = [], [], square
+    def __init__(self, root, names, dropouts, layers_at):
+        self.links, self.slots, self.layers_at = [], [], layers_at
         seen = set()
 
         def step(module, name):
@@ -100,9 +100,8 @@ class ModuleTree:
         for p in P:
             if p is None or p.dtype is not dtype:
                 return None
-        # the layers' parameters (everything but the first three and the last four): 64 wide throughout
-        for p in P[3:-4]:
-            if p.shape[0] != self.square or p.shape[-1] != self.square:
+        for p in P[self.layers_at:-4]:      # the layers' parameters (the last four are the final norm and the head): 64 wide throughout
+            if p.shape[0] != 64 or p.shape[-1] != 64:
                 return None
         return P
 
@@ -217,7 +216,7 @@ class Graphormer(nn.Module):
             return None
         tree = _TREES.get(self)
         if tree is None or not tree.current():
-            tree = _TREES[self] = ModuleTree(self, self._parameter_names(), ["self_attention_dropout", "ffn_dropout", "input_dropout"])
+            tree = _TREES[self] = ModuleTree(self, self._parameter_names(), ["self_attention_dropout", "ffn_dropout", "input_dropout"], 3)
         return tree.parameters(x.dtype, self.training)
 
     def _parameter_names(self):
@@ -228,7 +227,8 @@ class Graphormer(nn.Module):
 
     def forward(self, x, attn_bias, edge_index, perturb=None, attn_type=None):
         P = self._one_operator(x, attn_bias, edge_index, perturb, attn_type)
-        if P is not None and P[-1].shape[0] <= 64 and all(layer.one_operator and layer.self_attention.one_operator for layer in self.layers):
+        if P is not None and P[-1].shape[0] <= 64 and all(
+                "one_operator" not in layer.__dict__ and layer.one_operator and layer.self_attention.one_operator for layer in self.layers):
             # the whole model as one operator and one autograd node over kernels that take a layer's node-local part
             # in one pass each way
             plan = edge_index if isinstance(edge_index, GraphPlan) else get_plan(edge_index, x.shape[0] + self.num_global_node)

@@ -11,7 +11,7 @@ import torch.nn as nn
 
 from . import _ext, _lib
 from .core_attention import GraphBiasIds
-from .encoder import FeedForwardNetwork, init_params
+from .encoder import LAYER_PARAMETERS, _TREES, FeedForwardNetwork, ModuleTree, init_params
 from .graph_bias import GraphAttnBias
 from .multi_head_attention import MultiHeadAttention, fused_linear
 
@@ -192,7 +192,51 @@ class Graphormer(nn.Module):
         # the id histogram the tensor form runs once per step (1.85 against 2.30 ms per training step on that batch).
         self.bias_from_ids = False
 
+    one_operator = True      # False: always run the model layer by layer
+
+    def _one_operator(self, batched_data):
+        """The model's parameters in the operator's order when ``torch.ops.torchgt.graph_graphormer`` covers this call - the
+        bias as a tensor, hidden and feed-forward width 64, at most 64 outputs, no dropout at work but the attention's, one
+        dtype - else None."""
+        if not self.one_operator or self.bias_from_ids or not batched_data.attn_bias.is_cuda or len(self.layers) == 0 or batched_data.x.numel() == 0:
+            return None
+        multi_hop = self.graph_attn_bias.edge_type == "multi_hop"
+        head = "out_proj" if hasattr(self, "out_proj") else "downstream_out_proj"
+        tree = _TREES.get(self)
+        if tree is None or not tree.current():
+            names = [f"graph_node_feature.{k}.weight" for k in ("atom_encoder", "in_degree_encoder", "out_degree_encoder", "graph_token")]
+            names += [f"graph_attn_bias.{k}.weight" for k in ("spatial_pos_encoder", "edge_encoder", "graph_token_virtual_distance") +
+                      (("edge_dis_encoder",) if multi_hop else ())]
+            for i in range(len(self.layers)):
+                names += [f"layers.{i}.{k}" for k in LAYER_PARAMETERS]
+            names += ["final_ln.weight", "final_ln.bias", f"{head}.weight", f"{head}.bias"]
+            tree = _TREES[self] = ModuleTree(self, names, ["self_attention_dropout", "ffn_dropout", "input_dropout"], 8 if multi_hop else 7)
+        first = self.layers[0].self_attention.dist_attn.local_attn
+        for layer in self.layers:
+            core = layer.self_attention.dist_attn.local_attn
+            # (a flag set on a layer itself asks for that layer's own way of running, either one)
+            if "one_operator" in layer.__dict__ or not layer.one_operator or layer.self_attention.num_heads not in (2, 4, 8) or \
+                    core.attention_dropout_rate != first.attention_dropout_rate or core.dense_bf16_products != first.dense_bf16_products:
+                return None
+        P = tree.parameters(self.final_ln.weight.dtype, self.training)
+        if P is None or P[0].dtype not in _DT or P[0].shape[1] != 64 or P[-1].shape[0] > 64 or P[4].shape[1] != self.layers[0].self_attention.num_heads:
+            return None
+        return P
+
     def forward(self, batched_data, perturb=None):
+        P = self._one_operator(batched_data)
+        if P is not None:
+            # the whole model as one operator and one autograd node: node features, bias, layers, head
+            multi_hop = self.graph_attn_bias.edge_type == "multi_hop"
+            att = self.layers[0].self_attention
+            core = att.dist_attn.local_attn
+            p = float(core.attention_dropout_rate) if self.training else 0.0
+            seeds = [int(torch.randint(0, 2 ** 62, (1,)).item()) if p > 0 else 0 for _ in self.layers]
+            eps = [e for layer in self.layers for e in (layer.self_attention_norm.eps, layer.ffn_norm.eps)] + [self.final_ln.eps]
+            d = batched_data
+            return _ext.op("graph_graphormer")(d.x, d.in_degree, d.out_degree, d.attn_bias, d.spatial_pos, d.edge_input if multi_hop else d.attn_edge_type,
+                                               P, multi_hop, int(self.graph_attn_bias.multi_hop_max_dist), att.num_heads, eps, p, seeds,
+                                               bool(core.dense_bf16_products))
         x = self.graph_node_feature(batched_data)            # [b, s + 1, h]
         attn_bias = self.graph_attn_bias(batched_data, as_ids=self.bias_from_ids)       # [b, H, s + 1, s + 1], or its ids
         output = self.input_dropout(x)
