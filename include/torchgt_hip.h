@@ -601,10 +601,12 @@ int tgt_node_pack(const void* const* mats, const int* ld, const int* rows, int n
  * first `tokens` rows are taken from `token` and written to s_out; s_in and s_out are the same array).  w_post: packed Wo,
  * W1, W2; v_post: bo, gamma, beta, b1, b2.  q, k, v: rows for the next attention (w_next: packed Wq, Wk, Wv; v_next: gamma,
  * beta, bq, bk, bv), or NULL.  logp: [rows - tokens, classes] log_softmax(LN(s') Wh^T + bh) without the token rows (w_next:
- * packed Wh; v_next: gamma, beta, bh), or NULL. */
+ * packed Wh; v_next: gamma, beta, bh), or NULL; with `linear` the logits themselves (the outputs of a regression).
+ * same_bits (bf16): every sum in the order of the separate kernels (tgt_linear_fwd, tgt_layer_norm_fwd, tgt_gelu_fwd), so that the
+ * results are theirs bit for bit. */
 typedef struct {
     int64_t rows;
-    int32_t dtype, tokens, classes;
+    int32_t dtype, tokens, classes, linear, same_bits;
     float eps_post, eps_next;
     const void *attn, *s_in, *token;
     void* s_out;
@@ -614,13 +616,13 @@ typedef struct {
 } tgt_node_fwd_args;
 int tgt_node_fwd(const tgt_node_fwd_args* args, void* stream);
 /* Backward of the part in front of an attention: g_out = g_in + d LN'(...) for dq, dk, dv (w_back: the transposed packed Wq,
- * Wk, Wv; s: the rows LN' normalised), or of the classes (dlogp, logp; no g_in, dq, dk, dv; w_back: transposed packed Wh).
+ * Wk, Wv; s: the rows LN' normalised), or of the classes (dlogp, logp - not needed with `linear` -; no g_in, dq, dk, dv; w_back: transposed packed Wh).
  * d_token: the first `tokens` rows of g_out once more (the gradient of the global tokens behind the first layer), or NULL.
  * partial: tgt_node_bwd_workers(rows) partial sums of the gradients of (Wq, Wk, Wv, bq, bk, bv, gamma, beta) or of
  * (Wh, bh, gamma, beta), each mats * 4096 + (mats + 2) * 64 floats: see tgt_node_sums. */
 typedef struct {
     int64_t rows;
-    int32_t dtype, tokens, classes;
+    int32_t dtype, tokens, classes, linear;
     float eps;
     const void *dq, *dk, *dv, *g_in, *s, *dlogp, *logp;
     const void* w_back;
@@ -635,7 +637,7 @@ int tgt_node_bwd_pre(const tgt_node_bwd_pre_args* args, void* stream);
  * (tgt_sparse_attn_bwd_from_nd), or NULL.  partial: sums for (Wo, W1, W2, bo, b1, b2, gamma, beta). */
 typedef struct {
     int64_t rows;
-    int32_t dtype, heads;
+    int32_t dtype, heads, same_bits;
     float eps;
     const void *g_in, *s, *attn;
     const void *w_post, *w_back;
@@ -653,13 +655,18 @@ typedef struct {
     void* out[8];
 } tgt_node_sum;
 int tgt_node_sums(const tgt_node_sum* sums, int count, int dtype, void* stream);
-/* The head of the graph-level models (models/graphormer_graph_level.py:383-388: final LayerNorm, the virtual node's row, output
- * projection): y[g] = LN(s[g, 0]) W^T + bias for s [b, S, 64], W [outputs, 64], 1 to 64 outputs.  Backward: g_out [b, S, 64] =
- * gradient of s (zero but for the virtual nodes' rows), dW, dbias, dgamma, dbeta (added in a fixed order). */
-int tgt_graph_head_fwd(const void* d_s, const void* d_gamma, const void* d_beta, float eps, const void* d_W, const void* d_bias, int b, int S,
-                       int outputs, int dtype, void* d_y, void* stream);
-int tgt_graph_head_bwd(const void* d_s, const void* d_gamma, const void* d_beta, float eps, const void* d_W, const void* d_dy, int b, int S,
-                       int outputs, int dtype, void* d_g_out, void* d_dW, void* d_dbias, void* d_dgamma, void* d_dbeta, void* stream);
+/* The dense biased attention for query 0 only: the last layer of the graph-level models, whose output is read at the virtual node
+ * (models/graphormer_graph_level.py:387).  Tensors as for tgt_dense_attn_dropout_fwd (H <= 8, d 8, 16 or 32, S <= 1024, dtype
+ * TGT_DTYPE_F32 or TGT_DTYPE_BF16); a0 [b, H d] = the attention's row 0 of every graph, s0 = the rows 0 of d_s [b, S, H d],
+ * lse [b, H].  Backward: da0, g0 [b, H d] = gradients of a0 and of s0; dq, dk, dv and g (the gradient of s) come back as full
+ * [b, S, H d] arrays, dvirt [b, H] = sums over the keys of the bias gradient's row 0 - a virtual node's row: it belongs to the
+ * virtual distance, to whose gradient tgt_dense_row0_virtual adds it. */
+int tgt_dense_row0_fwd(const void* d_q, const void* d_k, const void* d_v, const void* d_bias, const void* d_s, int b, int S, int H, int d, int dtype,
+                       float p_drop, uint64_t seed, void* d_a0, void* d_s0, float* d_lse, void* stream);
+int tgt_dense_row0_bwd(const void* d_q, const void* d_k, const void* d_v, const void* d_bias, int b, int S, int H, int d, int dtype, float p_drop,
+                       uint64_t seed, const void* d_a0, const float* d_lse, const void* d_da0, const void* d_g0, void* d_dq, void* d_dk, void* d_dv,
+                       void* d_g, float* d_dvirt, void* stream);
+int tgt_dense_row0_virtual(const float* d_dvirt, int b, int H, int dtype, void* d_dvirtual_dist, void* stream);
 /* tgt_sparse_attn_bwd for a caller that has already written the per-node side to the head of the workspace
  * (tgt_node_bwd_post with nd = d_workspace): no bias, and out and Z are not read. */
 int tgt_sparse_attn_bwd_from_nd(const tgt_plan_t* plan, const void* d_q, const void* d_k, const void* d_v, int H, int d, int dtype,

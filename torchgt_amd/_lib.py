@@ -95,8 +95,10 @@ SIGNATURES = {
     "tgt_graph_attn_bias_bwd_workspace_bytes": (_i64, [_i32, _i32, _i32]),
     "tgt_graph_attn_bias_bwd": (_i32, [_vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i64, _vp]),
     "tgt_graph_attn_bias_bwd_sum": (_i32, [_vp, _i32, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i64, _vp]),
-    "tgt_graph_head_fwd": (_i32, [_vp, _vp, _vp, _c.c_float, _vp, _vp, _i32, _i32, _i32, _i32, _vp, _vp]),
-    "tgt_graph_head_bwd": (_i32, [_vp, _vp, _vp, _c.c_float, _vp, _vp, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "tgt_dense_row0_fwd": (_i32, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _c.c_float, _c.c_uint64, _vp, _vp, _vp, _vp]),
+    "tgt_dense_row0_bwd": (_i32, [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _c.c_float, _c.c_uint64, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                                  _vp, _vp, _vp]),
+    "tgt_dense_row0_virtual": (_i32, [_vp, _i32, _i32, _i32, _vp, _vp]),
     "tgt_floyd_warshall": (_i32, [_vp, _vp, _i32, _i32, _vp, _vp, _vp]),
     "tgt_graph_attn_bias_multi_hop_fwd": (_i32, [_vp, _vp, _vp, _i32, _i32, _vp, _i32, _vp, _i32, _vp, _i32, _vp, _i32, _i32, _i32,
                                                  _i32, _i32, _vp, _vp]),

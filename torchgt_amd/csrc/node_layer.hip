@@ -101,18 +101,51 @@ template <typename T> __global__ __launch_bounds__(512) void k_node_pack(const P
     for (int q = 0; q < P; ++q) dst[(sm * P + q) * 64 + lane] = __builtin_bit_cast(vec16, p[q]);
 }
 
+// ---- GELU of a tile of pre-activations (and its slope) ---------------------------------------------------------------------
+// SAME (bf16): every sum and rounding as the separate kernels have it - GELU by the device library's error function, products of
+// half the depth, the bias behind the products, LayerNorm's sums in their order.  The graph-level models ask for it: they multiply
+// queries by sqrt(d), their attention is often all but a choice of one key, and in bf16 a rounding that falls the other way in one
+// activation moves every gradient of that graph by a per cent (0.019 of the gradients' norm without, 0.010 with it).
+template <typename T, bool SAME> __device__ __forceinline__ float cdf_and_bell(float v, float& bell) {
+    float cdf;
+    if constexpr (SAME) {
+        cdf = 0.5f * (1.f + erff(v * 0.70710678118654752f));
+        bell = __expf(-0.5f * v * v);
+    } else normal_cdf(v, cdf, bell);
+    return cdf;
+}
+template <typename T, bool SAME> __device__ __forceinline__ void gelu(Tile& u) {
+    TGT_EACH(i) {
+        const float v = stored(u.get(i), (const T*)nullptr);
+        float bell;
+        if constexpr (SAME) u.set(i, act_value<false>(v));
+        else u.set(i, v * cdf_and_bell<T, SAME>(v, bell));
+        if (i % 8 == 7) fence_schedule();
+    }
+}
+template <typename T, bool SAME> __device__ __forceinline__ void gelu(Tile& u, Tile& slope) {
+    TGT_EACH(i) {
+        const float v = stored(u.get(i), (const T*)nullptr);
+        float bell;
+        const float cdf = cdf_and_bell<T, SAME>(v, bell);
+        u.set(i, v * cdf);
+        slope.set(i, cdf + v * bell * 0.39894228040143268f);
+        if (i % 8 == 7) fence_schedule();
+    }
+}
+
 // ---- forward ------------------------------------------------------------------------------------------------------------
 enum { NEXT_NONE = 0, NEXT_QKV = 1, NEXT_CLASSES = 2 };
 
-template <typename T> constexpr int fwd_waves() { return sizeof(T) == 4 ? 8 : 16; }
+template <typename T, bool SAME> constexpr int fwd_waves() { return sizeof(T) == 4 || SAME ? 8 : 16; }
 // bf16 keeps all weights of a launch in LDS for the life of the workgroup; float32 planes of six weights (144 KB) do not
 // leave room for the row images, so its two halves take turns (the L2 has them)
 template <typename T, bool POST, int NEXT> constexpr int fwd_resident_mats() {
     const int post = POST ? 3 : 0, next = NEXT == NEXT_QKV ? 3 : (NEXT == NEXT_CLASSES ? 1 : 0);
     return sizeof(T) == 4 ? (post > next ? post : next) : post + next;
 }
-template <typename T, bool POST, int NEXT> constexpr int fwd_lds() {
-    return fwd_resident_mats<T, POST, NEXT>() * kFragVecs<Num<T>::P> * 16 + 10 * kVec * 4 + fwd_waves<T>() * RowShape<T>::kVecs * 16;
+template <typename T, bool SAME, bool POST, int NEXT> constexpr int fwd_lds() {
+    return fwd_resident_mats<T, POST, NEXT>() * kFragVecs<Num<T>::P> * 16 + 10 * kVec * 4 + fwd_waves<T, SAME>() * RowShape<T>::kVecs * 16;
 }
 
 // Rows of class values.  A wave's 32 rows are 32 C consecutive elements of the [N - tokens, C] array and travel through its
@@ -174,9 +207,9 @@ template <typename T> __device__ __forceinline__ T to_elem(float v);
 template <> __device__ __forceinline__ float to_elem<float>(float v) { return v; }
 template <> __device__ __forceinline__ nbf16 to_elem<nbf16>(float v) { return nbf16{__builtin_bit_cast(uint16_t, static_cast<__bf16>(v))}; }
 
-template <typename T, bool POST, int NEXT>
-__global__ __launch_bounds__(fwd_waves<T>() * 64) void k_node_fwd(const tgt_node_fwd_args a) {
-    constexpr int P = Num<T>::P, NW = fwd_waves<T>(), THREADS = NW * 64, FV = kFragVecs<P>;
+template <typename T, bool SAME, bool POST, int NEXT>
+__global__ __launch_bounds__((fwd_waves<T, SAME>() * 64)) void k_node_fwd(const tgt_node_fwd_args a) {
+    constexpr int P = Num<T>::P, NW = fwd_waves<T, SAME>(), THREADS = NW * 64, FV = kFragVecs<P>;
     constexpr bool RESIDENT = sizeof(T) == 2;
     constexpr int NMP = NEXT == NEXT_QKV ? 3 : (NEXT == NEXT_CLASSES ? 1 : 0);
     extern __shared__ __align__(16) unsigned char smem[];
@@ -225,23 +258,15 @@ __global__ __launch_bounds__(fwd_waves<T>() * 64) void k_node_fwd(const tgt_node
             if (POST) {
                 Tile x, y;
                 settle<T, false>(x, raw_a, stage, rows, lane);
-                load_vec(y, vec, h);                              // bo
-                TGT_EACH(i) s.set(i, s.get(i) + y.get(i));
-                gemm<P>(s, x, w, lane);                           // s1 = s + a Wo^T + bo
+                linear<P, SAME>(y, x, w, vec, lane);
+                TGT_EACH(i) s.set(i, s.get(i) + stored(y.get(i), (const T*)nullptr));      // s1 = s + (a Wo^T + bo)
                 x = s;
-                normalise(x, a.eps_post);
+                normalise<SAME>(x, a.eps_post);
                 affine(x, x, vec + kVec, vec + 2 * kVec, h);      // y2
-                load_vec(y, vec + 3 * kVec, h);
-                gemm<P>(y, x, w + FV, lane);                      // u
-                TGT_EACH(i) {
-                    float cdf, bell;
-                    normal_cdf(y.get(i), cdf, bell);
-                    y.set(i, y.get(i) * cdf);
-                    if (i % 8 == 7) fence_schedule();
-                }
-                load_vec(x, vec + 4 * kVec, h);
-                TGT_EACH(i) s.set(i, s.get(i) + x.get(i));
-                gemm<P>(s, y, w + 2 * FV, lane);                  // s' = s1 + h W2^T + b2
+                linear<P, SAME>(y, x, w + FV, vec + 3 * kVec, lane);    // u
+                gelu<T, SAME>(y);
+                linear<P, SAME>(x, y, w + 2 * FV, vec + 4 * kVec, lane);
+                TGT_EACH(i) s.set(i, stored(s.get(i), (const T*)nullptr) + stored(x.get(i), (const T*)nullptr));      // s'
                 put_rows(reinterpret_cast<T*>(a.s_out), s, stage, rows, lane);
             }
         }
@@ -251,29 +276,30 @@ __global__ __launch_bounds__(fwd_waves<T>() * 64) void k_node_fwd(const tgt_node
             __syncthreads();
         }
         if (NEXT && active) {
-            normalise(s, a.eps_next);
+            normalise<SAME>(s, a.eps_next);
             affine(s, s, vn, vn + kVec, h);
             if (NEXT == NEXT_QKV) {
 #pragma unroll
                 for (int j = 0; j < 3; ++j) {
                     Tile y;
-                    load_vec(y, vn + (2 + j) * kVec, h);
-                    gemm<P>(y, s, w_next + j * FV, lane);
+                    linear<P, SAME>(y, s, w_next + j * FV, vn + (2 + j) * kVec, lane);
                     put_rows(reinterpret_cast<T*>(j == 0 ? a.q : (j == 1 ? a.k : a.v)), y, stage, rows, lane);
                 }
             } else {
                 Tile y;
-                load_vec(y, vn + 2 * kVec, h);
-                gemm<P>(y, s, w_next, lane);
+                linear<P, SAME>(y, s, w_next, vn + 2 * kVec, lane);
                 const int C = a.classes;
-                float top = -INFINITY, sum = 0.f;
-                TGT_EACH(i) {      // rounded first: log_softmax reads the logits as a T tensor would hold them
-                    y.set(i, stored(y.get(i), (const T*)nullptr));
-                    if (32 * h + i < C) top = fmaxf(top, y.get(i));
+                float lse = 0.f;
+                if (!a.linear) {
+                    float top = -INFINITY, sum = 0.f;
+                    TGT_EACH(i) {      // rounded first: log_softmax reads the logits as a T tensor would hold them
+                        y.set(i, stored(y.get(i), (const T*)nullptr));
+                        if (32 * h + i < C) top = fmaxf(top, y.get(i));
+                    }
+                    top = fmaxf(top, __shfl_xor(top, 32, 64));
+                    TGT_EACH(i) if (32 * h + i < C) sum += expf(y.get(i) - top);
+                    lse = top + logf(both_halves(sum));
                 }
-                top = fmaxf(top, __shfl_xor(top, 32, 64));
-                TGT_EACH(i) if (32 * h + i < C) sum += expf(y.get(i) - top);
-                const float lse = top + logf(both_halves(sum));
                 const ClassRows<T> out(stage, row0, N, a.tokens, C);
                 wave_sync();
                 TGT_EACH(i) if (32 * h + i < C) out.img[(lane & 31) * C + 32 * h + i] = to_elem<T>(y.get(i) - lse);
@@ -317,8 +343,8 @@ template <int NM, int NV> __device__ __forceinline__ void write_partial(float* _
     for (int i = threadIdx.x; i < NV * 64; i += kBwdThreads) mine[NM * 4096 + i] = (buf[i] + buf[NV * 64 + i]) + (buf[2 * NV * 64 + i] + buf[3 * NV * 64 + i]);
 }
 
-// Class gradients of a wave's 32 rows: d logits = d logp - softmax * sum(d logp); zero for tokens and past the end.
-template <typename T> __device__ __forceinline__ void class_grads(Tile& d, const T* __restrict__ dlogp, const T* __restrict__ logp, int C, int tokens, int64_t row0, int64_t N,
+// Class gradients of a wave's 32 rows: d logits = d logp - softmax * sum(d logp) (linear: d logits as they come); zero for tokens and past the end.
+template <typename T> __device__ __forceinline__ void class_grads(Tile& d, const T* __restrict__ dlogp, const T* __restrict__ logp, bool linear, int C, int tokens, int64_t row0, int64_t N,
                                                                   vec16* stage, int lane) {
     const int n = lane & 31, h = lane >> 5;
     ClassRows<T> rows(stage, row0, N, tokens, C);
@@ -330,6 +356,7 @@ template <typename T> __device__ __forceinline__ void class_grads(Tile& d, const
         d.set(i, in && 32 * h + i < C ? as_float(mine[i]) : 0.f);
         sum += d.get(i);
     }
+    if (linear) return;
     sum = both_halves(sum);
     rows.load(logp, lane);
     TGT_EACH(i) if (in && 32 * h + i < C) d.set(i, d.get(i) - expf(as_float(mine[i])) * sum);
@@ -371,11 +398,11 @@ __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_pre(const tgt_node_bwd
             Tile xhat, dy, d;
             Frags<P> f;
             settle<T, false>(xhat, raw_s, stage, rows, lane);
-            const float rstd = normalise(xhat, a.eps);
+            const float rstd = normalise<false>(xhat, a.eps);
             zero(dy);
 #pragma unroll
             for (int j = 0; j < NM; ++j) {
-                if (CLASSES) class_grads(d, reinterpret_cast<const T*>(a.dlogp), reinterpret_cast<const T*>(a.logp), a.classes, a.tokens, (4 * g0 + wave) * 32, N, stage, lane);
+                if (CLASSES) class_grads(d, reinterpret_cast<const T*>(a.dlogp), reinterpret_cast<const T*>(a.logp), a.linear, a.classes, a.tokens, (4 * g0 + wave) * 32, N, stage, lane);
                 else {
                     settle<T, true>(d, raw_d, stage, rows, lane);
                     fetch(raw_d, j + 1 < NM ? src[j + 1] : reinterpret_cast<const T*>(a.g_in), rows, lane);
@@ -396,6 +423,7 @@ __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_pre(const tgt_node_bwd
                 __syncthreads();                       // planes j are there, weight j has been used
             }
             if (g0 + gridDim.x < groups) fetch(raw_s, reinterpret_cast<const T*>(a.s), Rows(4 * (g0 + gridDim.x) + wave, N), lane);
+            TGT_EACH(i) dy.set(i, stored(dy.get(i), (const T*)nullptr));
             col[NM + 1] += column_sums(dy, lane);
             TGT_EACH(i) d.set(i, dy.get(i) * xhat.get(i));
             col[NM] += column_sums(d, lane);
@@ -434,7 +462,7 @@ __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_pre(const tgt_node_bwd
 }
 
 // ---- backward of the part behind an attention -------------------------------------------------------------------------------
-template <typename T>
+template <typename T, bool SAME>
 __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_post(const tgt_node_bwd_post_args a) {
     using L = BwdLds<T>;
     constexpr int P = Num<T>::P, FV = kFragVecs<P>;
@@ -474,32 +502,28 @@ __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_post(const tgt_node_bw
                 fetch(raw_g, reinterpret_cast<const T*>(a.g_in), ahead, lane);
             };
             Tile g, xhat, slope, t;
-            Frags<P> f;
+            Frags<P> f, fy;      // fy: LayerNorm's output, kept in its one plane for bf16, formed again from xhat for float32
             settle<T, false>(t, raw_a, stage, rows, lane);
             make_frags(f, t);
             settle<T, false>(xhat, raw_s, stage, rows, lane);
-            load_vec(t, vec, h);
-            TGT_EACH(i) xhat.set(i, xhat.get(i) + t.get(i));
             settle<T, true>(g, raw_g, stage, rows, lane);
             col[2] += column_sums(g, lane);
             __syncthreads();                                        // Wo is there; product Wo of the round before is done
-            gemm<P>(xhat, f, w, lane);                              // s1
+            linear<P, SAME>(t, f, w, vec, lane);
             __syncthreads();                                        // Wo has been used
-            const float rstd = normalise(xhat, a.eps);
-            affine(t, xhat, vec + kVec, vec + 2 * kVec, h);
-            make_frags(f, t);
-            load_vec(t, vec + 3 * kVec, h);
-            __syncthreads();                                        // W1
-            gemm<P>(t, f, w, lane);                                 // u
-            __syncthreads();                                        // W1 has been used
-            TGT_EACH(i) {
-                const float u = t.get(i);
-                float cdf, bell;
-                normal_cdf(u, cdf, bell);
-                t.set(i, u * cdf);
-                slope.set(i, cdf + u * bell * 0.39894228040143268f);
-                if (i % 8 == 7) fence_schedule();
+            TGT_EACH(i) xhat.set(i, xhat.get(i) + stored(t.get(i), (const T*)nullptr));      // s1
+            t = xhat;
+            const MeanRstd stat = row_stats<SAME>(t, a.eps);
+            TGT_EACH(i) {      // LayerNorm's output is made of s1, its backward reads s1 as the stream holds it
+                t.set(i, (t.get(i) - stat.mean) * stat.rstd);
+                xhat.set(i, (stored(xhat.get(i), (const T*)nullptr) - stat.mean) * stat.rstd);
             }
+            affine(t, t, vec + kVec, vec + 2 * kVec, h);
+            make_frags(fy, t);
+            __syncthreads();                                        // W1
+            linear<P, SAME>(t, fy, w, vec + 3 * kVec, lane);           // u
+            __syncthreads();                                        // W1 has been used
+            gelu<T, SAME>(t, slope);
             make_frags(f, t);
             put_planes<P>(p_x, row, h, f);
             make_frags(f, g);
@@ -507,23 +531,25 @@ __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_post(const tgt_node_bw
             __syncthreads();                                        // planes of W2; W2^T
             zero(t);
             gemm<P>(t, f, w, lane);                                 // d gelu, beside product W2
-            TGT_EACH(i) t.set(i, t.get(i) * slope.get(i));          // du
+            TGT_EACH(i) t.set(i, stored(t.get(i) * slope.get(i), (const T*)nullptr));      // du
             col[1] += column_sums(t, lane);
             make_frags(f, t);
-            affine(t, xhat, vec + kVec, vec + 2 * kVec, h);
+            if (P != 1) {
+                forget(xhat);
+                affine(t, xhat, vec + kVec, vec + 2 * kVec, h);
+            }
             __syncthreads();                                        // product W2 is done, W2^T has been used
             put_planes<P>(p_dy, row, h, f);
-            {
-                Frags<P> fx;
-                make_frags(fx, t);
-                put_planes<P>(p_x, row, h, fx);
-            }
+            if (P != 1) make_frags(fy, t);
+            put_planes<P>(p_x, row, h, fy);
             __syncthreads();                                        // planes of W1; W1^T
             fetch(raw_a, reinterpret_cast<const T*>(a.attn), rows, lane);
             zero(t);
             gemm<P>(t, f, w, lane);                                 // d LN, beside product W1
+            TGT_EACH(i) t.set(i, stored(t.get(i), (const T*)nullptr));
             col[4] += column_sums(t, lane);
-            ln_back(g, t, xhat, rstd, vec + kVec, h);
+            ln_back(g, t, xhat, stat.rstd, vec + kVec, h);
+            TGT_EACH(i) g.set(i, stored(g.get(i), (const T*)nullptr));
             TGT_EACH(i) t.set(i, t.get(i) * xhat.get(i));
             col[3] += column_sums(t, lane);
             col[0] += column_sums(g, lane);
@@ -634,84 +660,6 @@ template <typename T> __global__ __launch_bounds__(1024) void k_node_sums(const 
     }
 }
 
-// ---- head of the graph-level models ---------------------------------------------------------------------------------------
-// One row per graph (the virtual node's): a few microseconds of latency whatever the shape.  Lane = feature.
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-template <typename T> __device__ __forceinline__ float head_row(const T* __restrict__ s, int64_t row, float eps, int lane, float& rstd) {
-    const float v = as_float(s[row * 64 + lane]), mean = wave_sum(v) * (1.f / 64), d = v - mean;
-    rstd = rsqrtf(wave_sum(d * d) * (1.f / 64) + eps);
-    return d * rstd;
-}
-template <typename T>
-__global__ __launch_bounds__(256) void k_graph_head_fwd(const T* __restrict__ s, const T* __restrict__ gamma, const T* __restrict__ beta, float eps, const T* __restrict__ W,
-                                                         const T* __restrict__ bias, int b, int S, int O, T* __restrict__ y) {
-    const int lane = threadIdx.x & 63, g = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (g >= b) return;
-    float rstd;
-    const float xhat = head_row(s, (int64_t)g * S, eps, lane, rstd);
-    const float v = stored(xhat * as_float(gamma[lane]) + as_float(beta[lane]), (const T*)nullptr);
-    for (int o = 0; o < O; ++o) {
-        const float t = wave_sum(v * as_float(W[o * 64 + lane]));
-        if (lane == 0) y[(int64_t)g * O + o] = to_elem<T>(t + as_float(bias[o]));
-    }
-}
-// Workgroup 0: the virtual nodes' rows and all parameter gradients, sixteen graphs at a time (wave = graph for the rows; wave =
-// slice of the outputs for the sums over graphs).  The others write the zero rows.
-template <typename T>
-__global__ __launch_bounds__(1024) void k_graph_head_bwd(const T* __restrict__ s, const T* __restrict__ gamma, const T* __restrict__ beta, float eps, const T* __restrict__ W,
-                                                          const T* __restrict__ dy, int b, int S, int O, T* __restrict__ g_out, T* __restrict__ dW, T* __restrict__ db,
-                                                          T* __restrict__ dgamma, T* __restrict__ dbeta) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (blockIdx.x > 0) {
-        constexpr int PP = RowShape<T>::kPieces;
-        const int64_t n = (int64_t)b * S * PP;
-        for (int64_t i = (int64_t)(blockIdx.x - 1) * 1024 + threadIdx.x; i < n; i += (int64_t)(gridDim.x - 1) * 1024)
-            if ((i / PP) % S != 0) reinterpret_cast<vec16*>(g_out)[i] = vec16{0u, 0u, 0u, 0u};
-        return;
-    }
-    __shared__ float sy[16][64], sd[16][64], sx[16][64], sdy[16][64];
-    float aw[4] = {0.f, 0.f, 0.f, 0.f}, ab[4] = {0.f, 0.f, 0.f, 0.f}, ag = 0.f, abt = 0.f;
-    const float gm = as_float(gamma[lane]), bt = as_float(beta[lane]);
-    for (int g0 = 0; g0 < b; g0 += 16) {
-        const int g = g0 + wave;
-        float d = 0.f, xhat = 0.f, rstd = 0.f, v = 0.f;
-        if (g < b) {
-            xhat = head_row(s, (int64_t)g * S, eps, lane, rstd);
-            v = stored(xhat * gm + bt, (const T*)nullptr);
-            for (int o = 0; o < O; ++o) d += as_float(dy[(int64_t)g * O + o]) * as_float(W[o * 64 + lane]);
-            const float t = d * gm, c1 = wave_sum(t) * (1.f / 64), c2 = wave_sum(t * xhat) * (1.f / 64);
-            g_out[(int64_t)g * S * 64 + lane] = to_elem<T>(rstd * (t - c1 - xhat * c2));
-        }
-        sy[wave][lane] = v; sd[wave][lane] = d; sx[wave][lane] = d * xhat;
-        sdy[wave][lane] = g < b && lane < O ? as_float(dy[(int64_t)g * O + lane]) : 0.f;
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int o = wave + 16 * k;
-            if (o < O)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) { aw[k] += sdy[i][o] * sy[i][lane]; ab[k] += sdy[i][o]; }
-        }
-        if (wave == 0)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) { abt += sd[i][lane]; ag += sx[i][lane]; }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int o = wave + 16 * k;
-        if (o < O) {
-            dW[o * 64 + lane] = to_elem<T>(aw[k]);
-            if (lane == 0) db[o] = to_elem<T>(ab[k]);
-        }
-    }
-    if (wave == 0) { dgamma[lane] = to_elem<T>(ag); dbeta[lane] = to_elem<T>(abt); }
-}
-
 int bad(const char* who, const char* what) { set_error("%s: %s", who, what); return TGT_ERR_INVALID_ARG; }
 int num_cus() {
     static const int n = [] { int dev = 0, v = 256; if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev); return v > 0 ? v : 256; }();
@@ -737,22 +685,22 @@ template <typename... Args> int launch(void (*kernel)(Args...), std::atomic<uint
     return TGT_OK;
 }
 
-template <typename T, bool POST, int NEXT> int launch_fwd(const tgt_node_fwd_args& a, hipStream_t st) {
+template <typename T, bool SAME, bool POST, int NEXT> int launch_fwd(const tgt_node_fwd_args& a, hipStream_t st) {
     static std::atomic<uint64_t> done{0};
-    return launch(&k_node_fwd<T, POST, NEXT>, done, grid_for(a.rows, fwd_waves<T>()), fwd_waves<T>() * 64, fwd_lds<T, POST, NEXT>(), st, a);
+    return launch(&k_node_fwd<T, SAME, POST, NEXT>, done, grid_for(a.rows, fwd_waves<T, SAME>()), fwd_waves<T, SAME>() * 64, fwd_lds<T, SAME, POST, NEXT>(), st, a);
 }
-template <typename T> int dispatch_fwd(const tgt_node_fwd_args& a, hipStream_t st) {
-    if (a.attn) return a.logp ? launch_fwd<T, true, NEXT_CLASSES>(a, st) : (a.q ? launch_fwd<T, true, NEXT_QKV>(a, st) : launch_fwd<T, true, NEXT_NONE>(a, st));
-    return launch_fwd<T, false, NEXT_QKV>(a, st);
+template <typename T, bool SAME> int dispatch_fwd(const tgt_node_fwd_args& a, hipStream_t st) {
+    if (a.attn) return a.logp ? launch_fwd<T, SAME, true, NEXT_CLASSES>(a, st) : (a.q ? launch_fwd<T, SAME, true, NEXT_QKV>(a, st) : launch_fwd<T, SAME, true, NEXT_NONE>(a, st));
+    return launch_fwd<T, SAME, false, NEXT_QKV>(a, st);
 }
 template <typename T> int dispatch_bwd_pre(const tgt_node_bwd_pre_args& a, int workers, hipStream_t st) {
     static std::atomic<uint64_t> done[2];
     return a.dlogp ? launch(&k_node_bwd_pre<T, true>, done[1], workers, kBwdThreads, BwdLds<T>::kBytes, st, a)
                    : launch(&k_node_bwd_pre<T, false>, done[0], workers, kBwdThreads, BwdLds<T>::kBytes, st, a);
 }
-template <typename T> int dispatch_bwd_post(const tgt_node_bwd_post_args& a, int workers, hipStream_t st) {
+template <typename T, bool SAME> int dispatch_bwd_post(const tgt_node_bwd_post_args& a, int workers, hipStream_t st) {
     static std::atomic<uint64_t> done{0};
-    return launch(&k_node_bwd_post<T>, done, workers, kBwdThreads, BwdLds<T>::kBytes, st, a);
+    return launch(&k_node_bwd_post<T, SAME>, done, workers, kBwdThreads, BwdLds<T>::kBytes, st, a);
 }
 bool dtype_ok(int dtype) { return dtype == TGT_DTYPE_F32 || dtype == TGT_DTYPE_BF16; }
 
@@ -800,7 +748,9 @@ int tgt_node_fwd(const tgt_node_fwd_args* a, void* stream) {
     if (a->tokens < 0 || (!a->attn && a->tokens > 0 && (!a->token || !a->s_out))) return bad("tgt_node_fwd", "tokens need their table and s_out");
     if (a->rows == 0) return TGT_OK;
     KernelTimer t(KS_LINEAR_FWD, (hipStream_t)stream);
-    return a->dtype == TGT_DTYPE_F32 ? dispatch_fwd<float>(*a, (hipStream_t)stream) : dispatch_fwd<nbf16>(*a, (hipStream_t)stream);
+    const hipStream_t st = (hipStream_t)stream;
+    if (a->dtype == TGT_DTYPE_F32) return dispatch_fwd<float, false>(*a, st);
+    return a->same_bits ? dispatch_fwd<nbf16, true>(*a, st) : dispatch_fwd<nbf16, false>(*a, st);
 }
 
 int tgt_node_bwd_workers(int64_t rows) { return rows < 0 ? -1 : tgt::grid_for(rows, 4); }
@@ -808,7 +758,7 @@ int tgt_node_bwd_workers(int64_t rows) { return rows < 0 ? -1 : tgt::grid_for(ro
 int tgt_node_bwd_pre(const tgt_node_bwd_pre_args* a, void* stream) {
     using namespace tgt;
     if (!a || a->rows < 1 || !dtype_ok(a->dtype) || !a->s || !a->g_out || !a->w_back || !a->v_next || !a->partial) return bad("tgt_node_bwd_pre", "null or bad argument");
-    if (a->dlogp ? (!a->logp || a->classes < 1 || a->classes > 64 || a->tokens < 0) : (!a->dq || !a->dk || !a->dv || !a->g_in))
+    if (a->dlogp ? ((!a->logp && !a->linear) || a->classes < 1 || a->classes > 64 || a->tokens < 0) : (!a->dq || !a->dk || !a->dv || !a->g_in))
         return bad("tgt_node_bwd_pre", "dq, dk, dv, g_in or dlogp, logp and 1 to 64 classes are needed");
     KernelTimer t(KS_LINEAR_DX, (hipStream_t)stream);
     const int workers = grid_for(a->rows, 4);
@@ -821,41 +771,10 @@ int tgt_node_bwd_post(const tgt_node_bwd_post_args* a, void* stream) {
         return bad("tgt_node_bwd_post", "null or bad argument");
     if (a->nd && (!a->Z || (a->heads != 8 && a->heads != 4 && a->heads != 2))) return bad("tgt_node_bwd_post", "nd needs Z and 8, 4 or 2 heads");
     KernelTimer t(KS_LINEAR_DX, (hipStream_t)stream);
+    const hipStream_t st = (hipStream_t)stream;
     const int workers = grid_for(a->rows, 4);
-    return a->dtype == TGT_DTYPE_F32 ? dispatch_bwd_post<float>(*a, workers, (hipStream_t)stream) : dispatch_bwd_post<nbf16>(*a, workers, (hipStream_t)stream);
-}
-
-int tgt_graph_head_fwd(const void* d_s, const void* d_gamma, const void* d_beta, float eps, const void* d_W, const void* d_bias, int b, int S,
-                       int outputs, int dtype, void* d_y, void* stream) {
-    using namespace tgt;
-    if (!d_s || !d_gamma || !d_beta || !d_W || !d_bias || !d_y || b < 0 || S < 1 || outputs < 1 || outputs > 64 || !dtype_ok(dtype)) return bad("tgt_graph_head_fwd", "null or bad argument");
-    if (b == 0) return TGT_OK;
-    KernelTimer t(KS_LINEAR_FWD, (hipStream_t)stream);
-    const auto run = [&](auto tag) {
-        using T = decltype(tag);
-        hipLaunchKernelGGL((k_graph_head_fwd<T>), dim3((b + 3) / 4), dim3(256), 0, (hipStream_t)stream, (const T*)d_s, (const T*)d_gamma, (const T*)d_beta, eps, (const T*)d_W,
-                           (const T*)d_bias, b, S, outputs, (T*)d_y);
-    };
-    if (dtype == TGT_DTYPE_F32) run(float()); else run(nbf16());
-    TGT_HIP_CHECK(hipGetLastError());
-    return TGT_OK;
-}
-
-int tgt_graph_head_bwd(const void* d_s, const void* d_gamma, const void* d_beta, float eps, const void* d_W, const void* d_dy, int b, int S,
-                       int outputs, int dtype, void* d_g_out, void* d_dW, void* d_dbias, void* d_dgamma, void* d_dbeta, void* stream) {
-    using namespace tgt;
-    if (!d_s || !d_gamma || !d_beta || !d_W || !d_dy || !d_g_out || !d_dW || !d_dbias || !d_dgamma || !d_dbeta || b < 1 || S < 1 || outputs < 1 || outputs > 64 || !dtype_ok(dtype))
-        return bad("tgt_graph_head_bwd", "null or bad argument");
-    KernelTimer t(KS_LINEAR_DX, (hipStream_t)stream);
-    const int zeros = (int)std::min<int64_t>(num_cus(), ((int64_t)b * S * 16 + 1023) / 1024);
-    const auto run = [&](auto tag) {
-        using T = decltype(tag);
-        hipLaunchKernelGGL((k_graph_head_bwd<T>), dim3(1 + zeros), dim3(1024), 0, (hipStream_t)stream, (const T*)d_s, (const T*)d_gamma, (const T*)d_beta, eps, (const T*)d_W,
-                           (const T*)d_dy, b, S, outputs, (T*)d_g_out, (T*)d_dW, (T*)d_dbias, (T*)d_dgamma, (T*)d_dbeta);
-    };
-    if (dtype == TGT_DTYPE_F32) run(float()); else run(nbf16());
-    TGT_HIP_CHECK(hipGetLastError());
-    return TGT_OK;
+    if (a->dtype == TGT_DTYPE_F32) return dispatch_bwd_post<float, false>(*a, workers, st);
+    return a->same_bits ? dispatch_bwd_post<nbf16, true>(*a, workers, st) : dispatch_bwd_post<nbf16, false>(*a, workers, st);
 }
 
 int tgt_node_sums(const tgt_node_sum* sums, int count, int dtype, void* stream) {

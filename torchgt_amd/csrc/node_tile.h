@@ -9,7 +9,8 @@
 // linears, residual adds, LayerNorms and activations never leaves the registers.  LayerNorm sums are 32 adds in a lane
 // and one exchange between the halves.
 //
-// Number formats.  float32 rows go through the matrix unit as three bf16 planes (see linear.hip: hi + mid + lo is exact,
+// Number formats.  bf16 kernels round where a chain of separate kernels would have stored a tensor (`stored`), so a model gives
+// the same numbers whichever way it runs, up to the order of float32 sums.  float32 rows go through the matrix unit as three bf16 planes (see linear.hip: hi + mid + lo is exact,
 // six products per pair of planes give the float32 product to a few 2^-23); bf16 rows as one.  P = number of planes.
 #pragma once
 #include "common.h"
@@ -83,6 +84,13 @@ __device__ __forceinline__ float16_t mma_planes(const bf16x8_t (&a)[3], const bf
     return mma(a[0], b[0], c);
 }
 __device__ __forceinline__ float16_t mma_planes(const bf16x8_t (&a)[1], const bf16x8_t (&b)[1], float16_t c) { return mma(a[0], b[0], c); }
+// one plane as two products of half the depth, in the order linear.hip adds them
+__device__ __forceinline__ float16_t mma_halves(bf16x8_t a, bf16x8_t b, float16_t c) {
+    typedef short short8_t __attribute__((ext_vector_type(8)));
+    const short8_t x = __builtin_bit_cast(short8_t, a), y = __builtin_bit_cast(short8_t, b);
+    c = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(short4_t{x[0], x[1], x[2], x[3]}, short4_t{y[0], y[1], y[2], y[3]}, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(short4_t{x[4], x[5], x[6], x[7]}, short4_t{y[4], y[5], y[6], y[7]}, c, 0, 0, 0);
+}
 
 // A packed 64 x 64 weight: operand A of step s and row block m, plane p, at ((2 s + m) P + p) * 64 + lane (16 bytes per
 // lane): row block m, row 8 j + 4 hh + t is output feature 32 hh + 16 m + 4 j + t; a lane's eight contraction indices are
@@ -114,7 +122,8 @@ template <int P> __device__ __forceinline__ void step_operand(bf16x8_t (&x)[P], 
 #pragma unroll
     for (int p = 0; p < P; ++p) x[p] = b.p[s][p];
 }
-template <int P, typename B> __device__ __forceinline__ void gemm(Tile& acc, const B& b, const vec16* w, int lane) {
+// HALVES: bits of the separate linears (linear.hip), for one plane
+template <int P, bool HALVES = false, typename B> __device__ __forceinline__ void gemm(Tile& acc, const B& b, const vec16* w, int lane) {
     StepWeights<P> f[2];
     step_weights<P>(f[0], w, 0, lane);
     float16_t c[2];
@@ -125,7 +134,10 @@ template <int P, typename B> __device__ __forceinline__ void gemm(Tile& acc, con
         bf16x8_t x[P];
         step_operand<P>(x, b, s);
 #pragma unroll
-        for (int m = 0; m < 2; ++m) c[m] = mma_planes(f[s & 1].a[m], x, c[m]);
+        for (int m = 0; m < 2; ++m) {
+            if constexpr (HALVES && P == 1) c[m] = mma_halves(f[s & 1].a[m][0], x[0], c[m]);
+            else c[m] = mma_planes(f[s & 1].a[m], x, c[m]);
+        }
         fence_schedule();
     }
     TGT_EACH(i) acc.set(i, c[i >> 4][i & 15]);
@@ -275,16 +287,52 @@ __device__ __forceinline__ void load_vec(Tile& t, const float* vec, int h) {
         t.set(4 * i, f.x); t.set(4 * i + 1, f.y); t.set(4 * i + 2, f.z); t.set(4 * i + 3, f.w);
     }
 }
-// x -> (x - mean) * rstd over the 64 features; returns rstd
-__device__ __forceinline__ float normalise(Tile& x, float eps) {
-    float s = 0.f;
-    TGT_EACH(i) s += x.get(i);
-    const float mean = both_halves(s) * (1.f / 64);
-    float v = 0.f;
-    TGT_EACH(i) { const float d = x.get(i) - mean; v += d * d; }
-    const float rstd = rsqrtf(both_halves(v) * (1.f / 64) + eps);
-    TGT_EACH(i) x.set(i, (x.get(i) - mean) * rstd);
-    return rstd;
+// y = W x + bias (vec: 64 floats in LDS).  SAME: the bits of linear.hip, which adds the bias behind the products.
+template <int P, bool SAME, typename B> __device__ __forceinline__ void linear(Tile& y, const B& x, const vec16* w, const float* vec, int lane) {
+    if constexpr (SAME) {
+        zero(y);
+        gemm<P, true>(y, x, w, lane);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float4 f = *reinterpret_cast<const float4*>(vec + 32 * (lane >> 5) + 4 * i);
+            y.set(4 * i, y.get(4 * i) + f.x); y.set(4 * i + 1, y.get(4 * i + 1) + f.y);
+            y.set(4 * i + 2, y.get(4 * i + 2) + f.z); y.set(4 * i + 3, y.get(4 * i + 3) + f.w);
+        }
+    } else {
+        load_vec(y, vec, lane >> 5);
+        gemm<P>(y, x, w, lane);
+    }
+}
+
+struct MeanRstd { float mean, rstd; };
+// sum of f(i) over the 64 features; SAME: eights in order, then the eights as elementwise.hip's lanes exchange them
+template <bool SAME, typename F> __device__ __forceinline__ float sum_features(const F& f) {
+    if constexpr (SAME) {
+        float t[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float s = 0.f;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) s += f(8 * i + k);
+            t[i] = both_halves(s);
+        }
+        return (t[0] + t[2]) + (t[1] + t[3]);
+    } else {
+        float s = 0.f;
+        TGT_EACH(i) s += f(i);
+        return both_halves(s);
+    }
+}
+template <bool SAME> __device__ __forceinline__ MeanRstd row_stats(const Tile& x, float eps) {
+    const float mean = sum_features<SAME>([&](int i) { return x.get(i); }) * (1.f / 64);
+    const float var = sum_features<SAME>([&](int i) { const float d = x.get(i) - mean; return d * d; }) * (1.f / 64);
+    return {mean, rsqrtf(var + eps)};
+}
+// x -> (x - mean) * rstd; returns rstd
+template <bool SAME> __device__ __forceinline__ float normalise(Tile& x, float eps) {
+    const MeanRstd m = row_stats<SAME>(x, eps);
+    TGT_EACH(i) x.set(i, (x.get(i) - m.mean) * m.rstd);
+    return m.rstd;
 }
 // xhat * gamma + beta, vectors in LDS
 __device__ __forceinline__ void affine(Tile& y, const Tile& xhat, const float* gamma, const float* beta, int h) {

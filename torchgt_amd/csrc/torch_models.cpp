@@ -3,7 +3,7 @@
 //
 //   torchgt::node_graphormer(x, params[7 + 16 L], plan holder, workspace, heads, tokens, eps[2 L + 1]) -> log-probabilities
 //   torchgt::graph_graphormer(x, in_degree, out_degree, attn_bias, spatial_pos, edge_ids, params[11 (12) + 16 L], multi_hop, max_dist,
-//                             heads, eps[2 L + 1], p_drop, seeds[L], bf16_products) -> predictions
+//                             heads, eps[2 L + 1], p_drop, seeds[L]) -> predictions
 //
 // A step's intermediate rows live in one allocation, its parameter gradients in another: with some seventy parameters the
 // host's time for tensors of their own would be longer than the kernels of a small graph take.
@@ -298,7 +298,7 @@ Tensor node_graphormer(const Tensor& x, at::TensorList P, const c10::intrusive_p
 // params: atom, in-degree, out-degree tables, graph token; spatial table, edge table, virtual distance (, hop matrices);
 // 16 per layer; gamma, beta (final norm), Wh, bh
 struct GraphCall {
-    bool multi_hop = false, bf16_products = false;
+    bool multi_hop = false;
     int64_t max_dist = 0, H = 0;
     double p_drop = 0;
     std::vector<double> eps;
@@ -309,24 +309,33 @@ struct GraphBatch { Tensor x, in_degree, out_degree, spatial, edges; };      // 
 
 struct GraphGraphormerFn : public torch::autograd::Function<GraphGraphormerFn> {
     static constexpr int kFixed = 7;
-    // dlse etc. of the layers live next to the rows: s_0 .. s_L, then q, k, v, a of every layer
+    // rows of the buffer: s_0 .. s_{L-1}, then q, k, v, a of every layer but the last, then q, k, v of the last, whose attention
+    // and everything behind it is needed at one row per graph only: a, s and s' of those rows follow
+    struct Layout {
+        int64_t N, b, L, ns;
+        bool keep;
+        Layout(int64_t N_, int64_t b_, int64_t L_, bool k) : N(N_), b(b_), L(L_), ns(k ? L_ : 1), keep(k) {}
+        int64_t s(int64_t l) const { return keep ? l * N : 0; }
+        int64_t a(int64_t l, int i) const { return (ns + (keep ? 4 * l : 0) + i) * N; }
+        int64_t thin(int i) const { return (ns + (keep ? 4 * L - 1 : 4)) * N + i * b; }      // 0: a, 1: s, 2: s'
+        int64_t rows() const { return thin(3); }
+    };
     static Tensor compute(const GraphBatch& in, const Tensor& attn_bias, const std::vector<Tensor>& p, const GraphCall& c, bool keep, Tensor& rows, Tensor& lse, Tensor& bias,
                           Packed& packed) {
-        const int code = dtype_code(p[0]), H = (int)c.H, tables = kFixed + (c.multi_hop ? 1 : 0);
-        const int dense = code == TGT_DTYPE_F32 && c.bf16_products ? TGT_DTYPE_F32_BF16_PRODUCTS : code;
+        const int code = dtype_code(p[0]), H = (int)c.H, d = (int)(kWidth / c.H), tables = kFixed + (c.multi_hop ? 1 : 0);
         const int64_t L = (int64_t)(p.size() - tables - 4) / 16, b = in.x.size(0), s = in.x.size(1), S = s + 1, N = b * S;
         const auto opt = p[0].options();
         void* stream = stream_of(p[0]);
-        const int64_t ns = keep ? L + 1 : 1, na = keep ? 4 * L : 4;
-        rows = at::empty({(ns + na) * N, kWidth}, opt);
-        lse = at::empty({keep ? L * b * H * S : b * H * S}, opt.dtype(at::kFloat));
+        const Layout at(N, b, L, keep);
+        rows = at::empty({at.rows(), kWidth}, opt);
+        lse = at::empty({(keep ? (L - 1) * b * H * S : b * H * S) + b * H}, opt.dtype(at::kFloat));
+        float* thin_lse = lse.data_ptr<float>() + lse.numel() - b * H;
         bias = at::empty({b, H, S, S}, opt);
-        packed = Packed(p.data() + tables, L, nullptr, code, opt, stream);
-        auto s_row = [&](int64_t l) { return at_row(rows, keep ? l * N : 0); };
-        auto a_row = [&](int64_t l, int i) { return at_row(rows, (ns + (keep ? 4 * l : 0) + i) * N); };
+        const Tensor* head = p.data() + tables + 16 * L;
+        packed = Packed(p.data() + tables, L, head, code, opt, stream);
         check(tgt_graph_node_feature_fwd(in.x.data_ptr<int64_t>(), in.in_degree.data_ptr<int64_t>(), in.out_degree.data_ptr<int64_t>(), (int)in.x.size(2), p[0].data_ptr(),
                                          (int)p[0].size(0), p[1].data_ptr(), (int)p[1].size(0), p[2].data_ptr(), (int)p[2].size(0), p[3].data_ptr(), (int)b, (int)s,
-                                         (int)kWidth, code, s_row(0), stream),
+                                         (int)kWidth, code, at_row(rows, 0), stream),
               "tgt_graph_node_feature_fwd");
         if (c.multi_hop)
             check(tgt_graph_attn_bias_multi_hop_fwd(attn_bias.data_ptr(), in.spatial.data_ptr<int64_t>(), in.edges.data_ptr<int64_t>(), (int)in.edges.size(3),
@@ -337,29 +346,33 @@ struct GraphGraphormerFn : public torch::autograd::Function<GraphGraphormerFn> {
             check(tgt_graph_attn_bias_fwd(attn_bias.data_ptr(), in.spatial.data_ptr<int64_t>(), in.edges.data_ptr<int64_t>(), (int)in.edges.size(3), p[4].data_ptr(),
                                           (int)p[4].size(0), p[5].data_ptr(), (int)p[5].size(0), p[6].data_ptr(), (int)b, (int)s, H, code, bias.data_ptr(), stream),
                   "tgt_graph_attn_bias_fwd");
-        for (int64_t l = 0; l <= L; ++l) {
+        for (int64_t l = 0; l < L; ++l) {
             tgt_node_fwd_args a{};
-            a.rows = N; a.dtype = code;
-            a.s_in = s_row(l ? l - 1 : 0); a.s_out = s_row(l);
+            a.rows = N; a.dtype = code; a.same_bits = code == TGT_DTYPE_BF16;
+            a.s_in = at_row(rows, at.s(l ? l - 1 : 0)); a.s_out = at_row(rows, at.s(l));
             if (l > 0) {
-                a.attn = a_row(l - 1, 3);
+                a.attn = at_row(rows, at.a(l - 1, 3));
                 a.w_post = packed.weight(6 * (l - 1)); a.v_post = packed.vec(10 * (l - 1)); a.eps_post = (float)c.eps[2 * (l - 1) + 1];
             }
-            if (l < L) {
-                a.q = a_row(l, 0); a.k = a_row(l, 1); a.v = a_row(l, 2);
-                a.w_next = packed.weight(6 * l + 3); a.v_next = packed.vec(10 * l + 5); a.eps_next = (float)c.eps[2 * l];
-            }
+            a.q = at_row(rows, at.a(l, 0)); a.k = at_row(rows, at.a(l, 1)); a.v = at_row(rows, at.a(l, 2));
+            a.w_next = packed.weight(6 * l + 3); a.v_next = packed.vec(10 * l + 5); a.eps_next = (float)c.eps[2 * l];
             check(tgt_node_fwd(&a, stream), "tgt_node_fwd");
-            if (l < L)
-                check(tgt_dense_attn_dropout_fwd(a.q, a.k, a.v, bias.data_ptr(), (int)b, (int)S, H, (int)(kWidth / H), dense, (float)c.p_drop, (uint64_t)c.seeds[l], a_row(l, 3),
+            if (l + 1 < L)
+                check(tgt_dense_attn_dropout_fwd(a.q, a.k, a.v, bias.data_ptr(), (int)b, (int)S, H, d, code, (float)c.p_drop, (uint64_t)c.seeds[l], at_row(rows, at.a(l, 3)),
                                                  lse.data_ptr<float>() + (keep ? l * b * H * S : 0), stream),
                       "tgt_dense_attn_dropout_fwd");
+            else
+                check(tgt_dense_row0_fwd(a.q, a.k, a.v, bias.data_ptr(), a.s_out, (int)b, (int)S, H, d, code, (float)c.p_drop, (uint64_t)c.seeds[l], at_row(rows, at.thin(0)),
+                                         at_row(rows, at.thin(1)), thin_lse, stream),
+                      "tgt_dense_row0_fwd");
         }
-        const Tensor* head = p.data() + tables + 16 * L;
         Tensor y = at::empty({b, head[2].size(0)}, opt);
-        check(tgt_graph_head_fwd(s_row(L), head[0].data_ptr(), head[1].data_ptr(), (float)c.eps[2 * L], head[2].data_ptr(), head[3].data_ptr(), (int)b, (int)S,
-                                 (int)head[2].size(0), code, y.data_ptr(), stream),
-              "tgt_graph_head_fwd");
+        tgt_node_fwd_args a{};
+        a.rows = b; a.dtype = code; a.classes = (int)head[2].size(0); a.linear = 1; a.same_bits = code == TGT_DTYPE_BF16;
+        a.attn = at_row(rows, at.thin(0)); a.s_in = at_row(rows, at.thin(1)); a.s_out = at_row(rows, at.thin(2));
+        a.w_post = packed.weight(6 * (L - 1)); a.v_post = packed.vec(10 * (L - 1)); a.eps_post = (float)c.eps[2 * L - 1];
+        a.logp = y.data_ptr(); a.w_next = packed.weight(6 * L); a.v_next = packed.vec(10 * L); a.eps_next = (float)c.eps[2 * L];
+        check(tgt_node_fwd(&a, stream), "tgt_node_fwd");
         return y;
     }
     static Tensor forward(AutogradContext* ctx, at::TensorList P, Tensor x, Tensor in_degree, Tensor out_degree, Tensor attn_bias, Tensor spatial, Tensor edges, GraphCall c) {
@@ -370,12 +383,9 @@ struct GraphGraphormerFn : public torch::autograd::Function<GraphGraphormerFn> {
         Tensor rows, lse, bias;
         Packed packed;
         Tensor y = compute(GraphBatch{x, in_degree, out_degree, spatial, edges}, attn_bias, p, c, true, rows, lse, bias, packed);
-        const size_t head = p.size() - 4;
-        ctx->save_for_backward({x, in_degree, out_degree, spatial, edges, rows, lse, bias, packed.frags, p[0], p[1], p[2], p[4], p[5], c.multi_hop ? p[7] : Tensor(), p[head],
-                                p[head + 1], p[head + 2], p[3], p[6]});
+        ctx->save_for_backward({x, in_degree, out_degree, spatial, edges, rows, lse, bias, packed.frags, p[0], p[1], p[2], p[4], p[5], c.multi_hop ? p[7] : Tensor(), p[3], p[6]});
         ctx->saved_data["multi_hop"] = c.multi_hop;
-        ctx->saved_data["dense"] = c.bf16_products;
-        ctx->saved_data["ints"] = std::vector<int64_t>{c.max_dist, c.H, (int64_t)p.size()};
+        ctx->saved_data["ints"] = std::vector<int64_t>{c.max_dist, c.H, (int64_t)p.size(), y.size(1)};
         ctx->saved_data["p"] = c.p_drop;
         ctx->saved_data["eps"] = c.eps;
         ctx->saved_data["seeds"] = c.seeds;
@@ -384,19 +394,20 @@ struct GraphGraphormerFn : public torch::autograd::Function<GraphGraphormerFn> {
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         auto sv = ctx->get_saved_variables();
         const Tensor &x = sv[0], &ind = sv[1], &outd = sv[2], &spatial = sv[3], &edges = sv[4], &rows = sv[5], &lse = sv[6], &bias = sv[7], &atom = sv[9], &tin = sv[10],
-                     &tout = sv[11], &sp = sv[12], &et = sv[13], &hops = sv[14], &gamma = sv[15], &beta = sv[16], &Wh = sv[17], &token = sv[18], &vd = sv[19];
+                     &tout = sv[11], &sp = sv[12], &et = sv[13], &hops = sv[14], &token = sv[15], &vd = sv[16];
         const bool multi_hop = ctx->saved_data["multi_hop"].toBool();
         const auto ints = ctx->saved_data["ints"].toIntVector();
         const auto eps = ctx->saved_data["eps"].toDoubleVector();
         const auto seeds = ctx->saved_data["seeds"].toIntVector();
         const double p_drop = ctx->saved_data["p"].toDouble();
-        const int tables = kFixed + (multi_hop ? 1 : 0), H = (int)ints[1];
-        const int64_t L = (ints[2] - tables - 4) / 16, b = x.size(0), s = x.size(1), S = s + 1, N = b * S, O = Wh.size(0);
-        const int code = dtype_code(atom), dense = code == TGT_DTYPE_F32 && ctx->saved_data["dense"].toBool() ? TGT_DTYPE_F32_BF16_PRODUCTS : code;
+        const int tables = kFixed + (multi_hop ? 1 : 0), H = (int)ints[1], hd = (int)(kWidth / H);
+        const int64_t L = (ints[2] - tables - 4) / 16, b = x.size(0), s = x.size(1), S = s + 1, N = b * S, O = ints[3];
+        const int code = dtype_code(atom);
+        const Layout lay(N, b, L, true);
         c10::DeviceGuard guard(atom.device());
         void* stream = stream_of(atom);
         const auto opt = atom.options(), bytes_opt = opt.dtype(at::kByte);
-        const Packed packed(sv[8], (int)(6 * L), code);
+        const Packed packed(sv[8], (int)(6 * L + 1), code);
         std::vector<std::vector<int64_t>> shapes;
         for (const Tensor* t : {&atom, &tin, &tout, &token, &sp, &et, &vd}) shapes.push_back(t->sizes().vec());
         if (multi_hop) shapes.push_back(hops.sizes().vec());
@@ -408,53 +419,69 @@ struct GraphGraphormerFn : public torch::autograd::Function<GraphGraphormerFn> {
         shapes.push_back({O});
         FlatGrads G(shapes, opt);
         const Tensor dy = grads[0].contiguous();
-        const int workers = tgt_node_bwd_workers(N);
-        Tensor work = at::empty({6 * N, kWidth}, opt);
-        Tensor partial = at::empty({workers * 2 * L * kLayerPartial}, opt.dtype(at::kFloat));
+        const int workers = tgt_node_bwd_workers(N), thin_workers = tgt_node_bwd_workers(b);
+        Tensor work = at::empty({6 * N + 3 * b, kWidth}, opt);
+        Tensor partial = at::empty({workers * (2 * L - 1) * kLayerPartial + thin_workers * (kLayerPartial + kClassPartial) + b * H}, opt.dtype(at::kFloat));
         char *g[2] = {at_row(work, 0), at_row(work, N)}, *da = at_row(work, 2 * N), *dq = at_row(work, 3 * N), *dk = at_row(work, 4 * N), *dv = at_row(work, 5 * N);
-        float* next_partial = partial.data_ptr<float>();
+        char *thin_g = at_row(work, 6 * N), *thin_g2 = at_row(work, 6 * N + b), *thin_da = at_row(work, 6 * N + 2 * b);
+        float *dvirt = partial.data_ptr<float>(), *next_partial = dvirt + b * H;
         std::vector<tgt_node_sum> sums;
-        auto new_sum = [&]() -> tgt_node_sum& {
+        auto new_sum = [&](int n, int mats, int n_rows) -> tgt_node_sum& {
             sums.push_back(tgt_node_sum{});
-            sums.back().partial = next_partial; sums.back().workers = workers; sums.back().mats = 3; sums.back().rows = (int)kWidth;
-            next_partial += workers * kLayerPartial;
+            sums.back().partial = next_partial; sums.back().workers = n; sums.back().mats = mats; sums.back().rows = n_rows;
+            next_partial += (int64_t)n * (mats * 4096 + (mats + 2) * 64);
             return sums.back();
         };
-        const Tensor* head = G.t.data() + tables + 16 * L;
-        check(tgt_graph_head_bwd(at_row(rows, L * N), gamma.data_ptr(), beta.data_ptr(), (float)eps[2 * L], Wh.data_ptr(), dy.data_ptr(), (int)b, (int)S, (int)O, code, g[0],
-                                 head[2].data_ptr(), head[3].data_ptr(), head[0].data_ptr(), head[1].data_ptr(), stream),
-              "tgt_graph_head_bwd");
+        {      // the head, one row per graph
+            tgt_node_bwd_pre_args a{};
+            a.rows = b; a.dtype = code; a.classes = (int)O; a.linear = 1; a.eps = (float)eps[2 * L];
+            a.s = at_row(rows, lay.thin(2)); a.dlogp = dy.data_ptr(); a.w_back = packed.transposed(6 * L); a.v_next = packed.vec(10 * L);
+            a.g_out = thin_g; a.partial = next_partial;
+            tgt_node_sum& sm = new_sum(thin_workers, 1, (int)O);
+            const Tensor* head = G.t.data() + tables + 16 * L;
+            sm.out[0] = head[2].data_ptr(); sm.out[1] = head[3].data_ptr(); sm.out[2] = head[0].data_ptr(); sm.out[3] = head[1].data_ptr();
+            check(tgt_node_bwd_pre(&a, stream), "tgt_node_bwd_pre");
+        }
         // the layers share one bias: their gradients of it are added where they are folded into the tables, four at a time
         const bool side_by_side = !multi_hop && H <= 8 && edges.size(3) == 1;
         std::vector<Tensor> dbias;
         for (int64_t l = L - 1; l >= 0; --l) {
+            const bool last = l == L - 1;
             const Tensor* w = G.t.data() + tables + 16 * l;
-            const int64_t unit = N * kWidth * rows.element_size();
-            const char *q = at_row(rows, (L + 1 + 4 * l) * N), *k = q + unit, *v = k + unit, *at = v + unit;
+            const char *q = at_row(rows, lay.a(l, 0)), *k = at_row(rows, lay.a(l, 1)), *v = at_row(rows, lay.a(l, 2));
             tgt_node_bwd_post_args post{};
-            post.rows = N; post.dtype = code; post.heads = H; post.eps = (float)eps[2 * l + 1];
-            post.g_in = g[0]; post.s = at_row(rows, l * N); post.attn = at; post.w_post = packed.weight(6 * l); post.w_back = packed.transposed(6 * l);
-            post.v_post = packed.vec(10 * l); post.g_out = g[1]; post.d_attn = da; post.partial = next_partial;
+            post.rows = last ? b : N; post.dtype = code; post.same_bits = code == TGT_DTYPE_BF16; post.heads = H; post.eps = (float)eps[2 * l + 1];
+            post.g_in = last ? thin_g : g[0]; post.s = at_row(rows, last ? lay.thin(1) : lay.s(l)); post.attn = at_row(rows, last ? lay.thin(0) : lay.a(l, 3));
+            post.w_post = packed.weight(6 * l); post.w_back = packed.transposed(6 * l);
+            post.v_post = packed.vec(10 * l); post.g_out = last ? thin_g2 : g[1]; post.d_attn = last ? thin_da : da; post.partial = next_partial;
             static const int to_post[8] = {8, 12, 14, 9, 13, 15, 10, 11}, to_pre[8] = {2, 4, 6, 3, 5, 7, 0, 1};
-            tgt_node_sum& s1 = new_sum();
+            tgt_node_sum& s1 = new_sum(last ? thin_workers : workers, 3, (int)kWidth);
             for (int i = 0; i < 8; ++i) s1.out[i] = w[to_post[i]].data_ptr();
             check(tgt_node_bwd_post(&post, stream), "tgt_node_bwd_post");
-            Tensor db = at::empty_like(bias);
-            check(tgt_dense_attn_dropout_bwd(q, k, v, bias.data_ptr(), (int)b, (int)S, H, (int)(kWidth / H), dense, (float)p_drop, (uint64_t)seeds[l], at,
-                                             lse.data_ptr<float>() + l * b * H * S, da, dq, dk, dv, db.data_ptr(), stream),
-                  "tgt_dense_attn_dropout_bwd");
-            if (dbias.empty() || (side_by_side && dbias.size() < 4)) dbias.push_back(db);
-            else dbias.back().add_(db);
+            if (last)
+                check(tgt_dense_row0_bwd(q, k, v, bias.data_ptr(), (int)b, (int)S, H, hd, code, (float)p_drop, (uint64_t)seeds[l], post.attn,
+                                         lse.data_ptr<float>() + lse.numel() - b * H, thin_da, thin_g2, dq, dk, dv, g[1], dvirt, stream),
+                      "tgt_dense_row0_bwd");
+            else {
+                Tensor db = at::empty_like(bias);
+                check(tgt_dense_attn_dropout_bwd(q, k, v, bias.data_ptr(), (int)b, (int)S, H, hd, code, (float)p_drop, (uint64_t)seeds[l], post.attn,
+                                                 lse.data_ptr<float>() + l * b * H * S, da, dq, dk, dv, db.data_ptr(), stream),
+                      "tgt_dense_attn_dropout_bwd");
+                if (dbias.empty() || (side_by_side && dbias.size() < 4)) dbias.push_back(db);
+                else dbias.back().add_(db);
+            }
             tgt_node_bwd_pre_args pre{};
             pre.rows = N; pre.dtype = code; pre.eps = (float)eps[2 * l];
-            pre.dq = dq; pre.dk = dk; pre.dv = dv; pre.g_in = g[1]; pre.s = at_row(rows, l * N);
+            pre.dq = dq; pre.dk = dk; pre.dv = dv; pre.g_in = g[1]; pre.s = at_row(rows, lay.s(l));
             pre.w_back = packed.transposed(6 * l + 3); pre.v_next = packed.vec(10 * l + 5); pre.g_out = g[0]; pre.partial = next_partial;
-            tgt_node_sum& s2 = new_sum();
+            tgt_node_sum& s2 = new_sum(workers, 3, (int)kWidth);
             for (int i = 0; i < 8; ++i) s2.out[i] = w[to_pre[i]].data_ptr();
             check(tgt_node_bwd_pre(&pre, stream), "tgt_node_bwd_pre");
         }
         check(tgt_node_sums(sums.data(), (int)sums.size(), code, stream), "tgt_node_sums");
-        if (multi_hop) {
+        if (dbias.empty())
+            for (int i = 4; i < tables; ++i) G.t[i].zero_();      // one layer: only the virtual distance below
+        else if (multi_hop) {
             const int D0 = (int)edges.size(3), md = (int)ints[0], D = md > 0 && md < D0 ? md : D0;
             const int64_t bytes = tgt_graph_attn_bias_multi_hop_bwd_workspace_bytes((int)sp.size(0), (int)et.size(0), H, D);
             Tensor ws = at::empty({bytes}, bytes_opt);
@@ -471,6 +498,7 @@ struct GraphGraphormerFn : public torch::autograd::Function<GraphGraphormerFn> {
                                               (int)b, (int)s, H, code, G.t[4].data_ptr(), G.t[5].data_ptr(), G.t[6].data_ptr(), ws.data_ptr(), bytes, stream),
                   "tgt_graph_attn_bias_bwd_sum");
         }
+        check(tgt_dense_row0_virtual(dvirt, (int)b, H, code, G.t[6].data_ptr(), stream), "tgt_dense_row0_virtual");
         {
             const int64_t bytes = tgt_graph_node_feature_bwd_workspace_bytes((int)atom.size(0), (int)tin.size(0), (int)tout.size(0), (int)kWidth);
             Tensor ws = at::empty({bytes}, bytes_opt);
@@ -488,7 +516,7 @@ struct GraphGraphormerFn : public torch::autograd::Function<GraphGraphormerFn> {
 };
 
 Tensor graph_graphormer(const Tensor& x, const Tensor& in_degree, const Tensor& out_degree, const Tensor& attn_bias, const Tensor& spatial_pos, const Tensor& edge_ids,
-                        at::TensorList P, bool multi_hop, int64_t max_dist, int64_t H, at::ArrayRef<double> eps, double p_drop, at::IntArrayRef seeds, bool bf16_products) {
+                        at::TensorList P, bool multi_hop, int64_t max_dist, int64_t H, at::ArrayRef<double> eps, double p_drop, at::IntArrayRef seeds) {
     on_gpu(attn_bias, "graph_graphormer");
     const int64_t tables = GraphGraphormerFn::kFixed + (multi_hop ? 1 : 0);
     TORCH_CHECK((int64_t)P.size() >= tables + 4 && (P.size() - tables - 4) % 16 == 0, "graph_graphormer takes ", tables + 4, " + 16 L parameter tensors");
@@ -517,7 +545,7 @@ Tensor graph_graphormer(const Tensor& x, const Tensor& in_degree, const Tensor& 
                     edge_ids.dim() == (multi_hop ? 5 : 4) && edge_ids.size(0) == b && edge_ids.size(1) == s && edge_ids.size(2) == s,
                 "graph_graphormer: x [b, s, F], degrees [b, s], attn_bias [b, s + 1, s + 1], spatial_pos [b, s, s], edge ids [b, s, s, ...]");
     GraphCall c;
-    c.multi_hop = multi_hop; c.bf16_products = bf16_products; c.max_dist = max_dist; c.H = H; c.p_drop = p_drop;
+    c.multi_hop = multi_hop; c.max_dist = max_dist; c.H = H; c.p_drop = p_drop;
     c.eps.assign(eps.begin(), eps.end());
     c.seeds.assign(seeds.begin(), seeds.end());
     const auto ids = [](const Tensor& t) { return t.to(at::kLong).contiguous(); };
@@ -537,7 +565,7 @@ TORCH_LIBRARY_FRAGMENT(torchgt, m) {
     m.def("node_graphormer(Tensor x, Tensor[] params, __torch__.torch.classes.torchgt.PlanHolder plan, Tensor workspace, int heads, int tokens, "
           "float[] eps) -> Tensor");
     m.def("graph_graphormer(Tensor x, Tensor in_degree, Tensor out_degree, Tensor attn_bias, Tensor spatial_pos, Tensor edge_ids, Tensor[] params, "
-          "bool multi_hop, int max_dist, int heads, float[] eps, float p_drop, int[] seeds, bool bf16_products) -> Tensor");
+          "bool multi_hop, int max_dist, int heads, float[] eps, float p_drop, int[] seeds) -> Tensor");
 }
 TORCH_LIBRARY_IMPL(torchgt, CompositeImplicitAutograd, m) {
     m.impl("node_graphormer", node_graphormer);

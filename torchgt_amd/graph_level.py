@@ -216,7 +216,7 @@ class Graphormer(nn.Module):
             core = layer.self_attention.dist_attn.local_attn
             # (a flag set on a layer itself asks for that layer's own way of running, either one)
             if "one_operator" in layer.__dict__ or not layer.one_operator or layer.self_attention.num_heads not in (2, 4, 8) or \
-                    core.attention_dropout_rate != first.attention_dropout_rate or core.dense_bf16_products != first.dense_bf16_products:
+                    core.attention_dropout_rate != first.attention_dropout_rate or core.dense_bf16_products:
                 return None
         P = tree.parameters(self.final_ln.weight.dtype, self.training)
         if P is None or P[0].dtype not in _DT or P[0].shape[1] != 64 or P[-1].shape[0] > 64 or P[4].shape[1] != self.layers[0].self_attention.num_heads:
@@ -226,7 +226,8 @@ class Graphormer(nn.Module):
     def forward(self, batched_data, perturb=None):
         P = self._one_operator(batched_data)
         if P is not None:
-            # the whole model as one operator and one autograd node: node features, bias, layers, head
+            # the whole model as one operator and one autograd node: node features, bias, layers, head (the last layer's
+            # attention and what follows it at the virtual nodes only: no other row of it is read)
             multi_hop = self.graph_attn_bias.edge_type == "multi_hop"
             att = self.layers[0].self_attention
             core = att.dist_attn.local_attn
@@ -235,8 +236,7 @@ class Graphormer(nn.Module):
             eps = [e for layer in self.layers for e in (layer.self_attention_norm.eps, layer.ffn_norm.eps)] + [self.final_ln.eps]
             d = batched_data
             return _ext.op("graph_graphormer")(d.x, d.in_degree, d.out_degree, d.attn_bias, d.spatial_pos, d.edge_input if multi_hop else d.attn_edge_type,
-                                               P, multi_hop, int(self.graph_attn_bias.multi_hop_max_dist), att.num_heads, eps, p, seeds,
-                                               bool(core.dense_bf16_products))
+                                               P, multi_hop, int(self.graph_attn_bias.multi_hop_max_dist), att.num_heads, eps, p, seeds)
         x = self.graph_node_feature(batched_data)            # [b, s + 1, h]
         attn_bias = self.graph_attn_bias(batched_data, as_ids=self.bias_from_ids)       # [b, H, s + 1, s + 1], or its ids
         output = self.input_dropout(x)
