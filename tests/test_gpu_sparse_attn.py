@@ -459,3 +459,26 @@ def test_plan_order_needs_the_map(cuda):
     assert L.tgt_sparse_attn_fwd(plan.handle, q.data_ptr(), q.data_ptr(), q.data_ptr(), b.data_ptr(), 0x23, H, d,
                                  _lib.DTYPE_F32, q.data_ptr(), Z.data_ptr(), ws.data_ptr(), ws.numel(), None) == _lib.ERR_INVALID_ARG
     plan.close()
+
+
+@pytest.mark.parametrize("bias_kind", ["none", "edge", "edge_head"])
+def test_rows_beyond_four_gib(cuda, bias_kind):
+    """2-byte arrays of 4 GiB and more take 64-bit offsets in the walks: the same bits as the same edges among few nodes."""
+    H, d, n, N = 8, 16, 300, (1 << 24) + 1000                 # rows of 256 bytes
+    g = torch.Generator().manual_seed(5)
+    ei = torch.cat([torch.randint(0, n, (2, 3000), generator=g), torch.stack([torch.randint(0, n, (400,), generator=g), torch.zeros(400, dtype=torch.int64)])], 1)
+    q, k, v, bias, dout = make_inputs(n, ei.shape[1], H, d, torch.bfloat16, bias_kind, 6)
+    o, Z, grads = hip_fwd_bwd(q, k, v, bias, ei, dout, cuda)
+    at = torch.randint(0, N // 4096, (n,), generator=g).sort()[0] * 4096 + torch.arange(n)      # increasing: the edge order is the same
+    at[-1] = N - 1
+    at = at.to(cuda)
+
+    def spread(x):
+        big = torch.zeros(N, H, d, dtype=torch.bfloat16, device=cuda)
+        big[at] = x.to(cuda)
+        return big
+
+    ob, Zb, gb = hip_fwd_bwd(spread(q), spread(k), spread(v), bias, at[ei.to(cuda)], spread(dout), cuda)
+    assert torch.equal(ob[at], o) and torch.equal(Zb[at], Z)
+    for i, (b, s) in enumerate(zip(gb, grads)):
+        assert torch.equal(b[at] if i < 3 else b, s), i

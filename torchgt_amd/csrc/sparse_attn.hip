@@ -19,6 +19,7 @@
 #include <stdlib.h>
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 namespace tgt {
 
@@ -28,6 +29,10 @@ __device__ __forceinline__ float bf16_to_f32(uint32_t bits16) { return __uint_as
 __device__ __forceinline__ uint32_t f32_to_bf16(float f) {   // gfx950 converts in hardware (round to nearest even)
     const __bf16 b = static_cast<__bf16>(f);
     return (uint32_t)__builtin_bit_cast(uint16_t, b);
+}
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {      // one instruction for the two
+    return __builtin_bit_cast(uint32_t, bf16x2_t{static_cast<__bf16>(lo), static_cast<__bf16>(hi)});
 }
 
 __device__ __forceinline__ void load8(const float* __restrict__ p, float (&x)[8]) {
@@ -48,12 +53,7 @@ __device__ __forceinline__ void store8(float* __restrict__ p, const float (&x)[8
     *reinterpret_cast<float4*>(p + 4) = make_float4(x[4], x[5], x[6], x[7]);
 }
 __device__ __forceinline__ void store8(bf16_t* __restrict__ p, const float (&x)[8]) {
-    uint4 u;
-    u.x = f32_to_bf16(x[0]) | (f32_to_bf16(x[1]) << 16);
-    u.y = f32_to_bf16(x[2]) | (f32_to_bf16(x[3]) << 16);
-    u.z = f32_to_bf16(x[4]) | (f32_to_bf16(x[5]) << 16);
-    u.w = f32_to_bf16(x[6]) | (f32_to_bf16(x[7]) << 16);
-    *reinterpret_cast<uint4*>(p) = u;
+    *reinterpret_cast<uint4*>(p) = make_uint4(pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3]), pack_bf16(x[4], x[5]), pack_bf16(x[6], x[7]));
 }
 // A gathered row chunk as it arrives from memory.  The walk issues all gathers of a step first and
 // converts only when a value is used: a conversion placed next to its load would make the wave
@@ -80,9 +80,12 @@ __device__ __forceinline__ void zero_raw(Raw8<float>& r) {
     for (int i = 0; i < 8; ++i) r.x[i] = 0.f;
 }
 __device__ __forceinline__ void zero_raw(Raw8<bf16_t>& r) { r.u = make_uint4(0u, 0u, 0u, 0u); }
+__device__ __forceinline__ void arrive_here(const Raw8<float>& r) {
+    asm volatile("" ::"v"(r.x[0]), "v"(r.x[1]), "v"(r.x[2]), "v"(r.x[3]), "v"(r.x[4]), "v"(r.x[5]), "v"(r.x[6]), "v"(r.x[7]));
+}
+__device__ __forceinline__ void arrive_here(const Raw8<bf16_t>& r) { asm volatile("" ::"v"(r.u.x), "v"(r.u.y), "v"(r.u.z), "v"(r.u.w)); }
 // Dot product of two chunks as they arrived.  bf16 pairs go through v_dot2_f32_bf16 (exact products,
 // fp32 sum): four instructions and no conversion of either operand.
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
     return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b), c, false);
 }
@@ -149,15 +152,51 @@ __device__ __forceinline__ float dot8(const float (&a)[8], const float (&b)[8]) 
     for (int c = 1; c < 8; ++c) s = fmaf(a[c], b[c], s);
     return s;
 }
+// x of lane (l ^ OFF) for OFF < 16, as a DPP move that the add behind it takes as an operand.
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+template <int OFF>
+__device__ __forceinline__ float lane_xor(float x) {
+    static_assert(OFF == 1 || OFF == 2 || OFF == 4 || OFF == 8, "within a row of 16 lanes");
+    if constexpr (OFF == 1) return dpp<0xB1>(x);                 // quad_perm [1, 0, 3, 2]
+    else if constexpr (OFF == 2) return dpp<0x4E>(x);            // quad_perm [2, 3, 0, 1]
+    else if constexpr (OFF == 4) return dpp<0x1B>(dpp<0x141>(x));   // row_half_mirror (l ^ 7), quad_perm [3, 2, 1, 0] (l ^ 3)
+    else return dpp<0x128>(x);                                   // row_ror:8
+}
+// Lanes l of `lo` and l + OFF of `hi` (OFF 16, 32) with bit OFF of l clear, at lane l; the two others at lane l + OFF.
+template <int OFF>
+__device__ __forceinline__ void lane_swap(float& lo, float& hi) {
+    const uint32_t a = __float_as_uint(lo), b = __float_as_uint(hi);
+    if constexpr (OFF == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+        lo = __uint_as_float(r[0]); hi = __uint_as_float(r[1]);
+    } else {
+        const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+        lo = __uint_as_float(r[0]); hi = __uint_as_float(r[1]);
+    }
+}
+// x + x of lane (l ^ OFF)
+template <int OFF>
+__device__ __forceinline__ float add_xor(float x) {
+    if constexpr (OFF >= 16) {
+        float y = x;
+        lane_swap<OFF>(x, y);
+        return x + y;
+    } else return x + lane_xor<OFF>(x);
+}
+// sum over lanes that differ in the bits FROM, 2 FROM, ... below TO
+template <int FROM, int TO>
+__device__ __forceinline__ float lanes_sum(float x) {
+    if constexpr (FROM < TO) return lanes_sum<2 * FROM, TO>(add_xor<FROM>(x));
+    else return x;
+}
 // sum over the LPH lanes that share a head (adjacent lanes)
 template <int LPH>
-__device__ __forceinline__ float head_sum(float x) {
-#pragma unroll
-    for (int off = 1; off < LPH; off <<= 1) x += __shfl_xor(x, off);
-    return x;
-}
-// clamp that keeps NaN (like torch.clamp)
-__device__ __forceinline__ float clamp5(float x) { return x < -5.0f ? -5.0f : (x > 5.0f ? 5.0f : x); }
+__device__ __forceinline__ float head_sum(float x) { return lanes_sum<1, LPH>(x); }
+// clamp that keeps NaN (like torch.clamp): one v_maximum3 and one v_minimum3
+__device__ __forceinline__ float clamp5(float x) { return __builtin_elementwise_minimum(__builtin_elementwise_maximum(x, -5.0f), 5.0f); }
 
 constexpr float kEps = 1e-6f;   // attn_module.py:187
 constexpr int kUnroll = 4;      // edges in flight per slot
@@ -174,8 +213,8 @@ struct Common {
     const void* bias;
     const void* bias_src; // the bias as the walk by source reads it (same array, or its source-sorted copy)
     const float2* nd;     // [N, H] (1/(Z+eps), D) (backward)
-    int32_t bias_mode;
     int32_t bias_se, bias_sh;   // element strides of the bias per edge / per head: (H, 1) or (1, 0)
+    int32_t narrow;       // every array is below 4 GiB: 32-bit offsets
     float inv_scale;
 };
 
@@ -214,6 +253,32 @@ __host__ __device__ constexpr int part_stride() {
     return MODE == MODE_FWD ? HD + H : (MODE == MODE_BWD_DST ? HD : 2 * HD);
 }
 
+constexpr int ilog2(int n) { return n <= 1 ? 0 : 1 + ilog2(n / 2); }
+// Element i * stride + k of an array (stride a power of two, k below it).  An unsigned 32-bit byte offset (O) is an operand of the load itself
+// (scalar base, vector offset); a 64-bit one takes three to six instructions for every gathered row.
+template <typename T, typename O>
+__device__ __forceinline__ T* at(const void* base, const int i, const int stride, const int k) {
+    T* b = static_cast<T*>(const_cast<void*>(base));
+    if constexpr (std::is_unsigned<O>::value) return reinterpret_cast<T*>(reinterpret_cast<char*>(b) + ((O)(uint32_t)i * (O)(stride * sizeof(T)) | (O)(k * sizeof(T))));
+    else return b + ((O)i * stride + k);
+}
+// f(offset type): 32 bits where every array is below 4 GiB and the elements have 2 bytes.  Those walks spend most of
+// their time issuing vector instructions (262 K nodes, 5 M edges, H d = 64: 118 -> 105 us forward, 339 -> 309 us
+// backward, with the lane exchanges below as DPP operands and swaps); those of 4-byte elements wait for memory, and
+// their backward has no registers for a second form of the addresses.  The two asm statements keep the compiler from
+// merging the two copies of f into one that works with 64-bit addresses.
+template <typename T, typename F>
+__device__ __forceinline__ void with_offsets(const bool narrow, const F& f) {
+    if constexpr (sizeof(T) == 4) f(int64_t(0));
+    else if (narrow) {
+        f(uint32_t(0));
+        asm volatile("; 32-bit offsets");
+    } else {
+        f(uint64_t(0));
+        asm volatile("; 64-bit offsets");
+    }
+}
+
 // What a lane group keeps of its own row while it walks the row's edges.
 template <typename T>
 struct RowRegs {
@@ -226,103 +291,103 @@ __device__ __forceinline__ void load_row(const Common& c, const int row, const i
                                          RowRegs<T>& rr, Acc& acc) {
     constexpr int H = LPE / LPH;
     constexpr int HD = LPE * 8;
-    const T* __restrict__ Q = static_cast<const T*>(c.q);
-    const T* __restrict__ K = static_cast<const T*>(c.k);
-    const T* __restrict__ V = static_cast<const T*>(c.v);
-    const T* __restrict__ Gd = static_cast<const T*>(c.g);
-    const int64_t row_off = (int64_t)row * HD + el * 8;
     rr.rz = 0.f; rr.Dh = 0.f;
     zero_raw(rr.r0); zero_raw(rr.r1);
 #pragma unroll
     for (int i = 0; i < 8; ++i) { acc.a0[i] = 0.f; acc.a1[i] = 0.f; }
     acc.z = 0.f;
     if (valid) {
-        if (MODE == MODE_FWD) {
-            load_raw(Q + row_off, rr.r0);
-        } else if (MODE == MODE_BWD_DST) {
-            load_raw(Q + row_off, rr.r0);
-            load_raw(Gd + row_off, rr.r1);
-            const float2 nd = c.nd[(int64_t)row * H + el / LPH];
-            rr.rz = nd.x; rr.Dh = nd.y;
-        } else {
-            load_raw(K + row_off, rr.r0);
-            load_raw(V + row_off, rr.r1);
-        }
+        with_offsets<T>(c.narrow, [&](auto zero) {
+            using O = decltype(zero);
+            load_raw(at<T, O>(MODE == MODE_BWD_SRC ? c.k : c.q, row, HD, el * 8), rr.r0);
+            if (MODE == MODE_BWD_DST) load_raw(at<T, O>(c.g, row, HD, el * 8), rr.r1);
+            if (MODE == MODE_BWD_SRC) load_raw(at<T, O>(c.v, row, HD, el * 8), rr.r1);
+            if (MODE == MODE_BWD_DST) {
+                const float2 nd = *at<float2, O>(c.nd, row, H, el / LPH);
+                rr.rz = nd.x; rr.Dh = nd.y;
+            }
+        });
     }
 }
 
+// Whether the lanes of a missing edge load nothing.  Without lane-dependent branches around them the gathers of a step go out
+// back to back and are waited for one edge at a time; the walks with four gathered float rows per lane and step and two rows of
+// their own do not have the registers for it (64 K nodes, 0.53 M edges, float32: forward 35.9 -> 35.4 us, 4 K nodes 13.1 -> 11.9 us,
+// but the backward 79 -> 88 us).
+template <typename T, int MODE> constexpr bool masked_gathers() { return sizeof(T) == 4 && MODE != MODE_FWD; }
+
 // kUnroll edges of one slot: nb[u] = the other endpoint, ed[u] = the row of the bias / dbias arrays, ok[u] =
-// whether the edge exists.  All gathers of the step are issued before anything is used.  For 4-byte
-// elements the lanes of a missing edge load nothing; for 2-byte elements every lane loads (a missing edge
-// must then name a valid node and bias row - callers repeat the row's last edge - and only the
-// arithmetic is skipped): with no lane-dependent branch around them the loads go out back to back, and
-// the rows stay packed until they are used.
+// whether the edge exists.  All gathers of the step are issued before anything is used.  Unless the gathers are
+// masked, every lane loads: a missing edge must then name a valid node and bias row - callers repeat the row's
+// last edge - and only the arithmetic is skipped.
 template <typename T, int LPE, int LPH, int MODE, int HASB>
 __device__ __forceinline__ void edge_step(const Common& c, const SideArgs& s, const RowRegs<T>& rr,
                                           const int (&nb)[kUnroll], const int (&ed)[kUnroll],
                                           const bool (&ok)[kUnroll], const int el, Acc& acc) {
     constexpr int H = LPE / LPH;
     constexpr int HD = LPE * 8;
+    constexpr bool MASKED = masked_gathers<T, MODE>();
     const int head = el / LPH;
-    const T* __restrict__ Q = static_cast<const T*>(c.q);
-    const T* __restrict__ K = static_cast<const T*>(c.k);
-    const T* __restrict__ V = static_cast<const T*>(c.v);
-    const T* __restrict__ Gd = static_cast<const T*>(c.g);
-    const T* __restrict__ B = static_cast<const T*>(MODE == MODE_BWD_SRC ? c.bias_src : c.bias);
-    const int bias_se = c.bias_se, bias_sh = c.bias_sh;
     const float inv_scale = c.inv_scale;
+    const int bias_se = c.bias_se, bias_sh = c.bias_sh;
+    const int bias_shift = ilog2(sizeof(T)) + (bias_sh != 0 ? ilog2(H) : 0);      // log2 of the bytes of a bias row
+    const uint32_t bias_el = head * bias_sh * sizeof(T);
     Raw8<T> g0[kUnroll], g1[kUnroll];          // gathered rows, unconverted
-    decltype(raw1(B)) braw[kUnroll];
+    decltype(raw1((const T*)nullptr)) braw[kUnroll];
     float2 ndv[kUnroll];
-    if constexpr (sizeof(T) == 4) {
+    if constexpr (MASKED) {
         // The edge ids are waited for here, on every path.  Otherwise the wait sits inside the first lane-masked
         // block below, and behind that block the compiler must assume the ids may still be in flight: it then
         // waits for everything outstanding - the first edge's rows - before it asks for the second edge's.
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) asm volatile("" ::"v"(nb[u]), "v"(ed[u]));
     }
+    if (MASKED) {
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-        braw[u] = 0;
-        ndv[u] = make_float2(0.f, 0.f);
-        if constexpr (sizeof(T) == 4) { zero_raw(g0[u]); zero_raw(g1[u]); }
-        if (sizeof(T) != 4 || ok[u]) {
-            const int64_t o = (int64_t)nb[u] * HD + el * 8;
-            if (MODE == MODE_BWD_SRC) {
-                load_raw(Q + o, g0[u]);
-                load_raw(Gd + o, g1[u]);
-                ndv[u] = c.nd[(int64_t)nb[u] * H + head];
-            } else {
-                load_raw(K + o, g0[u]);
-                load_raw(V + o, g1[u]);
-            }
-            if (HASB) braw[u] = raw1(B + (int64_t)ed[u] * bias_se + head * bias_sh);
+        for (int u = 0; u < kUnroll; ++u) {
+            braw[u] = 0;
+            ndv[u] = make_float2(0.f, 0.f);
+            zero_raw(g0[u]);
+            zero_raw(g1[u]);
         }
     }
+    with_offsets<T>(c.narrow, [&](auto zero) {
+        using O = decltype(zero);
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            if (!MASKED || ok[u]) {
+                load_raw(at<T, O>(MODE == MODE_BWD_SRC ? c.q : c.k, nb[u], HD, el * 8), g0[u]);
+                load_raw(at<T, O>(MODE == MODE_BWD_SRC ? c.g : c.v, nb[u], HD, el * 8), g1[u]);
+                if (MODE == MODE_BWD_SRC) ndv[u] = *at<float2, O>(c.nd, nb[u], H, head);
+                if (HASB) {
+                    const void* const bias = MODE == MODE_BWD_SRC ? c.bias_src : c.bias;
+                    if (std::is_unsigned<O>::value) braw[u] = raw1(reinterpret_cast<const T*>(static_cast<const char*>(bias) + (((O)(uint32_t)ed[u] << bias_shift) + bias_el)));
+                    else braw[u] = raw1(at<T, O>(bias, ed[u], bias_se, head * bias_sh));
+                }
+            }
+        }
+    });
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
-        if constexpr (sizeof(T) == 2) {
-            // The edge's rows are named here, outside the lane-masked block that uses them: the compiler otherwise
-            // moves their loads into that block (its only user), where they are asked for and waited for one edge
-            // at a time instead of with the other gathers of the step.
-            asm volatile("" ::"v"(g0[u].u.x), "v"(g0[u].u.y), "v"(g0[u].u.z), "v"(g0[u].u.w), "v"(g1[u].u.x), "v"(g1[u].u.y),
-                         "v"(g1[u].u.z), "v"(g1[u].u.w));
-        }
+        // The edge's rows are named here, outside the lane-masked block that uses them: the compiler otherwise
+        // moves their loads into that block (its only user), where they are asked for and waited for one edge
+        // at a time instead of with the other gathers of the step.
+        if (!MASKED) { arrive_here(g0[u]); arrive_here(g1[u]); }
         if (ok[u]) {
             float x0[8], x1[8];
             unpack(g0[u], x0);
             unpack(g1[u], x1);
-            const float bbu = HASB ? cvt1(braw[u]) : 0.f;
             // raw score: identical arithmetic in all three walks so that the
             // recomputed weights and the clamp mask agree bit for bit
             const float raw = head_sum<LPH>(dot_raw(rr.r0, g0[u])) * inv_scale;
-            const float w = __expf(clamp5(raw) + bbu);
+            const float cl = clamp5(raw);
+            const float w = __expf(HASB ? cl + cvt1(braw[u]) : cl);
             if (MODE == MODE_FWD) {
                 acc.z += w;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) acc.a0[i] = fmaf(w, x1[i], acc.a0[i]);
             } else {
-                const bool inside = (raw >= -5.0f) & (raw <= 5.0f);   // torch clamp backward: inclusive
+                const bool inside = cl == raw;   // torch clamp backward: inclusive (and not for NaN)
                 if (MODE == MODE_BWD_DST) {
                     const float t = head_sum<LPH>(dot_raw(rr.r1, g1[u]));   // g_dst . v_src
                     const float dS = w * rr.rz * (t - rr.Dh);
@@ -331,9 +396,7 @@ __device__ __forceinline__ void edge_step(const Common& c, const SideArgs& s, co
                         if (bias_sh != 0) {       // one value per edge and head
                             if (el % LPH == 0) store1(dB + (int64_t)ed[u] * H + head, dS);
                         } else {                  // one value per edge: sum over heads
-                            float t2 = dS;   // sum over heads; every head is held by LPH lanes
-#pragma unroll
-                            for (int off = 1; off < LPE; off <<= 1) t2 += __shfl_xor(t2, off);
+                            const float t2 = lanes_sum<1, LPE>(dS);   // every head is held by LPH lanes
                             if (el == 0) store1(dB + ed[u], t2 * (1.0f / LPH));
                         }
                     }
@@ -360,26 +423,11 @@ __device__ __forceinline__ void edge_step(const Common& c, const SideArgs& s, co
 template <int LPE, int S, int MODE>
 __device__ __forceinline__ void add_slots(Acc& acc) {
     constexpr int G = LPE * S;
+    if (MODE == MODE_FWD) acc.z = lanes_sum<LPE, G>(acc.z);
 #pragma unroll
-    for (int off = LPE; off < G; off <<= 1) {
-        if (MODE == MODE_FWD) acc.z += __shfl_xor(acc.z, off);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            acc.a0[i] += __shfl_xor(acc.a0[i], off);
-            if (MODE == MODE_BWD_SRC) acc.a1[i] += __shfl_xor(acc.a1[i], off);
-        }
-    }
-}
-
-// x of lane (l ^ OFF).  The exchange between the two halves of a row of 16 lanes is a DPP operand of the
-// add that uses it, the others go through the LDS crossbar.
-template <int OFF>
-__device__ __forceinline__ float lane_xor(float x) {
-    if constexpr (OFF == 8) {
-        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x128 /* row_ror:8 */,
-                                                                     0xf, 0xf, false));
-    } else {
-        return __shfl_xor(x, OFF);
+    for (int i = 0; i < 8; ++i) {
+        acc.a0[i] = lanes_sum<LPE, G>(acc.a0[i]);
+        if (MODE == MODE_BWD_SRC) acc.a1[i] = lanes_sum<LPE, G>(acc.a1[i]);
     }
 }
 
@@ -387,9 +435,12 @@ __device__ __forceinline__ float lane_xor(float x) {
 // the lower (bit OFF of the lane clear) or upper (set) half of them.
 template <int N, int OFF>
 __device__ __forceinline__ void halve(float (&a)[8], const bool upper) {
-    if constexpr (N >= 1) {
 #pragma unroll
-        for (int i = 0; i < N; ++i) {
+    for (int i = 0; i < N; ++i) {
+        if constexpr (OFF >= 16) {
+            lane_swap<OFF>(a[i], a[i + N]);
+            a[i] += a[i + N];
+        } else {
             const float keep = upper ? a[i + N] : a[i];
             const float send = upper ? a[i] : a[i + N];
             a[i] = keep + lane_xor<OFF>(send);
@@ -420,10 +471,8 @@ __device__ __forceinline__ void store_n(float* __restrict__ p, const float (&x)[
 template <int CNT>
 __device__ __forceinline__ void store_n(bf16_t* __restrict__ p, const float (&x)[8]) {
     if constexpr (CNT == 1) p->x = (uint16_t)f32_to_bf16(x[0]);
-    else if constexpr (CNT == 2) *reinterpret_cast<uint32_t*>(p) = f32_to_bf16(x[0]) | (f32_to_bf16(x[1]) << 16);
-    else if constexpr (CNT == 4)
-        *reinterpret_cast<uint2*>(p) = make_uint2(f32_to_bf16(x[0]) | (f32_to_bf16(x[1]) << 16),
-                                                  f32_to_bf16(x[2]) | (f32_to_bf16(x[3]) << 16));
+    else if constexpr (CNT == 2) *reinterpret_cast<uint32_t*>(p) = pack_bf16(x[0], x[1]);
+    else if constexpr (CNT == 4) *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3]));
     else store8(p, x);
 }
 template <int CNT>
@@ -443,29 +492,23 @@ __device__ __forceinline__ void finish_row(const Common& c, const SideArgs& s, c
     constexpr int CNT = 8 / SR;
     if constexpr (S > SR) {               // more slots than elements: the upper slot bits are plain sums
 #pragma unroll
-        for (int off = LPE * SR; off < LPE * S; off <<= 1) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                acc.a0[i] += __shfl_xor(acc.a0[i], off);
-                if (MODE == MODE_BWD_SRC) acc.a1[i] += __shfl_xor(acc.a1[i], off);
-            }
+        for (int i = 0; i < 8; ++i) {
+            acc.a0[i] = lanes_sum<LPE * SR, LPE * S>(acc.a0[i]);
+            if (MODE == MODE_BWD_SRC) acc.a1[i] = lanes_sum<LPE * SR, LPE * S>(acc.a1[i]);
         }
     }
     const int sl = slot % SR;
     reduce_slots<LPE, SR>(acc.a0, sl);
     if (MODE == MODE_BWD_SRC) reduce_slots<LPE, SR>(acc.a1, sl);
-    if (MODE == MODE_FWD) {
-#pragma unroll
-        for (int off = LPE; off < LPE * S; off <<= 1) acc.z += __shfl_xor(acc.z, off);
-    }
+    if (MODE == MODE_FWD) acc.z = lanes_sum<LPE, LPE * S>(acc.z);
     if (!valid || slot >= SR) return;
-    const int64_t off = (int64_t)row * HD + el * 8 + sl * CNT;
     if (MODE != MODE_FWD) {
 #pragma unroll
         for (int i = 0; i < CNT; ++i) acc.a0[i] *= c.inv_scale;
     }
     if (TILES) {   // sums of the dense tiles of the block path for this row, if it has any
         if (s.cover[row] != 0) {
+            const int64_t off = (int64_t)row * HD + el * 8 + sl * CNT;
             add_n<CNT>(s.init0 + off, acc.a0);
             if (MODE == MODE_FWD) acc.z += s.initZ[(int64_t)row * H + el / LPH];
             if (MODE == MODE_BWD_SRC) add_n<CNT>(s.init1 + off, acc.a1);
@@ -475,10 +518,13 @@ __device__ __forceinline__ void finish_row(const Common& c, const SideArgs& s, c
         const float inv = 1.0f / (acc.z + kEps);
 #pragma unroll
         for (int i = 0; i < CNT; ++i) acc.a0[i] *= inv;
-        if (sl == 0 && el % LPH == 0) s.Z[(int64_t)row * H + el / LPH] = acc.z;
     }
-    store_n<CNT>(static_cast<T*>(s.out0) + off, acc.a0);
-    if (MODE == MODE_BWD_SRC) store_n<CNT>(static_cast<T*>(s.out1) + off, acc.a1);
+    with_offsets<T>(c.narrow, [&](auto zero) {
+        using O = decltype(zero);
+        if (MODE == MODE_FWD && sl == 0 && el % LPH == 0) *at<float, O>(s.Z, row, H, el / LPH) = acc.z;
+        store_n<CNT>(at<T, O>(s.out0, row, HD, el * 8 + sl * CNT), acc.a0);
+        if (MODE == MODE_BWD_SRC) store_n<CNT>(at<T, O>(s.out1, row, HD, el * 8 + sl * CNT), acc.a1);
+    });
 }
 
 // Walks `len` edges starting at sorted position `start` of node `row` with S edge
@@ -500,7 +546,7 @@ __device__ __forceinline__ void walk_range(const Common& c, const SideArgs& s, c
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) {
             const int e = e0 + u * S;
-            if constexpr (sizeof(T) == 4) {
+            if constexpr (masked_gathers<T, MODE>()) {
                 nb[u] = 0; ed[u] = 0;
                 if (e < n) {
                     nb[u] = col[e];
@@ -1010,14 +1056,21 @@ struct Call {
     bool no_alloc;         // fail instead of building the launch descriptors of a shape seen for the first time
 };
 
+// Rows, node sides (8 bytes per node and head), sorted edge lists and bias rows all below 4 GiB
+template <typename T>
+static bool narrow_offsets(const Call& c) {
+    const int64_t row = std::max<int64_t>((int64_t)c.H * c.d * sizeof(T), 8 * c.H), edge = std::max<int64_t>(4, (int64_t)c.H * sizeof(T));
+    return c.plan->N * row < (1ll << 32) && c.plan->E * edge < (1ll << 32);
+}
+
 template <typename T, int LPE, int LPH>
 static int run_fwd(const Call& c) {
     const WsLayout L = ws_layout(c.plan, c.H, c.d);
     Common cm{};
     cm.q = c.q; cm.k = c.k; cm.v = c.v; cm.g = nullptr; cm.bias = c.bias; cm.bias_src = c.bias; cm.nd = nullptr;
-    cm.bias_mode = c.bias_mode;
     cm.bias_se = (c.bias_mode & 0xf) == TGT_BIAS_EDGE_HEAD ? c.H : 1;
     cm.bias_sh = (c.bias_mode & 0xf) == TGT_BIAS_EDGE_HEAD ? 1 : 0;
+    cm.narrow = narrow_offsets<T>(c);
     cm.inv_scale = 1.0f / sqrtf((float)c.d);
     SideArgs a{};
     fill_side(a, c.plan->dst);
@@ -1084,9 +1137,9 @@ static int run_bwd(const Call& c) {
     cm.bias_src = both_orders ? static_cast<const char*>(c.bias) +
                                     (size_t)c.plan->E * ((c.bias_mode & 0xf) == TGT_BIAS_EDGE_HEAD ? c.H : 1) * sizeof(T)
                               : c.bias;
-    cm.bias_mode = c.bias_mode;
     cm.bias_se = (c.bias_mode & 0xf) == TGT_BIAS_EDGE_HEAD ? c.H : 1;
     cm.bias_sh = (c.bias_mode & 0xf) == TGT_BIAS_EDGE_HEAD ? 1 : 0;
+    cm.narrow = narrow_offsets<T>(c);
     cm.inv_scale = 1.0f / sqrtf((float)c.d);
     int32_t* counters = reinterpret_cast<int32_t*>(c.ws + L.counters);
     SideArgs sd{}, ss{};
