@@ -8,7 +8,7 @@ import types
 import pytest
 import torch
 
-from torchgt_amd import GraphLevelGraphormer, Graphormer, GraphPlan
+from torchgt_amd import GT, GraphLevelGraphormer, Graphormer, GraphPlan
 from torchgt_amd.graph_prep import fix_edge_index
 
 pytestmark = pytest.mark.gpu
@@ -117,3 +117,32 @@ def test_graph_graphormer_as_one_operator(cuda, dtype, b, s, outputs, heads, lay
         floor = worst * (1.0 if k.endswith("linear_k.bias") else 1e-2)
         err = float((g1[k].float() - g0[k].float()).abs().max()) / max(float(g0[k].float().abs().max()), floor)
         assert err <= tol, f"{k}: {err}"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("kind,n,features,classes,heads,hidden,ffn,layers", [("gt", 1, 32, 3, 8, 64, 64, 1), ("gt", 999, 100, 47, 8, 64, 64, 3), ("gt", 3000, 51, 40, 8, 128, 128, 2),
+                                                                          ("graphormer", 1, 32, 3, 8, 128, 128, 1), ("graphormer", 999, 100, 47, 8, 128, 128, 3),
+                                                                          ("graphormer", 777, 64, 65, 4, 64, 64, 2), ("graphormer", 500, 51, 40, 4, 64, 96, 2)])
+def test_other_widths_as_one_operator(cuda, dtype, kind, n, features, classes, heads, hidden, ffn, layers):
+    """The models the fused kernels do not have: the same kernels in the same order as step by step, so the same bits."""
+    print(f"layered case: {kind} n={n} features={features} classes={classes} heads={heads} hidden={hidden} ffn={ffn} {dtype}", flush=True)
+    torch.manual_seed(n)
+    cls, tokens = (GT, 0) if kind == "gt" else (Graphormer, 1)
+    model = scaled(cls(layers, heads, features, hidden, classes, 1, 0.0, 0.0, 0.0, ffn, tokens), n + 1, dtype, cuda)
+    x = torch.randn(n, features).to(cuda, dtype)
+    plan = GraphPlan(random_edges(n, tokens, n + 2, cuda), n + tokens)
+    w = torch.randn(n, classes, generator=torch.Generator().manual_seed(3)).to(cuda)
+    got = []
+    for one in (True, False):
+        model.one_operator = one
+        model.zero_grad(set_to_none=True)
+        xr = x.clone().requires_grad_(True)
+        out = model(xr, None, plan, attn_type="sparse")
+        assert (type(out.grad_fn).__name__ == "LogSoftmaxBackward0") != one
+        (out.float() * w).sum().backward()
+        got.append([out.detach(), xr.grad] + [p.grad for p in model.parameters() if p.grad is not None])
+        with torch.no_grad():
+            assert torch.equal(model(x, None, plan, attn_type="sparse"), out)
+    assert len(got[0]) == len(got[1])
+    for i, (a, b) in enumerate(zip(*got)):
+        assert torch.equal(a, b), (i, float((a.float() - b.float()).abs().max()))

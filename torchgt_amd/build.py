@@ -14,7 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(CSRC, "build")
 LIB_PATH = os.path.join(HERE, "libtorchgt_hip.so")
-EXT_SRCS = [os.path.join(CSRC, f) for f in ("torch_binding.cpp", "torch_models.cpp")]
+EXT_SRCS = [os.path.join(CSRC, f) for f in ("torch_binding.cpp", "torch_models.cpp", "torch_layered.cpp")]
 EXT_PATH = os.path.join(HERE, "_torchgt_ext.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -49,4 +49,34 @@ inline void rows_match_plan(const c10::intrusive_ptr<PlanHolder>& holder, int64_
     TORCH_CHECK(info[0] == N, op, ": ", N, " rows, but the plan was built for ", info[0], " nodes");
 }
 
+// A tensor of the given sizes on `base`'s memory from element `offset` (no dispatch, no autograd view: base is a plain
+// buffer made here)
+inline Tensor part_of(const Tensor& base, int64_t offset, at::IntArrayRef sizes) {
+    auto impl = c10::make_intrusive<c10::TensorImpl>(c10::Storage(base.storage()), base.unsafeGetTensorImpl()->key_set(), base.dtype());
+    impl->set_storage_offset(base.storage_offset() + offset);
+    impl->set_sizes_contiguous(sizes);
+    return Tensor(std::move(impl));
+}
+inline int64_t rounded(int64_t n) { return (n + 15) / 16 * 16; }      // parameter gradients start on their own 16 elements
+
+
+// gradient buffers of a list of shapes in one allocation
+struct FlatGrads {
+    Tensor flat;
+    std::vector<Tensor> t;
+    FlatGrads(const std::vector<std::vector<int64_t>>& shapes, const at::TensorOptions& opt) {
+        int64_t total = 0;
+        std::vector<int64_t> off;
+        for (const auto& s : shapes) {
+            off.push_back(total);
+            int64_t n = 1;
+            for (int64_t d : s) n *= d;
+            total += rounded(n);
+        }
+        flat = at::empty({total}, opt);
+        t.reserve(shapes.size());
+        for (size_t i = 0; i < shapes.size(); ++i) t.push_back(part_of(flat, off[i], shapes[i]));
+    }
+};
+
 }  // namespace tgt_torch

@@ -15,36 +15,7 @@ using namespace tgt_torch;
 
 constexpr int64_t kWidth = 64;
 
-// A tensor of the given sizes on `base`'s memory from element `offset` (no dispatch, no autograd view: base is a plain
-// buffer made here)
-Tensor part_of(const Tensor& base, int64_t offset, at::IntArrayRef sizes) {
-    auto impl = c10::make_intrusive<c10::TensorImpl>(c10::Storage(base.storage()), base.unsafeGetTensorImpl()->key_set(), base.dtype());
-    impl->set_storage_offset(base.storage_offset() + offset);
-    impl->set_sizes_contiguous(sizes);
-    return Tensor(std::move(impl));
-}
 char* at_row(const Tensor& buf, int64_t row) { return static_cast<char*>(buf.data_ptr()) + row * kWidth * buf.element_size(); }
-int64_t rounded(int64_t n) { return (n + 15) / 16 * 16; }      // parameter gradients start on their own 16 elements
-
-// gradient buffers of a list of shapes in one allocation
-struct FlatGrads {
-    Tensor flat;
-    std::vector<Tensor> t;
-    FlatGrads(const std::vector<std::vector<int64_t>>& shapes, const at::TensorOptions& opt) {
-        int64_t total = 0;
-        std::vector<int64_t> off;
-        for (const auto& s : shapes) {
-            off.push_back(total);
-            int64_t n = 1;
-            for (int64_t d : s) n *= d;
-            total += rounded(n);
-        }
-        flat = at::empty({total}, opt);
-        t.reserve(shapes.size());
-        for (size_t i = 0; i < shapes.size(); ++i) t.push_back(part_of(flat, off[i], shapes[i]));
-    }
-};
-
 // Packed parameters of the layers: fragments of six weights per layer (Wo, W1, W2, Wq, Wk, Wv), then the classes'; vectors
 // per layer (bo, gamma2, beta2, b1, b2; gamma1, beta1, bq, bk, bv), then (gamma, beta, bh) of the classes.
 // Order of a layer's parameters: gamma1, beta1, Wq, bq, Wk, bk, Wv, bv, Wo, bo, gamma2, beta2, W1, b1, W2, b2.

@@ -54,8 +54,8 @@ class ModuleTree:
     attribute look-ups of seventy parameters through ``nn.Module`` would be a third of it.  Remembers the dictionaries of the
     modules, not the parameters, and notices when a module of the tree was exchanged (``current``)."""
 
-    def __init__(self, root, names, dropouts, layers_at):
-        self.links, self.slots, self.layers_at = [], [], layers_at
+    def __init__(self, root, names, dropouts):
+        self.links, self.slots = [], []
         seen = set()
 
         def step(module, name):
@@ -78,7 +78,6 @@ class ModuleTree:
         self.count = len(root.layers)
         self.layers = root.layers._modules
         self.dropouts = [m for n, m in root.named_modules() if n.rsplit(".", 1)[-1] in dropouts]
-        self.shapes = None
 
     def current(self):
         if self.missing or len(self.layers) != self.count:
@@ -89,7 +88,7 @@ class ModuleTree:
         return True
 
     def parameters(self, dtype, training):
-        """The parameters in order, or None: one is absent, has another dtype, a layer is not square, or dropout is at work."""
+        """The parameters in order, or None: one is absent or has another dtype, or dropout is at work."""
         if self.missing or self.count == 0:
             return None
         if training:
@@ -100,13 +99,36 @@ class ModuleTree:
         for p in P:
             if p is None or p.dtype is not dtype:
                 return None
-        for p in P[self.layers_at:-4]:      # the layers' parameters (the last four are the final norm and the head): 64 wide throughout
-            if p.shape[0] != 64 or p.shape[-1] != 64:
-                return None
         return P
+
+    def by_layer(self):
+        """Whether no layer was asked to run step by step."""
+        for layer in self.layers.values():
+            if "one_operator" in layer.__dict__ or not layer.one_operator or not layer.self_attention.one_operator:
+                return False
+        return True
 
 
 _TREES = weakref.WeakKeyDictionary()      # model -> ModuleTree (which holds the model's modules, not the model)
+
+
+def model_parameters(model, dtype):
+    """Parameters of a model in the order of its whole-model operators, or None where they do not cover its state."""
+    tree = _TREES.get(model)
+    if tree is None or not tree.current():
+        tree = _TREES[model] = ModuleTree(model, model._parameter_names(), model.dropouts)
+    return tree.parameters(dtype, model.training) if tree.by_layer() else None
+
+
+def padded(P, x, at, last):
+    """Zero-pads what the linears read in 16-byte pieces: the features of x and of P[at], the classes of P[last] and P[last + 1]."""
+    ve = 4 if x.dtype == torch.float32 else 8
+    pad, out = (-x.shape[1]) % ve, (-P[last].shape[0]) % ve
+    if pad:
+        x, P[at] = F.pad(x, (0, pad)), F.pad(P[at], (0, pad))
+    if out:
+        P[last], P[last + 1] = F.pad(P[last], (0, 0, 0, out)), F.pad(P[last + 1], (0, out))
+    return x.contiguous()
 
 
 class FeedForwardNetwork(nn.Module):
@@ -206,18 +228,21 @@ class Graphormer(nn.Module):
 
     one_operator = True      # False: always run the model layer by layer
 
+    dropouts = ("self_attention_dropout", "ffn_dropout", "input_dropout")
+
     def _one_operator(self, x, attn_bias, edge_index, perturb, attn_type):
-        """The model's parameters in the operator's order when ``torch.ops.torchgt.node_graphormer`` covers this call - sparse
-        attention without a bias, hidden and feed-forward width 64, at most 64 classes, no dropout at work, every linear with
-        its bias, one dtype - else None."""
+        """The model's parameters in the order of the whole-model operators when one of them covers this call - sparse
+        attention without a bias, no dropout at work, every linear with its bias, one dtype - else None."""
         if not self.one_operator or attn_type != "sparse" or attn_bias is not None or perturb is not None or edge_index is None:
             return None
-        if self.hidden_dim != 64 or self.num_heads not in (2, 4, 8) or x.dim() != 2 or not x.is_cuda or x.dtype not in _DT:
+        if x.dim() != 2 or not x.is_cuda or x.dtype not in _DT:
             return None
-        tree = _TREES.get(self)
-        if tree is None or not tree.current():
-            tree = _TREES[self] = ModuleTree(self, self._parameter_names(), ["self_attention_dropout", "ffn_dropout", "input_dropout"], 3)
-        return tree.parameters(x.dtype, self.training)
+        return model_parameters(self, x.dtype)
+
+    @staticmethod
+    def _fused(P, heads):
+        """Whether the fused per-node kernels have this model: 64 wide throughout, at most 64 classes."""
+        return heads in (2, 4, 8) and P[-1].shape[0] <= 64 and all(p.shape[0] == 64 and p.shape[-1] == 64 for p in P[3:-4])
 
     def _parameter_names(self):
         names = ["node_encoder.weight", "node_encoder.bias", "graph_token.weight"]
@@ -227,19 +252,21 @@ class Graphormer(nn.Module):
 
     def forward(self, x, attn_bias, edge_index, perturb=None, attn_type=None):
         P = self._one_operator(x, attn_bias, edge_index, perturb, attn_type)
-        if P is not None and P[-1].shape[0] <= 64 and all(
-                "one_operator" not in layer.__dict__ and layer.one_operator and layer.self_attention.one_operator for layer in self.layers):
-            # the whole model as one operator and one autograd node over kernels that take a layer's node-local part
-            # in one pass each way
+        if P is not None:
+            # the whole model as one operator and one autograd node
             plan = edge_index if isinstance(edge_index, GraphPlan) else get_plan(edge_index, x.shape[0] + self.num_global_node)
             plan.handle      # raises if the plan was closed
-            pad = (-x.shape[1]) % (4 if x.dtype == torch.float32 else 8)
-            if pad:
-                x = F.pad(x, (0, pad))
-                P[0] = F.pad(P[0], (0, pad))
             eps = [e for layer in self.layers for e in (layer.self_attention_norm.eps, layer.ffn_norm.eps)] + [self.final_ln.eps]
-            return _ext.op("node_graphormer")(x.contiguous(), P, plan.holder, plan.workspace(self.num_heads, 64 // self.num_heads),
-                                              self.num_heads, self.num_global_node, eps)
+            H, tokens, classes, ve = self.num_heads, self.num_global_node, P[-1].shape[0], 4 if x.dtype == torch.float32 else 8
+            if self._fused(P, H):      # kernels that take a layer's node-local part in one pass each way
+                if x.shape[1] % ve:
+                    pad = (-x.shape[1]) % ve
+                    x, P[0] = F.pad(x, (0, pad)), F.pad(P[0], (0, pad))
+                return _ext.op("node_graphormer")(x.contiguous(), P, plan.holder, plan.workspace(H, 64 // H), H, tokens, eps)
+            C, ff = P[0].shape[0], P[15].shape[0]
+            if C % ve == 0 and ff % ve == 0 and C % H == 0:
+                x = padded(P, x, 0, -2)
+                return _ext.op("layered_graphormer")(x, P, plan.holder, plan.workspace(H, C // H), H, tokens, classes, eps)
         x = x.unsqueeze(0)
         n_graph = x.shape[0]
         (node_feature,) = fused_linear(x, self.node_encoder)

@@ -210,7 +210,7 @@ class Graphormer(nn.Module):
             for i in range(len(self.layers)):
                 names += [f"layers.{i}.{k}" for k in LAYER_PARAMETERS]
             names += ["final_ln.weight", "final_ln.bias", f"{head}.weight", f"{head}.bias"]
-            tree = _TREES[self] = ModuleTree(self, names, ["self_attention_dropout", "ffn_dropout", "input_dropout"], 8 if multi_hop else 7)
+            tree = _TREES[self] = ModuleTree(self, names, ["self_attention_dropout", "ffn_dropout", "input_dropout"])
         first = self.layers[0].self_attention.dist_attn.local_attn
         for layer in self.layers:
             core = layer.self_attention.dist_attn.local_attn
@@ -219,7 +219,8 @@ class Graphormer(nn.Module):
                     core.attention_dropout_rate != first.attention_dropout_rate or core.dense_bf16_products:
                 return None
         P = tree.parameters(self.final_ln.weight.dtype, self.training)
-        if P is None or P[0].dtype not in _DT or P[0].shape[1] != 64 or P[-1].shape[0] > 64 or P[4].shape[1] != self.layers[0].self_attention.num_heads:
+        if P is None or P[0].dtype not in _DT or P[0].shape[1] != 64 or P[-1].shape[0] > 64 or P[4].shape[1] != self.layers[0].self_attention.num_heads or \
+                any(p.shape[0] != 64 or p.shape[-1] != 64 for p in P[8 if multi_hop else 7:-4]):
             return None
         return P
 

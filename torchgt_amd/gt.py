@@ -10,8 +10,9 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _ext, _lib
-from .encoder import init_params
+from .encoder import init_params, model_parameters, padded
 from .multi_head_attention import MultiHeadAttention, fused_linear
+from .plan import GraphPlan, get_plan
 
 _DT = {torch.float32: _lib.DTYPE_F32, torch.bfloat16: _lib.DTYPE_BF16}
 
@@ -43,6 +44,8 @@ class EncoderLayer(nn.Module):
         self.FFN_layer1 = nn.Linear(hidden_size, hidden_size * 2)
         self.FFN_layer2 = nn.Linear(hidden_size * 2, hidden_size)
         self.layer_norm2 = nn.LayerNorm(hidden_size)
+
+    one_operator = True      # False: the model runs this layer operator by operator
 
     def forward(self, x, attn_bias=None, edge_index=None, attn_type=None):
         n1, n2 = self.layer_norm1, self.layer_norm2
@@ -91,7 +94,29 @@ class GT(nn.Module):
         self.downstream_out_proj = nn.Linear(hidden_dim, output_dim)      # constructed, not used (:321)
         self.apply(lambda module: init_params(module, n_layers=n_layers))
 
+    one_operator = True      # False: always run the model layer by layer
+    dropouts = ("self_attention_dropout", "input_dropout")
+
+    def _parameter_names(self):
+        both = lambda name: [f"{name}.weight", f"{name}.bias"]
+        names = both("node_encoder")
+        for i in range(len(self.layers)):
+            for part in ("self_attention.linear_q", "self_attention.linear_k", "self_attention.linear_v", "O", "layer_norm1", "FFN_layer1", "FFN_layer2",
+                         "layer_norm2"):
+                names += both(f"layers.{i}.{part}")
+        return names + [n for j in range(self.MLP_layer.L + 1) for n in both(f"MLP_layer.FC_layers.{j}")]
+
     def forward(self, x, attn_bias, edge_index, perturb=None, attn_type=None):
+        if self.one_operator and attn_type == "sparse" and edge_index is not None and x.dim() == 2 and x.is_cuda and x.dtype in _DT and self.MLP_layer.L == 2:
+            P = model_parameters(self, x.dtype)
+            ve, H = 4 if x.dtype == torch.float32 else 8, self.layers[0].self_attention.num_heads
+            if P is not None and all(p.shape[0] % ve == 0 for p in P[:-2]) and P[2].shape[0] % H == 0:
+                # the whole model as one operator and one autograd node
+                plan = edge_index if isinstance(edge_index, GraphPlan) else get_plan(edge_index, x.shape[0])
+                plan.handle      # raises if the plan was closed
+                eps, classes = [e for layer in self.layers for e in (layer.layer_norm1.eps, layer.layer_norm2.eps)], P[-1].shape[0]
+                x = padded(P, x, 0, -2)
+                return _ext.op("layered_gt")(x, P, plan.holder, plan.workspace(H, P[2].shape[0] // H), H, classes, eps)
         x = x.unsqueeze(0)
         (node_feature,) = fused_linear(x, self.node_encoder)
         output = self.input_dropout(node_feature)
