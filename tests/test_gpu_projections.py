@@ -71,6 +71,15 @@ def test_linear_shapes(cuda, dtype):
         run_linear("in-100-out-44", 333, 100, 44, 1, dtype, cuda, 8)     # multiples of 4 only (100-d node features)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N,in_f,out_f,n", [(1, 8, 8, 1), (31, 64, 128, 1), (32, 128, 64, 2), (33, 56, 72, 3), (127, 128, 128, 3), (129, 136, 64, 1), (64, 200, 40, 2),
+                                            (65, 500 // 8 * 8, 8, 1), (4100, 128, 136, 3), (70000, 104, 64, 1), (300000, 16, 40, 1)])
+def test_linears_of_any_width(cuda, dtype, N, in_f, out_f, n):
+    """Edges of the row panels (32 per wave, 128 per workgroup, 64 of the weight gradient), of the 64-wide pieces, contractions of one, two
+    (operands kept) and more pieces, columns shared out between workgroups, row counts on both sides of the two partial counts."""
+    run_linear("any-width", N, in_f, out_f, n, dtype, cuda, N + in_f)
+
+
 def test_linear_weight_gradient_is_reproducible(cuda):
     """The weight gradients are summed in a fixed order: two runs give the same bits."""
     a = run_linear("repro-a", 20000, 64, 64, 3, torch.float32, cuda, 9)[1]

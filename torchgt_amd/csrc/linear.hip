@@ -11,11 +11,9 @@
 // N (nodes) is large and the feature widths are small (64 in the node-level
 // configurations), so every kernel walks panels of node rows and keeps the
 // weights / weight gradients on chip:
-//   k_linear<DX=false>   y_j = x W_j^T + b_j         panel of 128 rows, x staged once
-//   k_linear<DX=true>    dx  = sum_j dy_j W_j         same walk, W staged transposed
-//   k_linear_gradw       dW_j = dy_j^T x, db_j = colsum(dy_j): each workgroup keeps a
-//                        64 x 64 tile of every dW_j in registers over its share of the
-//                        panels and writes one partial; the fixed-order sum of reduce.hip adds the
+//   k_linear_tiles       y_j = x W_j^T + b_j, dx = sum_j dy_j W_j for widths other than 64 (linear_tiles.hip)
+//   k_gradw_tiles        dW_j = dy_j^T x, db_j = colsum(dy_j) (linear_tiles.hip): each workgroup keeps its tiles in
+//                        registers over its share of the panels and writes one partial; reduce.hip adds the
 //                        partials in a fixed order (no atomics: results are reproducible)
 // Matrix instructions: v_mfma_f32_32x32x2_f32 for float32 (exact fp32 products,
 // fp32 accumulation; the 64-wide forward instead splits every float into three
@@ -30,6 +28,7 @@
 // 16-byte LDS read.  (Any assignment of contraction indices to instructions gives
 // the same product as long as A and B use the same one.)
 #include "common.h"
+#include "linear_tiles.h"
 #include <algorithm>
 
 namespace tgt {
@@ -40,11 +39,10 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
 struct pbf16 { uint16_t x; };
 
 constexpr int kThreads = 256;
-constexpr int kPanel = 128;     // node rows per workgroup of the forward / input-gradient kernel
 constexpr int kChunk = 64;      // contraction indices per LDS stage
 constexpr int kCols = 64;       // output columns per accumulation pass
 constexpr int kGradRows = 64;   // node rows per step of the weight-gradient kernel
-constexpr int kGradWorkers = 512;   // workgroups (partials) of the weight-gradient kernel per output tile set
+constexpr int kGradWorkers = 1024;   // most workgroups (partials) of the weight-gradient kernel per output tile set
 
 template <typename T> constexpr int lds_stride(int inner) { return inner + 16 / (int)sizeof(T); }
 
@@ -260,64 +258,6 @@ template <int KC> struct Mma<pbf16, KC> {
         }
     }
 };
-
-struct LinArgs {
-    const void* A[3];      // forward: A[0] = x [N, K]; input gradient: A[j] = dy_j [N, M]
-    const void* W[3];      // [M, K] row-major (nn.Linear.weight)
-    const void* bias[3];   // forward only; entries may be null
-    void* out[3];          // forward: y_j [N, M]; input gradient: out[0] = dx [N, K]
-    int nw;
-    int64_t N;
-    int K, M;
-};
-
-// One workgroup per panel of 128 node rows; wave w owns rows [32w, 32w+32) and two
-// 32-column blocks of the current 64 output columns.
-template <typename T, bool DX>
-__global__ __launch_bounds__(kThreads) void k_linear(LinArgs a) {
-    constexpr int S = lds_stride<T>(kChunk);
-    __shared__ __align__(16) T tA[kPanel * S];
-    __shared__ __align__(16) T tB[kCols * S];
-    const int L = DX ? a.M : a.K;          // contraction length
-    const int C = DX ? a.K : a.M;          // output columns
-    const int n_out = DX ? 1 : a.nw, n_src = DX ? a.nw : 1;
-    const int64_t row0 = (int64_t)blockIdx.x * kPanel;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, h = lane >> 5;
-    const bool a_resident = (n_src == 1 && L <= kChunk);   // the source panel is staged once for all outputs
-    bool a_loaded = false;
-    for (int o = 0; o < n_out; ++o) {
-        for (int c0 = 0; c0 < C; c0 += kCols) {
-            float16_t acc0 = zero16(), acc1 = zero16();
-            for (int s = 0; s < n_src; ++s) {
-                const T* W = reinterpret_cast<const T*>(a.W[DX ? s : o]);
-                for (int l0 = 0; l0 < L; l0 += kChunk) {
-                    __syncthreads();
-                    if (!(a_resident && a_loaded)) {
-                        stage_natural<T, kPanel, S>(tA, reinterpret_cast<const T*>(a.A[s]), L, row0, a.N, l0, L);
-                        a_loaded = true;
-                    }
-                    if (!DX) stage_natural<T, kCols, S>(tB, W, a.K, c0, a.M, l0, a.K);       // rows = output columns
-                    else stage_transposed<T, kChunk, S>(tB, W, a.K, l0, a.M, c0, a.K);       // rows of W = contraction
-                    __syncthreads();
-                    const T* ap = tA + (wave * 32 + l32) * S + h * (kChunk / 2);
-                    Mma<T, kChunk>::run(ap, tB + l32 * S + h * (kChunk / 2), acc0);
-                    Mma<T, kChunk>::run(ap, tB + (32 + l32) * S + h * (kChunk / 2), acc1);
-                }
-            }
-            T* out = reinterpret_cast<T*>(a.out[o]);
-            const T* bias = DX ? nullptr : reinterpret_cast<const T*>(a.bias[o]);
-#pragma unroll
-            for (int cb = 0; cb < 2; ++cb) {
-                const int col = c0 + 32 * cb + l32;
-                if (col >= C) continue;
-                const float bv = bias ? ld1(bias + col) : 0.f;
-                const float16_t& acc = cb ? acc1 : acc0;
-                const int64_t first = row0 + wave * 32 + 4 * h;
-                store_rows<T>(out + first * C + col, C, acc, bv, a.N - first);
-            }
-        }
-    }
-}
 
 // A 64-row x 64-column tile on its way from global memory to LDS: each thread
 // holds 16-byte pieces in registers, so the loads of the next panel can be in
@@ -611,95 +551,18 @@ int launch_linear(const LinArgs& a, hipStream_t st) {
         if (a.nw == 2) return launch_linear64<T, DX, 2>(a, st);
         return launch_linear64<T, DX, 3>(a, st);
     }
-    hipLaunchKernelGGL((k_linear<T, DX>), dim3((unsigned)((a.N + kPanel - 1) / kPanel)), dim3(kThreads), 0, st, a);
-    return TGT_OK;
-}
-
-struct GradWArgs {
-    const void* x;         // [N, K]
-    const void* dy[3];     // [N, M]
-    float* partial;        // [workers][nw][M*K + M]
-    int64_t N;
-    int K, M;
-};
-
-// blockIdx.y picks a 64 x 64 tile (mt, kt) of the weight gradients, blockIdx.x a
-// worker; wave w owns the 32 x 32 block (w/2, w%2) of the tile for every weight.
-template <typename T, int NW>
-__global__ __launch_bounds__(kThreads) void k_linear_gradw(GradWArgs a) {
-    constexpr int S = lds_stride<T>(kGradRows);
-    extern __shared__ __align__(16) unsigned char smem[];
-    T* tX = reinterpret_cast<T*>(smem);          // [64 k][64 nodes]
-    T* tD = tX + kCols * S;                      // NW x [64 m][64 nodes]
-    const int kt_n = (a.K + kCols - 1) / kCols;
-    const int mt = blockIdx.y / kt_n, kt = blockIdx.y % kt_n;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, h = lane >> 5;
-    const int mi = wave >> 1, ki = wave & 1;
-    float16_t acc[NW];
-#pragma unroll
-    for (int j = 0; j < NW; ++j) acc[j] = zero16();
-    float colsum = 0.f;
-    static_assert(kGradRows == 64, "piece layout");
-    const int64_t n_panels = (a.N + kGradRows - 1) / kGradRows;
-    PieceRegs<T> nx, nd[NW];
-    int64_t p = blockIdx.x;
-    if (p < n_panels) {
-        fetch_t(nx, reinterpret_cast<const T*>(a.x), a.K, p * kGradRows, a.N, kt * kCols, a.K);
-#pragma unroll
-        for (int j = 0; j < NW; ++j)
-            fetch_t(nd[j], reinterpret_cast<const T*>(a.dy[j]), a.M, p * kGradRows, a.N, mt * kCols, a.M);
-    }
-    for (; p < n_panels; p += gridDim.x) {
-        __syncthreads();
-        put_t<T, S>(nx, tX, p * kGradRows, a.N, kt * kCols, a.K);
-#pragma unroll
-        for (int j = 0; j < NW; ++j) put_t<T, S>(nd[j], tD + j * kCols * S, p * kGradRows, a.N, mt * kCols, a.M);
-        __syncthreads();
-        if (p + gridDim.x < n_panels) {
-            const int64_t q = p + gridDim.x;
-            fetch_t(nx, reinterpret_cast<const T*>(a.x), a.K, q * kGradRows, a.N, kt * kCols, a.K);
-#pragma unroll
-            for (int j = 0; j < NW; ++j)
-                fetch_t(nd[j], reinterpret_cast<const T*>(a.dy[j]), a.M, q * kGradRows, a.N, mt * kCols, a.M);
-        }
-        const T* bp = tX + (32 * ki + l32) * S + h * (kGradRows / 2);
-#pragma unroll
-        for (int j = 0; j < NW; ++j)
-            Mma<T, kGradRows>::run(tD + j * kCols * S + (32 * mi + l32) * S + h * (kGradRows / 2), bp, acc[j]);
-        if (kt == 0 && wave < NW) {      // wave j adds up the columns of dy_j: lane = column
-            const T* row = tD + wave * kCols * S + lane * S;
-            float s = 0.f;
-#pragma unroll 16
-            for (int i = 0; i < kGradRows; ++i) s += ld1(row + i);
-            colsum += s;
-        }
-    }
-    const int64_t per = (int64_t)a.M * a.K + a.M;
-    float* mine = a.partial + (int64_t)blockIdx.x * NW * per;
-#pragma unroll
-    for (int j = 0; j < NW; ++j) {
-        const int k = kt * kCols + 32 * ki + l32;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int m = mt * kCols + 32 * mi + 8 * (r >> 2) + 4 * h + (r & 3);
-            if (m < a.M && k < a.K) mine[j * per + (int64_t)m * a.K + k] = acc[j][r];
-        }
-    }
-    if (kt == 0 && wave < NW) {
-        const int m = mt * kCols + lane;
-        if (m < a.M) mine[wave * per + (int64_t)a.M * a.K + m] = colsum;
-    }
+    return linear_tiles(a, DX, sizeof(T) == 4 ? TGT_DTYPE_F32 : TGT_DTYPE_BF16, st);
 }
 
 // ---------------------------------------------------------------------------
 // in_features = out_features = 64: the whole backward in one pass over dy.  A workgroup walks panels of 64 node
 // rows; for each it forms the panel of dx = sum_j dy_j W_j (weights resident in LDS, transposed) and adds
 // dy_j^T x and the column sums of dy_j to the 64 x 64 weight-gradient tiles it keeps in registers; at its end it
-// writes one partial like k_linear_gradw (the fixed-order sum of reduce.hip adds them).  dy is read once instead of twice and
+// writes one partial like k_gradw_tiles (the fixed-order sum of reduce.hip adds them).  dy is read once instead of twice and
 // one launch replaces two.
 //   bf16 (k_linear64_bwd, four waves): wave w owns the 32 x 32 block (w/2, w%2) of the dx panel and of every dW_j;
 //            the products over nodes need the node index contiguous: dy and x are also scattered into transposed
-//            tiles, as in k_linear_gradw.
+//            tiles.
 //   float32 (k_linear64_bwd_split, eight waves): see there.
 // ---------------------------------------------------------------------------
 struct Bwd64Args {
@@ -1051,19 +914,6 @@ int grad_workers(int in_features, int out_features) {
     return std::max(1, kGradWorkers / tiles);
 }
 
-template <typename T, int NW>
-int launch_gradw(const GradWArgs& g, int workers, int tiles, hipStream_t st) {
-    const size_t lds = sizeof(T) * (size_t)(1 + NW) * kCols * lds_stride<T>(kGradRows);
-    static bool raised = false;   // per instantiation; the attribute is per function and sticks
-    if (!raised && lds > 48 * 1024) {
-        TGT_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_linear_gradw<T, NW>),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        raised = true;
-    }
-    hipLaunchKernelGGL((k_linear_gradw<T, NW>), dim3(workers, tiles), dim3(kThreads), lds, st, g);
-    return TGT_OK;
-}
-
 template <typename T>
 int linear_bwd_t(const void* d_x, const void* const* d_W, const void* const* d_dy, int n_out, int64_t N, int K, int M,
                  void* d_dx, void* const* d_dW, void* const* d_db, float* partial, hipStream_t st, tgt_reduce_desc* defer,
@@ -1121,19 +971,18 @@ int linear_bwd_t(const void* d_x, const void* const* d_W, const void* const* d_d
         if (rc != TGT_OK) return rc;
     }
     if (d_dW) {
-        const int tiles = ((K + kCols - 1) / kCols) * ((M + kCols - 1) / kCols);
         const int64_t n_panels = (N + kGradRows - 1) / kGradRows;
-        const int workers = (int)std::max<int64_t>(1, std::min<int64_t>(n_panels, grad_workers(K, M)));
+        // half of them below 256 K rows: there the partials, written and read again, weigh more than the emptier chip (64 K rows,
+        // 128 x 128 float32, three weights: 66 us with 512, 75 us with 1024; 870 K rows, 104 x 64 bf16: 73 and 53 us)
+        const int workers = (int)std::max<int64_t>(1, std::min<int64_t>(n_panels, grad_workers(K, M) / (N < (256 << 10) ? 2 : 1)));
         GradWArgs g{};
         g.x = d_x;
         for (int j = 0; j < n_out; ++j) g.dy[j] = d_dy[j];
-        g.partial = partial; g.N = N; g.K = K; g.M = M;
+        g.partial = partial; g.nw = n_out; g.N = N; g.K = K; g.M = M;
         int rc = TGT_OK;
         {
             KernelTimer t(KS_LINEAR_DW, st);
-            if (n_out == 1) rc = launch_gradw<T, 1>(g, workers, tiles, st);
-            else if (n_out == 2) rc = launch_gradw<T, 2>(g, workers, tiles, st);
-            else rc = launch_gradw<T, 3>(g, workers, tiles, st);
+            rc = gradw_tiles(g, workers, sizeof(T) == 4 ? TGT_DTYPE_F32 : TGT_DTYPE_BF16, st);
         }
         if (rc != TGT_OK) return rc;
         TGT_HIP_CHECK(hipGetLastError());

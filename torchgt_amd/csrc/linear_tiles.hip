@@ -1,0 +1,321 @@
+// Linears of any width (a multiple of 16 bytes per row): y_j = x W_j^T + b_j for up to three weights of one shape, and
+// dx = sum_j dy_j W_j.  The node-level models' encoder and classes, and every linear of hidden sizes other than 64.
+//
+// Bound by the traffic of x and y at 64 K nodes and more, by latency below.  A wave takes 32 node rows; 64 features of
+// them at a time become matrix operands in its registers (node_tile.h: float32 as three exact bf16 planes, six products), the
+// workgroup's four waves share 64 x 64 pieces of the weight, packed into operand order on their way to LDS, and 64 output columns
+// accumulate in registers.  A contraction of up to 128 keeps its operands in registers for all output columns, so x is read
+// once; a longer one reads it again for every 64 columns.  The next piece of the weight is asked for before the products of
+// this one.  With few rows the output columns are spread over blockIdx.y until there are two workgroups per CU.
+#include "linear_tiles.h"
+#include "node_tile.h"
+#include <algorithm>
+#include <atomic>
+
+namespace tgt {
+namespace {
+
+constexpr int kThreads = 256, kWaves = 4;
+
+// 16 bytes of row r's columns k0 + ... of an array with ld columns (16-byte pieces; K of them count)
+template <typename T> __device__ __forceinline__ void fetch_cols(Raw<T>& raw, const T* __restrict__ src, int ld, int k0, const Rows& rows, int lane) {
+    constexpr int PP = RowShape<T>::kPieces, PER = RowShape<T>::kPer, VE = 16 / (int)sizeof(T);
+    const int last = rows.left > 0 ? rows.left - 1 : 0, r0 = lane / PP, col = k0 + (lane % PP) * VE;
+    const T* p = src + rows.first * ld + (col < ld ? col : 0);
+#pragma unroll
+    for (int i = 0; i < RowShape<T>::kAcc; ++i) {
+        const int r = r0 + i * PER;
+        raw.v[i] = *reinterpret_cast<const vec16*>(p + (int64_t)(r < last ? r : last) * ld);
+    }
+    if (k0 + 64 > ld && col >= ld) {      // (the weights are zero there, the row's neighbour may be anything)
+#pragma unroll
+        for (int i = 0; i < RowShape<T>::kAcc; ++i) raw.v[i] = vec16{0u, 0u, 0u, 0u};
+    }
+}
+template <typename T> __device__ __forceinline__ void put_cols(T* __restrict__ dst, int ld, int c0, const Tile& t, vec16* stage, const Rows& rows, int lane) {
+    constexpr int PP = RowShape<T>::kPieces, PER = RowShape<T>::kPer, VE = 16 / (int)sizeof(T);
+    wave_sync();
+    const int nb = node_base<T>(lane);
+#pragma unroll
+    for (int i = 0; i < PP / 2; ++i) {
+        float f[VE];
+#pragma unroll
+        for (int e = 0; e < VE; ++e) f[e] = t.get(i * VE + e);
+        stage[nb ^ i] = pack16(f, (const T*)nullptr);
+    }
+    wave_sync();
+    const int rb = row_base<T>(lane), r0 = lane / PP, col = c0 + (lane % PP) * VE;
+    vec16 v[RowShape<T>::kAcc];
+#pragma unroll
+    for (int i = 0; i < RowShape<T>::kAcc; ++i) v[i] = stage[row_slot<T>(rb, i)];
+    if (col >= ld) return;
+    T* p = dst + rows.first * ld + col;
+#pragma unroll
+    for (int i = 0; i < RowShape<T>::kAcc; ++i)
+        if (r0 + i * PER < rows.left) *reinterpret_cast<vec16*>(p + (int64_t)(r0 + i * PER) * ld) = v[i];
+}
+
+__device__ __forceinline__ float as_float(float v) { return v; }
+__device__ __forceinline__ float as_float(nbf16 v) { return __uint_as_float((uint32_t)v.x << 16); }
+
+// A thread's share of a 64 x 64 piece of the weight on its way to LDS: two operand vectors (outputs o0 .., contraction k0 ..)
+template <typename T> struct Piece { T v[2][8]; };
+template <typename T, bool DX> __device__ __forceinline__ void fetch_piece(Piece<T>& w, const T* __restrict__ W, int ld, int o0, int outs, int k0, int len) {
+    const int lane = forgotten(threadIdx.x & 63), r = lane & 31;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int sm = (threadIdx.x >> 6) + 4 * j, s = sm >> 1, m = sm & 1;
+        int o = o0 + 32 * ((r >> 2) & 1) + 16 * m + 4 * (r >> 3) + (r & 3), k = k0 + 32 * (lane >> 5) + 8 * s;
+        o = o < outs ? o : outs - 1;
+        if (DX) {      // eight rows of W at one column
+            if (k0 + 64 <= len) {      // (one vector offset, the rows as scalar bases)
+                const uint32_t at = k * ld + o;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) w.v[j][i] = (W + i * ld)[at];
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) w.v[j][i] = W[(uint32_t)((k + i < len ? k + i : len - 1) * ld + o)];
+            }
+        } else {       // eight columns of one row, in 16-byte pieces that end with the row
+            constexpr int VE = 16 / (int)sizeof(T);
+#pragma unroll
+            for (int q = 0; q < 8 / VE; ++q) {
+                const int c = k + q * VE;
+                *reinterpret_cast<vec16*>(&w.v[j][q * VE]) = *reinterpret_cast<const vec16*>(W + (uint32_t)(o * ld + (c < len ? c : len - VE)));
+            }
+        }
+    }
+}
+template <typename T, int P> __device__ __forceinline__ void put_piece(vec16* dst, const Piece<T>& w, int o0, int outs, int k0, int len) {
+    const int lane = forgotten(threadIdx.x & 63), r = lane & 31;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int sm = (threadIdx.x >> 6) + 4 * j, s = sm >> 1, m = sm & 1;
+        const int o = o0 + 32 * ((r >> 2) & 1) + 16 * m + 4 * (r >> 3) + (r & 3), k = k0 + 32 * (lane >> 5) + 8 * s;
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = o < outs && k + i < len ? as_float(w.v[j][i]) : 0.f;
+        bf16x8_t p[P];
+        to_planes(v, p);
+#pragma unroll
+        for (int q = 0; q < P; ++q) dst[(sm * P + q) * 64 + lane] = __builtin_bit_cast(vec16, p[q]);
+    }
+}
+
+// (float32: 80 KB, two workgroups per CU)
+template <typename T> constexpr int lin_lds() { return 2 * kFragVecs<Num<T>::P> * 16 + kWaves * RowShape<T>::kVecs * 16; }
+
+// blockIdx.x: 128 rows; blockIdx.y: `per` of the 64-column pieces of all outputs
+template <typename T, bool DX, bool RESIDENT> __global__ __launch_bounds__(kThreads, 2) void k_linear_tiles(const LinArgs a, const int per) {
+    constexpr int P = Num<T>::P, FV = kFragVecs<P>;
+    extern __shared__ __align__(16) unsigned char smem[];
+    vec16* w = reinterpret_cast<vec16*>(smem);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    vec16* stage = w + 2 * FV + wave * RowShape<T>::kVecs;
+    const int L = DX ? a.M : a.K, C = DX ? a.K : a.M, nl = (L + 63) / 64, nk = (DX ? a.nw : 1) * nl, nc = (C + 63) / 64;
+    const int first = blockIdx.y * per, all = (DX ? 1 : a.nw) * nc, end = first + per < all ? first + per : all;
+    const Rows rows((int64_t)blockIdx.x * kWaves + wave, a.N);
+    Frags<P> f[RESIDENT ? 2 : 1];
+    Raw<T> raw;
+    const auto ask_rows = [&](int k) { fetch_cols(raw, reinterpret_cast<const T*>(a.A[k / nl]), L, (k % nl) * 64, rows, lane); };
+    const auto operands = [&](Frags<P>& to) {
+        Tile t;
+        settle<T, false>(t, raw, stage, rows, lane);
+        make_frags(to, t);
+    };
+    ask_rows(0);
+    Piece<T> next;
+    const auto ask = [&](int t, int k) { fetch_piece<T, DX>(next, reinterpret_cast<const T*>(a.W[DX ? k / nl : t / nc]), a.K, (t % nc) * 64, C, (k % nl) * 64, L); };
+    if constexpr (RESIDENT) {
+        operands(f[0]);
+        if (nk == 2) {
+            ask_rows(1);
+            operands(f[1]);
+        }
+    }
+    ask(first, 0);
+    int turn = 0;
+    for (int t = first; t < end; ++t) {
+        const int o = t / nc, c0 = (t - o * nc) * 64;
+        Tile acc;
+        zero(acc);
+        if (!DX && a.bias[o]) {
+            constexpr int VE = 16 / (int)sizeof(T);
+#pragma unroll
+            for (int i = 0; i < 32 / VE; ++i) {
+                const int c = c0 + 32 * (lane >> 5) + VE * i;
+                float v[VE];
+                unpack16(*reinterpret_cast<const vec16*>(reinterpret_cast<const T*>(a.bias[o]) + (c < C ? c : C - VE)), v, (const T*)nullptr);
+#pragma unroll
+                for (int e = 0; e < VE; ++e) acc.set(i * VE + e, v[e]);
+            }
+        }
+        for (int k = 0; k < nk; ++k, turn ^= 1) {
+            vec16* const mine = w + turn * FV;      // last read in the step before the one before: every wave has passed the barrier since
+            put_piece<T, P>(mine, next, c0, C, (k % nl) * 64, L);
+            if (k + 1 < nk) ask(t, k + 1);
+            else if (t + 1 < end) ask(t + 1, 0);
+            if constexpr (!RESIDENT) {
+                operands(f[0]);
+                if (k + 1 < nk || t + 1 < end) ask_rows(k + 1 < nk ? k + 1 : 0);
+            }
+            __syncthreads();
+            if (RESIDENT && k == 1) gemm<P>(acc, f[RESIDENT ? 1 : 0], mine, lane);
+            else gemm<P>(acc, f[0], mine, lane);
+        }
+        put_cols(reinterpret_cast<T*>(a.out[o]), C, c0, acc, stage, rows, lane);
+    }
+}
+
+// Raises the dynamic LDS limit of a kernel where it needs that, once per kernel and device (`done`: one bit per device)
+int allow_lds(const void* kernel, int bytes, std::atomic<uint64_t>& done) {
+    if (bytes <= 64 * 1024) return TGT_OK;
+    int dev = 0;
+    TGT_HIP_CHECK(hipGetDevice(&dev));
+    const uint64_t bit = 1ull << (dev & 63);
+    if (done.load(std::memory_order_relaxed) & bit) return TGT_OK;
+    TGT_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+    done.fetch_or(bit, std::memory_order_relaxed);
+    return TGT_OK;
+}
+
+template <typename T, bool DX, bool RESIDENT> int launch(const LinArgs& a, hipStream_t st) {
+    static std::atomic<uint64_t> done{0};
+    constexpr int lds = lin_lds<T>();
+    if (int rc = allow_lds(reinterpret_cast<const void*>(&k_linear_tiles<T, DX, RESIDENT>), lds, done)) return rc;
+    // two workgroups per CU: below that the columns are shared out
+    const int64_t panels = (a.N + 32 * kWaves - 1) / (32 * kWaves);
+    const int all = (DX ? 1 : a.nw) * (((DX ? a.K : a.M) + 63) / 64), splits = (int)std::min<int64_t>(all, std::max<int64_t>(1, 512 / panels)), per = (all + splits - 1) / splits;
+    hipLaunchKernelGGL((k_linear_tiles<T, DX, RESIDENT>), dim3((unsigned)panels, (unsigned)((all + per - 1) / per)), dim3(kThreads), lds, st, a, per);
+    TGT_HIP_CHECK(hipGetLastError());
+    return TGT_OK;
+}
+template <typename T, bool DX> int run(const LinArgs& a, hipStream_t st) {
+    return (DX ? a.nw * ((a.M + 63) / 64) : (a.K + 63) / 64) <= 2 ? launch<T, DX, true>(a, st) : launch<T, DX, false>(a, st);
+}
+
+// ---- weight gradients -------------------------------------------------------------------------------------------------
+// A workgroup keeps one 64-row piece of one dW_j against XT 64-column pieces of x in registers, one 32 x 32 block per wave, over
+// its share of 64-node panels.  The panel's rows arrive coalesced, are cut into bf16 planes on their way to LDS and are read back
+// transposed by the products (node_tile.h); the next panel is asked for before the products of this one.  Bound by the traffic
+// of x and dy: with two pieces of x at a time dy is read once per 128 columns of x.  XT = 1 where x has 64 columns or less.
+constexpr int kPanelBytes = 64 * 128;      // one plane of one operand
+
+template <typename T, int XT> __global__ __launch_bounds__(XT * 256) void k_gradw_tiles(const GradWArgs a) {
+    constexpr int P = Num<T>::P, NWV = 4 * XT, RPW = 64 / NWV, PP = RowShape<T>::kPieces, PER = RowShape<T>::kPer, ACC = RPW / PER, VE = 16 / (int)sizeof(T), NT = 1 + XT;
+    extern __shared__ __align__(16) unsigned char smem[];      // [NT][P][kPanelBytes]: dy, then x
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int groups = ((a.K + 63) / 64 + XT - 1) / XT, mts = (a.M + 63) / 64;
+    const int m = blockIdx.y / groups, g = blockIdx.y - m * groups, j = m / mts, m0 = (m - j * mts) * 64, k0 = g * XT * 64;
+    const T* src[NT];
+    int ld[NT], col[NT];
+    src[0] = reinterpret_cast<const T*>(a.dy[j]); ld[0] = a.M; col[0] = m0;
+#pragma unroll
+    for (int t = 1; t < NT; ++t) { src[t] = reinterpret_cast<const T*>(a.x); ld[t] = a.K; col[t] = k0 + 64 * (t - 1); }
+    const int q = lane % PP, r0 = wave * RPW + lane / PP;      // this lane's 16-byte piece and first row of a panel
+    const int64_t panels = (a.N + 63) / 64;
+    vec16 raw[NT][ACC];
+    const auto fetch = [&](int64_t p) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const int c = col[t] + q * VE;
+#pragma unroll
+            for (int i = 0; i < ACC; ++i) {
+                const int64_t r = p * 64 + r0 + i * PER;
+                raw[t][i] = *reinterpret_cast<const vec16*>(src[t] + (r < a.N ? r : a.N - 1) * ld[t] + (c < ld[t] ? c : ld[t] - VE));
+            }
+        }
+    };
+    float sums[VE];
+#pragma unroll
+    for (int e = 0; e < VE; ++e) sums[e] = 0.f;
+    float16_t acc;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+    const int block = wave & 3, base_dy = operand_base(block >> 1, lane), base_x = operand_base(block & 1, lane);
+    const unsigned char* const x_planes = smem + (1 + wave / 4) * P * kPanelBytes;
+    int64_t p = blockIdx.x;
+    if (p < panels) fetch(p);
+    for (; p < panels; p += gridDim.x) {
+        __syncthreads();      // the panel before has been used
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const bool in = col[t] + q * VE < ld[t];
+#pragma unroll
+            for (int i = 0; i < ACC; ++i) {
+                const int r = r0 + i * PER;
+                if (!in || p * 64 + r >= a.N) raw[t][i] = vec16{0u, 0u, 0u, 0u};
+                float v[VE];
+                unpack16(raw[t][i], v, (const T*)nullptr);
+                if (t == 0) {
+#pragma unroll
+                    for (int e = 0; e < VE; ++e) sums[e] += v[e];
+                }
+                unsigned char* const at = smem + t * P * kPanelBytes + r * 128 + (((q * VE / 8) ^ (r & 7)) << 4);
+                if constexpr (P == 1) *reinterpret_cast<vec16*>(at) = raw[t][i];
+                else {
+                    uint32_t w[3][4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) cut3(v[e], w[0][e], w[1][e], w[2][e]);
+#pragma unroll
+                    for (int s = 0; s < P; ++s)
+                        *reinterpret_cast<uint2*>(at + s * kPanelBytes + 8 * (q & 1)) =
+                            make_uint2(__builtin_amdgcn_perm(w[s][1], w[s][0], 0x07060302u), __builtin_amdgcn_perm(w[s][3], w[s][2], 0x07060302u));
+                }
+            }
+        }
+        __syncthreads();
+        if (p + gridDim.x < panels) fetch(p + gridDim.x);
+        node_product<P, kPanelBytes>(acc, smem, x_planes, base_dy, base_x);
+    }
+    const int64_t per = (int64_t)a.M * a.K + a.M;
+    float* const mine = a.partial + ((int64_t)blockIdx.x * a.nw + j) * per;
+    const int k = k0 + 64 * (wave / 4) + 32 * (block & 1) + (lane & 31);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int o = m0 + 32 * (block >> 1) + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+        if (o < a.M && k < a.K) mine[(int64_t)o * a.K + k] = acc[i];
+    }
+    if (g == 0) {      // column sums of dy: over the lanes of a piece, then over the waves
+        float* const part = reinterpret_cast<float*>(smem);
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < VE; ++e) {
+#pragma unroll
+            for (int off = PP; off < 64; off <<= 1) sums[e] += __shfl_xor(sums[e], off);
+            if (lane < PP) part[wave * 64 + q * VE + e] = sums[e];
+        }
+        __syncthreads();
+        if (threadIdx.x < 64 && m0 + (int)threadIdx.x < a.M) {
+            float s = 0.f;
+#pragma unroll
+            for (int w = 0; w < NWV; ++w) s += part[w * 64 + threadIdx.x];
+            mine[(int64_t)a.M * a.K + m0 + threadIdx.x] = s;
+        }
+    }
+}
+
+template <typename T, int XT> int launch_gradw(const GradWArgs& a, int workers, hipStream_t st) {
+    static std::atomic<uint64_t> done{0};
+    constexpr int lds = (1 + XT) * Num<T>::P * kPanelBytes;
+    if (int rc = allow_lds(reinterpret_cast<const void*>(&k_gradw_tiles<T, XT>), lds, done)) return rc;
+    const int groups = ((a.K + 63) / 64 + XT - 1) / XT;
+    hipLaunchKernelGGL((k_gradw_tiles<T, XT>), dim3((unsigned)workers, (unsigned)(a.nw * ((a.M + 63) / 64) * groups)), dim3(XT * 256), lds, st, a);
+    TGT_HIP_CHECK(hipGetLastError());
+    return TGT_OK;
+}
+
+}  // namespace
+
+int gradw_tiles(const GradWArgs& a, int workers, int dtype, hipStream_t st) {
+    // (one piece of x at a time where there is only one)
+    if (dtype == TGT_DTYPE_F32) return a.K <= 64 ? launch_gradw<float, 1>(a, workers, st) : launch_gradw<float, 2>(a, workers, st);
+    return a.K <= 64 ? launch_gradw<nbf16, 1>(a, workers, st) : launch_gradw<nbf16, 2>(a, workers, st);
+}
+
+int linear_tiles(const LinArgs& a, bool dx, int dtype, hipStream_t st) {
+    if (dtype == TGT_DTYPE_F32) return dx ? run<float, true>(a, st) : run<float, false>(a, st);
+    return dx ? run<nbf16, true>(a, st) : run<nbf16, false>(a, st);
+}
+
+}  // namespace tgt

@@ -434,29 +434,29 @@ __device__ __forceinline__ int operand_base(int block, int lane) {
     const int i = lane & 15, chunk = 4 * block + 2 * ((lane >> 4) & 1) + ((i & 3) >> 1);
     return (8 * (lane >> 5) + (i >> 2)) * 128 + ((chunk ^ (i >> 2)) << 4) + 8 * (i & 1);
 }
-template <int P> __device__ __forceinline__ void node_operand(bf16x8_t (&out)[P], const unsigned char* planes, int base, int node0) {
+template <int P, int BYTES = kPlaneBytes> __device__ __forceinline__ void node_operand(bf16x8_t (&out)[P], const unsigned char* planes, int base, int node0) {
     typedef __attribute__((address_space(3))) short4_t lds_short4;
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-        const unsigned char* q = planes + p * kPlaneBytes + node0 * 128;
+        const unsigned char* q = planes + p * BYTES + node0 * 128;
         const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(q + base));
         const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(q + (base ^ 64) + 512));     // rows + 4
         const uint2 a = __builtin_bit_cast(uint2, lo), b = __builtin_bit_cast(uint2, hi);
         out[p] = __builtin_bit_cast(bf16x8_t, vec16{a.x, a.y, b.x, b.y});
     }
 }
-// acc += dy^T x over the 128 nodes, one 32 x 32 block (bases of its rows and columns from operand_base); the operands of
+// acc += dy^T x over the nodes of the planes, one 32 x 32 block (bases of its rows and columns from operand_base); the operands of
 // the next sixteen nodes are asked for before the products of these
-template <int P> __device__ __forceinline__ void node_product(float16_t& acc, const unsigned char* dy, const unsigned char* x, int base_dy, int base_x) {
+template <int P, int BYTES = kPlaneBytes> __device__ __forceinline__ void node_product(float16_t& acc, const unsigned char* dy, const unsigned char* x, int base_dy, int base_x) {
     bf16x8_t a[2][P], b[2][P];
-    node_operand<P>(a[0], dy, base_dy, 0);
-    node_operand<P>(b[0], x, base_x, 0);
+    node_operand<P, BYTES>(a[0], dy, base_dy, 0);
+    node_operand<P, BYTES>(b[0], x, base_x, 0);
 #pragma unroll
-    for (int k = 0; k < 128; k += 16) {
+    for (int k = 0; k < BYTES / 128; k += 16) {
         const int now = (k >> 4) & 1;
-        if (k + 16 < 128) {
-            node_operand<P>(a[now ^ 1], dy, base_dy, k + 16);
-            node_operand<P>(b[now ^ 1], x, base_x, k + 16);
+        if (k + 16 < BYTES / 128) {
+            node_operand<P, BYTES>(a[now ^ 1], dy, base_dy, k + 16);
+            node_operand<P, BYTES>(b[now ^ 1], x, base_x, k + 16);
         }
         acc = mma_planes(a[now], b[now], acc);
         fence_schedule();
