@@ -335,6 +335,9 @@ int tgt_fix_edge_index(const int64_t* d_edge_index, int64_t E0, int64_t num_node
  * too small (*h_num_edges then holds the needed size). */
 int tgt_sub_edge_index(const int64_t* d_edge_index, int64_t E, int64_t N, const int64_t* d_idx_batch, int64_t S,
                        int64_t* d_out, int64_t capacity, int64_t* h_num_edges, void* stream);
+/* The same with the two rows of the result one behind the other: row 1 starts at d_out + *h_num_edges. */
+int tgt_sub_edge_index_packed(const int64_t* d_edge_index, int64_t E, int64_t N, const int64_t* d_idx_batch, int64_t S,
+                              int64_t* d_out, int64_t capacity, int64_t* h_num_edges, void* stream);
 
 /* reformat_graph (gt_sp/utils.py:319-359) with the METIS call replaced by the
  * explicit d_partition_ids int64 [N] in [0, k):
@@ -345,7 +348,7 @@ int tgt_sub_edge_index(const int64_t* d_edge_index, int64_t E, int64_t N, const 
  *     (including its compact-count quirk and p hard-wired to 1);
  *   blockize == 0: keep the real edges (the alternative commented out at :347);
  *   stable sort of the new edge list by source (:354-356).
- * Synchronises `stream`.  Results are read with tgt_reformat_export:
+ * Synchronises `stream` once, for the counts; what follows is complete in stream order.  Results are read with tgt_reformat_export:
  * d_edge_index int64 [2, E'] (E' = tgt_reformat_num_edges), d_sorted_indices
  * int64 [N] = argsort(new_id_mapping) (new id -> old id, :352). */
 typedef struct tgt_reformat tgt_reformat_t;
@@ -355,6 +358,9 @@ int tgt_reformat_create(const int64_t* d_src, const int64_t* d_dst, int64_t E, i
 int64_t tgt_reformat_num_edges(const tgt_reformat_t* r);
 int tgt_reformat_export(const tgt_reformat_t* r, int64_t* d_edge_index, int64_t* d_sorted_indices, void* stream);
 int tgt_reformat_destroy(tgt_reformat_t* r);
+/* The rows of a batch in its new order (gt_sp/utils.py:463-472): d_rows[j] = d_idx_batch[old id - tokens] over the new ids,
+ * without the global node (old id 0) when tokens is 1; int64 [N - tokens]. */
+int tgt_reformat_rows(const tgt_reformat_t* r, const int64_t* d_idx_batch, int tokens, int64_t* d_rows, void* stream);
 /* The same result as a tile list: every emitted block as (first source, first
  * destination) in new ids (h_tiles, HOST int32 [T, 2], T = tgt_reformat_num_tiles)
  * plus the edges that were kept as they are (d_raw_edge_index, DEVICE int64

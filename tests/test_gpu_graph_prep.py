@@ -169,3 +169,21 @@ def test_prepare_batch_composes_the_reference_steps(cuda):
         return torch.as_tensor(part)
     out2 = graph_prep.prepare_batch(x.to(cuda), y.to(cuda), torch.as_tensor(idx), torch.as_tensor(e).to(cuda), n, k, bs, partition)
     assert seen["args"] == ((2, sub.shape[1]), S + 1, k) and torch.equal(out2[2], ei)
+
+
+@pytest.mark.parametrize("model,part_of_first", [("graphormer", 0), ("graphormer", 1), ("graphormer", 3), ("gt", 2)])
+def test_batch_rows_follow_the_new_order(cuda, model, part_of_first):
+    """Features and labels are gathered once, in the new order, wherever the global node's part (or the first node's) lies."""
+    g = torch.Generator().manual_seed(part_of_first)
+    n, S, k = 700, 333, 4
+    idx = torch.randperm(n, generator=g)[:S]
+    e = torch.randint(0, n, (2, 4000), generator=g)
+    tokens = 1 if model == "graphormer" else 0
+    part = torch.randint(0, k, (S + tokens,), generator=g)
+    part[0] = part_of_first
+    x, y = torch.randn(n, 5, generator=g), torch.arange(n)
+    x_i, y_i, ei, _ = graph_prep.prepare_batch(x.to(cuda), y.to(cuda), idx, e.to(cuda), n, k, 16, part, model=model, blockize=False)
+    order = torch.argsort(part, stable=True)
+    rows = idx[order[order != 0] - 1] if tokens else idx[order]
+    assert torch.equal(y_i.cpu(), rows) and torch.equal(x_i.cpu(), x[rows])
+    assert int(ei.max()) < S + tokens and ei.is_contiguous()

@@ -72,6 +72,8 @@ SIGNATURES = {
     "tgt_reformat_num_edges": (_i64, [_vp]),
     "tgt_reformat_export": (_i32, [_vp, _vp, _vp, _vp]),
     "tgt_reformat_destroy": (_i32, [_vp]),
+    "tgt_reformat_rows": (_i32, [_vp, _vp, _i32, _vp, _vp]),
+    "tgt_sub_edge_index_packed": (_i32, [_vp, _i64, _i64, _vp, _i64, _vp, _i64, _c.POINTER(_i64), _vp]),
     "tgt_np_legacy_randint": (_i32, [_c.c_uint32, _vp, _i32, _vp]),
     "tgt_linear_fwd": (_i32, [_vp, _vp, _vp, _vp, _i32, _i64, _i32, _i32, _i32, _vp]),
     "tgt_linear_bwd_workspace_bytes": (_i64, [_i32, _i32, _i32]),

@@ -154,16 +154,20 @@ int bits_for(int64_t n);   // bits needed to hold values in [0, n)
 // Stable LSD radix sort of (uint32 key, uint32 value) pairs (radix_sort.hip).
 class RadixSorter {
 public:
-    int init(int64_t capacity, hipStream_t st = nullptr);
-    // Sorts by the low `bits` bits of the keys.  vals_in == nullptr means values 0..n-1.
+    int init(int64_t capacity, hipStream_t st = nullptr, int sorts = 1);
+    // Sorts `sorts` key arrays by their low `bits` bits, side by side.  vals_in == nullptr means values 0..n-1.
     // The results live in the sorter's buffers until the next sort() call; copy a
     // result before passing it as input of another sort().
-    int sort(const uint32_t* keys_in, const uint32_t* vals_in, int64_t n, int bits, hipStream_t st,
+    int sort(const uint32_t* const* keys_in, const uint32_t* const* vals_in, int sorts, int64_t n, int bits, hipStream_t st,
              const uint32_t** keys_out, const uint32_t** vals_out);
+    int sort(const uint32_t* keys_in, const uint32_t* vals_in, int64_t n, int bits, hipStream_t st, const uint32_t** keys_out,
+             const uint32_t** vals_out) {
+        return sort(&keys_in, vals_in ? &vals_in : nullptr, 1, n, bits, st, keys_out, vals_out);
+    }
 private:
-    DevBuf keysA_, keysB_, valsA_, valsB_, hist_, totals_;
+    DevBuf buf_;
     int64_t cap_ = 0;
-    int nblocks_ = 0;
+    int nblocks_ = 0, sorts_ = 1;
 };
 
 // nn.GELU() (exact erf form) and F.relu on one value, and dh * d act / du.  One definition for the elementwise kernels

@@ -21,16 +21,18 @@ namespace tgt {
 // numpy legacy RandomState: MT19937 seeded with init_genrand, randint(0, high)
 // by masked rejection on 32-bit outputs.
 // ---------------------------------------------------------------------------
+// A stream here is short (the blocks of one pair of partitions) and there is one per pair: state words are seeded and twisted when
+// they are first needed, the same numbers as whole blocks of 624 (64 pairs: 180 us of host time with them).
 class LegacyMT {
 public:
-    explicit LegacyMT(uint32_t seed) {
-        mt_[0] = seed;
-        for (int i = 1; i < 624; ++i) mt_[i] = 1812433253u * (mt_[i - 1] ^ (mt_[i - 1] >> 30)) + (uint32_t)i;
-        pos_ = 624;
-    }
+    explicit LegacyMT(uint32_t seed) { mt_[0] = seed; }
     uint32_t next() {
-        if (pos_ == 624) refill();
-        uint32_t y = mt_[pos_++];
+        const uint32_t UP = 0x80000000u, LO = 0x7fffffffu, MAG = 0x9908b0dfu;
+        const int i = pos_, i1 = i + 1 < 624 ? i + 1 : 0, im = i + 397 < 624 ? i + 397 : i - 227;
+        seeded(im > i1 ? im : i1);
+        const uint32_t t = (mt_[i] & UP) | (mt_[i1] & LO);
+        uint32_t y = mt_[i] = mt_[im] ^ (t >> 1) ^ ((t & 1u) ? MAG : 0u);
+        pos_ = i1;
         y ^= y >> 11;
         y ^= (y << 7) & 0x9d2c5680u;
         y ^= (y << 15) & 0xefc60000u;
@@ -48,23 +50,11 @@ public:
         return (int64_t)v;
     }
 private:
-    void refill() {
-        const uint32_t UP = 0x80000000u, LO = 0x7fffffffu, MAG = 0x9908b0dfu;
-        int i = 0;
-        for (; i < 624 - 397; ++i) {
-            uint32_t y = (mt_[i] & UP) | (mt_[i + 1] & LO);
-            mt_[i] = mt_[i + 397] ^ (y >> 1) ^ ((y & 1u) ? MAG : 0u);
-        }
-        for (; i < 623; ++i) {
-            uint32_t y = (mt_[i] & UP) | (mt_[i + 1] & LO);
-            mt_[i] = mt_[i + (397 - 624)] ^ (y >> 1) ^ ((y & 1u) ? MAG : 0u);
-        }
-        uint32_t y = (mt_[623] & UP) | (mt_[0] & LO);
-        mt_[623] = mt_[396] ^ (y >> 1) ^ ((y & 1u) ? MAG : 0u);
-        pos_ = 0;
+    void seeded(int upto) {
+        for (; seeded_ <= upto; ++seeded_) mt_[seeded_] = 1812433253u * (mt_[seeded_ - 1] ^ (mt_[seeded_ - 1] >> 30)) + (uint32_t)seeded_;
     }
     uint32_t mt_[624];
-    int pos_;
+    int pos_ = 0, seeded_ = 1;
 };
 
 // ---------------------------------------------------------------------------
@@ -84,20 +74,12 @@ __global__ void k_fix_edge_index(const int64_t* __restrict__ in, int64_t E0, int
 }
 
 __global__ void k_check_partition(const int64_t* __restrict__ part, int64_t N, int k, uint32_t* __restrict__ p32,
-                                  int* __restrict__ flag) {
+                                  unsigned long long* __restrict__ flag) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
     int64_t p = part[i];
     if (p < 0 || p >= k) { flag[0] = 1; p = 0; }
     p32[i] = (uint32_t)p;
-}
-
-__global__ void k_check_edges(const int64_t* __restrict__ src, const int64_t* __restrict__ dst, int64_t E,
-                              int64_t N, int* __restrict__ flag) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= E) return;
-    const int64_t s = src[i], d = dst[i];
-    if ((s < 0) | (s >= N) | (d < 0) | (d >= N)) flag[0] = 1;
 }
 
 // mapping[old] = new position; sorted[new] = old (as int64 for the caller)
@@ -150,13 +132,15 @@ __global__ __launch_bounds__(256) void k_count(const uint32_t* __restrict__ keys
     }
 }
 
-// per-edge keys: pair = part[src]*k + part[dst], s32 = src, d32 = dst
-__global__ void k_edge_keys(const int64_t* __restrict__ src, const int64_t* __restrict__ dst, int64_t E,
+// per-edge keys: pair = part[src]*k + part[dst], s32 = src, d32 = dst; an endpoint outside [0, N) is flagged and taken as node 0
+__global__ void k_edge_keys(const int64_t* __restrict__ src, const int64_t* __restrict__ dst, int64_t E, int64_t N,
                             const uint32_t* __restrict__ p32, int k, uint32_t* __restrict__ pair,
-                            uint32_t* __restrict__ s32, uint32_t* __restrict__ d32) {
+                            uint32_t* __restrict__ s32, uint32_t* __restrict__ d32, unsigned long long* __restrict__ flag) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= E) return;
-    const uint32_t s = (uint32_t)src[i], d = (uint32_t)dst[i];
+    int64_t s64 = src[i], d64 = dst[i];
+    if ((s64 < 0) | (s64 >= N) | (d64 < 0) | (d64 >= N)) { flag[0] = 1; s64 = 0; d64 = 0; }
+    const uint32_t s = (uint32_t)s64, d = (uint32_t)d64;
     s32[i] = s;
     d32[i] = d;
     pair[i] = p32[s] * (uint32_t)k + p32[d];
@@ -182,11 +166,11 @@ __global__ void k_emit_raw(const uint32_t* __restrict__ order, int64_t lo, int64
 }
 
 // dense bs x bs block, pairs (a, b) row-major (gt_sp/utils.py:218-220); one workgroup per block
-__global__ void k_emit_blocks(const int64_t* __restrict__ blk_off, const uint32_t* __restrict__ blk_r0,
-                              const uint32_t* __restrict__ blk_c0, int bs, uint32_t* __restrict__ ns,
-                              uint32_t* __restrict__ nd) {
-    const int64_t off = blk_off[blockIdx.x];
-    const uint32_t r0 = blk_r0[blockIdx.x], c0 = blk_c0[blockIdx.x];
+struct Block { int64_t off; uint32_t r0, c0; };
+__global__ void k_emit_blocks(const Block* __restrict__ blocks, int bs, uint32_t* __restrict__ ns, uint32_t* __restrict__ nd) {
+    const Block b = blocks[blockIdx.x];
+    const int64_t off = b.off;
+    const uint32_t r0 = b.r0, c0 = b.c0;
     for (int p = threadIdx.x; p < bs * bs; p += blockDim.x) {
         ns[off + p] = r0 + (uint32_t)(p / bs);
         nd[off + p] = c0 + (uint32_t)(p % bs);
@@ -215,11 +199,21 @@ static inline unsigned nblk(int64_t n, int t = 256) { return (unsigned)((n + t -
 
 struct tgt_reformat {
     int64_t N = 0, E_out = 0;
-    tgt::DevBuf edge_index;       // int64 [2, E_out], stably sorted by source
+    tgt::RadixSorter sorter;      // the edges sorted by new source (stable): keys and order ...
+    const uint32_t *keys = nullptr, *order = nullptr;
+    tgt::DevBuf nd;               // ... and the new destinations in emission order
+    tgt::DevBuf mapping;          // uint32 [N], old id -> new id
     tgt::DevBuf sorted_indices;   // int64 [N], new id -> old id
     std::vector<int32_t> tiles;   // (first source, first destination) of every emitted block, emission order
     int64_t E_raw = 0;            // edges kept as they are (the sparsity > p branch, or everything if !blockize)
     tgt::DevBuf raw;              // int64 [2, E_raw], relabelled, emission order
+    std::vector<tgt::Block> blocks;      // feeds an asynchronous copy, which `copied` marks the end of
+    hipEvent_t copied = nullptr;
+    ~tgt_reformat() {
+        if (!copied) return;
+        (void)hipEventSynchronize(copied);
+        (void)hipEventDestroy(copied);
+    }
 };
 
 namespace tgt {
@@ -227,64 +221,51 @@ namespace tgt {
 static int reformat_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, int64_t N,
                          const int64_t* d_part, int k, int bs, int blockize, hipStream_t st, tgt_reformat* R) {
     R->N = N;
-    DevBuf flag, p32, mapping, sorted_old;
-    TGT_HIP_CHECK(flag.alloc(sizeof(int)));
-    TGT_HIP_CHECK(p32.alloc(sizeof(uint32_t) * N));
-    TGT_HIP_CHECK(mapping.alloc(sizeof(uint32_t) * N));
-    TGT_HIP_CHECK(R->sorted_indices.alloc(sizeof(int64_t) * N));
-    TGT_HIP_CHECK(hipMemsetAsync(flag.p, 0, sizeof(int), st));
-    hipLaunchKernelGGL(k_check_partition, dim3(nblk(N)), dim3(256), 0, st, d_part, N, k, p32.as<uint32_t>(),
-                       flag.as<int>());
-    if (E > 0)
-        hipLaunchKernelGGL(k_check_edges, dim3(nblk(E)), dim3(256), 0, st, d_src, d_dst, E, N, flag.as<int>());
-    int h_flag = 0;
-    TGT_HIP_CHECK(hipMemcpyAsync(&h_flag, flag.p, sizeof(int), hipMemcpyDeviceToHost, st));
+    DevBuf report, p32, pair, s32, d32;
+    const size_t eb = sizeof(uint32_t) * (size_t)(E ? E : 1);
+    // flag, nodes per part, edges per pair of parts: cleared and read back in one go
+    const size_t words = 1 + (size_t)k + (size_t)k * k;
+    TGT_HIP_CHECK(report.alloc(sizeof(unsigned long long) * words, st));
+    TGT_HIP_CHECK(p32.alloc(sizeof(uint32_t) * N, st));
+    TGT_HIP_CHECK(R->mapping.alloc(sizeof(uint32_t) * N, st));
+    TGT_HIP_CHECK(R->sorted_indices.alloc(sizeof(int64_t) * N, st));
+    TGT_HIP_CHECK(pair.alloc(eb, st));
+    TGT_HIP_CHECK(s32.alloc(eb, st));
+    TGT_HIP_CHECK(d32.alloc(eb, st));
+    const DevBuf& mapping = R->mapping;
+    unsigned long long *const flag = report.as<unsigned long long>(), *const cnt_nodes = flag + 1, *const cnt_pairs = cnt_nodes + k;
+    TGT_HIP_CHECK(hipMemsetAsync(report.p, 0, sizeof(unsigned long long) * words, st));
+    hipLaunchKernelGGL(k_check_partition, dim3(nblk(N)), dim3(256), 0, st, d_part, N, k, p32.as<uint32_t>(), flag);
+    const auto count_grid = [](int64_t n) { return dim3((unsigned)std::min<int64_t>(256, (n + 255) / 256)); };
+    hipLaunchKernelGGL(k_count, count_grid(N), dim3(256), 0, st, p32.as<uint32_t>(), N, k, bits_for(k), cnt_nodes);
+    if (E > 0) {
+        hipLaunchKernelGGL(k_edge_keys, dim3(nblk(E)), dim3(256), 0, st, d_src, d_dst, E, N, p32.as<uint32_t>(), k,
+                           pair.as<uint32_t>(), s32.as<uint32_t>(), d32.as<uint32_t>(), flag);
+        hipLaunchKernelGGL(k_count, count_grid(E), dim3(256), 0, st, pair.as<uint32_t>(), E, k * k,
+                           bits_for((int64_t)k * k), cnt_pairs);
+    }
+    std::vector<unsigned long long> h_report(words);
+    TGT_HIP_CHECK(hipMemcpyAsync(h_report.data(), report.p, sizeof(unsigned long long) * words, hipMemcpyDeviceToHost, st));
     TGT_HIP_CHECK(hipStreamSynchronize(st));
-    if (h_flag) {
+    if (h_report[0]) {
         set_error("partition id outside [0, %d) or edge endpoint outside [0, %lld)", k, (long long)N);
         return TGT_ERR_INDEX_RANGE;
     }
+    const unsigned long long *const h_nodes = h_report.data() + 1, *const h_pairs = h_nodes + k;
     // relabel: parts in order, members in ascending old id (gt_sp/utils.py:329-335) = stable sort by part
     RadixSorter node_sorter;
-    int rc = node_sorter.init(N);
+    int rc = node_sorter.init(N, st);
     if (rc) return rc;
     const uint32_t *ks = nullptr, *vs = nullptr;
     rc = node_sorter.sort(p32.as<uint32_t>(), nullptr, N, bits_for(k), st, &ks, &vs);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_invert, dim3(nblk(N)), dim3(256), 0, st, vs, N, mapping.as<uint32_t>(),
+    hipLaunchKernelGGL(k_invert, dim3(nblk(N)), dim3(256), 0, st, vs, N, R->mapping.as<uint32_t>(),
                        R->sorted_indices.as<int64_t>());
-    // node count per part
-    DevBuf cnt_nodes, cnt_pairs;
-    TGT_HIP_CHECK(cnt_nodes.alloc(sizeof(unsigned long long) * k));
-    TGT_HIP_CHECK(cnt_pairs.alloc(sizeof(unsigned long long) * k * k));
-    TGT_HIP_CHECK(hipMemsetAsync(cnt_nodes.p, 0, sizeof(unsigned long long) * k, st));
-    TGT_HIP_CHECK(hipMemsetAsync(cnt_pairs.p, 0, sizeof(unsigned long long) * k * k, st));
-    const auto count_grid = [](int64_t n) { return dim3((unsigned)std::min<int64_t>(256, (n + 255) / 256)); };
-    hipLaunchKernelGGL(k_count, count_grid(N), dim3(256), 0, st, p32.as<uint32_t>(), N, k, bits_for(k),
-                       cnt_nodes.as<unsigned long long>());
-    DevBuf pair, s32, d32;
-    const size_t eb = sizeof(uint32_t) * (size_t)(E ? E : 1);
-    TGT_HIP_CHECK(pair.alloc(eb));
-    TGT_HIP_CHECK(s32.alloc(eb));
-    TGT_HIP_CHECK(d32.alloc(eb));
-    if (E > 0) {
-        hipLaunchKernelGGL(k_edge_keys, dim3(nblk(E)), dim3(256), 0, st, d_src, d_dst, E, p32.as<uint32_t>(), k,
-                           pair.as<uint32_t>(), s32.as<uint32_t>(), d32.as<uint32_t>());
-        hipLaunchKernelGGL(k_count, count_grid(E), dim3(256), 0, st, pair.as<uint32_t>(), E, k * k,
-                           bits_for((int64_t)k * k), cnt_pairs.as<unsigned long long>());
-    }
-    std::vector<unsigned long long> h_nodes(k), h_pairs((size_t)k * k);
-    TGT_HIP_CHECK(hipMemcpyAsync(h_nodes.data(), cnt_nodes.p, sizeof(unsigned long long) * k,
-                                 hipMemcpyDeviceToHost, st));
-    TGT_HIP_CHECK(hipMemcpyAsync(h_pairs.data(), cnt_pairs.p, sizeof(unsigned long long) * k * k,
-                                 hipMemcpyDeviceToHost, st));
-    TGT_HIP_CHECK(hipStreamSynchronize(st));
 
     // ---- what to emit, in the reference's order ------------------------------
     struct RawSlice { int64_t lo, cnt, out_off; };
     std::vector<RawSlice> raws;
-    std::vector<int64_t> blk_off;
-    std::vector<uint32_t> blk_r0, blk_c0;
+    std::vector<Block>& blocks = R->blocks;
     int64_t E_out = 0;
     if (!blockize) {
         E_out = E;
@@ -320,9 +301,7 @@ static int reformat_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, 
                             const int64_t br = rng.randint(ni / bs);
                             const int64_t bc = rng.randint(nj / bs);
                             ++keep_cnt;
-                            blk_off.push_back(E_out);
-                            blk_r0.push_back((uint32_t)(br * bs + offs[i]));
-                            blk_c0.push_back((uint32_t)(bc * bs + offs[j]));
+                            blocks.push_back(Block{E_out, (uint32_t)(br * bs + offs[i]), (uint32_t)(bc * bs + offs[j])});
                             E_out += (int64_t)bs * bs;
                         }
                     }
@@ -332,12 +311,11 @@ static int reformat_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, 
     }
     if (E_out > 0x7fff0000LL) { set_error("reordered edge list does not fit 31 bits"); return TGT_ERR_INVALID_ARG; }
     R->E_out = E_out;
-    TGT_HIP_CHECK(R->edge_index.alloc(sizeof(int64_t) * 2 * (size_t)(E_out ? E_out : 1)));
-    DevBuf ns, nd;
-    TGT_HIP_CHECK(ns.alloc(sizeof(uint32_t) * (size_t)(E_out ? E_out : 1)));
-    TGT_HIP_CHECK(nd.alloc(sizeof(uint32_t) * (size_t)(E_out ? E_out : 1)));
-    RadixSorter sorter;
-    rc = sorter.init(E_out > E ? E_out : E);
+    DevBuf ns, &nd = R->nd;
+    TGT_HIP_CHECK(ns.alloc(sizeof(uint32_t) * (size_t)(E_out ? E_out : 1), st));
+    TGT_HIP_CHECK(nd.alloc(sizeof(uint32_t) * (size_t)(E_out ? E_out : 1), st));
+    RadixSorter& sorter = R->sorter;
+    rc = sorter.init(E_out > E ? E_out : E, st);
     if (rc) return rc;
 
     if (!blockize) {
@@ -350,8 +328,8 @@ static int reformat_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, 
             // edges sorted by ((part_src, part_dst), (src, dst)) (gt_sp/utils.py:230-235): LSD over
             // dst, src, pair with the stable sort
             DevBuf tmp, order;
-            TGT_HIP_CHECK(tmp.alloc(eb));
-            TGT_HIP_CHECK(order.alloc(eb));
+            TGT_HIP_CHECK(tmp.alloc(eb, st));
+            TGT_HIP_CHECK(order.alloc(eb, st));
             const uint32_t *ko = nullptr, *vo = nullptr;
             rc = sorter.sort(d32.as<uint32_t>(), nullptr, E, bits_for(N), st, &ko, &vo);
             if (rc) return rc;
@@ -370,32 +348,26 @@ static int reformat_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, 
                     hipLaunchKernelGGL(k_emit_raw, dim3(nblk(r.cnt)), dim3(256), 0, st, vo, r.lo, r.cnt,
                                        s32.as<uint32_t>(), d32.as<uint32_t>(), mapping.as<uint32_t>(), r.out_off,
                                        ns.as<uint32_t>(), nd.as<uint32_t>());
-            TGT_HIP_CHECK(hipStreamSynchronize(st));   // tmp / order die here
         }
-        if (!blk_off.empty()) {
-            DevBuf d_off, d_r0, d_c0;
-            const size_t nb = blk_off.size();
-            TGT_HIP_CHECK(d_off.alloc(sizeof(int64_t) * nb));
-            TGT_HIP_CHECK(d_r0.alloc(sizeof(uint32_t) * nb));
-            TGT_HIP_CHECK(d_c0.alloc(sizeof(uint32_t) * nb));
-            TGT_HIP_CHECK(hipMemcpyAsync(d_off.p, blk_off.data(), sizeof(int64_t) * nb, hipMemcpyHostToDevice, st));
-            TGT_HIP_CHECK(hipMemcpyAsync(d_r0.p, blk_r0.data(), sizeof(uint32_t) * nb, hipMemcpyHostToDevice, st));
-            TGT_HIP_CHECK(hipMemcpyAsync(d_c0.p, blk_c0.data(), sizeof(uint32_t) * nb, hipMemcpyHostToDevice, st));
-            hipLaunchKernelGGL(k_emit_blocks, dim3((unsigned)nb), dim3(256), 0, st, d_off.as<int64_t>(),
-                               d_r0.as<uint32_t>(), d_c0.as<uint32_t>(), bs, ns.as<uint32_t>(), nd.as<uint32_t>());
-            TGT_HIP_CHECK(hipStreamSynchronize(st));   // the descriptor buffers die here
+        if (!blocks.empty()) {
+            DevBuf d_blocks;
+            TGT_HIP_CHECK(d_blocks.alloc(sizeof(Block) * blocks.size(), st));
+            TGT_HIP_CHECK(hipMemcpyAsync(d_blocks.p, blocks.data(), sizeof(Block) * blocks.size(), hipMemcpyHostToDevice, st));
+            TGT_HIP_CHECK(hipEventCreateWithFlags(&R->copied, hipEventDisableTiming));
+            TGT_HIP_CHECK(hipEventRecord(R->copied, st));
+            hipLaunchKernelGGL(k_emit_blocks, dim3((unsigned)blocks.size()), dim3(256), 0, st, d_blocks.as<Block>(), bs, ns.as<uint32_t>(), nd.as<uint32_t>());
         }
     }
     // the blocks as a tile list and the edges kept as they are, for the block attention path
-    for (size_t i = 0; i < blk_r0.size(); ++i) {
-        R->tiles.push_back((int32_t)blk_r0[i]);
-        R->tiles.push_back((int32_t)blk_c0[i]);
+    for (const Block& b : blocks) {
+        R->tiles.push_back((int32_t)b.r0);
+        R->tiles.push_back((int32_t)b.c0);
     }
     {
         int64_t e_raw = blockize ? 0 : E;
         for (const RawSlice& r : raws) e_raw += r.cnt;
         R->E_raw = e_raw;
-        TGT_HIP_CHECK(R->raw.alloc(sizeof(int64_t) * 2 * (size_t)(e_raw ? e_raw : 1)));
+        TGT_HIP_CHECK(R->raw.alloc(sizeof(int64_t) * 2 * (size_t)(e_raw ? e_raw : 1), st));
         if (!blockize) {
             if (E > 0)
                 hipLaunchKernelGGL(k_write_raw, dim3(nblk(E)), dim3(256), 0, st, ns.as<uint32_t>(), nd.as<uint32_t>(),
@@ -412,15 +384,21 @@ static int reformat_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, 
     }
     // stable sort by new source (gt_sp/utils.py:354-356)
     if (E_out > 0) {
-        const uint32_t *ko = nullptr, *vo = nullptr;
-        rc = sorter.sort(ns.as<uint32_t>(), nullptr, E_out, bits_for(N), st, &ko, &vo);
+        rc = sorter.sort(ns.as<uint32_t>(), nullptr, E_out, bits_for(N), st, &R->keys, &R->order);
         if (rc) return rc;
-        hipLaunchKernelGGL(k_write_sorted, dim3(nblk(E_out)), dim3(256), 0, st, ko, vo, nd.as<uint32_t>(), E_out,
-                           R->edge_index.as<int64_t>());
     }
     TGT_HIP_CHECK(hipGetLastError());
-    TGT_HIP_CHECK(hipStreamSynchronize(st));
     return TGT_OK;
+}
+
+// The batch node behind every row of the reordered batch: idx[old id], without the `tokens` global nodes in front of the old ids
+// (at most one: the first member of its part, wherever that part lies)
+__global__ void k_batch_rows(const int64_t* __restrict__ sorted, int64_t N, const uint32_t* __restrict__ mapping, const int64_t* __restrict__ idx, int tokens,
+                             int64_t* __restrict__ out) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= N) return;
+    const int64_t token = tokens ? (int64_t)mapping[0] : N;      // the global node's new place
+    if (i != token) out[i > token ? i - 1 : i] = idx[sorted[i] - tokens];
 }
 
 // ---------------------------------------------------------------------------
@@ -437,8 +415,9 @@ static int reformat_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, 
 // ---------------------------------------------------------------------------
 constexpr int kSubItems = 1024;     // items per workgroup of the compaction (4 rounds of 256)
 
-__global__ void k_sub_fill(int32_t* __restrict__ pos, int64_t N) {
+__global__ void k_sub_fill(int32_t* __restrict__ pos, int64_t N, int* __restrict__ bad) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) *bad = 0;
     if (i < N) pos[i] = -1;
 }
 
@@ -539,28 +518,26 @@ __global__ __launch_bounds__(256) void k_sub_scan(uint32_t* __restrict__ counts,
 }
 
 static int sub_edge_index_impl(const int64_t* d_ei, int64_t E, int64_t N, const int64_t* d_idx, int64_t S,
-                               int64_t* d_out, int64_t capacity, int64_t* h_num, hipStream_t st) {
+                               int64_t* d_out, int64_t capacity, bool packed, int64_t* h_num, hipStream_t st) {
     const int64_t total = E + N;
     const int nblocks = (int)((total + kSubItems - 1) / kSubItems);
-    DevBuf pos, counts, bad, bits;
-    TGT_HIP_CHECK(pos.alloc(sizeof(int32_t) * (size_t)N));
-    TGT_HIP_CHECK(counts.alloc(sizeof(uint32_t) * (size_t)(nblocks + 1)));
-    TGT_HIP_CHECK(bits.alloc(sizeof(uint64_t) * (size_t)nblocks * (kSubItems / 64)));
-    TGT_HIP_CHECK(bad.alloc(sizeof(int)));
-    TGT_HIP_CHECK(hipMemsetAsync(bad.p, 0, sizeof(int), st));
-    hipLaunchKernelGGL(k_sub_fill, dim3(nblk(N)), dim3(256), 0, st, pos.as<int32_t>(), N);
+    DevBuf pos, counts, bits;      // counts: per workgroup, their total, the error flag
+    TGT_HIP_CHECK(pos.alloc(sizeof(int32_t) * (size_t)N, st));
+    TGT_HIP_CHECK(counts.alloc(sizeof(uint32_t) * (size_t)(nblocks + 2), st));
+    TGT_HIP_CHECK(bits.alloc(sizeof(uint64_t) * (size_t)nblocks * (kSubItems / 64), st));
+    int* const bad = counts.as<int>() + nblocks + 1;
+    hipLaunchKernelGGL(k_sub_fill, dim3(nblk(N)), dim3(256), 0, st, pos.as<int32_t>(), N, bad);
     if (S > 0)
         hipLaunchKernelGGL(k_sub_positions, dim3(nblk(S)), dim3(256), 0, st, d_idx, S, N, pos.as<int32_t>(),
-                           bad.as<int>());
+                           bad);
     hipLaunchKernelGGL((k_sub_compact<0>), dim3(nblocks), dim3(256), 0, st, d_ei, E, N, pos.as<int32_t>(),
-                       counts.as<uint32_t>(), bits.as<uint64_t>(), (int64_t*)nullptr, (int64_t)0, bad.as<int>());
+                       counts.as<uint32_t>(), bits.as<uint64_t>(), (int64_t*)nullptr, (int64_t)0, bad);
     hipLaunchKernelGGL(k_sub_scan, dim3(1), dim3(256), 0, st, counts.as<uint32_t>(), nblocks);
     TGT_HIP_CHECK(hipGetLastError());
-    uint32_t n_keep = 0;
-    int h_bad = 0;
-    TGT_HIP_CHECK(hipMemcpyAsync(&n_keep, counts.as<uint32_t>() + nblocks, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-    TGT_HIP_CHECK(hipMemcpyAsync(&h_bad, bad.p, sizeof(int), hipMemcpyDeviceToHost, st));
+    uint32_t back[2] = {0, 0};
+    TGT_HIP_CHECK(hipMemcpyAsync(back, counts.as<uint32_t>() + nblocks, sizeof(back), hipMemcpyDeviceToHost, st));
     TGT_HIP_CHECK(hipStreamSynchronize(st));
+    const uint32_t n_keep = back[0], h_bad = back[1];
     if (h_bad) {
         set_error("tgt_sub_edge_index: %s outside [0, %lld)", (h_bad & 1) ? "a batch node id is" : "an edge endpoint is",
                   (long long)N);
@@ -573,9 +550,8 @@ static int sub_edge_index_impl(const int64_t* d_ei, int64_t E, int64_t N, const 
     }
     if (n_keep > 0) {
         hipLaunchKernelGGL((k_sub_compact<1>), dim3(nblocks), dim3(256), 0, st, d_ei, E, N, pos.as<int32_t>(),
-                           counts.as<uint32_t>(), bits.as<uint64_t>(), d_out, capacity, bad.as<int>());
+                           counts.as<uint32_t>(), bits.as<uint64_t>(), d_out, packed ? (int64_t)n_keep : capacity, bad);
         TGT_HIP_CHECK(hipGetLastError());
-        TGT_HIP_CHECK(hipStreamSynchronize(st));      // the scratch buffers are freed on return
     }
     return TGT_OK;
 }
@@ -597,8 +573,8 @@ int tgt_fix_edge_index(const int64_t* d_edge_index, int64_t E0, int64_t num_node
     return TGT_OK;
 }
 
-int tgt_sub_edge_index(const int64_t* d_edge_index, int64_t E, int64_t N, const int64_t* d_idx_batch, int64_t S,
-                       int64_t* d_out, int64_t capacity, int64_t* h_num_edges, void* stream) {
+static int sub_edge_index_entry(const int64_t* d_edge_index, int64_t E, int64_t N, const int64_t* d_idx_batch, int64_t S, int64_t* d_out, int64_t capacity, bool packed,
+                                int64_t* h_num_edges, void* stream) {
     if (E < 0 || N < 1 || S < 0 || capacity < 0 || !h_num_edges || (E > 0 && !d_edge_index) || (S > 0 && !d_idx_batch) ||
         (capacity > 0 && !d_out)) {
         tgt::set_error("tgt_sub_edge_index: null pointer or bad size");
@@ -608,8 +584,17 @@ int tgt_sub_edge_index(const int64_t* d_edge_index, int64_t E, int64_t N, const 
         tgt::set_error("tgt_sub_edge_index: E, N and the batch size must fit 31 bits");
         return TGT_ERR_INVALID_ARG;
     }
-    return tgt::sub_edge_index_impl(d_edge_index, E, N, d_idx_batch, S, d_out, capacity, h_num_edges,
+    return tgt::sub_edge_index_impl(d_edge_index, E, N, d_idx_batch, S, d_out, capacity, packed, h_num_edges,
                                     (hipStream_t)stream);
+}
+
+int tgt_sub_edge_index(const int64_t* d_edge_index, int64_t E, int64_t N, const int64_t* d_idx_batch, int64_t S,
+                       int64_t* d_out, int64_t capacity, int64_t* h_num_edges, void* stream) {
+    return sub_edge_index_entry(d_edge_index, E, N, d_idx_batch, S, d_out, capacity, false, h_num_edges, stream);
+}
+int tgt_sub_edge_index_packed(const int64_t* d_edge_index, int64_t E, int64_t N, const int64_t* d_idx_batch, int64_t S,
+                              int64_t* d_out, int64_t capacity, int64_t* h_num_edges, void* stream) {
+    return sub_edge_index_entry(d_edge_index, E, N, d_idx_batch, S, d_out, capacity, true, h_num_edges, stream);
 }
 
 int tgt_np_legacy_randint(uint32_t seed, const int64_t* h_highs, int n, int64_t* h_out) {
@@ -652,10 +637,21 @@ int tgt_reformat_export(const tgt_reformat_t* r, int64_t* d_edge_index, int64_t*
     }
     hipStream_t st = (hipStream_t)stream;
     if (r->E_out > 0)
-        TGT_HIP_CHECK(hipMemcpyAsync(d_edge_index, r->edge_index.p, sizeof(int64_t) * 2 * r->E_out,
-                                     hipMemcpyDeviceToDevice, st));
+        hipLaunchKernelGGL(tgt::k_write_sorted, dim3(tgt::nblk(r->E_out)), dim3(256), 0, st, r->keys, r->order, r->nd.as<uint32_t>(), r->E_out, d_edge_index);
+    TGT_HIP_CHECK(hipGetLastError());
     TGT_HIP_CHECK(hipMemcpyAsync(d_sorted_indices, r->sorted_indices.p, sizeof(int64_t) * r->N,
                                  hipMemcpyDeviceToDevice, st));
+    return TGT_OK;
+}
+
+int tgt_reformat_rows(const tgt_reformat_t* r, const int64_t* d_idx_batch, int tokens, int64_t* d_rows, void* stream) {
+    if (!r || tokens < 0 || tokens > 1 || (r->N > tokens && (!d_idx_batch || !d_rows))) {
+        tgt::set_error("tgt_reformat_rows: null pointer, or tokens not 0 or 1");
+        return TGT_ERR_INVALID_ARG;
+    }
+    hipLaunchKernelGGL(tgt::k_batch_rows, dim3(tgt::nblk(r->N)), dim3(256), 0, (hipStream_t)stream, r->sorted_indices.as<int64_t>(), r->N, r->mapping.as<uint32_t>(),
+                       d_idx_batch, tokens, d_rows);
+    TGT_HIP_CHECK(hipGetLastError());
     return TGT_OK;
 }
 

@@ -17,6 +17,7 @@
 #include <utility>
 #include <algorithm>
 #include <stdlib.h>
+#include <string.h>
 
 namespace tgt {
 
@@ -45,11 +46,19 @@ __global__ void k_convert_validate(const int64_t* __restrict__ src, const int64_
     d32[i] = (uint32_t)d;
 }
 
+// The two views are made by the same launches (blockIdx.y: by destination, by source): a batch's edge list does not fill the
+// chip with one of them, and a launch costs as much host time as such a kernel runs.
+struct SideArrays {
+    const uint32_t *keys[2], *order[2], *other[2];      // sorted keys, edge of a sorted position, the edges' other endpoints
+    int32_t *rowptr[2], *col[2], *eid[2];
+};
+
 // rowptr[r] = first sorted position whose key is >= r (r = 0 .. N): one thread per row, binary
 // search in the sorted keys (a thread per position walking the gap to the next key would leave
 // all the work to one thread when the keys are few or far apart).
-__global__ void k_fill_rowptr(const uint32_t* __restrict__ keys, int64_t E, int64_t N,
-                              int32_t* __restrict__ rowptr) {
+__global__ void k_fill_rowptr(const SideArrays a, int64_t E, int64_t N) {
+    const uint32_t* __restrict__ keys = a.keys[blockIdx.y];
+    int32_t* __restrict__ rowptr = a.rowptr[blockIdx.y];
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (r > N) return;
     int64_t lo = 0, hi = E;            // answer in [lo, hi]
@@ -61,8 +70,9 @@ __global__ void k_fill_rowptr(const uint32_t* __restrict__ keys, int64_t E, int6
     rowptr[r] = (int32_t)lo;
 }
 
-__global__ void k_gather_col(const uint32_t* __restrict__ eid, const uint32_t* __restrict__ other,
-                             int64_t E, int32_t* __restrict__ col, int32_t* __restrict__ eid_out) {
+__global__ void k_gather_col(const SideArrays a, int64_t E) {
+    const uint32_t *__restrict__ eid = a.order[blockIdx.y], *__restrict__ other = a.other[blockIdx.y];
+    int32_t *__restrict__ col = a.col[blockIdx.y], *__restrict__ eid_out = a.eid[blockIdx.y];
     int64_t pos = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (pos >= E) return;
     uint32_t e = eid[pos];
@@ -88,9 +98,23 @@ __device__ __forceinline__ int sched_category(int len, int wave_row_max, bool sk
     return 4;
 }
 
+// Per side, written by the device and read back once: how many of everything the schedule holds.
+struct SchedHeader { int32_t n_wave, n_long, n_block, n_split, n_parts, n_groups, pad0, pad1; };
+struct BlockMeta;
+// What the schedule kernels read and write, of both views (blockIdx.y)
+struct SchedArgs {
+    const int32_t *rowptr[2], *col[2];
+    uint32_t *counts[2], *offs[2];
+    SchedHeader* hdr[2];
+    Item *items[2], *block_items[2];
+    int32_t *long_rows[2], *row_item_off[2], *row_split_idx[2], *row_part_off[2], *split_row[2], *split_off[2], *split_grp[2], *part2split[2];
+    BlockMeta* meta[2];
+};
+
 // counts[window * kSchedCats + cat] = rows of that category among the window's rows (blockDim.x rows)
-__global__ void k_sched_count(const int32_t* __restrict__ rowptr, int64_t N, int wave_row_max, bool skip_empty,
-                              uint32_t* __restrict__ counts) {
+__global__ void k_sched_count(const SchedArgs a, int64_t N, int wave_row_max, bool skip_empty) {
+    const int32_t* __restrict__ rowptr = a.rowptr[blockIdx.y];
+    uint32_t* __restrict__ counts = a.counts[blockIdx.y];
     __shared__ uint32_t c[kSchedCats];
     if (threadIdx.x < kSchedCats) c[threadIdx.x] = 0;
     __syncthreads();
@@ -105,13 +129,12 @@ __global__ void k_sched_count(const int32_t* __restrict__ rowptr, int64_t N, int
     if (threadIdx.x < kSchedCats) counts[(int64_t)blockIdx.x * kSchedCats + threadIdx.x] = c[threadIdx.x];
 }
 
-// Per side, written by the device and read back once: how many of everything the schedule holds.
-struct SchedHeader { int32_t n_wave, n_long, n_block, n_split, n_parts, n_groups, pad0, pad1; };
-
 // offs[window, cat]: first position of the window's rows of a category - wave classes count through
-// (window, class) in that order, long rows through the windows - and the two totals.  One workgroup.
-__global__ __launch_bounds__(1024) void k_sched_scan(const uint32_t* __restrict__ counts, int nwin,
-                                                     uint32_t* __restrict__ offs, SchedHeader* __restrict__ hdr) {
+// (window, class) in that order, long rows through the windows - and the two totals.  One workgroup per view.
+__global__ __launch_bounds__(1024) void k_sched_scan(const SchedArgs a, int nwin) {
+    const uint32_t* __restrict__ counts = a.counts[blockIdx.y];
+    uint32_t* __restrict__ offs = a.offs[blockIdx.y];
+    SchedHeader* __restrict__ hdr = a.hdr[blockIdx.y];
     __shared__ uint32_t sw[1024], sl[1024];
     const int tid = threadIdx.x;
     const int chunk = (nwin + 1023) / 1024;
@@ -141,9 +164,11 @@ __global__ __launch_bounds__(1024) void k_sched_scan(const uint32_t* __restrict_
 // Rows keep their order inside a (window, category): position = offs[window, cat] + rank among the
 // window's rows.  Wave-class rows become wave items at items[position]; long rows are listed (row, first
 // edge, length) for the kernels that cut them into workgroup items.
-__global__ void k_sched_fill(const int32_t* __restrict__ rowptr, int64_t N, int wave_row_max, bool skip_empty,
-                             const uint32_t* __restrict__ offs, Item* __restrict__ items,
-                             int32_t* __restrict__ long_rows, int64_t cap_long) {
+__global__ void k_sched_fill(const SchedArgs a, int64_t N, int wave_row_max, bool skip_empty, int64_t cap_long) {
+    const int32_t* __restrict__ rowptr = a.rowptr[blockIdx.y];
+    const uint32_t* __restrict__ offs = a.offs[blockIdx.y];
+    Item* __restrict__ items = a.items[blockIdx.y];
+    int32_t* __restrict__ long_rows = a.long_rows[blockIdx.y];
     __shared__ uint32_t wave_cnt[kSchedMaxWaves][kSchedCats];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -185,14 +210,15 @@ __host__ __device__ inline void cut_row(const CutParams& cp, int len, int& nseg,
     seg = (len + nseg - 1) / nseg;
 }
 
-// Long rows -> where their workgroup items, partial slots and combine groups start.  One workgroup: every
+// Long rows -> where their workgroup items, partial slots and combine groups start.  One workgroup per view: every
 // thread takes a run of consecutive rows of the list (it is short: rows of more than a wave row's edges), the
 // runs' totals are scanned in LDS, then every thread writes its rows.
-__global__ __launch_bounds__(1024) void k_cut_rows(const int32_t* __restrict__ long_rows, SchedHeader* __restrict__ hdr,
-                                                   CutParams cp, int32_t* __restrict__ row_item_off,
-                                                   int32_t* __restrict__ row_split_idx, int32_t* __restrict__ row_part_off,
-                                                   int32_t* __restrict__ split_row, int32_t* __restrict__ split_off,
-                                                   int32_t* __restrict__ split_grp) {
+__global__ __launch_bounds__(1024) void k_cut_rows(const SchedArgs a, CutParams cp) {
+    const int32_t* __restrict__ long_rows = a.long_rows[blockIdx.y];
+    SchedHeader* __restrict__ hdr = a.hdr[blockIdx.y];
+    int32_t *__restrict__ row_item_off = a.row_item_off[blockIdx.y], *__restrict__ row_split_idx = a.row_split_idx[blockIdx.y],
+            *__restrict__ row_part_off = a.row_part_off[blockIdx.y], *__restrict__ split_row = a.split_row[blockIdx.y],
+            *__restrict__ split_off = a.split_off[blockIdx.y], *__restrict__ split_grp = a.split_grp[blockIdx.y];
     __shared__ uint32_t sh[4][1024];
     const int n_long = hdr->n_long;
     const int tid = threadIdx.x;
@@ -255,11 +281,14 @@ __global__ __launch_bounds__(1024) void k_cut_rows(const int32_t* __restrict__ l
 struct BlockMeta { int32_t home, len, spread; };
 
 // One thread per workgroup item: finds its row in the offsets and writes the item.
-__global__ void k_emit_items(const int32_t* __restrict__ long_rows, const SchedHeader* __restrict__ hdr, CutParams cp,
-                             const int32_t* __restrict__ row_item_off, const int32_t* __restrict__ row_split_idx,
-                             const int32_t* __restrict__ row_part_off, const int32_t* __restrict__ col,
-                             Item* __restrict__ block_items, BlockMeta* __restrict__ meta,
-                             int32_t* __restrict__ part2split) {
+__global__ void k_emit_items(const SchedArgs a, CutParams cp) {
+    const int32_t* __restrict__ long_rows = a.long_rows[blockIdx.y];
+    const SchedHeader* __restrict__ hdr = a.hdr[blockIdx.y];
+    const int32_t *__restrict__ row_item_off = a.row_item_off[blockIdx.y], *__restrict__ row_split_idx = a.row_split_idx[blockIdx.y],
+                  *__restrict__ row_part_off = a.row_part_off[blockIdx.y], *__restrict__ col = a.col[blockIdx.y];
+    Item* __restrict__ block_items = a.block_items[blockIdx.y];
+    BlockMeta* __restrict__ meta = a.meta[blockIdx.y];
+    int32_t* __restrict__ part2split = a.part2split[blockIdx.y];
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= hdr->n_block) return;
     int lo = 0, hi = hdr->n_long - 1;               // last row whose first item is <= j
@@ -282,35 +311,48 @@ __global__ void k_emit_items(const int32_t* __restrict__ long_rows, const SchedH
     if (part >= 0) part2split[part] = sidx;
 }
 
-// A run: `waves` consecutive waves of the list of XCD `xcd` that do the same kind of thing.
+// A run: consecutive waves of the list of one XCD that do the same kind of thing, from wave `wave0` of the list.
 //   rows:       the wave items [first, first + n) of one (window, class), rows_per_wave of them per wave
 //   block item: workgroup item `first`; its four waves carry the same record
-//   nothing:    padding to whole workgroups, and behind the end of a list
-struct Run { int32_t wave0, waves, first, n; uint32_t code; int32_t xcd; int32_t pad[2]; };
+//   nothing:    padding to whole workgroups, and behind the end of a list; n waves
+// code: descriptor code (kind, view), the XCD in bits 8 .. 10, bit 11: of the backward's launch.
+struct Run { int32_t wave0, first, n; uint32_t code; };
+constexpr uint32_t kRunBackward = 1u << 11;
+__host__ __device__ inline int32_t run_waves(uint32_t kind, int32_t n, int lpe) {
+    if (kind == kDescBlock) return 4;
+    if (kind == kDescNone) return n;
+    const int ipw = rows_per_wave(lpe, (int)kind);
+    return (n + ipw - 1) / ipw;
+}
 
-// One workgroup per run; its waves write the run's wave records in turn (layout: WaveRec in common.h).  Wave lw of
+// One workgroup per run, for the forward's and the backward's launch together; its sixteen waves write the run's wave records
+// in turn (layout: WaveRec in common.h), the lanes of a wave one edge or bias row each.  Wave lw of
 // XCD x's list is wave lw % 4 of that XCD's (lw / 4)-th workgroup, and workgroup b of the launch runs on XCD b mod 8:
 // record ((lw / 4) * 8 + x) * 4 + lw % 4.  Everything a kernel uses of a record is written: no clearing pass.
-__global__ __launch_bounds__(256) void k_build_records(const Run* __restrict__ runs, const Item* __restrict__ items_d,
+// Bound by the two dependent reads (item, edges) of a record; 390 K edges: 27 us for each of the two launches with four waves
+// per run and eight lanes at work.
+constexpr int kRecordWaves = 16;
+__global__ __launch_bounds__(64 * kRecordWaves) void k_build_records(const Run* __restrict__ runs, const Item* __restrict__ items_d,
                                                        const Item* __restrict__ items_s, const Item* __restrict__ bitems_d,
                                                        const Item* __restrict__ bitems_s, const int32_t* __restrict__ col_d,
                                                        const int32_t* __restrict__ eid_d, const int32_t* __restrict__ col_s,
                                                        const int32_t* __restrict__ eid_s, WaveRecLayout L, int lpe,
-                                                       int32_t* __restrict__ recs) {
+                                                       int32_t* __restrict__ recs_fwd, int32_t* __restrict__ recs_bwd) {
     const Run run = runs[blockIdx.x];
     const int t = threadIdx.x & 63;
-    const uint32_t kind = run.code & 7u;
+    const uint32_t kind = run.code & 7u, xcd = (run.code >> 8) & 7u;
     const bool src = (run.code & kDescSrcSide) != 0;
     const Item* items = src ? items_s : items_d;
     const int32_t* col = src ? col_s : col_d;
     const int32_t* eid = src ? eid_s : eid_d;
+    int32_t* const recs = run.code & kRunBackward ? recs_bwd : recs_fwd;
     const int ipw = kind < (uint32_t)kNumClass ? rows_per_wave(lpe, (int)kind) : 1;
     const int S = kind < (uint32_t)kNumClass ? slots_for_class(lpe, (int)kind) : 1;
     const bool inl = kind < (uint32_t)kNumClass && class_inline(lpe, (int)kind);
-    const int groups = kWave / lpe;
-    for (int w = threadIdx.x >> 6; w < run.waves; w += 4) {
+    const int groups = kWave / lpe, waves = run_waves(kind, run.n, lpe);
+    for (int w = threadIdx.x >> 6; w < waves; w += kRecordWaves) {
         const int lw = run.wave0 + w;
-        int32_t* out = recs + (((int64_t)(lw >> 2) * 8 + run.xcd) * 4 + (lw & 3)) * L.stride;
+        int32_t* out = recs + (((int64_t)(lw >> 2) * 8 + xcd) * 4 + (lw & 3)) * L.stride;
         if (kind == kDescNone) {
             if (t == 0) out[0] = (int32_t)kDescNone;
             continue;
@@ -318,7 +360,7 @@ __global__ __launch_bounds__(256) void k_build_records(const Run* __restrict__ r
         if (kind == kDescBlock) {
             if (t == 0) {
                 const Item it = (src ? bitems_s : bitems_d)[run.first];
-                out[0] = (int32_t)run.code;
+                out[0] = (int32_t)desc_code(kDescBlock, src, 0);
                 out[4] = it.row; out[5] = it.start; out[6] = it.len; out[7] = it.part;
             }
             continue;
@@ -327,18 +369,20 @@ __global__ __launch_bounds__(256) void k_build_records(const Run* __restrict__ r
         const int count = min(ipw, run.n - w * ipw);
         if (t == 0) out[0] = (int32_t)desc_code(kind, src, (uint32_t)count);
         if (t < groups) {                               // every lane group's entries, zeros behind the last row
-            const int i = t / S, sl = t % S;
+            const int i = t / S;
             Item it{0, 0, 0, -1};
             if (i < count) it = items[first + i];
             out[L.off_row + t] = it.row;                // per lane group: a lane finds its row without knowing the class
             out[L.off_start + t] = it.start;
             out[L.off_len + t] = it.len;
-            if (inl) for (int u = 0; u < 4; ++u) {
-                const int e = sl + u * S;
-                const int ec = e < it.len ? e : it.len - 1;
-                out[L.off_col + 4 * t + u] = it.len > 0 ? col[it.start + ec] : 0;
-                out[L.off_eid + 4 * t + u] = it.len > 0 ? eid[it.start + ec] : 0;
-            }
+        }
+        if (inl) for (int k = t; k < 4 * groups; k += 64) {      // entry k: edge k % 4 of lane group k / 4
+            const int g = k >> 2, i = g / S;
+            Item it{0, 0, 0, -1};
+            if (i < count) it = items[first + i];
+            const int e = g % S + (k & 3) * S, ec = e < it.len ? e : it.len - 1;
+            out[L.off_col + k] = it.len > 0 ? col[it.start + ec] : 0;
+            out[L.off_eid + k] = it.len > 0 ? eid[it.start + ec] : 0;
         }
     }
 }
@@ -346,21 +390,22 @@ __global__ __launch_bounds__(256) void k_build_records(const Run* __restrict__ r
 // ---------------------------------------------------------------------------
 // host helpers
 // ---------------------------------------------------------------------------
-// Sort edge ids by `keys32` (stable) and fill one Side's rowptr / col / eid.
-static int build_side(const uint32_t* keys32, const uint32_t* other32, int64_t E, int64_t N,
-                      RadixSorter& sorter, Side& side, hipStream_t st) {
-    const uint32_t* kin = keys32;
-    const uint32_t* vin = nullptr;
+// Sort edge ids by destination and by source (stable) and fill both views' rowptr / col / eid.
+static int build_sides(const uint32_t* d32, const uint32_t* s32, int64_t E, int64_t N, RadixSorter& sorter, Side& dst, Side& src, hipStream_t st) {
+    SideArrays a{};
+    a.keys[0] = d32; a.keys[1] = s32;
+    a.other[0] = s32; a.other[1] = d32;
+    a.rowptr[0] = dst.rowptr; a.rowptr[1] = src.rowptr;
+    a.col[0] = dst.col; a.col[1] = src.col;
+    a.eid[0] = dst.eid; a.eid[1] = src.eid;
     if (E > 0) {
-        int rc = sorter.sort(keys32, nullptr, E, bits_for(N), st, &kin, &vin);
+        const uint32_t* in[2] = {d32, s32};
+        int rc = sorter.sort(in, nullptr, 2, E, bits_for(N), st, a.keys, a.order);
         if (rc) return rc;
     }
     const int T = 256;
-    hipLaunchKernelGGL(k_fill_rowptr, dim3((unsigned)((N + 1 + T - 1) / T)), dim3(T), 0, st, kin, E, N,
-                       side.rowptr);
-    if (E > 0)
-        hipLaunchKernelGGL(k_gather_col, dim3((unsigned)((E + T - 1) / T)), dim3(T), 0, st, vin, other32,
-                           E, side.col, side.eid);
+    hipLaunchKernelGGL(k_fill_rowptr, dim3((unsigned)((N + 1 + T - 1) / T), 2), dim3(T), 0, st, a, E, N);
+    if (E > 0) hipLaunchKernelGGL(k_gather_col, dim3((unsigned)((E + T - 1) / T), 2), dim3(T), 0, st, a, E);
     TGT_HIP_CHECK(hipGetLastError());
     return TGT_OK;
 }
@@ -388,58 +433,65 @@ static int window_rows() {
 // both views, together with the range-check flag) and, if there are long rows, what it needs to place
 // their workgroup items.
 struct SideScratch {
-    DevBuf long_rows, row_item_off, row_split_idx, row_part_off, meta;
+    DevBuf rows;      // rows: per long row (row, first edge, length), its first split, partial slot and item
     int64_t cap_long = 0, cap_block = 0;
     CutParams cp{};
     int wave_row_max = 0, W = 0, nwin = 0;
 };
 
+// bounds known before anything is counted: a long row has more than wave_row_max edges, a row of len edges
+// is cut into at most len / min(block_seg, spread_seg) + 1 segments
+static int64_t cap_long_rows(int64_t N, int64_t E) { return std::min<int64_t>(N, E / (env_int("TGT_WAVE_ROW_MAX", tgt::kWaveRowMax) + 1)) + 1; }
+static int64_t cap_block_items(int64_t N, int64_t E) {
+    return E / std::max(1, std::min(env_int("TGT_BLOCK_SEG", tgt::kBlockSeg), env_int("TGT_SPREAD_SEG", tgt::kSpreadSeg))) + cap_long_rows(N, E) + 1;
+}
+
 // ints of the report in front of the per-window counts: two headers, the flag, padding
 constexpr int kReportHead = 32;
 constexpr int kReportFlag = 16;
+constexpr size_t kOneCopyBytes = 256 << 10;
 
-static int schedule_device(int64_t N, int64_t E, Side& side, SideScratch& sc, int32_t* report, int side_idx,
-                           bool skip_empty, hipStream_t st) {
-    // tuning overrides (experiments only; the defaults are the measured best)
-    sc.wave_row_max = env_int("TGT_WAVE_ROW_MAX", tgt::kWaveRowMax);
-    sc.cp.block_seg = env_int("TGT_BLOCK_SEG", tgt::kBlockSeg);
-    sc.cp.spread_seg = env_int("TGT_SPREAD_SEG", tgt::kSpreadSeg);
-    sc.cp.spread_segs = kSpreadSegs;
-    sc.cp.combine_fan = kCombineFan;
-    sc.W = window_rows();
-    sc.cp.window = sc.W;
-    sc.nwin = (int)((N + sc.W - 1) / sc.W);
-    side.n_windows = sc.nwin;
-    const size_t ncnt = (size_t)kSchedCats * sc.nwin;
-    SchedHeader* hdr = reinterpret_cast<SchedHeader*>(report) + side_idx;
-    uint32_t* counts = reinterpret_cast<uint32_t*>(report) + kReportHead + (size_t)side_idx * 2 * ncnt;
-    uint32_t* offs = counts + ncnt;
-    // bounds known before anything is counted: a long row has more than wave_row_max edges, a row of len edges
-    // is cut into at most len / min(block_seg, spread_seg) + 1 segments
-    sc.cap_long = std::min<int64_t>(N, E / (sc.wave_row_max + 1)) + 1;
-    const int min_seg = std::max(1, std::min(sc.cp.block_seg, sc.cp.spread_seg));
-    sc.cap_block = E / min_seg + sc.cap_long + 1;
-    TGT_HIP_CHECK(dev_alloc((void**)&side.items, sizeof(Item) * (size_t)(N + 1), st));
-    TGT_HIP_CHECK(dev_alloc((void**)&side.block_items, sizeof(Item) * (size_t)sc.cap_block, st));
-    TGT_HIP_CHECK(dev_alloc((void**)&side.split_row, sizeof(int32_t) * (size_t)(sc.cap_long + 1), st));
-    TGT_HIP_CHECK(dev_alloc((void**)&side.split_off, sizeof(int32_t) * (size_t)(sc.cap_long + 1), st));
-    TGT_HIP_CHECK(dev_alloc((void**)&side.split_grp, sizeof(int32_t) * (size_t)(sc.cap_long + 1), st));
-    TGT_HIP_CHECK(dev_alloc((void**)&side.part2split, sizeof(int32_t) * (size_t)(sc.cap_block + 1), st));
-    TGT_HIP_CHECK(sc.long_rows.alloc(sizeof(int32_t) * 3 * (size_t)sc.cap_long, st));
-    TGT_HIP_CHECK(sc.row_item_off.alloc(sizeof(int32_t) * (size_t)(sc.cap_long + 1), st));
-    TGT_HIP_CHECK(sc.row_split_idx.alloc(sizeof(int32_t) * (size_t)sc.cap_long, st));
-    TGT_HIP_CHECK(sc.row_part_off.alloc(sizeof(int32_t) * (size_t)sc.cap_long, st));
-    TGT_HIP_CHECK(sc.meta.alloc(sizeof(BlockMeta) * (size_t)sc.cap_block, st));
-    hipLaunchKernelGGL(k_sched_count, dim3(sc.nwin), dim3(sc.W), 0, st, side.rowptr, N, sc.wave_row_max, skip_empty, counts);
-    hipLaunchKernelGGL(k_sched_scan, dim3(1), dim3(1024), 0, st, counts, sc.nwin, offs, hdr);
-    hipLaunchKernelGGL(k_sched_fill, dim3(sc.nwin), dim3(sc.W), 0, st, side.rowptr, N, sc.wave_row_max, skip_empty, offs, side.items,
-                       sc.long_rows.as<int32_t>(), sc.cap_long);
-    hipLaunchKernelGGL(k_cut_rows, dim3(1), dim3(1024), 0, st, sc.long_rows.as<int32_t>(), hdr, sc.cp,
-                       sc.row_item_off.as<int32_t>(), sc.row_split_idx.as<int32_t>(), sc.row_part_off.as<int32_t>(),
-                       side.split_row, side.split_off, side.split_grp);
-    hipLaunchKernelGGL(k_emit_items, dim3((unsigned)((sc.cap_block + 255) / 256)), dim3(256), 0, st, sc.long_rows.as<int32_t>(),
-                       hdr, sc.cp, sc.row_item_off.as<int32_t>(), sc.row_split_idx.as<int32_t>(), sc.row_part_off.as<int32_t>(),
-                       side.col, side.block_items, sc.meta.as<BlockMeta>(), side.part2split);
+static int schedule_device(int64_t N, int64_t E, Side* const (&sides)[2], SideScratch (&scr)[2], int32_t* report, BlockMeta* metas, bool skip_empty,
+                           hipStream_t st) {
+    SchedArgs a{};
+    for (int i = 0; i < 2; ++i) {
+        Side& side = *sides[i];
+        SideScratch& sc = scr[i];
+        // tuning overrides (experiments only; the defaults are the measured best)
+        sc.wave_row_max = env_int("TGT_WAVE_ROW_MAX", tgt::kWaveRowMax);
+        sc.cp.block_seg = env_int("TGT_BLOCK_SEG", tgt::kBlockSeg);
+        sc.cp.spread_seg = env_int("TGT_SPREAD_SEG", tgt::kSpreadSeg);
+        sc.cp.spread_segs = kSpreadSegs;
+        sc.cp.combine_fan = kCombineFan;
+        sc.W = window_rows();
+        sc.cp.window = sc.W;
+        sc.nwin = (int)((N + sc.W - 1) / sc.W);
+        side.n_windows = sc.nwin;
+        const size_t ncnt = (size_t)kSchedCats * sc.nwin;
+        a.hdr[i] = reinterpret_cast<SchedHeader*>(report) + i;
+        a.counts[i] = reinterpret_cast<uint32_t*>(report) + kReportHead + (size_t)i * 2 * ncnt;
+        a.offs[i] = a.counts[i] + ncnt;
+        sc.cap_long = cap_long_rows(N, E);
+        sc.cap_block = cap_block_items(N, E);
+        TGT_HIP_CHECK(dev_alloc((void**)&side.items, sizeof(Item) * (size_t)(N + 1), st));
+        TGT_HIP_CHECK(dev_alloc((void**)&side.block_items, sizeof(Item) * (size_t)sc.cap_block, st));
+        TGT_HIP_CHECK(dev_alloc((void**)&side.split_row, sizeof(int32_t) * (size_t)(sc.cap_long + 1), st));
+        TGT_HIP_CHECK(dev_alloc((void**)&side.split_off, sizeof(int32_t) * (size_t)(sc.cap_long + 1), st));
+        TGT_HIP_CHECK(dev_alloc((void**)&side.split_grp, sizeof(int32_t) * (size_t)(sc.cap_long + 1), st));
+        TGT_HIP_CHECK(dev_alloc((void**)&side.part2split, sizeof(int32_t) * (size_t)(sc.cap_block + 1), st));
+        TGT_HIP_CHECK(sc.rows.alloc(sizeof(int32_t) * (6 * (size_t)sc.cap_long + 1), st));
+        a.rowptr[i] = side.rowptr; a.col[i] = side.col; a.items[i] = side.items; a.block_items[i] = side.block_items;
+        a.long_rows[i] = sc.rows.as<int32_t>();
+        a.row_split_idx[i] = a.long_rows[i] + 3 * sc.cap_long; a.row_part_off[i] = a.row_split_idx[i] + sc.cap_long; a.row_item_off[i] = a.row_part_off[i] + sc.cap_long;
+        a.split_row[i] = side.split_row; a.split_off[i] = side.split_off; a.split_grp[i] = side.split_grp; a.part2split[i] = side.part2split;
+        a.meta[i] = metas + i * sc.cap_block;
+    }
+    const SideScratch& sc = scr[0];      // (sizes and parameters are the same)
+    hipLaunchKernelGGL(k_sched_count, dim3(sc.nwin, 2), dim3(sc.W), 0, st, a, N, sc.wave_row_max, skip_empty);
+    hipLaunchKernelGGL(k_sched_scan, dim3(1, 2), dim3(1024), 0, st, a, sc.nwin);
+    hipLaunchKernelGGL(k_sched_fill, dim3(sc.nwin, 2), dim3(sc.W), 0, st, a, N, sc.wave_row_max, skip_empty, sc.cap_long);
+    hipLaunchKernelGGL(k_cut_rows, dim3(1, 2), dim3(1024), 0, st, a, sc.cp);
+    hipLaunchKernelGGL(k_emit_items, dim3((unsigned)((sc.cap_block + 255) / 256), 2), dim3(256), 0, st, a, sc.cp);
     TGT_HIP_CHECK(hipGetLastError());
     return TGT_OK;
 }
@@ -468,48 +520,56 @@ static void schedule_counts(Side& side, const SideScratch& sc, const int32_t* re
 // load (their own q/k/v/dout rows, the rows of their self-loops, the window's share of a global node's
 // segment) then meets in one L2 at about the same time.
 namespace {
+// Waves of n rows of a class (rows per wave are powers of two)
+struct WaveShift {
+    int sh[kNumClass];
+    explicit WaveShift(int lpe) {
+        for (int c = 0; c < kNumClass; ++c) { sh[c] = 0; while ((1 << sh[c]) < rows_per_wave(lpe, c)) ++sh[c]; }
+    }
+    int32_t waves(int c, int64_t n) const { return (int32_t)((n + (1 << sh[c]) - 1) >> sh[c]); }
+};
 // One XCD's list as runs of waves.
 struct XcdList {
     std::vector<Run> runs;
-    int32_t waves = 0, xcd = 0;
-    void add(uint32_t code, int32_t first, int32_t n, int32_t waves_of_run) {
-        if (waves_of_run <= 0) return;
-        runs.push_back(Run{waves, waves_of_run, first, n, code, xcd, {0, 0}});
-        waves += waves_of_run;
+    int32_t waves = 0;
+    const WaveShift* ws = nullptr;
+    uint32_t where = 0;      // the list's bits of a run's code
+    void add(uint32_t code, int32_t first, int32_t n) {
+        if (n <= 0) return;
+        runs.push_back(Run{waves, first, n, code | where});
+        const uint32_t kind = code & 7u;
+        waves += kind == kDescBlock ? 4 : (kind == kDescNone ? n : ws->waves((int)kind, n));
     }
-    void pad4() { if (waves % 4) add(kDescNone, 0, 0, 4 - waves % 4); }
+    void pad4() { if (waves % 4) add(kDescNone, 0, 4 - waves % 4); }
 };
 
 // Workgroup items homed at window w_items and the waves of window w of one view (either may be -1: none), appended
 // to the list.  part 0: the heavy share (segments of ordinary long rows and the rows of the longest class, which
 // run for many steps and whose edges have no tie to the window), part 1: the rest (segments of a row that
 // spans the graph, which gather exactly the window's rows, and the short rows).
-void append_side(XcdList& xl, const Side& s, int w, int w_items, int lpe, bool src_side, int part) {
+void append_side(XcdList& xl, const Side& s, int w, int w_items, bool src_side, int part) {
     if (w_items >= 0) {
         for (int32_t q = s.homed_off[w_items]; q < s.homed_off[w_items + 1]; ++q) {
             const int32_t it = s.homed_idx[q];
             if ((s.block_spread[it] != 0) != (part == 1)) continue;
             xl.pad4();      // close a partly filled workgroup first: a workgroup item takes all four waves
-            xl.add(desc_code(kDescBlock, src_side, 0), it, 1, 4);
+            xl.add(desc_code(kDescBlock, src_side, 0), it, 1);
         }
     }
     if (w < 0) return;
     for (int c = (part == 0 ? 0 : 1); c < (part == 0 ? 1 : kNumClass); ++c) {
         const uint32_t n = s.win_class_cnt[(size_t)w * (kNumClass + 1) + c];
-        const int ipw = rows_per_wave(lpe, c);
-        xl.add(desc_code((uint32_t)c, src_side, 0), (int32_t)s.win_class_off[(size_t)w * (kNumClass + 1) + c], (int32_t)n,
-               (int32_t)((n + ipw - 1) / ipw));
+        xl.add(desc_code((uint32_t)c, src_side, 0), (int32_t)s.win_class_off[(size_t)w * (kNumClass + 1) + c], (int32_t)n);
     }
 }
 
 // runs of all windows -> block order.  XCD x gets a contiguous range of windows; it first walks the
 // heavy share of all its windows (long work first keeps the end of the launch short), then window by window.
-// The host vectors and device buffers handed back feed an asynchronous copy and the kernel behind it: the caller
-// keeps them until the stream has been synchronised.
-int place(const std::vector<const Side*>& sides, int lpe, void** d_out, int32_t* n_blocks, hipStream_t st,
-          std::vector<Run>& all_runs, DevBuf& runs_d) {
+// Appends one launch's runs to `all_runs`.
+void place(const std::vector<const Side*>& sides, int lpe, bool backward, int32_t* n_blocks, std::vector<Run>& all_runs) {
     const int nwin = sides[0]->n_windows;
     const bool heavy_first = env_int("TGT_HEAVY_FIRST", 1) == 1;
+    const WaveShift shift(lpe);
     // 8 contiguous window ranges with about equal numbers of edges and rows
     int bound[9];
     bound[0] = 0;
@@ -521,8 +581,7 @@ int place(const std::vector<const Side*>& sides, int lpe, void** d_out, int32_t*
                 const Side* sd = sides[k];
                 for (int32_t q = sd->homed_off[w]; q < sd->homed_off[w + 1]; ++q) c += 1.0 + sd->block_len[sd->homed_idx[q]] / 128.0;
                 for (int kk = 0; kk < kNumClass; ++kk)
-                    c += (kk == 0 ? 0.75 : 0.25) * ((sd->win_class_cnt[(size_t)w * (kNumClass + 1) + kk] + rows_per_wave(lpe, kk) - 1) /
-                                                    rows_per_wave(lpe, kk));
+                    c += (kk == 0 ? 0.75 : 0.25) * shift.waves(kk, sd->win_class_cnt[(size_t)w * (kNumClass + 1) + kk]);
             }
             cost[w + 1] = cost[w] + c;
         }
@@ -535,11 +594,12 @@ int place(const std::vector<const Side*>& sides, int lpe, void** d_out, int32_t*
     // part 1 the segments homed at a window run `lead` windows ahead of the window's rows: close enough in
     // time for the rows to meet in the L2, and the last windows of a range end with short rows only - the
     // chain of a split row (partial slot, arrival, sums of the group and of the row) is not left for the end.
-    const int lead = env_int("TGT_SEGMENT_LEAD", 3);
+    const int lead = env_int("TGT_SEGMENT_LEAD", 3), early_share = env_int("TGT_EARLY_SHARE", 2);
     XcdList xl[8];
     for (int x = 0; x < 8; ++x) {
         XcdList& wv = xl[x];
-        wv.xcd = x;
+        wv.ws = &shift;
+        wv.where = ((uint32_t)x << 8) | (backward ? kRunBackward : 0u);
         wv.runs.reserve((size_t)(bound[x + 1] - bound[x] + 8) * 8 * sides.size());
         const int w0 = bound[x], w1 = bound[x + 1];
         if (heavy_first) {
@@ -547,43 +607,44 @@ int place(const std::vector<const Side*>& sides, int lpe, void** d_out, int32_t*
             // view q, dout and the per-node scalars; side by side the two sets compete for the L2 (870 K nodes with
             // 50 edges per row: 3 % faster one after the other; no difference where long rows are few)
             for (size_t k = 0; k < sides.size(); ++k)
-                for (int w = w0; w < w1; ++w) append_side(wv, *sides[k], w, w, lpe, k == 1, 0);
+                for (int w = w0; w < w1; ++w) append_side(wv, *sides[k], w, w, k == 1, 0);
             wv.pad4();
         }
         // the segments of the last half of the range go first: when the launch ends no split row is still
         // being added up (those windows give up meeting their segment in the L2)
-        const int w_early = w1 - (w1 - w0) / env_int("TGT_EARLY_SHARE", 2);
+        const int w_early = w1 - (w1 - w0) / early_share;
         for (int w = w_early; w < w1; ++w)
-            for (size_t k = 0; k < sides.size(); ++k) append_side(wv, *sides[k], -1, w, lpe, k == 1, 1);
+            for (size_t k = 0; k < sides.size(); ++k) append_side(wv, *sides[k], -1, w, k == 1, 1);
         for (int w = w0 - lead; w < w1; ++w) {
             const int wi = w + lead < w_early ? w + lead : -1;        // segments of the window `lead` ahead
             for (size_t k = 0; k < sides.size(); ++k) {
-                if (!heavy_first) append_side(wv, *sides[k], w >= w0 ? w : -1, w >= w0 ? w : -1, lpe, k == 1, 0);
-                append_side(wv, *sides[k], w >= w0 ? w : -1, wi >= w0 ? wi : -1, lpe, k == 1, 1);
+                if (!heavy_first) append_side(wv, *sides[k], w >= w0 ? w : -1, w >= w0 ? w : -1, k == 1, 0);
+                append_side(wv, *sides[k], w >= w0 ? w : -1, wi >= w0 ? wi : -1, k == 1, 1);
             }
             wv.pad4();
         }
     }
     int32_t per = 0;
     for (int x = 0; x < 8; ++x) per = std::max(per, (xl[x].waves + 3) / 4);
-    const size_t nb = (size_t)per * 8;
-    const WaveRecLayout L(lpe);
-    const size_t n_rec = nb * 4;
-    *n_blocks = (int32_t)nb;
-    if (n_rec == 0) return TGT_OK;
-    all_runs.clear();
+    *n_blocks = per * 8;
     for (int x = 0; x < 8; ++x) {
-        xl[x].add(kDescNone, 0, 0, per * 4 - xl[x].waves);       // behind the end of the list: records that say "nothing"
+        xl[x].add(kDescNone, 0, per * 4 - xl[x].waves);       // behind the end of the list: records that say "nothing"
         all_runs.insert(all_runs.end(), xl[x].runs.begin(), xl[x].runs.end());
     }
-    TGT_HIP_CHECK(runs_d.alloc(sizeof(Run) * all_runs.size(), st));
-    TGT_HIP_CHECK(hipMemcpyAsync(runs_d.p, all_runs.data(), sizeof(Run) * all_runs.size(), hipMemcpyHostToDevice, st));
-    const size_t bytes = n_rec * (size_t)L.stride * sizeof(int32_t);
-    TGT_HIP_CHECK(dev_alloc(d_out, bytes, st));
-    const Side* sd = sides[0];
-    const Side* ss = sides.size() > 1 ? sides[1] : sides[0];
-    hipLaunchKernelGGL(k_build_records, dim3((unsigned)all_runs.size()), dim3(256), 0, st, runs_d.as<Run>(), sd->items, ss->items,
-                       sd->block_items, ss->block_items, sd->col, sd->eid, ss->col, ss->eid, L, lpe, static_cast<int32_t*>(*d_out));
+}
+
+// The records of both launches.  `runs` feeds an asynchronous copy: it lives until the stream has been synchronised.
+int build_records(const tgt_plan* plan, int lpe, Schedule& sc, const std::vector<Run>& runs, DevBuf& runs_d, hipStream_t st) {
+    const WaveRecLayout L(lpe);
+    const size_t rec = (size_t)L.stride * sizeof(int32_t) * 4;
+    if (runs.empty()) return TGT_OK;
+    TGT_HIP_CHECK(runs_d.alloc(sizeof(Run) * runs.size(), st));
+    TGT_HIP_CHECK(hipMemcpyAsync(runs_d.p, runs.data(), sizeof(Run) * runs.size(), hipMemcpyHostToDevice, st));
+    if (sc.fwd_blocks) TGT_HIP_CHECK(dev_alloc(&sc.fwd, rec * sc.fwd_blocks, st));
+    if (sc.bwd_blocks) TGT_HIP_CHECK(dev_alloc(&sc.bwd, rec * sc.bwd_blocks, st));
+    const Side &d = plan->dst, &s = plan->src;
+    hipLaunchKernelGGL(k_build_records, dim3((unsigned)runs.size()), dim3(64 * kRecordWaves), 0, st, runs_d.as<Run>(), d.items, s.items, d.block_items, s.block_items, d.col,
+                       d.eid, s.col, s.eid, L, lpe, static_cast<int32_t*>(sc.fwd), static_cast<int32_t*>(sc.bwd));
     TGT_HIP_CHECK(hipGetLastError());
     return TGT_OK;
 }
@@ -604,11 +665,12 @@ const Schedule* plan_schedule(const tgt_plan* plan_c, int lpe, hipStream_t st) {
     // the descriptors of a shape are made once, whichever thread or stream asks first
     std::lock_guard<std::mutex> lock(plan->sched_mutex);
     if (sc.ready) return &sc;
-    std::vector<Run> runs_f, runs_b;
-    DevBuf rf, rb;
-    int rc = place({&plan->dst}, lpe, &sc.fwd, &sc.fwd_blocks, st, runs_f, rf);
-    if (rc == TGT_OK) rc = place({&plan->dst, &plan->src}, lpe, &sc.bwd, &sc.bwd_blocks, st, runs_b, rb);
-    // the host vectors feed asynchronous copies: they may go once the stream is idle
+    std::vector<Run> runs;
+    DevBuf runs_d;
+    place({&plan->dst}, lpe, false, &sc.fwd_blocks, runs);
+    place({&plan->dst, &plan->src}, lpe, true, &sc.bwd_blocks, runs);
+    int rc = build_records(plan, lpe, sc, runs, runs_d, st);
+    // the host vector feeds an asynchronous copy: it may go once the stream is idle
     if (hipStreamSynchronize(st) != hipSuccess && rc == TGT_OK) { set_error("hipStreamSynchronize failed"); rc = TGT_ERR_HIP; }
     if (rc != TGT_OK) {
         dev_free(sc.fwd); dev_free(sc.bwd);
@@ -679,15 +741,18 @@ static int create_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, in
     TGT_HIP_CHECK(s32.alloc(eb, st));
     TGT_HIP_CHECK(d32.alloc(eb, st));
     {
-        int rc0 = sorter.init(E, st);
+        int rc0 = sorter.init(E, st, 2);
         if (rc0) return rc0;
     }
-    // what comes back to the host, in one copy: the two schedule headers, the range-check flag, and per view the
-    // per-window row counts and their offsets
+    // what comes back to the host, in one copy: the two schedule headers, the range-check flag, per view the
+    // per-window row counts and their offsets, and where the workgroup items go if there is room for few of them (else that
+    // is a second copy, of the items there are)
     const int W = window_rows();
     const int nwin = (int)((N + W - 1) / W);
     const size_t report_ints = kReportHead + 4 * (size_t)kSchedCats * nwin;
-    TGT_HIP_CHECK(report_d.alloc(sizeof(int32_t) * report_ints, st));
+    const size_t cap_meta = (size_t)cap_block_items(N, E), meta_bytes = 2 * sizeof(BlockMeta) * cap_meta;
+    const bool one_copy = meta_bytes <= kOneCopyBytes;
+    TGT_HIP_CHECK(report_d.alloc(sizeof(int32_t) * report_ints + meta_bytes, st));
     TGT_HIP_CHECK(hipMemsetAsync(report_d.p, 0, sizeof(int32_t) * kReportHead, st));
     int32_t* report = report_d.as<int32_t>();
     if (E > 0) {
@@ -697,32 +762,32 @@ static int create_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, in
         TGT_HIP_CHECK(hipGetLastError());
     }
     // out-of-range endpoints were replaced by node 0 (and flagged): everything below runs on valid ids
-    int rc = build_side(d32.as<uint32_t>(), s32.as<uint32_t>(), E, N, sorter, plan->dst, st);
+    int rc = build_sides(d32.as<uint32_t>(), s32.as<uint32_t>(), E, N, sorter, plan->dst, plan->src, st);
     if (rc) return rc;
-    rc = build_side(s32.as<uint32_t>(), d32.as<uint32_t>(), E, N, sorter, plan->src, st);
+    SideScratch scr[2];
+    Side* const views[2] = {&plan->dst, &plan->src};
+    BlockMeta* const metas = reinterpret_cast<BlockMeta*>(report + report_ints);
+    rc = schedule_device(N, E, views, scr, report, metas, plan->rows_with_edges_only, st);
     if (rc) return rc;
-    SideScratch scr_d, scr_s;
-    rc = schedule_device(N, E, plan->dst, scr_d, report, 0, plan->rows_with_edges_only, st);
-    if (rc) return rc;
-    rc = schedule_device(N, E, plan->src, scr_s, report, 1, plan->rows_with_edges_only, st);
-    if (rc) return rc;
-    std::vector<int32_t> h_report(report_ints);
-    TGT_HIP_CHECK(hipMemcpyAsync(h_report.data(), report, sizeof(int32_t) * report_ints, hipMemcpyDeviceToHost, st));
+    std::vector<int32_t> h_report(report_ints + (one_copy ? meta_bytes / 4 : 0));
+    TGT_HIP_CHECK(hipMemcpyAsync(h_report.data(), report, sizeof(int32_t) * h_report.size(), hipMemcpyDeviceToHost, st));
     TGT_HIP_CHECK(hipStreamSynchronize(st));
     if (h_report[kReportFlag]) {
         set_error("edge_index holds a node id outside [0, %lld)", (long long)N);
         return TGT_ERR_INDEX_RANGE;
     }
-    schedule_counts(plan->dst, scr_d, h_report.data(), 0);
-    schedule_counts(plan->src, scr_s, h_report.data(), 1);
-    // graphs with rows longer than a wave row: where their workgroup items go (second and last read-back)
-    std::vector<BlockMeta> meta_d(plan->dst.n_block_items), meta_s(plan->src.n_block_items);
-    if (!meta_d.empty())
-        TGT_HIP_CHECK(hipMemcpyAsync(meta_d.data(), scr_d.meta.p, sizeof(BlockMeta) * meta_d.size(), hipMemcpyDeviceToHost, st));
-    if (!meta_s.empty())
-        TGT_HIP_CHECK(hipMemcpyAsync(meta_s.data(), scr_s.meta.p, sizeof(BlockMeta) * meta_s.size(), hipMemcpyDeviceToHost, st));
-    if (!meta_d.empty() || !meta_s.empty()) TGT_HIP_CHECK(hipStreamSynchronize(st));
-    for (auto sm : {std::make_pair(&plan->dst, &meta_d), std::make_pair(&plan->src, &meta_s)}) {
+    schedule_counts(plan->dst, scr[0], h_report.data(), 0);
+    schedule_counts(plan->src, scr[1], h_report.data(), 1);
+    // graphs with rows longer than a wave row: where their workgroup items go
+    std::vector<BlockMeta> meta[2];
+    for (int i = 0; i < 2; ++i) {
+        meta[i].resize(views[i]->n_block_items);
+        if (meta[i].empty()) continue;
+        if (one_copy) memcpy(meta[i].data(), reinterpret_cast<const BlockMeta*>(h_report.data() + report_ints) + i * cap_meta, sizeof(BlockMeta) * meta[i].size());
+        else TGT_HIP_CHECK(hipMemcpyAsync(meta[i].data(), metas + i * cap_meta, sizeof(BlockMeta) * meta[i].size(), hipMemcpyDeviceToHost, st));
+    }
+    if (!one_copy && !(meta[0].empty() && meta[1].empty())) TGT_HIP_CHECK(hipStreamSynchronize(st));
+    for (auto sm : {std::make_pair(&plan->dst, &meta[0]), std::make_pair(&plan->src, &meta[1])}) {
         Side& sd = *sm.first;
         const std::vector<BlockMeta>& m = *sm.second;
         sd.block_home.resize(m.size()); sd.block_len.resize(m.size()); sd.block_spread.resize(m.size());

@@ -17,10 +17,17 @@ constexpr int RS_ITEMS = 16;
 constexpr int RS_TILE = RS_THREADS * RS_ITEMS;   // 4096 keys per workgroup
 constexpr int RS_WAVE_SPAN = kWave * RS_ITEMS;   // 1024 consecutive keys per wave
 
+// One or two sorts of the same size in a launch (blockIdx.y): the two views of a plan are sorted side by side - at half a
+// million keys one of them is a hundred workgroups.
+struct RsArgs {
+    const uint32_t *keys_in[2], *vals_in[2];
+    uint32_t *keys_out[2], *vals_out[2], *hist[2], *totals[2];
+};
+
 // Per-workgroup digit histogram, stored digit-major: hist[digit * nblocks + block].
-__global__ __launch_bounds__(RS_THREADS) void k_rs_hist(const uint32_t* __restrict__ keys, int64_t n,
-                                                        int shift, uint32_t* __restrict__ hist,
-                                                        int nblocks) {
+__global__ __launch_bounds__(RS_THREADS) void k_rs_hist(const RsArgs a, int64_t n, int shift, int nblocks) {
+    const uint32_t* __restrict__ keys = a.keys_in[blockIdx.y];
+    uint32_t* __restrict__ hist = a.hist[blockIdx.y];
     __shared__ uint32_t h[256];
     const int tid = threadIdx.x;
     h[tid] = 0;
@@ -37,8 +44,8 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_hist(const uint32_t* __restri
 
 // Workgroup `digit` turns its row of per-block counts into exclusive offsets and
 // records the row total.
-__global__ __launch_bounds__(256) void k_rs_scan_rows(uint32_t* __restrict__ hist, int nblocks,
-                                                      uint32_t* __restrict__ totals) {
+__global__ __launch_bounds__(256) void k_rs_scan_rows(const RsArgs a, int nblocks) {
+    uint32_t *__restrict__ hist = a.hist[blockIdx.y], *__restrict__ totals = a.totals[blockIdx.y];
     __shared__ uint32_t part[256];
     const int tid = threadIdx.x;
     uint32_t* row = hist + (int64_t)blockIdx.x * nblocks;
@@ -70,10 +77,10 @@ __global__ __launch_bounds__(256) void k_rs_scan_rows(uint32_t* __restrict__ his
 // is then put in digit order in LDS (stable), so that the writes to global memory go
 // out as runs of consecutive addresses, one run per digit, instead of one scattered
 // 4-byte store per key.
-__global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(
-    const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in,
-    uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out, int64_t n, int shift,
-    const uint32_t* __restrict__ hist, const uint32_t* __restrict__ totals, int nblocks) {
+__global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const RsArgs a, int64_t n, int shift, int nblocks) {
+    const uint32_t *__restrict__ keys_in = a.keys_in[blockIdx.y], *__restrict__ vals_in = a.vals_in[blockIdx.y];
+    uint32_t *__restrict__ keys_out = a.keys_out[blockIdx.y], *__restrict__ vals_out = a.vals_out[blockIdx.y];
+    const uint32_t *__restrict__ hist = a.hist[blockIdx.y], *__restrict__ totals = a.totals[blockIdx.y];
     __shared__ uint32_t cnt[4][256];
     __shared__ uint32_t base[256];        // first output position of this tile's keys of a digit
     __shared__ uint32_t scan[256];        // scan of the global digit totals
@@ -205,45 +212,39 @@ int bits_for(int64_t n) {
     return bits;
 }
 
-int RadixSorter::init(int64_t n, hipStream_t st) {
+int RadixSorter::init(int64_t n, hipStream_t st, int sorts) {
     cap_ = n > 0 ? n : 1;
     nblocks_ = (int)((cap_ + RS_TILE - 1) / RS_TILE);
-    const size_t eb = sizeof(uint32_t) * (size_t)cap_;
-    TGT_HIP_CHECK(keysA_.alloc(eb, st));
-    TGT_HIP_CHECK(keysB_.alloc(eb, st));
-    TGT_HIP_CHECK(valsA_.alloc(eb, st));
-    TGT_HIP_CHECK(valsB_.alloc(eb, st));
-    TGT_HIP_CHECK(hist_.alloc(sizeof(uint32_t) * 256 * (size_t)nblocks_, st));
-    TGT_HIP_CHECK(totals_.alloc(sizeof(uint32_t) * 256, st));
+    sorts_ = sorts;
+    TGT_HIP_CHECK(buf_.alloc(sizeof(uint32_t) * sorts * (4 * (size_t)cap_ + 256 * (size_t)nblocks_ + 256), st));
     return TGT_OK;
 }
 
-int RadixSorter::sort(const uint32_t* keys_in, const uint32_t* vals_in, int64_t n, int bits, hipStream_t st,
+int RadixSorter::sort(const uint32_t* const* keys_in, const uint32_t* const* vals_in, int sorts, int64_t n, int bits, hipStream_t st,
                       const uint32_t** keys_out, const uint32_t** vals_out) {
-    if (n > cap_) { set_error("RadixSorter: n exceeds capacity"); return TGT_ERR_INVALID_ARG; }
+    if (n > cap_ || sorts > sorts_) { set_error("RadixSorter: n exceeds capacity"); return TGT_ERR_INVALID_ARG; }
     const int passes = (bits + 7) / 8 > 0 ? (bits + 7) / 8 : 1;
     const int nblocks = (int)((n + RS_TILE - 1) / RS_TILE);
-    const uint32_t* kin = keys_in;
-    const uint32_t* vin = vals_in;
-    uint32_t* kout = keysA_.as<uint32_t>();
-    uint32_t* vout = valsA_.as<uint32_t>();
+    RsArgs a{};
+    uint32_t *key[2][2], *val[2][2];      // [sort][ping, pong]
+    uint32_t* at = buf_.as<uint32_t>();
+    for (int i = 0; i < sorts; ++i) {
+        for (int j = 0; j < 2; ++j) { key[i][j] = at; val[i][j] = at + cap_; at += 2 * cap_; }
+        a.hist[i] = at; a.totals[i] = at + 256 * (size_t)nblocks_;
+        at += 256 * (size_t)nblocks_ + 256;
+        a.keys_in[i] = keys_in[i];
+        a.vals_in[i] = vals_in ? vals_in[i] : nullptr;
+    }
     for (int p = 0; p < passes && n > 0; ++p) {
         const int shift = 8 * p;
-        hipLaunchKernelGGL(k_rs_hist, dim3(nblocks), dim3(RS_THREADS), 0, st, kin, n, shift,
-                           hist_.as<uint32_t>(), nblocks);
-        hipLaunchKernelGGL(k_rs_scan_rows, dim3(256), dim3(256), 0, st, hist_.as<uint32_t>(), nblocks,
-                           totals_.as<uint32_t>());
-        hipLaunchKernelGGL(k_rs_scatter, dim3(nblocks), dim3(RS_THREADS), 0, st, kin, vin, kout, vout, n,
-                           shift, hist_.as<uint32_t>(), totals_.as<uint32_t>(), nblocks);
-        kin = kout;
-        vin = vout;
-        const bool toB = (kout == keysA_.as<uint32_t>());
-        kout = toB ? keysB_.as<uint32_t>() : keysA_.as<uint32_t>();
-        vout = toB ? valsB_.as<uint32_t>() : valsA_.as<uint32_t>();
+        for (int i = 0; i < sorts; ++i) { a.keys_out[i] = key[i][p & 1]; a.vals_out[i] = val[i][p & 1]; }
+        hipLaunchKernelGGL(k_rs_hist, dim3(nblocks, sorts), dim3(RS_THREADS), 0, st, a, n, shift, nblocks);
+        hipLaunchKernelGGL(k_rs_scan_rows, dim3(256, sorts), dim3(256), 0, st, a, nblocks);
+        hipLaunchKernelGGL(k_rs_scatter, dim3(nblocks, sorts), dim3(RS_THREADS), 0, st, a, n, shift, nblocks);
+        for (int i = 0; i < sorts; ++i) { a.keys_in[i] = a.keys_out[i]; a.vals_in[i] = a.vals_out[i]; }
     }
     TGT_HIP_CHECK(hipGetLastError());
-    *keys_out = kin;
-    *vals_out = vin;
+    for (int i = 0; i < sorts; ++i) { keys_out[i] = a.keys_in[i]; vals_out[i] = a.vals_in[i]; }
     return TGT_OK;
 }
 

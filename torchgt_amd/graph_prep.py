@@ -35,6 +35,10 @@ def gen_sub_edge_index(edge_index, idx_batch, N):
     self-loops of the input dropped and one self-loop per batch node appended - the result of the
     reference's remove_self_loops / add_self_loops / subgraph(relabel_nodes=True) chain, in the
     same order.  edge_index: int64 [2, E] CUDA tensor over nodes 0..N-1."""
+    return _sub_edges(edge_index, idx_batch, N).clone()      # (of its own size: the buffer has room for every edge)
+
+
+def _sub_edges(edge_index, idx_batch, N):
     if not edge_index.is_cuda:
         raise RuntimeError("gen_sub_edge_index needs GPU tensors (no CPU implementation)")
     dev = edge_index.device
@@ -45,9 +49,9 @@ def gen_sub_edge_index(edge_index, idx_batch, N):
     out = torch.empty((2, cap), dtype=torch.int64, device=dev)
     n = ctypes.c_int64()
     with torch.cuda.device(dev):
-        _lib.check(_lib.lib().tgt_sub_edge_index(ei.data_ptr() if E else None, E, N, idx.data_ptr() if S else None, S,
-                                                 out.data_ptr() if cap else None, cap, ctypes.byref(n), _stream(dev)))
-    return out[:, :n.value].contiguous()
+        _lib.check(_lib.lib().tgt_sub_edge_index_packed(ei.data_ptr() if E else None, E, N, idx.data_ptr() if S else None, S,
+                                                        out.data_ptr() if cap else None, cap, ctypes.byref(n), _stream(dev)))
+    return out.view(-1)[:2 * n.value].view(2, n.value)
 
 
 def adjust_edge_index_nomerge(edge_index, sub_seq_len):
@@ -70,6 +74,13 @@ def reformat_graph(edge_index, k, block_size, beta_coeffi="1", partition_ids=Non
     ``return_tiles=True`` additionally returns the emitted blocks as a tile list (numpy int32
     [T, 2], first source / first destination in new ids) and the edges that were kept as they
     are (int64 [2, E_raw]), the inputs of ``torchgt_amd.block_attention``."""
+    res = _reformat(edge_index, k, block_size, partition_ids, blockize, return_tiles)
+    return res[:4] if return_tiles else res[:2]
+
+
+def _reformat(edge_index, k, block_size, partition_ids, blockize, return_tiles, batch=None, tokens=0):
+    """``(edges, sorted_indices, tiles, raw edges, rows)``; rows: the nodes of ``batch`` in the new order (without the global
+    node in front of them when ``tokens`` is 1)."""
     if partition_ids is None:
         raise ValueError("reformat_graph: partition_ids must be given (METIS is not available)")
     if not edge_index.is_cuda:
@@ -82,16 +93,16 @@ def reformat_graph(edge_index, k, block_size, beta_coeffi="1", partition_ids=Non
     handle = ctypes.c_void_p()
     with torch.cuda.device(dev):
         st = _stream(dev)
-        _lib.check(L.tgt_reformat_create(ei[0].data_ptr() if E else None, ei[1].data_ptr() if E else None, E, N,
-                                         part.data_ptr(), int(k), int(block_size), 1 if blockize else 0, st,
-                                         ctypes.byref(handle)))
+        src = ei.data_ptr() if E else None
+        _lib.check(L.tgt_reformat_create(src, src + 8 * E if E else None, E, N, part.data_ptr(), int(k), int(block_size),
+                                         1 if blockize else 0, st, ctypes.byref(handle)))
         try:
             E_out = L.tgt_reformat_num_edges(handle)
             out = torch.empty((2, E_out), dtype=torch.int64, device=dev)
             sorted_indices = torch.empty(N, dtype=torch.int64, device=dev)
             _lib.check(L.tgt_reformat_export(handle, out.data_ptr() if E_out else None,
                                              sorted_indices.data_ptr(), st))
-            tiles = raw = None
+            tiles = raw = rows = None
             if return_tiles:
                 import numpy as np
                 T, E_raw = L.tgt_reformat_num_tiles(handle), L.tgt_reformat_num_raw_edges(handle)
@@ -99,12 +110,12 @@ def reformat_graph(edge_index, k, block_size, beta_coeffi="1", partition_ids=Non
                 raw = torch.empty((2, E_raw), dtype=torch.int64, device=dev)
                 _lib.check(L.tgt_reformat_export_tiles(handle, tiles.ctypes.data_as(ctypes.c_void_p) if T else None,
                                                        raw.data_ptr() if E_raw else None, st))
-            torch.cuda.current_stream(dev).synchronize()
+            if batch is not None:
+                rows = torch.empty(N - tokens, dtype=torch.int64, device=dev)
+                _lib.check(L.tgt_reformat_rows(handle, batch.data_ptr() if N > tokens else None, tokens, rows.data_ptr(), st))
         finally:
             L.tgt_reformat_destroy(handle)
-    if return_tiles:
-        return out, sorted_indices, tiles, raw
-    return out, sorted_indices
+    return out, sorted_indices, tiles, raw, rows
 
 
 def prepare_batch(x, y, idx_batch, edge_index, N, k, block_size, partition, model="graphormer", reorder=True,
@@ -120,25 +131,19 @@ def prepare_batch(x, y, idx_batch, edge_index, N, k, block_size, partition, mode
     sub-graph, :326).  Returns (x_i, y_i, edge_index_i, attn_bias=None) like the reference, plus
     (tiles, raw_edge_index) when ``return_tiles``."""
     idx_batch = idx_batch.to(edge_index.device)
-    x_i, y_i = x[idx_batch], y[idx_batch]
     S = idx_batch.shape[0]
-    ei = gen_sub_edge_index(edge_index, idx_batch, N)
-    n_sub = S
-    if model == "graphormer":
-        ei = fix_edge_index(ei, S)
-        n_sub = S + 1
+    tokens = 1 if model == "graphormer" else 0
+    ei = fix_edge_index(_sub_edges(edge_index, idx_batch, N), S) if tokens else gen_sub_edge_index(edge_index, idx_batch, N)
+    n_sub = S + tokens
     extra = ()
+    rows = idx_batch
     if reorder:
         part = partition(ei, n_sub, k) if callable(partition) else partition
         if part.numel() != n_sub:
             raise ValueError(f"partition ids for {part.numel()} nodes, the sub-graph has {n_sub}")
-        res = reformat_graph(ei, k, block_size, partition_ids=part, blockize=blockize, return_tiles=return_tiles)
-        ei, sorted_indices = res[0], res[1]
-        extra = tuple(res[2:])
-        if model == "graphormer":
-            sorted_indices = sorted_indices[sorted_indices != 0] - 1      # drop the global node, back to batch positions
-        x_i = torch.index_select(x_i, 0, sorted_indices)
-        y_i = torch.index_select(y_i, 0, sorted_indices)
-    if model == "graphormer":
-        ei = adjust_edge_index_nomerge(ei, S)
-    return (x_i, y_i, ei, None) + extra
+        # x and y are gathered once, in the new order (the global node has no row)
+        batch = idx_batch.to(torch.int64).contiguous()
+        ei, _, tiles, raw, rows = _reformat(ei, k, block_size, part, blockize, return_tiles, batch, tokens)
+        extra = (tiles, raw) if return_tiles else ()
+    # (adjust_edge_index_nomerge leaves every id of one rank, 0 .. S, as it is)
+    return (x[rows], y[rows], ei, None) + extra
