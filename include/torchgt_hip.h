@@ -623,6 +623,7 @@ typedef struct {
 int tgt_node_fwd(const tgt_node_fwd_args* args, void* stream);
 /* Backward of the part in front of an attention: g_out = g_in + d LN'(...) for dq, dk, dv (w_back: the transposed packed Wq,
  * Wk, Wv; s: the rows LN' normalised), or of the classes (dlogp, logp - not needed with `linear` -; no g_in, dq, dk, dv; w_back: transposed packed Wh).
+ * v_next NULL: q, k, v were made of the rows s themselves (GT), no LayerNorm.
  * d_token: the first `tokens` rows of g_out once more (the gradient of the global tokens behind the first layer), or NULL.
  * partial: tgt_node_bwd_workers(rows) partial sums of the gradients of (Wq, Wk, Wv, bq, bk, bv, gamma, beta) or of
  * (Wh, bh, gamma, beta), each mats * 4096 + (mats + 2) * 64 floats: see tgt_node_sums. */
@@ -657,10 +658,39 @@ int tgt_node_bwd_post(const tgt_node_bwd_post_args* args, void* stream);
  * gamma, beta [64] (NULL: not wanted). */
 typedef struct {
     const float* partial;
-    int32_t workers, mats, rows;
+    int32_t workers, mats, rows, ld;      /* ld: elements between rows of the weights (0: 64) */
     void* out[8];
 } tgt_node_sum;
 int tgt_node_sums(const tgt_node_sum* sums, int count, int dtype, void* stream);
+/* The same for the GT layers (models/gt_dist_node_level.py:218-267), hidden 64, feed-forward 128:
+ *     y = a O^T + bo;  x1 = LN1(x + y);  s2 = x1 + W2 relu(W1 y + b1) + b2;  x' = LN2(s2);   q, k, v = x' W^T + b
+ * w: packed O, W1 (rows 0 .. 63, 64 .. 127), W2 (columns 0 .. 63, 64 .. 127) with unit frag_bytes(1) / 2; v: bo, gamma1, beta1, b1 (two
+ * vectors), b2, gamma2, beta2.  s2: kept for the backward (NULL: not).  q, k, v: rows for the next attention (w_next: packed Wq, Wk,
+ * Wv; v_next: bq, bk, bv), or NULL. */
+typedef struct {
+    int64_t rows;
+    int32_t dtype;
+    float eps1, eps2;
+    const void *attn, *x;
+    void *s2, *x_out, *q, *k, *v;
+    const void *w, *w_next;
+    const float *vec, *v_next;
+} tgt_gt_fwd_args;
+int tgt_gt_fwd(const tgt_gt_fwd_args* args, void* stream);
+/* g_in = dx' -> g_out = dx (residual path) and d_attn = da, nd as in tgt_node_bwd_post.  w_back: the transposed packed weights in the
+ * order of w.  partial_a: sums for (O, W1 lower and upper half, bo, b1 (two), gamma1, beta1), partial_b: for (W2 left and right half,
+ * b2, nothing, gamma2, beta2), tgt_node_bwd_workers(rows) of them each. */
+typedef struct {
+    int64_t rows;
+    int32_t dtype, heads;
+    float eps1, eps2;
+    const void *g_in, *x, *attn, *s2;
+    const void *w, *w_back;
+    const float *vec, *Z;
+    void *g_out, *d_attn;
+    float *nd, *partial_a, *partial_b;
+} tgt_gt_bwd_args;
+int tgt_gt_bwd(const tgt_gt_bwd_args* args, void* stream);
 /* The dense biased attention for query 0 only: the last layer of the graph-level models, whose output is read at the virtual node
  * (models/graphormer_graph_level.py:387).  Tensors as for tgt_dense_attn_dropout_fwd (H <= 8, d 8, 16 or 32, S <= 1024, dtype
  * TGT_DTYPE_F32 or TGT_DTYPE_BF16); a0 [b, H d] = the attention's row 0 of every graph, s0 = the rows 0 of d_s [b, S, H d],

@@ -3,6 +3,7 @@ test_gpu_encoder.py): output and every parameter gradient, at the sizes where th
 a wave's 32 rows and a workgroup's 128 and 256, class counts around the halves of a row, odd feature widths, all head shapes.
 
 Bars: float32 1e-5 of the largest value of the tensor, bf16 6e-2 (the layer-by-layer path rounds every intermediate tensor)."""
+import copy
 import types
 
 import pytest
@@ -120,7 +121,7 @@ def test_graph_graphormer_as_one_operator(cuda, dtype, b, s, outputs, heads, lay
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("kind,n,features,classes,heads,hidden,ffn,layers", [("gt", 1, 32, 3, 8, 64, 64, 1), ("gt", 999, 100, 47, 8, 64, 64, 3), ("gt", 3000, 51, 40, 8, 128, 128, 2),
+@pytest.mark.parametrize("kind,n,features,classes,heads,hidden,ffn,layers", [("gt", 1, 32, 3, 8, 128, 64, 1), ("gt", 999, 100, 47, 4, 32, 64, 3), ("gt", 3000, 51, 40, 8, 128, 128, 2),
                                                                           ("graphormer", 1, 32, 3, 8, 128, 128, 1), ("graphormer", 999, 100, 47, 8, 128, 128, 3),
                                                                           ("graphormer", 777, 64, 65, 4, 64, 64, 2), ("graphormer", 500, 51, 40, 4, 64, 96, 2)])
 def test_other_widths_as_one_operator(cuda, dtype, kind, n, features, classes, heads, hidden, ffn, layers):
@@ -146,3 +147,30 @@ def test_other_widths_as_one_operator(cuda, dtype, kind, n, features, classes, h
     assert len(got[0]) == len(got[1])
     for i, (a, b) in enumerate(zip(*got)):
         assert torch.equal(a, b), (i, float((a.float() - b.float()).abs().max()))
+
+
+@pytest.mark.parametrize("n,features,classes,heads,layers", [(1, 32, 3, 8, 1), (31, 64, 8, 4, 2), (32, 100, 47, 8, 1), (129, 51, 40, 2, 3), (256, 64, 16, 8, 2), (4097, 128, 40, 8, 4),
+                                                             (40000, 64, 5, 8, 2)])
+def test_gt_on_fused_layers(cuda, n, features, classes, heads, layers):
+    """float32 against the kernels step by step; bf16, where a ReLU's input of nearly 0 may change its side, by how far both are from float32"""
+    print(f"fused gt case: n={n} features={features} classes={classes} heads={heads} layers={layers}", flush=True)
+    torch.manual_seed(n)
+    model = scaled(GT(layers, heads, features, 64, classes, 1, 0.0, 0.0, 0.0, 64, 0), n + 1, torch.bfloat16, cuda)
+    x, plan = torch.randn(n, features).to(cuda, torch.bfloat16), GraphPlan(random_edges(n, 0, n + 2, cuda), n)
+    exact = copy.deepcopy(model).float()
+    compare(GT, exact, x.float(), plan, n + 3)
+    w = torch.randn(n, classes, generator=torch.Generator().manual_seed(n + 4)).to(cuda)
+    got = []
+    for m, fused in ((exact, False), (model, True), (model, False)):
+        GT.one_operator = fused
+        try:
+            m.zero_grad(set_to_none=True)
+            xr = x.to(next(m.parameters()).dtype).requires_grad_(True)
+            out = m(xr, None, plan, attn_type="sparse")
+            (out.float() * w).sum().backward()
+            got.append([t.float() for t in (out.detach(), xr.grad, torch.cat([p.grad.flatten() for p in m.parameters() if p.grad is not None]))])
+        finally:
+            GT.one_operator = True
+    for name, f32, one, steps in zip(("output", "input gradient", "parameter gradients"), *got):
+        off, most = float((one - f32).norm() / f32.norm()), float((steps - f32).norm() / f32.norm())
+        assert off <= 1.1 * most + 2e-3, f"{name}: {off}, step by step {most}"

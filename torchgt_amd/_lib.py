@@ -122,6 +122,8 @@ SIGNATURES = {
     "tgt_node_bwd_pre": (_i32, [_vp, _vp]),
     "tgt_node_bwd_post": (_i32, [_vp, _vp]),
     "tgt_node_sums": (_i32, [_vp, _i32, _i32, _vp]),
+    "tgt_gt_fwd": (_i32, [_vp, _vp]),
+    "tgt_gt_bwd": (_i32, [_vp, _vp]),
     "tgt_sparse_attn_bwd_from_nd": (_i32, [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),
     "tgt_timing_enable": (_i32, [_i32]),
     "tgt_timing_reset": (_i32, []),

@@ -15,50 +15,10 @@
 // written and read).  A wave takes 32 nodes and keeps them in registers through the whole chain (node_tile.h); the waves of
 // a workgroup share the packed weights in LDS.  Weight gradients contract over nodes: the waves put the bf16 planes of both
 // operands into LDS, four waves (128 nodes) at a time, and every wave adds one 32 x 32 block over its share of the nodes.
-#include "node_tile.h"
-#include <algorithm>
-#include <atomic>
+#include "node_roles.h"
 
 namespace tgt {
 namespace {
-
-constexpr int kVec = 64;      // floats per parameter vector
-
-// N 16-byte vectors from global memory to LDS by all THREADS threads of a workgroup, every load issued before the first write
-template <int N, int THREADS> __device__ __forceinline__ void copy_vecs(vec16* dst, const vec16* __restrict__ src) {
-    constexpr int R = (N + THREADS - 1) / THREADS;
-    vec16 v[R];
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-        const int at = threadIdx.x + i * THREADS;
-        if (N % THREADS == 0 || at < N) v[i] = src[at];
-    }
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-        const int at = threadIdx.x + i * THREADS;
-        if (N % THREADS == 0 || at < N) dst[at] = v[i];
-    }
-}
-
-// A packed weight on its way from memory to LDS through the registers of the four block waves
-template <int N> struct WeightsAhead {
-    static_assert(N % 256 == 0, "whole vectors per thread");
-    vec16 v[N / 256];
-    __device__ __forceinline__ void fetch(const vec16* __restrict__ src) {
-#pragma unroll
-        for (int i = 0; i < N / 256; ++i) v[i] = src[(threadIdx.x & 255) + i * 256];
-    }
-    __device__ __forceinline__ void put(vec16* dst) const {
-#pragma unroll
-        for (int i = 0; i < N / 256; ++i) dst[(threadIdx.x & 255) + i * 256] = v[i];
-    }
-    // the weight at hand to LDS, the next one asked for, and the barrier that says so
-    __device__ __forceinline__ void hand_over(vec16* dst, const vec16* __restrict__ src) {
-        put(dst);
-        fetch(src);
-        __syncthreads();
-    }
-};
 
 // ---- packing of the parameters ---------------------------------------------------------------------------------------
 constexpr int kPackMats = 96, kPackVecs = 160;
@@ -310,39 +270,6 @@ __global__ __launch_bounds__((fwd_waves<T, SAME>() * 64)) void k_node_fwd(const 
     }
 }
 
-// ---- backward: shared pieces ----------------------------------------------------------------------------------------------
-// Eight waves, two roles, one of each per SIMD: waves 0 .. 3 ("chain") carry 32 nodes each through the chain of products and
-// LayerNorms and leave the planes of both operands of every weight gradient in LDS; waves 4 .. 7 ("blocks") keep one 32 x 32
-// block of every weight gradient in registers and add the products over the 128 nodes while the chain is in its next step,
-// and hand the chain its packed weights one at a time.  So the matrix work of one role runs beside the vector work of the
-// other, and neither has to hold the other's registers (with all waves in both roles, 16 KB of accumulators per wave next to
-// the tiles spilled: 106 us for k_node_bwd_post and 55 us for k_node_bwd_pre at 64 K nodes in float32).
-constexpr int kChainNodes = 128, kBwdThreads = 512;
-
-template <typename T> struct BwdLds {
-    static constexpr int P = Num<T>::P;
-    static constexpr int kW = 2 * P * kPlaneBytes, kStage = kW + kFragVecs<P> * 16, kVecs = kStage + 4 * RowShape<T>::kVecs * 16;
-    static constexpr int kBytes = kVecs + 5 * kVec * 4;
-};
-
-// The workgroup's sums to its partial: NM 64 x 64 blocks (registers of the block waves), then NV vectors of 64 (a register
-// of each chain wave; added through LDS).
-template <int NM, int NV> __device__ __forceinline__ void write_partial(float* __restrict__ mine, const float16_t (&acc)[NM], const float (&col)[NV], float* buf, int wave, int lane) {
-    __syncthreads();
-    if (wave < 4) {
-#pragma unroll
-        for (int c = 0; c < NV; ++c) buf[(wave * NV + c) * 64 + lane] = col[c];
-    } else {
-        const int q = wave - 4, h = lane >> 5;
-#pragma unroll
-        for (int j = 0; j < NM; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) mine[j * 4096 + (32 * (q >> 1) + 8 * (r >> 2) + 4 * h + (r & 3)) * 64 + 32 * (q & 1) + (lane & 31)] = acc[j][r];
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < NV * 64; i += kBwdThreads) mine[NM * 4096 + i] = (buf[i] + buf[NV * 64 + i]) + (buf[2 * NV * 64 + i] + buf[3 * NV * 64 + i]);
-}
-
 // Class gradients of a wave's 32 rows: d logits = d logp - softmax * sum(d logp) (linear: d logits as they come); zero for tokens and past the end.
 template <typename T> __device__ __forceinline__ void class_grads(Tile& d, const T* __restrict__ dlogp, const T* __restrict__ logp, bool linear, int C, int tokens, int64_t row0, int64_t N,
                                                                   vec16* stage, int lane) {
@@ -363,7 +290,8 @@ template <typename T> __device__ __forceinline__ void class_grads(Tile& d, const
 }
 
 // ---- backward of the part in front of an attention (or of the classes) ------------------------------------------------------
-template <typename T, bool CLASSES>
+// NORM false (GT): q, k, v are made of the rows s themselves.
+template <typename T, bool CLASSES, bool NORM>
 __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_pre(const tgt_node_bwd_pre_args a) {
     using L = BwdLds<T>;
     constexpr int P = Num<T>::P, FV = kFragVecs<P>, NM = CLASSES ? 1 : 3;
@@ -373,7 +301,7 @@ __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_pre(const tgt_node_bwd
     float* vec = reinterpret_cast<float*>(smem + L::kVecs);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5;
     const int64_t N = a.rows, groups = (N + kChainNodes - 1) / kChainNodes;
-    copy_vecs<2 * kVec / 4, kBwdThreads>(reinterpret_cast<vec16*>(vec), reinterpret_cast<const vec16*>(a.v_next));
+    if constexpr (NORM) copy_vecs<2 * kVec / 4, kBwdThreads>(reinterpret_cast<vec16*>(vec), reinterpret_cast<const vec16*>(a.v_next));
     __syncthreads();
     float16_t acc[NM];
     float col[NM + 2];
@@ -398,7 +326,8 @@ __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_pre(const tgt_node_bwd
             Tile xhat, dy, d;
             Frags<P> f;
             settle<T, false>(xhat, raw_s, stage, rows, lane);
-            const float rstd = normalise<false>(xhat, a.eps);
+            float rstd = 1.f;
+            if constexpr (NORM) rstd = normalise<false>(xhat, a.eps);
             zero(dy);
 #pragma unroll
             for (int j = 0; j < NM; ++j) {
@@ -414,7 +343,8 @@ __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_pre(const tgt_node_bwd
                 if (j > 0) __syncthreads();            // product j - 1 is done
                 else {
                     Tile y;
-                    affine(y, xhat, vec, vec + kVec, h);
+                    if constexpr (NORM) affine(y, xhat, vec, vec + kVec, h);
+                    else y = xhat;
                     Frags<P> fx;
                     make_frags(fx, y);
                     put_planes<P>(p_x, row, h, fx);
@@ -424,15 +354,18 @@ __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_pre(const tgt_node_bwd
             }
             if (g0 + gridDim.x < groups) fetch(raw_s, reinterpret_cast<const T*>(a.s), Rows(4 * (g0 + gridDim.x) + wave, N), lane);
             TGT_EACH(i) dy.set(i, stored(dy.get(i), (const T*)nullptr));
-            col[NM + 1] += column_sums(dy, lane);
-            TGT_EACH(i) d.set(i, dy.get(i) * xhat.get(i));
-            col[NM] += column_sums(d, lane);
+            if constexpr (NORM) {
+                col[NM + 1] += column_sums(dy, lane);
+                TGT_EACH(i) d.set(i, dy.get(i) * xhat.get(i));
+                col[NM] += column_sums(d, lane);
+            }
             if (CLASSES) zero(d);
             else {
                 settle<T, true>(d, raw_d, stage, rows, lane);
                 if (g0 + gridDim.x < groups) fetch(raw_d, src[0], Rows(4 * (g0 + gridDim.x) + wave, N), lane);
             }
-            ln_back(d, dy, xhat, rstd, vec, h);
+            if constexpr (NORM) ln_back(d, dy, xhat, rstd, vec, h);
+            else TGT_EACH(i) d.set(i, d.get(i) + dy.get(i));
             put_rows(reinterpret_cast<T*>(a.g_out), d, stage, rows, lane);
             if (a.d_token && 4 * g0 + wave < (a.tokens + 31) / 32) put_rows(reinterpret_cast<T*>(a.d_token), d, stage, Rows(4 * g0 + wave, a.tokens), lane);
         }
@@ -569,29 +502,7 @@ __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_post(const tgt_node_bw
             gemm<P>(g, f, w, lane);                                 // da, beside product Wo
             __syncthreads();                                        // Wo^T has been used
             put_rows(reinterpret_cast<T*>(a.d_attn), g, stage, rows, lane);
-            if (a.nd && n < rows.left) {
-                float dot[4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    dot[k] = 0.f;
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) dot[k] += stored(g.get(8 * k + i), (const T*)nullptr) * t.get(8 * k + i);
-                }
-                const int heads = a.heads;      // 8, 4 or 2: one, two or four groups of 8 features per head
-                const float* Z = a.Z + (rows.first + n) * heads;
-                float2* nd = reinterpret_cast<float2*>(a.nd) + (rows.first + n) * heads;
-                if (heads == 8) {
-                    const float4 z = *reinterpret_cast<const float4*>(Z + 4 * h);
-                    float4* o = reinterpret_cast<float4*>(nd + 4 * h);
-                    o[0] = make_float4(1.f / (z.x + 1e-6f), dot[0], 1.f / (z.y + 1e-6f), dot[1]);
-                    o[1] = make_float4(1.f / (z.z + 1e-6f), dot[2], 1.f / (z.w + 1e-6f), dot[3]);
-                } else if (heads == 4) {
-                    const float2 z = *reinterpret_cast<const float2*>(Z + 2 * h);
-                    *reinterpret_cast<float4*>(nd + 2 * h) = make_float4(1.f / (z.x + 1e-6f), dot[0] + dot[1], 1.f / (z.y + 1e-6f), dot[2] + dot[3]);
-                } else {
-                    nd[h] = make_float2(1.f / (Z[h] + 1e-6f), dot[0] + dot[1] + (dot[2] + dot[3]));
-                }
-            }
+            if (a.nd && n < rows.left) put_node_side<T>(g, t, a.Z, a.nd, a.heads, rows.first + n, h);
             if (P != 1) fetch_next();
         }
     } else {
@@ -624,7 +535,7 @@ struct SumArgs {
     const float* partial[kMaxSums];
     int workers[kMaxSums], n[kMaxSums];
     void* out[kMaxSums][kMaxOut];      // mats x 4096 elements, then vectors of 64 (a null entry is not wanted)
-    int16_t mats[kMaxSums], rows[kMaxSums];   // rows: of the 64 in each matrix and the vectors that follow them (classes)
+    int16_t mats[kMaxSums], rows[kMaxSums], ld[kMaxSums];   // rows: of the 64 in each matrix and the vectors that follow them (classes)
 };
 __device__ __forceinline__ void put_elem(float* p, float v) { *p = v; }
 __device__ __forceinline__ void put_elem(nbf16* p, float v) { p->x = __builtin_bit_cast(uint16_t, static_cast<__bf16>(v)); }
@@ -656,33 +567,8 @@ template <typename T> __global__ __launch_bounds__(1024) void k_node_sums(const 
         const int mats = a.mats[d], rows = a.rows[d];
         const int seg = e < mats * 4096 ? e >> 12 : mats + ((e - mats * 4096) >> 6), at = e < mats * 4096 ? e & 4095 : (e - mats * 4096) & 63;
         const int limit = seg < mats ? rows * 64 : (seg < 2 * mats ? rows : 64);
-        if (a.out[d][seg] && at < limit) put_elem(reinterpret_cast<T*>(a.out[d][seg]) + at, t);
+        if (a.out[d][seg] && at < limit) put_elem(reinterpret_cast<T*>(a.out[d][seg]) + (seg < mats ? (at >> 6) * a.ld[d] + (at & 63) : at), t);
     }
-}
-
-int bad(const char* who, const char* what) { set_error("%s: %s", who, what); return TGT_ERR_INVALID_ARG; }
-int num_cus() {
-    static const int n = [] { int dev = 0, v = 256; if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev); return v > 0 ? v : 256; }();
-    return n;
-}
-// a workgroup of `waves` waves per CU (LDS), fewer when there is less work
-int grid_for(int64_t rows, int waves) { return (int)std::max<int64_t>(1, std::min<int64_t>(num_cus(), ((rows + 31) / 32 + waves - 1) / waves)); }
-
-// Raises the dynamic LDS limit of a kernel, once per kernel and device (`done`: one bit per device, kept by the caller)
-int allow_lds(const void* kernel, int bytes, std::atomic<uint64_t>& done) {
-    int dev = 0;
-    TGT_HIP_CHECK(hipGetDevice(&dev));
-    const uint64_t bit = 1ull << (dev & 63);
-    if (done.load(std::memory_order_relaxed) & bit) return TGT_OK;
-    TGT_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
-    done.fetch_or(bit, std::memory_order_relaxed);
-    return TGT_OK;
-}
-template <typename... Args> int launch(void (*kernel)(Args...), std::atomic<uint64_t>& done, int grid, int threads, int lds, hipStream_t st, Args... args) {
-    if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), lds, done)) return rc;
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds, st, args...);
-    TGT_HIP_CHECK(hipGetLastError());
-    return TGT_OK;
 }
 
 template <typename T, bool SAME, bool POST, int NEXT> int launch_fwd(const tgt_node_fwd_args& a, hipStream_t st) {
@@ -694,9 +580,10 @@ template <typename T, bool SAME> int dispatch_fwd(const tgt_node_fwd_args& a, hi
     return launch_fwd<T, SAME, false, NEXT_QKV>(a, st);
 }
 template <typename T> int dispatch_bwd_pre(const tgt_node_bwd_pre_args& a, int workers, hipStream_t st) {
-    static std::atomic<uint64_t> done[2];
-    return a.dlogp ? launch(&k_node_bwd_pre<T, true>, done[1], workers, kBwdThreads, BwdLds<T>::kBytes, st, a)
-                   : launch(&k_node_bwd_pre<T, false>, done[0], workers, kBwdThreads, BwdLds<T>::kBytes, st, a);
+    static std::atomic<uint64_t> done[3];
+    if (a.dlogp) return launch(&k_node_bwd_pre<T, true, true>, done[1], workers, kBwdThreads, BwdLds<T>::kBytes, st, a);
+    return a.v_next ? launch(&k_node_bwd_pre<T, false, true>, done[0], workers, kBwdThreads, BwdLds<T>::kBytes, st, a)
+                    : launch(&k_node_bwd_pre<T, false, false>, done[2], workers, kBwdThreads, BwdLds<T>::kBytes, st, a);
 }
 template <typename T, bool SAME> int dispatch_bwd_post(const tgt_node_bwd_post_args& a, int workers, hipStream_t st) {
     static std::atomic<uint64_t> done{0};
@@ -757,7 +644,7 @@ int tgt_node_bwd_workers(int64_t rows) { return rows < 0 ? -1 : tgt::grid_for(ro
 
 int tgt_node_bwd_pre(const tgt_node_bwd_pre_args* a, void* stream) {
     using namespace tgt;
-    if (!a || a->rows < 1 || !dtype_ok(a->dtype) || !a->s || !a->g_out || !a->w_back || !a->v_next || !a->partial) return bad("tgt_node_bwd_pre", "null or bad argument");
+    if (!a || a->rows < 1 || !dtype_ok(a->dtype) || !a->s || !a->g_out || !a->w_back || (a->dlogp && !a->v_next) || !a->partial) return bad("tgt_node_bwd_pre", "null or bad argument");
     if (a->dlogp ? ((!a->logp && !a->linear) || a->classes < 1 || a->classes > 64 || a->tokens < 0) : (!a->dq || !a->dk || !a->dv || !a->g_in))
         return bad("tgt_node_bwd_pre", "dq, dk, dv, g_in or dlogp, logp and 1 to 64 classes are needed");
     KernelTimer t(KS_LINEAR_DX, (hipStream_t)stream);
@@ -787,8 +674,8 @@ int tgt_node_sums(const tgt_node_sum* sums, int count, int dtype, void* stream) 
         int longest = 0;
         for (int i = 0; i < m; ++i) {
             const tgt_node_sum& s = sums[c + i];
-            if (!s.partial || s.workers < 1 || s.mats < 1 || s.mats > 3 || s.rows < 1 || s.rows > 64) return bad("tgt_node_sums", "bad descriptor");
-            a.partial[i] = s.partial; a.workers[i] = s.workers; a.mats[i] = (int16_t)s.mats; a.rows[i] = (int16_t)s.rows;
+            if (!s.partial || s.workers < 1 || s.mats < 1 || s.mats > 3 || s.rows < 1 || s.rows > 64 || s.ld < 0 || s.ld > 32767) return bad("tgt_node_sums", "bad descriptor");
+            a.partial[i] = s.partial; a.workers[i] = s.workers; a.mats[i] = (int16_t)s.mats; a.rows[i] = (int16_t)s.rows; a.ld[i] = (int16_t)(s.ld ? s.ld : 64);
             a.n[i] = s.mats * 4096 + (s.mats + 2) * 64;
             for (int o = 0; o < 2 * s.mats + 2; ++o) a.out[i][o] = s.out[o];
             longest = std::max(longest, a.n[i]);

@@ -2,9 +2,10 @@
 // (linears, LayerNorms, activations, attention): the models whose widths the fused per-node kernels do not have.  The numbers
 // are those of the modules step by step; what goes away is the host's time between the launches - a step of four layers
 // passes through some forty operators and autograd nodes otherwise, 1.3 ms of host time whatever the graph's size.
+// GT of hidden size 64 runs its layers on the fused kernels of gt_layer.hip instead.
 //
 //   torchgt::layered_graphormer(x, params[7 + 16 L], plan holder, workspace, heads, tokens, classes, eps[2 L + 1]) -> log-probabilities
-//   torchgt::layered_gt(x, params[8 + 16 L], plan holder, workspace, heads, classes, eps[2 L]) -> log-probabilities
+//   torchgt::node_gt(x, params[8 + 16 L], plan holder, workspace, heads, classes, eps[2 L]) -> log-probabilities
 //
 // classes: output columns that count (the last weight may be padded to a width the linears read in 16-byte pieces).
 #include "torch_common.h"
@@ -118,9 +119,10 @@ struct Layer {
     Norm n1, n2;
 };
 struct Saved {
-    void *rows_in, *out, *m1, *r1, *m2, *r2, *logits;      // readout: graphormer: out = rows of the final norm; gt: out = last layer's rows
+    void *packed, *rows_in, *out, *m1, *r1, *m2, *r2, *logits;      // readout: graphormer: out = rows of the final norm; gt: out = last layer's rows
     Norm last;
     std::vector<Layer> l;
+    const std::vector<double>* eps;
 };
 
 Norm take_norm(Tape& t, const Dims& D, bool with_sum) { return {with_sum ? t.take(D.N * D.C * D.size) : nullptr, (float*)t.take(4 * D.N), (float*)t.take(4 * D.N)}; }
@@ -241,6 +243,24 @@ struct GtModel {
         const int64_t e = kHead + 16 * D.L;
         is(e, D.M1, D.C); is(e + 2, D.M2, D.M1); is(e + 4, D.Cp, D.M2);
     }
+    // models/gt_dist_node_level.py:270-286
+    static void readout(Tape& t, const Dims& D, const std::vector<Tensor>& p, void* in, Saved& s) {
+        auto P = [&](int64_t i) { return p[i].data_ptr(); };
+        const int64_t b = kHead + 16 * D.L;
+        s.out = in;
+        s.m1 = t.take(D.N * D.M1 * D.size); s.r1 = t.take(D.N * D.M1 * D.size); s.m2 = t.take(D.N * D.M2 * D.size); s.r2 = t.take(D.N * D.M2 * D.size);
+        s.logits = t.take(D.n * D.Cp * D.size);
+        linear_act(t, D, in, {P(b), P(b + 1)}, TGT_ACT_RELU, s.m1, s.r1, D.N, D.C, D.M1);
+        linear_act(t, D, s.r1, {P(b + 2), P(b + 3)}, TGT_ACT_RELU, s.m2, s.r2, D.N, D.M1, D.M2);
+        linear(t, D, s.r2, {{P(b + 4), P(b + 5)}}, {s.logits}, D.n, D.M2, D.Cp);
+    }
+    static void readout_back(Tape& t, const Dims& D, const std::vector<const void*>& P, const std::vector<void*>& G, const void* dlogits, void* dm, void* du, void* g,
+                             const Saved& s, Sums& sums) {
+        const int64_t e = kHead + 16 * D.L;
+        linear_act_back(t, D, s.r2, P[e + 4], dlogits, s.m2, TGT_ACT_RELU, dm, G[e + 4], G[e + 5], D.n, D.M2, D.Cp, sums);
+        linear_act_back(t, D, s.r1, P[e + 2], dm, s.m1, TGT_ACT_RELU, du, G[e + 2], G[e + 3], D.N, D.M1, D.M2, sums);
+        linear_back(t, D, s.out, {P[e]}, {du}, g, {G[e]}, {G[e + 1]}, D.N, D.C, D.M1, sums);
+    }
     static void forward(Tape& t, const Dims& D, const std::vector<Tensor>& p, const void* x, const tgt_plan_t* plan, const Tensor& ws, const std::vector<double>& eps, bool keep,
                         Saved& s) {
         const int64_t row = D.N * D.C * D.size;
@@ -270,13 +290,7 @@ struct GtModel {
             add_norm(t, D, x1, f, P(b + 14), P(b + 15), eps[2 * i + 1], l.n2, l.y1);      // y1: the layer's output
             in = l.y1;
         }
-        const int64_t b = kHead + 16 * D.L;
-        s.out = in;
-        s.m1 = t.take(D.N * D.M1 * D.size); s.r1 = t.take(D.N * D.M1 * D.size); s.m2 = t.take(D.N * D.M2 * D.size); s.r2 = t.take(D.N * D.M2 * D.size);
-        s.logits = t.take(D.n * D.Cp * D.size);
-        linear_act(t, D, in, {P(b), P(b + 1)}, TGT_ACT_RELU, s.m1, s.r1, D.N, D.C, D.M1);
-        linear_act(t, D, s.r1, {P(b + 2), P(b + 3)}, TGT_ACT_RELU, s.m2, s.r2, D.N, D.M1, D.M2);
-        linear(t, D, s.r2, {{P(b + 4), P(b + 5)}}, {s.logits}, D.n, D.M2, D.Cp);
+        readout(t, D, p, in, s);
     }
     static void backward(Tape& t, const Dims& D, const std::vector<const void*>& P, const std::vector<void*>& G, const void* x, void* dx, const void* dlogits,
                          const tgt_plan_t* plan, const Tensor& ws, const Saved& s) {
@@ -284,12 +298,10 @@ struct GtModel {
         void *g = t.take(row), *d2 = t.take(row), *d1 = t.take(row), *dy = t.take(row), *d_o = t.take(heads), *dq = t.take(heads), *dk = t.take(heads), *dv = t.take(heads),
              *du = t.take(D.N * std::max(D.ff, D.M1) * D.size), *dm = t.take(D.N * D.M2 * D.size);
         Sums sums;
-        const int64_t mark = t.used, e = kHead + 16 * D.L;
+        const int64_t mark = t.used;
         int64_t high = mark;
         auto done = [&] { sums.run(t, D); high = std::max(high, t.used); t.used = mark; };
-        linear_act_back(t, D, s.r2, P[e + 4], dlogits, s.m2, TGT_ACT_RELU, dm, G[e + 4], G[e + 5], D.n, D.M2, D.Cp, sums);
-        linear_act_back(t, D, s.r1, P[e + 2], dm, s.m1, TGT_ACT_RELU, du, G[e + 2], G[e + 3], D.N, D.M1, D.M2, sums);
-        linear_back(t, D, s.out, {P[e]}, {du}, g, {G[e]}, {G[e + 1]}, D.N, D.C, D.M1, sums);
+        readout_back(t, D, P, G, dlogits, dm, du, g, s, sums);
         done();
         for (int64_t i = D.L - 1; i >= 0; --i) {
             const Layer& l = s.l[i];
@@ -308,6 +320,109 @@ struct GtModel {
         linear_back(t, D, x, {P[0]}, {g}, dx, {G[0]}, {G[1]}, D.n, D.F, D.C, sums);
         done();
         t.used = high;
+    }
+};
+
+// The same with hidden size 64 and 8, 4 or 2 heads, layers on gt_layer.hip.  Packed per layer: O, W1 (two halves of its rows), W2 (two
+// halves of its columns), Wq, Wk, Wv and bo, gamma1, beta1, b1 (two), b2, gamma2, beta2, bq, bk, bv.
+struct FusedGtModel : GtModel {
+    static constexpr int kMats = 8, kVecs = 11;
+    static constexpr int64_t kPre = 3 * 4096 + 5 * 64, kPostA = kPre, kPostB = 2 * 4096 + 4 * 64;      // floats of a worker's partials
+    static bool covers(const Dims& D) { return D.C == 64 && D.W == 64 && D.ff == 128 && (D.H == 8 || D.H == 4 || D.H == 2); }
+    static int64_t unit(const Dims& D) { return tgt_node_frag_bytes(1, D.code) / 2; }
+    static char* weight(const Dims& D, const Saved& s, int64_t l, int i) { return (char*)s.packed + (kMats * l + i) * unit(D); }
+    static char* transposed(const Dims& D, const Saved& s, int64_t l, int i) { return weight(D, s, l + D.L, i); }
+    static float* vec(const Dims& D, const Saved& s, int64_t l, int i) { return (float*)((char*)s.packed + 2 * kMats * D.L * unit(D)) + (kVecs * l + i) * 64; }
+    static void pack(Tape& t, const Dims& D, const std::vector<Tensor>& p, Saved& s) {
+        s.packed = t.take(2 * kMats * D.L * unit(D) + kVecs * D.L * 64 * 4);
+        if (t.dry()) return;
+        std::vector<const void*> m, v;
+        std::vector<int> ld, rows(kMats * D.L, 64), len(kVecs * D.L, 64);
+        for (int64_t l = 0; l < D.L; ++l) {
+            const Tensor* w = &p[kHead + 16 * l];
+            auto part = [&](int i, int64_t elements) { return static_cast<char*>(w[i].data_ptr()) + elements * D.size; };
+            for (const void* q : {part(6, 0), part(10, 0), part(10, 64 * 64), part(12, 0), part(12, 64), part(0, 0), part(2, 0), part(4, 0)}) m.push_back(q);
+            for (int i : {64, 64, 64, 128, 128, 64, 64, 64}) ld.push_back(i);
+            for (const void* q : {part(7, 0), part(8, 0), part(9, 0), part(11, 0), part(11, 64), part(13, 0), part(14, 0), part(15, 0), part(1, 0), part(3, 0), part(5, 0)}) v.push_back(q);
+        }
+        check(tgt_node_pack(m.data(), ld.data(), rows.data(), (int)m.size(), v.data(), len.data(), (int)v.size(), D.code, s.packed, vec(D, s, 0, 0), D.stream), "tgt_node_pack");
+    }
+    static void forward(Tape& t, const Dims& D, const std::vector<Tensor>& p, const void* x, const tgt_plan_t* plan, const Tensor& ws, const std::vector<double>& eps, bool keep,
+                        Saved& s) {
+        const int64_t row = D.N * 64 * D.size;
+        auto P = [&](int64_t i) { return p[i].data_ptr(); };
+        s.l.assign(D.L, Layer{});
+        pack(t, D, p, s);
+        s.rows_in = t.take(row);
+        linear(t, D, x, {{P(0), P(1)}}, {s.rows_in}, D.n, D.F, 64);
+        for (int64_t i = 0; i < D.L; ++i) {
+            Layer& l = s.l[i];
+            if (i > 0 && !keep) l = s.l[0];
+            else {
+                l.q = t.take(row); l.k = t.take(row); l.v = t.take(row); l.o = t.take(row);
+                l.Z = (float*)t.take(4 * D.N * D.H);
+                if (keep) { l.n2.s = t.take(row); l.y1 = t.take(row); }
+            }
+            l.x = i == 0 || !keep ? s.rows_in : s.l[i - 1].y1;      // (without a backward the stream is rewritten in place)
+            if (!keep) l.y1 = l.x;
+        }
+        const int64_t b = kHead;
+        linear(t, D, s.rows_in, {{P(b), P(b + 1)}, {P(b + 2), P(b + 3)}, {P(b + 4), P(b + 5)}}, {s.l[0].q, s.l[0].k, s.l[0].v}, D.N, 64, 64);
+        for (int64_t i = 0; i < D.L; ++i) {
+            const Layer& l = s.l[i];
+            attention(t, D, l, plan, ws);
+            tgt_gt_fwd_args a{};
+            a.rows = D.N; a.dtype = D.code; a.eps1 = (float)eps[2 * i]; a.eps2 = (float)eps[2 * i + 1];
+            a.attn = l.o; a.x = l.x; a.s2 = keep ? l.n2.s : nullptr; a.x_out = l.y1; a.w = weight(D, s, i, 0); a.vec = vec(D, s, i, 0);
+            if (i + 1 < D.L) {
+                const Layer& n = s.l[i + 1];
+                a.q = n.q; a.k = n.k; a.v = n.v; a.w_next = weight(D, s, i + 1, 5); a.v_next = vec(D, s, i + 1, 8);
+            }
+            if (!t.dry()) check(tgt_gt_fwd(&a, D.stream), "tgt_gt_fwd");
+        }
+        readout(t, D, p, s.l[D.L - 1].y1, s);
+    }
+    static void backward(Tape& t, const Dims& D, const std::vector<const void*>& P, const std::vector<void*>& G, const void* x, void* dx, const void* dlogits,
+                         const tgt_plan_t* plan, const Tensor& ws, const Saved& s) {
+        const int64_t row = D.N * 64 * D.size;
+        void *g = t.take(row), *d1 = t.take(row), *d_o = t.take(row), *dq = t.take(row), *dk = t.take(row), *dv = t.take(row), *du = t.take(D.N * D.M1 * D.size),
+             *dm = t.take(D.N * D.M2 * D.size);
+        const int workers = tgt_node_bwd_workers(D.N);
+        float* partial = (float*)t.take(4 * workers * D.L * (kPre + kPostA + kPostB));
+        Sums sums;
+        readout_back(t, D, P, G, dlogits, dm, du, g, s, sums);
+        std::vector<tgt_node_sum> later;
+        auto partial_of = [&](int mats, int ld, std::initializer_list<void*> out) {
+            tgt_node_sum d{};
+            d.partial = partial; d.workers = workers; d.mats = mats; d.rows = 64; d.ld = ld;
+            int i = 0;
+            for (void* o : out) d.out[i++] = o;
+            later.push_back(d);
+            partial += (int64_t)workers * (mats * 4096 + (mats + 2) * 64);
+            return const_cast<float*>(d.partial);
+        };
+        for (int64_t i = D.L - 1; i >= 0; --i) {
+            const Layer& l = s.l[i];
+            void* const* w = &G[kHead + 16 * i];
+            auto part = [&](int k, int64_t elements) { return static_cast<char*>(w[k]) + elements * D.size; };
+            tgt_gt_bwd_args a{};
+            a.rows = D.N; a.dtype = D.code; a.heads = (int)D.H; a.eps1 = (float)(*s.eps)[2 * i]; a.eps2 = (float)(*s.eps)[2 * i + 1];
+            a.g_in = g; a.x = l.x; a.attn = l.o; a.s2 = l.n2.s; a.w = weight(D, s, i, 0); a.w_back = transposed(D, s, i, 0); a.vec = vec(D, s, i, 0); a.Z = l.Z;
+            a.g_out = d1; a.d_attn = d_o; a.nd = static_cast<float*>(ws.data_ptr());
+            tgt_node_bwd_pre_args b{};
+            b.rows = D.N; b.dtype = D.code; b.dq = dq; b.dk = dk; b.dv = dv; b.g_in = d1; b.s = l.x; b.w_back = transposed(D, s, i, 5); b.g_out = g;
+            if (t.dry()) continue;
+            a.partial_a = partial_of(3, 64, {w[6], w[10], part(10, 64 * 64), w[7], w[11], part(11, 64), w[8], w[9]});
+            a.partial_b = partial_of(2, 128, {w[12], part(12, 64), w[13], nullptr, w[14], w[15]});
+            b.partial = partial_of(3, 64, {w[0], w[2], w[4], w[1], w[3], w[5], nullptr, nullptr});
+            check(tgt_gt_bwd(&a, D.stream), "tgt_gt_bwd");
+            check(tgt_sparse_attn_bwd_from_nd(plan, l.q, l.k, l.v, (int)D.H, (int)(64 / D.H), D.code, d_o, dq, dk, dv, ws.data_ptr(), ws.numel(), D.stream),
+                  "tgt_sparse_attn_bwd_from_nd");
+            check(tgt_node_bwd_pre(&b, D.stream), "tgt_node_bwd_pre");
+        }
+        linear_back(t, D, x, {P[0]}, {g}, dx, {G[0]}, {G[1]}, D.n, D.F, 64, sums);
+        if (!t.dry()) check(tgt_node_sums(later.data(), (int)later.size(), D.code, D.stream), "tgt_node_sums");
+        sums.run(t, D);
     }
 };
 
@@ -335,7 +450,7 @@ struct LayeredFn : public torch::autograd::Function<LayeredFn<M>> {
         std::vector<Tensor> save;
         save.reserve(P.size() + 4);
         for (const Tensor& t : P) save.push_back(t.contiguous());
-        Saved s;
+        Saved s{};
         const auto* plan = reinterpret_cast<const tgt_plan_t*>(holder->h);
         Tensor mem = record(x.options(), [&](Tape& t) { M::forward(t, D, save, x.data_ptr(), plan, ws, eps, true, s); });
         Tensor logp = log_probabilities(s, D, classes, x.options());
@@ -358,7 +473,8 @@ struct LayeredFn : public torch::autograd::Function<LayeredFn<M>> {
         const auto* plan = reinterpret_cast<const tgt_plan_t*>(holder->h);
         const Dims D = dims_of<M>(x, sv, dv[0], dv[1], (int64_t)(np - M::kHead - M::kTail) / 16);
         const int64_t classes = dv[2];
-        Saved s;
+        Saved s{};
+        s.eps = &eps;
         Tape where;
         where.base = static_cast<char*>(mem.data_ptr());
         M::forward(where, D, sv, x.data_ptr(), plan, ws, eps, true, s);
@@ -404,7 +520,7 @@ Tensor layered(const char* name, const Tensor& x, at::TensorList P, const c10::i
     c10::DeviceGuard guard(x.device());
     std::vector<Tensor> p;
     for (const Tensor& t : P) p.push_back(t.contiguous());
-    Saved s;
+    Saved s{};
     Tensor mem = record(x.options(), [&](Tape& t) { M::forward(t, D, p, x.data_ptr(), reinterpret_cast<const tgt_plan_t*>(holder->h), ws, e, false, s); });
     return log_probabilities(s, D, classes, x.options());
 }
@@ -412,8 +528,9 @@ Tensor layered_graphormer(const Tensor& x, at::TensorList P, const c10::intrusiv
                           at::ArrayRef<double> eps) {
     return layered<GraphormerModel>("layered_graphormer", x, P, holder, ws, H, tokens, classes, eps);
 }
-Tensor layered_gt(const Tensor& x, at::TensorList P, const c10::intrusive_ptr<PlanHolder>& holder, const Tensor& ws, int64_t H, int64_t classes, at::ArrayRef<double> eps) {
-    return layered<GtModel>("layered_gt", x, P, holder, ws, H, 0, classes, eps);
+Tensor node_gt(const Tensor& x, at::TensorList P, const c10::intrusive_ptr<PlanHolder>& holder, const Tensor& ws, int64_t H, int64_t classes, at::ArrayRef<double> eps) {
+    const bool fused = P.size() >= 24 && FusedGtModel::covers(dims_of<GtModel>(x, P, H, 0, (int64_t)(P.size() - 8) / 16));
+    return fused ? layered<FusedGtModel>("node_gt", x, P, holder, ws, H, 0, classes, eps) : layered<GtModel>("node_gt", x, P, holder, ws, H, 0, classes, eps);
 }
 
 }  // namespace
@@ -421,9 +538,9 @@ Tensor layered_gt(const Tensor& x, at::TensorList P, const c10::intrusive_ptr<Pl
 TORCH_LIBRARY_FRAGMENT(torchgt, m) {
     m.def("layered_graphormer(Tensor x, Tensor[] params, __torch__.torch.classes.torchgt.PlanHolder plan, Tensor workspace, int heads, int tokens, int classes, "
           "float[] eps) -> Tensor");
-    m.def("layered_gt(Tensor x, Tensor[] params, __torch__.torch.classes.torchgt.PlanHolder plan, Tensor workspace, int heads, int classes, float[] eps) -> Tensor");
+    m.def("node_gt(Tensor x, Tensor[] params, __torch__.torch.classes.torchgt.PlanHolder plan, Tensor workspace, int heads, int classes, float[] eps) -> Tensor");
 }
 TORCH_LIBRARY_IMPL(torchgt, CompositeImplicitAutograd, m) {
     m.impl("layered_graphormer", layered_graphormer);
-    m.impl("layered_gt", layered_gt);
+    m.impl("node_gt", node_gt);
 }

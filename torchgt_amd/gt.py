@@ -116,7 +116,7 @@ class GT(nn.Module):
                 plan.handle      # raises if the plan was closed
                 eps, classes = [e for layer in self.layers for e in (layer.layer_norm1.eps, layer.layer_norm2.eps)], P[-1].shape[0]
                 x = padded(P, x, 0, -2)
-                return _ext.op("layered_gt")(x, P, plan.holder, plan.workspace(H, P[2].shape[0] // H), H, classes, eps)
+                return _ext.op("node_gt")(x, P, plan.holder, plan.workspace(H, P[2].shape[0] // H), H, classes, eps)
         x = x.unsqueeze(0)
         (node_feature,) = fused_linear(x, self.node_encoder)
         output = self.input_dropout(node_feature)
