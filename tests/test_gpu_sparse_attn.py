@@ -482,3 +482,37 @@ def test_rows_beyond_four_gib(cuda, bias_kind):
     assert torch.equal(ob[at], o) and torch.equal(Zb[at], Z)
     for i, (b, s) in enumerate(zip(gb, grads)):
         assert torch.equal(b[at] if i < 3 else b, s), i
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("copies", [1, 2])
+@pytest.mark.parametrize("per_head", [False, True])
+def test_plan_order_bias_with_isolated_last_rows(cuda, dtype, copies, per_head):
+    """Rows without edges behind the last edge: their lanes start one position past the end of the bias."""
+    N, E, H, d = 300, 900, 8, 8
+    ei = rand_graph(N - 130, E, 3)
+    q, k, v, bias, dout = make_inputs(N, E, H, d, dtype, "edge_head" if per_head else "edge", 4)
+    want = oracle_fwd_bwd(q, k, v, bias, ei, dout)
+    plan = GraphPlan(ei.to(cuda), N)
+    b = bias.to(cuda).requires_grad_(True)
+    t = [x.to(cuda).requires_grad_(True) for x in (q, k, v)]
+    in_order = plan.sort_bias(b) if copies == 2 else b[plan.edge_order()]
+    assert in_order.shape[0] == copies * E
+    out, Z = sparse_attention(t[0], t[1], t[2], plan=plan, edge_bias=in_order, return_z=True, bias_in_plan_order=True)
+    grads = torch.autograd.grad(out, t + [b], dout.to(cuda))
+    for name, a, r in zip(("out", "Z", "dq", "dk", "dv", "dbias"), (out, Z) + grads, want[:2] + want[2]):
+        assert err(a, r) <= TOL[dtype], f"{name}: {err(a, r)}"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("plan_order", [False, True])
+@pytest.mark.parametrize("shape", [(0,), (0, 8)])
+def test_bias_of_a_graph_without_edges(cuda, dtype, plan_order, shape):
+    """An empty bias has no memory behind it: nothing of it may be asked for."""
+    N, H, d = 70, 8, 8
+    plan = GraphPlan(torch.zeros(2, 0, dtype=torch.long, device=cuda), N)
+    q, k, v, _, dout = make_inputs(N, 1, H, d, dtype, "none", 1)
+    t = [x.to(cuda).requires_grad_(True) for x in (q, k, v)] + [torch.zeros(shape, dtype=dtype, device=cuda, requires_grad=True)]
+    out = sparse_attention(t[0], t[1], t[2], plan=plan, edge_bias=t[3], bias_in_plan_order=plan_order)
+    grads = torch.autograd.grad(out, t, dout.to(cuda))
+    assert not out.any() and grads[3].shape == shape and not any(g.any() for g in grads[:3])

@@ -16,6 +16,7 @@
 // walked by whole workgroups in segments of kBlockSeg edges whose partial sums the
 // last-arriving workgroup adds in a fixed order.
 #include "common.h"
+#include "edge_slots.h"
 #include <stdlib.h>
 #include <algorithm>
 #include <mutex>
@@ -635,11 +636,11 @@ __device__ __forceinline__ void walk_record(const Common& c, const SideArgs& s, 
     for (int u = 0; u < kUnroll; ++u) ok[u] = slot + u * S < n;
     if (HASB == 2) {          // bias rows in this view's sorted order: row = sorted position
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) ed[u] = start + min(slot + u * S, max(n - 1, 0));
+        for (int u = 0; u < kUnroll; ++u) ed[u] = edge_of_slot(start, n, slot + u * S);
     } else if (HASB) {
         if (s.eid_is_map) {   // the bias rows are named by a map from sorted positions, not by the caller's edge ids
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) ed[u] = s.eid[start + min(slot + u * S, max(n - 1, 0))];
+            for (int u = 0; u < kUnroll; ++u) ed[u] = s.eid[edge_of_slot(start, n, slot + u * S)];
         } else {
             const int4 e4 = rec_edges_early<T, MODE>() ? rec.eids : *reinterpret_cast<const int4*>(rec.eid_p);
             ed[0] = e4.x; ed[1] = e4.y; ed[2] = e4.z; ed[3] = e4.w;
@@ -1091,7 +1092,7 @@ static int run_fwd(const Call& c) {
     const int nb = sch->fwd_blocks;
     if (nb > 0) {
         KernelTimer t(KS_FWD, c.st, !c.no_alloc);       // the entry point that allocates nothing creates no events either
-        const bool hb = c.bias_mode != TGT_BIAS_NONE;
+        const bool hb = c.bias_mode != TGT_BIAS_NONE && c.plan->E > 0;       // (a graph without edges has no bias row that a lane could read)
         if (c.init != nullptr && (c.bias_mode & TGT_BIAS_PLAN_ORDER)) {
             set_error("block attention takes the bias in the caller's edge order");
             return TGT_ERR_UNSUPPORTED;
@@ -1162,7 +1163,7 @@ static int run_bwd(const Call& c) {
     const int nb = sch->bwd_blocks;
     if (nb > 0) {
         KernelTimer t(KS_BWD, c.st);
-        const bool hb = c.bias_mode != TGT_BIAS_NONE;
+        const bool hb = c.bias_mode != TGT_BIAS_NONE && c.plan->E > 0;       // (a graph without edges has no bias row that a lane could read)
         if (c.init != nullptr && (c.bias_mode & TGT_BIAS_PLAN_ORDER)) {
             set_error("block attention takes the bias in the caller's edge order");
             return TGT_ERR_UNSUPPORTED;
