@@ -1,0 +1,49 @@
+"""Which calls the whole-model operators take: a call that they do not cover gives what the layers one by one give."""
+import pytest
+import torch
+
+from oracle import encoder_layer as oel
+from torchgt_amd import Graphormer, GraphPlan
+
+pytestmark = pytest.mark.gpu
+
+
+def edges_of(n, tokens, seed):
+    g = torch.Generator().manual_seed(seed)
+    e = torch.cat([torch.randint(0, n, (2, 4 * n), generator=g), torch.arange(n).repeat(2, 1)], 1)
+    for t in range(tokens):      # a token is joined to every row in front of it
+        old = torch.arange(n + t)
+        e = torch.cat([e + 1, torch.stack([torch.zeros_like(old), old + 1]), torch.stack([old + 1, torch.zeros_like(old)])], 1)
+    return e
+
+
+def scaled(model, seed, dtype, device):
+    g = torch.Generator().manual_seed(seed)
+    with torch.no_grad():
+        for p in model.parameters():
+            p.copy_(p + torch.randn(p.shape, generator=g) * 0.1 if p.dim() == 1 else torch.randn(p.shape, generator=g) / p.shape[-1] ** 0.5)
+    return model.to(device, dtype)
+
+
+@pytest.mark.parametrize("hidden", [64, 128])
+@pytest.mark.parametrize("tokens", [0, 1, 2, 3])
+def test_token_counts(cuda, tokens, hidden):
+    """Rows 1 .. of the sequence come back (models/graphormer_dist_node_level.py:391) for any number of global tokens."""
+    n, layers, heads, classes = 100, 2, 8, 7
+    print(f"tokens case: {tokens} hidden={hidden}", flush=True)
+    torch.manual_seed(tokens)
+    model = scaled(Graphormer(layers, heads, 20, hidden, classes, 1, 0.0, 0.0, 0.0, hidden, tokens), 2, torch.float32, cuda)
+    x, e = torch.randn(n, 20), edges_of(n, tokens, 3)
+    want = torch.from_numpy(oel.graphormer_forward(x.numpy(), {k: v.double().cpu().numpy() for k, v in model.state_dict().items()}, e.numpy(), layers, heads))
+    plan = GraphPlan(e.to(cuda), n + tokens)
+    w = torch.randn(want.shape, generator=torch.Generator().manual_seed(4)).to(cuda)
+    grads = []
+    for one in (True, False):
+        model.one_operator = one
+        model.zero_grad(set_to_none=True)
+        out = model(x.to(cuda), None, plan, attn_type="sparse")
+        assert out.shape == want.shape == (n + tokens - 1, classes)
+        assert float((out.double().cpu() - want).abs().max()) <= 3e-5 * float(want.abs().max())
+        (out * w).sum().backward()
+        grads.append(torch.cat([p.grad.flatten() for p in model.parameters() if p.grad is not None]))
+    assert float((grads[0] - grads[1]).norm()) <= 2e-5 * float(grads[1].norm())

@@ -526,6 +526,7 @@ Tensor layered(const char* name, const Tensor& x, at::TensorList P, const c10::i
 }
 Tensor layered_graphormer(const Tensor& x, at::TensorList P, const c10::intrusive_ptr<PlanHolder>& holder, const Tensor& ws, int64_t H, int64_t tokens, int64_t classes,
                           at::ArrayRef<double> eps) {
+    TORCH_CHECK(tokens == 1, "layered_graphormer: one global token (its rows are the nodes', the model's are 1 .. of the sequence)");
     return layered<GraphormerModel>("layered_graphormer", x, P, holder, ws, H, tokens, classes, eps);
 }
 Tensor node_gt(const Tensor& x, at::TensorList P, const c10::intrusive_ptr<PlanHolder>& holder, const Tensor& ws, int64_t H, int64_t classes, at::ArrayRef<double> eps) {

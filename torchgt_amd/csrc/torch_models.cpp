@@ -228,6 +228,7 @@ Tensor node_graphormer(const Tensor& x, at::TensorList P, const c10::intrusive_p
     on_gpu(x, "node_graphormer");
     TORCH_CHECK(x.dim() == 2 && x.is_contiguous(), "node_graphormer: x must be a contiguous [n, features]");
     TORCH_CHECK(P.size() >= 7 && (P.size() - 7) % 16 == 0, "node_graphormer takes 7 + 16 L parameter tensors");
+    TORCH_CHECK(tokens == 1, "node_graphormer: one global token (its rows are the nodes', the model's are 1 .. of the sequence)");
     GraphormerDims D{};
     D.L = (int64_t)(P.size() - 7) / 16; D.n = x.size(0); D.tokens = tokens; D.N = D.n + tokens; D.F = x.size(1); D.H = H;
     TORCH_CHECK((int64_t)eps.size() == 2 * D.L + 1, "node_graphormer: 2 L + 1 values of eps");

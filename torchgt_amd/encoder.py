@@ -232,8 +232,10 @@ class Graphormer(nn.Module):
 
     def _one_operator(self, x, attn_bias, edge_index, perturb, attn_type):
         """The model's parameters in the order of the whole-model operators when one of them covers this call - sparse
-        attention without a bias, no dropout at work, every linear with its bias, one dtype - else None."""
-        if not self.one_operator or attn_type != "sparse" or attn_bias is not None or perturb is not None or edge_index is None:
+        attention without a bias, no dropout at work, every linear with its bias, one dtype, one global token (the rows that
+        come back are 1 .. of the sequence, :391, whatever the number of tokens: the operators return the nodes' rows) -
+        else None."""
+        if not self.one_operator or self.num_global_node != 1 or attn_type != "sparse" or attn_bias is not None or perturb is not None or edge_index is None:
             return None
         if x.dim() != 2 or not x.is_cuda or x.dtype not in _DT:
             return None
@@ -254,10 +256,10 @@ class Graphormer(nn.Module):
         P = self._one_operator(x, attn_bias, edge_index, perturb, attn_type)
         if P is not None:
             # the whole model as one operator and one autograd node
-            plan = edge_index if isinstance(edge_index, GraphPlan) else get_plan(edge_index, x.shape[0] + self.num_global_node)
+            plan = edge_index if isinstance(edge_index, GraphPlan) else get_plan(edge_index, x.shape[0] + 1)
             plan.handle      # raises if the plan was closed
             eps = [e for layer in self.layers for e in (layer.self_attention_norm.eps, layer.ffn_norm.eps)] + [self.final_ln.eps]
-            H, tokens, classes, ve = self.num_heads, self.num_global_node, P[-1].shape[0], 4 if x.dtype == torch.float32 else 8
+            H, tokens, classes, ve = self.num_heads, 1, P[-1].shape[0], 4 if x.dtype == torch.float32 else 8
             if self._fused(P, H):      # kernels that take a layer's node-local part in one pass each way
                 if x.shape[1] % ve:
                     pad = (-x.shape[1]) % ve
