@@ -3,7 +3,7 @@ import pytest
 import torch
 
 from oracle import encoder_layer as oel
-from torchgt_amd import Graphormer, GraphPlan
+from torchgt_amd import GT, Graphormer, GraphPlan
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +47,28 @@ def test_token_counts(cuda, tokens, hidden):
         (out * w).sum().backward()
         grads.append(torch.cat([p.grad.flatten() for p in model.parameters() if p.grad is not None]))
     assert float((grads[0] - grads[1]).norm()) <= 2e-5 * float(grads[1].norm())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("kind,hidden,classes", [("gt", 64, 40), ("gt", 128, 47), ("graphormer", 64, 40), ("graphormer", 128, 40)])
+def test_autocast(cuda, kind, hidden, classes, dtype):
+    """Under autocast the log-probabilities are float32, whichever way the model runs, and the gradients those of the model's dtype."""
+    n, layers, heads = 200, 2, 8
+    print(f"autocast case: {kind} hidden={hidden} {dtype}", flush=True)
+    cls, tokens = (GT, 0) if kind == "gt" else (Graphormer, 1)
+    torch.manual_seed(1)
+    model = scaled(cls(layers, heads, 32, hidden, classes, 1, 0.0, 0.0, 0.0, hidden, tokens), 2, dtype, cuda)
+    x, plan = torch.randn(n, 32).to(cuda, dtype), GraphPlan(edges_of(n, tokens, 3).to(cuda), n + tokens)
+    w = torch.randn(n, classes, generator=torch.Generator().manual_seed(4)).to(cuda)
+    got = []
+    for one in (True, False):
+        model.one_operator = one
+        model.zero_grad(set_to_none=True)
+        with torch.autocast("cuda", torch.bfloat16):
+            out = model(x, None, plan, attn_type="sparse")
+            loss = (out.float() * w).sum()
+        loss.backward()
+        assert out.dtype == torch.float32
+        got.append([out.detach(), torch.cat([p.grad.float().flatten() for p in model.parameters() if p.grad is not None])])
+    for a, b in zip(*got):      # two orders of float32 sums; bf16: two orders of roundings
+        assert float((a - b).norm()) <= (2e-5 if dtype == torch.float32 else 3e-2) * float(b.norm())

@@ -437,7 +437,9 @@ Dims dims_of(const Tensor& x, at::TensorList P, int64_t H, int64_t tokens, int64
     D.code = dtype_code(x); D.size = (int)x.element_size(); D.stream = stream_of(x);
     return D;
 }
+// In the dtype of x also under autocast: the kernels of the backward are told that its gradient has that dtype.
 Tensor log_probabilities(const Saved& s, const Dims& D, int64_t classes, const at::TensorOptions& opt) {
+    c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
     return at::log_softmax(at::from_blob(s.logits, {D.n, D.Cp}, opt).narrow(1, 0, classes), 1);
 }
 
@@ -480,6 +482,7 @@ struct LayeredFn : public torch::autograd::Function<LayeredFn<M>> {
         M::forward(where, D, sv, x.data_ptr(), plan, ws, eps, true, s);
         Tensor dlogits = at::_log_softmax_backward_data(grads[0], logp, 1, logp.scalar_type());
         if (D.Cp != classes) dlogits = at::constant_pad_nd(dlogits, {0, D.Cp - classes});
+        TORCH_CHECK(dlogits.scalar_type() == x.scalar_type(), "gradient of the logits in another dtype than x");
         dlogits = dlogits.contiguous();
         std::vector<std::vector<int64_t>> shapes;
         std::vector<const void*> W;

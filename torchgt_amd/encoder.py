@@ -120,6 +120,11 @@ def model_parameters(model, dtype):
     return tree.parameters(dtype, model.training) if tree.by_layer() else None
 
 
+def autocast_to_float32(x):
+    """Whether autocast makes the log-softmax of rows of x's dtype float32: the operators compute it in x's dtype."""
+    return x.dtype is not torch.float32 and torch.is_autocast_enabled("cuda")
+
+
 def padded(P, x, at, last):
     """Zero-pads what the linears read in 16-byte pieces: the features of x and of P[at], the classes of P[last] and P[last + 1]."""
     ve = 4 if x.dtype == torch.float32 else 8
@@ -237,7 +242,7 @@ class Graphormer(nn.Module):
         else None."""
         if not self.one_operator or self.num_global_node != 1 or attn_type != "sparse" or attn_bias is not None or perturb is not None or edge_index is None:
             return None
-        if x.dim() != 2 or not x.is_cuda or x.dtype not in _DT:
+        if x.dim() != 2 or not x.is_cuda or x.dtype not in _DT or autocast_to_float32(x):
             return None
         return model_parameters(self, x.dtype)
 

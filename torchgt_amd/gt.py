@@ -10,7 +10,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _ext, _lib
-from .encoder import init_params, model_parameters, padded
+from .encoder import autocast_to_float32, init_params, model_parameters, padded
 from .multi_head_attention import MultiHeadAttention, fused_linear
 from .plan import GraphPlan, get_plan
 
@@ -107,7 +107,8 @@ class GT(nn.Module):
         return names + [n for j in range(self.MLP_layer.L + 1) for n in both(f"MLP_layer.FC_layers.{j}")]
 
     def forward(self, x, attn_bias, edge_index, perturb=None, attn_type=None):
-        if self.one_operator and attn_type == "sparse" and edge_index is not None and x.dim() == 2 and x.is_cuda and x.dtype in _DT and self.MLP_layer.L == 2:
+        if self.one_operator and attn_type == "sparse" and edge_index is not None and x.dim() == 2 and x.is_cuda and x.dtype in _DT and \
+                self.MLP_layer.L == 2 and not autocast_to_float32(x):
             P = model_parameters(self, x.dtype)
             ve, H = 4 if x.dtype == torch.float32 else 8, self.layers[0].self_attention.num_heads
             if P is not None and all(p.shape[0] % ve == 0 for p in P[:-2]) and P[2].shape[0] % H == 0:
