@@ -244,3 +244,21 @@ def test_dense_layer_as_one_operator_equals_layer_op_by_op(cuda, dtype, from_ids
             assert (a.double() - r.double()).abs().max().item() <= 1e-5 * max(r.double().abs().max().item(), 1e-30), name
         else:
             assert torch.equal(a, r), name
+
+
+@pytest.mark.parametrize("edge_type", ["single_hop", "multi_hop"])
+@pytest.mark.parametrize("one_operator", [True, False])
+def test_batches_that_are_not_on_the_gpu_are_refused(cuda, edge_type, one_operator):
+    """Every tensor of the batch is looked at before a kernel is given its address."""
+    b, s = 2, 5
+    m = Graphormer(2, 8, 64, 0.0, 0.0, 64, "ZINC", edge_type, 5, 0.0, 1).to(cuda)
+    m.one_operator = one_operator
+    ids = lambda *shape: torch.ones(shape, dtype=torch.long, device=cuda)
+    batch = dict(x=ids(b, s, 1), in_degree=ids(b, s), out_degree=ids(b, s), attn_bias=torch.zeros(b, s + 1, s + 1, device=cuda), spatial_pos=ids(b, s, s),
+                 attn_edge_type=ids(b, s, s, 1), edge_input=ids(b, s, s, 3, 1))
+    assert (m._one_operator(types.SimpleNamespace(**batch)) is not None) == one_operator
+    for name in batch:
+        if name != ("attn_edge_type" if edge_type == "multi_hop" else "edge_input"):
+            with pytest.raises(RuntimeError, match="on the GPU|GPU only"):
+                m(types.SimpleNamespace(**{**batch, name: batch[name].cpu()}))
+    assert m(types.SimpleNamespace(**batch)).shape == (b, 1)

@@ -236,6 +236,7 @@ Tensor dense_attention_ids(const Tensor& q, const Tensor& k, const Tensor& v, co
 // the reference's int64 ids to the packed form, once per batch
 std::tuple<Tensor, Tensor> dense_ids_pack(const Tensor& spatial_pos, const Tensor& edge_type, int64_t num_spatial, int64_t num_edges) {
     on_gpu(spatial_pos, "dense_ids_pack");
+    same_gpu(edge_type, spatial_pos, "dense_ids_pack", "edge_type");
     TORCH_CHECK(spatial_pos.dim() == 3 && edge_type.dim() == 4 && spatial_pos.size(1) == spatial_pos.size(2) &&
                     edge_type.size(0) == spatial_pos.size(0) && edge_type.size(1) == spatial_pos.size(1) &&
                     edge_type.size(2) == spatial_pos.size(1), "spatial_pos [b, s, s] and attn_edge_type [b, s, s, F] expected");

@@ -31,6 +31,11 @@ inline void on_gpu(const Tensor& t, const char* op) {
     TORCH_CHECK(t.is_cuda(), op, " needs GPU tensors (there is no CPU implementation)");
 }
 
+// what a kernel reads has to be on the GPU of its first operand: a host pointer or another GPU's is a fault there
+inline void same_gpu(const Tensor& t, const Tensor& first, const char* op, const char* name) {
+    TORCH_CHECK(t.defined() && t.is_cuda() && t.device() == first.device(), op, ": ", name, " must be on the GPU ", first.device(), " like the other operands");
+}
+
 // Owner of a tgt_plan_t: the Python plan object holds one, and so does every autograd node that will need the plan
 // in its backward - the plan lives until the last of them lets go.
 struct PlanHolder : torch::CustomClassHolder {

@@ -511,9 +511,11 @@ Tensor layered(const char* name, const Tensor& x, at::TensorList P, const c10::i
     TORCH_CHECK(L >= 1 && per % 16 == 0 && (int64_t)eps.size() == 2 * L + (M::kTail == 4 ? 1 : 0), name, ": 16 parameters and two eps per layer");
     bool train = x.requires_grad();
     for (const Tensor& t : P) {
-        TORCH_CHECK(t.defined() && t.is_cuda() && t.scalar_type() == x.scalar_type(), name, ": parameters must be GPU tensors of x's dtype");
+        same_gpu(t, x, name, "every parameter");
+        TORCH_CHECK(t.scalar_type() == x.scalar_type(), name, ": parameters must be GPU tensors of x's dtype");
         train = train || t.requires_grad();
     }
+    same_gpu(ws, x, name, "the plan");
     const Dims D = dims_of<M>(x, P, H, tokens, L);
     M::check_shapes(name, D, P);
     TORCH_CHECK(classes >= 1 && classes <= D.Cp && D.W % H == 0, name, ": classes or heads");

@@ -234,9 +234,11 @@ Tensor node_graphormer(const Tensor& x, at::TensorList P, const c10::intrusive_p
     TORCH_CHECK((int64_t)eps.size() == 2 * D.L + 1, "node_graphormer: 2 L + 1 values of eps");
     bool train = false;
     for (const Tensor& t : P) {
-        TORCH_CHECK(t.defined() && t.is_cuda() && t.scalar_type() == x.scalar_type(), "parameters must be GPU tensors of x's dtype");
+        same_gpu(t, x, "node_graphormer", "every parameter");
+        TORCH_CHECK(t.scalar_type() == x.scalar_type(), "parameters must be GPU tensors of x's dtype");
         train = train || t.requires_grad();
     }
+    same_gpu(ws, x, "node_graphormer", "the plan");
     const Tensor* q = P.data() + 3;
     TORCH_CHECK(P[0].dim() == 2 && P[0].size(0) == kWidth && P[0].size(1) == D.F && P[1].numel() == kWidth && P[2].dim() == 2 && P[2].size(0) == tokens &&
                     P[2].size(1) == kWidth, "node_graphormer: encoder shapes");
@@ -497,9 +499,15 @@ Tensor graph_graphormer(const Tensor& x, const Tensor& in_degree, const Tensor& 
     TORCH_CHECK(H == 8 || H == 4 || H == 2, "graph_graphormer: 8, 4 or 2 heads");
     bool train = false;
     for (const Tensor& t : P) {
-        TORCH_CHECK(t.defined() && t.is_cuda() && t.scalar_type() == P[0].scalar_type(), "graph_graphormer: parameters must be GPU tensors of one dtype");
+        same_gpu(t, attn_bias, "graph_graphormer", "every parameter");
+        TORCH_CHECK(t.scalar_type() == P[0].scalar_type(), "graph_graphormer: parameters must be GPU tensors of one dtype");
         train = train || t.requires_grad();
     }
+    same_gpu(x, attn_bias, "graph_graphormer", "x");
+    same_gpu(in_degree, attn_bias, "graph_graphormer", "in_degree");
+    same_gpu(out_degree, attn_bias, "graph_graphormer", "out_degree");
+    same_gpu(spatial_pos, attn_bias, "graph_graphormer", "spatial_pos");
+    same_gpu(edge_ids, attn_bias, "graph_graphormer", multi_hop ? "edge_input" : "attn_edge_type");
     for (int i : {0, 1, 2, 3}) TORCH_CHECK(P[i].dim() == 2 && P[i].size(1) == kWidth, "graph_graphormer: feature tables are [rows, 64]");
     for (int i : {4, 5, 6}) TORCH_CHECK(P[i].dim() == 2 && P[i].size(1) == H, "graph_graphormer: bias tables are [rows, heads]");
     TORCH_CHECK(!multi_hop || P[7].numel() % (H * H) == 0, "graph_graphormer: hop matrices");

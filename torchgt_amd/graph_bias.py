@@ -22,11 +22,17 @@ def _stream(t):
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
+def same_gpu(who, first, *others):
+    """Refuses what a kernel of the first operand's GPU cannot read: a host pointer there is a fault."""
+    if not first.is_cuda or any(t.device != first.device for t in others):
+        raise RuntimeError(f"{who} runs on the GPU only (no CPU fallback): all operands have to be on one GPU, got "
+                           f"{', '.join(str(t.device) for t in (first,) + others)}")
+
+
 class GraphAttnBiasFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, attn_bias, spatial_pos, attn_edge_type, spatial_table, edge_table, virtual_dist):
-        if not attn_bias.is_cuda:
-            raise RuntimeError("GraphAttnBias runs on the GPU only (no CPU fallback)")
+        same_gpu("GraphAttnBias", attn_bias, spatial_pos, attn_edge_type, spatial_table, edge_table, virtual_dist)
         dt = spatial_table.dtype
         if dt not in _DT:
             raise TypeError(f"unsupported dtype {dt}")
@@ -69,8 +75,7 @@ class GraphAttnBiasMultiHopFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, attn_bias, spatial_pos, edge_input, spatial_table, edge_table, edge_dis_weight, virtual_dist,
                 multi_hop_max_dist):
-        if not attn_bias.is_cuda:
-            raise RuntimeError("GraphAttnBias runs on the GPU only (no CPU fallback)")
+        same_gpu("GraphAttnBias", attn_bias, spatial_pos, edge_input, spatial_table, edge_table, edge_dis_weight, virtual_dist)
         dt = spatial_table.dtype
         if dt not in _DT:
             raise TypeError(f"unsupported dtype {dt}")
@@ -136,8 +141,7 @@ class GraphAttnBias(nn.Module):
             from . import _ext
             from .core_attention import GraphBiasIds
             sp_w, e_w, vd_w = self.spatial_pos_encoder.weight, self.edge_encoder.weight, self.graph_token_virtual_distance.weight
-            if not batched_data.attn_bias.is_cuda:
-                raise RuntimeError("GraphAttnBias runs on the GPU only (no CPU fallback)")
+            same_gpu("GraphAttnBias", batched_data.attn_bias, batched_data.spatial_pos, batched_data.attn_edge_type, sp_w, e_w, vd_w)
             sp16, et16 = _ext.op("dense_ids_pack")(batched_data.spatial_pos, batched_data.attn_edge_type, sp_w.shape[0], e_w.shape[0])
             build = lambda: GraphAttnBiasFunction.apply(batched_data.attn_bias, batched_data.spatial_pos,
                                                         batched_data.attn_edge_type, sp_w, e_w, vd_w)

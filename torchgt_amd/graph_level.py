@@ -12,7 +12,7 @@ import torch.nn as nn
 from . import _ext, _lib
 from .core_attention import GraphBiasIds
 from .encoder import LAYER_PARAMETERS, _TREES, FeedForwardNetwork, ModuleTree, init_params
-from .graph_bias import GraphAttnBias
+from .graph_bias import GraphAttnBias, same_gpu
 from .multi_head_attention import MultiHeadAttention, fused_linear
 
 _DT = {torch.float32: _lib.DTYPE_F32, torch.bfloat16: _lib.DTYPE_BF16}
@@ -25,8 +25,7 @@ def _stream(t):
 class GraphNodeFeatureFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, in_degree, out_degree, atom_table, in_table, out_table, graph_token):
-        if not x.is_cuda:
-            raise RuntimeError("GraphNodeFeature runs on the GPU only (no CPU fallback)")
+        same_gpu("GraphNodeFeature", x, in_degree, out_degree, atom_table, in_table, out_table, graph_token)
         dt = atom_table.dtype
         if dt not in _DT:
             raise TypeError(f"unsupported dtype {dt}")

@@ -11,6 +11,7 @@ import torch.nn.functional as F
 
 from . import _ext, _lib
 from .encoder import autocast_to_float32, init_params, model_parameters, padded
+from .graph_bias import same_gpu
 from .multi_head_attention import MultiHeadAttention, fused_linear
 from .plan import GraphPlan, get_plan
 
@@ -132,8 +133,7 @@ class EmbeddingSumFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, table):
-        if not x.is_cuda:
-            raise RuntimeError("torchgt_amd kernels run on the GPU only (no CPU fallback)")
+        same_gpu("EmbeddingSum", x, table)
         dt = table.dtype
         if dt not in _DT:
             raise TypeError(f"unsupported dtype {dt}")
