@@ -1,0 +1,42 @@
+"""What keeps a model off the whole-model operators, as far as the model itself decides it (no GPU needed): a model that they do not
+cover has to run module by module, not raise and not lose what its modules do."""
+import pytest
+import torch
+import torch.nn as nn
+
+from torchgt_amd import GT, GraphLevelGraphormer, Graphormer
+from torchgt_amd.encoder import model_parameters
+
+
+def build(kind, dropout=0.0, input_dropout=0.0, attention_dropout=0.0, layers=2):
+    if kind == "graph":
+        return GraphLevelGraphormer(layers, 8, 64, dropout, input_dropout, 64, "ZINC", "single_hop", 5, attention_dropout, 1)
+    cls, tokens = (GT, 0) if kind == "gt" else (Graphormer, 1)
+    return cls(layers, 8, 16, 64, 4, 1, dropout, input_dropout, attention_dropout, 64, tokens)
+
+
+def parameters(model):
+    return model._operator_parameters() if isinstance(model, GraphLevelGraphormer) else model_parameters(model, torch.float32)
+
+
+KINDS = ["graphormer", "gt", "graph"]
+
+
+class Attention(nn.Module):      # a module of the user's own, without the parameters of the library's
+    def forward(self, x, attn_bias=None, edge_index=None, attn_type=None):
+        return x
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("where", ["layer", "attention", "last", "no layers"])
+def test_a_module_of_another_kind_in_the_tree(kind, where):
+    """``parameters`` says no, before and after, and yes again once the library's module is back."""
+    model = build(kind)
+    assert parameters(model) is not None
+    owner, name = {"layer": (model.layers, "0"), "attention": (model.layers[1], "self_attention"), "no layers": (model, "layers"),
+                   "last": (model, "MLP_layer" if kind == "gt" else "final_ln")}[where]
+    kept = owner._modules[name]
+    setattr(owner, name, {"last": nn.Identity(), "no layers": nn.ModuleList()}.get(where, Attention()))
+    assert parameters(model) is None and parameters(model) is None
+    setattr(owner, name, kept)
+    assert parameters(model) is not None

@@ -65,7 +65,8 @@ class ModuleTree:
                 self.links.append((module._modules, name, child))
             return child
 
-        self.missing = False
+        step(root, "layers")
+        self.missing = False      # a module of the names is not there: somebody's own module stands in its place
         for full in names:
             *path, leaf = full.split(".")
             m = root
@@ -73,14 +74,14 @@ class ModuleTree:
                 m = step(m, part) if m is not None else None
             if m is None:
                 self.missing = True
-                return
+                break
             self.slots.append((m._parameters, leaf))
         self.count = len(root.layers)
         self.layers = root.layers._modules
         self.dropouts = [m for n, m in root.named_modules() if n.rsplit(".", 1)[-1] in dropouts]
 
     def current(self):
-        if self.missing or len(self.layers) != self.count:
+        if len(self.layers) != self.count:
             return False
         for d, name, child in self.links:
             if d.get(name) is not child:
@@ -102,7 +103,9 @@ class ModuleTree:
         return P
 
     def by_layer(self):
-        """Whether no layer was asked to run step by step."""
+        """Whether every layer has the modules of a layer and none was asked to run step by step."""
+        if self.missing:
+            return False
         for layer in self.layers.values():
             if "one_operator" in layer.__dict__ or not layer.one_operator or not layer.self_attention.one_operator:
                 return False

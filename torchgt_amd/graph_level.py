@@ -195,11 +195,15 @@ class Graphormer(nn.Module):
 
     def _one_operator(self, batched_data):
         """The model's parameters in the operator's order when ``torch.ops.torchgt.graph_graphormer`` covers this call - the
-        bias as a tensor, hidden and feed-forward width 64, at most 64 outputs, no dropout at work but the attention's, one
-        dtype - else None."""
-        if not self.one_operator or self.bias_from_ids or not batched_data.attn_bias.is_cuda or len(self.layers) == 0 or batched_data.x.numel() == 0:
+        bias as a tensor and what ``_operator_parameters`` asks of the model - else None."""
+        if not self.one_operator or self.bias_from_ids or not batched_data.attn_bias.is_cuda or batched_data.x.numel() == 0:
             return None
-        multi_hop = self.graph_attn_bias.edge_type == "multi_hop"
+        return self._operator_parameters()
+
+    def _operator_parameters(self):
+        """The parameters in the operator's order if the model has hidden and feed-forward width 64, at most 64 outputs, no
+        dropout at work but the attention's and one dtype, else None."""
+        multi_hop = getattr(self.graph_attn_bias, "edge_type", None) == "multi_hop"
         head = "out_proj" if hasattr(self, "out_proj") else "downstream_out_proj"
         tree = _TREES.get(self)
         if tree is None or not tree.current():
@@ -210,15 +214,16 @@ class Graphormer(nn.Module):
                 names += [f"layers.{i}.{k}" for k in LAYER_PARAMETERS]
             names += ["final_ln.weight", "final_ln.bias", f"{head}.weight", f"{head}.bias"]
             tree = _TREES[self] = ModuleTree(self, names, ["self_attention_dropout", "ffn_dropout", "input_dropout"])
+        dtype = getattr(getattr(self.final_ln, "weight", None), "dtype", None)
+        P = tree.parameters(dtype, self.training) if tree.by_layer() else None
+        if P is None:
+            return None
         first = self.layers[0].self_attention.dist_attn.local_attn
         for layer in self.layers:
             core = layer.self_attention.dist_attn.local_attn
-            # (a flag set on a layer itself asks for that layer's own way of running, either one)
-            if "one_operator" in layer.__dict__ or not layer.one_operator or layer.self_attention.num_heads not in (2, 4, 8) or \
-                    core.attention_dropout_rate != first.attention_dropout_rate or core.dense_bf16_products:
+            if layer.self_attention.num_heads not in (2, 4, 8) or core.attention_dropout_rate != first.attention_dropout_rate or core.dense_bf16_products:
                 return None
-        P = tree.parameters(self.final_ln.weight.dtype, self.training)
-        if P is None or P[0].dtype not in _DT or P[0].shape[1] != 64 or P[-1].shape[0] > 64 or P[4].shape[1] != self.layers[0].self_attention.num_heads or \
+        if P[0].dtype not in _DT or P[0].shape[1] != 64 or P[-1].shape[0] > 64 or P[4].shape[1] != self.layers[0].self_attention.num_heads or \
                 any(p.shape[0] != 64 or p.shape[-1] != 64 for p in P[8 if multi_hop else 7:-4]):
             return None
         return P

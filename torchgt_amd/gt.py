@@ -105,20 +105,29 @@ class GT(nn.Module):
             for part in ("self_attention.linear_q", "self_attention.linear_k", "self_attention.linear_v", "O", "layer_norm1", "FFN_layer1", "FFN_layer2",
                          "layer_norm2"):
                 names += both(f"layers.{i}.{part}")
-        return names + [n for j in range(self.MLP_layer.L + 1) for n in both(f"MLP_layer.FC_layers.{j}")]
+        return names + [n for j in range(3) for n in both(f"MLP_layer.FC_layers.{j}")]
+
+    def _one_operator(self, x, edge_index, attn_type):
+        """The model's parameters in the operator's order when ``torch.ops.torchgt.node_gt`` covers this call, else None."""
+        if not self.one_operator or attn_type != "sparse" or edge_index is None or x.dim() != 2 or not x.is_cuda or x.dtype not in _DT or \
+                autocast_to_float32(x) or getattr(self.MLP_layer, "L", None) != 2:
+            return None
+        P = model_parameters(self, x.dtype)
+        ve = 4 if x.dtype == torch.float32 else 8
+        if P is None or any(p.shape[0] % ve for p in P[:-2]) or P[2].shape[0] % self.layers[0].self_attention.num_heads:
+            return None
+        return P
 
     def forward(self, x, attn_bias, edge_index, perturb=None, attn_type=None):
-        if self.one_operator and attn_type == "sparse" and edge_index is not None and x.dim() == 2 and x.is_cuda and x.dtype in _DT and \
-                self.MLP_layer.L == 2 and not autocast_to_float32(x):
-            P = model_parameters(self, x.dtype)
-            ve, H = 4 if x.dtype == torch.float32 else 8, self.layers[0].self_attention.num_heads
-            if P is not None and all(p.shape[0] % ve == 0 for p in P[:-2]) and P[2].shape[0] % H == 0:
-                # the whole model as one operator and one autograd node
-                plan = edge_index if isinstance(edge_index, GraphPlan) else get_plan(edge_index, x.shape[0])
-                plan.handle      # raises if the plan was closed
-                eps, classes = [e for layer in self.layers for e in (layer.layer_norm1.eps, layer.layer_norm2.eps)], P[-1].shape[0]
-                x = padded(P, x, 0, -2)
-                return _ext.op("node_gt")(x, P, plan.holder, plan.workspace(H, P[2].shape[0] // H), H, classes, eps)
+        P = self._one_operator(x, edge_index, attn_type)
+        if P is not None:
+            # the whole model as one operator and one autograd node
+            H = self.layers[0].self_attention.num_heads
+            plan = edge_index if isinstance(edge_index, GraphPlan) else get_plan(edge_index, x.shape[0])
+            plan.handle      # raises if the plan was closed
+            eps, classes = [e for layer in self.layers for e in (layer.layer_norm1.eps, layer.layer_norm2.eps)], P[-1].shape[0]
+            x = padded(P, x, 0, -2)
+            return _ext.op("node_gt")(x, P, plan.holder, plan.workspace(H, P[2].shape[0] // H), H, classes, eps)
         x = x.unsqueeze(0)
         (node_feature,) = fused_linear(x, self.node_encoder)
         output = self.input_dropout(node_feature)
