@@ -4,6 +4,7 @@ import torch
 
 from oracle import encoder_layer as oel
 from torchgt_amd import GT, Graphormer, GraphPlan
+from torchgt_amd.encoder import EncoderLayer
 
 pytestmark = pytest.mark.gpu
 
@@ -72,3 +73,41 @@ def test_autocast(cuda, kind, hidden, classes, dtype):
         got.append([out.detach(), torch.cat([p.grad.float().flatten() for p in model.parameters() if p.grad is not None])])
     for a, b in zip(*got):      # two orders of float32 sums; bf16: two orders of roundings
         assert float((a - b).norm()) <= (2e-5 if dtype == torch.float32 else 3e-2) * float(b.norm())
+
+
+class OwnLayer(EncoderLayer):
+    calls = 0
+
+    def forward(self, *args, **kwargs):
+        OwnLayer.calls += 1
+        return super().forward(*args, **kwargs)
+
+
+@pytest.mark.parametrize("path", ["input_dropout", "layers.0", "layers.1.self_attention", "layers.1.self_attention.dist_attn", "layers.0.self_attention.dist_attn.local_attn",
+                                  "layers.0.self_attention_dropout", "layers.1.ffn", "layers.1.ffn_dropout"])
+def test_hooks_fire_and_may_change_what_they_see(cuda, path):
+    """A hook on a module of the model sees one call a pass, and what it returns goes on through the model."""
+    n = 100
+    torch.manual_seed(1)
+    model = scaled(Graphormer(2, 8, 32, 64, 5, 1, 0.0, 0.0, 0.0, 64, 1), 2, torch.float32, cuda)
+    x, plan = torch.randn(n, 32).to(cuda), GraphPlan(edges_of(n, 1, 3).to(cuda), n + 1)
+    before = model(x, None, plan, attn_type="sparse")
+    seen = []
+    handle = model.get_submodule(path).register_forward_hook(lambda m, args, out: seen.append(1) or (tuple(0.5 * t for t in out) if isinstance(out, tuple) else 0.5 * out))
+    changed = model(x, None, plan, attn_type="sparse")
+    assert seen == [1] and float((changed - before).abs().max()) > 1e-3
+    handle.remove()
+    after = model(x, None, plan, attn_type="sparse")
+    assert seen == [1] and torch.equal(after, before)
+
+
+def test_a_subclass_of_the_layer_keeps_its_forward(cuda):
+    n = 100
+    torch.manual_seed(1)
+    model = scaled(Graphormer(2, 8, 32, 64, 5, 1, 0.0, 0.0, 0.0, 64, 1), 2, torch.float32, cuda)
+    x, plan = torch.randn(n, 32).to(cuda), GraphPlan(edges_of(n, 1, 3).to(cuda), n + 1)
+    before = model(x, None, plan, attn_type="sparse")
+    model.layers[1].__class__ = OwnLayer
+    OwnLayer.calls = 0
+    out = model(x, None, plan, attn_type="sparse")
+    assert OwnLayer.calls == 1 and float((out - before).abs().max()) <= 1e-5 * float(before.abs().max())

@@ -5,7 +5,7 @@ import torch
 import torch.nn as nn
 
 from torchgt_amd import GT, GraphLevelGraphormer, Graphormer
-from torchgt_amd.encoder import model_parameters
+from torchgt_amd.module_tree import model_parameters
 
 
 def build(kind, dropout=0.0, input_dropout=0.0, attention_dropout=0.0, layers=2):
@@ -40,3 +40,56 @@ def test_a_module_of_another_kind_in_the_tree(kind, where):
     assert parameters(model) is None and parameters(model) is None
     setattr(owner, name, kept)
     assert parameters(model) is not None
+
+
+def called(model):
+    return [(path, model.get_submodule(path)) for path, _ in model._called_modules()]
+
+
+LISTENERS = {
+    "forward hook": lambda m: m.register_forward_hook(lambda *a: None),
+    "forward pre-hook": lambda m: m.register_forward_pre_hook(lambda *a: None),
+    "backward hook": lambda m: m.register_full_backward_hook(lambda *a: None),
+    "backward pre-hook": lambda m: m.register_full_backward_pre_hook(lambda *a: None),
+}
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_modules_that_somebody_listens_to_are_called(kind):
+    model = build(kind)
+    assert len(called(model)) >= 2 * 5 + 1
+    for path, m in called(model):
+        for name, listen in LISTENERS.items():
+            handle = listen(m)
+            assert parameters(model) is None, (path, name)
+            handle.remove()
+            assert parameters(model) is not None, (path, name)
+        m.forward = lambda *a, **k: None
+        assert parameters(model) is None, path
+        del m.forward
+        cls = type(m)
+        m.__class__ = type("Own", (cls,), {"forward": lambda *a, **k: None})
+        assert parameters(model) is None, path
+        m.__class__ = cls
+        assert parameters(model) is not None, path
+        forward = cls.forward
+        cls.forward = lambda *a, **k: None
+        try:
+            assert parameters(model) is None, path
+        finally:
+            cls.forward = forward
+    for listen in (nn.modules.module.register_module_forward_hook, nn.modules.module.register_module_forward_pre_hook,
+                   nn.modules.module.register_module_full_backward_hook):
+        handle = listen(lambda *a: None)
+        assert parameters(model) is None
+        handle.remove()
+    assert parameters(model) is not None
+
+
+def test_layers_of_unlike_head_counts():
+    """Every layer has its own number of heads: the operators take one for all."""
+    for kind in KINDS:
+        model, other = build(kind), build(kind)
+        other.layers[1].self_attention.num_heads = 4
+        model.layers[1] = other.layers[1]
+        assert parameters(model) is None

@@ -13,14 +13,14 @@ supports); with a positive rate in training mode torch's dropout is applied at
 the reference's places, with torch's random stream.
 """
 import math
-import weakref
 
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _ext, _lib
-from .multi_head_attention import MultiHeadAttention, fused_linear, _DT
+from .module_tree import DROPOUT, all_plain, kind, model_parameters
+from .multi_head_attention import MultiHeadAttention, attention_modules, fused_linear, plain_attention, _DT
 from .plan import GraphPlan, get_plan
 
 
@@ -47,80 +47,6 @@ def init_params(module, n_layers):
 # a layer's parameters in the order of the whole-model operators
 LAYER_PARAMETERS = [f"{m}.{k}" for m in ("self_attention_norm", "self_attention.linear_q", "self_attention.linear_k", "self_attention.linear_v",
                                          "self_attention.output_layer", "ffn_norm", "ffn.layer1", "ffn.layer2") for k in ("weight", "bias")]
-
-
-class ModuleTree:
-    """Where a model's parameters are: for the whole-model operators, whose host time is counted in microseconds, the
-    attribute look-ups of seventy parameters through ``nn.Module`` would be a third of it.  Remembers the dictionaries of the
-    modules, not the parameters, and notices when a module of the tree was exchanged (``current``)."""
-
-    def __init__(self, root, names, dropouts):
-        self.links, self.slots = [], []
-        seen = set()
-
-        def step(module, name):
-            child = module._modules.get(name)
-            if (id(module), name) not in seen:
-                seen.add((id(module), name))
-                self.links.append((module._modules, name, child))
-            return child
-
-        step(root, "layers")
-        self.missing = False      # a module of the names is not there: somebody's own module stands in its place
-        for full in names:
-            *path, leaf = full.split(".")
-            m = root
-            for part in path:
-                m = step(m, part) if m is not None else None
-            if m is None:
-                self.missing = True
-                break
-            self.slots.append((m._parameters, leaf))
-        self.count = len(root.layers)
-        self.layers = root.layers._modules
-        self.dropouts = [m for n, m in root.named_modules() if n.rsplit(".", 1)[-1] in dropouts]
-
-    def current(self):
-        if len(self.layers) != self.count:
-            return False
-        for d, name, child in self.links:
-            if d.get(name) is not child:
-                return False
-        return True
-
-    def parameters(self, dtype, training):
-        """The parameters in order, or None: one is absent or has another dtype, or dropout is at work."""
-        if self.missing or self.count == 0:
-            return None
-        if training:
-            for m in self.dropouts:
-                if m.p > 0:
-                    return None
-        P = [d.get(name) for d, name in self.slots]
-        for p in P:
-            if p is None or p.dtype is not dtype:
-                return None
-        return P
-
-    def by_layer(self):
-        """Whether every layer has the modules of a layer and none was asked to run step by step."""
-        if self.missing:
-            return False
-        for layer in self.layers.values():
-            if "one_operator" in layer.__dict__ or not layer.one_operator or not layer.self_attention.one_operator:
-                return False
-        return True
-
-
-_TREES = weakref.WeakKeyDictionary()      # model -> ModuleTree (which holds the model's modules, not the model)
-
-
-def model_parameters(model, dtype):
-    """Parameters of a model in the order of its whole-model operators, or None where they do not cover its state."""
-    tree = _TREES.get(model)
-    if tree is None or not tree.current():
-        tree = _TREES[model] = ModuleTree(model, model._parameter_names(), model.dropouts)
-    return tree.parameters(dtype, model.training) if tree.by_layer() else None
 
 
 def autocast_to_float32(x):
@@ -158,6 +84,9 @@ class FeedForwardNetwork(nn.Module):
         return y
 
 
+FFN = kind(FeedForwardNetwork)
+
+
 class EncoderLayer(nn.Module):
     def __init__(self, hidden_size, ffn_size, dropout_rate, attention_dropout_rate, num_heads, attn_bias_dim):
         super().__init__()
@@ -178,6 +107,8 @@ class EncoderLayer(nn.Module):
         if self.training and (self.self_attention_dropout.p > 0 or self.ffn_dropout.p > 0):
             return False
         att = self.self_attention
+        if not plain_attention(att) or not all_plain((self.self_attention_dropout, DROPOUT), (self.ffn, FFN), (self.ffn_dropout, DROPOUT)):
+            return False
         if att.output_layer is None or x.dtype not in _DT:
             return False
         ve = 4 if x.dtype == torch.float32 else 8
@@ -213,6 +144,19 @@ class EncoderLayer(nn.Module):
         return _ext.op("add")(x, y)
 
 
+_LAYER = kind(EncoderLayer)
+
+
+def layer_modules(count, layer):
+    """(path, kind) of the modules that the layers of a Graphormer call, themselves among them."""
+    out = []
+    for i in range(count):
+        at = f"layers.{i}."
+        out += [(at[:-1], layer)] + attention_modules(at + "self_attention")
+        out += [(at + "self_attention_dropout", DROPOUT), (at + "ffn", FFN), (at + "ffn_dropout", DROPOUT)]
+    return out
+
+
 class Graphormer(nn.Module):
     """Graphormer for node-level tasks, global token at index 0
     (models/graphormer_dist_node_level.py:316-392)."""
@@ -236,8 +180,6 @@ class Graphormer(nn.Module):
 
     one_operator = True      # False: always run the model layer by layer
 
-    dropouts = ("self_attention_dropout", "ffn_dropout", "input_dropout")
-
     def _one_operator(self, x, attn_bias, edge_index, perturb, attn_type):
         """The model's parameters in the order of the whole-model operators when one of them covers this call - sparse
         attention without a bias, no dropout at work, every linear with its bias, one dtype, one global token (the rows that
@@ -247,7 +189,8 @@ class Graphormer(nn.Module):
             return None
         if x.dim() != 2 or not x.is_cuda or x.dtype not in _DT or autocast_to_float32(x):
             return None
-        return model_parameters(self, x.dtype)
+        P = model_parameters(self, x.dtype)
+        return P if P is not None and self.layers[0].self_attention.num_heads == self.num_heads else None
 
     @staticmethod
     def _fused(P, heads):
@@ -259,6 +202,9 @@ class Graphormer(nn.Module):
         for i in range(len(self.layers)):
             names += [f"layers.{i}.{k}" for k in LAYER_PARAMETERS]
         return names + ["final_ln.weight", "final_ln.bias", "downstream_out_proj.weight", "downstream_out_proj.bias"]
+
+    def _called_modules(self):
+        return [("input_dropout", DROPOUT)] + layer_modules(len(self.layers), _LAYER)
 
     def forward(self, x, attn_bias, edge_index, perturb=None, attn_type=None):
         P = self._one_operator(x, attn_bias, edge_index, perturb, attn_type)

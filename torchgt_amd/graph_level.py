@@ -11,9 +11,10 @@ import torch.nn as nn
 
 from . import _ext, _lib
 from .core_attention import GraphBiasIds
-from .encoder import LAYER_PARAMETERS, _TREES, FeedForwardNetwork, ModuleTree, init_params
+from .encoder import FFN, LAYER_PARAMETERS, FeedForwardNetwork, init_params, layer_modules
 from .graph_bias import GraphAttnBias, same_gpu
-from .multi_head_attention import MultiHeadAttention, fused_linear
+from .module_tree import DROPOUT, all_plain, kind, model_parameters
+from .multi_head_attention import MultiHeadAttention, fused_linear, plain_attention
 
 _DT = {torch.float32: _lib.DTYPE_F32, torch.bfloat16: _lib.DTYPE_BF16}
 
@@ -106,6 +107,8 @@ class EncoderLayer(nn.Module):
         if self.training and (self.self_attention_dropout.p > 0 or self.ffn_dropout.p > 0):
             return None
         att = self.self_attention
+        if not plain_attention(att) or not all_plain((self.self_attention_dropout, DROPOUT), (self.ffn, FFN), (self.ffn_dropout, DROPOUT)):
+            return None
         core = att.dist_attn.local_attn
         ve = 4 if x.dtype == torch.float32 else 8
         if att.output_layer is None or any(w % ve for w in (x.shape[-1], self.ffn.layer1.out_features)) or \
@@ -159,6 +162,9 @@ class EncoderLayer(nn.Module):
         return _ext.op("add")(x, y)
 
 
+_LAYER, _NODE_FEATURE, _ATTN_BIAS = kind(EncoderLayer), kind(GraphNodeFeature), kind(GraphAttnBias)
+
+
 class Graphormer(nn.Module):
     """Graphormer for graph-level tasks: one graph, one sequence (graphormer_graph_level.py:309-389)."""
 
@@ -200,22 +206,26 @@ class Graphormer(nn.Module):
             return None
         return self._operator_parameters()
 
+    def _multi_hop(self):
+        return getattr(self.graph_attn_bias, "edge_type", None) == "multi_hop"
+
+    def _parameter_names(self):
+        head = "out_proj" if hasattr(self, "out_proj") else "downstream_out_proj"
+        names = [f"graph_node_feature.{k}.weight" for k in ("atom_encoder", "in_degree_encoder", "out_degree_encoder", "graph_token")]
+        names += [f"graph_attn_bias.{k}.weight" for k in ("spatial_pos_encoder", "edge_encoder", "graph_token_virtual_distance") +
+                  (("edge_dis_encoder",) if self._multi_hop() else ())]
+        for i in range(len(self.layers)):
+            names += [f"layers.{i}.{k}" for k in LAYER_PARAMETERS]
+        return names + ["final_ln.weight", "final_ln.bias", f"{head}.weight", f"{head}.bias"]
+
+    def _called_modules(self):
+        return [("graph_node_feature", _NODE_FEATURE), ("graph_attn_bias", _ATTN_BIAS), ("input_dropout", DROPOUT)] + layer_modules(len(self.layers), _LAYER)
+
     def _operator_parameters(self):
         """The parameters in the operator's order if the model has hidden and feed-forward width 64, at most 64 outputs, no
         dropout at work but the attention's and one dtype, else None."""
-        multi_hop = getattr(self.graph_attn_bias, "edge_type", None) == "multi_hop"
-        head = "out_proj" if hasattr(self, "out_proj") else "downstream_out_proj"
-        tree = _TREES.get(self)
-        if tree is None or not tree.current():
-            names = [f"graph_node_feature.{k}.weight" for k in ("atom_encoder", "in_degree_encoder", "out_degree_encoder", "graph_token")]
-            names += [f"graph_attn_bias.{k}.weight" for k in ("spatial_pos_encoder", "edge_encoder", "graph_token_virtual_distance") +
-                      (("edge_dis_encoder",) if multi_hop else ())]
-            for i in range(len(self.layers)):
-                names += [f"layers.{i}.{k}" for k in LAYER_PARAMETERS]
-            names += ["final_ln.weight", "final_ln.bias", f"{head}.weight", f"{head}.bias"]
-            tree = _TREES[self] = ModuleTree(self, names, ["self_attention_dropout", "ffn_dropout", "input_dropout"])
-        dtype = getattr(getattr(self.final_ln, "weight", None), "dtype", None)
-        P = tree.parameters(dtype, self.training) if tree.by_layer() else None
+        multi_hop = self._multi_hop()
+        P = model_parameters(self, getattr(getattr(self.final_ln, "weight", None), "dtype", None))
         if P is None:
             return None
         first = self.layers[0].self_attention.dist_attn.local_attn

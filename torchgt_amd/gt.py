@@ -10,9 +10,10 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _ext, _lib
-from .encoder import autocast_to_float32, init_params, model_parameters, padded
+from .encoder import autocast_to_float32, init_params, padded
 from .graph_bias import same_gpu
-from .multi_head_attention import MultiHeadAttention, fused_linear
+from .module_tree import DROPOUT, kind, model_parameters
+from .multi_head_attention import MultiHeadAttention, attention_modules, fused_linear
 from .plan import GraphPlan, get_plan
 
 _DT = {torch.float32: _lib.DTYPE_F32, torch.bfloat16: _lib.DTYPE_BF16}
@@ -81,6 +82,9 @@ class MLPReadout(nn.Module):
         return y
 
 
+_LAYER, _READOUT = kind(EncoderLayer), kind(MLPReadout)
+
+
 class GT(nn.Module):
     """GT for node-level tasks, no global token (gt_dist_node_level.py:290-341)."""
 
@@ -96,7 +100,6 @@ class GT(nn.Module):
         self.apply(lambda module: init_params(module, n_layers=n_layers))
 
     one_operator = True      # False: always run the model layer by layer
-    dropouts = ("self_attention_dropout", "input_dropout")
 
     def _parameter_names(self):
         both = lambda name: [f"{name}.weight", f"{name}.bias"]
@@ -106,6 +109,12 @@ class GT(nn.Module):
                          "layer_norm2"):
                 names += both(f"layers.{i}.{part}")
         return names + [n for j in range(3) for n in both(f"MLP_layer.FC_layers.{j}")]
+
+    def _called_modules(self):
+        out = [("input_dropout", DROPOUT), ("MLP_layer", _READOUT)]
+        for i in range(len(self.layers)):
+            out += [(f"layers.{i}", _LAYER), (f"layers.{i}.self_attention_dropout", DROPOUT)] + attention_modules(f"layers.{i}.self_attention")
+        return out
 
     def _one_operator(self, x, edge_index, attn_type):
         """The model's parameters in the operator's order when ``torch.ops.torchgt.node_gt`` covers this call, else None."""

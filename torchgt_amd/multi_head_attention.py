@@ -19,6 +19,7 @@ import torch.nn as nn
 
 from . import _ext, _lib
 from .core_attention import CoreAttention
+from .module_tree import all_plain, kind
 from .plan import GraphPlan, get_plan
 
 _DT = {torch.float32: _lib.DTYPE_F32, torch.bfloat16: _lib.DTYPE_BF16}
@@ -75,6 +76,9 @@ class _LocalAttention(nn.Module):
         return self.local_attn(query, key, value, attn_bias, edge_index, attn_type, *args)
 
 
+_LOCAL, _CORE = kind(_LocalAttention), kind(CoreAttention)
+
+
 class MultiHeadAttention(nn.Module):
     """``MultiHeadAttention(hidden_size, attention_dropout_rate, num_heads, attn_bias_dim)``:
     the Graphormer flavour with an output layer (graphormer_dist_node_level.py:228-241).
@@ -103,9 +107,16 @@ class MultiHeadAttention(nn.Module):
         widths the kernels read without padding, every layer with its bias."""
         if not self.one_operator or attn_type != "sparse" or attn_bias is not None or edge_index is None or not x.is_cuda:
             return False
+        if not self.plain_core():
+            return False
         ve = 4 if x.dtype == torch.float32 else 8
         layers = [self.linear_q, self.linear_k, self.linear_v] + ([] if self.output_layer is None else [self.output_layer])
         return all(l.bias is not None and l.in_features % ve == 0 and l.out_features % ve == 0 for l in layers)
+
+    def plain_core(self):
+        """Whether the modules behind the projections are the library's and nobody listens to them."""
+        d = self.dist_attn
+        return all_plain((d, _LOCAL)) and all_plain((d.local_attn, _CORE))
 
     def forward(self, x, attn_bias=None, edge_index=None, attn_type=None):
         if self._one_operator(x, attn_bias, edge_index, attn_type):
@@ -127,3 +138,16 @@ class MultiHeadAttention(nn.Module):
         if self.output_layer is not None:
             (x,) = fused_linear(x, self.output_layer)
         return x
+
+
+_MHA = kind(MultiHeadAttention)
+
+
+def plain_attention(att):
+    """Whether an operator may do the work of this attention module."""
+    return all_plain((att, _MHA)) and att.plain_core()
+
+
+def attention_modules(path):
+    """(path, kind) of the modules that calling an attention module of the library calls."""
+    return [(path, _MHA), (path + ".dist_attn", _LOCAL), (path + ".dist_attn.local_attn", _CORE)]
