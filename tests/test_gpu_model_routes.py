@@ -111,3 +111,31 @@ def test_a_subclass_of_the_layer_keeps_its_forward(cuda):
     OwnLayer.calls = 0
     out = model(x, None, plan, attn_type="sparse")
     assert OwnLayer.calls == 1 and float((out - before).abs().max()) <= 1e-5 * float(before.abs().max())
+
+
+@pytest.mark.parametrize("where", ["input_dropout", "layers.1.ffn_dropout", "layers.0.self_attention_dropout"])
+def test_one_dropout_in_training_mode(cuda, where):
+    """A dropout module set to training in a model in eval mode drops (and the others don't), as does none in a model in training mode
+    whose dropouts are in eval mode."""
+    n = 100
+    torch.manual_seed(1)
+    model = scaled(Graphormer(2, 8, 32, 64, 5, 1, 0.2, 0.2, 0.0, 64, 1), 2, torch.float32, cuda).eval()
+    x, plan = torch.randn(n, 32).to(cuda), GraphPlan(edges_of(n, 1, 3).to(cuda), n + 1)
+    run = lambda: model(x, None, plan, attn_type="sparse").detach()
+    still = run()
+    dropout = model.get_submodule(where)
+    dropout.train()
+    with torch.random.fork_rng(devices=[cuda]):
+        torch.manual_seed(5)
+        dropped = run()
+        seen = []
+        handle = dropout.register_forward_hook(lambda m, args, out: seen.append(int((out == 0).sum()) > args[0].numel() // 10))
+        torch.manual_seed(5)
+        assert torch.equal(run(), dropped) and seen == [True]
+        handle.remove()
+    assert float((dropped - still).abs().max()) > 1e-3
+    model.train()
+    for m in model.modules():
+        if isinstance(m, torch.nn.Dropout):
+            m.eval()
+    assert torch.equal(run(), still)

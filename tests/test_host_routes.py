@@ -93,3 +93,31 @@ def test_layers_of_unlike_head_counts():
         other.layers[1].self_attention.num_heads = 4
         model.layers[1] = other.layers[1]
         assert parameters(model) is None
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_every_dropout_has_its_own_mode(kind):
+    model = build(kind, dropout=0.1, input_dropout=0.3)
+    assert parameters(model) is None
+    model.eval()
+    assert parameters(model) is not None
+    dropouts = [m for _, m in called(model) if isinstance(m, nn.Dropout)]
+    assert len(dropouts) == (3 if kind == "gt" else 5)
+    for m in dropouts:
+        m.train()      # drops in a model in eval mode
+        assert parameters(model) is None
+        m.eval()
+    model.train()
+    for m in dropouts:
+        m.eval()       # (the model's own flag says nothing)
+    assert model.training and parameters(model) is not None
+
+
+def test_attention_dropout_has_each_modules_mode():
+    model = build("graph", attention_dropout=0.5)
+    cores = [layer.self_attention.dist_attn.local_attn for layer in model.layers]
+    assert parameters(model) is not None and cores[0].dropout_at_work() == 0.5
+    cores[1].eval()      # the operator has one rate for all layers
+    assert parameters(model) is None
+    cores[0].eval()
+    assert parameters(model) is not None and cores[0].dropout_at_work() == 0.0

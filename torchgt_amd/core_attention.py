@@ -231,6 +231,10 @@ class CoreAttention(nn.Module):
         # bf16 matrix cores (faster, about 2e-2 instead of 1e-5)
         self.dense_bf16_products = False
 
+    def dropout_at_work(self):
+        """The rate at which the dense attention drops probabilities in this module's mode."""
+        return float(self.attention_dropout_rate) if self.training else 0.0
+
     # -- helpers ---------------------------------------------------------
     def _edge_bias(self, attn_bias, edge_index):
         if attn_bias is None:
@@ -278,7 +282,7 @@ class CoreAttention(nn.Module):
                                       "it is not supported")
         # the reference applies att_dropout to the softmax output (graphormer_graph_level.py:207-209); here the
         # kernels do, in training mode
-        p = float(self.attention_dropout_rate) if self.training else 0.0
+        p = self.dropout_at_work()
         return dense_attention(q, k, v, attn_bias, p_drop=p, bf16_products=self.dense_bf16_products)
 
     def forward(self, q, k, v, attn_bias=None, edge_index=None, attn_type=None, mask=None,

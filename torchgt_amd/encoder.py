@@ -19,7 +19,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _ext, _lib
-from .module_tree import DROPOUT, all_plain, kind, model_parameters
+from .module_tree import DROPOUT, all_plain, at_work, kind, model_parameters
 from .multi_head_attention import MultiHeadAttention, attention_modules, fused_linear, plain_attention, _DT
 from .plan import GraphPlan, get_plan
 
@@ -104,10 +104,10 @@ class EncoderLayer(nn.Module):
         work, feature widths the kernels read without padding."""
         if not self.one_operator or attn_type != "sparse" or attn_bias is not None or edge_index is None or not x.is_cuda:
             return False
-        if self.training and (self.self_attention_dropout.p > 0 or self.ffn_dropout.p > 0):
-            return False
         att = self.self_attention
         if not plain_attention(att) or not all_plain((self.self_attention_dropout, DROPOUT), (self.ffn, FFN), (self.ffn_dropout, DROPOUT)):
+            return False
+        if at_work(self.self_attention_dropout) or at_work(self.ffn_dropout):
             return False
         if att.output_layer is None or x.dtype not in _DT:
             return False

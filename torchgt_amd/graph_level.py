@@ -13,7 +13,7 @@ from . import _ext, _lib
 from .core_attention import GraphBiasIds
 from .encoder import FFN, LAYER_PARAMETERS, FeedForwardNetwork, init_params, layer_modules
 from .graph_bias import GraphAttnBias, same_gpu
-from .module_tree import DROPOUT, all_plain, kind, model_parameters
+from .module_tree import DROPOUT, all_plain, at_work, kind, model_parameters
 from .multi_head_attention import MultiHeadAttention, fused_linear, plain_attention
 
 _DT = {torch.float32: _lib.DTYPE_F32, torch.bfloat16: _lib.DTYPE_BF16}
@@ -104,10 +104,10 @@ class EncoderLayer(nn.Module):
         (no torch dropout at work, widths the kernels read without padding, a bias it can take as it is), else None."""
         if not self.one_operator or not x.is_cuda or x.dim() != 3 or x.dtype not in (torch.float32, torch.bfloat16):
             return None
-        if self.training and (self.self_attention_dropout.p > 0 or self.ffn_dropout.p > 0):
-            return None
         att = self.self_attention
         if not plain_attention(att) or not all_plain((self.self_attention_dropout, DROPOUT), (self.ffn, FFN), (self.ffn_dropout, DROPOUT)):
+            return None
+        if at_work(self.self_attention_dropout) or at_work(self.ffn_dropout):
             return None
         core = att.dist_attn.local_attn
         ve = 4 if x.dtype == torch.float32 else 8
@@ -138,7 +138,7 @@ class EncoderLayer(nn.Module):
             extra, ab, sp16, et16 = fused
             att = self.self_attention
             core = att.dist_attn.local_attn
-            p = float(core.attention_dropout_rate) if self.training else 0.0
+            p = core.dropout_at_work()
             seed = int(torch.randint(0, 2 ** 62, (1,)).item()) if p > 0 else 0
             params = [n1.weight, n1.bias, att.linear_q.weight, att.linear_q.bias, att.linear_k.weight, att.linear_k.bias,
                       att.linear_v.weight, att.linear_v.bias, att.output_layer.weight, att.output_layer.bias, n2.weight, n2.bias,
@@ -228,10 +228,10 @@ class Graphormer(nn.Module):
         P = model_parameters(self, getattr(getattr(self.final_ln, "weight", None), "dtype", None))
         if P is None:
             return None
-        first = self.layers[0].self_attention.dist_attn.local_attn
+        p = self.layers[0].self_attention.dist_attn.local_attn.dropout_at_work()
         for layer in self.layers:
             core = layer.self_attention.dist_attn.local_attn
-            if layer.self_attention.num_heads not in (2, 4, 8) or core.attention_dropout_rate != first.attention_dropout_rate or core.dense_bf16_products:
+            if layer.self_attention.num_heads not in (2, 4, 8) or core.dropout_at_work() != p or core.dense_bf16_products:
                 return None
         if P[0].dtype not in _DT or P[0].shape[1] != 64 or P[-1].shape[0] > 64 or P[4].shape[1] != self.layers[0].self_attention.num_heads or \
                 any(p.shape[0] != 64 or p.shape[-1] != 64 for p in P[8 if multi_hop else 7:-4]):
@@ -245,8 +245,7 @@ class Graphormer(nn.Module):
             # attention and what follows it at the virtual nodes only: no other row of it is read)
             multi_hop = self.graph_attn_bias.edge_type == "multi_hop"
             att = self.layers[0].self_attention
-            core = att.dist_attn.local_attn
-            p = float(core.attention_dropout_rate) if self.training else 0.0
+            p = att.dist_attn.local_attn.dropout_at_work()
             seeds = [int(torch.randint(0, 2 ** 62, (1,)).item()) if p > 0 else 0 for _ in self.layers]
             eps = [e for layer in self.layers for e in (layer.self_attention_norm.eps, layer.ffn_norm.eps)] + [self.final_ln.eps]
             d = batched_data

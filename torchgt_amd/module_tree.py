@@ -30,6 +30,10 @@ def all_plain(*pairs):
     return not watched_everywhere() and all(plain(m, *k) for m, k in pairs)
 
 
+def at_work(dropout):
+    return dropout.training and dropout.p > 0
+
+
 def watched_everywhere():
     m = _torch_module
     return bool(m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks or m._global_backward_pre_hooks)
@@ -88,18 +92,17 @@ class ModuleTree:
                 return False
         return True
 
-    def parameters(self, dtype, training):
+    def parameters(self, dtype):
         """The parameters in order, or None: one is absent or has another dtype, a module is not plain or was asked to run step by
-        step, or dropout is at work."""
+        step, or dropout is at work (each dropout module has its own mode, whatever the model's)."""
         if self.missing or self.count == 0 or watched_everywhere():
             return None
         for m, cls, forward in self.called:
             if not plain(m, cls, forward):
                 return None
-        if training:
-            for d in self.dropouts:
-                if d["p"] > 0:
-                    return None
+        for d in self.dropouts:
+            if d["training"] and d["p"] > 0:
+                return None
         heads = None
         for layer in self.layers.values():
             att = layer._modules["self_attention"]
@@ -121,4 +124,4 @@ def model_parameters(model, dtype):
     tree = _TREES.get(model)
     if tree is None or not tree.current():
         tree = _TREES[model] = ModuleTree(model, model._parameter_names(), model._called_modules())
-    return tree.parameters(dtype, model.training)
+    return tree.parameters(dtype)
