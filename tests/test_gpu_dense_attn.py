@@ -270,3 +270,22 @@ def test_node_level_bias_layout_is_reinterpreted_like_the_reference(cuda):
     assert torch.equal(got, want)
     o_ref = oda.dense_attention(q.double().cpu(), k.double().cpu(), v.double().cpu(), bias.double().cpu().contiguous().view(b, H, S, S))
     assert err(got, o_ref) <= TOL
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("d", [8, 16, 32])
+def test_query_0_backward_forms_the_forwards_score(cuda, dtype, d):
+    """One key: its probability is exactly 1 whatever the score, if the backward's score has the bits of the one in the log-sum-exp."""
+    b, H = 256, 8
+    code = _lib.DTYPE_F32 if dtype == torch.float32 else _lib.DTYPE_BF16
+    g = torch.Generator().manual_seed(d)
+    q, k, v, s, da0 = (torch.randn(b, 1, H * d, generator=g).mul(8).to(cuda, dtype) for _ in range(5))
+    bias = torch.randn(b, H, 1, 1, generator=g).to(cuda, dtype)
+    a0, s0, dq, dk, dv, ds, g0 = (torch.empty_like(q) for _ in range(7))
+    g0.zero_()
+    lse, dvirt = (torch.empty(b, H, device=cuda) for _ in range(2))
+    at, stream, L = (lambda t: t.data_ptr()), torch.cuda.current_stream(cuda).cuda_stream, _lib.lib()
+    _lib.check(L.tgt_dense_row0_fwd(at(q), at(k), at(v), at(bias), at(s), b, 1, H, d, code, 0.0, 0, at(a0), at(s0), at(lse), stream))
+    _lib.check(L.tgt_dense_row0_bwd(at(q), at(k), at(v), at(bias), b, 1, H, d, code, 0.0, 0, at(a0), at(lse), at(da0), at(g0), at(dq), at(dk), at(dv), at(ds), at(dvirt), stream))
+    assert float(lse.abs().max()) > 100 and torch.equal(a0, v) and torch.equal(s0, s)
+    assert torch.equal(dv, da0)

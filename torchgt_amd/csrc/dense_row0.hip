@@ -84,6 +84,18 @@ template <typename T> struct Row0Args {
     float* dvirt;
 };
 
+// The score of a key in one expression for forward and backward: the backward's exp(score - lse) is only as good as their last bits
+// agree (scores reach the hundreds).  float32: the reference scales the query; bf16: the matrix-core kernels scale the product.
+template <typename T, int D> __device__ __forceinline__ void scaled_query(const Row0Args<T>& a, int64_t row, float (&q)[D]) {
+    load_vec<D>(a.q + row, q);
+    if (sizeof(T) == 4)
+#pragma unroll
+        for (int c = 0; c < D; ++c) q[c] *= a.scale;
+}
+template <typename T, int D> __device__ __forceinline__ float score_of(const Row0Args<T>& a, const float (&q)[D], const float (&k)[D], float bias) {
+    return sizeof(T) == 2 ? fmaf(dot<D>(q, k), a.scale, bias) : dot<D>(q, k) + bias;
+}
+
 template <typename T, int D, bool DROP> __global__ __launch_bounds__(512) void k_row0_fwd(const Row0Args<T> a, const DropArgs da) {
     extern __shared__ float lds[];
     constexpr bool MATRIX = sizeof(T) == 2;      // rounds like the matrix-core kernels
@@ -92,10 +104,7 @@ template <typename T, int D, bool DROP> __global__ __launch_bounds__(512) void k
     float *score = lds + h * (kRow0Max + 2 * (kRow0Max / 32)), *tile_max = score + kRow0Max, *factor = tile_max + kRow0Max / 32;
     const int64_t row = ((int64_t)g * S * H + h) * D, pitch = (int64_t)H * D;
     float q[D];
-    load_vec<D>(a.q + row, q);
-    if (!MATRIX)
-#pragma unroll
-        for (int c = 0; c < D; ++c) q[c] *= a.scale;      // the reference scales the query
+    scaled_query(a, row, q);
     const T* bias = a.bias ? a.bias + ((int64_t)g * H + h) * S * S : nullptr;
     for (int k0 = 0; k0 < S; k0 += 64) {
         const int key = k0 + lane;
@@ -104,7 +113,7 @@ template <typename T, int D, bool DROP> __global__ __launch_bounds__(512) void k
             float kv[D];
             load_vec<D>(a.k + row + key * pitch, kv);
             const float bv = bias ? ld(bias + key) : 0.f;
-            sc = MATRIX ? fmaf(dot<D>(q, kv), a.scale, bv) : dot<D>(q, kv) + bv;
+            sc = score_of(a, q, kv, bv);
             score[key] = sc;
         }
         float m = sc;
@@ -165,7 +174,7 @@ template <typename T, int D, bool DROP> __global__ __launch_bounds__(512) void k
     const int g = blockIdx.x, h = threadIdx.x >> 6, lane = threadIdx.x & 63, S = a.S, H = a.H;
     const int64_t row = ((int64_t)g * S * H + h) * D, pitch = (int64_t)H * D, at = ((int64_t)g * H + h) * D;
     float q[D], o[D], gv[D], g0[D], dq[D], none[D];
-    load_vec<D>(a.q + row, q);
+    scaled_query(a, row, q);
     load_vec<D>(a.a0 + at, o);
     load_vec<D>(a.da0 + at, gv);
     load_vec<D>(a.g0 + at, g0);
@@ -179,14 +188,14 @@ template <typename T, int D, bool DROP> __global__ __launch_bounds__(512) void k
         float kv[D], vv[D];
         load_vec<D>(a.k + row + key * pitch, kv);
         load_vec<D>(a.v + row + key * pitch, vv);
-        const float sc = fmaf(dot<D>(q, kv), a.scale, bias ? ld(bias + key) : 0.f);
+        const float sc = score_of(a, q, kv, bias ? ld(bias + key) : 0.f);
         const float p = exp_of(sc - lse, tag), ks = !DROP ? 1.f : (drop_keep(da, rh, key) ? da.inv_keep : 0.f);
         const float ds = rounded(p * (dot<D>(gv, vv) * ks - delta), tag), pb = rounded(p * ks, tag);
         dv_sum += ds;
 #pragma unroll
         for (int c = 0; c < D; ++c) {
             dq[c] = fmaf(ds, kv[c], dq[c]);
-            kv[c] = ds * q[c] * a.scale;
+            kv[c] = sizeof(T) == 2 ? ds * q[c] * a.scale : ds * q[c];
             vv[c] = pb * gv[c];
         }
         store_vec<D>(a.dk + row + key * pitch, kv);
