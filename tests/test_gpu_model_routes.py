@@ -1,9 +1,11 @@
 """Which calls the whole-model operators take: a call that they do not cover gives what the layers one by one give."""
+import types
+
 import pytest
 import torch
 
 from oracle import encoder_layer as oel
-from torchgt_amd import GT, Graphormer, GraphPlan
+from torchgt_amd import GT, GraphLevelGraphormer, Graphormer, GraphPlan
 from torchgt_amd.encoder import EncoderLayer
 
 pytestmark = pytest.mark.gpu
@@ -139,3 +141,28 @@ def test_one_dropout_in_training_mode(cuda, where):
         if isinstance(m, torch.nn.Dropout):
             m.eval()
     assert torch.equal(run(), still)
+
+
+def test_bias_gradients_of_a_large_batch_go_into_a_running_sum(cuda):
+    """The layers share one bias; where its gradient is large only a running sum and the next layer's are held."""
+    b, s, layers = 64, 384, 5
+    torch.manual_seed(1)
+    model = scaled(GraphLevelGraphormer(layers, 8, 64, 0.0, 0.0, 64, "ZINC", "single_hop", 5, 0.0, 1), 2, torch.float32, cuda)
+    g = torch.Generator().manual_seed(3)
+    ids = lambda hi, *shape: torch.randint(0, hi, shape, generator=g).to(cuda)
+    batch = types.SimpleNamespace(x=ids(64, b, s, 1), in_degree=ids(64, b, s), out_degree=ids(64, b, s), attn_bias=torch.zeros(b, s + 1, s + 1, device=cuda),
+                                  spatial_pos=ids(40, b, s, s), attn_edge_type=ids(64, b, s, s, 1))
+    one_bias = b * 8 * (s + 1) ** 2 * 4
+    assert one_bias > 256 << 20
+    got = []
+    for one in (True, False):
+        model.one_operator = one
+        model.zero_grad(set_to_none=True)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        model(batch).sum().backward()
+        torch.cuda.synchronize()
+        got.append((torch.cuda.max_memory_allocated() - before, torch.cat([p.grad.flatten() for p in model.parameters() if p.grad is not None])))
+    assert got[0][0] <= 4.5 * one_bias      # the bias, the sum, one layer's gradient, all rows of the step (1 to 1.5 of a bias)
+    assert float((got[0][1] - got[1][1]).norm()) <= 3e-5 * float(got[1][1].norm())
