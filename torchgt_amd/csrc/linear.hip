@@ -914,6 +914,22 @@ int grad_workers(int in_features, int out_features) {
     return std::max(1, kGradWorkers / tiles);
 }
 
+// Workgroups per output tile for k_gradw_tiles.  Half of grad_workers where that many would be more than two workgroups per CU over all
+// tiles, or would have less than eight panels each: the partials, written and read again, then weigh more than the emptier chip.
+// From 256 K rows on always all of them: narrow shapes would gain up to 14 % from half, but a worker's chain of float32 adds would
+// pass 512 rows, and the sums be less accurate.
+// Kernel and sum of the partials, us, all / half of them, at 32 K, 64 K, 256 K, 512 K, 870 K rows:
+//   128 -> 64 float32 (512 of them, one tile)       16.2/13.7  19.4/16.7  40.6/40.2  78.2/84.5   131.6/133.8
+//   128 -> 64 bf16                                  16.2/12.1  15.5/13.6  24.2/22.6  37.5/36.1   62.7/69.2
+//   496 -> 64 bf16 (128, four tiles)                15.4/16.1  20.1/23.1  55.7/81.0  108.6/155   173/252
+//   128 -> 256 float32 (128, four tiles)            24.7/24.8  38.9/39.9  132/146    272/282     453/469
+//   64 -> 40 float32 (1024, one tile)               11.8/11.8  17.8/13.0  29.8/24.7  46.2/40.1   81.8/70.6
+//   128 -> 128 float32, three weights (256, six)    41.3/33.8  63.9/55.3  209/203    451/412     752/685
+int gradw_workers(int64_t n_panels, int nw, int K, int M) {
+    const int all = grad_workers(K, M), tiles = nw * ((M + kCols - 1) / kCols) * ((K + 2 * kCols - 1) / (2 * kCols));
+    return (int)std::max<int64_t>(1, std::min<int64_t>(n_panels, n_panels < 4096 && (all * tiles > 512 || n_panels < 8 * all) ? all / 2 : all));
+}
+
 template <typename T>
 int linear_bwd_t(const void* d_x, const void* const* d_W, const void* const* d_dy, int n_out, int64_t N, int K, int M,
                  void* d_dx, void* const* d_dW, void* const* d_db, float* partial, hipStream_t st, tgt_reduce_desc* defer,
@@ -972,9 +988,7 @@ int linear_bwd_t(const void* d_x, const void* const* d_W, const void* const* d_d
     }
     if (d_dW) {
         const int64_t n_panels = (N + kGradRows - 1) / kGradRows;
-        // half of them below 256 K rows: there the partials, written and read again, weigh more than the emptier chip (64 K rows,
-        // 128 x 128 float32, three weights: 66 us with 512, 75 us with 1024; 870 K rows, 104 x 64 bf16: 73 and 53 us)
-        const int workers = (int)std::max<int64_t>(1, std::min<int64_t>(n_panels, grad_workers(K, M) / (N < (256 << 10) ? 2 : 1)));
+        const int workers = gradw_workers(n_panels, n_out, K, M);
         GradWArgs g{};
         g.x = d_x;
         for (int j = 0; j < n_out; ++j) g.dy[j] = d_dy[j];
