@@ -4,12 +4,13 @@ a wave's 32 rows and a workgroup's 128 and 256, class counts around the halves o
 
 Bars: float32 1e-5 of the largest value of the tensor, bf16 6e-2 (the layer-by-layer path rounds every intermediate tensor)."""
 import copy
+import ctypes
 import types
 
 import pytest
 import torch
 
-from torchgt_amd import GT, GraphLevelGraphormer, Graphormer, GraphPlan
+from torchgt_amd import GT, GraphLevelGraphormer, Graphormer, GraphPlan, _ext, _lib
 from torchgt_amd.graph_prep import fix_edge_index
 
 pytestmark = pytest.mark.gpu
@@ -174,3 +175,36 @@ def test_gt_on_fused_layers(cuda, n, features, classes, heads, layers):
     for name, f32, one, steps in zip(("output", "input gradient", "parameter gradients"), *got):
         off, most = float((one - f32).norm() / f32.norm()), float((steps - f32).norm() / f32.norm())
         assert off <= 1.1 * most + 2e-3, f"{name}: {off}, step by step {most}"
+
+
+class NodeFwdArgs(ctypes.Structure):      # tgt_node_fwd_args
+    _fields_ = [("rows", ctypes.c_int64)] + [(k, ctypes.c_int32) for k in ("dtype", "tokens", "classes", "linear", "same_bits")] + \
+        [(k, ctypes.c_float) for k in ("eps_post", "eps_next")] + \
+        [(k, ctypes.c_void_p) for k in ("attn", "s_in", "token", "s_out", "w_post", "w_next", "v_post", "v_next", "q", "k", "v", "logp")]
+
+
+@pytest.mark.parametrize("scale", [0.3, 1.0, 2.0])
+def test_gelu_of_the_fused_layers_is_as_exact_as_the_error_function(cuda, scale):
+    """The activation of the fused kernels against 64 bits, next to 0.5 u (1 + erff(u / sqrt 2)) of the separate kernel.  With zero rows,
+    W1 = 0 and W2 = 1 the layer's output is the activation of its bias b1, 64 values a launch, behind a product with W2 that rounds a
+    little of its own: the separate kernel's values go through the same product."""
+    launches, L = 1024, _lib.lib()
+    u = (torch.randn(launches, 64, generator=torch.Generator().manual_seed(3)) * scale).to(cuda)
+    zero, one = torch.zeros(64, 64, device=cuda), torch.eye(64, device=cuda)
+    frags = torch.empty(L.tgt_node_frag_bytes(3, _lib.DTYPE_F32), dtype=torch.uint8, device=cuda)
+    vecs, stream = torch.zeros(5, 64, device=cuda), torch.cuda.current_stream(cuda).cuda_stream      # bo, gamma, beta, b1, b2
+    mats, ld = (ctypes.c_void_p * 3)(zero.data_ptr(), zero.data_ptr(), one.data_ptr()), (ctypes.c_int * 3)(64, 64, 64)
+    rows, lens, packed = (ctypes.c_void_p * 5)(*[vecs[i].data_ptr() for i in range(5)]), (ctypes.c_int * 5)(*[64] * 5), torch.empty_like(vecs)
+    _lib.check(L.tgt_node_pack(ctypes.addressof(mats), ctypes.addressof(ld), ctypes.addressof(ld), 3, ctypes.addressof(rows), ctypes.addressof(lens), 5,
+                               _lib.DTYPE_F32, frags.data_ptr(), packed.data_ptr(), stream))
+    fused = torch.empty_like(u)
+    for i in range(launches):
+        vecs[3] = u[i]
+        args = NodeFwdArgs(rows=1, dtype=_lib.DTYPE_F32, eps_post=1e-5, attn=zero.data_ptr(), s_in=zero.data_ptr(), s_out=fused[i].data_ptr(), w_post=frags.data_ptr(),
+                           v_post=vecs.data_ptr())
+        _lib.check(L.tgt_node_fwd(ctypes.addressof(args), stream))
+    exact = 0.5 * u.double() * torch.special.erfc(-u.double() * 2 ** -0.5)
+    rms = lambda t: float((t.double() - exact).pow(2).mean().sqrt())
+    (separate,) = _ext.op("linear")(_ext.op("gelu")(u), [one], [zero[0]])
+    print(f"gelu, u ~ N(0, {scale}): rms error {rms(fused):.3e}, of the separate kernel {rms(separate):.3e}", flush=True)
+    assert rms(fused) <= rms(separate) and float((fused - exact).abs().max()) <= 5e-7
