@@ -80,6 +80,40 @@ def test_linears_of_any_width(cuda, dtype, N, in_f, out_f, n):
     run_linear("any-width", N, in_f, out_f, n, dtype, cuda, N + in_f)
 
 
+@pytest.mark.parametrize("N,in_f,out_f,n", [(70, 128, 64, 1), (33, 56, 72, 3), (257, 200, 40, 2), (64, 8, 128, 1)])
+@pytest.mark.parametrize("what", ["x", "W", "dy", "both signs"])
+def test_infinities_and_nan_stay_where_they_belong(cuda, N, in_f, out_f, n, what):
+    """float32 operands go through the matrix unit in three parts, and an infinity has none: every output is +-inf, NaN or finite as the
+    float32 products and sums have it, and the finite ones have their accuracy."""
+    print(f"infinities case: N={N} in={in_f} out={out_f} n={n} {what}", flush=True)
+    g = torch.Generator().manual_seed(N)
+    x = torch.randn(N, in_f, generator=g)
+    Ws = [torch.randn(out_f, in_f, generator=g) for _ in range(n)]
+    dys = [torch.randn(N, out_f, generator=g) for _ in range(n)]
+    Ws[0][3, 1] = 0.5      # (representable in one part: the other two are zeros)
+    inf = float("inf")
+    if what == "x":
+        x[N // 2, 1], x[N - 1, in_f - 1], x[0, 0] = inf, -inf, float("nan")
+    elif what == "W":
+        Ws[n - 1][out_f // 2, in_f - 1], Ws[0][0, 0] = inf, -inf
+    elif what == "dy":
+        dys[n - 1][N - 1, 0], dys[0][N // 3, out_f - 1] = -inf, inf
+    else:
+        x[N // 2, 1], x[N // 2, 2], dys[0][0, 0], dys[0][0, 1] = inf, -inf, inf, -inf
+    xc = x.to(cuda).requires_grad_(True)
+    Wc = [W.to(cuda).requires_grad_(True) for W in Ws]
+    bc = [torch.zeros(out_f, device=cuda, requires_grad=True) for _ in range(n)]
+    ys = LinearFunction.apply(xc, *[t for pair in zip(Wc, bc) for t in pair])
+    grads = torch.autograd.grad(ys, [xc] + Wc + bc, [dy.to(cuda) for dy in dys])
+    product = lambda a, b: (a.double().unsqueeze(2) * b.double().unsqueeze(0)).sum(1)      # (every product formed and added)
+    want = [product(x, W.t()) for W in Ws] + [sum(product(dy, W) for dy, W in zip(dys, Ws))] + [product(dy.t(), x) for dy in dys] + [dy.double().sum(0) for dy in dys]
+    for i, (a, b) in enumerate(zip(list(ys) + list(grads), want)):
+        a = a.detach().double().cpu()
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isposinf(), b.isposinf()) and torch.equal(a.isneginf(), b.isneginf()), i
+        fin = b.isfinite()
+        assert not fin.any() or float((a - b)[fin].abs().max()) <= 1e-5 * float(b[fin].abs().max()), i
+
+
 def test_linear_weight_gradient_is_reproducible(cuda):
     """The weight gradients are summed in a fixed order: two runs give the same bits."""
     a = run_linear("repro-a", 20000, 64, 64, 3, torch.float32, cuda, 9)[1]

@@ -102,6 +102,34 @@ template <typename T, int P> __device__ __forceinline__ void put_piece(vec16* ds
     }
 }
 
+// Whether a lane of the wave holds a NaN.  An infinity has no planes (what is left of it behind hi is NaN, and an infinite hi times the
+// mid plane of the other operand has any sign): every output that it touches comes out as NaN and is formed again by plain float32
+// multiply-adds, which give the +-inf or NaN that it has.  The look costs one multiply-add per output (128 -> 64 of 64 K rows: below
+// the runs' difference); the second computation runs for waves with a NaN only.
+template <typename V> __device__ __forceinline__ bool holds_nan(const V& value, int n) {
+    float t = 0.f;
+#pragma unroll
+    for (int i = 0; i < n; ++i) t = fmaf(value(i), 0.f, t);      // (infinities too: they may have become what they are on the way)
+    return __ballot(t != 0.f) != 0;
+}
+
+// the wave's 32 rows of 64 output columns from c0 on, lane = its node's half as in Tile
+template <bool DX> __device__ __forceinline__ void rows_again(const LinArgs& a, int o, int c0, const Rows& rows, int lane) {
+    const int L = DX ? a.M : a.K, C = DX ? a.K : a.M, n = lane & 31;
+    if (n >= rows.left) return;
+    const int64_t row = rows.first + n;
+    for (int i = 0; i < 32; ++i) {
+        const int c = c0 + 32 * (lane >> 5) + i;
+        if (c >= C) return;
+        float t = !DX && a.bias[o] ? reinterpret_cast<const float*>(a.bias[o])[c] : 0.f;
+        for (int j = DX ? 0 : o; j < (DX ? a.nw : o + 1); ++j) {
+            const float *x = reinterpret_cast<const float*>(a.A[DX ? j : 0]) + row * L, *W = reinterpret_cast<const float*>(a.W[j]);
+            for (int k = 0; k < L; ++k) t = fmaf(x[k], DX ? W[k * a.K + c] : W[c * a.K + k], t);
+        }
+        reinterpret_cast<float*>(a.out[o])[row * C + c] = t;
+    }
+}
+
 // (float32: 80 KB, two workgroups per CU)
 template <typename T> constexpr int lin_lds() { return 2 * kFragVecs<Num<T>::P> * 16 + kWaves * RowShape<T>::kVecs * 16; }
 
@@ -163,7 +191,14 @@ template <typename T, bool DX, bool RESIDENT> __global__ __launch_bounds__(kThre
             if (RESIDENT && k == 1) gemm<P>(acc, f[RESIDENT ? 1 : 0], mine, lane);
             else gemm<P>(acc, f[0], mine, lane);
         }
+        bool again = false;
+        if constexpr (P == 3) again = holds_nan([&](int i) { return acc.get(i); }, 32);
         put_cols(reinterpret_cast<T*>(a.out[o]), C, c0, acc, stage, rows, lane);
+        if constexpr (P == 3)
+            if (again) {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // (the rows as they were first are on their way)
+                rows_again<DX>(a, o, c0, rows, lane);
+            }
     }
 }
 
@@ -276,6 +311,18 @@ template <typename T, int XT> __global__ __launch_bounds__(XT * 256) void k_grad
         const int o = m0 + 32 * (block >> 1) + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
         if (o < a.M && k < a.K) mine[(int64_t)o * a.K + k] = acc[i];
     }
+    if constexpr (P == 3)
+        if (holds_nan([&](int i) { return acc[i]; }, 16) && k < a.K) {      // as in rows_again: this worker's share of the nodes
+            const float *x = reinterpret_cast<const float*>(a.x) + k, *dy = reinterpret_cast<const float*>(a.dy[j]);
+            for (int i = 0; i < 16; ++i) {
+                const int o = m0 + 32 * (block >> 1) + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+                if (o >= a.M) break;
+                float t = 0.f;
+                for (int64_t q0 = blockIdx.x; q0 < panels; q0 += gridDim.x)
+                    for (int64_t r = q0 * 64; r < a.N && r < q0 * 64 + 64; ++r) t = fmaf(dy[r * a.M + o], x[r * a.K], t);
+                mine[(int64_t)o * a.K + k] = t;
+            }
+        }
     if (g == 0) {      // column sums of dy: over the lanes of a piece, then over the waves
         float* const part = reinterpret_cast<float*>(smem);
         __syncthreads();
