@@ -417,3 +417,25 @@ def test_module_as_one_operator_on_the_benchmark_graph(cuda, dtype):
     for a, b in zip(*results):
         assert torch.isfinite(a).all()
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("N,in_f,out_f,n", [(4096, 32, 64, 1), (64000, 128, 64, 1), (20000, 500, 64, 1), (64000, 128, 128, 3), (64000, 64, 40, 1)])
+def test_float32_linears_of_any_width_are_as_exact_as_float32_products(cuda, N, in_f, out_f, n):
+    """rms error against 64 bits, of the rms of the result.  Bound: the float32 matrix instructions round the running sum once per two
+    products, by an rms of 2^-24 / sqrt 3 of it; the sum's square grows evenly to that of the result, so k products leave
+    2^-24 sqrt(k / 12) and the store another 2^-24 / sqrt 3: below 2^-24 sqrt(1 + k / 12).  k: the contraction, for dW the 320 rows of
+    a worker's share at most."""
+    print(f"exactness case: N={N} in={in_f} out={out_f} n={n}", flush=True)
+    g = torch.Generator(device=cuda).manual_seed(N)
+    rand = lambda *s: torch.randn(*s, generator=g, device=cuda)
+    x, Ws, bs, dys = rand(N, in_f), [rand(out_f, in_f) / in_f ** 0.5 for _ in range(n)], [torch.zeros(out_f, device=cuda) for _ in range(n)], [rand(N, out_f) for _ in range(n)]
+    leaves = [x.requires_grad_(True)] + [W.requires_grad_(True) for W in Ws]
+    ys = LinearFunction.apply(x, *[t for pair in zip(Ws, bs) for t in pair])
+    grads = torch.autograd.grad(ys, leaves, dys)
+    X, W64, D = x.detach().double(), [W.detach().double() for W in Ws], [d.double() for d in dys]
+    rms = lambda a, b: float((a.double() - b).norm() / b.norm())
+    for name, k, got, want in (("y", in_f, ys[0], X @ W64[0].t()), ("dx", n * out_f, grads[0], sum(d @ W for d, W in zip(D, W64))), ("dW", 320, grads[1], D[0].t().contiguous() @ X)):
+        bound = 2 ** -24 * (1 + k / 12) ** 0.5
+        err = rms(got, want)
+        print(f"  {name}: {err:.2e} (bound {bound:.2e})", flush=True)
+        assert err <= bound, name

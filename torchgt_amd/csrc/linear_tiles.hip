@@ -7,6 +7,16 @@
 // accumulate in registers.  A contraction of up to 128 keeps its operands in registers for all output columns, so x is read
 // once; a longer one reads it again for every 64 columns.  The next piece of the weight is asked for before the products of
 // this one.  With few rows the output columns are spread over blockIdx.y until there are two workgroups per CU.
+//
+// float32: six of the nine products of planes (mid lo, lo mid, lo lo are below 2^-24 of the product), the five small ones in a sum of
+// their own.  rms error against 64 bits of the result's rms, here / v_mfma_f32_32x32x2_f32 (exact products, one rounding per two of
+// them) / all six in one sum, x, W, dy ~ normal:
+//   128 -> 64, 64 K rows     y 9.2e-8 / 1.5e-7 / 2.1e-7   dx 7.7e-8 / 1.5e-7 / 1.3e-7   dW 1.5e-7 / 3.1e-7 / 3.5e-7
+//   128 -> 64, 300 K rows    y 9.2e-8 / 1.5e-7 / 2.1e-7   dx 7.7e-8 / 1.4e-7 / 1.2e-7   dW 2.0e-7 / 6.1e-7 / 7.7e-7
+//   500 -> 64, 20 K rows     y 1.8e-7 / 2.7e-7 / 4.3e-7   dx 7.7e-8 / 1.4e-7 / 1.2e-7   dW 1.5e-7 / 3.3e-7 / 3.1e-7
+//   16 -> 40, 64 K rows      y 5.8e-8 / 5.9e-8 / 8.1e-8   dx 7.2e-8 / 1.1e-7 / 1.0e-7   dW 1.7e-7 / 2.4e-7 / 2.9e-7
+// and smaller than with the float32 instruction at every other shape of eleven (16 to 500 features, 16 to 128 columns, 1 K to 500 K rows).
+// us for 128 -> 64, 64 K rows: y 14.9 / 18.3 / 14.4, dx 15.6 / 19.1 / 18.4, dW with its sum 17.4 / 20.2 / 17.0.
 #include "linear_tiles.h"
 #include "node_tile.h"
 #include <algorithm>
@@ -188,8 +198,8 @@ template <typename T, bool DX, bool RESIDENT> __global__ __launch_bounds__(kThre
                 if (k + 1 < nk || t + 1 < end) ask_rows(k + 1 < nk ? k + 1 : 0);
             }
             __syncthreads();
-            if (RESIDENT && k == 1) gemm<P>(acc, f[RESIDENT ? 1 : 0], mine, lane);
-            else gemm<P>(acc, f[0], mine, lane);
+            if (RESIDENT && k == 1) gemm_apart<P>(acc, f[RESIDENT ? 1 : 0], mine, lane);
+            else gemm_apart<P>(acc, f[0], mine, lane);
         }
         bool again = false;
         if constexpr (P == 3) again = holds_nan([&](int i) { return acc.get(i); }, 32);
@@ -264,9 +274,9 @@ template <typename T, int XT> __global__ __launch_bounds__(XT * 256) void k_grad
     float sums[VE];
 #pragma unroll
     for (int e = 0; e < VE; ++e) sums[e] = 0.f;
-    float16_t acc;
+    float16_t acc, small;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+    for (int i = 0; i < 16; ++i) acc[i] = small[i] = 0.f;
     const int block = wave & 3, base_dy = operand_base(block >> 1, lane), base_x = operand_base(block & 1, lane);
     const unsigned char* const x_planes = smem + (1 + wave / 4) * P * kPanelBytes;
     int64_t p = blockIdx.x;
@@ -301,8 +311,9 @@ template <typename T, int XT> __global__ __launch_bounds__(XT * 256) void k_grad
         }
         __syncthreads();
         if (p + gridDim.x < panels) fetch(p + gridDim.x);
-        node_product<P, kPanelBytes>(acc, smem, x_planes, base_dy, base_x);
+        node_product<P, kPanelBytes, true>(acc, smem, x_planes, base_dy, base_x, &small);
     }
+    if constexpr (P == 3) acc += small;
     const int64_t per = (int64_t)a.M * a.K + a.M;
     float* const mine = a.partial + ((int64_t)blockIdx.x * a.nw + j) * per;
     const int k = k0 + 64 * (wave / 4) + 32 * (block & 1) + (lane & 31);
