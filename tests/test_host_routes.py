@@ -121,3 +121,24 @@ def test_attention_dropout_has_each_modules_mode():
     assert parameters(model) is None
     cores[0].eval()
     assert parameters(model) is not None and cores[0].dropout_at_work() == 0.0
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_data_parallel_wrapper_gets_gradients_layer_by_layer(kind, tmp_path):
+    """Its reduction overlaps with the backward only if gradients become ready one after the other; gradients that nobody waits for (no
+    wrapper, no gradients wanted) leave the operators their work."""
+    model, alone = build(kind), build(kind)
+    assert parameters(model) is not None
+    torch.distributed.init_process_group("gloo", init_method=f"file://{tmp_path}/store", rank=0, world_size=1)
+    try:
+        assert parameters(model) is not None
+        wrapped = torch.nn.parallel.DistributedDataParallel(model, find_unused_parameters=True)
+        assert parameters(model) is None and parameters(alone) is not None
+        with torch.no_grad():
+            assert parameters(model) is not None
+        del wrapped
+        handle = alone.layers[0].self_attention.linear_q.weight.register_post_accumulate_grad_hook(lambda p: None)
+        assert parameters(alone) is None
+        handle.remove()
+    finally:
+        torch.distributed.destroy_process_group()

@@ -6,7 +6,11 @@
 //                             heads, eps[2 L + 1], p_drop, seeds[L]) -> predictions
 //
 // A step's intermediate rows live in one allocation, its parameter gradients in another: with some seventy parameters the
-// host's time for tensors of their own would be longer than the kernels of a small graph take.
+// host's time for tensors of their own would be longer than the kernels of a small graph take.  So every parameter's gradient is a
+// part of one storage (a kept one keeps them all, 0.5 MB for the slim models; clone() it to keep one), and all of them are ready when the
+// node ends.  Where somebody waits for single gradients (gradients_watched) the model runs layer by layer instead.
+//
+//   torchgt::gradients_watched(params[]) -> bool
 #include "torch_common.h"
 
 namespace {
@@ -545,15 +549,29 @@ Tensor graph_graphormer(const Tensor& x, const Tensor& in_degree, const Tensor& 
     return GraphGraphormerFn::compute(GraphBatch{ids(x), ids(in_degree), ids(out_degree), ids(spatial_pos), ids(edge_ids)}, ab, p, c, false, rows, lse, bias, packed);
 }
 
+// Whether somebody waits for single gradients of these parameters: a data-parallel wrapper hooks every parameter's accumulation, to
+// reduce gradients while the backward goes on.
+bool gradients_watched(at::TensorList params) {
+    for (const Tensor& t : params) {
+        if (!t.defined() || !t.requires_grad()) continue;
+        if (!torch::autograd::impl::hooks(t).empty() || torch::autograd::impl::post_acc_grad_hooks(t) != nullptr) return true;
+        const auto node = torch::autograd::impl::try_get_grad_accumulator(t);
+        if (node && (!node->post_hooks().empty() || !node->pre_hooks().empty())) return true;
+    }
+    return false;
+}
+
 }  // namespace
 
 TORCH_LIBRARY_FRAGMENT(torchgt, m) {
+    m.def("gradients_watched(Tensor[] params) -> bool");
     m.def("node_graphormer(Tensor x, Tensor[] params, __torch__.torch.classes.torchgt.PlanHolder plan, Tensor workspace, int heads, int tokens, "
           "float[] eps) -> Tensor");
     m.def("graph_graphormer(Tensor x, Tensor in_degree, Tensor out_degree, Tensor attn_bias, Tensor spatial_pos, Tensor edge_ids, Tensor[] params, "
           "bool multi_hop, int max_dist, int heads, float[] eps, float p_drop, int[] seeds) -> Tensor");
 }
 TORCH_LIBRARY_IMPL(torchgt, CompositeImplicitAutograd, m) {
+    m.impl("gradients_watched", gradients_watched);
     m.impl("node_graphormer", node_graphormer);
     m.impl("graph_graphormer", graph_graphormer);
 }

@@ -5,8 +5,11 @@ every module it passes by is the library's own and nobody listens to it: ``plain
 import weakref
 
 import torch
+import torch.distributed
 import torch.nn as nn
 from torch.nn.modules import module as _torch_module
+
+from . import _ext
 
 
 def kind(cls):
@@ -116,6 +119,14 @@ class ModuleTree:
         return P
 
 
+def gradients_watched(parameters):
+    """Whether a data-parallel wrapper reduces these gradients while the backward goes on.  An operator for the whole model hands over
+    all of them at its end, its layers one by one hand over a layer's at a time: such a wrapper gets the layers.  Asked in jobs with a
+    process group only; gradients that are reduced after the backward (one flat all-reduce) do not ask for anything else."""
+    d = torch.distributed
+    return d.is_available() and d.is_initialized() and torch.is_grad_enabled() and _ext.op("gradients_watched")(parameters)
+
+
 _TREES = weakref.WeakKeyDictionary()      # model -> ModuleTree (which holds the model's modules, not the model)
 
 
@@ -124,4 +135,5 @@ def model_parameters(model, dtype):
     tree = _TREES.get(model)
     if tree is None or not tree.current():
         tree = _TREES[model] = ModuleTree(model, model._parameter_names(), model._called_modules())
-    return tree.parameters(dtype)
+    P = tree.parameters(dtype)
+    return None if P is None or gradients_watched(P) else P
