@@ -668,6 +668,7 @@ def bench_model(args):
         torch.cuda.synchronize()
         graph_ms = (time.perf_counter() - t0) / args.steps * 1e3
     groups = {"attention": ("attn_fwd", "bwd_node_side", "attn_bwd"), "projections and ffn linears": ("linear_fwd", "linear_dx", "linear_dw"),
+              "fused layers": ("node_pack", "node_fwd", "node_bwd_pre", "node_bwd_post", "node_sums", "gt_fwd", "gt_bwd"),
               "layer norm + residual": ("layer_norm_fwd", "layer_norm_bwd"), "gelu": ("gelu",), "nll loss": ("nll_loss",)}
     result = {
         "metric": "training step of the 4-layer " + ("GT" if gt else "Graphormer-Slim") + " on one 64 K-node sequence",
@@ -790,7 +791,8 @@ def bench_graph_model(args):
         graph_ms = (time.perf_counter() - t0) / args.steps * 1e3
     else:
         loss_value = float(loss.detach())
-    groups = {"dense attention": ("dense_fwd", "dense_bwd"), "bias builder": ("graph_bias_fwd", "graph_bias_bwd"),
+    groups = {"dense attention": ("dense_fwd", "dense_bwd", "dense_row0_fwd", "dense_row0_bwd"),
+              "fused layers": ("node_pack", "node_fwd", "node_bwd_pre", "node_bwd_post", "node_sums"), "bias builder": ("graph_bias_fwd", "graph_bias_bwd"),
               "projections and ffn linears": ("linear_fwd", "linear_dx", "linear_dw"),
               "layer norm + residual": ("layer_norm_fwd", "layer_norm_bwd"), "gelu": ("gelu",)}
     result = {

@@ -190,7 +190,8 @@ __device__ __forceinline__ float act_grad(float u, float dh) {
 // Kernel names of the optional per-kernel timing (timing.hip).
 enum KernelSlot { KS_FWD = 0, KS_NODE_SIDE, KS_BWD, KS_DENSE_FWD, KS_DENSE_BWD, KS_TILE_FWD, KS_TILE_BWD, KS_LINEAR_FWD,
                   KS_LINEAR_DX, KS_LINEAR_DW, KS_LAYER_NORM_FWD, KS_LAYER_NORM_BWD, KS_GELU, KS_GRAPH_BIAS_FWD,
-                  KS_GRAPH_BIAS_BWD, KS_LOSS, KS_COUNT };
+                  KS_GRAPH_BIAS_BWD, KS_LOSS, KS_NODE_PACK, KS_NODE_FWD, KS_NODE_BWD_PRE, KS_NODE_BWD_POST, KS_NODE_SUMS, KS_GT_FWD, KS_GT_BWD,
+                  KS_ROW0_FWD, KS_ROW0_BWD, KS_COUNT };
 
 // Scope guard: records a hipEvent on `st` before and after the launches made in
 // its scope when timing is enabled; does nothing otherwise.

@@ -262,7 +262,7 @@ int tgt_dense_row0_fwd(const void* d_q, const void* d_k, const void* d_v, const 
     using namespace tgt;
     if (int rc = row0_check("tgt_dense_row0_fwd", d_q, d_k, d_v, b, S, H, d, dtype, p_drop)) return rc;
     if (!d_s || !d_a0 || !d_s0 || !d_lse) { set_error("tgt_dense_row0_fwd: null pointer"); return TGT_ERR_INVALID_ARG; }
-    KernelTimer t(KS_DENSE_FWD, (hipStream_t)stream);
+    KernelTimer t(KS_ROW0_FWD, (hipStream_t)stream);
     const auto run = [&](auto tag) {
         using T = decltype(tag);
         Row0Args<T> a{};
@@ -278,7 +278,7 @@ int tgt_dense_row0_bwd(const void* d_q, const void* d_k, const void* d_v, const 
     using namespace tgt;
     if (int rc = row0_check("tgt_dense_row0_bwd", d_q, d_k, d_v, b, S, H, d, dtype, p_drop)) return rc;
     if (!d_a0 || !d_lse || !d_da0 || !d_g0 || !d_dq || !d_dk || !d_dv || !d_g || !d_dvirt) { set_error("tgt_dense_row0_bwd: null pointer"); return TGT_ERR_INVALID_ARG; }
-    KernelTimer t(KS_DENSE_BWD, (hipStream_t)stream);
+    KernelTimer t(KS_ROW0_BWD, (hipStream_t)stream);
     const auto run = [&](auto tag) {
         using T = decltype(tag);
         Row0Args<T> a{};

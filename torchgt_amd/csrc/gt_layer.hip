@@ -283,7 +283,7 @@ int tgt_gt_fwd(const tgt_gt_fwd_args* a, void* stream) {
     if (a->q && (!a->k || !a->v || !a->w_next || !a->v_next)) return bad("tgt_gt_fwd", "q needs k, v, w_next and v_next");
     if (a->rows == 0) return TGT_OK;
     const hipStream_t st = (hipStream_t)stream;
-    KernelTimer t(KS_LINEAR_FWD, st);
+    KernelTimer t(KS_GT_FWD, st);
     if (a->dtype == TGT_DTYPE_F32) return a->q ? run_fwd<float, true>(*a, st) : run_fwd<float, false>(*a, st);
     return a->q ? run_fwd<nbf16, true>(*a, st) : run_fwd<nbf16, false>(*a, st);
 }
@@ -295,7 +295,7 @@ int tgt_gt_bwd(const tgt_gt_bwd_args* a, void* stream) {
         return bad("tgt_gt_bwd", "null or bad argument");
     if (!a->nd || !a->Z || (a->heads != 8 && a->heads != 4 && a->heads != 2)) return bad("tgt_gt_bwd", "nd, Z and 8, 4 or 2 heads");
     const hipStream_t st = (hipStream_t)stream;
-    KernelTimer t(KS_LINEAR_DX, st);
+    KernelTimer t(KS_GT_BWD, st);
     return a->dtype == TGT_DTYPE_F32 ? run_bwd<float>(*a, st) : run_bwd<nbf16>(*a, st);
 }
 

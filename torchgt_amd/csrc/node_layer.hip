@@ -609,7 +609,7 @@ int tgt_node_pack(const void* const* mats, const int* ld, const int* rows, int n
         if (!mats[i] || rows[i] < 1 || rows[i] > 64 || ld[i] < 64 || ld[i] > 32767) return bad("tgt_node_pack", "weights are [1..64, >= 64]");
     for (int i = 0; i < n_vecs; ++i)
         if (!vecs[i] || lens[i] < 1 || lens[i] > 64) return bad("tgt_node_pack", "vectors have 1 to 64 elements");
-    KernelTimer t(KS_LINEAR_FWD, (hipStream_t)stream);
+    KernelTimer t(KS_NODE_PACK, (hipStream_t)stream);
     for (int m = 0, v = 0; m < n_mats || v < n_vecs;) {
         PackArgs a{};
         a.n_mats = std::min(kPackMats, n_mats - m); a.n_vecs = std::min(kPackVecs, n_vecs - v);
@@ -634,7 +634,7 @@ int tgt_node_fwd(const tgt_node_fwd_args* a, void* stream) {
     if (a->logp && (!a->attn || !a->w_next || !a->v_next || a->classes < 1 || a->classes > 64)) return bad("tgt_node_fwd", "logp needs attention rows, w_next, v_next and 1 to 64 classes");
     if (a->tokens < 0 || (!a->attn && a->tokens > 0 && (!a->token || !a->s_out))) return bad("tgt_node_fwd", "tokens need their table and s_out");
     if (a->rows == 0) return TGT_OK;
-    KernelTimer t(KS_LINEAR_FWD, (hipStream_t)stream);
+    KernelTimer t(KS_NODE_FWD, (hipStream_t)stream);
     const hipStream_t st = (hipStream_t)stream;
     if (a->dtype == TGT_DTYPE_F32) return dispatch_fwd<float, false>(*a, st);
     return a->same_bits ? dispatch_fwd<nbf16, true>(*a, st) : dispatch_fwd<nbf16, false>(*a, st);
@@ -647,7 +647,7 @@ int tgt_node_bwd_pre(const tgt_node_bwd_pre_args* a, void* stream) {
     if (!a || a->rows < 1 || !dtype_ok(a->dtype) || !a->s || !a->g_out || !a->w_back || (a->dlogp && !a->v_next) || !a->partial) return bad("tgt_node_bwd_pre", "null or bad argument");
     if (a->dlogp ? ((!a->logp && !a->linear) || a->classes < 1 || a->classes > 64 || a->tokens < 0) : (!a->dq || !a->dk || !a->dv || !a->g_in))
         return bad("tgt_node_bwd_pre", "dq, dk, dv, g_in or dlogp, logp and 1 to 64 classes are needed");
-    KernelTimer t(KS_LINEAR_DX, (hipStream_t)stream);
+    KernelTimer t(KS_NODE_BWD_PRE, (hipStream_t)stream);
     const int workers = grid_for(a->rows, 4);
     return a->dtype == TGT_DTYPE_F32 ? dispatch_bwd_pre<float>(*a, workers, (hipStream_t)stream) : dispatch_bwd_pre<nbf16>(*a, workers, (hipStream_t)stream);
 }
@@ -657,7 +657,7 @@ int tgt_node_bwd_post(const tgt_node_bwd_post_args* a, void* stream) {
     if (!a || a->rows < 1 || !dtype_ok(a->dtype) || !a->s || !a->attn || !a->g_in || !a->g_out || !a->d_attn || !a->w_post || !a->w_back || !a->v_post || !a->partial)
         return bad("tgt_node_bwd_post", "null or bad argument");
     if (a->nd && (!a->Z || (a->heads != 8 && a->heads != 4 && a->heads != 2))) return bad("tgt_node_bwd_post", "nd needs Z and 8, 4 or 2 heads");
-    KernelTimer t(KS_LINEAR_DX, (hipStream_t)stream);
+    KernelTimer t(KS_NODE_BWD_POST, (hipStream_t)stream);
     const hipStream_t st = (hipStream_t)stream;
     const int workers = grid_for(a->rows, 4);
     if (a->dtype == TGT_DTYPE_F32) return dispatch_bwd_post<float, false>(*a, workers, st);
@@ -667,7 +667,7 @@ int tgt_node_bwd_post(const tgt_node_bwd_post_args* a, void* stream) {
 int tgt_node_sums(const tgt_node_sum* sums, int count, int dtype, void* stream) {
     using namespace tgt;
     if (!sums || count < 1 || !dtype_ok(dtype)) return bad("tgt_node_sums", "null or bad argument");
-    KernelTimer t(KS_LINEAR_DW, (hipStream_t)stream);
+    KernelTimer t(KS_NODE_SUMS, (hipStream_t)stream);
     for (int c = 0; c < count; c += kMaxSums) {
         SumArgs a{};
         const int m = std::min(kMaxSums, count - c);

@@ -15,6 +15,7 @@ static const char* kSlotNames[KS_COUNT] = {
     "attn_fwd", "bwd_node_side", "attn_bwd", "dense_fwd", "dense_bwd", "tile_fwd", "tile_bwd",
     "linear_fwd", "linear_dx", "linear_dw", "layer_norm_fwd", "layer_norm_bwd", "gelu",
     "graph_bias_fwd", "graph_bias_bwd", "nll_loss",
+    "node_pack", "node_fwd", "node_bwd_pre", "node_bwd_post", "node_sums", "gt_fwd", "gt_bwd", "dense_row0_fwd", "dense_row0_bwd",
 };
 
 struct Pending { hipEvent_t start, stop; int slot; };
