@@ -4,6 +4,7 @@
 #include <stdint.h>
 #include <stdio.h>
 #include <stdarg.h>
+#include <atomic>
 #include <mutex>
 #include <vector>
 #include "../../include/torchgt_hip.h"
@@ -33,6 +34,22 @@ int reduce_partials(const tgt_reduce_desc* descs, int count, int dtype, hipStrea
             return TGT_ERR_HIP;                                                    \
         }                                                                          \
     } while (0)
+
+inline int num_cus() {
+    static const int n = [] { int dev = 0, v = 256; if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev); return v > 0 ? v : 256; }();
+    return n;
+}
+
+// Raises the dynamic LDS limit of a kernel, once per kernel and device (`done`: one bit per device, kept by the caller)
+inline int allow_lds(const void* kernel, int bytes, std::atomic<uint64_t>& done) {
+    int dev = 0;
+    TGT_HIP_CHECK(hipGetDevice(&dev));
+    const uint64_t bit = 1ull << (dev & 63);
+    if (done.load(std::memory_order_relaxed) & bit) return TGT_OK;
+    TGT_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+    done.fetch_or(bit, std::memory_order_relaxed);
+    return TGT_OK;
+}
 
 // One schedule entry: `len` consecutive edges starting at sorted position
 // `start`, all belonging to node `row`.  part < 0: the item covers the whole row

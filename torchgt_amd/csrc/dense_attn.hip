@@ -19,6 +19,7 @@
 // The bias is read straight from global memory in the layout each walk needs (see
 // key_of_row and the backward kernel); only q/k/v/dout heads are staged in LDS.
 #include "common.h"
+#include "dense_rows.h"
 #include "dense_dropout.h"
 #include <algorithm>
 #include <stdlib.h>
@@ -29,13 +30,6 @@ typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef float float16_t __attribute__((ext_vector_type(16)));
 
-struct dbf16 { uint16_t x; };
-
-__device__ __forceinline__ short f2bf(float f) {
-    const __bf16 b = static_cast<__bf16>(f);
-    return __builtin_bit_cast(short, b);
-}
-__device__ __forceinline__ float bf2f(short s) { return __uint_as_float(((uint32_t)(uint16_t)s) << 16); }
 // two / four floats -> bf16 (round to nearest even), two values per conversion instruction
 __device__ __forceinline__ uint32_t cvt_pk(float lo, float hi) {
     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -69,11 +63,6 @@ __device__ __forceinline__ void st4(float* p, float a, float b, float c, float d
     r.x = a; r.y = b; r.z = c; r.w = d;
     *reinterpret_cast<float4_t*>(p) = r;
 }
-__device__ __forceinline__ float ld1(const float* p) { return *p; }
-__device__ __forceinline__ float ld1(const dbf16* p) { return __uint_as_float(((uint32_t)p->x) << 16); }
-__device__ __forceinline__ void st1(float* p, float v) { *p = v; }
-__device__ __forceinline__ void st1(dbf16* p, float v) { p->x = (uint16_t)f2bf(v); }
-
 __device__ __forceinline__ float16_t mfma(short4_t a, short4_t b, float16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, b, c, 0, 0, 0);
 }
@@ -379,17 +368,11 @@ constexpr int kLdsLimit = 160 * 1024;
 // products from the LDS images, reductions over the wave.  Probabilities and dS are rounded to bf16
 // where the matrix path rounds them.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) x += __shfl_xor(x, off);
-    return x;
-}
 __device__ __forceinline__ float wave_max(float x) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) x = fmaxf(x, __shfl_xor(x, off));
     return x;
 }
-__device__ __forceinline__ float round_bf(float x) { return bf2f(f2bf(x)); }
 template <int D>
 __device__ __forceinline__ void lds_row(const short* __restrict__ rm, int row, float (&x)[D]) {
 #pragma unroll
@@ -397,13 +380,6 @@ __device__ __forceinline__ void lds_row(const short* __restrict__ rm, int row, f
         const short4_t v = *reinterpret_cast<const short4_t*>(&rm[row * D + 4 * c]);
         x[4 * c + 0] = bf2f(v.x); x[4 * c + 1] = bf2f(v.y); x[4 * c + 2] = bf2f(v.z); x[4 * c + 3] = bf2f(v.w);
     }
-}
-template <int D>
-__device__ __forceinline__ float dot_d(const float (&a)[D], const float (&b)[D]) {
-    float t = 0.f;
-#pragma unroll
-    for (int c = 0; c < D; ++c) t = fmaf(a[c], b[c], t);
-    return t;
 }
 template <typename T, int D>
 __device__ __forceinline__ void store_row(T* __restrict__ p, const float (&x)[D], float f) {

@@ -9,6 +9,7 @@
 // matrix-core kernels of dense_attn.hip round (scores in tiles of 32 keys with a running maximum, probabilities and dS to bf16),
 // float32 is float32 throughout (dense_attn_f32.hip).  Latency bound: a handful of dependent round trips.
 #include "dense_dropout.h"
+#include "dense_rows.h"
 #include <cmath>
 
 namespace tgt {
@@ -17,13 +18,8 @@ namespace {
 constexpr int kRow0Max = 1024;      // longest sequence (its scores sit in LDS)
 constexpr float kLog2e = 1.4426950408889634f;
 
-struct rbf16 { uint16_t x; };
-__device__ __forceinline__ float ld(const float* p) { return *p; }
-__device__ __forceinline__ float ld(const rbf16* p) { return __uint_as_float((uint32_t)p->x << 16); }
-__device__ __forceinline__ void st(float* p, float v) { *p = v; }
-__device__ __forceinline__ void st(rbf16* p, float v) { p->x = __builtin_bit_cast(uint16_t, static_cast<__bf16>(v)); }
 __device__ __forceinline__ float rounded(float v, const float*) { return v; }
-__device__ __forceinline__ float rounded(float v, const rbf16*) { return static_cast<float>(static_cast<__bf16>(v)); }
+__device__ __forceinline__ float rounded(float v, const dbf16*) { return round_bf(v); }
 
 template <int D> __device__ __forceinline__ void load_vec(const float* p, float (&x)[D]) {
 #pragma unroll
@@ -32,7 +28,7 @@ template <int D> __device__ __forceinline__ void load_vec(const float* p, float 
         x[c] = f.x; x[c + 1] = f.y; x[c + 2] = f.z; x[c + 3] = f.w;
     }
 }
-template <int D> __device__ __forceinline__ void load_vec(const rbf16* p, float (&x)[D]) {
+template <int D> __device__ __forceinline__ void load_vec(const dbf16* p, float (&x)[D]) {
 #pragma unroll
     for (int c = 0; c < D; c += 8) {
         const uint4 u = *reinterpret_cast<const uint4*>(p + c);
@@ -48,7 +44,7 @@ template <int D> __device__ __forceinline__ void store_vec(float* p, const float
 #pragma unroll
     for (int c = 0; c < D; c += 4) *reinterpret_cast<float4*>(p + c) = make_float4(x[c], x[c + 1], x[c + 2], x[c + 3]);
 }
-template <int D> __device__ __forceinline__ void store_vec(rbf16* p, const float (&x)[D]) {
+template <int D> __device__ __forceinline__ void store_vec(dbf16* p, const float (&x)[D]) {
 #pragma unroll
     for (int c = 0; c < D; c += 8) {
         uint32_t w[4];
@@ -58,19 +54,8 @@ template <int D> __device__ __forceinline__ void store_vec(rbf16* p, const float
         *reinterpret_cast<uint4*>(p + c) = make_uint4(w[0], w[1], w[2], w[3]);
     }
 }
-template <int D> __device__ __forceinline__ float dot(const float (&a)[D], const float (&b)[D]) {
-    float t = 0.f;
-#pragma unroll
-    for (int c = 0; c < D; ++c) t = fmaf(a[c], b[c], t);
-    return t;
-}
-__device__ __forceinline__ float sum64(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
 __device__ __forceinline__ float exp_of(float x, const float*) { return expf(x); }
-__device__ __forceinline__ float exp_of(float x, const rbf16*) { return __builtin_amdgcn_exp2f(x * kLog2e); }
+__device__ __forceinline__ float exp_of(float x, const dbf16*) { return __builtin_amdgcn_exp2f(x * kLog2e); }
 
 template <typename T> struct Row0Args {
     const T *q, *k, *v, *bias, *s;
@@ -93,7 +78,7 @@ template <typename T, int D> __device__ __forceinline__ void scaled_query(const 
         for (int c = 0; c < D; ++c) q[c] *= a.scale;
 }
 template <typename T, int D> __device__ __forceinline__ float score_of(const Row0Args<T>& a, const float (&q)[D], const float (&k)[D], float bias) {
-    return sizeof(T) == 2 ? fmaf(dot<D>(q, k), a.scale, bias) : dot<D>(q, k) + bias;
+    return sizeof(T) == 2 ? fmaf(dot_d<D>(q, k), a.scale, bias) : dot_d<D>(q, k) + bias;
 }
 
 template <typename T, int D, bool DROP> __global__ __launch_bounds__(512) void k_row0_fwd(const Row0Args<T> a, const DropArgs da) {
@@ -112,7 +97,7 @@ template <typename T, int D, bool DROP> __global__ __launch_bounds__(512) void k
         if (key < S) {
             float kv[D];
             load_vec<D>(a.k + row + key * pitch, kv);
-            const float bv = bias ? ld(bias + key) : 0.f;
+            const float bv = bias ? ld1(bias + key) : 0.f;
             sc = score_of(a, q, kv, bv);
             score[key] = sc;
         }
@@ -157,10 +142,10 @@ template <typename T, int D, bool DROP> __global__ __launch_bounds__(512) void k
 #pragma unroll
         for (int c = 0; c < D; ++c) o[c] = fmaf(w, vv[c], o[c]);
     }
-    l = sum64(l);
+    l = wave_sum(l);
     const float inv = (DROP ? da.inv_keep : 1.f) / l;
 #pragma unroll
-    for (int c = 0; c < D; ++c) o[c] = sum64(o[c]) * inv;
+    for (int c = 0; c < D; ++c) o[c] = wave_sum(o[c]) * inv;
     const int64_t at = ((int64_t)g * H + h) * D;
     if (lane == 0) {
         store_vec<D>(a.a0 + at, o);
@@ -180,7 +165,7 @@ template <typename T, int D, bool DROP> __global__ __launch_bounds__(512) void k
     load_vec<D>(a.g0 + at, g0);
 #pragma unroll
     for (int c = 0; c < D; ++c) { dq[c] = 0.f; none[c] = 0.f; }
-    const float delta = dot<D>(o, gv), lse = a.lse[g * H + h];
+    const float delta = dot_d<D>(o, gv), lse = a.lse[g * H + h];
     const uint32_t rh = DROP ? drop_row_hash(da, g * H + h, 0) : 0u;
     const T* bias = a.bias ? a.bias + ((int64_t)g * H + h) * S * S : nullptr;
     float dv_sum = 0.f;
@@ -188,9 +173,9 @@ template <typename T, int D, bool DROP> __global__ __launch_bounds__(512) void k
         float kv[D], vv[D];
         load_vec<D>(a.k + row + key * pitch, kv);
         load_vec<D>(a.v + row + key * pitch, vv);
-        const float sc = score_of(a, q, kv, bias ? ld(bias + key) : 0.f);
+        const float sc = score_of(a, q, kv, bias ? ld1(bias + key) : 0.f);
         const float p = exp_of(sc - lse, tag), ks = !DROP ? 1.f : (drop_keep(da, rh, key) ? da.inv_keep : 0.f);
-        const float ds = rounded(p * (dot<D>(gv, vv) * ks - delta), tag), pb = rounded(p * ks, tag);
+        const float ds = rounded(p * (dot_d<D>(gv, vv) * ks - delta), tag), pb = rounded(p * ks, tag);
         dv_sum += ds;
 #pragma unroll
         for (int c = 0; c < D; ++c) {
@@ -206,8 +191,8 @@ template <typename T, int D, bool DROP> __global__ __launch_bounds__(512) void k
         }
     }
 #pragma unroll
-    for (int c = 0; c < D; ++c) dq[c] = sum64(dq[c]) * a.scale;
-    dv_sum = sum64(dv_sum);
+    for (int c = 0; c < D; ++c) dq[c] = wave_sum(dq[c]) * a.scale;
+    dv_sum = wave_sum(dv_sum);
     if (lane == 0) {
         store_vec<D>(a.dq + row, dq);
         store_vec<D>(a.g + row, g0);
@@ -219,8 +204,8 @@ template <typename T, int D, bool DROP> __global__ __launch_bounds__(512) void k
 template <typename T> __global__ __launch_bounds__(64) void k_row0_virtual(const float* __restrict__ dvirt, int b, int H, T* __restrict__ d) {
     float t = 0.f;
     for (int g = threadIdx.x; g < b; g += 64) t += dvirt[g * H + blockIdx.x];
-    t = sum64(t);
-    if (threadIdx.x == 0) st(d + blockIdx.x, ld(d + blockIdx.x) + t);
+    t = wave_sum(t);
+    if (threadIdx.x == 0) st1(d + blockIdx.x, ld1(d + blockIdx.x) + t);
 }
 
 int row0_check(const char* who, const void* q, const void* k, const void* v, int b, int S, int H, int d, int dtype, float p_drop) {
@@ -270,7 +255,7 @@ int tgt_dense_row0_fwd(const void* d_q, const void* d_k, const void* d_v, const 
         a.b = b; a.S = S; a.H = H; a.a0 = (T*)d_a0; a.s0 = (T*)d_s0; a.lse = d_lse;
         return row0(a, d, p_drop, seed, false, (hipStream_t)stream);
     };
-    return dtype == TGT_DTYPE_F32 ? run(float()) : run(rbf16());
+    return dtype == TGT_DTYPE_F32 ? run(float()) : run(dbf16());
 }
 
 int tgt_dense_row0_bwd(const void* d_q, const void* d_k, const void* d_v, const void* d_bias, int b, int S, int H, int d, int dtype, float p_drop, uint64_t seed, const void* d_a0,
@@ -287,7 +272,7 @@ int tgt_dense_row0_bwd(const void* d_q, const void* d_k, const void* d_v, const 
         a.dq = (T*)d_dq; a.dk = (T*)d_dk; a.dv = (T*)d_dv; a.g = (T*)d_g; a.dvirt = d_dvirt;
         return row0(a, d, p_drop, seed, true, (hipStream_t)stream);
     };
-    return dtype == TGT_DTYPE_F32 ? run(float()) : run(rbf16());
+    return dtype == TGT_DTYPE_F32 ? run(float()) : run(dbf16());
 }
 
 int tgt_dense_row0_virtual(const float* d_dvirt, int b, int H, int dtype, void* d_dvirtual_dist, void* stream) {
@@ -295,7 +280,7 @@ int tgt_dense_row0_virtual(const float* d_dvirt, int b, int H, int dtype, void* 
     if (!d_dvirt || b < 1 || H < 1 || !d_dvirtual_dist || (dtype != TGT_DTYPE_F32 && dtype != TGT_DTYPE_BF16)) { set_error("tgt_dense_row0_virtual: null or bad argument"); return TGT_ERR_INVALID_ARG; }
     KernelTimer t(KS_GRAPH_BIAS_BWD, (hipStream_t)stream);
     if (dtype == TGT_DTYPE_F32) hipLaunchKernelGGL((k_row0_virtual<float>), dim3(H), dim3(64), 0, (hipStream_t)stream, d_dvirt, b, H, (float*)d_dvirtual_dist);
-    else hipLaunchKernelGGL((k_row0_virtual<rbf16>), dim3(H), dim3(64), 0, (hipStream_t)stream, d_dvirt, b, H, (rbf16*)d_dvirtual_dist);
+    else hipLaunchKernelGGL((k_row0_virtual<dbf16>), dim3(H), dim3(64), 0, (hipStream_t)stream, d_dvirt, b, H, (dbf16*)d_dvirtual_dist);
     TGT_HIP_CHECK(hipGetLastError());
     return TGT_OK;
 }

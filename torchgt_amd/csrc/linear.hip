@@ -15,9 +15,8 @@
 //   k_gradw_tiles        dW_j = dy_j^T x, db_j = colsum(dy_j) (linear_tiles.hip): each workgroup keeps its tiles in
 //                        registers over its share of the panels and writes one partial; reduce.hip adds the
 //                        partials in a fixed order (no atomics: results are reproducible)
-// Matrix instructions: v_mfma_f32_32x32x2_f32 for float32 (exact fp32 products,
-// fp32 accumulation; the 64-wide forward instead splits every float into three
-// bf16 and uses the bf16 instructions, see k_linear64_split),
+// Matrix instructions: float32 operands are split into three bf16 parts and go through the bf16 instructions (see k_linear64_split and
+// linear_tiles.hip), but for the 64-wide input gradient on its own, which uses v_mfma_f32_32x32x2_f32 (exact fp32 products);
 // v_mfma_f32_32x32x8_bf16_1k for bf16 (fp32 accumulation).
 //   A 32xk : lane l holds A[l%32][k-slice of half l/32]
 //   B kx32 : lane l holds B[k-slice of half l/32][l%32]
@@ -505,19 +504,6 @@ __global__ __launch_bounds__(kThreads) void k_linear64_split(LinArgs a) {
             store_rows<float>(out, 64, acc, 0.f, a.N - (p * 64 + 32 * rb + 4 * h));
         }
     }
-}
-
-int num_cus() {
-    static int cus = 0;
-    if (cus == 0) {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
-            cus = n;
-        else
-            cus = 256;
-    }
-    return cus;
 }
 
 template <typename T, bool DX, int NW, int ACT = 0>

@@ -20,7 +20,6 @@
 #include "linear_tiles.h"
 #include "node_tile.h"
 #include <algorithm>
-#include <atomic>
 
 namespace tgt {
 namespace {
@@ -210,18 +209,6 @@ template <typename T, bool DX, bool RESIDENT> __global__ __launch_bounds__(kThre
                 rows_again<DX>(a, o, c0, rows, lane);
             }
     }
-}
-
-// Raises the dynamic LDS limit of a kernel where it needs that, once per kernel and device (`done`: one bit per device)
-int allow_lds(const void* kernel, int bytes, std::atomic<uint64_t>& done) {
-    if (bytes <= 64 * 1024) return TGT_OK;
-    int dev = 0;
-    TGT_HIP_CHECK(hipGetDevice(&dev));
-    const uint64_t bit = 1ull << (dev & 63);
-    if (done.load(std::memory_order_relaxed) & bit) return TGT_OK;
-    TGT_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
-    done.fetch_or(bit, std::memory_order_relaxed);
-    return TGT_OK;
 }
 
 template <typename T, bool DX, bool RESIDENT> int launch(const LinArgs& a, hipStream_t st) {

@@ -13,8 +13,9 @@
 // features per node forward and 47 backward through memory; here it moves 6 and 12 (q, k, v, the residual stream and the
 // attention rows; the intermediate activations are recomputed in the backward from s and a: two products, against two rows
 // written and read).  A wave takes 32 nodes and keeps them in registers through the whole chain (node_tile.h); the waves of
-// a workgroup share the packed weights in LDS.  Weight gradients contract over nodes: the waves put the bf16 planes of both
-// operands into LDS, four waves (128 nodes) at a time, and every wave adds one 32 x 32 block over its share of the nodes.
+// a workgroup share the packed weights in LDS.  Weight gradients contract over nodes: in the backward kernels four waves carry 32
+// nodes each through the chain and put the bf16 planes of both operands into LDS, four others keep one 32 x 32 block of every
+// weight gradient each and add the products over these 128 nodes beside it (node_roles.h).
 #include "node_roles.h"
 
 namespace tgt {

@@ -3,7 +3,6 @@
 #pragma once
 #include "node_tile.h"
 #include <algorithm>
-#include <atomic>
 
 namespace tgt {
 namespace {
@@ -104,23 +103,9 @@ template <typename T> __device__ __forceinline__ void put_node_side(const Tile& 
 }
 
 int bad(const char* who, const char* what) { set_error("%s: %s", who, what); return TGT_ERR_INVALID_ARG; }
-int num_cus() {
-    static const int n = [] { int dev = 0, v = 256; if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev); return v > 0 ? v : 256; }();
-    return n;
-}
 // a workgroup of `waves` waves per CU (LDS), fewer when there is less work
 int grid_for(int64_t rows, int waves) { return (int)std::max<int64_t>(1, std::min<int64_t>(num_cus(), ((rows + 31) / 32 + waves - 1) / waves)); }
 
-// Raises the dynamic LDS limit of a kernel, once per kernel and device (`done`: one bit per device, kept by the caller)
-int allow_lds(const void* kernel, int bytes, std::atomic<uint64_t>& done) {
-    int dev = 0;
-    TGT_HIP_CHECK(hipGetDevice(&dev));
-    const uint64_t bit = 1ull << (dev & 63);
-    if (done.load(std::memory_order_relaxed) & bit) return TGT_OK;
-    TGT_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
-    done.fetch_or(bit, std::memory_order_relaxed);
-    return TGT_OK;
-}
 template <typename... Args> int launch(void (*kernel)(Args...), std::atomic<uint64_t>& done, int grid, int threads, int lds, hipStream_t st, Args... args) {
     if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), lds, done)) return rc;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds, st, args...);

@@ -9,9 +9,13 @@
 // linears, residual adds, LayerNorms and activations never leaves the registers.  LayerNorm sums are 32 adds in a lane
 // and one exchange between the halves.
 //
-// Number formats.  bf16 kernels round where a chain of separate kernels would have stored a tensor (`stored`), so a model gives
-// the same numbers whichever way it runs, up to the order of float32 sums.  float32 rows go through the matrix unit as three bf16 planes (see linear.hip: hi + mid + lo is exact,
-// six products per pair of planes give the float32 product to a few 2^-23); bf16 rows as one.  P = number of planes.
+// Number formats.  bf16 kernels round where a chain of separate kernels would have stored a tensor (`stored`).  The numbers are those
+// of the separate kernels up to the order of float32 sums and, in the node-level Graphormer, to another evaluation of GELU
+// (normal_cdf): in float32 both are a few 2^-24 of a row; in bf16 a sum that rounds the other way moves a value by 2^-8 of it, and a
+// model's outputs and gradients differ by 0.2 to 1 % of their norm between the two ways of running it, each as far from float32 as
+// the other.  Where bits of the separate kernels are wanted (`SAME`), sums and GELU follow them.
+// float32 rows go through the matrix unit as three bf16 planes (see linear.hip: hi + mid + lo is exact, six products per pair of planes
+// give the float32 product to a few 2^-23); bf16 rows as one.  P = number of planes.
 #pragma once
 #include "common.h"
 
