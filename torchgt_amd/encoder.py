@@ -181,7 +181,7 @@ class Graphormer(nn.Module):
     one_operator = True      # False: always run the model layer by layer
 
     def _one_operator(self, x, attn_bias, edge_index, perturb, attn_type):
-        """The model's parameters in the order of the whole-model operators when one of them covers this call - sparse
+        """(parameters, eps of the norms) in the order of the whole-model operators when one of them covers this call - sparse
         attention without a bias, no dropout at work, every linear with its bias, one dtype, one global token (the rows that
         come back are 1 .. of the sequence, :391, whatever the number of tokens: the operators return the nodes' rows) -
         else None."""
@@ -189,8 +189,8 @@ class Graphormer(nn.Module):
             return None
         if x.dim() != 2 or not x.is_cuda or x.dtype not in _DT or autocast_to_float32(x):
             return None
-        P = model_parameters(self, x.dtype)
-        return P if P is not None and self.layers[0].self_attention.num_heads == self.num_heads else None
+        found = model_parameters(self, x.dtype)
+        return found if found is not None and self.layers[0].self_attention.num_heads == self.num_heads else None
 
     @staticmethod
     def _fused(P, heads):
@@ -203,16 +203,19 @@ class Graphormer(nn.Module):
             names += [f"layers.{i}.{k}" for k in LAYER_PARAMETERS]
         return names + ["final_ln.weight", "final_ln.bias", "downstream_out_proj.weight", "downstream_out_proj.bias"]
 
+    def _norm_names(self):
+        return [f"layers.{i}.{k}" for i in range(len(self.layers)) for k in ("self_attention_norm", "ffn_norm")] + ["final_ln"]
+
     def _called_modules(self):
         return [("input_dropout", DROPOUT)] + layer_modules(len(self.layers), _LAYER)
 
     def forward(self, x, attn_bias, edge_index, perturb=None, attn_type=None):
-        P = self._one_operator(x, attn_bias, edge_index, perturb, attn_type)
-        if P is not None:
+        found = self._one_operator(x, attn_bias, edge_index, perturb, attn_type)
+        if found is not None:
             # the whole model as one operator and one autograd node
             plan = edge_index if isinstance(edge_index, GraphPlan) else get_plan(edge_index, x.shape[0] + 1)
             plan.handle      # raises if the plan was closed
-            eps = [e for layer in self.layers for e in (layer.self_attention_norm.eps, layer.ffn_norm.eps)] + [self.final_ln.eps]
+            P, eps = found
             H, tokens, classes, ve = self.num_heads, 1, P[-1].shape[0], 4 if x.dtype == torch.float32 else 8
             if self._fused(P, H):      # kernels that take a layer's node-local part in one pass each way
                 if x.shape[1] % ve:

@@ -200,7 +200,7 @@ class Graphormer(nn.Module):
     one_operator = True      # False: always run the model layer by layer
 
     def _one_operator(self, batched_data):
-        """The model's parameters in the operator's order when ``torch.ops.torchgt.graph_graphormer`` covers this call - the
+        """(parameters, eps of the norms) in the operator's order when ``torch.ops.torchgt.graph_graphormer`` covers this call - the
         bias as a tensor and what ``_operator_parameters`` asks of the model - else None."""
         if not self.one_operator or self.bias_from_ids or not batched_data.attn_bias.is_cuda or batched_data.x.numel() == 0:
             return None
@@ -218,16 +218,20 @@ class Graphormer(nn.Module):
             names += [f"layers.{i}.{k}" for k in LAYER_PARAMETERS]
         return names + ["final_ln.weight", "final_ln.bias", f"{head}.weight", f"{head}.bias"]
 
+    def _norm_names(self):
+        return [f"layers.{i}.{k}" for i in range(len(self.layers)) for k in ("self_attention_norm", "ffn_norm")] + ["final_ln"]
+
     def _called_modules(self):
         return [("graph_node_feature", _NODE_FEATURE), ("graph_attn_bias", _ATTN_BIAS), ("input_dropout", DROPOUT)] + layer_modules(len(self.layers), _LAYER)
 
     def _operator_parameters(self):
-        """The parameters in the operator's order if the model has hidden and feed-forward width 64, at most 64 outputs, no
+        """(parameters, eps of the norms) in the operator's order if the model has hidden and feed-forward width 64, at most 64 outputs, no
         dropout at work but the attention's and one dtype, else None."""
         multi_hop = self._multi_hop()
-        P = model_parameters(self, getattr(getattr(self.final_ln, "weight", None), "dtype", None))
-        if P is None:
+        found = model_parameters(self, getattr(getattr(self.final_ln, "weight", None), "dtype", None))
+        if found is None:
             return None
+        P = found[0]
         p = self.layers[0].self_attention.dist_attn.local_attn.dropout_at_work()
         for layer in self.layers:
             core = layer.self_attention.dist_attn.local_attn
@@ -236,18 +240,18 @@ class Graphormer(nn.Module):
         if P[0].dtype not in _DT or P[0].shape[1] != 64 or P[-1].shape[0] > 64 or P[4].shape[1] != self.layers[0].self_attention.num_heads or \
                 any(p.shape[0] != 64 or p.shape[-1] != 64 for p in P[8 if multi_hop else 7:-4]):
             return None
-        return P
+        return found
 
     def forward(self, batched_data, perturb=None):
-        P = self._one_operator(batched_data)
-        if P is not None:
+        found = self._one_operator(batched_data)
+        if found is not None:
             # the whole model as one operator and one autograd node: node features, bias, layers, head (the last layer's
             # attention and what follows it at the virtual nodes only: no other row of it is read)
             multi_hop = self.graph_attn_bias.edge_type == "multi_hop"
             att = self.layers[0].self_attention
             p = att.dist_attn.local_attn.dropout_at_work()
             seeds = [int(torch.randint(0, 2 ** 62, (1,)).item()) if p > 0 else 0 for _ in self.layers]
-            eps = [e for layer in self.layers for e in (layer.self_attention_norm.eps, layer.ffn_norm.eps)] + [self.final_ln.eps]
+            P, eps = found
             d = batched_data
             return _ext.op("graph_graphormer")(d.x, d.in_degree, d.out_degree, d.attn_bias, d.spatial_pos, d.edge_input if multi_hop else d.attn_edge_type,
                                                P, multi_hop, int(self.graph_attn_bias.multi_hop_max_dist), att.num_heads, eps, p, seeds)

@@ -110,6 +110,9 @@ class GT(nn.Module):
                 names += both(f"layers.{i}.{part}")
         return names + [n for j in range(3) for n in both(f"MLP_layer.FC_layers.{j}")]
 
+    def _norm_names(self):
+        return [f"layers.{i}.{k}" for i in range(len(self.layers)) for k in ("layer_norm1", "layer_norm2")]
+
     def _called_modules(self):
         out = [("input_dropout", DROPOUT), ("MLP_layer", _READOUT)]
         for i in range(len(self.layers)):
@@ -117,24 +120,24 @@ class GT(nn.Module):
         return out
 
     def _one_operator(self, x, edge_index, attn_type):
-        """The model's parameters in the operator's order when ``torch.ops.torchgt.node_gt`` covers this call, else None."""
+        """(parameters, eps of the norms) in the operator's order when ``torch.ops.torchgt.node_gt`` covers this call, else None."""
         if not self.one_operator or attn_type != "sparse" or edge_index is None or x.dim() != 2 or not x.is_cuda or x.dtype not in _DT or \
                 autocast_to_float32(x) or getattr(self.MLP_layer, "L", None) != 2:
             return None
-        P = model_parameters(self, x.dtype)
+        found = model_parameters(self, x.dtype)
         ve = 4 if x.dtype == torch.float32 else 8
-        if P is None or any(p.shape[0] % ve for p in P[:-2]) or P[2].shape[0] % self.layers[0].self_attention.num_heads:
+        if found is None or any(p.shape[0] % ve for p in found[0][:-2]) or found[0][2].shape[0] % self.layers[0].self_attention.num_heads:
             return None
-        return P
+        return found
 
     def forward(self, x, attn_bias, edge_index, perturb=None, attn_type=None):
-        P = self._one_operator(x, edge_index, attn_type)
-        if P is not None:
+        found = self._one_operator(x, edge_index, attn_type)
+        if found is not None:
             # the whole model as one operator and one autograd node
             H = self.layers[0].self_attention.num_heads
             plan = edge_index if isinstance(edge_index, GraphPlan) else get_plan(edge_index, x.shape[0])
             plan.handle      # raises if the plan was closed
-            eps, classes = [e for layer in self.layers for e in (layer.layer_norm1.eps, layer.layer_norm2.eps)], P[-1].shape[0]
+            (P, eps), classes = found, found[0][-1].shape[0]
             x = padded(P, x, 0, -2)
             return _ext.op("node_gt")(x, P, plan.holder, plan.workspace(H, P[2].shape[0] // H), H, classes, eps)
         x = x.unsqueeze(0)

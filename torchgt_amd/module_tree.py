@@ -25,7 +25,7 @@ def plain(module, cls, forward):
     object or the class, no hook, no compiled call."""
     d = module.__dict__
     return type(module) is cls and cls.forward is forward and "forward" not in d and not (
-        d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"] or d.get("_compiled_call_impl"))
+        d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"] or "_compiled_call_impl" in d)
 
 
 def all_plain(*pairs):
@@ -47,11 +47,11 @@ class ModuleTree:
     attribute look-ups of seventy parameters through ``nn.Module`` would be a third of it.  Remembers the dictionaries of the
     modules, not the parameters, and notices when a module of the tree was exchanged (``current``).
 
-    names: the parameters in the operator's order; called: (path, kind) of the modules that the model calls when it runs module by
-    module."""
+    names: the parameters in the operator's order; norms: the modules whose ``eps`` it takes; called: (path, kind) of the modules that
+    the model calls when it runs module by module."""
 
-    def __init__(self, root, names, called):
-        self.links, self.slots, self.called, self.dropouts = [], [], [], []
+    def __init__(self, root, names, norms, called):
+        self.links, self.slots, self.norms, self.called, self.dropouts, self.layers = [], [], [], [], [], []
         seen = set()
 
         def step(module, name):
@@ -67,28 +67,35 @@ class ModuleTree:
                 m = step(m, part) if m is not None else None
             return m
 
-        step(root, "layers")
-        self.missing = False      # a module of the names is not there: somebody's own module stands in its place
+        self.count = len(root.layers)
+        self.all_layers = step(root, "layers")._modules
+        self.missing = self.count == 0      # a module of the names is not there: somebody's own module stands in its place
         for full in names:
             *path, leaf = full.split(".")
             m = at(path)
             if m is None:
                 self.missing = True
-                break
+                return
             self.slots.append((m._parameters, leaf))
+        for path in norms:
+            m = at(path.split("."))
+            if m is None or "eps" not in m.__dict__:
+                self.missing = True
+                return
+            self.norms.append(m.__dict__)
         for path, (cls, forward) in called:
             m = at(path.split("."))
             if m is None:
                 self.missing = True
-                break
-            self.called.append((m, cls, forward))
+                return
+            self.called.append((m, m.__dict__, cls))
             if cls is nn.Dropout:
                 self.dropouts.append(m.__dict__)
-        self.count = len(root.layers)
-        self.layers = root.layers._modules
+        self.classes = list({kind for _, kind in called})
+        self.layers = [(layer, layer.__dict__, layer._modules.get("self_attention")) for layer in self.all_layers.values()]
 
     def current(self):
-        if len(self.layers) != self.count:
+        if len(self.all_layers) != self.count:
             return False
         for d, name, child in self.links:
             if d.get(name) is not child:
@@ -96,27 +103,30 @@ class ModuleTree:
         return True
 
     def parameters(self, dtype):
-        """The parameters in order, or None: one is absent or has another dtype, a module is not plain or was asked to run step by
-        step, or dropout is at work (each dropout module has its own mode, whatever the model's)."""
-        if self.missing or self.count == 0 or watched_everywhere():
+        """(parameters, eps of the norms), each in order, or None: one is absent or has another dtype, a module is not plain or was asked
+        to run step by step, or dropout is at work (each dropout module has its own mode, whatever the model's)."""
+        if self.missing or watched_everywhere():
             return None
-        for m, cls, forward in self.called:
-            if not plain(m, cls, forward):
+        for cls, forward in self.classes:
+            if cls.forward is not forward:
+                return None
+        for m, d, cls in self.called:      # ``plain``, without a call for each of the thirty
+            if type(m) is not cls or "forward" in d or d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or \
+                    d["_backward_pre_hooks"] or "_compiled_call_impl" in d:
                 return None
         for d in self.dropouts:
             if d["training"] and d["p"] > 0:
                 return None
         heads = None
-        for layer in self.layers.values():
-            att = layer._modules["self_attention"]
-            if "one_operator" in layer.__dict__ or not layer.one_operator or not att.one_operator or att.num_heads != (heads or att.num_heads):
+        for layer, d, att in self.layers:
+            if "one_operator" in d or not layer.one_operator or not att.one_operator or att.num_heads != (heads or att.num_heads):
                 return None
             heads = att.num_heads
         P = [d.get(name) for d, name in self.slots]
         for p in P:
             if p is None or p.dtype is not dtype:
                 return None
-        return P
+        return P, [d["eps"] for d in self.norms]
 
 
 def gradients_watched(parameters):
@@ -131,9 +141,9 @@ _TREES = weakref.WeakKeyDictionary()      # model -> ModuleTree (which holds the
 
 
 def model_parameters(model, dtype):
-    """Parameters of a model in the order of its whole-model operators, or None where they do not cover its state."""
+    """(parameters, eps of the norms) of a model in the order of its whole-model operators, or None where they do not cover its state."""
     tree = _TREES.get(model)
     if tree is None or not tree.current():
-        tree = _TREES[model] = ModuleTree(model, model._parameter_names(), model._called_modules())
-    P = tree.parameters(dtype)
-    return None if P is None or gradients_watched(P) else P
+        tree = _TREES[model] = ModuleTree(model, model._parameter_names(), model._norm_names(), model._called_modules())
+    found = tree.parameters(dtype)
+    return None if found is None or gradients_watched(found[0]) else found
