@@ -166,3 +166,18 @@ def test_bias_gradients_of_a_large_batch_go_into_a_running_sum(cuda):
         got.append((torch.cuda.max_memory_allocated() - before, torch.cat([p.grad.flatten() for p in model.parameters() if p.grad is not None])))
     assert got[0][0] <= 4.5 * one_bias      # the bias, the sum, one layer's gradient, all rows of the step (1 to 1.5 of a bias)
     assert float((got[0][1] - got[1][1]).norm()) <= 3e-5 * float(got[1][1].norm())
+
+
+@pytest.mark.parametrize("kind,hidden", [("gt", 64), ("gt", 128), ("graphormer", 64), ("graphormer", 128)])
+def test_forward_mode_is_refused_not_dropped(cuda, kind, hidden):
+    """A tangent of x that no operator carries on raises, with gradients off too."""
+    n, tokens = 50, 0 if kind == "gt" else 1
+    torch.manual_seed(1)
+    model = (Graphormer if tokens else GT)(2, 8, 32, hidden, 5, 1, 0.0, 0.0, 0.0, hidden, tokens).to(cuda).requires_grad_(False)
+    x, plan = torch.randn(n, 32).to(cuda), GraphPlan(edges_of(n, tokens, 3).to(cuda), n + tokens)
+    for one in (True, False):
+        model.one_operator = one
+        with torch.autograd.forward_ad.dual_level(), torch.no_grad():
+            with pytest.raises(RuntimeError, match="jvp"):
+                model(torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)), None, plan, attn_type="sparse")
+        assert model(x, None, plan, attn_type="sparse").shape == (n, 5)

@@ -31,6 +31,16 @@ inline void on_gpu(const Tensor& t, const char* op) {
     TORCH_CHECK(t.is_cuda(), op, " needs GPU tensors (there is no CPU implementation)");
 }
 
+// Whether an operator has to go through its autograd node: somebody wants gradients, or a tangent comes with the tensor (forward mode is
+// refused there; passing the node by would drop the tangent without a word)
+struct Wanted {
+    bool gradients = false, tangents = false;
+    void look(const Tensor& t) {
+        gradients = gradients || t.requires_grad();
+        tangents = tangents || t._fw_grad(0).defined();
+    }
+    bool node() const { return tangents || (gradients && at::GradMode::is_enabled()); }
+};
 // what a kernel reads has to be on the GPU of its first operand: a host pointer or another GPU's is a fault there
 inline void same_gpu(const Tensor& t, const Tensor& first, const char* op, const char* name) {
     TORCH_CHECK(t.defined() && t.is_cuda() && t.device() == first.device(), op, ": ", name, " must be on the GPU ", first.device(), " like the other operands");

@@ -509,11 +509,12 @@ Tensor layered(const char* name, const Tensor& x, at::TensorList P, const c10::i
     TORCH_CHECK(x.dim() == 2 && x.is_contiguous(), name, ": x must be a contiguous [n, features]");
     const int64_t per = (int64_t)P.size() - M::kHead - M::kTail, L = per / 16;
     TORCH_CHECK(L >= 1 && per % 16 == 0 && (int64_t)eps.size() == 2 * L + (M::kTail == 4 ? 1 : 0), name, ": 16 parameters and two eps per layer");
-    bool train = x.requires_grad();
+    Wanted wanted;
+    wanted.look(x);
     for (const Tensor& t : P) {
         same_gpu(t, x, name, "every parameter");
         TORCH_CHECK(t.scalar_type() == x.scalar_type(), name, ": parameters must be GPU tensors of x's dtype");
-        train = train || t.requires_grad();
+        wanted.look(t);
     }
     same_gpu(ws, x, name, "the plan");
     const Dims D = dims_of<M>(x, P, H, tokens, L);
@@ -521,7 +522,7 @@ Tensor layered(const char* name, const Tensor& x, at::TensorList P, const c10::i
     TORCH_CHECK(classes >= 1 && classes <= D.Cp && D.W % H == 0, name, ": classes or heads");
     rows_match_plan(holder, D.N, name);
     std::vector<double> e(eps.begin(), eps.end());
-    if (train && at::GradMode::is_enabled()) return LayeredFn<M>::apply(x, P, holder, ws, H, tokens, classes, e);
+    if (wanted.node()) return LayeredFn<M>::apply(x, P, holder, ws, H, tokens, classes, e);
     c10::DeviceGuard guard(x.device());
     std::vector<Tensor> p;
     for (const Tensor& t : P) p.push_back(t.contiguous());

@@ -236,11 +236,11 @@ Tensor node_graphormer(const Tensor& x, at::TensorList P, const c10::intrusive_p
     GraphormerDims D{};
     D.L = (int64_t)(P.size() - 7) / 16; D.n = x.size(0); D.tokens = tokens; D.N = D.n + tokens; D.F = x.size(1); D.H = H;
     TORCH_CHECK((int64_t)eps.size() == 2 * D.L + 1, "node_graphormer: 2 L + 1 values of eps");
-    bool train = false;
+    Wanted wanted;
     for (const Tensor& t : P) {
         same_gpu(t, x, "node_graphormer", "every parameter");
         TORCH_CHECK(t.scalar_type() == x.scalar_type(), "parameters must be GPU tensors of x's dtype");
-        train = train || t.requires_grad();
+        wanted.look(t);
     }
     same_gpu(ws, x, "node_graphormer", "the plan");
     const Tensor* q = P.data() + 3;
@@ -256,9 +256,9 @@ Tensor node_graphormer(const Tensor& x, at::TensorList P, const c10::intrusive_p
                 "node_graphormer: 1 to 64 classes on 64 features");
     TORCH_CHECK(H == 8 || H == 4 || H == 2, "node_graphormer: 8, 4 or 2 heads");
     rows_match_plan(holder, D.N, "node_graphormer");
-    train = at::GradMode::is_enabled() && (train || x.requires_grad());
+    wanted.look(x);
     std::vector<double> e(eps.begin(), eps.end());
-    if (train) return NodeGraphormerFn::apply(x, P, holder, ws, D, e);
+    if (wanted.node()) return NodeGraphormerFn::apply(x, P, holder, ws, D, e);
     GraphormerState st;
     std::vector<Tensor> p;
     p.reserve(P.size());
@@ -507,11 +507,11 @@ Tensor graph_graphormer(const Tensor& x, const Tensor& in_degree, const Tensor& 
     const int64_t L = (int64_t)(P.size() - tables - 4) / 16;
     TORCH_CHECK((int64_t)eps.size() == 2 * L + 1 && (int64_t)seeds.size() == L, "graph_graphormer: 2 L + 1 values of eps, L seeds");
     TORCH_CHECK(H == 8 || H == 4 || H == 2, "graph_graphormer: 8, 4 or 2 heads");
-    bool train = false;
+    Wanted wanted;
     for (const Tensor& t : P) {
         same_gpu(t, attn_bias, "graph_graphormer", "every parameter");
         TORCH_CHECK(t.scalar_type() == P[0].scalar_type(), "graph_graphormer: parameters must be GPU tensors of one dtype");
-        train = train || t.requires_grad();
+        wanted.look(t);
     }
     same_gpu(x, attn_bias, "graph_graphormer", "x");
     same_gpu(in_degree, attn_bias, "graph_graphormer", "in_degree");
@@ -541,7 +541,7 @@ Tensor graph_graphormer(const Tensor& x, const Tensor& in_degree, const Tensor& 
     const auto ids = [](const Tensor& t) { return t.to(at::kLong).contiguous(); };
     c10::DeviceGuard guard(P[0].device());
     const Tensor ab = attn_bias.to(P[0].scalar_type()).contiguous();
-    if (at::GradMode::is_enabled() && train) return GraphGraphormerFn::apply(P, ids(x), ids(in_degree), ids(out_degree), ab, ids(spatial_pos), ids(edge_ids), c);
+    if (wanted.node()) return GraphGraphormerFn::apply(P, ids(x), ids(in_degree), ids(out_degree), ab, ids(spatial_pos), ids(edge_ids), c);
     std::vector<Tensor> p;
     for (const Tensor& t : P) p.push_back(t.contiguous());
     Tensor rows, lse, bias;
