@@ -181,3 +181,22 @@ def test_forward_mode_is_refused_not_dropped(cuda, kind, hidden):
             with pytest.raises(RuntimeError, match="jvp"):
                 model(torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)), None, plan, attn_type="sparse")
         assert model(x, None, plan, attn_type="sparse").shape == (n, 5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("hidden", [64, 128])
+def test_a_batch_without_nodes(cuda, dtype, hidden):
+    """No node, the global token alone: no rows come back, and every gradient is zero."""
+    torch.manual_seed(1)
+    model = Graphormer(2, 8, 32, hidden, 5, 1, 0.0, 0.0, 0.0, hidden, 1).to(cuda, dtype)
+    x, plan = torch.zeros(0, 32, device=cuda, dtype=dtype), GraphPlan(torch.zeros(2, 1, dtype=torch.long, device=cuda), 1)
+    for one in (True, False):
+        model.one_operator = one
+        model.zero_grad(set_to_none=True)
+        out = model(x, None, plan, attn_type="sparse")
+        assert out.shape == (0, 5)
+        out.float().sum().backward()
+        grads = [p.grad for p in model.parameters() if p.grad is not None]
+        assert len(grads) > 30 and not any(g.any() for g in grads)
+        with torch.no_grad():
+            assert model(x, None, plan, attn_type="sparse").shape == (0, 5)

@@ -187,7 +187,7 @@ class Graphormer(nn.Module):
         else None."""
         if not self.one_operator or self.num_global_node != 1 or attn_type != "sparse" or attn_bias is not None or perturb is not None or edge_index is None:
             return None
-        if x.dim() != 2 or not x.is_cuda or x.dtype not in _DT or autocast_to_float32(x):
+        if x.dim() != 2 or x.shape[0] == 0 or not x.is_cuda or x.dtype not in _DT or autocast_to_float32(x):
             return None
         found = model_parameters(self, x.dtype)
         return found if found is not None and self.layers[0].self_attention.num_heads == self.num_heads else None

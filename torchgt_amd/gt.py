@@ -121,7 +121,7 @@ class GT(nn.Module):
 
     def _one_operator(self, x, edge_index, attn_type):
         """(parameters, eps of the norms) in the operator's order when ``torch.ops.torchgt.node_gt`` covers this call, else None."""
-        if not self.one_operator or attn_type != "sparse" or edge_index is None or x.dim() != 2 or not x.is_cuda or x.dtype not in _DT or \
+        if not self.one_operator or attn_type != "sparse" or edge_index is None or x.dim() != 2 or x.shape[0] == 0 or not x.is_cuda or x.dtype not in _DT or \
                 autocast_to_float32(x) or getattr(self.MLP_layer, "L", None) != 2:
             return None
         found = model_parameters(self, x.dtype)
