@@ -136,7 +136,7 @@ def cpu_baseline(e, n, H, d, seconds_budget=30.0):
 def reference_ops_on_gpu(ei, q, k, v, bias, dout, steps=20):
     """The reference's formulation on this GPU: its chain of stock PyTorch-ROCm ops (gathers,
     elementwise ops, index_add_ scatter-adds, autograd backward; attn_module.py:146-187), fp32, same
-    inputs.  A datapoint beside the HIP path, not a checker: nothing is compared with it."""
+    inputs.  A datapoint beside the HIP path: nothing is compared with it."""
     import torch
     H, d = q.shape[1], q.shape[2]
     src, dst = ei[0], ei[1]

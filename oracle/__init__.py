@@ -2,7 +2,7 @@
 
 TEST INFRASTRUCTURE ONLY.  Nothing in the shipped package may import this
 directory: only ``tests/``, ``__graft_entry__.smoke()`` and the ``cpu_baseline``
-leg of ``bench.py`` use it, and there only as the checker (or as the CPU
+leg of ``bench.py`` use it, and there only to compare with (or as the CPU
 baseline being timed), never as the thing that produces a result.
 
 Every function restates, in plain PyTorch / numpy, the algorithm of a reference
