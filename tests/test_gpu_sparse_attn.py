@@ -127,6 +127,21 @@ def test_all_length_classes_and_ragged_rows(cuda):
     run_case("ragged-T", N, ei.flip(0).contiguous(), 8, 8, torch.float32, "edge", 12, cuda)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("bias_kind", ["none", "edge", "edge_head"])
+@pytest.mark.parametrize("H,d", [(8, 8), (8, 16), (1, 8)])
+def test_rows_that_end_at_and_beside_a_step(cuda, H, d, dtype, bias_kind):
+    # a long row's gathers are asked for one step (16, 32 or 256 edges, by the shape) ahead: rows that end with a step, one edge
+    # behind it and one short of it, and segments of longer ones, in both views
+    degs = [15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 95, 96, 97, 127, 128, 129, 255, 256, 257, 288, 511, 512, 513, 1056]
+    rng = np.random.default_rng(11)
+    N = 1200
+    hub = np.repeat(np.arange(len(degs)), degs)
+    leaf = np.concatenate([rng.permutation(N - len(degs))[:n] for n in degs]) + len(degs)
+    ei = torch.from_numpy(np.concatenate([np.stack([leaf, hub]), np.stack([hub, leaf])], axis=1)[:, rng.permutation(2 * len(hub))].copy())
+    run_case("steps", N, ei, H, d, dtype, bias_kind, 13, cuda)
+
+
 def test_large_scores_hit_the_clamp(cuda):
     N, E = 500, 5000
     ei = rand_graph(N, E, 21)

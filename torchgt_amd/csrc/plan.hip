@@ -371,7 +371,6 @@ __global__ __launch_bounds__(64 * kRecordWaves) void k_build_records(const Run* 
     int32_t* const recs = run.code & kRunBackward ? recs_bwd : recs_fwd;
     const int ipw = kind < (uint32_t)kNumClass ? rows_per_wave(lpe, (int)kind) : 1;
     const int S = kind < (uint32_t)kNumClass ? slots_for_class(lpe, (int)kind) : 1;
-    const bool inl = kind < (uint32_t)kNumClass && class_inline(lpe, (int)kind);
     const int groups = kWave / lpe, waves = run_waves(kind, run.n, lpe);
     for (int w = threadIdx.x >> 6; w < waves; w += kRecordWaves) {
         const int lw = run.wave0 + w;
@@ -399,7 +398,7 @@ __global__ __launch_bounds__(64 * kRecordWaves) void k_build_records(const Run* 
             out[L.off_start + t] = it.start;
             out[L.off_len + t] = it.len;
         }
-        if (inl) for (int k = t; k < 4 * groups; k += 64) {      // entry k: edge k % 4 of lane group k / 4
+        for (int k = t; k < 4 * groups; k += 64) {      // entry k: edge k % 4 of lane group k / 4
             const int g = k >> 2, i = g / S;
             Item it{0, 0, 0, -1};
             if (i < count) it = items[first + i];

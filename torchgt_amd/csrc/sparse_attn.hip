@@ -317,6 +317,80 @@ __device__ __forceinline__ void load_row(const Common& c, const int row, const i
 // but the backward 79 -> 88 us).
 template <typename T, int MODE> constexpr bool masked_gathers() { return sizeof(T) == 4 && MODE != MODE_FWD; }
 
+// What a lane holds of one edge between asking for it and using it: the gathered rows (unconverted), the bias, the destination's
+// (1 / (Z + eps), D).
+template <typename T>
+struct Gathered {
+    Raw8<T> g0, g1;
+    decltype(raw1((const T*)nullptr)) b;
+    float2 nd;
+};
+// Asks for everything of one edge: nb = the other endpoint, ed = the row of the bias array.
+template <typename T, int LPE, int LPH, int MODE, int HASB, typename O>
+__device__ __forceinline__ void ask_edge(const Common& c, const int nb, const int ed, const int el, Gathered<T>& g) {
+    constexpr int H = LPE / LPH;
+    constexpr int HD = LPE * 8;
+    const int head = el / LPH;
+    load_raw(at<T, O>(MODE == MODE_BWD_SRC ? c.q : c.k, nb, HD, el * 8), g.g0);
+    load_raw(at<T, O>(MODE == MODE_BWD_SRC ? c.g : c.v, nb, HD, el * 8), g.g1);
+    if (MODE == MODE_BWD_SRC) g.nd = *at<float2, O>(c.nd, nb, H, head);
+    if (HASB) {
+        const void* const bias = MODE == MODE_BWD_SRC ? c.bias_src : c.bias;
+        const int bias_shift = ilog2(sizeof(T)) + (c.bias_sh != 0 ? ilog2(H) : 0);      // log2 of the bytes of a bias row
+        const uint32_t bias_el = head * c.bias_sh * sizeof(T);
+        if (std::is_unsigned<O>::value) g.b = raw1(reinterpret_cast<const T*>(static_cast<const char*>(bias) + (((O)(uint32_t)ed << bias_shift) + bias_el)));
+        else g.b = raw1(at<T, O>(bias, ed, c.bias_se, head * c.bias_sh));
+    }
+}
+// Adds one edge to the sums of its slot.
+template <typename T, int LPE, int LPH, int MODE, int HASB>
+__device__ __forceinline__ void use_edge(const Common& c, const SideArgs& s, const RowRegs<T>& rr, const Gathered<T>& g, const int ed,
+                                         const int el, Acc& acc) {
+    constexpr int H = LPE / LPH;
+    const int head = el / LPH;
+    float x0[8], x1[8];
+    unpack(g.g0, x0);
+    unpack(g.g1, x1);
+    // raw score: identical arithmetic in all three walks so that the
+    // recomputed weights and the clamp mask agree bit for bit
+    const float raw = head_sum<LPH>(dot_raw(rr.r0, g.g0)) * c.inv_scale;
+    const float cl = clamp5(raw);
+    const float w = __expf(HASB ? cl + cvt1(g.b) : cl);
+    if (MODE == MODE_FWD) {
+        acc.z += w;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc.a0[i] = fmaf(w, x1[i], acc.a0[i]);
+    } else {
+        const bool inside = cl == raw;   // torch clamp backward: inclusive (and not for NaN)
+        if (MODE == MODE_BWD_DST) {
+            const float t = head_sum<LPH>(dot_raw(rr.r1, g.g1));   // g_dst . v_src
+            const float dS = w * rr.rz * (t - rr.Dh);
+            T* __restrict__ dB = static_cast<T*>(s.out1);
+            if (HASB && dB != nullptr) {
+                if (c.bias_sh != 0) {     // one value per edge and head
+                    if (el % LPH == 0) store1(dB + (int64_t)ed * H + head, dS);
+                } else {                  // one value per edge: sum over heads
+                    const float t2 = lanes_sum<1, LPE>(dS);   // every head is held by LPH lanes
+                    if (el == 0) store1(dB + ed, t2 * (1.0f / LPH));
+                }
+            }
+            const float md = inside ? dS : 0.f;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) acc.a0[i] = fmaf(md, x0[i], acc.a0[i]);
+        } else {
+            const float p = w * g.nd.x;
+            const float t = head_sum<LPH>(dot_raw(g.g1, rr.r1));   // g_dst . v_src
+            const float dS = p * (t - g.nd.y);
+            const float md = inside ? dS : 0.f;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                acc.a0[i] = fmaf(md, x0[i], acc.a0[i]);   // dk += m dS q_dst
+                acc.a1[i] = fmaf(p, x1[i], acc.a1[i]);    // dv += p g_dst
+            }
+        }
+    }
+}
+
 // kUnroll edges of one slot: nb[u] = the other endpoint, ed[u] = the row of the bias / dbias arrays, ok[u] =
 // whether the edge exists.  All gathers of the step are issued before anything is used.  Unless the gathers are
 // masked, every lane loads: a missing edge must then name a valid node and bias row - callers repeat the row's
@@ -325,98 +399,34 @@ template <typename T, int LPE, int LPH, int MODE, int HASB>
 __device__ __forceinline__ void edge_step(const Common& c, const SideArgs& s, const RowRegs<T>& rr,
                                           const int (&nb)[kUnroll], const int (&ed)[kUnroll],
                                           const bool (&ok)[kUnroll], const int el, Acc& acc) {
-    constexpr int H = LPE / LPH;
-    constexpr int HD = LPE * 8;
     constexpr bool MASKED = masked_gathers<T, MODE>();
-    const int head = el / LPH;
-    const float inv_scale = c.inv_scale;
-    const int bias_se = c.bias_se, bias_sh = c.bias_sh;
-    const int bias_shift = ilog2(sizeof(T)) + (bias_sh != 0 ? ilog2(H) : 0);      // log2 of the bytes of a bias row
-    const uint32_t bias_el = head * bias_sh * sizeof(T);
-    Raw8<T> g0[kUnroll], g1[kUnroll];          // gathered rows, unconverted
-    decltype(raw1((const T*)nullptr)) braw[kUnroll];
-    float2 ndv[kUnroll];
+    Gathered<T> g[kUnroll];
     if constexpr (MASKED) {
         // The edge ids are waited for here, on every path.  Otherwise the wait sits inside the first lane-masked
         // block below, and behind that block the compiler must assume the ids may still be in flight: it then
         // waits for everything outstanding - the first edge's rows - before it asks for the second edge's.
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) asm volatile("" ::"v"(nb[u]), "v"(ed[u]));
-    }
-    if (MASKED) {
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) {
-            braw[u] = 0;
-            ndv[u] = make_float2(0.f, 0.f);
-            zero_raw(g0[u]);
-            zero_raw(g1[u]);
+            g[u].b = 0;
+            g[u].nd = make_float2(0.f, 0.f);
+            zero_raw(g[u].g0);
+            zero_raw(g[u].g1);
         }
     }
     with_offsets<T>(c.narrow, [&](auto zero) {
-        using O = decltype(zero);
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-            if (!MASKED || ok[u]) {
-                load_raw(at<T, O>(MODE == MODE_BWD_SRC ? c.q : c.k, nb[u], HD, el * 8), g0[u]);
-                load_raw(at<T, O>(MODE == MODE_BWD_SRC ? c.g : c.v, nb[u], HD, el * 8), g1[u]);
-                if (MODE == MODE_BWD_SRC) ndv[u] = *at<float2, O>(c.nd, nb[u], H, head);
-                if (HASB) {
-                    const void* const bias = MODE == MODE_BWD_SRC ? c.bias_src : c.bias;
-                    if (std::is_unsigned<O>::value) braw[u] = raw1(reinterpret_cast<const T*>(static_cast<const char*>(bias) + (((O)(uint32_t)ed[u] << bias_shift) + bias_el)));
-                    else braw[u] = raw1(at<T, O>(bias, ed[u], bias_se, head * bias_sh));
-                }
-            }
-        }
+        for (int u = 0; u < kUnroll; ++u)
+            if (!MASKED || ok[u]) ask_edge<T, LPE, LPH, MODE, HASB, decltype(zero)>(c, nb[u], ed[u], el, g[u]);
     });
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
         // The edge's rows are named here, outside the lane-masked block that uses them: the compiler otherwise
         // moves their loads into that block (its only user), where they are asked for and waited for one edge
         // at a time instead of with the other gathers of the step.
-        if (!MASKED) { arrive_here(g0[u]); arrive_here(g1[u]); }
-        if (ok[u]) {
-            float x0[8], x1[8];
-            unpack(g0[u], x0);
-            unpack(g1[u], x1);
-            // raw score: identical arithmetic in all three walks so that the
-            // recomputed weights and the clamp mask agree bit for bit
-            const float raw = head_sum<LPH>(dot_raw(rr.r0, g0[u])) * inv_scale;
-            const float cl = clamp5(raw);
-            const float w = __expf(HASB ? cl + cvt1(braw[u]) : cl);
-            if (MODE == MODE_FWD) {
-                acc.z += w;
-#pragma unroll
-                for (int i = 0; i < 8; ++i) acc.a0[i] = fmaf(w, x1[i], acc.a0[i]);
-            } else {
-                const bool inside = cl == raw;   // torch clamp backward: inclusive (and not for NaN)
-                if (MODE == MODE_BWD_DST) {
-                    const float t = head_sum<LPH>(dot_raw(rr.r1, g1[u]));   // g_dst . v_src
-                    const float dS = w * rr.rz * (t - rr.Dh);
-                    T* __restrict__ dB = static_cast<T*>(s.out1);
-                    if (HASB && dB != nullptr) {
-                        if (bias_sh != 0) {       // one value per edge and head
-                            if (el % LPH == 0) store1(dB + (int64_t)ed[u] * H + head, dS);
-                        } else {                  // one value per edge: sum over heads
-                            const float t2 = lanes_sum<1, LPE>(dS);   // every head is held by LPH lanes
-                            if (el == 0) store1(dB + ed[u], t2 * (1.0f / LPH));
-                        }
-                    }
-                    const float md = inside ? dS : 0.f;
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) acc.a0[i] = fmaf(md, x0[i], acc.a0[i]);
-                } else {
-                    const float p = w * ndv[u].x;
-                    const float t = head_sum<LPH>(dot_raw(g1[u], rr.r1));   // g_dst . v_src
-                    const float dS = p * (t - ndv[u].y);
-                    const float md = inside ? dS : 0.f;
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        acc.a0[i] = fmaf(md, x0[i], acc.a0[i]);   // dk += m dS q_dst
-                        acc.a1[i] = fmaf(p, x1[i], acc.a1[i]);    // dv += p g_dst
-                    }
-                }
-            }
-        }
+        if (!MASKED) { arrive_here(g[u].g0); arrive_here(g[u].g1); }
+        if (ok[u]) use_edge<T, LPE, LPH, MODE, HASB>(c, s, rr, g[u], ed[u], el, acc);
     }
 }
 
@@ -528,68 +538,6 @@ __device__ __forceinline__ void finish_row(const Common& c, const SideArgs& s, c
     });
 }
 
-// Walks `len` edges starting at sorted position `start` of node `row` with S edge
-// slots (this lane is slot `slot`, element chunk `el`), reading the plan's sorted view.  On return
-// every lane holds the sums of its own slot (add_slots or reduce_slots adds the slots).
-template <typename T, int LPE, int LPH, int S, int MODE, int HASB>
-__device__ __forceinline__ void walk_range(const Common& c, const SideArgs& s, const int row, const int start,
-                                           const int len, const int slot, const int el, const bool valid,
-                                           Acc& acc) {
-    RowRegs<T> rr;
-    load_row<T, LPE, LPH, MODE>(c, row, el, valid, rr, acc);
-    const int32_t* __restrict__ col = s.col + start;
-    // HASB == 2: no edge-id array, the bias rows are in this side's own sorted order (row = sorted position)
-    constexpr bool ident = HASB == 2;
-    const int32_t* __restrict__ eid = ident ? nullptr : s.eid + start;
-    const int n = valid ? len : 0;
-    // endpoints and bias rows of the step that starts at edge e0 of the row
-    auto load_ids = [&](const int e0, int (&nb)[kUnroll], int (&ed)[kUnroll]) {
-#pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-            const int e = e0 + u * S;
-            if constexpr (masked_gathers<T, MODE>()) {
-                nb[u] = 0; ed[u] = 0;
-                if (e < n) {
-                    nb[u] = col[e];
-                    if (HASB) ed[u] = ident ? start + e : eid[e];
-                }
-            } else {   // lanes past the end of the row repeat its last edge (a line the wave is reading anyway)
-                const int ec = min(e, n - 1);
-                nb[u] = col[ec];
-                ed[u] = HASB ? (ident ? start + ec : eid[ec]) : 0;
-            }
-        }
-    };
-    if (n <= 0) return;
-    if constexpr (sizeof(T) == 4) {
-#pragma unroll 1
-        for (int e0 = slot; e0 < n; e0 += S * kUnroll) {
-            int nb[kUnroll], ed[kUnroll];
-            bool ok[kUnroll];
-#pragma unroll
-            for (int u = 0; u < kUnroll; ++u) ok[u] = e0 + u * S < n;
-            load_ids(e0, nb, ed);
-            edge_step<T, LPE, LPH, MODE, HASB>(c, s, rr, nb, ed, ok, el, acc);
-        }
-    } else {
-        // the ids of the next step are asked for before this step's gathers: a step waits for one memory
-        // round trip, not for two in a row (2-byte elements leave the registers for it)
-        int nb[kUnroll], ed[kUnroll];
-        load_ids(slot, nb, ed);
-#pragma unroll 1
-        for (int e0 = slot; e0 < n; e0 += S * kUnroll) {
-            int nb2[kUnroll], ed2[kUnroll];
-            bool ok[kUnroll];
-#pragma unroll
-            for (int u = 0; u < kUnroll; ++u) ok[u] = e0 + u * S < n;
-            load_ids(e0 + S * kUnroll, nb2, ed2);
-            edge_step<T, LPE, LPH, MODE, HASB>(c, s, rr, nb, ed, ok, el, acc);
-#pragma unroll
-            for (int u = 0; u < kUnroll; ++u) { nb[u] = nb2[u]; ed[u] = ed2[u]; }
-        }
-    }
-}
-
 // What one lane takes from its wave's record, asked for in one go when the kernel starts: none of the addresses
 // depends on the row class (the record lists row, start and length per lane group), so the wave has its rows and
 // its edges after one memory round trip, whatever the code then says they are.
@@ -619,6 +567,111 @@ __device__ __forceinline__ RecLane load_rec_lane(const WaveRec<LPE>& rec) {
     return r;
 }
 template <typename T, int MODE> constexpr bool rec_edges_early() { return sizeof(T) == 2 || MODE == MODE_FWD; }
+
+// Whether the walk of a long row keeps its queue of gathers filled (walk_range).  The float32 backward has no registers for it (128 with two
+// rows of its own and two gathered ones per edge) and its gathers are masked.
+template <typename T, int MODE> constexpr bool piped_walk() { return sizeof(T) == 2 || MODE == MODE_FWD; }
+
+// Walks `len` edges starting at sorted position `start` of node `row` with S edge
+// slots (this lane is slot `slot`, element chunk `el`), reading the plan's sorted view.  On return
+// every lane holds the sums of its own slot (add_slots or reduce_slots adds the slots).
+// FIRST: the edges of the first step came with the wave's record.
+template <typename T, int LPE, int LPH, int S, int MODE, int HASB, bool FIRST>
+__device__ __forceinline__ void walk_range(const Common& c, const SideArgs& s, const RecLane& rec, const int row, const int start,
+                                           const int len, const int slot, const int el, const bool valid,
+                                           Acc& acc) {
+    RowRegs<T> rr;
+    // HASB == 2: no edge-id array, the bias rows are in this side's own sorted order (row = sorted position)
+    constexpr bool ident = HASB == 2;
+    if constexpr (!piped_walk<T, MODE>()) {
+        load_row<T, LPE, LPH, MODE>(c, row, el, valid, rr, acc);
+        const int32_t* __restrict__ col = s.col + start;
+        const int32_t* __restrict__ eid = ident ? nullptr : s.eid + start;
+        const int n = valid ? len : 0;
+#pragma unroll 1
+        for (int e0 = slot; e0 < n; e0 += S * kUnroll) {
+            int nb[kUnroll], ed[kUnroll];
+            bool ok[kUnroll];
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u) {
+                const int e = e0 + u * S;
+                ok[u] = e < n;
+                nb[u] = 0; ed[u] = 0;
+                if (ok[u]) {
+                    nb[u] = col[e];
+                    if (HASB) ed[u] = ident ? start + e : eid[e];
+                }
+            }
+            edge_step<T, LPE, LPH, MODE, HASB>(c, s, rr, nb, ed, ok, el, acc);
+        }
+    } else {
+        // The edges of a slot are a queue of kUnroll: when one has been used its place is asked for again, with the edge one
+        // step on, so the wave's gathers never run dry between two steps; the edge ids are asked for a step before that, in front of
+        // the gathers (loads return in order: behind them, a wait for the ids would be one for all gathers).  The first step's ids
+        // come with the wave's record where there is one.  Bound by vector issue and this chain rather than by memory: 870 K nodes with 50
+        // edges each take 819 + 2292 us in bf16 when all neighbours are within 500 rows, 895 + 2490 us over 64 clusters.  Step by
+        // step / as a queue, forward + backward: 870 K nodes in 64 clusters 3386 / 3288 us, 200 K nodes, 8 M edges 717 / 683 us, 262 K
+        // nodes, 4.5 M edges, four heads of 16 438 / 419 us; rows of 5 edges have no second step: no difference.
+        constexpr bool ONE_ROW = LPE * S == kWave;      // one row per wave: its numbers are scalars
+        const int n = ONE_ROW ? __builtin_amdgcn_readfirstlane(valid ? len : 0) : (valid ? len : 0);
+        const int first = ONE_ROW ? __builtin_amdgcn_readfirstlane(start) : start;
+        const int32_t* __restrict__ col = s.col + first;
+        const int32_t* __restrict__ eid = HASB == 1 ? s.eid + first : nullptr;
+        const auto load_ids = [&](const int base, int (&nb)[kUnroll], int (&ed)[kUnroll]) {
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u) {      // past the end of the row: its last edge (a line the wave is reading anyway)
+                const uint32_t e = min(base + slot + u * S, n - 1);
+                nb[u] = col[e];
+                ed[u] = HASB ? (ident ? first + (int)e : eid[e]) : 0;
+            }
+        };
+        if (n <= 0) {
+            load_row<T, LPE, LPH, MODE>(c, row, el, valid, rr, acc);
+            return;
+        }
+        int nb[kUnroll], ed[kUnroll], nb2[kUnroll], ed2[kUnroll];
+        if constexpr (FIRST) {
+            nb[0] = rec.cols.x; nb[1] = rec.cols.y; nb[2] = rec.cols.z; nb[3] = rec.cols.w;
+            if (HASB == 1 && !s.eid_is_map) {
+                ed[0] = rec.eids.x; ed[1] = rec.eids.y; ed[2] = rec.eids.z; ed[3] = rec.eids.w;
+            } else {
+#pragma unroll
+                for (int u = 0; u < kUnroll; ++u) {
+                    const uint32_t e = min(slot + u * S, n - 1);
+                    ed[u] = HASB ? (ident ? first + (int)e : eid[e]) : 0;
+                }
+            }
+        } else load_ids(0, nb, ed);
+        load_ids(S * kUnroll, nb2, ed2);
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) asm volatile("" ::"v"(nb[u]), "v"(ed[u]));
+        load_row<T, LPE, LPH, MODE>(c, row, el, valid, rr, acc);
+        with_offsets<T>(c.narrow, [&](auto zero) {
+            using O = decltype(zero);
+            Gathered<T> g[kUnroll];
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u) ask_edge<T, LPE, LPH, MODE, HASB, O>(c, nb[u], ed[u], el, g[u]);
+            int base = 0;
+#pragma unroll 1
+            for (; base + S * kUnroll < n; base += S * kUnroll) {      // another step follows: every edge of this one exists
+                int nb3[kUnroll], ed3[kUnroll];
+                load_ids(base + 2 * S * kUnroll, nb3, ed3);
+#pragma unroll
+                for (int u = 0; u < kUnroll; ++u) {
+                    use_edge<T, LPE, LPH, MODE, HASB>(c, s, rr, g[u], ed[u], el, acc);
+                    __builtin_amdgcn_sched_barrier(0);      // (asked for earlier, the edge would need registers of its own)
+                    ask_edge<T, LPE, LPH, MODE, HASB, O>(c, nb2[u], ed2[u], el, g[u]);
+                    ed[u] = ed2[u]; nb2[u] = nb3[u]; ed2[u] = ed3[u];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u) {
+                arrive_here(g[u].g0); arrive_here(g[u].g1);      // (see edge_step)
+                if (base + slot + u * S < n) use_edge<T, LPE, LPH, MODE, HASB>(c, s, rr, g[u], ed[u], el, acc);
+            }
+        });
+    }
+}
 
 // The same for a row of at most S * kUnroll edges whose endpoints and bias rows come with the wave's
 // record (one step, no loop): the record lists them in lane order, four consecutive entries per
@@ -708,7 +761,7 @@ __device__ __forceinline__ void wave_rows(const Common& c, const SideArgs& s, co
     // (the row's own loads below) makes the compiler wait for everything outstanding behind that block - the
     // row's data - before the gathers may go out.
     asm volatile("" ::"v"(row), "v"(start), "v"(len));
-    if (INLINE && rec_edges_early<T, MODE>())
+    if ((INLINE && rec_edges_early<T, MODE>()) || (!INLINE && piped_walk<T, MODE>()))
         asm volatile("" ::"v"(rec.cols.x), "v"(rec.cols.y), "v"(rec.cols.z), "v"(rec.cols.w), "v"(rec.eids.x), "v"(rec.eids.y),
                      "v"(rec.eids.z), "v"(rec.eids.w));
     if (!valid) { row = 0; start = 0; len = 0; }
@@ -717,7 +770,7 @@ __device__ __forceinline__ void wave_rows(const Common& c, const SideArgs& s, co
     if (TILES) valid = valid && !(len == 0 && s.cover[row] != 0);
     Acc acc;
     if (INLINE) walk_record<T, LPE, LPH, S, MODE, HASB>(c, s, rec, row, start, len, slot, el, valid, acc);
-    else walk_range<T, LPE, LPH, S, MODE, HASB>(c, s, row, start, len, slot, el, valid, acc);
+    else walk_range<T, LPE, LPH, S, MODE, HASB, true>(c, s, rec, row, start, len, slot, el, valid, acc);
     finish_row<T, LPE, LPH, S, MODE, TILES>(c, s, row, slot, el, valid, acc);
 }
 
@@ -890,7 +943,7 @@ __device__ __forceinline__ void block_item(const Common& c, const SideArgs& s, c
     const int lo = min(grp * share, it.len);
     const int hi = min(lo + share, it.len);
     Acc acc;
-    walk_range<T, LPE, LPH, S, MODE, HASB>(c, s, it.row, it.start + lo, hi - lo, slot, el, true, acc);
+    walk_range<T, LPE, LPH, S, MODE, HASB, false>(c, s, RecLane{}, it.row, it.start + lo, hi - lo, slot, el, true, acc);
     add_slots<LPE, S, MODE>(acc);
     if (slot == 0) {
         float* r = lds.red + grp * STRIDE;
@@ -943,10 +996,17 @@ __device__ __forceinline__ void block_item(const Common& c, const SideArgs& s, c
     if (tid < LPE) write_row<T, LPE, LPH, MODE, TILES>(c, s, it.row, tid, acc);
 }
 
+// Waves per SIMD that the registers of the forward are kept down for: seven without a bias in bf16 rows of 32 and 64 elements, where that
+// costs nothing (72 registers, 76 without the bound, none in scratch; other shapes would spill); four in float32 (128 elements with
+// a bias take 130 registers unbounded: three waves, 38.9 us instead of 37.9 for 20 K nodes and 0.4 M edges)
+template <typename T, int LPE, int HASB, bool TILES> constexpr int fwd_waves() {
+    return sizeof(T) == 4 ? 4 : ((LPE == 4 || LPE == 8) && HASB == 0 && !TILES ? 7 : 1);
+}
+
 // Forward.  Workgroup b does what the records 4b .. 4b+3 say: one workgroup item, or four waves of
 // rows.  Which rows meet in which workgroup, on which XCD and when is the plan's business.
 template <typename T, int LPE, int LPH, int HASB, bool TILES>
-__global__ __launch_bounds__(kBlock) void k_attn_fwd(const Common c, const SideArgs s,
+__global__ __launch_bounds__(kBlock, (fwd_waves<T, LPE, HASB, TILES>())) void k_attn_fwd(const Common c, const SideArgs s,
                                                      const WaveRec<LPE>* __restrict__ recs) {
     __shared__ BlockLds<LPE> lds;
     const WaveRec<LPE>* r0 = recs + (int64_t)blockIdx.x * (kBlock / kWave);
