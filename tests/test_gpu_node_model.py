@@ -177,6 +177,42 @@ def test_gt_on_fused_layers(cuda, n, features, classes, heads, layers):
         assert off <= 1.1 * most + 2e-3, f"{name}: {off}, step by step {most}"
 
 
+@pytest.mark.parametrize("n,heads", [(15, 8), (16, 4), (17, 2), (64, 2), (65, 4), (16383, 8), (16384, 4), (32767, 2), (32768, 8), (40000, 4), (49152, 2), (49153, 8), (65535, 4), (65537, 2)])
+def test_rows_beside_the_lines_between_variants(cuda, n, heads):
+    """Sixteen or thirty-two rows per wave, 64 or 128 nodes per group (256 CUs: 16384, 32768, 49152 and 65536 rows), beside their edges"""
+    for dtype in (torch.float32, torch.bfloat16):
+        print(f"rows beside the lines: n={n} heads={heads} {dtype}", flush=True)
+        model = scaled(Graphormer(1, heads, 32, 64, 5, 1, 0.0, 0.0, 0.0, 64, 1), n, dtype, cuda)
+        x = torch.randn(n - 1, 32, generator=torch.Generator().manual_seed(n)).to(cuda, dtype)      # (one more row: the global token)
+        compare(Graphormer, model, x, GraphPlan(random_edges(n - 1, 1, n + 2, cuda), n), n + 3)
+    if n < 1000:
+        return test_gt_on_fused_layers(cuda, n, 32, 5, heads, 1)
+    # GT: among 128 n normal inputs of a ReLU those within rounding (1e-7) of 0 change their side between the two ways of summing, one for
+    # 40 K nodes and as many in the readout; each moves one of 128 (32) features of one node, 1 / sqrt(128 n) (1 / sqrt(32 n)) of a
+    # gradient's norm.  At 65 K nodes two of either kind, all in the same direction, are 0.5 / sqrt(n); the bar is 0.7 / sqrt(n), a
+    # single row gone wrong would be 1 / sqrt(n).  The output is continuous.
+    for dtype in (torch.float32, torch.bfloat16):
+        model = scaled(GT(1, heads, 32, 64, 5, 1, 0.0, 0.0, 0.0, 64, 0), n, dtype, cuda)
+        x, plan = torch.randn(n, 32, generator=torch.Generator().manual_seed(n)).to(cuda, dtype), GraphPlan(random_edges(n, 0, n + 2, cuda), n)
+        w = torch.randn(n, 5, generator=torch.Generator().manual_seed(n + 4)).to(cuda)
+        got = []
+        for fused in (True, False):
+            GT.one_operator = fused
+            try:
+                model.zero_grad(set_to_none=True)
+                xr = x.clone().requires_grad_(True)
+                out = model(xr, None, plan, attn_type="sparse")
+                (out.float() * w).sum().backward()
+                got.append([t.double() for t in [out.detach(), xr.grad] + [p.grad for p in model.parameters() if p.grad is not None]])
+            finally:
+                GT.one_operator = True
+        off = [float((a - b).norm() / b.norm().clamp(min=1e-30)) for a, b in zip(*got)]
+        names = ["output", "input gradient"] + [k for k, p in model.named_parameters() if p.grad is not None]
+        for name, o in zip(names, off):
+            if not name.endswith("linear_k.bias"):      # (rounding noise: it moves all scores of a query alike)
+                assert o <= (2e-2 if dtype == torch.bfloat16 else 1e-6 if name == "output" else (2 * n) ** -0.5), f"{name}: {o}"
+
+
 class NodeFwdArgs(ctypes.Structure):      # tgt_node_fwd_args
     _fields_ = [("rows", ctypes.c_int64)] + [(k, ctypes.c_int32) for k in ("dtype", "tokens", "classes", "linear", "same_bits")] + \
         [(k, ctypes.c_float) for k in ("eps_post", "eps_next")] + \

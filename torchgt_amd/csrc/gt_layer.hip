@@ -19,9 +19,9 @@ namespace {
 enum { V_BO = 0, V_GAMMA1, V_BETA1, V_B1A, V_B1B, V_B2, V_GAMMA2, V_BETA2, kVecs8 };
 enum { W_O = 0, W_1A, W_1B, W_2A, W_2B };
 
-template <typename T> __device__ __forceinline__ void round_to(Tile& t) { TGT_EACH(i) t.set(i, stored(t.get(i), (const T*)nullptr)); }
+template <typename T, int R> __device__ __forceinline__ void round_to(TileOf<R>& t) { TGT_EACH(i) t.set(i, stored(t.get(i), (const T*)nullptr)); }
 // relu(u), and (bit i) where u > 0
-template <typename T> __device__ __forceinline__ uint32_t relu(Tile& u) {
+template <typename T, int R> __device__ __forceinline__ uint32_t relu(TileOf<R>& u) {
     uint32_t on = 0;
     TGT_EACH(i) {
         const float v = stored(u.get(i), (const T*)nullptr);
@@ -31,89 +31,92 @@ template <typename T> __device__ __forceinline__ uint32_t relu(Tile& u) {
     return on;
 }
 
-constexpr int kFwdWaves = 8;
+// waves of a workgroup at most
+template <int R> constexpr int gt_fwd_waves() { return R == 32 ? 8 : 16; }
 // float32 takes its packed weights in turns (O and W1, W2, then q, k, v: 72 KB at most next to the row images), bf16 keeps all of them
 template <typename T> constexpr int gt_fwd_mats() { return sizeof(T) == 4 ? 3 : 8; }
-template <typename T> constexpr int gt_fwd_lds() { return gt_fwd_mats<T>() * kFragVecs<Num<T>::P> * 16 + (kVecs8 + 3) * kVec * 4 + kFwdWaves * RowShape<T>::kVecs * 16; }
+template <typename T, int R> constexpr int gt_fwd_lds(int waves) { return gt_fwd_mats<T>() * kFragVecs<Num<T>::P> * 16 + (kVecs8 + 3) * kVec * 4 + waves * RowShape<T, R>::kVecs * 16; }
 
-template <typename T, bool NEXT> __global__ __launch_bounds__(kFwdWaves * 64) void k_gt_fwd(const tgt_gt_fwd_args a) {
-    constexpr int P = Num<T>::P, THREADS = kFwdWaves * 64, FV = kFragVecs<P>;
+template <typename T, int R, bool NEXT> __global__ __launch_bounds__((gt_fwd_waves<R>() * 64)) void k_gt_fwd(const tgt_gt_fwd_args a) {
+    constexpr int P = Num<T>::P, FV = kFragVecs<P>;
+    constexpr bool CUT_AGAIN = P != 1 && R == 32;      // (no registers to keep a tile's planes)
+    const int threads = blockDim.x, kFwdWaves = threads >> 6;
     constexpr bool RESIDENT = sizeof(T) == 2;
     extern __shared__ __align__(16) unsigned char smem[];
     vec16* w = reinterpret_cast<vec16*>(smem);
     float* vec = reinterpret_cast<float*>(w + gt_fwd_mats<T>() * FV);
     float* vn = vec + kVecs8 * kVec;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    vec16* stage = reinterpret_cast<vec16*>(vn + 3 * kVec) + wave * RowShape<T>::kVecs;
+    vec16* stage = reinterpret_cast<vec16*>(vn + 3 * kVec) + wave * RowShape<T, R>::kVecs;
     const vec16 *gw = reinterpret_cast<const vec16*>(a.w), *gn = reinterpret_cast<const vec16*>(a.w_next);
-    const int64_t N = a.rows, tiles = (N + 31) / 32;
-    copy_vecs<kVecs8 * kVec / 4, THREADS>(reinterpret_cast<vec16*>(vec), reinterpret_cast<const vec16*>(a.vec));
-    if constexpr (NEXT) copy_vecs<3 * kVec / 4, THREADS>(reinterpret_cast<vec16*>(vn), reinterpret_cast<const vec16*>(a.v_next));
+    const int64_t N = a.rows, tiles = (N + R - 1) / R;
+    copy_params<kVecs8 * kVec>(threads, vec, a.vec);
+    if constexpr (NEXT) copy_params<3 * kVec>(threads, vn, a.v_next);
     if (RESIDENT) {
-        copy_vecs<5 * FV, THREADS>(w, gw);
-        if constexpr (NEXT) copy_vecs<3 * FV, THREADS>(w + 5 * FV, gn);
+        copy_vecs_by<5 * FV>(threads, w, gw);
+        if constexpr (NEXT) copy_vecs_by<3 * FV>(threads, w + 5 * FV, gn);
         __syncthreads();
     }
     const vec16 *w2 = RESIDENT ? w + 3 * FV : w, *wn = RESIDENT ? w + 5 * FV : w;
     for (int64_t t0 = (int64_t)blockIdx.x * kFwdWaves; t0 < tiles; t0 += (int64_t)gridDim.x * kFwdWaves) {
-        const Rows rows(t0 + wave, N);
+        const Rows rows(t0 + wave, N, R);
         const bool active = rows.left > 0;
-        Raw<T> raw_x, raw_a;
+        Raw<T, R> raw_x, raw_a;
         if (active) {
             fetch(raw_a, reinterpret_cast<const T*>(a.attn), rows, lane);
             fetch(raw_x, reinterpret_cast<const T*>(a.x), rows, lane);
         }
         if (!RESIDENT) {
             __syncthreads();
-            copy_vecs<3 * FV, THREADS>(w, gw);
+            copy_vecs_by<3 * FV>(threads, w, gw);
             __syncthreads();
         }
-        Tile s, r[2];
+        TileOf<R> s, r[2];
         if (active) {
-            Tile x, y;
+            TileOf<R> x, y;
             settle<T, false>(x, raw_a, stage, rows, lane);
             linear<P, false>(y, x, w, vec + V_BO * kVec, lane);
             round_to<T>(y);
             settle<T, false>(s, raw_x, stage, rows, lane);
             TGT_EACH(i) s.set(i, s.get(i) + y.get(i));
             normalise<false>(s, a.eps1);
-            affine(s, s, vec + V_GAMMA1 * kVec, vec + V_BETA1 * kVec, lane >> 5);
+            affine(s, s, vec + V_GAMMA1 * kVec, vec + V_BETA1 * kVec, lane / R);
             round_to<T>(s);      // x1
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                if (P != 1) forget(y);      // (its planes are formed again: there are no registers to keep them)
+                if (CUT_AGAIN) forget(y);
                 linear<P, false>(r[j], y, w + (W_1A + j) * FV, vec + (V_B1A + j) * kVec, lane);
                 relu<T>(r[j]);
             }
         }
         if (!RESIDENT) {
             __syncthreads();
-            copy_vecs<2 * FV, THREADS>(w, gw + W_2A * FV);
+            copy_vecs_by<2 * FV>(threads, w, gw + W_2A * FV);
             __syncthreads();
         }
         if (active) {
-            Tile y;
-            load_vec(y, vec + V_B2 * kVec, lane >> 5);
+            TileOf<R> y;
+            load_vec(y, vec + V_B2 * kVec, lane / R);
             gemm<P>(y, r[0], w2, lane);
             gemm<P>(y, r[1], w2 + FV, lane);
             TGT_EACH(i) s.set(i, s.get(i) + stored(y.get(i), (const T*)nullptr));
             if (a.s2) put_rows(reinterpret_cast<T*>(a.s2), s, stage, rows, lane);
             normalise<false>(s, a.eps2);
-            affine(s, s, vec + V_GAMMA2 * kVec, vec + V_BETA2 * kVec, lane >> 5);
+            affine(s, s, vec + V_GAMMA2 * kVec, vec + V_BETA2 * kVec, lane / R);
             round_to<T>(s);
             put_rows(reinterpret_cast<T*>(a.x_out), s, stage, rows, lane);
         }
         if constexpr (NEXT) {
             if (!RESIDENT) {
                 __syncthreads();
-                copy_vecs<3 * FV, THREADS>(w, gn);
+                copy_vecs_by<3 * FV>(threads, w, gn);
                 __syncthreads();
             }
             if (active) {
 #pragma unroll
                 for (int j = 0; j < 3; ++j) {
-                    Tile y;
-                    if (P != 1) forget(s);
+                    TileOf<R> y;
+                    if (CUT_AGAIN) forget(s);
                     linear<P, false>(y, s, wn + j * FV, vn + j * kVec, lane);
                     put_rows(reinterpret_cast<T*>(j == 0 ? a.q : (j == 1 ? a.k : a.v)), y, stage, rows, lane);
                 }
@@ -125,16 +128,17 @@ template <typename T, bool NEXT> __global__ __launch_bounds__(kFwdWaves * 64) vo
 // ---- backward -------------------------------------------------------------------------------------------------------------
 // Weights in the order the chain uses them: O, W1a, W2a^T, W1a^T, W1b, W2b^T, W1b^T, O^T.  Every step has two barriers: its weight
 // (and the planes of its weight gradient) are there; they have been used.
-template <typename T> __global__ __launch_bounds__(kBwdThreads) void k_gt_bwd(const tgt_gt_bwd_args a) {
-    using L = BwdLds<T, kVecs8>;
-    constexpr int P = Num<T>::P, FV = kFragVecs<P>;
+template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN, kVecs8>::kThreads)) void k_gt_bwd(const tgt_gt_bwd_args a) {
+    using L = Bwd<T, R, CN, kVecs8>;
+    constexpr int P = Num<T>::P, FV = kFragVecs<P>, PB = L::kPlane, NC = L::kChain;
+    constexpr bool CUT_AGAIN = P != 1;
     extern __shared__ __align__(16) unsigned char smem[];
-    unsigned char *p_dy = smem, *p_x = smem + P * kPlaneBytes;
+    unsigned char *p_dy = smem, *p_x = smem + P * PB;
     vec16* w = reinterpret_cast<vec16*>(smem + L::kW);
     float* vec = reinterpret_cast<float*>(smem + L::kVecs);
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 31, h = lane >> 5;
-    const int64_t N = a.rows, groups = (N + kChainNodes - 1) / kChainNodes;
-    copy_vecs<kVecs8 * kVec / 4, kBwdThreads>(reinterpret_cast<vec16*>(vec), reinterpret_cast<const vec16*>(a.vec));
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane % R, h = lane / R;
+    const int64_t N = a.rows, groups = (N + CN - 1) / CN;
+    copy_vecs<kVecs8 * kVec / 4, L::kThreads>(reinterpret_cast<vec16*>(vec), reinterpret_cast<const vec16*>(a.vec));
     __syncthreads();
     float16_t acc_a[3], acc_b[2];      // O, W1a, W1b; W2a, W2b
     float col_a[5], col_b[4];          // bo, b1a, b1b, gamma1, beta1; b2, -, gamma2, beta2
@@ -148,13 +152,13 @@ template <typename T> __global__ __launch_bounds__(kBwdThreads) void k_gt_bwd(co
     for (int j = 0; j < 5; ++j) col_a[j] = 0.f;
 #pragma unroll
     for (int j = 0; j < 4; ++j) col_b[j] = 0.f;
-    if (wave < 4) {
-        vec16* stage = reinterpret_cast<vec16*>(smem + L::kStage) + wave * RowShape<T>::kVecs;
-        const int row = 32 * wave + n;
+    if (wave < NC) {
+        vec16* stage = reinterpret_cast<vec16*>(smem + L::kStage) + wave * RowShape<T, R>::kVecs;
+        const int row = R * wave + n;
         for (int64_t g0 = blockIdx.x; g0 < groups; g0 += gridDim.x) {
-            const Rows rows(4 * g0 + wave, N);
-            Raw<T> raw;
-            Tile y, ds2, dy, t;
+            const Rows rows(NC * g0 + wave, N, R);
+            Raw<T, R> raw;
+            TileOf<R> y, ds2, dy, t;
             fetch(raw, reinterpret_cast<const T*>(a.attn), rows, lane);
             settle<T, false>(t, raw, stage, rows, lane);
             fetch(raw, reinterpret_cast<const T*>(a.s2), rows, lane);
@@ -163,7 +167,7 @@ template <typename T> __global__ __launch_bounds__(kBwdThreads) void k_gt_bwd(co
             round_to<T>(y);
             __syncthreads();
             {
-                Tile g;
+                TileOf<R> g;
                 settle<T, false>(t, raw, stage, rows, lane);
                 fetch(raw, reinterpret_cast<const T*>(a.g_in), rows, lane);
                 const float rstd = normalise<false>(t, a.eps2);
@@ -179,28 +183,26 @@ template <typename T> __global__ __launch_bounds__(kBwdThreads) void k_gt_bwd(co
             zero(dy);
 #pragma unroll
             for (int j = 0; j < 2; ++j) {      // the two halves of the feed-forward features
-                Frags<P> f;
-                if (P != 1) forget(y);      // (planes are formed again where they are used: there are no registers to keep them)
+                Frags<P, R> f;
+                if (CUT_AGAIN) forget(y);      // (planes are formed again where they are used: there are no registers to keep them)
                 __syncthreads();                                    // W1
                 linear<P, false>(t, y, w, vec + (V_B1A + j) * kVec, lane);
                 __syncthreads();
                 const uint32_t on = relu<T>(t);
-                make_frags(f, t);
-                put_planes<P>(p_x, row, h, f);
-                if (P != 1) forget(ds2);
+                put_tile_planes<PB, P>(p_x, row, h, t);
+                if (CUT_AGAIN) forget(ds2);
                 make_frags(f, ds2);
-                put_planes<P>(p_dy, row, h, f);
+                put_planes<PB>(p_dy, row, h, f);
                 __syncthreads();                                    // W2^T; planes of W2
                 zero(t);
                 gemm<P>(t, f, w, lane);
                 TGT_EACH(i) t.set(i, on & (1u << i) ? stored(t.get(i), (const T*)nullptr) : 0.f);      // du
                 col_a[1 + j] += column_sums(t, lane);
-                if (P != 1) forget(y);
+                if (CUT_AGAIN) forget(y);
                 __syncthreads();
-                make_frags(f, y);
-                put_planes<P>(p_x, row, h, f);
+                put_tile_planes<PB, P>(p_x, row, h, y);
                 make_frags(f, t);
-                put_planes<P>(p_dy, row, h, f);
+                put_planes<PB>(p_dy, row, h, f);
                 __syncthreads();                                    // W1^T; planes of W1
                 gemm<P>(dy, f, w, lane);
                 __syncthreads();
@@ -221,20 +223,19 @@ template <typename T> __global__ __launch_bounds__(kBwdThreads) void k_gt_bwd(co
             TGT_EACH(i) dy.set(i, stored(stored(dy.get(i), (const T*)nullptr) + y.get(i), (const T*)nullptr));
             col_a[0] += column_sums(dy, lane);
             settle<T, false>(t, raw, stage, rows, lane);
-            Frags<P> f;
-            make_frags(f, t);
-            put_planes<P>(p_x, row, h, f);
+            Frags<P, R> f;
+            put_tile_planes<PB, P>(p_x, row, h, t);
             make_frags(f, dy);
-            put_planes<P>(p_dy, row, h, f);
+            put_planes<PB>(p_dy, row, h, f);
             __syncthreads();                                        // O^T; planes of O
             zero(dy);
             gemm<P>(dy, f, w, lane);
             __syncthreads();
             put_rows(reinterpret_cast<T*>(a.d_attn), dy, stage, rows, lane);
-            if (n < rows.left) put_node_side<T>(dy, t, a.Z, a.nd, a.heads, rows.first + n, h);
+            put_node_side<T>(dy, t, a.Z, a.nd, a.heads, rows.first + n, h, n < rows.left);
         }
     } else {
-        const int q = wave - 4, base_dy = operand_base(q >> 1, lane), base_x = operand_base(q & 1, lane);
+        const int q = wave - NC, base_dy = operand_base(q >> 1, lane), base_x = operand_base(q & 1, lane);
         const vec16 *fw = reinterpret_cast<const vec16*>(a.w), *bw = reinterpret_cast<const vec16*>(a.w_back);
         WeightsAhead<FV> next;
         next.fetch(fw + W_O * FV);
@@ -246,29 +247,35 @@ template <typename T> __global__ __launch_bounds__(kBwdThreads) void k_gt_bwd(co
                 next.hand_over(w, bw + (W_2A + j) * FV);      // W1
                 __syncthreads();
                 next.hand_over(w, bw + (W_1A + j) * FV);      // W2^T
-                node_product<P>(acc_b[j], p_dy, p_x, base_dy, base_x);
+                node_product<P, PB>(acc_b[j], p_dy, p_x, base_dy, base_x);
                 __syncthreads();
                 next.hand_over(w, j == 0 ? fw + W_1B * FV : bw + W_O * FV);      // W1^T
-                node_product<P>(acc_a[1 + j], p_dy, p_x, base_dy, base_x);
+                node_product<P, PB>(acc_a[1 + j], p_dy, p_x, base_dy, base_x);
                 __syncthreads();
             }
             next.hand_over(w, fw + W_O * FV);           // O^T
-            node_product<P>(acc_a[0], p_dy, p_x, base_dy, base_x);
+            node_product<P, PB>(acc_a[0], p_dy, p_x, base_dy, base_x);
             __syncthreads();
         }
     }
     float* buf = reinterpret_cast<float*>(smem);
-    write_partial<3, 5>(a.partial_a + (int64_t)blockIdx.x * (3 * 4096 + 5 * 64), acc_a, col_a, buf, wave, lane);
-    write_partial<2, 4>(a.partial_b + (int64_t)blockIdx.x * (2 * 4096 + 4 * 64), acc_b, col_b, buf, wave, lane);
+    write_partial<L, 3, 5>(a.partial_a + (int64_t)blockIdx.x * (3 * 4096 + 5 * 64), acc_a, col_a, buf, wave, lane);
+    write_partial<L, 2, 4>(a.partial_b + (int64_t)blockIdx.x * (2 * 4096 + 4 * 64), acc_b, col_b, buf, wave, lane);
 }
 
-template <typename T, bool NEXT> int run_fwd(const tgt_gt_fwd_args& a, hipStream_t st) {
+template <typename T, int R, bool NEXT> int run_fwd(const tgt_gt_fwd_args& a, hipStream_t st) {
     static std::atomic<uint64_t> done{0};
-    return launch(&k_gt_fwd<T, NEXT>, done, grid_for(a.rows, kFwdWaves), kFwdWaves * 64, gt_fwd_lds<T>(), st, a);
+    constexpr int most = gt_fwd_waves<R>();
+    const int waves = fwd_waves_for(a.rows, R, most);
+    if (int rc = allow_lds(reinterpret_cast<const void*>(&k_gt_fwd<T, R, NEXT>), gt_fwd_lds<T, R>(most), done)) return rc;
+    hipLaunchKernelGGL((k_gt_fwd<T, R, NEXT>), dim3(fwd_grid(a.rows, R, waves)), dim3(waves * 64), (gt_fwd_lds<T, R>(waves)), st, a);
+    TGT_HIP_CHECK(hipGetLastError());
+    return TGT_OK;
 }
-template <typename T> int run_bwd(const tgt_gt_bwd_args& a, hipStream_t st) {
+template <typename T, int R, int CN> int run_bwd(const tgt_gt_bwd_args& a, hipStream_t st) {
+    using L = Bwd<T, R, CN, kVecs8>;
     static std::atomic<uint64_t> done{0};
-    return launch(&k_gt_bwd<T>, done, grid_for(a.rows, 4), kBwdThreads, BwdLds<T, kVecs8>::kBytes, st, a);
+    return launch(&k_gt_bwd<T, R, CN>, done, bwd_workers(a.rows), L::kThreads, L::kBytes, st, a);
 }
 bool dtype_ok(int dtype) { return dtype == TGT_DTYPE_F32 || dtype == TGT_DTYPE_BF16; }
 
@@ -284,8 +291,11 @@ int tgt_gt_fwd(const tgt_gt_fwd_args* a, void* stream) {
     if (a->rows == 0) return TGT_OK;
     const hipStream_t st = (hipStream_t)stream;
     KernelTimer t(KS_GT_FWD, st);
-    if (a->dtype == TGT_DTYPE_F32) return a->q ? run_fwd<float, true>(*a, st) : run_fwd<float, false>(*a, st);
-    return a->q ? run_fwd<nbf16, true>(*a, st) : run_fwd<nbf16, false>(*a, st);
+    // rows per wave: 16 in float32 (us with 16 / 32: 4 K nodes 20.5 / 31.1, 64 K 42.7 / 47.1, 200 K 147 / 152), in bf16 while the CUs are
+    // less than three quarters full in one round (4 K 10.7 / 12.2, 37605 14.4 / 14.7, 64 K 17.0 / 16.1, 200 K 43.9 / 43.9)
+    if (a->dtype == TGT_DTYPE_F32) return a->q ? run_fwd<float, 16, true>(*a, st) : run_fwd<float, 16, false>(*a, st);
+    if (4 * a->rows <= 3 * one_round()) return a->q ? run_fwd<nbf16, 16, true>(*a, st) : run_fwd<nbf16, 16, false>(*a, st);
+    return a->q ? run_fwd<nbf16, 32, true>(*a, st) : run_fwd<nbf16, 32, false>(*a, st);
 }
 
 int tgt_gt_bwd(const tgt_gt_bwd_args* a, void* stream) {
@@ -296,7 +306,11 @@ int tgt_gt_bwd(const tgt_gt_bwd_args* a, void* stream) {
     if (!a->nd || !a->Z || (a->heads != 8 && a->heads != 4 && a->heads != 2)) return bad("tgt_gt_bwd", "nd, Z and 8, 4 or 2 heads");
     const hipStream_t st = (hipStream_t)stream;
     KernelTimer t(KS_GT_BWD, st);
-    return a->dtype == TGT_DTYPE_F32 ? run_bwd<float>(*a, st) : run_bwd<nbf16>(*a, st);
+    // (node_roles.h; eight chain waves of sixteen rows and the blocks' accumulators of five weights do not fit the registers in float32: 64 nodes
+    // per group as soon as that leaves the number of workgroups alone - 64 K nodes 77 us, 200 K 222, with 128 nodes and 32 rows per
+    // wave 80 and 232 -, those in between)
+    if (a->dtype == TGT_DTYPE_F32) return groups_of_64(a->rows, true) || a->rows >= (int64_t)128 * num_cus() ? run_bwd<float, 16, 64>(*a, st) : run_bwd<float, 32, 128>(*a, st);
+    return groups_of_64(a->rows, false) ? run_bwd<nbf16, 16, 64>(*a, st) : run_bwd<nbf16, 16, 128>(*a, st);
 }
 
 }  // extern "C"

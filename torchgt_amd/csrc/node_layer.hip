@@ -47,8 +47,8 @@ template <typename T> __global__ __launch_bounds__(512) void k_node_pack(const P
     const int j = b >> 1, back = b & 1;
     const T* W = reinterpret_cast<const T*>(a.mat[j]);
     const int ld = a.ld[j], rows = a.rows[j];
-    const int lane = threadIdx.x & 63, sm = threadIdx.x >> 6, s = sm >> 1, m = sm & 1;
-    const int r = lane & 31, out_f = 32 * ((r >> 2) & 1) + 16 * m + 4 * (r >> 3) + (r & 3), in0 = 32 * (lane >> 5) + 8 * s;
+    const int lane = threadIdx.x & 63, sm = threadIdx.x >> 6, s = sm >> 2, m = sm & 3;
+    const int out_f = 16 * gray2((lane >> 2) & 3) + 4 * m + (lane & 3), in0 = 16 * (lane >> 4) + 8 * s;
     float v[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -75,7 +75,7 @@ template <typename T, bool SAME> __device__ __forceinline__ float cdf_and_bell(f
     } else normal_cdf(v, cdf, bell);
     return cdf;
 }
-template <typename T, bool SAME> __device__ __forceinline__ void gelu(Tile& u) {
+template <typename T, bool SAME, int R> __device__ __forceinline__ void gelu(TileOf<R>& u) {
     TGT_EACH(i) {
         const float v = stored(u.get(i), (const T*)nullptr);
         float bell;
@@ -84,7 +84,7 @@ template <typename T, bool SAME> __device__ __forceinline__ void gelu(Tile& u) {
         if (i % 8 == 7) fence_schedule();
     }
 }
-template <typename T, bool SAME> __device__ __forceinline__ void gelu(Tile& u, Tile& slope) {
+template <typename T, bool SAME, int R> __device__ __forceinline__ void gelu(TileOf<R>& u, TileOf<R>& slope) {
     TGT_EACH(i) {
         const float v = stored(u.get(i), (const T*)nullptr);
         float bell;
@@ -98,20 +98,21 @@ template <typename T, bool SAME> __device__ __forceinline__ void gelu(Tile& u, T
 // ---- forward ------------------------------------------------------------------------------------------------------------
 enum { NEXT_NONE = 0, NEXT_QKV = 1, NEXT_CLASSES = 2 };
 
-template <typename T, bool SAME> constexpr int fwd_waves() { return sizeof(T) == 4 || SAME ? 8 : 16; }
+// waves of a workgroup at most
+template <typename T, int R, bool SAME> constexpr int fwd_waves() { return R == 32 && (sizeof(T) == 4 || SAME) ? 8 : 16; }
 // bf16 keeps all weights of a launch in LDS for the life of the workgroup; float32 planes of six weights (144 KB) do not
 // leave room for the row images, so its two halves take turns (the L2 has them)
 template <typename T, bool POST, int NEXT> constexpr int fwd_resident_mats() {
     const int post = POST ? 3 : 0, next = NEXT == NEXT_QKV ? 3 : (NEXT == NEXT_CLASSES ? 1 : 0);
     return sizeof(T) == 4 ? (post > next ? post : next) : post + next;
 }
-template <typename T, bool SAME, bool POST, int NEXT> constexpr int fwd_lds() {
-    return fwd_resident_mats<T, POST, NEXT>() * kFragVecs<Num<T>::P> * 16 + 10 * kVec * 4 + fwd_waves<T, SAME>() * RowShape<T>::kVecs * 16;
+template <typename T, int R, bool POST, int NEXT> constexpr int fwd_lds(int waves) {
+    return fwd_resident_mats<T, POST, NEXT>() * kFragVecs<Num<T>::P> * 16 + 10 * kVec * 4 + waves * RowShape<T, R>::kVecs * 16;
 }
 
-// Rows of class values.  A wave's 32 rows are 32 C consecutive elements of the [N - tokens, C] array and travel through its
+// Rows of class values.  A wave's R rows are R C consecutive elements of the [N - tokens, C] array and travel through its
 // row image, in words: for bf16 the image starts one element late where the rows begin in the middle of a word.
-template <typename T> struct ClassRows {
+template <typename T, int R> struct ClassRows {
     static constexpr int kPerWord = 4 / (int)sizeof(T);
     T* img;
     int C, lo, hi;            // elements of the wave's rows that exist: [lo, hi)
@@ -121,8 +122,8 @@ template <typename T> struct ClassRows {
         C = classes;
         const int64_t r = row0 - tokens, left = N - row0;
         first = r * C; total = (N - tokens) * C;
-        lo = r < 0 ? (int)(-r < 32 ? -r : 32) * C : 0;
-        hi = (int)(left < 0 ? 0 : (left < 32 ? left : 32)) * C;
+        lo = r < 0 ? (int)(-r < R ? -r : R) * C : 0;
+        hi = (int)(left < 0 ? 0 : (left < R ? left : R)) * C;
         shift = kPerWord == 2 ? (int)(first & 1) : 0;
         img = reinterpret_cast<T*>(stage) + shift;
     }
@@ -132,9 +133,8 @@ template <typename T> struct ClassRows {
         const int n = words();
         const int64_t w0 = (first - shift) / kPerWord, last = total / kPerWord - 1;
         const uint32_t* p = reinterpret_cast<const uint32_t*>(src);
-        uint32_t v[32];
-#pragma unroll
-        for (int i = 0; i < 32; ++i)
+        uint32_t v[R];
+        TGT_EACH(i)
             if (i * 64 < n && last >= 0) {
                 int64_t w = w0 + i * 64 + lane;
                 w = w < 0 ? 0 : (w > last ? last : w);
@@ -142,8 +142,7 @@ template <typename T> struct ClassRows {
             }
         wave_sync();
         uint32_t* d = reinterpret_cast<uint32_t*>(img - shift);
-#pragma unroll
-        for (int i = 0; i < 32; ++i)
+        TGT_EACH(i)
             if (i * 64 < n && last >= 0 && i * 64 + lane < n) d[i * 64 + lane] = v[i];
         wave_sync();
         if (kPerWord == 2 && (total & 1) && first + hi == total && hi > lo && lane == 0) img[hi - 1] = src[total - 1];      // half a word at the end
@@ -168,46 +167,48 @@ template <typename T> __device__ __forceinline__ T to_elem(float v);
 template <> __device__ __forceinline__ float to_elem<float>(float v) { return v; }
 template <> __device__ __forceinline__ nbf16 to_elem<nbf16>(float v) { return nbf16{__builtin_bit_cast(uint16_t, static_cast<__bf16>(v))}; }
 
-template <typename T, bool SAME, bool POST, int NEXT>
-__global__ __launch_bounds__((fwd_waves<T, SAME>() * 64)) void k_node_fwd(const tgt_node_fwd_args a) {
-    constexpr int P = Num<T>::P, NW = fwd_waves<T, SAME>(), THREADS = NW * 64, FV = kFragVecs<P>;
+template <typename T, int R, bool SAME, bool POST, int NEXT>
+__global__ __launch_bounds__((fwd_waves<T, R, SAME>() * 64)) void k_node_fwd(const tgt_node_fwd_args a) {
+    constexpr int P = Num<T>::P, FV = kFragVecs<P>;
     constexpr bool RESIDENT = sizeof(T) == 2;
     constexpr int NMP = NEXT == NEXT_QKV ? 3 : (NEXT == NEXT_CLASSES ? 1 : 0);
+    using Shape = RowShape<T, R>;
     extern __shared__ __align__(16) unsigned char smem[];
     vec16* w = reinterpret_cast<vec16*>(smem);
     vec16* w_next = w + (RESIDENT && POST ? 3 * FV : 0);
     float* vec = reinterpret_cast<float*>(w + fwd_resident_mats<T, POST, NEXT>() * FV);
     float* vn = vec + 5 * kVec;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5;
-    vec16* stage = reinterpret_cast<vec16*>(vec + 10 * kVec) + wave * RowShape<T>::kVecs;
-    const int64_t N = a.rows, tiles = (N + 31) / 32;
-    if constexpr (POST) copy_vecs<5 * kVec / 4, THREADS>(reinterpret_cast<vec16*>(vec), reinterpret_cast<const vec16*>(a.v_post));
-    if constexpr (NEXT != NEXT_NONE) copy_vecs<(2 + NMP) * kVec / 4, THREADS>(reinterpret_cast<vec16*>(vn), reinterpret_cast<const vec16*>(a.v_next));
+    const int threads = blockDim.x, NW = threads >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane / R;
+    vec16* stage = reinterpret_cast<vec16*>(vec + 10 * kVec) + wave * Shape::kVecs;
+    const int64_t N = a.rows, tiles = (N + R - 1) / R;
+    if constexpr (POST) copy_params<5 * kVec>(threads, vec, a.v_post);
+    if constexpr (NEXT != NEXT_NONE) copy_params<(2 + NMP) * kVec>(threads, vn, a.v_next);
     if (RESIDENT) {
-        if constexpr (POST) copy_vecs<3 * FV, THREADS>(w, reinterpret_cast<const vec16*>(a.w_post));
-        if constexpr (NEXT != NEXT_NONE) copy_vecs<NMP * FV, THREADS>(w_next, reinterpret_cast<const vec16*>(a.w_next));
+        if constexpr (POST) copy_vecs_by<3 * FV>(threads, w, reinterpret_cast<const vec16*>(a.w_post));
+        if constexpr (NEXT != NEXT_NONE) copy_vecs_by<NMP * FV>(threads, w_next, reinterpret_cast<const vec16*>(a.w_next));
         __syncthreads();
     }
     for (int64_t t0 = (int64_t)blockIdx.x * NW; t0 < tiles; t0 += (int64_t)gridDim.x * NW) {
-        const Rows rows(t0 + wave, N);
-        const int64_t row0 = (t0 + wave) * 32;
+        const Rows rows(t0 + wave, N, R);
+        const int64_t row0 = (t0 + wave) * R;
         const bool active = rows.left > 0;
-        Raw<T> raw_a, raw_s;
+        Raw<T, R> raw_a, raw_s;
         if (active) {
             fetch(raw_s, reinterpret_cast<const T*>(a.s_in), rows, lane);
             if (POST) fetch(raw_a, reinterpret_cast<const T*>(a.attn), rows, lane);
         }
         if (!RESIDENT && POST) {
             __syncthreads();
-            copy_vecs<3 * FV, THREADS>(w, reinterpret_cast<const vec16*>(a.w_post));
+            copy_vecs_by<3 * FV>(threads, w, reinterpret_cast<const vec16*>(a.w_post));
             __syncthreads();
         }
-        Tile s;
+        TileOf<R> s;
         if (active) {
             if (!POST && row0 < a.tokens) {      // the global tokens in front of the nodes: from their table, and into the stream
-                constexpr int PP = RowShape<T>::kPieces, PER = RowShape<T>::kPer;
+                constexpr int PP = Shape::kPieces, PER = Shape::kPer;
 #pragma unroll
-                for (int i = 0; i < RowShape<T>::kAcc; ++i) {
+                for (int i = 0; i < Shape::kAcc; ++i) {
                     const int64_t r = row0 + i * PER + lane / PP;
                     if (r < a.tokens) {
                         raw_s.v[i] = reinterpret_cast<const vec16*>(a.token)[r * PP + lane % PP];
@@ -217,13 +218,13 @@ __global__ __launch_bounds__((fwd_waves<T, SAME>() * 64)) void k_node_fwd(const 
             }
             settle<T, false>(s, raw_s, stage, rows, lane);
             if (POST) {
-                Tile x, y;
+                TileOf<R> x, y;
                 settle<T, false>(x, raw_a, stage, rows, lane);
                 linear<P, SAME>(y, x, w, vec, lane);
                 TGT_EACH(i) s.set(i, s.get(i) + stored(y.get(i), (const T*)nullptr));      // s1 = s + (a Wo^T + bo)
                 x = s;
                 normalise<SAME>(x, a.eps_post);
-                affine(x, x, vec + kVec, vec + 2 * kVec, h);      // y2
+                affine(x, x, vec + kVec, vec + 2 * kVec, g);      // y2
                 linear<P, SAME>(y, x, w + FV, vec + 3 * kVec, lane);    // u
                 gelu<T, SAME>(y);
                 linear<P, SAME>(x, y, w + 2 * FV, vec + 4 * kVec, lane);
@@ -233,21 +234,26 @@ __global__ __launch_bounds__((fwd_waves<T, SAME>() * 64)) void k_node_fwd(const 
         }
         if constexpr (!RESIDENT && NEXT != NEXT_NONE) {
             __syncthreads();
-            copy_vecs<NMP * FV, THREADS>(w, reinterpret_cast<const vec16*>(a.w_next));
+            copy_vecs_by<NMP * FV>(threads, w, reinterpret_cast<const vec16*>(a.w_next));
             __syncthreads();
         }
         if (NEXT && active) {
             normalise<SAME>(s, a.eps_next);
-            affine(s, s, vn, vn + kVec, h);
-            if (NEXT == NEXT_QKV) {
+            affine(s, s, vn, vn + kVec, g);
+            if constexpr (NEXT == NEXT_QKV) {
+                // float32: sixteen rows' planes fit beside a product, thirty-two rows' are cut again for each of the three
+                using Operand = std::conditional_t<R == 16, Frags<P, R>, TileOf<R>>;
+                Operand f;
+                if constexpr (R == 16) make_frags(f, s);
+                else f = s;
 #pragma unroll
                 for (int j = 0; j < 3; ++j) {
-                    Tile y;
-                    linear<P, SAME>(y, s, w_next + j * FV, vn + (2 + j) * kVec, lane);
+                    TileOf<R> y;
+                    linear<P, SAME>(y, f, w_next + j * FV, vn + (2 + j) * kVec, lane);
                     put_rows(reinterpret_cast<T*>(j == 0 ? a.q : (j == 1 ? a.k : a.v)), y, stage, rows, lane);
                 }
             } else {
-                Tile y;
+                TileOf<R> y;
                 linear<P, SAME>(y, s, w_next, vn + 2 * kVec, lane);
                 const int C = a.classes;
                 float lse = 0.f;
@@ -255,15 +261,16 @@ __global__ __launch_bounds__((fwd_waves<T, SAME>() * 64)) void k_node_fwd(const 
                     float top = -INFINITY, sum = 0.f;
                     TGT_EACH(i) {      // rounded first: log_softmax reads the logits as a T tensor would hold them
                         y.set(i, stored(y.get(i), (const T*)nullptr));
-                        if (32 * h + i < C) top = fmaxf(top, y.get(i));
+                        if (R * g + i < C) top = fmaxf(top, y.get(i));
                     }
-                    top = fmaxf(top, __shfl_xor(top, 32, 64));
-                    TGT_EACH(i) if (32 * h + i < C) sum += expf(y.get(i) - top);
-                    lse = top + logf(both_halves(sum));
+#pragma unroll
+                    for (int off = R; off < 64; off <<= 1) top = fmaxf(top, __shfl_xor(top, off, 64));
+                    TGT_EACH(i) if (R * g + i < C) sum += expf(y.get(i) - top);
+                    lse = top + logf(node_sum<R>(sum));
                 }
-                const ClassRows<T> out(stage, row0, N, a.tokens, C);
+                const ClassRows<T, R> out(stage, row0, N, a.tokens, C);
                 wave_sync();
-                TGT_EACH(i) if (32 * h + i < C) out.img[(lane & 31) * C + 32 * h + i] = to_elem<T>(y.get(i) - lse);
+                TGT_EACH(i) if (R * g + i < C) out.img[(lane % R) * C + R * g + i] = to_elem<T>(y.get(i) - lse);
                 wave_sync();
                 out.store(reinterpret_cast<T*>(a.logp), lane);
             }
@@ -271,38 +278,38 @@ __global__ __launch_bounds__((fwd_waves<T, SAME>() * 64)) void k_node_fwd(const 
     }
 }
 
-// Class gradients of a wave's 32 rows: d logits = d logp - softmax * sum(d logp) (linear: d logits as they come); zero for tokens and past the end.
-template <typename T> __device__ __forceinline__ void class_grads(Tile& d, const T* __restrict__ dlogp, const T* __restrict__ logp, bool linear, int C, int tokens, int64_t row0, int64_t N,
-                                                                  vec16* stage, int lane) {
-    const int n = lane & 31, h = lane >> 5;
-    ClassRows<T> rows(stage, row0, N, tokens, C);
+// Class gradients of a wave's R rows: d logits = d logp - softmax * sum(d logp) (linear: d logits as they come); zero for tokens and past the end.
+template <typename T, int R> __device__ __forceinline__ void class_grads(TileOf<R>& d, const T* __restrict__ dlogp, const T* __restrict__ logp, bool linear, int C, int tokens, int64_t row0, int64_t N,
+                                                                         vec16* stage, int lane) {
+    const int n = lane % R, g = lane / R;
+    ClassRows<T, R> rows(stage, row0, N, tokens, C);
     const bool in = n * C >= rows.lo && n * C < rows.hi;
-    const T* mine = rows.img + (in ? n * C + 32 * h : 0);
+    const T* mine = rows.img + (in ? n * C + R * g : 0);
     rows.load(dlogp, lane);
     float sum = 0.f;
     TGT_EACH(i) {
-        d.set(i, in && 32 * h + i < C ? as_float(mine[i]) : 0.f);
+        d.set(i, in && R * g + i < C ? as_float(mine[i]) : 0.f);
         sum += d.get(i);
     }
     if (linear) return;
-    sum = both_halves(sum);
+    sum = node_sum<R>(sum);
     rows.load(logp, lane);
-    TGT_EACH(i) if (in && 32 * h + i < C) d.set(i, d.get(i) - expf(as_float(mine[i])) * sum);
+    TGT_EACH(i) if (in && R * g + i < C) d.set(i, d.get(i) - expf(as_float(mine[i])) * sum);
 }
 
 // ---- backward of the part in front of an attention (or of the classes) ------------------------------------------------------
 // NORM false (GT): q, k, v are made of the rows s themselves.
-template <typename T, bool CLASSES, bool NORM>
-__global__ __launch_bounds__(kBwdThreads) void k_node_bwd_pre(const tgt_node_bwd_pre_args a) {
-    using L = BwdLds<T>;
-    constexpr int P = Num<T>::P, FV = kFragVecs<P>, NM = CLASSES ? 1 : 3;
+template <typename T, int R, int CN, bool CLASSES, bool NORM>
+__global__ __launch_bounds__((Bwd<T, R, CN>::kThreads)) void k_node_bwd_pre(const tgt_node_bwd_pre_args a) {
+    using L = Bwd<T, R, CN>;
+    constexpr int P = Num<T>::P, FV = kFragVecs<P>, NM = CLASSES ? 1 : 3, PB = L::kPlane, NC = L::kChain;
     extern __shared__ __align__(16) unsigned char smem[];
-    unsigned char *p_dy = smem, *p_x = smem + P * kPlaneBytes;
+    unsigned char *p_dy = smem, *p_x = smem + P * PB;
     vec16* w = reinterpret_cast<vec16*>(smem + L::kW);
     float* vec = reinterpret_cast<float*>(smem + L::kVecs);
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5;
-    const int64_t N = a.rows, groups = (N + kChainNodes - 1) / kChainNodes;
-    if constexpr (NORM) copy_vecs<2 * kVec / 4, kBwdThreads>(reinterpret_cast<vec16*>(vec), reinterpret_cast<const vec16*>(a.v_next));
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane / R;
+    const int64_t N = a.rows, groups = (N + CN - 1) / CN;
+    if constexpr (NORM) copy_vecs<2 * kVec / 4, L::kThreads>(reinterpret_cast<vec16*>(vec), reinterpret_cast<const vec16*>(a.v_next));
     __syncthreads();
     float16_t acc[NM];
     float col[NM + 2];
@@ -312,27 +319,27 @@ __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_pre(const tgt_node_bwd
         for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
 #pragma unroll
     for (int j = 0; j < NM + 2; ++j) col[j] = 0.f;
-    if (wave < 4) {
-        vec16* stage = reinterpret_cast<vec16*>(smem + L::kStage) + wave * RowShape<T>::kVecs;
+    if (wave < NC) {
+        vec16* stage = reinterpret_cast<vec16*>(smem + L::kStage) + wave * RowShape<T, R>::kVecs;
         const T* src[3] = {reinterpret_cast<const T*>(a.dq), reinterpret_cast<const T*>(a.dk), reinterpret_cast<const T*>(a.dv)};
-        const int row = 32 * wave + (lane & 31);
-        Raw<T> raw_s, raw_d;
+        const int row = R * wave + lane % R;
+        Raw<T, R> raw_s, raw_d;
         {
-            const Rows rows(4 * (int64_t)blockIdx.x + wave, N);
+            const Rows rows(NC * (int64_t)blockIdx.x + wave, N, R);
             fetch(raw_s, reinterpret_cast<const T*>(a.s), rows, lane);
             if (!CLASSES) fetch(raw_d, src[0], rows, lane);
         }
         for (int64_t g0 = blockIdx.x; g0 < groups; g0 += gridDim.x) {
-            const Rows rows(4 * g0 + wave, N);
-            Tile xhat, dy, d;
-            Frags<P> f;
+            const Rows rows(NC * g0 + wave, N, R);
+            TileOf<R> xhat, dy, d;
+            Frags<P, R> f;
             settle<T, false>(xhat, raw_s, stage, rows, lane);
             float rstd = 1.f;
             if constexpr (NORM) rstd = normalise<false>(xhat, a.eps);
             zero(dy);
 #pragma unroll
             for (int j = 0; j < NM; ++j) {
-                if (CLASSES) class_grads(d, reinterpret_cast<const T*>(a.dlogp), reinterpret_cast<const T*>(a.logp), a.linear, a.classes, a.tokens, (4 * g0 + wave) * 32, N, stage, lane);
+                if (CLASSES) class_grads(d, reinterpret_cast<const T*>(a.dlogp), reinterpret_cast<const T*>(a.logp), a.linear, a.classes, a.tokens, (NC * g0 + wave) * R, N, stage, lane);
                 else {
                     settle<T, true>(d, raw_d, stage, rows, lane);
                     fetch(raw_d, j + 1 < NM ? src[j + 1] : reinterpret_cast<const T*>(a.g_in), rows, lane);
@@ -343,17 +350,15 @@ __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_pre(const tgt_node_bwd
                 gemm<P>(dy, f, w, lane);               // beside product j - 1 of the block waves
                 if (j > 0) __syncthreads();            // product j - 1 is done
                 else {
-                    Tile y;
+                    TileOf<R> y;
                     if constexpr (NORM) affine(y, xhat, vec, vec + kVec, h);
                     else y = xhat;
-                    Frags<P> fx;
-                    make_frags(fx, y);
-                    put_planes<P>(p_x, row, h, fx);
+                    put_tile_planes<PB, P>(p_x, row, h, y);
                 }
-                put_planes<P>(p_dy, row, h, f);
+                put_planes<PB>(p_dy, row, h, f);
                 __syncthreads();                       // planes j are there, weight j has been used
             }
-            if (g0 + gridDim.x < groups) fetch(raw_s, reinterpret_cast<const T*>(a.s), Rows(4 * (g0 + gridDim.x) + wave, N), lane);
+            if (g0 + gridDim.x < groups) fetch(raw_s, reinterpret_cast<const T*>(a.s), Rows(NC * (g0 + gridDim.x) + wave, N, R), lane);
             TGT_EACH(i) dy.set(i, stored(dy.get(i), (const T*)nullptr));
             if constexpr (NORM) {
                 col[NM + 1] += column_sums(dy, lane);
@@ -363,15 +368,15 @@ __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_pre(const tgt_node_bwd
             if (CLASSES) zero(d);
             else {
                 settle<T, true>(d, raw_d, stage, rows, lane);
-                if (g0 + gridDim.x < groups) fetch(raw_d, src[0], Rows(4 * (g0 + gridDim.x) + wave, N), lane);
+                if (g0 + gridDim.x < groups) fetch(raw_d, src[0], Rows(NC * (g0 + gridDim.x) + wave, N, R), lane);
             }
             if constexpr (NORM) ln_back(d, dy, xhat, rstd, vec, h);
             else TGT_EACH(i) d.set(i, d.get(i) + dy.get(i));
             put_rows(reinterpret_cast<T*>(a.g_out), d, stage, rows, lane);
-            if (a.d_token && 4 * g0 + wave < (a.tokens + 31) / 32) put_rows(reinterpret_cast<T*>(a.d_token), d, stage, Rows(4 * g0 + wave, a.tokens), lane);
+            if (a.d_token && NC * g0 + wave < (a.tokens + R - 1) / R) put_rows(reinterpret_cast<T*>(a.d_token), d, stage, Rows(NC * g0 + wave, a.tokens, R), lane);
         }
     } else {
-        const int q = wave - 4, base_dy = operand_base(q >> 1, lane), base_x = operand_base(q & 1, lane);
+        const int q = wave - NC, base_dy = operand_base(q >> 1, lane), base_x = operand_base(q & 1, lane);
         const vec16* weights = reinterpret_cast<const vec16*>(a.w_back);
         WeightsAhead<FV> next;
         next.fetch(weights);
@@ -387,26 +392,27 @@ __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_pre(const tgt_node_bwd
                     next.fetch(weights + (j + 2 < NM ? j + 2 : 0) * FV);
                     __syncthreads();                   // weight j + 1
                 }
-                node_product<P>(acc[j], p_dy, p_x, base_dy, base_x);
+                node_product<P, PB>(acc[j], p_dy, p_x, base_dy, base_x);
                 if (j + 1 < NM) __syncthreads();       // product j is done
             }
         }
     }
-    write_partial<NM, NM + 2>(a.partial + (int64_t)blockIdx.x * (NM * 4096 + (NM + 2) * 64), acc, col, reinterpret_cast<float*>(smem), wave, lane);
+    write_partial<L, NM, NM + 2>(a.partial + (int64_t)blockIdx.x * (NM * 4096 + (NM + 2) * 64), acc, col, reinterpret_cast<float*>(smem), wave, lane);
 }
 
 // ---- backward of the part behind an attention -------------------------------------------------------------------------------
-template <typename T, bool SAME>
-__global__ __launch_bounds__(kBwdThreads) void k_node_bwd_post(const tgt_node_bwd_post_args a) {
-    using L = BwdLds<T>;
-    constexpr int P = Num<T>::P, FV = kFragVecs<P>;
+template <typename T, int R, int CN, bool SAME>
+__global__ __launch_bounds__((Bwd<T, R, CN>::kThreads)) void k_node_bwd_post(const tgt_node_bwd_post_args a) {
+    using L = Bwd<T, R, CN>;
+    constexpr int P = Num<T>::P, FV = kFragVecs<P>, PB = L::kPlane, NC = L::kChain;
+    constexpr bool KEEP = P == 1 || CN == 64;      // whether there are registers for the planes of LayerNorm's output
     extern __shared__ __align__(16) unsigned char smem[];
-    unsigned char *p_dy = smem, *p_x = smem + P * kPlaneBytes;
+    unsigned char *p_dy = smem, *p_x = smem + P * PB;
     vec16* w = reinterpret_cast<vec16*>(smem + L::kW);
     float* vec = reinterpret_cast<float*>(smem + L::kVecs);
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 31, h = lane >> 5;
-    const int64_t N = a.rows, groups = (N + kChainNodes - 1) / kChainNodes;
-    copy_vecs<5 * kVec / 4, kBwdThreads>(reinterpret_cast<vec16*>(vec), reinterpret_cast<const vec16*>(a.v_post));
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane % R, h = lane / R;
+    const int64_t N = a.rows, groups = (N + CN - 1) / CN;
+    copy_vecs<5 * kVec / 4, L::kThreads>(reinterpret_cast<vec16*>(vec), reinterpret_cast<const vec16*>(a.v_post));
     __syncthreads();
     float16_t acc[3];       // Wo, W1, W2
     float col[5];           // bo, b1, b2, gamma, beta
@@ -416,27 +422,27 @@ __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_post(const tgt_node_bw
         for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
 #pragma unroll
     for (int j = 0; j < 5; ++j) col[j] = 0.f;
-    if (wave < 4) {
-        vec16* stage = reinterpret_cast<vec16*>(smem + L::kStage) + wave * RowShape<T>::kVecs;
-        const int row = 32 * wave + n;
-        Raw<T> raw_a, raw_s, raw_g;
+    if (wave < NC) {
+        vec16* stage = reinterpret_cast<vec16*>(smem + L::kStage) + wave * RowShape<T, R>::kVecs;
+        const int row = R * wave + n;
+        Raw<T, R> raw_a, raw_s, raw_g;
         {
-            const Rows rows(4 * (int64_t)blockIdx.x + wave, N);
+            const Rows rows(NC * (int64_t)blockIdx.x + wave, N, R);
             fetch(raw_a, reinterpret_cast<const T*>(a.attn), rows, lane);
             fetch(raw_s, reinterpret_cast<const T*>(a.s), rows, lane);
             fetch(raw_g, reinterpret_cast<const T*>(a.g_in), rows, lane);
         }
         for (int64_t g0 = blockIdx.x; g0 < groups; g0 += gridDim.x) {
-            const Rows rows(4 * g0 + wave, N);
+            const Rows rows(NC * g0 + wave, N, R);
             const auto fetch_next = [&]() {
                 if (g0 + gridDim.x >= groups) return;
-                const Rows ahead(4 * (g0 + gridDim.x) + wave, N);
+                const Rows ahead(NC * (g0 + gridDim.x) + wave, N, R);
                 fetch(raw_a, reinterpret_cast<const T*>(a.attn), ahead, lane);
                 fetch(raw_s, reinterpret_cast<const T*>(a.s), ahead, lane);
                 fetch(raw_g, reinterpret_cast<const T*>(a.g_in), ahead, lane);
             };
-            Tile g, xhat, slope, t;
-            Frags<P> f, fy;      // fy: LayerNorm's output, kept in its one plane for bf16, formed again from xhat for float32
+            TileOf<R> g, xhat, slope, t;
+            Frags<P, R> f, fy;      // fy: LayerNorm's output, formed again from xhat where it is not kept
             settle<T, false>(t, raw_a, stage, rows, lane);
             make_frags(f, t);
             settle<T, false>(xhat, raw_s, stage, rows, lane);
@@ -458,24 +464,23 @@ __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_post(const tgt_node_bw
             linear<P, SAME>(t, fy, w, vec + 3 * kVec, lane);           // u
             __syncthreads();                                        // W1 has been used
             gelu<T, SAME>(t, slope);
-            make_frags(f, t);
-            put_planes<P>(p_x, row, h, f);
+            put_tile_planes<PB, P>(p_x, row, h, t);
             make_frags(f, g);
-            put_planes<P>(p_dy, row, h, f);
+            put_planes<PB>(p_dy, row, h, f);
             __syncthreads();                                        // planes of W2; W2^T
             zero(t);
             gemm<P>(t, f, w, lane);                                 // d gelu, beside product W2
             TGT_EACH(i) t.set(i, stored(t.get(i) * slope.get(i), (const T*)nullptr));      // du
             col[1] += column_sums(t, lane);
             make_frags(f, t);
-            if (P != 1) {
+            if (!KEEP) {
                 forget(xhat);
                 affine(t, xhat, vec + kVec, vec + 2 * kVec, h);
             }
             __syncthreads();                                        // product W2 is done, W2^T has been used
-            put_planes<P>(p_dy, row, h, f);
-            if (P != 1) make_frags(fy, t);
-            put_planes<P>(p_x, row, h, fy);
+            put_planes<PB>(p_dy, row, h, f);
+            if constexpr (KEEP) put_planes<PB>(p_x, row, h, fy);
+            else put_tile_planes<PB, P>(p_x, row, h, t);
             __syncthreads();                                        // planes of W1; W1^T
             fetch(raw_a, reinterpret_cast<const T*>(a.attn), rows, lane);
             zero(t);
@@ -491,23 +496,19 @@ __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_post(const tgt_node_bw
             make_frags(f, g);
             settle<T, false>(t, raw_a, stage, rows, lane);
             __syncthreads();                                        // product W1 is done, W1^T has been used
-            put_planes<P>(p_dy, row, h, f);
-            {
-                Frags<P> fx;
-                make_frags(fx, t);
-                put_planes<P>(p_x, row, h, fx);
-            }
+            put_planes<PB>(p_dy, row, h, f);
+            put_tile_planes<PB, P>(p_x, row, h, t);
             __syncthreads();                                        // planes of Wo; Wo^T
             if (P == 1) fetch_next();      // float32 has the registers only after the products
             zero(g);
             gemm<P>(g, f, w, lane);                                 // da, beside product Wo
             __syncthreads();                                        // Wo^T has been used
             put_rows(reinterpret_cast<T*>(a.d_attn), g, stage, rows, lane);
-            if (a.nd && n < rows.left) put_node_side<T>(g, t, a.Z, a.nd, a.heads, rows.first + n, h);
+            if (a.nd) put_node_side<T>(g, t, a.Z, a.nd, a.heads, rows.first + n, h, n < rows.left);
             if (P != 1) fetch_next();
         }
     } else {
-        const int q = wave - 4, base_dy = operand_base(q >> 1, lane), base_x = operand_base(q & 1, lane);
+        const int q = wave - NC, base_dy = operand_base(q >> 1, lane), base_x = operand_base(q & 1, lane);
         const vec16 *fw = reinterpret_cast<const vec16*>(a.w_post), *bw = reinterpret_cast<const vec16*>(a.w_back);
         WeightsAhead<FV> next;
         next.fetch(fw);
@@ -517,17 +518,17 @@ __global__ __launch_bounds__(kBwdThreads) void k_node_bwd_post(const tgt_node_bw
             next.hand_over(w, bw + 2 * FV);         // W1
             __syncthreads();
             next.hand_over(w, bw + FV);             // W2^T and the planes of W2
-            node_product<P>(acc[2], p_dy, p_x, base_dy, base_x);
+            node_product<P, PB>(acc[2], p_dy, p_x, base_dy, base_x);
             __syncthreads();
             next.hand_over(w, bw);                  // W1^T and the planes of W1
-            node_product<P>(acc[1], p_dy, p_x, base_dy, base_x);
+            node_product<P, PB>(acc[1], p_dy, p_x, base_dy, base_x);
             __syncthreads();
             next.hand_over(w, fw);                  // Wo^T and the planes of Wo
-            node_product<P>(acc[0], p_dy, p_x, base_dy, base_x);
+            node_product<P, PB>(acc[0], p_dy, p_x, base_dy, base_x);
             __syncthreads();
         }
     }
-    write_partial<3, 5>(a.partial + (int64_t)blockIdx.x * (3 * 4096 + 5 * 64), acc, col, reinterpret_cast<float*>(smem), wave, lane);
+    write_partial<L, 3, 5>(a.partial + (int64_t)blockIdx.x * (3 * 4096 + 5 * 64), acc, col, reinterpret_cast<float*>(smem), wave, lane);
 }
 
 // ---- sums of the partials -----------------------------------------------------------------------------------------------
@@ -541,30 +542,39 @@ struct SumArgs {
 __device__ __forceinline__ void put_elem(float* p, float v) { *p = v; }
 __device__ __forceinline__ void put_elem(nbf16* p, float v) { p->x = __builtin_bit_cast(uint16_t, static_cast<__bf16>(v)); }
 
-// 64 consecutive elements x 16 slices of the workers per workgroup: slices in worker order, then the slice sums in order
-template <typename T> __global__ __launch_bounds__(1024) void k_node_sums(const SumArgs a) {
-    __shared__ float part[16][64];
-    const int d = blockIdx.y, n = a.n[d];
-    if ((int)blockIdx.x * 64 >= n) return;
-    const int el = threadIdx.x & 63, sl = threadIdx.x >> 6, e = blockIdx.x * 64 + el;
-    const int w0 = a.workers[d] * sl / 16, w1 = a.workers[d] * (sl + 1) / 16;
-    const float* __restrict__ src = a.partial[d] + e;
-    float s = 0.f;
-    int w = w0;
-    for (; w + 8 <= w1; w += 8) {
-        float t[8];
+// 64 consecutive elements x 16 slices of the workers per workgroup: slices in worker order, then the slice sums in order.  Bound by
+// its reads, 50 KB of partials from every worker of every launch of a backward (108 MB for four Graphormer layers): sixteen lanes of a
+// wave take 16 bytes each of a slice's 64 elements, eight workers in flight.  A lane per element and a wave per slice / this / 256 elements
+// and a wave per slice, us with 64, 250 and 256 workers of four layers: 14.2 / 8.9 / 8.9, 24.3 / 19.8 / 20.0, 27.2 / 26.3 / 25.9 (GT: 34 / 34 / 39).
+constexpr int kSumElems = 64;
+template <int W> __device__ __forceinline__ void add_workers(float4& s, const float* __restrict__ src, int64_t n) {
+    float4 t[W];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) t[i] = src[(int64_t)(w + i) * n];
+    for (int i = 0; i < W; ++i) t[i] = *reinterpret_cast<const float4*>(src + i * n);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) s += t[i];
+    for (int i = 0; i < W; ++i) { s.x += t[i].x; s.y += t[i].y; s.z += t[i].z; s.w += t[i].w; }
+}
+template <typename T> __global__ __launch_bounds__(256) void k_node_sums(const SumArgs a) {
+    __shared__ float part[16][kSumElems];
+    const int d = blockIdx.y, n = a.n[d], e0 = blockIdx.x * kSumElems;      // (n is a multiple of 64)
+    if (e0 >= n) return;
+    {
+        const int sl = threadIdx.x >> 4, el = 4 * (threadIdx.x & 15);
+        const int w0 = a.workers[d] * sl / 16, w1 = a.workers[d] * (sl + 1) / 16;
+        const float* __restrict__ src = a.partial[d] + e0 + el;
+        float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+        int w = w0;
+        for (; w + 8 <= w1; w += 8) add_workers<8>(s, src + (int64_t)w * n, n);
+        for (; w + 2 <= w1; w += 2) add_workers<2>(s, src + (int64_t)w * n, n);
+        if (w < w1) add_workers<1>(s, src + (int64_t)w * n, n);
+        *reinterpret_cast<float4*>(&part[sl][el]) = s;
     }
-    for (; w < w1; ++w) s += src[(int64_t)w * n];
-    part[sl][el] = s;
     __syncthreads();
-    if (sl == 0) {
+    if (threadIdx.x < kSumElems) {
+        const int e = e0 + threadIdx.x;
         float t = 0.f;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) t += part[i][el];
+        for (int i = 0; i < 16; ++i) t += part[i][threadIdx.x];
         const int mats = a.mats[d], rows = a.rows[d];
         const int seg = e < mats * 4096 ? e >> 12 : mats + ((e - mats * 4096) >> 6), at = e < mats * 4096 ? e & 4095 : (e - mats * 4096) & 63;
         const int limit = seg < mats ? rows * 64 : (seg < 2 * mats ? rows : 64);
@@ -572,23 +582,32 @@ template <typename T> __global__ __launch_bounds__(1024) void k_node_sums(const 
     }
 }
 
-template <typename T, bool SAME, bool POST, int NEXT> int launch_fwd(const tgt_node_fwd_args& a, hipStream_t st) {
+template <typename T, int R, bool SAME, bool POST, int NEXT> int launch_fwd(const tgt_node_fwd_args& a, hipStream_t st) {
     static std::atomic<uint64_t> done{0};
-    return launch(&k_node_fwd<T, SAME, POST, NEXT>, done, grid_for(a.rows, fwd_waves<T, SAME>()), fwd_waves<T, SAME>() * 64, fwd_lds<T, SAME, POST, NEXT>(), st, a);
+    constexpr int most = fwd_waves<T, R, SAME>();
+    const int waves = fwd_waves_for(a.rows, R, most);
+    if (int rc = allow_lds(reinterpret_cast<const void*>(&k_node_fwd<T, R, SAME, POST, NEXT>), fwd_lds<T, R, POST, NEXT>(most), done)) return rc;
+    hipLaunchKernelGGL((k_node_fwd<T, R, SAME, POST, NEXT>), dim3(fwd_grid(a.rows, R, waves)), dim3(waves * 64), (fwd_lds<T, R, POST, NEXT>(waves)), st, a);
+    TGT_HIP_CHECK(hipGetLastError());
+    return TGT_OK;
 }
-template <typename T, bool SAME> int dispatch_fwd(const tgt_node_fwd_args& a, hipStream_t st) {
-    if (a.attn) return a.logp ? launch_fwd<T, SAME, true, NEXT_CLASSES>(a, st) : (a.q ? launch_fwd<T, SAME, true, NEXT_QKV>(a, st) : launch_fwd<T, SAME, true, NEXT_NONE>(a, st));
-    return launch_fwd<T, SAME, false, NEXT_QKV>(a, st);
+template <typename T, int R, bool SAME> int dispatch_fwd(const tgt_node_fwd_args& a, hipStream_t st) {
+    if (a.attn) return a.logp ? launch_fwd<T, R, SAME, true, NEXT_CLASSES>(a, st) : (a.q ? launch_fwd<T, R, SAME, true, NEXT_QKV>(a, st) : launch_fwd<T, R, SAME, true, NEXT_NONE>(a, st));
+    return launch_fwd<T, R, SAME, false, NEXT_QKV>(a, st);
 }
-template <typename T> int dispatch_bwd_pre(const tgt_node_bwd_pre_args& a, int workers, hipStream_t st) {
-    static std::atomic<uint64_t> done[3];
-    if (a.dlogp) return launch(&k_node_bwd_pre<T, true, true>, done[1], workers, kBwdThreads, BwdLds<T>::kBytes, st, a);
-    return a.v_next ? launch(&k_node_bwd_pre<T, false, true>, done[0], workers, kBwdThreads, BwdLds<T>::kBytes, st, a)
-                    : launch(&k_node_bwd_pre<T, false, false>, done[2], workers, kBwdThreads, BwdLds<T>::kBytes, st, a);
-}
-template <typename T, bool SAME> int dispatch_bwd_post(const tgt_node_bwd_post_args& a, int workers, hipStream_t st) {
+template <typename T, int R, int CN, bool CLASSES, bool NORM> int launch_bwd_pre(const tgt_node_bwd_pre_args& a, hipStream_t st) {
+    using L = Bwd<T, R, CN>;
     static std::atomic<uint64_t> done{0};
-    return launch(&k_node_bwd_post<T, SAME>, done, workers, kBwdThreads, BwdLds<T>::kBytes, st, a);
+    return launch(&k_node_bwd_pre<T, R, CN, CLASSES, NORM>, done, bwd_workers(a.rows), L::kThreads, L::kBytes, st, a);
+}
+template <typename T, int R, int CN> int dispatch_bwd_pre(const tgt_node_bwd_pre_args& a, hipStream_t st) {
+    if (a.dlogp) return launch_bwd_pre<T, R, CN, true, true>(a, st);
+    return a.v_next ? launch_bwd_pre<T, R, CN, false, true>(a, st) : launch_bwd_pre<T, R, CN, false, false>(a, st);
+}
+template <typename T, int R, int CN, bool SAME> int launch_bwd_post(const tgt_node_bwd_post_args& a, hipStream_t st) {
+    using L = Bwd<T, R, CN>;
+    static std::atomic<uint64_t> done{0};
+    return launch(&k_node_bwd_post<T, R, CN, SAME>, done, bwd_workers(a.rows), L::kThreads, L::kBytes, st, a);
 }
 bool dtype_ok(int dtype) { return dtype == TGT_DTYPE_F32 || dtype == TGT_DTYPE_BF16; }
 
@@ -637,11 +656,16 @@ int tgt_node_fwd(const tgt_node_fwd_args* a, void* stream) {
     if (a->rows == 0) return TGT_OK;
     KernelTimer t(KS_NODE_FWD, (hipStream_t)stream);
     const hipStream_t st = (hipStream_t)stream;
-    if (a->dtype == TGT_DTYPE_F32) return dispatch_fwd<float, false>(*a, st);
-    return a->same_bits ? dispatch_fwd<nbf16, true>(*a, st) : dispatch_fwd<nbf16, false>(*a, st);
+    // Sixteen rows per wave while that is one round (the chain of a wave is what the launch takes, and more CUs have one), thirty-two
+    // with more rows: us with 16 / 32, float32 4 K nodes 16.6 / 21.8, 37605 23.3 / 26.5, 64 K 31.4 / 30.7, 200 K 107 / 103; bf16
+    // 4 K 10.9 / 18.3, 37605 15.3 / 20.2, 64 K 18.3 / 18.9, 200 K 43.1 / 38.8.  In float32 the weights' way out of LDS is as long as the
+    // products with sixteen rows, so the line lies where the CUs are three quarters full.
+    if (a->dtype == TGT_DTYPE_F32) return 4 * a->rows <= 3 * one_round() ? dispatch_fwd<float, 16, false>(*a, st) : dispatch_fwd<float, 32, false>(*a, st);
+    if (a->same_bits) return dispatch_fwd<nbf16, 32, true>(*a, st);
+    return a->rows <= one_round() ? dispatch_fwd<nbf16, 16, false>(*a, st) : dispatch_fwd<nbf16, 32, false>(*a, st);
 }
 
-int tgt_node_bwd_workers(int64_t rows) { return rows < 0 ? -1 : tgt::grid_for(rows, 4); }
+int tgt_node_bwd_workers(int64_t rows) { return rows < 0 ? -1 : tgt::bwd_workers(rows); }
 
 int tgt_node_bwd_pre(const tgt_node_bwd_pre_args* a, void* stream) {
     using namespace tgt;
@@ -649,8 +673,9 @@ int tgt_node_bwd_pre(const tgt_node_bwd_pre_args* a, void* stream) {
     if (a->dlogp ? ((!a->logp && !a->linear) || a->classes < 1 || a->classes > 64 || a->tokens < 0) : (!a->dq || !a->dk || !a->dv || !a->g_in))
         return bad("tgt_node_bwd_pre", "dq, dk, dv, g_in or dlogp, logp and 1 to 64 classes are needed");
     KernelTimer t(KS_NODE_BWD_PRE, (hipStream_t)stream);
-    const int workers = grid_for(a->rows, 4);
-    return a->dtype == TGT_DTYPE_F32 ? dispatch_bwd_pre<float>(*a, workers, (hipStream_t)stream) : dispatch_bwd_pre<nbf16>(*a, workers, (hipStream_t)stream);
+    const hipStream_t st = (hipStream_t)stream;
+    if (a->dtype == TGT_DTYPE_F32) return groups_of_64(a->rows, true) ? dispatch_bwd_pre<float, 16, 64>(*a, st) : dispatch_bwd_pre<float, 16, 128>(*a, st);
+    return groups_of_64(a->rows, false) ? dispatch_bwd_pre<nbf16, 16, 64>(*a, st) : dispatch_bwd_pre<nbf16, 16, 128>(*a, st);
 }
 
 int tgt_node_bwd_post(const tgt_node_bwd_post_args* a, void* stream) {
@@ -660,9 +685,10 @@ int tgt_node_bwd_post(const tgt_node_bwd_post_args* a, void* stream) {
     if (a->nd && (!a->Z || (a->heads != 8 && a->heads != 4 && a->heads != 2))) return bad("tgt_node_bwd_post", "nd needs Z and 8, 4 or 2 heads");
     KernelTimer t(KS_NODE_BWD_POST, (hipStream_t)stream);
     const hipStream_t st = (hipStream_t)stream;
-    const int workers = grid_for(a->rows, 4);
-    if (a->dtype == TGT_DTYPE_F32) return dispatch_bwd_post<float, false>(*a, workers, st);
-    return a->same_bits ? dispatch_bwd_post<nbf16, true>(*a, workers, st) : dispatch_bwd_post<nbf16, false>(*a, workers, st);
+    if (a->dtype == TGT_DTYPE_F32) return groups_of_64(a->rows, true) ? launch_bwd_post<float, 16, 64, false>(*a, st) : launch_bwd_post<float, 16, 128, false>(*a, st);
+    const bool small = groups_of_64(a->rows, false);
+    if (a->same_bits) return small ? launch_bwd_post<nbf16, 32, 64, true>(*a, st) : launch_bwd_post<nbf16, 32, 128, true>(*a, st);
+    return small ? launch_bwd_post<nbf16, 16, 64, false>(*a, st) : launch_bwd_post<nbf16, 16, 128, false>(*a, st);
 }
 
 int tgt_node_sums(const tgt_node_sum* sums, int count, int dtype, void* stream) {
@@ -681,9 +707,9 @@ int tgt_node_sums(const tgt_node_sum* sums, int count, int dtype, void* stream) 
             for (int o = 0; o < 2 * s.mats + 2; ++o) a.out[i][o] = s.out[o];
             longest = std::max(longest, a.n[i]);
         }
-        const dim3 grid((unsigned)(longest / 64), (unsigned)m);
-        if (dtype == TGT_DTYPE_F32) hipLaunchKernelGGL((k_node_sums<float>), grid, dim3(1024), 0, (hipStream_t)stream, a);
-        else hipLaunchKernelGGL((k_node_sums<nbf16>), grid, dim3(1024), 0, (hipStream_t)stream, a);
+        const dim3 grid((unsigned)(longest / kSumElems), (unsigned)m);
+        if (dtype == TGT_DTYPE_F32) hipLaunchKernelGGL((k_node_sums<float>), grid, dim3(256), 0, (hipStream_t)stream, a);
+        else hipLaunchKernelGGL((k_node_sums<nbf16>), grid, dim3(256), 0, (hipStream_t)stream, a);
         TGT_HIP_CHECK(hipGetLastError());
     }
     return TGT_OK;

@@ -25,6 +25,36 @@ template <int N, int THREADS> __device__ __forceinline__ void copy_vecs(vec16* d
     }
 }
 
+// The same for a workgroup of any number of whole waves; N is a number of whole waves' accesses
+template <int K> __device__ __forceinline__ void copy_batch(int threads, vec16* dst, const vec16* __restrict__ src) {
+    vec16 v[K];
+#pragma unroll
+    for (int i = 0; i < K; ++i) v[i] = src[i * threads];
+#pragma unroll
+    for (int i = 0; i < K; ++i) dst[i * threads] = v[i];
+}
+template <int N> __device__ __forceinline__ void copy_vecs_by(int threads, vec16* dst, const vec16* __restrict__ src) {
+    static_assert(N % 64 == 0, "whole waves");
+    const int wave0 = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63);
+    int k = wave0 < N ? (N - wave0 + threads - 1) / threads : 0, at = threadIdx.x;      // accesses of this wave
+    for (; k > 8; k -= 8, at += 8 * threads) copy_batch<8>(threads, dst + at, src + at);
+    switch (k) {      // the rest in one round trip
+        case 1: copy_batch<1>(threads, dst + at, src + at); break;
+        case 2: copy_batch<2>(threads, dst + at, src + at); break;
+        case 3: copy_batch<3>(threads, dst + at, src + at); break;
+        case 4: copy_batch<4>(threads, dst + at, src + at); break;
+        case 5: copy_batch<5>(threads, dst + at, src + at); break;
+        case 6: copy_batch<6>(threads, dst + at, src + at); break;
+        case 7: copy_batch<7>(threads, dst + at, src + at); break;
+        case 8: copy_batch<8>(threads, dst + at, src + at); break;
+        default: break;
+    }
+}
+// a few parameter vectors
+template <int N> __device__ __forceinline__ void copy_params(int threads, float* dst, const float* __restrict__ src) {
+    for (int at = threadIdx.x; at < N / 4; at += threads) reinterpret_cast<vec16*>(dst)[at] = reinterpret_cast<const vec16*>(src)[at];
+}
+
 // A packed weight on its way from memory to LDS through the registers of the four block waves
 template <int N> struct WeightsAhead {
     static_assert(N % 256 == 0, "whole vectors per thread");
@@ -46,65 +76,106 @@ template <int N> struct WeightsAhead {
 };
 
 // ---- backward: shared pieces ----------------------------------------------------------------------------------------------
-// Eight waves, two roles, one of each per SIMD: waves 0 .. 3 ("chain") carry 32 nodes each through the chain of products and
-// LayerNorms and leave the planes of both operands of every weight gradient in LDS; waves 4 .. 7 ("blocks") keep one 32 x 32
-// block of every weight gradient in registers and add the products over the 128 nodes while the chain is in its next step,
+// Two roles per workgroup: the first CN / R waves ("chain") carry R of its CN nodes each through the chain of products and
+// LayerNorms and leave the planes of both operands of every weight gradient in LDS; four more ("blocks") keep one 32 x 32
+// block of every weight gradient in registers and add the products over the CN nodes while the chain is in its next step,
 // and hand the chain its packed weights one at a time.  So the matrix work of one role runs beside the vector work of the
 // other, and neither has to hold the other's registers (with all waves in both roles, 16 KB of accumulators per wave next to
 // the tiles spilled: 106 us for k_node_bwd_post and 55 us for k_node_bwd_pre at 64 K nodes in float32).
-constexpr int kChainNodes = 128, kBwdThreads = 512;
+constexpr int kBlockWaves = 4;
 
-template <typename T, int NV = 5> struct BwdLds {
-    static constexpr int P = Num<T>::P;
-    static constexpr int kW = 2 * P * kPlaneBytes, kStage = kW + kFragVecs<P> * 16, kVecs = kStage + 4 * RowShape<T>::kVecs * 16;
-    static constexpr int kBytes = kVecs + NV * kVec * 4;      // NV: parameter vectors
+template <typename T, int R_, int CN_, int NV = 5> struct Bwd {      // NV: parameter vectors
+    static constexpr int R = R_, CN = CN_, P = Num<T>::P, kChain = CN / R, kThreads = (kChain + kBlockWaves) * 64, kPlane = CN * 128;
+    static constexpr int kW = 2 * P * kPlane, kStage = kW + kFragVecs<P> * 16, kVecs = kStage + kChain * RowShape<T, R>::kVecs * 16;
+    static constexpr int kBytes = kVecs + NV * kVec * 4;
+    static_assert(kChain * 5 * 64 * 4 <= kW, "the column sums of the chain waves meet where the planes were");
 };
 
 // The workgroup's sums to its partial: NM 64 x 64 blocks (registers of the block waves), then NV vectors of 64 (a register
 // of each chain wave; added through LDS).
-template <int NM, int NV> __device__ __forceinline__ void write_partial(float* __restrict__ mine, const float16_t (&acc)[NM], const float (&col)[NV], float* buf, int wave, int lane) {
+template <typename L, int NM, int NV> __device__ __forceinline__ void write_partial(float* __restrict__ mine, const float16_t (&acc)[NM], const float (&col)[NV], float* buf, int wave, int lane) {
     __syncthreads();
-    if (wave < 4) {
+    if (wave < L::kChain) {
 #pragma unroll
         for (int c = 0; c < NV; ++c) buf[(wave * NV + c) * 64 + lane] = col[c];
     } else {
-        const int q = wave - 4, h = lane >> 5;
+        const int q = wave - L::kChain, h = lane >> 5;
 #pragma unroll
         for (int j = 0; j < NM; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) mine[j * 4096 + (32 * (q >> 1) + 8 * (r >> 2) + 4 * h + (r & 3)) * 64 + 32 * (q & 1) + (lane & 31)] = acc[j][r];
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < NV * 64; i += kBwdThreads) mine[NM * 4096 + i] = (buf[i] + buf[NV * 64 + i]) + (buf[2 * NV * 64 + i] + buf[3 * NV * 64 + i]);
+    for (int i = threadIdx.x; i < NV * 64; i += L::kThreads) {
+        float t = 0.f;
+#pragma unroll
+        for (int c = 0; c < L::kChain; c += 2) t += buf[c * NV * 64 + i] + buf[(c + 1) * NV * 64 + i];
+        mine[NM * 4096 + i] = t;
+    }
 }
 
-// Per head of a node (1 / (Z + 1e-6), da . a): what the sparse attention's backward begins with.  da, a: the lane's half of the node.
-template <typename T> __device__ __forceinline__ void put_node_side(const Tile& da, const Tile& a, const float* __restrict__ Z0, float* __restrict__ nd0, int heads, int64_t node, int h) {
-    float dot[4];
+// Per head of a node (1 / (Z + 1e-6), da . a): what the sparse attention's backward begins with.  da, a: the lane's share of the node.
+// All lanes take part (`in`: whether the node exists).
+template <typename T, int R> __device__ __forceinline__ void put_node_side(const TileOf<R>& da, const TileOf<R>& a, const float* __restrict__ Z0, float* __restrict__ nd0, int heads, int64_t node, int g, bool in) {
+    float dot[R / 8];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < R / 8; ++k) {
         dot[k] = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; ++i) dot[k] += stored(da.get(8 * k + i), (const T*)nullptr) * a.get(8 * k + i);
     }
+    if constexpr (R == 16) {      // two heads of 32 features: two lanes each
+        if (heads == 2) {
+            const float t = dot[0] + dot[1];
+            const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(t), __float_as_uint(t), false, false);
+            dot[0] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        }
+    }
+    if (!in) return;
     const float* Z = Z0 + node * heads;      // 8, 4 or 2 heads: one, two or four groups of 8 features each
     float2* nd = reinterpret_cast<float2*>(nd0) + node * heads;
-    if (heads == 8) {
-        const float4 z = *reinterpret_cast<const float4*>(Z + 4 * h);
-        float4* o = reinterpret_cast<float4*>(nd + 4 * h);
+    if constexpr (R == 16) {
+        if (heads == 8) {
+            const float2 z = *reinterpret_cast<const float2*>(Z + 2 * g);
+            *reinterpret_cast<float4*>(nd + 2 * g) = make_float4(1.f / (z.x + 1e-6f), dot[0], 1.f / (z.y + 1e-6f), dot[1]);
+        } else if (heads == 4) nd[g] = make_float2(1.f / (Z[g] + 1e-6f), dot[0] + dot[1]);
+        else if ((g & 1) == 0) nd[g >> 1] = make_float2(1.f / (Z[g >> 1] + 1e-6f), dot[0]);
+    } else if (heads == 8) {
+        const float4 z = *reinterpret_cast<const float4*>(Z + 4 * g);
+        float4* o = reinterpret_cast<float4*>(nd + 4 * g);
         o[0] = make_float4(1.f / (z.x + 1e-6f), dot[0], 1.f / (z.y + 1e-6f), dot[1]);
         o[1] = make_float4(1.f / (z.z + 1e-6f), dot[2], 1.f / (z.w + 1e-6f), dot[3]);
     } else if (heads == 4) {
-        const float2 z = *reinterpret_cast<const float2*>(Z + 2 * h);
-        *reinterpret_cast<float4*>(nd + 2 * h) = make_float4(1.f / (z.x + 1e-6f), dot[0] + dot[1], 1.f / (z.y + 1e-6f), dot[2] + dot[3]);
+        const float2 z = *reinterpret_cast<const float2*>(Z + 2 * g);
+        *reinterpret_cast<float4*>(nd + 2 * g) = make_float4(1.f / (z.x + 1e-6f), dot[0] + dot[1], 1.f / (z.y + 1e-6f), dot[2] + dot[3]);
     } else {
-        nd[h] = make_float2(1.f / (Z[h] + 1e-6f), dot[0] + dot[1] + (dot[2] + dot[3]));
+        nd[g] = make_float2(1.f / (Z[g] + 1e-6f), dot[0] + dot[1] + (dot[2] + dot[3]));
     }
 }
 
 int bad(const char* who, const char* what) { set_error("%s: %s", who, what); return TGT_ERR_INVALID_ARG; }
-// a workgroup of `waves` waves per CU (LDS), fewer when there is less work
-int grid_for(int64_t rows, int waves) { return (int)std::max<int64_t>(1, std::min<int64_t>(num_cus(), ((rows + 31) / 32 + waves - 1) / waves)); }
+int64_t groups_of(int64_t rows, int per) { return std::max<int64_t>(1, (rows + per - 1) / per); }
+// Forward: a workgroup per CU (LDS), of as many waves as give every CU one, four to `most` (a workgroup copies the weights of a layer to
+// LDS: with fewer waves the copies are more traffic than the rows)
+int fwd_waves_for(int64_t rows, int per, int most) { return (int)std::min<int64_t>(most, std::max<int64_t>(4, (groups_of(rows, per) + num_cus() - 1) / num_cus())); }
+int fwd_grid(int64_t rows, int per, int waves) { return (int)std::min<int64_t>(num_cus(), groups_of(rows, per * waves)); }
+// Rows that sixteen waves of 16 (or eight of 32) on every CU take in one round
+int64_t one_round(void) { return (int64_t)256 * num_cus(); }
+
+// Backward: nodes of a workgroup's group.  64 while there is a CU for every group of 64 (the chain of a workgroup is what such a launch
+// takes), 128 with more: the products of a group run while its chain goes on, and a barrier costs the same for 64 nodes and for 128.
+// In between the last round decides: float32 takes about 1.75 times as long for a group of 128 as for one of 64 (37605 nodes, three rounds
+// of 64 / two of 128: k_node_bwd_pre 27.4 / 30.4 us, k_node_bwd_post 42.4 / 49.0; 64000, four / two: 35.9 / 33.7, 56.8 / 55.4), bf16 1.45
+// times (37605: 18.6 / 17.8, 27.0 / 25.0).  The number of workgroups - and of partial sums - does not depend on the type: it is the same
+// for both choices as soon as every CU has a group of 128.
+int bwd_workers(int64_t rows) { return (int)std::min<int64_t>(num_cus(), groups_of(rows, rows <= (int64_t)64 * num_cus() ? 64 : 128)); }
+bool groups_of_64(int64_t rows, bool f32) {
+    const int64_t cus = num_cus();
+    if (rows <= 64 * cus) return true;
+    if (!f32 || rows < 128 * cus) return false;
+    const int64_t r64 = (groups_of(rows, 64) + cus - 1) / cus, r128 = (groups_of(rows, 128) + cus - 1) / cus;
+    return 4 * r64 <= 7 * r128;
+}
 
 template <typename... Args> int launch(void (*kernel)(Args...), std::atomic<uint64_t>& done, int grid, int threads, int lds, hipStream_t st, Args... args) {
     if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), lds, done)) return rc;

@@ -1,13 +1,17 @@
 // Building blocks of the fused per-node kernels (node_layer.hip): everything between two attention launches of an
-// encoder layer works on node rows of 64 features, so a wave takes 32 rows and keeps them in registers from the first
-// load to the last store.
+// encoder layer works on node rows of 64 features, so a wave takes R = 32 or 16 rows and keeps them in registers from the
+// first load to the last store.
 //
 // Register layout.  v_mfma_f32_32x32x16_bf16 leaves D[8 j + 4 h + t][c] in lane c + 32 h (register 4 j + t) and takes
-// operand B[k][c] in lane c + 32 h (eight k per lane).  With node rows as columns (c = node) and the rows of the
-// weights handed over in a permuted order, lane (node n, half h) of a product holds the output features 32 h .. 32 h + 31
-// of its node in register order, and these registers are the B operand of the next product as they stand: a chain of
-// linears, residual adds, LayerNorms and activations never leaves the registers.  LayerNorm sums are 32 adds in a lane
-// and one exchange between the halves.
+// operand B[k][c] in lane c + 32 h (eight k per lane); v_mfma_f32_16x16x32_bf16 leaves D[4 g + t][c] in lane c + 16 g and
+// takes B[k][c] there (eight k per lane, four groups of lanes).  With node rows as columns (c = node) and the rows of the
+// weights handed over in a permuted order, lane (node n, group g = lane / R) of a product holds the output features
+// R g .. R g + R - 1 of its node in register order, and these registers are the B operand of the next product as they stand: a
+// chain of linears, residual adds, LayerNorms and activations never leaves the registers.  LayerNorm sums are R adds in a
+// lane and one or two exchanges between the groups.
+//
+// R = 32 reads every weight once per 32 rows and takes 256 registers in float32; R = 16 halves what a wave holds and the length
+// of its chain, and reads the weights twice as often from LDS (in float32 about as long as the products take).
 //
 // Number formats.  bf16 kernels round where a chain of separate kernels would have stored a tensor (`stored`).  The numbers are those
 // of the separate kernels up to the order of float32 sums and, in the node-level Graphormer, to another evaluation of GELU
@@ -24,6 +28,7 @@ namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float float16_t __attribute__((ext_vector_type(16)));
+typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t vec16 __attribute__((ext_vector_type(4)));      // 16 bytes in registers
 struct nbf16 { uint16_t x; };
@@ -32,15 +37,16 @@ template <typename T> struct Num;
 template <> struct Num<float> { static constexpr int P = 3; };
 template <> struct Num<nbf16> { static constexpr int P = 1; };
 
-// Lane (n = lane % 32, h = lane / 32) holds features 32 h .. 32 h + 31 of node n: at(i) is feature 32 h + i.
-struct Tile {
-    float v[32];
+// Lane (n = lane % R, g = lane / R) holds features R g .. R g + R - 1 of node n: get(i) is feature R g + i.
+template <int R> struct TileOf {
+    float v[R];
     __device__ __forceinline__ float get(int i) const { return v[i]; }
     __device__ __forceinline__ void set(int i, float x) { v[i] = x; }
 };
-#define TGT_EACH(i) _Pragma("unroll") for (int i = 0; i < 32; ++i)
+using Tile = TileOf<32>;
+#define TGT_EACH(i) _Pragma("unroll") for (int i = 0; i < R; ++i)      // R: rows per wave and features per lane
 
-__device__ __forceinline__ void zero(Tile& t) { TGT_EACH(i) t.set(i, 0.f); }
+template <int R> __device__ __forceinline__ void zero(TileOf<R>& t) { TGT_EACH(i) t.set(i, 0.f); }
 
 // The three parts of a float as float words whose lower half is zero (hi, mid) or unused (lo).  The subtractions are of x itself: joined
 // with a product that made x (a fused multiply-add), they would be of the unrounded one, whose parts do not end where lo does - the cut
@@ -71,7 +77,7 @@ __device__ __forceinline__ void to_planes(const float (&v)[8], bf16x8_t (&p)[1])
     for (int i = 0; i < 8; ++i) p[0][i] = static_cast<__bf16>(v[i]);
 }
 // the eight contraction indices of step s as matrix operands
-template <int P> __device__ __forceinline__ void step_planes(const Tile& t, int s, bf16x8_t (&p)[P]) {
+template <int P, int R> __device__ __forceinline__ void step_planes(const TileOf<R>& t, int s, bf16x8_t (&p)[P]) {
     float v[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = t.get(8 * s + i);
@@ -81,8 +87,11 @@ template <int P> __device__ __forceinline__ void step_planes(const Tile& t, int 
 __device__ __forceinline__ float16_t mma(bf16x8_t a, bf16x8_t b, float16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
+__device__ __forceinline__ float4_t mma(bf16x8_t a, bf16x8_t b, float4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
 // c += a b for one contraction step in P planes each, small terms first
-__device__ __forceinline__ float16_t mma_planes(const bf16x8_t (&a)[3], const bf16x8_t (&b)[3], float16_t c) {
+template <typename C> __device__ __forceinline__ C mma_planes(const bf16x8_t (&a)[3], const bf16x8_t (&b)[3], C c) {
     c = mma(a[2], b[0], c);
     c = mma(a[0], b[2], c);
     c = mma(a[1], b[1], c);
@@ -90,7 +99,7 @@ __device__ __forceinline__ float16_t mma_planes(const bf16x8_t (&a)[3], const bf
     c = mma(a[0], b[1], c);
     return mma(a[0], b[0], c);
 }
-__device__ __forceinline__ float16_t mma_planes(const bf16x8_t (&a)[1], const bf16x8_t (&b)[1], float16_t c) { return mma(a[0], b[0], c); }
+template <typename C> __device__ __forceinline__ C mma_planes(const bf16x8_t (&a)[1], const bf16x8_t (&b)[1], C c) { return mma(a[0], b[0], c); }
 // The same with the five small terms in a sum of their own, 2^-8 of c: c is rounded once per step instead of six times, the small sum's
 // roundings hardly count
 __device__ __forceinline__ void mma_planes(const bf16x8_t (&a)[3], const bf16x8_t (&b)[3], float16_t& c, float16_t& small) {
@@ -110,9 +119,14 @@ __device__ __forceinline__ float16_t mma_halves(bf16x8_t a, bf16x8_t b, float16_
     return __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(short4_t{x[4], x[5], x[6], x[7]}, short4_t{y[4], y[5], y[6], y[7]}, c, 0, 0, 0);
 }
 
-// A packed 64 x 64 weight: operand A of step s and row block m, plane p, at ((2 s + m) P + p) * 64 + lane (16 bytes per
-// lane): row block m, row 8 j + 4 hh + t is output feature 32 hh + 16 m + 4 j + t; a lane's eight contraction indices are
-// the input features 32 (lane / 32) + 8 s ... + 7.
+// A packed 64 x 64 weight is one layout for both R, 16-byte vectors of eight contraction indices.  R = 16: operand A of step s and block
+// m of 16 rows, plane p, is in the 64 vectors from ((4 s + m) P + p) * 64 on; row r of the block is output feature 16 (r / 4) + 4 m +
+// r % 4, the indices are the input features 16 (lane / 16) + 8 s ... + 7, and the vector is number 16 (lane / 16) + 4 gray(r / 4) + r % 4
+// of the 64.  R = 32 (step s of 16, block m of 32 rows) takes for its row r the output feature 32 ((r / 4) % 2) + 16 m + 4 (r / 8) +
+// r % 4 and the input features 32 (lane / 32) + 8 s ... + 7.  The Gray code 0 1 3 2 makes both reads free of bank conflicts: eight
+// neighbouring lanes differ in bit 4 of the output feature (R = 16) or in bit 5 (R = 32), and the slot has their exclusive or as its third bit
+// (without it the reads of R = 32 meet two by two: 200 K nodes forward in bf16 41.0 us instead of 38.8).
+__host__ __device__ constexpr int gray2(int a) { return a ^ (a >> 1); }      // its own inverse for two bits
 template <int P> constexpr int kFragVecs = 8 * P * 64;
 
 // Nothing is moved across: left alone, the scheduler asks for every operand of a product before its first instruction, and
@@ -120,35 +134,39 @@ template <int P> constexpr int kFragVecs = 8 * P * 64;
 __device__ __forceinline__ void fence_schedule() { __builtin_amdgcn_sched_barrier(0); }
 
 // B operands of a whole tile
-template <int P> struct Frags { bf16x8_t p[4][P]; };
-template <int P> __device__ __forceinline__ void make_frags(Frags<P>& f, const Tile& t) {
+template <int P, int R = 32> struct Frags { bf16x8_t p[R / 8][P]; };
+template <int P, int R> __device__ __forceinline__ void make_frags(Frags<P, R>& f, const TileOf<R>& t) {
 #pragma unroll
-    for (int s = 0; s < 4; ++s) step_planes<P>(t, s, f.p[s]);
+    for (int s = 0; s < R / 8; ++s) step_planes<P>(t, s, f.p[s]);
 }
 
 // acc += W b: w = packed weight in LDS, b = node rows (a tile, cut into planes one contraction step at a time, or planes);
 // the weight operands of the next step are asked for before the products of this one
 template <int P> struct StepWeights { bf16x8_t a[2][P]; };
-template <int P> __device__ __forceinline__ void step_weights(StepWeights<P>& f, const vec16* w, int s, int lane) {
+template <int P> __device__ __forceinline__ void step_weights(StepWeights<P>& f, const vec16* const (&w)[2], int s) {
 #pragma unroll
     for (int m = 0; m < 2; ++m)
 #pragma unroll
-        for (int p = 0; p < P; ++p) f.a[m][p] = __builtin_bit_cast(bf16x8_t, w[((2 * s + m) * P + p) * 64 + lane]);
+        for (int p = 0; p < P; ++p) f.a[m][p] = __builtin_bit_cast(bf16x8_t, w[m][((s & 1) * 4 * P + p) * 64 + 16 * (s >> 1)]);
 }
-template <int P> __device__ __forceinline__ void step_operand(bf16x8_t (&x)[P], const Tile& b, int s) { step_planes<P>(b, s, x); }
-template <int P> __device__ __forceinline__ void step_operand(bf16x8_t (&x)[P], const Frags<P>& b, int s) {
+template <int P, int R> __device__ __forceinline__ void step_operand(bf16x8_t (&x)[P], const TileOf<R>& b, int s) { step_planes<P>(b, s, x); }
+template <int P, int R> __device__ __forceinline__ void step_operand(bf16x8_t (&x)[P], const Frags<P, R>& b, int s) {
 #pragma unroll
     for (int p = 0; p < P; ++p) x[p] = b.p[s][p];
 }
 // HALVES: bits of the separate linears (linear.hip), for one plane
-template <int P, bool HALVES = false, typename B> __device__ __forceinline__ void gemm(Tile& acc, const B& b, const vec16* w, int lane) {
+template <int P, bool HALVES = false, typename B> __device__ __forceinline__ void gemm(TileOf<32>& acc, const B& b, const vec16* w0, int lane) {
+    const int r = lane & 31, upper = (r >> 2) & 1;
+    const vec16* const mine = w0 + (r >> 3) * P * 64 + (r & 3) + (lane & 32);
+    const vec16* const w[2] = {mine + 12 * upper, mine + 4 + 4 * upper};      // 4 gray(2 upper + m)
     StepWeights<P> f[2];
-    step_weights<P>(f[0], w, 0, lane);
+    step_weights<P>(f[0], w, 0);
     float16_t c[2];
-    TGT_EACH(i) c[i >> 4][i & 15] = acc.get(i);
+#pragma unroll
+    for (int i = 0; i < 32; ++i) c[i >> 4][i & 15] = acc.get(i);
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-        if (s < 3) step_weights<P>(f[(s + 1) & 1], w, s + 1, lane);
+        if (s < 3) step_weights<P>(f[(s + 1) & 1], w, s + 1);
         bf16x8_t x[P];
         step_operand<P>(x, b, s);
 #pragma unroll
@@ -158,11 +176,35 @@ template <int P, bool HALVES = false, typename B> __device__ __forceinline__ voi
         }
         fence_schedule();
     }
-    TGT_EACH(i) acc.set(i, c[i >> 4][i & 15]);
+#pragma unroll
+    for (int i = 0; i < 32; ++i) acc.set(i, c[i >> 4][i & 15]);
+}
+template <int P, bool HALVES = false, typename B> __device__ __forceinline__ void gemm(TileOf<16>& acc, const B& b, const vec16* w, int lane) {
+    static_assert(!HALVES, "products of half the depth are made by R = 32");
+    w += (lane & 0x33) | (gray2((lane >> 2) & 3) << 2);
+    bf16x8_t a[2][P], x[P];
+    const auto ask = [&](int q) {
+#pragma unroll
+        for (int p = 0; p < P; ++p) a[q & 1][p] = __builtin_bit_cast(bf16x8_t, w[(q * P + p) * 64]);
+    };
+    float4_t c[4];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) c[i >> 2][i & 3] = acc.get(i);
+    ask(0);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        if (q < 7) ask(q + 1);
+        if (q % 4 == 0) step_operand<P>(x, b, q / 4);
+        c[q & 3] = mma_planes(a[q & 1], x, c[q & 3]);
+        fence_schedule();
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc.set(i, c[i >> 2][i & 3]);
 }
 // acc += W b with the small terms of three planes in a sum of their own, one row block after the other and the weights of a step asked
 // for when it begins: beside 96 registers of operands there is room for one block's two sums and one step's weights - with the next
 // step's too, 22 registers go to scratch and 128 -> 64 of 64 K rows takes 19.6 us instead of 14.9.
+// (linear_tiles.hip packs its pieces of a weight for this: operand A of step s and block m of 32 rows, plane p, at ((2 s + m) P + p) * 64 + lane.)
 template <int P> __device__ __forceinline__ void gemm_apart(Tile& acc, const Frags<P>& b, const vec16* w, int lane) {
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
@@ -189,28 +231,29 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The 32 rows of a wave: first row and how many of them exist (wave-uniform, so the addresses have scalar bases)
+// The `per` rows of a wave: first row and how many of them exist (wave-uniform, so the addresses have scalar bases)
 struct Rows {
     int64_t first;
     int left;       // <= 0: none
-    __device__ __forceinline__ Rows(int64_t tile, int64_t N) {
-        const int64_t r = N - tile * 32;
-        left = r > 32 ? 32 : (int)r;
-        first = left > 0 ? tile * 32 : 0;
+    __device__ __forceinline__ Rows(int64_t tile, int64_t N, int per = 32) {
+        const int64_t r = N - tile * per;
+        left = r > per ? per : (int)r;
+        first = left > 0 ? tile * per : 0;
     }
 };
 
-// 32 node rows on their way between global memory (coalesced: consecutive lanes, consecutive 16-byte pieces) and the
+// A wave's node rows on their way between global memory (coalesced: consecutive lanes, consecutive 16-byte pieces) and the
 // register layout, through a wave-private LDS image of the rows.  Piece q of row r sits in slot q ^ (r mod pieces): both
 // the row-wise and the node-wise accesses spread over all banks, and the slots of a lane differ from its first one by an
 // exclusive or, which is formed at each access (kept in registers, the addresses of all accesses would crowd out the tiles).
-template <typename T> struct RowShape {
+template <typename T, int R = 32> struct RowShape {
     static constexpr int kPieces = 64 * (int)sizeof(T) / 16;      // 16-byte pieces of a row: 16 or 8
     static constexpr int kPer = 64 / kPieces;                     // rows per access of the wave
-    static constexpr int kAcc = 32 / kPer;                        // accesses per tile
-    static constexpr int kVecs = 32 * kPieces;                    // 16-byte vectors of the image
+    static constexpr int kAcc = R / kPer;                         // accesses per tile
+    static constexpr int kVecs = R * kPieces;                     // 16-byte vectors of the image
+    static constexpr int kMine = kPieces * R / 64;                // pieces of its node's row that a lane holds
 };
-template <typename T> struct Raw { vec16 v[RowShape<T>::kAcc]; };
+template <typename T, int R = 32> struct Raw { vec16 v[RowShape<T, R>::kAcc]; };
 
 __device__ __forceinline__ int forgotten(int v) { asm volatile("" : "+v"(v)); return v; }
 // slot of access i of the row-wise walk: rows i * kPer ..., consecutive lanes along a row
@@ -223,19 +266,19 @@ template <typename T> __device__ __forceinline__ int row_base(int lane) {
     const int r = lane / PP;
     return forgotten(r * PP + ((lane % PP) ^ r));
 }
-// slot of piece i of the lane's half of its node's row
-template <typename T> __device__ __forceinline__ int node_base(int lane) {
-    constexpr int PP = RowShape<T>::kPieces;
-    const int n = lane & 31, h = lane >> 5;
-    return forgotten(n * PP + ((h * (PP / 2)) ^ (n & (PP - 1))));
+// slot of the first piece of the lane's share of its node's row (piece i: exclusive or with i)
+template <typename T, int R = 32> __device__ __forceinline__ int node_base(int lane) {
+    constexpr int PP = RowShape<T, R>::kPieces;
+    const int n = lane % R, g = lane / R;
+    return forgotten(n * PP + ((g * RowShape<T, R>::kMine) ^ (n & (PP - 1))));
 }
 
-template <typename T> __device__ __forceinline__ void fetch(Raw<T>& raw, const T* __restrict__ src, const Rows& rows, int lane) {
-    constexpr int PP = RowShape<T>::kPieces, PER = RowShape<T>::kPer;
+template <typename T, int R> __device__ __forceinline__ void fetch(Raw<T, R>& raw, const T* __restrict__ src, const Rows& rows, int lane) {
+    constexpr int PP = RowShape<T, R>::kPieces, PER = RowShape<T, R>::kPer;
     const vec16* p = reinterpret_cast<const vec16*>(src) + rows.first * PP;
     const int last = rows.left > 0 ? rows.left - 1 : 0, r0 = forgotten(lane / PP), q = lane % PP;
 #pragma unroll
-    for (int i = 0; i < RowShape<T>::kAcc; ++i) {
+    for (int i = 0; i < RowShape<T, R>::kAcc; ++i) {
         const int r = r0 + i * PER;
         raw.v[i] = p[(uint32_t)((r < last ? r : last) * PP + q)];
     }
@@ -261,33 +304,35 @@ __device__ __forceinline__ vec16 pack16(const float (&f)[8], const nbf16*) {
     return __builtin_bit_cast(vec16, b);
 }
 // ZERO: rows past the end read as zero (they enter sums over nodes); otherwise they repeat the last row
-template <typename T, bool ZERO> __device__ __forceinline__ void settle(Tile& t, Raw<T>& raw, vec16* stage, const Rows& rows, int lane) {
-    constexpr int PP = RowShape<T>::kPieces, PER = RowShape<T>::kPer, VE = 16 / (int)sizeof(T);
-    if (ZERO && rows.left < 32) {
+template <typename T, bool ZERO, int R> __device__ __forceinline__ void settle(TileOf<R>& t, Raw<T, R>& raw, vec16* stage, const Rows& rows, int lane) {
+    using Shape = RowShape<T, R>;
+    constexpr int PP = Shape::kPieces, PER = Shape::kPer, VE = 16 / (int)sizeof(T);
+    if (ZERO && rows.left < R) {
 #pragma unroll
-        for (int i = 0; i < RowShape<T>::kAcc; ++i)
+        for (int i = 0; i < Shape::kAcc; ++i)
             if (i * PER + lane / PP >= rows.left) raw.v[i] = vec16{0u, 0u, 0u, 0u};
     }
     wave_sync();
     const int rb = row_base<T>(lane);
 #pragma unroll
-    for (int i = 0; i < RowShape<T>::kAcc; ++i) stage[row_slot<T>(rb, i)] = raw.v[i];
+    for (int i = 0; i < Shape::kAcc; ++i) stage[row_slot<T>(rb, i)] = raw.v[i];
     wave_sync();
-    const int nb = node_base<T>(lane);
+    const int nb = node_base<T, R>(lane);
 #pragma unroll
-    for (int i = 0; i < PP / 2; ++i) {
+    for (int i = 0; i < Shape::kMine; ++i) {
         float f[VE];
         unpack16(stage[nb ^ i], f, (const T*)nullptr);
 #pragma unroll
         for (int e = 0; e < VE; ++e) t.set(i * VE + e, f[e]);
     }
 }
-template <typename T> __device__ __forceinline__ void put_rows(T* __restrict__ dst, const Tile& t, vec16* stage, const Rows& rows, int lane) {
-    constexpr int PP = RowShape<T>::kPieces, PER = RowShape<T>::kPer, VE = 16 / (int)sizeof(T);
+template <typename T, int R> __device__ __forceinline__ void put_rows(T* __restrict__ dst, const TileOf<R>& t, vec16* stage, const Rows& rows, int lane) {
+    using Shape = RowShape<T, R>;
+    constexpr int PP = Shape::kPieces, PER = Shape::kPer, VE = 16 / (int)sizeof(T);
     wave_sync();
-    const int nb = node_base<T>(lane);
+    const int nb = node_base<T, R>(lane);
 #pragma unroll
-    for (int i = 0; i < PP / 2; ++i) {
+    for (int i = 0; i < Shape::kMine; ++i) {
         float f[VE];
 #pragma unroll
         for (int e = 0; e < VE; ++e) f[e] = t.get(i * VE + e);
@@ -296,15 +341,15 @@ template <typename T> __device__ __forceinline__ void put_rows(T* __restrict__ d
     wave_sync();
     vec16* p = reinterpret_cast<vec16*>(dst) + rows.first * PP;
     const int rb = row_base<T>(lane), r0 = forgotten(lane / PP), q = lane % PP;
-    vec16 v[RowShape<T>::kAcc];
+    vec16 v[Shape::kAcc];
 #pragma unroll
-    for (int i = 0; i < RowShape<T>::kAcc; ++i) v[i] = stage[row_slot<T>(rb, i)];
-    if (rows.left >= 32) {
+    for (int i = 0; i < Shape::kAcc; ++i) v[i] = stage[row_slot<T>(rb, i)];
+    if (rows.left >= R) {
 #pragma unroll
-        for (int i = 0; i < RowShape<T>::kAcc; ++i) p[(uint32_t)((r0 + i * PER) * PP + q)] = v[i];
+        for (int i = 0; i < Shape::kAcc; ++i) p[(uint32_t)((r0 + i * PER) * PP + q)] = v[i];
     } else {
 #pragma unroll
-        for (int i = 0; i < RowShape<T>::kAcc; ++i)
+        for (int i = 0; i < Shape::kAcc; ++i)
             if (r0 + i * PER < rows.left) p[(uint32_t)((r0 + i * PER) * PP + q)] = v[i];
     }
 }
@@ -312,41 +357,50 @@ template <typename T> __device__ __forceinline__ void put_rows(T* __restrict__ d
 __device__ __forceinline__ float stored(float v, const float*) { return v; }
 __device__ __forceinline__ float stored(float v, const nbf16*) { return static_cast<float>(static_cast<__bf16>(v)); }
 
-// v of this lane plus v of the lane that holds the other half of the node
+// v of this lane plus v of the lane that is 32 further on or back
 __device__ __forceinline__ float both_halves(float v) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
+// sum over the lanes that share a node
+template <int R> __device__ __forceinline__ float node_sum(float v) {
+    if constexpr (R == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    return both_halves(v);
+}
 
 // vec: 64 floats in LDS
-__device__ __forceinline__ void load_vec(Tile& t, const float* vec, int h) {
+template <int R> __device__ __forceinline__ void load_vec(TileOf<R>& t, const float* vec, int g) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const float4 f = *reinterpret_cast<const float4*>(vec + 32 * h + 4 * i);
+    for (int i = 0; i < R / 4; ++i) {
+        const float4 f = *reinterpret_cast<const float4*>(vec + R * g + 4 * i);
         t.set(4 * i, f.x); t.set(4 * i + 1, f.y); t.set(4 * i + 2, f.z); t.set(4 * i + 3, f.w);
     }
 }
 // y = W x + bias (vec: 64 floats in LDS).  SAME: the bits of linear.hip, which adds the bias behind the products.
-template <int P, bool SAME, typename B> __device__ __forceinline__ void linear(Tile& y, const B& x, const vec16* w, const float* vec, int lane) {
+template <int P, bool SAME, int R, typename B> __device__ __forceinline__ void linear(TileOf<R>& y, const B& x, const vec16* w, const float* vec, int lane) {
     if constexpr (SAME) {
         zero(y);
         gemm<P, true>(y, x, w, lane);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float4 f = *reinterpret_cast<const float4*>(vec + 32 * (lane >> 5) + 4 * i);
+        for (int i = 0; i < R / 4; ++i) {
+            const float4 f = *reinterpret_cast<const float4*>(vec + R * (lane / R) + 4 * i);
             y.set(4 * i, y.get(4 * i) + f.x); y.set(4 * i + 1, y.get(4 * i + 1) + f.y);
             y.set(4 * i + 2, y.get(4 * i + 2) + f.z); y.set(4 * i + 3, y.get(4 * i + 3) + f.w);
         }
     } else {
-        load_vec(y, vec, lane >> 5);
+        load_vec(y, vec, lane / R);
         gemm<P>(y, x, w, lane);
     }
 }
 
 struct MeanRstd { float mean, rstd; };
 // sum of f(i) over the 64 features; SAME: eights in order, then the eights as elementwise.hip's lanes exchange them
-template <bool SAME, typename F> __device__ __forceinline__ float sum_features(const F& f) {
+template <bool SAME, int R, typename F> __device__ __forceinline__ float sum_features(const F& f) {
     if constexpr (SAME) {
+        static_assert(R == 32, "the separate kernels' bits are made by R = 32");
         float t[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -359,36 +413,36 @@ template <bool SAME, typename F> __device__ __forceinline__ float sum_features(c
     } else {
         float s = 0.f;
         TGT_EACH(i) s += f(i);
-        return both_halves(s);
+        return node_sum<R>(s);
     }
 }
-template <bool SAME> __device__ __forceinline__ MeanRstd row_stats(const Tile& x, float eps) {
-    const float mean = sum_features<SAME>([&](int i) { return x.get(i); }) * (1.f / 64);
-    const float var = sum_features<SAME>([&](int i) { const float d = x.get(i) - mean; return d * d; }) * (1.f / 64);
+template <bool SAME, int R> __device__ __forceinline__ MeanRstd row_stats(const TileOf<R>& x, float eps) {
+    const float mean = sum_features<SAME, R>([&](int i) { return x.get(i); }) * (1.f / 64);
+    const float var = sum_features<SAME, R>([&](int i) { const float d = x.get(i) - mean; return d * d; }) * (1.f / 64);
     return {mean, rsqrtf(var + eps)};
 }
 // x -> (x - mean) * rstd; returns rstd
-template <bool SAME> __device__ __forceinline__ float normalise(Tile& x, float eps) {
+template <bool SAME, int R> __device__ __forceinline__ float normalise(TileOf<R>& x, float eps) {
     const MeanRstd m = row_stats<SAME>(x, eps);
     TGT_EACH(i) x.set(i, (x.get(i) - m.mean) * m.rstd);
     return m.rstd;
 }
 // xhat * gamma + beta, vectors in LDS
-__device__ __forceinline__ void affine(Tile& y, const Tile& xhat, const float* gamma, const float* beta, int h) {
+template <int R> __device__ __forceinline__ void affine(TileOf<R>& y, const TileOf<R>& xhat, const float* gamma, const float* beta, int g) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const float4 g = *reinterpret_cast<const float4*>(gamma + 32 * h + 4 * i);
-        const float4 b = *reinterpret_cast<const float4*>(beta + 32 * h + 4 * i);
-        y.set(4 * i, xhat.get(4 * i) * g.x + b.x);
-        y.set(4 * i + 1, xhat.get(4 * i + 1) * g.y + b.y);
-        y.set(4 * i + 2, xhat.get(4 * i + 2) * g.z + b.z);
-        y.set(4 * i + 3, xhat.get(4 * i + 3) * g.w + b.w);
+    for (int i = 0; i < R / 4; ++i) {
+        const float4 c = *reinterpret_cast<const float4*>(gamma + R * g + 4 * i);
+        const float4 b = *reinterpret_cast<const float4*>(beta + R * g + 4 * i);
+        y.set(4 * i, xhat.get(4 * i) * c.x + b.x);
+        y.set(4 * i + 1, xhat.get(4 * i + 1) * c.y + b.y);
+        y.set(4 * i + 2, xhat.get(4 * i + 2) * c.z + b.z);
+        y.set(4 * i + 3, xhat.get(4 * i + 3) * c.w + b.w);
     }
 }
 // g += LayerNorm backward of dy (gamma in LDS)
-__device__ __forceinline__ void ln_back(Tile& g, const Tile& dy, const Tile& xhat, float rstd, const float* gamma, int h) {
-    Tile d;
-    load_vec(d, gamma, h);
+template <int R> __device__ __forceinline__ void ln_back(TileOf<R>& g, const TileOf<R>& dy, const TileOf<R>& xhat, float rstd, const float* gamma, int group) {
+    TileOf<R> d;
+    load_vec(d, gamma, group);
     float c1 = 0.f, c2 = 0.f;
     TGT_EACH(i) {
         const float v = d.get(i) * dy.get(i);
@@ -396,8 +450,8 @@ __device__ __forceinline__ void ln_back(Tile& g, const Tile& dy, const Tile& xha
         c1 += v;
         c2 += v * xhat.get(i);
     }
-    c1 = both_halves(c1) * (1.f / 64);
-    c2 = both_halves(c2) * (1.f / 64);
+    c1 = node_sum<R>(c1) * (1.f / 64);
+    c2 = node_sum<R>(c2) * (1.f / 64);
     TGT_EACH(i) g.set(i, g.get(i) + rstd * (d.get(i) - c1 - xhat.get(i) * c2));
 }
 
@@ -431,8 +485,8 @@ __device__ __forceinline__ void normal_cdf(float u, float& cdf, float& bell) {
     cdf = z < 1.f ? fmaf(u, p, 0.5f) : outside;
 }
 
-// Sum over the 32 nodes of every feature: lane l returns the sum of feature l.  A reduce-scatter over the lanes of a
-// half: at each of the five steps a lane hands half of its values to a partner and keeps the other half.  All exchanges are
+// Sum over the R nodes of every feature: lane l returns the sum of feature l.  A reduce-scatter over the lanes of a
+// group: at each of the four or five steps a lane hands half of its values to a partner and keeps the other half.  All exchanges are
 // operands of vector instructions (row swap, mirrors within 16 and 8 lanes, quad permutes), none goes through the LDS.
 template <int CTRL> __device__ __forceinline__ float lane_permuted(float v) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
@@ -445,12 +499,14 @@ template <int BIT, int CTRL, int NV> __device__ __forceinline__ void scatter_ste
         v[i] = keep + lane_permuted<CTRL>(send);
     }
 }
-__device__ __forceinline__ float column_sums(const Tile& t, int lane) {
+template <int R> __device__ __forceinline__ float column_sums(const TileOf<R>& t, int lane) {
     float v[16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {      // rows of 16 lanes: the first keeps value i, the second value i + 16
-        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(t.get(i)), __float_as_uint(t.get(i + 16)), false, false);
-        v[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    for (int i = 0; i < 16; ++i) {
+        if constexpr (R == 32) {      // rows of 16 lanes: the first keeps value i, the second value i + 16
+            const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(t.get(i)), __float_as_uint(t.get(i + 16)), false, false);
+            v[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        } else v[i] = t.get(i);
     }
     scatter_step<8, 0x140>(v, lane);      // row_mirror
     scatter_step<4, 0x141>(v, lane);      // row_half_mirror
@@ -461,30 +517,39 @@ __device__ __forceinline__ float column_sums(const Tile& t, int lane) {
 
 // Makes the compiler forget what it knows about the values: without it, the planes of a tile that two products use (some
 // forty instructions' worth each) are computed once and kept in registers that are not there
-__device__ __forceinline__ void forget(Tile& t) {
+template <int R> __device__ __forceinline__ void forget(TileOf<R>& t) {
     TGT_EACH(i) asm volatile("" : "+v"(t.v[i]));
 }
 
 // ---- weight gradients: contraction over nodes ---------------------------------------------------------------------------
-// 128 node rows of an operand in LDS, P bf16 planes of 128 rows x 128 bytes; a wave writes its 32 rows as they sit in its
-// registers and the products read them back transposed (ds_read_b64_tr_b16: within 16 lanes, lane i hands over the address
+// The node rows of a workgroup's operand in LDS, P bf16 planes of 64 or 128 rows x 128 bytes (BYTES); a wave writes its rows as they
+// sit in its registers and the products read them back transposed (ds_read_b64_tr_b16: within 16 lanes, lane i hands over the address
 // of four consecutive elements of row i / 4 and receives column i of the four rows).  16-byte chunk c of row r sits in slot
 // c ^ (r mod 8): eight lanes of a write and sixteen of a transposed read touch different banks.
-constexpr int kPlaneBytes = 128 * 128;
-
-template <int P> __device__ __forceinline__ void put_planes(unsigned char* planes, int row, int h, const Frags<P>& f) {
-    const int base = forgotten(row * 128 + (((4 * h) ^ (row & 7)) << 4));
+template <int BYTES, int P, int R> __device__ __forceinline__ void put_planes(unsigned char* planes, int row, int g, const Frags<P, R>& f) {
+    const int base = forgotten(row * 128 + (((R / 8 * g) ^ (row & 7)) << 4));
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
+    for (int s = 0; s < R / 8; ++s)
 #pragma unroll
-        for (int p = 0; p < P; ++p) *reinterpret_cast<bf16x8_t*>(planes + p * kPlaneBytes + (base ^ (s << 4))) = f.p[s][p];
+        for (int p = 0; p < P; ++p) *reinterpret_cast<bf16x8_t*>(planes + p * BYTES + (base ^ (s << 4))) = f.p[s][p];
+}
+// the same of a tile, cut one contraction step at a time (its planes are not kept)
+template <int BYTES, int P, int R> __device__ __forceinline__ void put_tile_planes(unsigned char* planes, int row, int g, const TileOf<R>& t) {
+    const int base = forgotten(row * 128 + (((R / 8 * g) ^ (row & 7)) << 4));
+#pragma unroll
+    for (int s = 0; s < R / 8; ++s) {
+        bf16x8_t f[P];
+        step_planes<P>(t, s, f);
+#pragma unroll
+        for (int p = 0; p < P; ++p) *reinterpret_cast<bf16x8_t*>(planes + p * BYTES + (base ^ (s << 4))) = f[p];
+    }
 }
 // Address of a lane's first piece of the operand that has features 32 block .. + 31 as rows: nodes 8 (lane / 32) ... + 3
 __device__ __forceinline__ int operand_base(int block, int lane) {
     const int i = lane & 15, chunk = 4 * block + 2 * ((lane >> 4) & 1) + ((i & 3) >> 1);
     return (8 * (lane >> 5) + (i >> 2)) * 128 + ((chunk ^ (i >> 2)) << 4) + 8 * (i & 1);
 }
-template <int P, int BYTES = kPlaneBytes> __device__ __forceinline__ void node_operand(bf16x8_t (&out)[P], const unsigned char* planes, int base, int node0) {
+template <int P, int BYTES> __device__ __forceinline__ void node_operand(bf16x8_t (&out)[P], const unsigned char* planes, int base, int node0) {
     typedef __attribute__((address_space(3))) short4_t lds_short4;
 #pragma unroll
     for (int p = 0; p < P; ++p) {
@@ -498,7 +563,7 @@ template <int P, int BYTES = kPlaneBytes> __device__ __forceinline__ void node_o
 // acc += dy^T x over the nodes of the planes, one 32 x 32 block (bases of its rows and columns from operand_base); the operands of
 // the next sixteen nodes are asked for before the products of these
 // (APART: the small terms in a sum of their own)
-template <int P, int BYTES = kPlaneBytes, bool APART = false>
+template <int P, int BYTES, bool APART = false>
 __device__ __forceinline__ void node_product(float16_t& acc, const unsigned char* dy, const unsigned char* x, int base_dy, int base_x, float16_t* small = nullptr) {
     bf16x8_t a[2][P], b[2][P];
     node_operand<P, BYTES>(a[0], dy, base_dy, 0);
