@@ -289,3 +289,47 @@ def test_query_0_backward_forms_the_forwards_score(cuda, dtype, d):
     _lib.check(L.tgt_dense_row0_bwd(at(q), at(k), at(v), at(bias), b, 1, H, d, code, 0.0, 0, at(a0), at(lse), at(da0), at(g0), at(dq), at(dk), at(dv), at(ds), at(dvirt), stream))
     assert float(lse.abs().max()) > 100 and torch.equal(a0, v) and torch.equal(s0, s)
     assert torch.equal(dv, da0)
+
+
+# Sizes beside the lines between the kernels that keep the bias plane in LDS and those that read it in pieces, every tile count, thin last
+# tiles (one to four rows), rows a power of two of bytes apart.  The general kernels take the same numbers as float32 tensors by
+# bf16_products: the same roundings of operands, probabilities and dS, so what is left is the rounding of the results (2^-9 of each) and sums in
+# another order, which may move a probability or a dS to the neighbouring bf16 (2^-8 of a term): 2^-7 of the largest result.
+@pytest.mark.parametrize("b,S,H,d,offset,p_drop", [
+    (3, 25, 2, 8, 1, 0.0), (3, 28, 2, 8, 0, 0.3), (5, 33, 3, 16, 3, 0.0), (300, 34, 4, 8, 0, 0.0), (3, 40, 8, 8, 5, 0.0), (9, 59, 2, 32, 0, 0.0),
+    (2, 64, 2, 32, 1, 0.0), (3, 68, 2, 16, 0, 0.4), (3, 90, 2, 8, 7, 0.0), (90, 90, 8, 8, 0, 0.0), (3, 100, 2, 32, 2, 0.0), (9, 111, 8, 16, 0, 0.0),
+    (128, 129, 8, 8, 0, 0.0), (3, 129, 8, 8, 1, 0.2), (64, 130, 16, 16, 1, 0.0), (3, 132, 2, 32, 0, 0.0), (2, 161, 2, 8, 0, 0.0), (2, 164, 2, 16, 1, 0.0),
+    (2, 181, 2, 8, 1, 0.0), (2, 182, 2, 32, 0, 0.0), (2, 201, 2, 8, 1, 0.3), (2, 225, 2, 16, 0, 0.0), (2, 249, 2, 8, 1, 0.0), (2, 255, 2, 8, 0, 0.0)])
+def test_plane_in_lds_gives_what_the_general_kernels_give(cuda, b, S, H, d, offset, p_drop):
+    print(f"dense plane b={b} S={S} H={H} d={d} offset={offset} p_drop={p_drop}", flush=True)
+    g = torch.Generator(device=cuda).manual_seed(S + d)
+    q, k, v, dout = (torch.randn(b, S, H, d, generator=g, device=cuda).bfloat16() for _ in range(4))
+    q = q / d
+    flat = torch.randn(offset + b * H * S * S, generator=g, device=cuda).bfloat16()
+    bias = flat[offset:].view(b, H, S, S)      # a plane begins anywhere
+    real = torch.randint(1, S + 1, (b,), generator=g, device=cuda)
+    real[0] = S
+    bias.masked_fill_((torch.arange(S, device=cuda) >= real[:, None])[:, None, None, :], float("-inf"))
+    dout *= (torch.arange(S, device=cuda) < real[:, None])[:, :, None, None]      # nobody reads the padded rows
+    bias[1, 0] = float("-inf")                          # a head without any key
+    bias[1, 1, :, S // 2:] = torch.finfo(torch.bfloat16).min
+    if b > 2:
+        v[2, S - 1, 0, 1] = float("inf")                # tiles of masked keys count: 0 times inf
+        q[2, S // 2, 1, 0] = float("nan")
+        bias[2, :, :, S // 2 + 1:] = float("-inf")
+
+    def run(q, k, v, bias, dout, **kw):
+        ts = [t.detach().requires_grad_(True) for t in (q, k, v, bias) if t is not None]
+        o = dense_attention(*ts, p_drop=p_drop, seed=7, **kw)
+        return (o, *torch.autograd.grad(o, ts, dout.reshape(o.shape)))
+
+    for bb in (bias, None) if b <= 5 else (bias,):
+        got = run(q, k, v, bb, dout)
+        want = run(*(None if t is None else t.float() for t in (q, k, v, bb, dout)), bf16_products=True)
+        for name, x, y in zip(("out", "dq", "dk", "dv", "dbias"), got, want):
+            x, y = x.float(), y.float()
+            assert torch.equal(torch.isfinite(x), torch.isfinite(y)), name
+            e = err(x, y)
+            print("  ", name, f"{e:.1e}", flush=True)
+            # the backward's dout . out is taken from the stored output: bf16 there, float32 here (2^-9 of it more, twice in dq and dk)
+            assert e <= (2 ** -7 if name in ("out", "dv") else 2 ** -6), name

@@ -569,21 +569,22 @@ __device__ __forceinline__ RecLane load_rec_lane(const WaveRec<LPE>& rec) {
 template <typename T, int MODE> constexpr bool rec_edges_early() { return sizeof(T) == 2 || MODE == MODE_FWD; }
 
 // Whether the walk of a long row keeps its queue of gathers filled (walk_range).  The float32 backward has no registers for it (128 with two
-// rows of its own and two gathered ones per edge) and its gathers are masked.
-template <typename T, int MODE> constexpr bool piped_walk() { return sizeof(T) == 2 || MODE == MODE_FWD; }
+// rows of its own and two gathered ones per edge) and its gathers are masked.  Beside dense tiles the rows are short and the queue's registers
+// cost a wave per SIMD: 262 K nodes in clusters of 64, forward + backward 158.7 us step by step, 159.8 as a queue.
+template <typename T, int MODE, bool TILES> constexpr bool piped_walk() { return !TILES && (sizeof(T) == 2 || MODE == MODE_FWD); }
 
 // Walks `len` edges starting at sorted position `start` of node `row` with S edge
 // slots (this lane is slot `slot`, element chunk `el`), reading the plan's sorted view.  On return
 // every lane holds the sums of its own slot (add_slots or reduce_slots adds the slots).
 // FIRST: the edges of the first step came with the wave's record.
-template <typename T, int LPE, int LPH, int S, int MODE, int HASB, bool FIRST>
+template <typename T, int LPE, int LPH, int S, int MODE, int HASB, bool TILES, bool FIRST>
 __device__ __forceinline__ void walk_range(const Common& c, const SideArgs& s, const RecLane& rec, const int row, const int start,
                                            const int len, const int slot, const int el, const bool valid,
                                            Acc& acc) {
     RowRegs<T> rr;
     // HASB == 2: no edge-id array, the bias rows are in this side's own sorted order (row = sorted position)
     constexpr bool ident = HASB == 2;
-    if constexpr (!piped_walk<T, MODE>()) {
+    if constexpr (!piped_walk<T, MODE, TILES>()) {
         load_row<T, LPE, LPH, MODE>(c, row, el, valid, rr, acc);
         const int32_t* __restrict__ col = s.col + start;
         const int32_t* __restrict__ eid = ident ? nullptr : s.eid + start;
@@ -761,7 +762,7 @@ __device__ __forceinline__ void wave_rows(const Common& c, const SideArgs& s, co
     // (the row's own loads below) makes the compiler wait for everything outstanding behind that block - the
     // row's data - before the gathers may go out.
     asm volatile("" ::"v"(row), "v"(start), "v"(len));
-    if ((INLINE && rec_edges_early<T, MODE>()) || (!INLINE && piped_walk<T, MODE>()))
+    if ((INLINE && rec_edges_early<T, MODE>()) || (!INLINE && piped_walk<T, MODE, TILES>()))
         asm volatile("" ::"v"(rec.cols.x), "v"(rec.cols.y), "v"(rec.cols.z), "v"(rec.cols.w), "v"(rec.eids.x), "v"(rec.eids.y),
                      "v"(rec.eids.z), "v"(rec.eids.w));
     if (!valid) { row = 0; start = 0; len = 0; }
@@ -770,7 +771,7 @@ __device__ __forceinline__ void wave_rows(const Common& c, const SideArgs& s, co
     if (TILES) valid = valid && !(len == 0 && s.cover[row] != 0);
     Acc acc;
     if (INLINE) walk_record<T, LPE, LPH, S, MODE, HASB>(c, s, rec, row, start, len, slot, el, valid, acc);
-    else walk_range<T, LPE, LPH, S, MODE, HASB, true>(c, s, rec, row, start, len, slot, el, valid, acc);
+    else walk_range<T, LPE, LPH, S, MODE, HASB, TILES, true>(c, s, rec, row, start, len, slot, el, valid, acc);
     finish_row<T, LPE, LPH, S, MODE, TILES>(c, s, row, slot, el, valid, acc);
 }
 
@@ -943,7 +944,7 @@ __device__ __forceinline__ void block_item(const Common& c, const SideArgs& s, c
     const int lo = min(grp * share, it.len);
     const int hi = min(lo + share, it.len);
     Acc acc;
-    walk_range<T, LPE, LPH, S, MODE, HASB, false>(c, s, RecLane{}, it.row, it.start + lo, hi - lo, slot, el, true, acc);
+    walk_range<T, LPE, LPH, S, MODE, HASB, TILES, false>(c, s, RecLane{}, it.row, it.start + lo, hi - lo, slot, el, true, acc);
     add_slots<LPE, S, MODE>(acc);
     if (slot == 0) {
         float* r = lds.red + grp * STRIDE;
