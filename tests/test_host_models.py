@@ -6,7 +6,7 @@ import types
 import pytest
 import torch
 
-from torchgt_amd import GT, GraphLevelGT, GraphLevelGraphormer, GraphAttnBias
+from torchgt_amd import GT, GraphLevelGT, GraphLevelGraphormer, GraphAttnBias, Graphormer
 from torchgt_amd.graph_level import GraphNodeFeature
 
 
@@ -68,3 +68,40 @@ def test_models_refuse_cpu_tensors():
         GraphLevelGT(1, 8, 64, 0.0, 0.0, 64, "ZINC", "single_hop", 5, 0.0, 1)(batch, attn_type="sparse")
     with pytest.raises(RuntimeError):
         GT(1, 8, 16, 64, 4, 1, 0.0, 0.0, 0.0, 64, 0)(torch.zeros(5, 16), None, torch.zeros(2, 4, dtype=torch.long), attn_type="sparse")
+
+
+@pytest.mark.parametrize("change", ["none", "shared", "none_slot", "own_names", "own_child", "twice", "itself", "extra"])
+def test_parameters_are_the_named_parameters_in_their_order(change):
+    for m in (Graphormer(2, 8, 16, 64, 5, 1, 0.0, 0.0, 0.0, 64, 1), GT(2, 8, 16, 64, 5, 1, 0.0, 0.0, 0.0, 64, 0),
+              GraphLevelGraphormer(2, 8, 64, 0.0, 0.0, 64, "ZINC", "multi_hop", 5, 0.0, 1)):
+        first = m.layers[0]
+        if change == "shared":
+            m.layers[1].extra = torch.nn.Linear(3, 3)
+            m.layers[1].extra.weight = next(first.parameters())
+        if change == "none_slot":
+            first.register_parameter("nothing", None)
+            first.register_module("nobody", None)
+        if change == "own_names":
+            class Mine(type(m)):
+                def named_parameters(self, *a, **k):
+                    return iter(list(super().named_parameters(*a, **k))[:3])
+            m.__class__ = Mine
+        if change == "own_child":
+            class Hidden(torch.nn.Linear):
+                def named_modules(self, *a, **k):
+                    return iter(())
+            first.hidden = Hidden(4, 4)
+        if change == "twice":
+            m.layers.append(first)
+        if change == "itself":
+            first.register_module("up", m)
+        if change == "extra":
+            m.extra = torch.nn.ParameterList([torch.nn.Parameter(torch.zeros(2)), torch.nn.Parameter(torch.zeros(3))])
+        for recurse in (True, False):
+            want = [p for _, p in m.named_parameters(recurse=recurse)]
+            got = list(m.parameters(recurse))
+            assert len(got) == len(want) and all(a is b for a, b in zip(got, want))
+        for p in m.parameters():
+            p.grad = torch.zeros_like(p)
+        m.zero_grad()
+        assert all(p.grad is None for p in m.parameters())

@@ -19,7 +19,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _ext, _lib
-from .module_tree import DROPOUT, all_plain, at_work, kind, model_parameters
+from .module_tree import DROPOUT, OneWalk, all_plain, at_work, kind, model_parameters
 from .multi_head_attention import MultiHeadAttention, attention_modules, fused_linear, plain_attention, _DT
 from .plan import GraphPlan, get_plan
 
@@ -157,7 +157,7 @@ def layer_modules(count, layer):
     return out
 
 
-class Graphormer(nn.Module):
+class Graphormer(OneWalk):
     """Graphormer for node-level tasks, global token at index 0
     (models/graphormer_dist_node_level.py:316-392)."""
 

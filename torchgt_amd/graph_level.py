@@ -13,7 +13,7 @@ from . import _ext, _lib
 from .core_attention import GraphBiasIds
 from .encoder import FFN, LAYER_PARAMETERS, FeedForwardNetwork, init_params, layer_modules
 from .graph_bias import GraphAttnBias, same_gpu
-from .module_tree import DROPOUT, all_plain, at_work, kind, model_parameters
+from .module_tree import DROPOUT, OneWalk, all_plain, at_work, kind, model_parameters
 from .multi_head_attention import MultiHeadAttention, fused_linear, plain_attention
 
 _DT = {torch.float32: _lib.DTYPE_F32, torch.bfloat16: _lib.DTYPE_BF16}
@@ -165,7 +165,7 @@ class EncoderLayer(nn.Module):
 _LAYER, _NODE_FEATURE, _ATTN_BIAS = kind(EncoderLayer), kind(GraphNodeFeature), kind(GraphAttnBias)
 
 
-class Graphormer(nn.Module):
+class Graphormer(OneWalk):
     """Graphormer for graph-level tasks: one graph, one sequence (graphormer_graph_level.py:309-389)."""
 
     def __init__(self, n_layers, num_heads, hidden_dim, dropout_rate, intput_dropout_rate, ffn_dim, dataset_name, edge_type,

@@ -12,7 +12,7 @@ import torch.nn.functional as F
 from . import _ext, _lib
 from .encoder import autocast_to_float32, init_params, padded
 from .graph_bias import same_gpu
-from .module_tree import DROPOUT, kind, model_parameters
+from .module_tree import DROPOUT, OneWalk, kind, model_parameters
 from .multi_head_attention import MultiHeadAttention, attention_modules, fused_linear
 from .plan import GraphPlan, get_plan
 
@@ -85,7 +85,7 @@ class MLPReadout(nn.Module):
 _LAYER, _READOUT = kind(EncoderLayer), kind(MLPReadout)
 
 
-class GT(nn.Module):
+class GT(OneWalk):
     """GT for node-level tasks, no global token (gt_dist_node_level.py:290-341)."""
 
     def __init__(self, n_layers, num_heads, input_dim, hidden_dim, output_dim, attn_bias_dim, dropout_rate,
@@ -193,7 +193,7 @@ class GraphLevelEncoderLayer(EncoderLayer):
         return super().forward(x, attn_bias, edge_index=edge_index, attn_type=attn_type)
 
 
-class GraphLevelGT(nn.Module):
+class GraphLevelGT(OneWalk):
     """GT for graph-level tasks, one sequence per graph (models/gt_graph_level.py:276-363; class ``GT`` there).
     The node rows are the summed embeddings of the integer features, the edges of all graphs of the batch
     index the flattened [b * s] axis, the graph representation is the mean over all s rows (padding included,

@@ -42,6 +42,45 @@ def watched_everywhere():
     return bool(m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks or m._global_backward_pre_hooks)
 
 
+class OneWalk(nn.Module):
+    """``parameters()`` of a model in one walk over its modules.  ``zero_grad``, a gradient clip and a flattening all-reduce each ask for
+    them on every step, and ``nn.Module`` spells out the name of every parameter through a generator per module for it: 92 us for
+    the 72 parameters of four layers, 38 here (half a step of 4 K nodes is host time).  Names are only left out where nobody could
+    see them: a class that brings its own ``named_parameters`` or ``named_modules`` is asked in the general way."""
+
+    def parameters(self, recurse=True):
+        if not recurse or not _plain_names(type(self)):
+            yield from super().parameters(recurse)
+            return
+        seen, parents, known, stack = set(), set(), {type(self)}, [self]
+        while stack:
+            m = stack.pop()
+            own, children = m._parameters, m._modules
+            if children:
+                if id(m) in parents:      # (a leaf that is there twice has nothing new the second time)
+                    continue
+                parents.add(id(m))
+            if own:
+                for p in own.values():
+                    if p is not None and id(p) not in seen:
+                        seen.add(id(p))
+                        yield p
+            if children:
+                for child in reversed(children.values()):
+                    if child is not None:
+                        if type(child) not in known:
+                            if not _plain_names(type(child)):
+                                yield from [q for q in super().parameters() if id(q) not in seen]
+                                return
+                            known.add(type(child))
+                        stack.append(child)
+
+
+def _plain_names(cls):
+    M = nn.Module
+    return cls.named_parameters is M.named_parameters and cls.named_modules is M.named_modules and cls._named_members is M._named_members
+
+
 class ModuleTree:
     """Where a model's parameters are: for the whole-model operators, whose host time is counted in microseconds, the
     attribute look-ups of seventy parameters through ``nn.Module`` would be a third of it.  Remembers the dictionaries of the
