@@ -76,6 +76,36 @@ def test_graph_node_feature_matches_oracle(cuda, dtype, C, Fx, num_atoms, num_de
             assert not a[0].any()
 
 
+# Table gradients in LDS (one to four copies, runs of rows that end inside eight, token rows in any place of a run, more channels than lanes)
+# and beyond it.  Sums of up to n float32 terms in another order: n 2^-24 of the sum of their magnitudes; bf16 results round once more.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("b,s,C,Fx,atoms,deg", [(1, 1, 64, 1, 64, 64), (5, 7, 64, 1, 64, 64), (3, 8, 40, 2, 9, 5), (40, 9, 64, 1, 64, 64), (7, 128, 64, 3, 64, 64),
+                                                (300, 20, 64, 1, 30, 20), (2, 30, 128, 1, 200, 40), (2, 30, 128, 1, 230, 40), (3, 11, 200, 1, 20, 10)])
+def test_node_feature_gradients_at_every_size_of_tables(cuda, b, s, C, Fx, atoms, deg, dtype):
+    print(f"node feature gradients b={b} s={s} C={C} Fx={Fx} tables {atoms} / {deg} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(b + s)
+    m = GraphNodeFeature(8, atoms, deg, deg + 1, C).to(cuda, dtype)
+    ids = lambda n, *shape: torch.randint(-1, n + 1, shape, generator=g)      # the ends are clamped
+    x, ind, outd = ids(atoms, b, s, Fx), ids(deg, b, s), ids(deg + 1, b, s)
+    batch = types.SimpleNamespace(x=x.to(cuda), in_degree=ind.to(cuda), out_degree=outd.to(cuda))
+    dout = torch.randn(b, s + 1, C, generator=g).to(dtype)
+    tables = [m.atom_encoder.weight, m.in_degree_encoder.weight, m.out_degree_encoder.weight, m.graph_token.weight]
+    got = torch.autograd.grad(m(batch), tables, dout.to(cuda))
+    d = dout.double()
+    for name, t, i in zip(("atom", "in", "out"), got, (x, ind.unsqueeze(-1), outd.unsqueeze(-1))):
+        n = t.shape[0]
+        want, size = torch.zeros(n, C, dtype=torch.double), torch.zeros(n, C, dtype=torch.double)
+        for f in range(i.shape[-1]):
+            at = i[..., f].clamp(0, n - 1).reshape(-1)
+            want.index_add_(0, at, d[:, 1:].reshape(-1, C))
+            size.index_add_(0, at, d[:, 1:].abs().reshape(-1, C))
+        want[0] = size[0] = 0                           # padding
+        bound = size * (b * s * Fx * 2.0 ** -24) + want.abs() * (2.0 ** -8 if dtype == torch.bfloat16 else 0)
+        assert ((t.double().cpu() - want).abs() <= bound).all(), name
+    want, size = d[:, 0].sum(0), d[:, 0].abs().sum(0)
+    assert ((got[3].double().cpu().view(-1) - want).abs() <= size * (b * 2.0 ** -24) + want.abs() * (2.0 ** -8 if dtype == torch.bfloat16 else 0)).all()
+
+
 def test_graph_node_feature_empty_batch_and_bad_arguments(cuda):
     m = GraphNodeFeature(8, 64, 64, 64, 64).to(cuda)
     out = m(types.SimpleNamespace(x=torch.zeros(0, 5, 1, dtype=torch.long, device=cuda),

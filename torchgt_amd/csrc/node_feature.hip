@@ -6,14 +6,15 @@
 //                      + out_degree_table[out_degree[g, i]]
 //
 // The reference runs three embedding lookups, a sum over the features, two adds, a repeat and a
-// concatenation; here one kernel reads the ids and writes every output row once.  The backward adds
-// the output gradient into float copies of the tables with vector-memory atomics (row 0 of the three
-// lookup tables is the padding index and gets none) and a last kernel hands the sums over in the
-// caller's type: results agree to rounding between runs, not bit for bit.  With a few dozen atom types every
-// table row is shared by hundreds of node rows and atomics on one address serialise (55 us for the 33 K rows of
-// 256 padded graphs; summing a workgroup's share in LDS first costs the same, the LDS float atomics of a CU
-// serialise likewise), so neighbouring workgroups add into different copies of the sums (up to 64, at most 16 MB
-// in all) that the last kernel adds up: 21 us.
+// concatenation; here one kernel reads the ids and writes every output row once.  The backward adds the output gradient
+// into float copies of the tables (row 0 of the three lookup tables is the padding index and gets none) and a
+// last kernel adds the copies up and hands the sums over in the caller's type.
+//
+// With a few dozen atom types every table row is shared by hundreds of node rows, and atomics on one address serialise
+// (55 us for the 33 K rows of 256 padded graphs into one copy, 43 with the fill into 64, in LDS as slow as in memory).  Tables that
+// fit a workgroup's LDS are summed there without atomics: a wave has a table to itself.  Larger ones are added to
+// with vector-memory atomics, neighbouring workgroups into different copies (up to 64, at most 16 MB in all): their results agree to
+// rounding between runs, not bit for bit.
 #include "common.h"
 #include <algorithm>
 
@@ -119,8 +120,89 @@ __global__ __launch_bounds__(256) void k_node_feature_bwd(NodeFeatArgs a, const 
     if (row < n_rows) node_feature_bwd_row(a, dout, row, threadIdx.x % 64, acc + (blockIdx.x % copies) * n_acc);
 }
 
+// Tables in LDS.  A workgroup takes a run of rows for all tables: wave w adds the rows of set w / tables to that set's copy of table w % tables,
+// lane = channel, so nobody else writes there and the sums come in row order.  Bound by that chain, one LDS read, add and write per row, and
+// by the loads in front of it, eight rows at a time.  33 K rows of 64 channels, tables of 64 + 64 + 64 + 1 rows: 20 us, and 5
+// for the sum of 256 copies; with atomics 33, 6 for their fill and 4.
+constexpr int kFeatRows = 16, kFeatSets = 4;
+template <typename T>
+__global__ __launch_bounds__(64 * 3 * kFeatSets) void k_node_feature_bwd_lds(NodeFeatArgs a, const T* __restrict__ dout, float* __restrict__ partial,
+                                                                             int n_acc, int tables, int sets) {
+    extern __shared__ __align__(16) float sums[];      // [sets][n_acc]
+    const bool fours = n_acc % 4 == 0;
+    if (fours) {
+#pragma unroll 4
+        for (int i = threadIdx.x; i < sets * n_acc / 4; i += blockDim.x) reinterpret_cast<float4*>(sums)[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    } else
+        for (int i = threadIdx.x; i < sets * n_acc; i += blockDim.x) sums[i] = 0.f;
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), table = wave % tables, set = wave / tables;
+    float* mine = sums + set * n_acc;
+    float* token = mine + (a.num_atoms + a.num_in + a.num_out) * a.C;
+    const int64_t* ids = a.x;
+    int F = a.Fx, num = a.num_atoms, least = a.pad_rows;
+    if (table == 1) { ids = a.in_degree; F = 1; num = a.num_in; least = 1; mine += a.num_atoms * a.C; }
+    if (table == 2) { ids = a.out_degree; F = 1; num = a.num_out; least = 1; mine += (a.num_atoms + a.num_in) * a.C; }
+    if (a.s == 0) F = 0;      // token rows only
+    const int rows = a.s + a.has_token, n_rows = a.b * rows, per = (n_rows + gridDim.x - 1) / gridDim.x;
+    const int r0 = per * blockIdx.x, r1 = min(r0 + per, n_rows), last = a.b * a.s - 1;
+    // every load of eight rows is asked for before the first is used, also where there is nothing to add (another row's is read then)
+    for (int row = r0 + kFeatRows * set; row < r1; row += kFeatRows * sets) {
+        const int g0 = (uint32_t)row / (uint32_t)rows;
+        int at = row - g0 * rows, p = g0 * a.s + at - a.has_token;      // the row's place in its graph, the position of its ids
+        int pos[kFeatRows];
+        bool node[kFeatRows];
+#pragma unroll
+        for (int u = 0; u < kFeatRows; ++u) {
+            node[u] = !(a.has_token && at == 0);
+            pos[u] = max(0, min(p, last));
+            at = at + 1 == rows ? 0 : at + 1;
+            p += !(a.has_token && at == 0);
+        }
+        for (int c = lane; c < a.C; c += 64) {
+            float d[kFeatRows];
+#pragma unroll
+            for (int u = 0; u < kFeatRows; ++u) d[u] = ldf(dout + (int64_t)min(row + u, r1 - 1) * a.C + c);
+            for (int f = 0; f < F; ++f) {
+                int64_t id[kFeatRows];
+#pragma unroll
+                for (int u = 0; u < kFeatRows; ++u) id[u] = ids[(int64_t)pos[u] * F + f];
+#pragma unroll
+                for (int u = 0; u < kFeatRows; ++u) {
+                    const int to = clamp_id(id[u], num);
+                    if (row + u < r1 && node[u] && to >= least) mine[to * a.C + c] += d[u];
+                }
+            }
+            if (table == 0) {
+#pragma unroll
+                for (int u = 0; u < kFeatRows; ++u)
+                    if (row + u < r1 && !node[u]) token[c] += d[u];
+            }
+        }
+    }
+    __syncthreads();
+    float* __restrict__ out = partial + (int64_t)blockIdx.x * n_acc;
+    if (fours) {
+#pragma unroll 2
+        for (int i = threadIdx.x; i < n_acc / 4; i += blockDim.x) {
+            float4 t[kFeatSets];
+#pragma unroll
+            for (int k = 0; k < kFeatSets; ++k) t[k] = reinterpret_cast<const float4*>(sums)[(k < sets ? k : 0) * (n_acc / 4) + i];
+#pragma unroll
+            for (int k = 1; k < kFeatSets; ++k)
+                if (k < sets) { t[0].x += t[k].x; t[0].y += t[k].y; t[0].z += t[k].z; t[0].w += t[k].w; }
+            reinterpret_cast<float4*>(out)[i] = t[0];
+        }
+    } else
+        for (int i = threadIdx.x; i < n_acc; i += blockDim.x) {
+            float t = sums[i];
+            for (int k = 1; k < sets; ++k) t += sums[k * n_acc + i];
+            out[i] = t;
+        }
+}
+
 // Sum of the copies, handed over in the caller's type.  64 entries per workgroup along the lanes; the four waves take
-// every fourth copy each (four loads in flight per lane) and their partial sums are added in wave order.
+// every fourth copy each (sixteen loads in flight per lane) and their partial sums are added in wave order.
 template <typename T>
 __global__ __launch_bounds__(256) void k_node_feature_finish(const float* __restrict__ acc, int64_t n_atom, int64_t n_in,
                                                              int64_t n_out, int64_t n_tok, int copies, T* __restrict__ d_atom,
@@ -131,11 +213,12 @@ __global__ __launch_bounds__(256) void k_node_feature_finish(const float* __rest
     const int64_t t = (int64_t)blockIdx.x * 64 + lane;
     float v = 0.f;
     if (t < n_acc) {
-        for (int c0 = wave; c0 < copies; c0 += 16) {
-            float x[4];
+        for (int c0 = wave; c0 < copies; c0 += 64) {
+            float x[16];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) x[u] = c0 + 4 * u < copies ? acc[(int64_t)(c0 + 4 * u) * n_acc + t] : 0.f;
-            v += (x[0] + x[1]) + (x[2] + x[3]);
+            for (int u = 0; u < 16; ++u) x[u] = c0 + 4 * u < copies ? acc[(int64_t)(c0 + 4 * u) * n_acc + t] : 0.f;
+#pragma unroll
+            for (int u = 0; u < 16; u += 4) v += (x[u] + x[u + 1]) + (x[u + 2] + x[u + 3]);
         }
     }
     part[wave][lane] = v;
@@ -148,8 +231,13 @@ __global__ __launch_bounds__(256) void k_node_feature_finish(const float* __rest
     else stf(d_tok + (t - n_atom - n_in - n_out), v);
 }
 
-// Copies of the float sums the backward spreads its atomics over: as many as stay under 16 MB in all, at most 64.
+// Copies of the tables that a workgroup's LDS holds (0: none): up to four, at less than a CU's 160 KB
+// (rows are counted in 32 bits there)
+inline int node_feat_sets(int64_t n_acc) { return (int)std::min<int64_t>(kFeatSets, (156 << 10) / (n_acc * (int64_t)sizeof(float))); }
+// Copies of the float sums in memory.  From LDS: one per workgroup, a workgroup per CU at most.  With atomics: as many as stay under 16 MB in
+// all, at most 64.
 inline int node_feat_copies(int64_t n_acc) {
+    if (node_feat_sets(n_acc) > 0) return num_cus();
     int copies = 64;
     while (copies > 1 && n_acc * copies * (int64_t)sizeof(float) > (16 << 20)) copies /= 2;
     return copies;
@@ -195,23 +283,37 @@ int node_feature_bwd_impl(NodeFeatArgs a, const void* d_dout, int dtype, void* d
     const int64_t n_acc = n_atom + n_in + n_out + n_tok;
     if (!a.has_degree) a.num_in = a.num_out = 0;          // the kernel's offsets of the sums that follow the atom table
     const int64_t n_rows = (int64_t)a.b * (a.s + a.has_token);
-    const int64_t total = n_rows * a.C;
+    int copies = node_feat_copies(n_acc);
+    if (const int sets = node_feat_sets(n_acc); sets > 0 && n_rows + kFeatRows * kFeatSets <= INT32_MAX) {
+        // a workgroup for every eight rows of each set, at most one per copy
+        copies = (int)std::min<int64_t>(copies, (n_rows + kFeatRows * sets - 1) / (kFeatRows * sets));
+        if (copies > 0) {
+            const int tables = a.has_degree ? 3 : 1, lds = (int)(sets * n_acc * sizeof(float));
+            static std::atomic<uint64_t> done[2];
+            const auto run = [&](auto kernel, const auto* dout, std::atomic<uint64_t>& d) {
+                if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), 156 << 10, d)) return rc;
+                hipLaunchKernelGGL(kernel, dim3(copies), dim3(64 * tables * sets), lds, st, a, dout, acc, (int)n_acc, tables, sets);
+                return (int)TGT_OK;
+            };
+            const int rc = dtype == TGT_DTYPE_F32 ? run(&k_node_feature_bwd_lds<float>, (const float*)d_dout, done[0])
+                                                  : run(&k_node_feature_bwd_lds<nbf16>, (const nbf16*)d_dout, done[1]);
+            if (rc != TGT_OK) return rc;
+        }
+    } else {
+        hipLaunchKernelGGL(k_fill_zero, dim3((unsigned)((n_acc * copies + 255) / 256)), dim3(256), 0, st, acc, n_acc * copies);
+        const dim3 grid((unsigned)((n_rows + 3) / 4));
+        if (n_rows > 0) {
+            if (dtype == TGT_DTYPE_F32) hipLaunchKernelGGL((k_node_feature_bwd<float>), grid, dim3(256), 0, st, a, (const float*)d_dout, acc, copies, n_acc);
+            else hipLaunchKernelGGL((k_node_feature_bwd<nbf16>), grid, dim3(256), 0, st, a, (const nbf16*)d_dout, acc, copies, n_acc);
+        }
+    }
     const dim3 fgrid((unsigned)((n_acc + 63) / 64));
-    const int copies = node_feat_copies(n_acc);
-    hipLaunchKernelGGL(k_fill_zero, dim3((unsigned)((n_acc * copies + 255) / 256)), dim3(256), 0, st, acc, n_acc * copies);
-    if (dtype == TGT_DTYPE_F32) {
-        if (total > 0)
-            hipLaunchKernelGGL((k_node_feature_bwd<float>), dim3((unsigned)((n_rows + 3) / 4)), dim3(256), 0, st, a,
-                               (const float*)d_dout, acc, copies, n_acc);
+    if (dtype == TGT_DTYPE_F32)
         hipLaunchKernelGGL((k_node_feature_finish<float>), fgrid, dim3(256), 0, st, (const float*)acc, n_atom, n_in, n_out, n_tok, copies,
                            (float*)d_datom, (float*)d_din, (float*)d_dout_table, (float*)d_dtoken);
-    } else {
-        if (total > 0)
-            hipLaunchKernelGGL((k_node_feature_bwd<nbf16>), dim3((unsigned)((n_rows + 3) / 4)), dim3(256), 0, st, a,
-                               (const nbf16*)d_dout, acc, copies, n_acc);
+    else
         hipLaunchKernelGGL((k_node_feature_finish<nbf16>), fgrid, dim3(256), 0, st, (const float*)acc, n_atom, n_in, n_out, n_tok, copies,
                            (nbf16*)d_datom, (nbf16*)d_din, (nbf16*)d_dout_table, (nbf16*)d_dtoken);
-    }
     TGT_HIP_CHECK(hipGetLastError());
     return TGT_OK;
 }
