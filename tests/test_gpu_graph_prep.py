@@ -131,6 +131,17 @@ def test_gen_sub_edge_index_matches_oracle(cuda):
     _check_sub(e, np.arange(n), n, cuda)                     # the whole graph: every edge survives
 
 
+# Members' bits: whole and part words and vectors, the last node count whose bits fit LDS and the first beyond; tiles of 1024 items that end
+# inside, at and behind the edge list; more tiles than waves in one round
+@pytest.mark.parametrize("N,E,S", [(1, 0, 1), (1, 5, 1), (31, 1023, 9), (32, 992, 32), (33, 1024, 33), (127, 897, 60), (128, 896, 1), (129, 5000, 70), (4097, 300000, 900),
+                                   (1 << 20, 2049, 700000), ((1 << 20) + 1, 2049, 700000), ((1 << 20) + 129, 4500000, 300000)])
+def test_sub_edge_index_at_the_edges_of_its_bits_and_tiles(cuda, N, E, S):
+    print(f"sub graph N={N} E={E} S={S}", flush=True)
+    rng = np.random.default_rng(N + E)
+    e = rng.integers(0, N, size=(2, E))
+    _check_sub(e, rng.integers(0, N, size=S), N, cuda)
+
+
 def test_gen_sub_edge_index_errors(cuda):
     e = torch.tensor([[0, 1], [1, 7]], device=cuda)
     with pytest.raises(_lib.TorchGTHipError) as ei:

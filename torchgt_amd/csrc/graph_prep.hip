@@ -413,83 +413,112 @@ __global__ void k_batch_rows(const int64_t* __restrict__ sorted, int64_t N, cons
 // self-loops.  A node that occurs more than once in idx_batch takes its LAST
 // position (what the sequential index assignment n_idx[subset] = arange gives).
 // ---------------------------------------------------------------------------
-constexpr int kSubItems = 1024;     // items per workgroup of the compaction (4 rounds of 256)
+constexpr int kSubItems = 1024;     // items of a tile of the compaction
 
-__global__ void k_sub_fill(int32_t* __restrict__ pos, int64_t N, int* __restrict__ bad) {
+__global__ void k_sub_fill(int32_t* __restrict__ pos, int64_t N, uint32_t* __restrict__ member, int64_t words, int* __restrict__ bad) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i == 0) *bad = 0;
     if (i < N) pos[i] = -1;
+    if (i < words) member[i] = 0;
 }
 
+// member: one bit per node of the batch
 __global__ void k_sub_positions(const int64_t* __restrict__ idx, int64_t S, int64_t N, int32_t* __restrict__ pos,
-                                int* __restrict__ bad) {
+                                uint32_t* __restrict__ member, int* __restrict__ bad) {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= S) return;
     const int64_t v = idx[p];
     if (v < 0 || v >= N) { atomicOr(bad, 1); return; }
     atomicMax(&pos[v], (int32_t)p);
+    atomicOr(&member[v >> 5], 1u << (v & 31));
 }
 
-// item i < E: edge i; item E + v: self-loop of node v.  Returns the renamed endpoints.
-__device__ __forceinline__ bool sub_item(const int64_t* __restrict__ ei, int64_t E, int64_t N,
-                                         const int32_t* __restrict__ pos, int64_t i, int32_t& a, int32_t& b,
-                                         int* __restrict__ bad) {
-    if (i < E) {
-        const int64_t s = ei[i], d = ei[E + i];
-        if (s < 0 || s >= N || d < 0 || d >= N) { atomicOr(bad, 2); return false; }
-        if (s == d) return false;
-        a = pos[s]; b = pos[d];
-        return a >= 0 && b >= 0;
+// The endpoints of item i (< E: edge i; E + v: the self-loop of node v).  An index past the end reads the last item's.
+__device__ __forceinline__ void sub_ends(const int64_t* __restrict__ ei, int64_t E, int64_t total, int64_t i, int64_t& s, int64_t& d) {
+    i = min(i, total - 1);
+    const bool edge = i < E;
+    const int64_t at = edge ? i : 0;
+    if (E > 0) { s = ei[at]; d = ei[E + at]; }
+    if (!edge) s = d = i - E;
+}
+
+// First pass: the kept items of every tile of kSubItems, as one bit per item and their number.  A wave takes a tile.  Two look-ups in a random place
+// for every edge are what this pass waits for when they go to the position table (a request to L2 per lane: 35 us for 3.1 M edges and
+// 256 K nodes, whose 16 bytes per edge take 10); whether a node is in the batch is one bit, and the bits of up to 1 M nodes stay in a
+// CU's LDS (IN_LDS): 15 us.  The loads of eight rounds go out before the first is used.
+constexpr int kSubWords = kSubItems / 64, kSubRounds = 8, kSubWaves = 16;
+template <bool IN_LDS>
+__global__ __launch_bounds__(64 * kSubWaves) void k_sub_mark(const int64_t* __restrict__ ei, int64_t E, int64_t N, const uint32_t* __restrict__ member,
+                                                             int words, int tiles, uint32_t* __restrict__ counts, uint64_t* __restrict__ keep_bits,
+                                                             int* __restrict__ bad) {
+    extern __shared__ __align__(16) uint32_t in_lds[];
+    if (IN_LDS) {
+        for (int i = threadIdx.x; i < words / 4; i += 64 * kSubWaves) reinterpret_cast<uint4*>(in_lds)[i] = reinterpret_cast<const uint4*>(member)[i];
+        __syncthreads();
     }
-    a = b = pos[i - E];
-    return a >= 0;
-}
-
-// pass 0 counts the kept items of every workgroup; pass 1 writes them behind the
-// workgroup's offset, in item order (ballot ranks inside a wave, wave totals in LDS).
-template <int PASS>
-__global__ __launch_bounds__(256) void k_sub_compact(const int64_t* __restrict__ ei, int64_t E, int64_t N,
-                                                     const int32_t* __restrict__ pos, uint32_t* __restrict__ counts,
-                                                     uint64_t* __restrict__ keep_bits, int64_t* __restrict__ out,
-                                                     int64_t capacity, int* __restrict__ bad) {
-    __shared__ uint32_t wave_n[4];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t* bits = IN_LDS ? in_lds : member;
+    const int lane = threadIdx.x & 63;
     const int64_t total = E + N;
-    uint32_t run = PASS ? counts[blockIdx.x] : 0u;          // pass 1: exclusive prefix of this workgroup
-    for (int round = 0; round < kSubItems / 256; ++round) {
-        const int64_t i = (int64_t)blockIdx.x * kSubItems + round * 256 + threadIdx.x;
-        int32_t a = 0, b = 0;
-        // one keep bit per item, a 64-bit word per wave and round: the writing pass reads the words and
-        // looks at the endpoints of the kept items only (a few per cent of the edge list)
-        const int64_t word = ((int64_t)blockIdx.x * (kSubItems / 256) + round) * 4 + wave;
-        bool keep;
-        uint64_t m;
-        if (PASS == 0) {
-            keep = i < total && sub_item(ei, E, N, pos, i, a, b, bad);
-            m = __ballot(keep);
-            if (lane == 0) keep_bits[word] = m;
-        } else {
-            m = keep_bits[word];
-            keep = (m >> lane) & 1ull;
-            if (keep) (void)sub_item(ei, E, N, pos, i, a, b, bad);
-        }
-        if (lane == 0) wave_n[wave] = (uint32_t)__popcll(m);
-        __syncthreads();
-        uint32_t before = 0, all = 0;
+    for (int tile = blockIdx.x * kSubWaves + (threadIdx.x >> 6); tile < tiles; tile += gridDim.x * kSubWaves) {
+        uint64_t mine = 0;      // lane w: word w
+        uint32_t kept = 0;
+#pragma unroll 1
+        for (int r0 = 0; r0 < kSubWords; r0 += kSubRounds) {
+            const int64_t i0 = (int64_t)tile * kSubItems + r0 * 64 + lane;
+            int64_t s[kSubRounds], d[kSubRounds];
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            if (w < wave) before += wave_n[w];
-            all += wave_n[w];
+            for (int r = 0; r < kSubRounds; ++r) sub_ends(ei, E, total, i0 + r * 64, s[r], d[r]);
+#pragma unroll
+            for (int r = 0; r < kSubRounds; ++r) {
+                const int64_t i = i0 + r * 64;
+                const bool in = s[r] >= 0 && s[r] < N && d[r] >= 0 && d[r] < N;
+                if (!in && i < E) atomicOr(bad, 2);
+                const uint32_t a = bits[in ? s[r] >> 5 : 0] >> (s[r] & 31), b = bits[in ? d[r] >> 5 : 0] >> (d[r] & 31);
+                const uint64_t m = __ballot(in && i < total && (a & b & 1u) && (i >= E || s[r] != d[r]));
+                mine = lane == r0 + r ? m : mine;
+                kept += (uint32_t)__popcll(m);
+            }
         }
-        if (PASS && keep) {
-            const int64_t o = (int64_t)run + before + __popcll(m & ((1ull << lane) - 1ull));
-            out[o] = a;
-            out[capacity + o] = b;
-        }
-        run += all;
-        __syncthreads();
+        if (lane < kSubWords) keep_bits[(int64_t)tile * kSubWords + lane] = mine;
+        if (lane == 0) counts[tile] = kept;
     }
-    if (!PASS && threadIdx.x == 0) counts[blockIdx.x] = run;
+}
+
+// Second pass: the kept items in item order, behind the tile's offset.  Every wave of a tile's workgroup reads all of its words, a lane each,
+// whose prefix is where a word's items go; only kept items look at their endpoints and positions.
+__global__ __launch_bounds__(256) void k_sub_write(const int64_t* __restrict__ ei, int64_t E, int64_t N, const int32_t* __restrict__ pos,
+                                                   const uint32_t* __restrict__ offsets, const uint64_t* __restrict__ keep_bits,
+                                                   int64_t* __restrict__ out, int64_t capacity) {
+    constexpr int kRounds = kSubWords / 4;      // words of a wave: wave, 4 + wave, ...
+    static_assert(kSubWords % 4 == 0 && kSubWords <= 64, "a lane per word");
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t total = E + N, item0 = (int64_t)blockIdx.x * kSubItems + threadIdx.x;
+    const uint64_t mine = lane < kSubWords ? keep_bits[(int64_t)blockIdx.x * kSubWords + lane] : 0ull;
+    const uint32_t n = (uint32_t)__popcll(mine);
+    uint32_t before = n;      // kept items up to this lane's word
+#pragma unroll
+    for (int off = 1; off < kSubWords; off <<= 1) {
+        const uint32_t x = __shfl_up(before, off);
+        if (lane >= off) before += x;
+    }
+    before += offsets[blockIdx.x] - n;
+    int64_t s[kRounds], d[kRounds];
+    uint64_t m[kRounds];
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+        m[r] = __shfl(mine, 4 * r + wave);
+        s[r] = d[r] = -1;
+        if ((m[r] >> lane) & 1ull) sub_ends(ei, E, total, item0 + r * 256, s[r], d[r]);
+    }
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+        const uint32_t first = __shfl(before, 4 * r + wave);
+        if (s[r] >= 0) {
+            const int64_t o = (int64_t)first + __popcll(m[r] & ((1ull << lane) - 1ull));
+            out[o] = pos[s[r]];
+            out[capacity + o] = pos[d[r]];
+        }
+    }
 }
 
 // exclusive prefix of the workgroup counts in place (one workgroup), total to counts[n]
@@ -521,17 +550,32 @@ static int sub_edge_index_impl(const int64_t* d_ei, int64_t E, int64_t N, const 
                                int64_t* d_out, int64_t capacity, bool packed, int64_t* h_num, hipStream_t st) {
     const int64_t total = E + N;
     const int nblocks = (int)((total + kSubItems - 1) / kSubItems);
-    DevBuf pos, counts, bits;      // counts: per workgroup, their total, the error flag
+    const int64_t words = (N + 127) / 128 * 4;      // of the members' bits, in whole vectors
+    DevBuf pos, counts, bits, member;      // counts: per tile, their total, the error flag
     TGT_HIP_CHECK(pos.alloc(sizeof(int32_t) * (size_t)N, st));
     TGT_HIP_CHECK(counts.alloc(sizeof(uint32_t) * (size_t)(nblocks + 2), st));
-    TGT_HIP_CHECK(bits.alloc(sizeof(uint64_t) * (size_t)nblocks * (kSubItems / 64), st));
+    TGT_HIP_CHECK(bits.alloc(sizeof(uint64_t) * (size_t)nblocks * kSubWords, st));
+    TGT_HIP_CHECK(member.alloc(sizeof(uint32_t) * (size_t)words, st));
     int* const bad = counts.as<int>() + nblocks + 1;
-    hipLaunchKernelGGL(k_sub_fill, dim3(nblk(N)), dim3(256), 0, st, pos.as<int32_t>(), N, bad);
+    hipLaunchKernelGGL(k_sub_fill, dim3(nblk(std::max(N, words))), dim3(256), 0, st, pos.as<int32_t>(), N, member.as<uint32_t>(), words, bad);
     if (S > 0)
         hipLaunchKernelGGL(k_sub_positions, dim3(nblk(S)), dim3(256), 0, st, d_idx, S, N, pos.as<int32_t>(),
-                           bad);
-    hipLaunchKernelGGL((k_sub_compact<0>), dim3(nblocks), dim3(256), 0, st, d_ei, E, N, pos.as<int32_t>(),
-                       counts.as<uint32_t>(), bits.as<uint64_t>(), (int64_t*)nullptr, (int64_t)0, bad);
+                           member.as<uint32_t>(), bad);
+    {
+        // a workgroup per CU; with the bits elsewhere (more than 1 M nodes) twice as many waves cover the requests
+        constexpr int kMost = 128 << 10;
+        const bool in_lds = words * (int64_t)sizeof(uint32_t) <= kMost;
+        const int grid = (int)std::min<int64_t>((int64_t)num_cus() * (in_lds ? 1 : 2), (nblocks + kSubWaves - 1) / kSubWaves);
+        static std::atomic<uint64_t> done;
+        const auto run = [&](auto kernel, int lds) {
+            hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * kSubWaves), lds, st, d_ei, E, N, (const uint32_t*)member.as<uint32_t>(), (int)words, nblocks,
+                               counts.as<uint32_t>(), bits.as<uint64_t>(), bad);
+        };
+        if (in_lds) {
+            if (int rc = allow_lds(reinterpret_cast<const void*>(&k_sub_mark<true>), kMost, done)) return rc;
+            run(&k_sub_mark<true>, (int)(words * sizeof(uint32_t)));
+        } else run(&k_sub_mark<false>, 0);
+    }
     hipLaunchKernelGGL(k_sub_scan, dim3(1), dim3(256), 0, st, counts.as<uint32_t>(), nblocks);
     TGT_HIP_CHECK(hipGetLastError());
     uint32_t back[2] = {0, 0};
@@ -549,8 +593,8 @@ static int sub_edge_index_impl(const int64_t* d_ei, int64_t E, int64_t N, const 
         return TGT_ERR_WORKSPACE;
     }
     if (n_keep > 0) {
-        hipLaunchKernelGGL((k_sub_compact<1>), dim3(nblocks), dim3(256), 0, st, d_ei, E, N, pos.as<int32_t>(),
-                           counts.as<uint32_t>(), bits.as<uint64_t>(), d_out, packed ? (int64_t)n_keep : capacity, bad);
+        hipLaunchKernelGGL(k_sub_write, dim3(nblocks), dim3(256), 0, st, d_ei, E, N, pos.as<int32_t>(),
+                           counts.as<uint32_t>(), bits.as<uint64_t>(), d_out, packed ? (int64_t)n_keep : capacity);
         TGT_HIP_CHECK(hipGetLastError());
     }
     return TGT_OK;
