@@ -69,6 +69,15 @@ def test_plan_config1_and_config2_graphs(cuda):
     _check_plan(e2, n2, cuda)
 
 
+# Tiles of 1024 and of 4096 keys: one that ends inside, at and behind a tile, the largest sort of small tiles (eight per CU, two views) and the
+# first of large ones
+def test_plan_at_the_edges_of_the_sorts_tiles(cuda):
+    rng = np.random.default_rng(3)
+    few = 4 * torch.cuda.get_device_properties(cuda).multi_processor_count * 1024
+    for N, E in ((40, 1023), (40, 1024), (40, 1025), (300, 2049), (5000, few), (5000, few + 1), (70000, few - 1), (70000, few + 4096)):
+        _check_plan(rng.integers(0, N, (2, E)), N, cuda)
+
+
 def test_plan_three_radix_passes(cuda):
     # N > 65536 needs three 8-bit passes; ids spread over the whole range
     rng = np.random.default_rng(2)

@@ -352,9 +352,10 @@ __host__ __device__ inline int32_t run_waves(uint32_t kind, int32_t n, int lpe) 
 // in turn (layout: WaveRec in common.h), the lanes of a wave one edge or bias row each.  Wave lw of
 // XCD x's list is wave lw % 4 of that XCD's (lw / 4)-th workgroup, and workgroup b of the launch runs on XCD b mod 8:
 // record ((lw / 4) * 8 + x) * 4 + lw % 4.  Everything a kernel uses of a record is written: no clearing pass.
-// Bound by the two dependent reads (item, edges) of a record; 390 K edges: 27 us for each of the two launches with four waves
-// per run and eight lanes at work.
-constexpr int kRecordWaves = 16;
+// Bound by the two dependent reads (item, edges) of a record, which the waves of a long run repeat: four records of a wave are asked for
+// together (64 K nodes, 0.53 M edges, 57 K records in 4.2 K runs of mostly 8 to 32: sixteen waves and one record at a time 33 us, four waves and four
+// records 23).
+constexpr int kRecordWaves = 4, kRecordStep = 4;
 __global__ __launch_bounds__(64 * kRecordWaves) void k_build_records(const Run* __restrict__ runs, const Item* __restrict__ items_d,
                                                        const Item* __restrict__ items_s, const Item* __restrict__ bitems_d,
                                                        const Item* __restrict__ bitems_s, const int32_t* __restrict__ col_d,
@@ -372,41 +373,73 @@ __global__ __launch_bounds__(64 * kRecordWaves) void k_build_records(const Run* 
     const int ipw = kind < (uint32_t)kNumClass ? rows_per_wave(lpe, (int)kind) : 1;
     const int S = kind < (uint32_t)kNumClass ? slots_for_class(lpe, (int)kind) : 1;
     const int groups = kWave / lpe, waves = run_waves(kind, run.n, lpe);
-    for (int w = threadIdx.x >> 6; w < waves; w += kRecordWaves) {
+    const auto record = [&](int w) {
         const int lw = run.wave0 + w;
-        int32_t* out = recs + (((int64_t)(lw >> 2) * 8 + xcd) * 4 + (lw & 3)) * L.stride;
-        if (kind == kDescNone) {
-            if (t == 0) out[0] = (int32_t)kDescNone;
-            continue;
-        }
-        if (kind == kDescBlock) {
-            if (t == 0) {
+        return recs + (((int64_t)(lw >> 2) * 8 + xcd) * 4 + (lw & 3)) * L.stride;
+    };
+    if (kind >= (uint32_t)kNumClass) {
+        for (int w = threadIdx.x >> 6; w < waves; w += kRecordWaves) {
+            int32_t* out = record(w);
+            if (t != 0) continue;
+            if (kind == kDescNone) out[0] = (int32_t)kDescNone;
+            else {
                 const Item it = (src ? bitems_s : bitems_d)[run.first];
                 out[0] = (int32_t)desc_code(kDescBlock, src, 0);
                 out[4] = it.row; out[5] = it.start; out[6] = it.len; out[7] = it.part;
             }
-            continue;
         }
-        const int first = run.first + w * ipw;
-        const int count = min(ipw, run.n - w * ipw);
-        if (t == 0) out[0] = (int32_t)desc_code(kind, src, (uint32_t)count);
-        if (t < groups) {                               // every lane group's entries, zeros behind the last row
-            const int i = t / S;
-            Item it{0, 0, 0, -1};
-            if (i < count) it = items[first + i];
-            out[L.off_row + t] = it.row;                // per lane group: a lane finds its row without knowing the class
-            out[L.off_start + t] = it.start;
-            out[L.off_len + t] = it.len;
+        return;
+    }
+    // the row of lane group g in the wave w; nothing behind the wave's last row (an item of it is read all the same)
+    const auto row_of = [&](int w, int g) {
+        const int i = g / S, last = run.n - 1 - w * ipw;
+        Item it = items[run.first + w * ipw + min(i, last)];
+        if (i > last) it = Item{0, 0, 0, -1};
+        return it;
+    };
+    const auto step = [&](int w0, auto records) {
+        constexpr int U = decltype(records)::value;
+        int32_t* out[U];
+        int wave[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            wave[u] = w0 + u * kRecordWaves;
+            out[u] = record(wave[u]);
+        }
+        if (t < groups) {                               // every lane group's entries: a lane finds its row without knowing the class
+            Item it[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) it[u] = row_of(wave[u], t);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (t == 0) out[u][0] = (int32_t)desc_code(kind, src, (uint32_t)min(ipw, run.n - wave[u] * ipw));
+                out[u][L.off_row + t] = it[u].row;
+                out[u][L.off_start + t] = it[u].start;
+                out[u][L.off_len + t] = it[u].len;
+            }
         }
         for (int k = t; k < 4 * groups; k += 64) {      // entry k: edge k % 4 of lane group k / 4
-            const int g = k >> 2, i = g / S;
-            Item it{0, 0, 0, -1};
-            if (i < count) it = items[first + i];
-            const int e = g % S + (k & 3) * S, ec = e < it.len ? e : it.len - 1;
-            out[L.off_col + k] = it.len > 0 ? col[it.start + ec] : 0;
-            out[L.off_eid + k] = it.len > 0 ? eid[it.start + ec] : 0;
+            Item it[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) it[u] = row_of(wave[u], k >> 2);
+            int c[U], e[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int at = it[u].len > 0 ? it[u].start + min((k >> 2) % S + (k & 3) * S, it[u].len - 1) : 0;
+                c[u] = col[at];
+                e[u] = eid[at];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                out[u][L.off_col + k] = it[u].len > 0 ? c[u] : 0;
+                out[u][L.off_eid + k] = it[u].len > 0 ? e[u] : 0;
+            }
         }
-    }
+    };
+    int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (; w + (kRecordStep - 1) * kRecordWaves < waves; w += kRecordWaves * kRecordStep) step(w, std::integral_constant<int, kRecordStep>{});
+    if (w + kRecordWaves < waves) { step(w, std::integral_constant<int, 2>{}); w += 2 * kRecordWaves; }
+    if (w < waves) step(w, std::integral_constant<int, 1>{});
 }
 
 // ---------------------------------------------------------------------------

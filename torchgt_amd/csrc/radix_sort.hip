@@ -13,9 +13,12 @@
 namespace tgt {
 
 constexpr int RS_THREADS = 256;
-constexpr int RS_ITEMS = 16;
-constexpr int RS_TILE = RS_THREADS * RS_ITEMS;   // 4096 keys per workgroup
-constexpr int RS_WAVE_SPAN = kWave * RS_ITEMS;   // 1024 consecutive keys per wave
+// Keys per thread (a workgroup's tile is 256 times as many; a wave takes a quarter of it, consecutive keys): 4 as long as every tile of a launch has
+// a place of its own (eight workgroups per CU), 16 with more.  Few keys are bound by the chain of one tile, sixteen rounds of ballots and
+// an LDS counter: 0.53 M keys of two sorts 8.6 us a pass with 4, 12 with 8, 14.5 with 16; 0.2 M of one 6.1, 8.1, 13.9.  Many pay for the
+// digits' counts of every tile: a plan of 2 M edges 584 us and 537 with 16, of 44 M 6.9 ms and 5.5.
+constexpr int kFewItems = 4, kManyItems = 16;
+static int rs_items(int64_t n, int sorts) { return n * sorts <= (int64_t)8 * num_cus() * RS_THREADS * kFewItems ? kFewItems : kManyItems; }
 
 // One or two sorts of the same size in a launch (blockIdx.y): the two views of a plan are sorted side by side - at half a
 // million keys one of them is a hundred workgroups.
@@ -25,6 +28,7 @@ struct RsArgs {
 };
 
 // Per-workgroup digit histogram, stored digit-major: hist[digit * nblocks + block].
+template <int RS_ITEMS>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_hist(const RsArgs a, int64_t n, int shift, int nblocks) {
     const uint32_t* __restrict__ keys = a.keys_in[blockIdx.y];
     uint32_t* __restrict__ hist = a.hist[blockIdx.y];
@@ -32,12 +36,13 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_hist(const RsArgs a, int64_t 
     const int tid = threadIdx.x;
     h[tid] = 0;
     __syncthreads();
-    const int64_t base = (int64_t)blockIdx.x * RS_TILE;
+    const int64_t base = (int64_t)blockIdx.x * RS_THREADS * RS_ITEMS;
+    uint32_t key[RS_ITEMS];
 #pragma unroll
-    for (int i = 0; i < RS_ITEMS; ++i) {
-        int64_t idx = base + i * RS_THREADS + tid;
-        if (idx < n) atomicAdd(&h[(keys[idx] >> shift) & 255u], 1u);   // integer count: order-free
-    }
+    for (int i = 0; i < RS_ITEMS; ++i) key[i] = keys[min(base + i * RS_THREADS + tid, n - 1)];
+#pragma unroll
+    for (int i = 0; i < RS_ITEMS; ++i)
+        if (base + i * RS_THREADS + tid < n) atomicAdd(&h[(key[i] >> shift) & 255u], 1u);   // integer count: order-free
     __syncthreads();
     hist[(int64_t)tid * nblocks + blockIdx.x] = h[tid];
 }
@@ -71,13 +76,15 @@ __global__ __launch_bounds__(256) void k_rs_scan_rows(const RsArgs a, int nblock
     if (tid == 255) totals[blockIdx.x] = part[255];
 }
 
-// Stable scatter of one radix pass.  Each wave owns 1024 consecutive keys of the
-// tile and ranks them in 16 rounds of 64; the rank of a key among equal digits is
+// Stable scatter of one radix pass.  Each wave owns a quarter of the tile, consecutive keys, and ranks them in rounds of 64; the rank of a key among equal digits is
 // (count in earlier rounds) + (number of lower lanes with the same digit).  The tile
 // is then put in digit order in LDS (stable), so that the writes to global memory go
 // out as runs of consecutive addresses, one run per digit, instead of one scattered
-// 4-byte store per key.
+// 4-byte store per key.  A wave asks for all its keys and values before it ranks the first (past the end: the last key's); loads inside
+// the branch that uses them went out one after the other (16.5 us for 0.53 M keys, 14.5 without).
+template <int RS_ITEMS>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const RsArgs a, int64_t n, int shift, int nblocks) {
+    constexpr int RS_TILE = RS_THREADS * RS_ITEMS;
     const uint32_t *__restrict__ keys_in = a.keys_in[blockIdx.y], *__restrict__ vals_in = a.vals_in[blockIdx.y];
     uint32_t *__restrict__ keys_out = a.keys_out[blockIdx.y], *__restrict__ vals_out = a.vals_out[blockIdx.y];
     const uint32_t *__restrict__ hist = a.hist[blockIdx.y], *__restrict__ totals = a.totals[blockIdx.y];
@@ -95,17 +102,18 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const RsArgs a, int64
     __syncthreads();
 
     volatile uint32_t* wcnt = &cnt[wave][0];
-    uint32_t key[RS_ITEMS], rank[RS_ITEMS];
+    uint32_t key[RS_ITEMS], val[RS_ITEMS], rank[RS_ITEMS];
     const int64_t tbase = (int64_t)blockIdx.x * RS_TILE;
-    const int64_t wbase = tbase + (int64_t)wave * RS_WAVE_SPAN;
+    const int64_t wbase = tbase + (int64_t)wave * kWave * RS_ITEMS;
     const uint64_t lower_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
 #pragma unroll
+    for (int r = 0; r < RS_ITEMS; ++r) key[r] = keys_in[min(wbase + r * kWave + lane, n - 1)];
+#pragma unroll
+    for (int r = 0; r < RS_ITEMS; ++r) val[r] = vals_in ? vals_in[min(wbase + r * kWave + lane, n - 1)] : (uint32_t)(wbase + r * kWave + lane);
+#pragma unroll
     for (int r = 0; r < RS_ITEMS; ++r) {
-        const int64_t idx = wbase + r * kWave + lane;
-        const bool valid = idx < n;
-        const uint32_t kk = valid ? keys_in[idx] : 0u;
-        key[r] = kk;
-        const uint32_t dg = (kk >> shift) & 255u;
+        const bool valid = wbase + r * kWave + lane < n;
+        const uint32_t dg = (key[r] >> shift) & 255u;
         uint64_t same = __ballot(valid);
 #pragma unroll
         for (int b = 0; b < 8; ++b) {
@@ -152,7 +160,7 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const RsArgs a, int64
             const uint32_t dg = (key[r] >> shift) & 255u;
             const uint32_t slot = tstart[dg] + cnt[wave][dg] + rank[r];
             lkey[slot] = key[r];
-            lval[slot] = vals_in ? vals_in[idx] : (uint32_t)idx;
+            lval[slot] = val[r];
         }
     }
     __syncthreads();
@@ -214,7 +222,8 @@ int bits_for(int64_t n) {
 
 int RadixSorter::init(int64_t n, hipStream_t st, int sorts) {
     cap_ = n > 0 ? n : 1;
-    nblocks_ = (int)((cap_ + RS_TILE - 1) / RS_TILE);
+    const int tile = RS_THREADS * rs_items(cap_, sorts);
+    nblocks_ = (int)((cap_ + tile - 1) / tile);
     sorts_ = sorts;
     TGT_HIP_CHECK(buf_.alloc(sizeof(uint32_t) * sorts * (4 * (size_t)cap_ + 256 * (size_t)nblocks_ + 256), st));
     return TGT_OK;
@@ -224,7 +233,8 @@ int RadixSorter::sort(const uint32_t* const* keys_in, const uint32_t* const* val
                       const uint32_t** keys_out, const uint32_t** vals_out) {
     if (n > cap_ || sorts > sorts_) { set_error("RadixSorter: n exceeds capacity"); return TGT_ERR_INVALID_ARG; }
     const int passes = (bits + 7) / 8 > 0 ? (bits + 7) / 8 : 1;
-    const int nblocks = (int)((n + RS_TILE - 1) / RS_TILE);
+    // of the capacity: a smaller sort never has more workgroups than there is room for
+    const int items = rs_items(cap_, sorts_), nblocks = (int)((n + RS_THREADS * items - 1) / (RS_THREADS * items));
     RsArgs a{};
     uint32_t *key[2][2], *val[2][2];      // [sort][ping, pong]
     uint32_t* at = buf_.as<uint32_t>();
@@ -238,9 +248,9 @@ int RadixSorter::sort(const uint32_t* const* keys_in, const uint32_t* const* val
     for (int p = 0; p < passes && n > 0; ++p) {
         const int shift = 8 * p;
         for (int i = 0; i < sorts; ++i) { a.keys_out[i] = key[i][p & 1]; a.vals_out[i] = val[i][p & 1]; }
-        hipLaunchKernelGGL(k_rs_hist, dim3(nblocks, sorts), dim3(RS_THREADS), 0, st, a, n, shift, nblocks);
+        hipLaunchKernelGGL(items == kFewItems ? &k_rs_hist<kFewItems> : &k_rs_hist<kManyItems>, dim3(nblocks, sorts), dim3(RS_THREADS), 0, st, a, n, shift, nblocks);
         hipLaunchKernelGGL(k_rs_scan_rows, dim3(256, sorts), dim3(256), 0, st, a, nblocks);
-        hipLaunchKernelGGL(k_rs_scatter, dim3(nblocks, sorts), dim3(RS_THREADS), 0, st, a, n, shift, nblocks);
+        hipLaunchKernelGGL(items == kFewItems ? &k_rs_scatter<kFewItems> : &k_rs_scatter<kManyItems>, dim3(nblocks, sorts), dim3(RS_THREADS), 0, st, a, n, shift, nblocks);
         for (int i = 0; i < sorts; ++i) { a.keys_in[i] = a.keys_out[i]; a.vals_in[i] = a.vals_out[i]; }
     }
     TGT_HIP_CHECK(hipGetLastError());
