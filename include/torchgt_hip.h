@@ -603,6 +603,9 @@ int tgt_floyd_warshall(const uint8_t* d_adj, const int32_t* d_n_nodes, int num_g
 int64_t tgt_node_frag_bytes(int n_mats, int dtype);
 int tgt_node_pack(const void* const* mats, const int* ld, const int* rows, int n_mats, const void* const* vecs, const int* lens,
                   int n_vecs, int dtype, void* d_frags, float* d_vecs, void* stream);
+/* The same for weights [rows[i] <= 64, cols[i] <= 64] with ld[i] >= cols[i] (columns behind cols[i] count as zero). */
+int tgt_node_pack_parts(const void* const* mats, const int* ld, const int* rows, const int* cols, int n_mats, const void* const* vecs,
+                        const int* lens, int n_vecs, int dtype, void* d_frags, float* d_vecs, void* stream);
 /* Forward.  attn: the attention's rows [rows, 64], or NULL for the part in front of the first layer (then s' = s_in, whose
  * first `tokens` rows are taken from `token` and written to s_out; s_in and s_out are the same array).  w_post: packed Wo,
  * W1, W2; v_post: bo, gamma, beta, b1, b2.  q, k, v: rows for the next attention (w_next: packed Wq, Wk, Wv; v_next: gamma,
@@ -691,6 +694,28 @@ typedef struct {
     float *nd, *partial_a, *partial_b;
 } tgt_gt_bwd_args;
 int tgt_gt_bwd(const tgt_gt_bwd_args* args, void* stream);
+/* The GT readout behind the layers (models/gt_dist_node_level.py:270-286, 337-341): log_softmax over the first `classes` of
+ * Wc relu(Wb relu(Wa x + ba) + bb) + bc for x [rows, 64]; Wa [m1, 64], Wb [m2, m1], Wc [out, m2], all widths up to 64.  w, v: the packed
+ * weights (tgt_node_pack_parts) and biases in this order, w_back: the transposed ones.  Backward: dx [rows, 64] and the gradients of
+ * (Wa, Wb, Wc, ba, bb, bc) in out (NULL: not wanted); partial: tgt_readout_partial_floats(...) floats. */
+typedef struct {
+    int64_t rows;
+    int32_t dtype, m1, m2, out, classes;
+    const void *x, *w;
+    const float* v;
+    void* logp;
+} tgt_readout_fwd_args;
+int tgt_readout_fwd(const tgt_readout_fwd_args* args, void* stream);
+typedef struct {
+    int64_t rows;
+    int32_t dtype, m1, m2, out, classes;
+    const void *x, *dlogp, *logp, *w, *w_back;
+    const float* v;
+    void *dx, *grads[6];
+    float* partial;
+} tgt_readout_bwd_args;
+int64_t tgt_readout_partial_floats(int64_t rows, int m1, int m2, int out);
+int tgt_readout_bwd(const tgt_readout_bwd_args* args, void* stream);
 /* The dense biased attention for query 0 only: the last layer of the graph-level models, whose output is read at the virtual node
  * (models/graphormer_graph_level.py:387).  Tensors as for tgt_dense_attn_dropout_fwd (H <= 8, d 8, 16 or 32, S <= 1024, dtype
  * TGT_DTYPE_F32 or TGT_DTYPE_BF16); a0 [b, H d] = the attention's row 0 of every graph, s0 = the rows 0 of d_s [b, S, H d],

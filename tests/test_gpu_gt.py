@@ -3,13 +3,15 @@ ReLU is exact.  The model: max|a - b| / max|b| against float64 on the same input
 log-probabilities and on every parameter gradient;
 bf16 three times the single-kernel bar of 2e-2 on the output.
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 from oracle import gt as ogt
 from torchgt_amd import _lib, workloads
-from torchgt_amd.gt import GT, ReluFunction
+from torchgt_amd.gt import _DT, GT, ReluFunction
 
 pytestmark = pytest.mark.gpu
 
@@ -179,3 +181,64 @@ def test_graph_level_gt_matches_oracle(cuda, attn_type):
     assert not bad, bad
     assert np.median(list(errs.values())) <= tol
     assert "embedding_h.weight" in errs and got_g[names.index("embedding_h.weight")][0].abs().max() > 0     # row 0 is an ordinary row
+
+
+class _ReadoutFwd(ctypes.Structure):
+    _fields_ = [("rows", ctypes.c_int64)] + [(k, ctypes.c_int32) for k in ("dtype", "m1", "m2", "out", "classes")] + [(k, ctypes.c_void_p) for k in ("x", "w", "v", "logp")]
+
+
+class _ReadoutBwd(ctypes.Structure):
+    _fields_ = ([("rows", ctypes.c_int64)] + [(k, ctypes.c_int32) for k in ("dtype", "m1", "m2", "out", "classes")] +
+                [(k, ctypes.c_void_p) for k in ("x", "dlogp", "logp", "w", "w_back", "v", "dx")] + [("grads", ctypes.c_void_p * 6), ("partial", ctypes.c_void_p)])
+
+
+# Weights and rows of -1, 0, 1 (times a power of two): the inputs of both ReLUs and the logits are the same numbers whatever the order of
+# the sums, so no activation changes its side.  What is left: a log-softmax (2^-8 of a bfloat16 result, 1e-5 in float32) and, backward, one rounding of
+# every d logits, du (bfloat16: 2^-9 each of three in a row, and of the results): 1e-2 of the largest; float32 1e-5.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,m1,m2,out,classes", [(1, 32, 16, 40, 40), (15, 5, 3, 7, 7), (16, 64, 64, 64, 63), (17, 33, 17, 8, 1), (63, 32, 16, 48, 47), (65, 32, 16, 1, 1),
+                                                 (129, 1, 1, 2, 2), (4097, 32, 16, 40, 40), (16385, 64, 32, 16, 13), (70001, 32, 16, 40, 40)])
+def test_readout_in_one_kernel(cuda, dtype, n, m1, m2, out, classes):
+    print(f"readout n={n} widths {m1} {m2} {out} classes={classes} {dtype}", flush=True)
+    L, code, st = _lib.lib(), _DT[dtype], ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    g = torch.Generator(device=cuda).manual_seed(n + out)
+    grid = lambda *s: torch.randint(-1, 2, s, generator=g, device=cuda).to(dtype)
+    W = [grid(m1, 64) * 0.25, grid(m2, m1) * 0.5, grid(out, m2) * 0.25]
+    b = [grid(m1), grid(m2), grid(out)]
+    x, dlogp = grid(n, 64), torch.randn(n, classes, generator=g, device=cuda).to(dtype)
+    ints = lambda *a: (ctypes.c_int * len(a))(*a)
+    ptrs = lambda ts: (ctypes.c_void_p * len(ts))(*[t.data_ptr() for t in ts])
+    unit = L.tgt_node_frag_bytes(3, code)
+    frags, vecs = torch.empty(unit, dtype=torch.uint8, device=cuda), torch.empty(192, device=cuda)
+    _lib.check(L.tgt_node_pack_parts(ptrs(W), ints(64, m1, m2), ints(m1, m2, out), ints(64, m1, m2), 3, ptrs(b), ints(m1, m2, out), 3, code, frags.data_ptr(), vecs.data_ptr(), st))
+    logp, dx, grads = torch.full((n, classes), 7., device=cuda).to(dtype), torch.full_like(x, 7), [torch.full_like(t, 7) for t in W + b]
+    f = _ReadoutFwd(n, code, m1, m2, out, classes, x.data_ptr(), frags.data_ptr(), vecs.data_ptr(), logp.data_ptr())
+    _lib.check(L.tgt_readout_fwd(ctypes.byref(f), st))
+    partial = torch.empty(L.tgt_readout_partial_floats(n, m1, m2, out), device=cuda)
+    r = _ReadoutBwd(n, code, m1, m2, out, classes, x.data_ptr(), dlogp.data_ptr(), logp.data_ptr(), frags.data_ptr(), frags.data_ptr() + unit // 2, vecs.data_ptr(), dx.data_ptr(),
+                    ptrs(grads), partial.data_ptr())
+    _lib.check(L.tgt_readout_bwd(ctypes.byref(r), st))
+    held = lambda t: t.to(dtype).double()      # as a row of this type holds it
+    Wd, bd, a0 = [t.double() for t in W], [t.double() for t in b], x.double()
+    a1 = held(a0 @ Wd[0].T + bd[0]).relu()
+    a2 = held(a1 @ Wd[1].T + bd[1]).relu()
+    want = torch.log_softmax(held(a2 @ Wd[2].T + bd[2])[:, :classes], 1)
+    assert float((logp.double() - want).abs().max()) <= (2 ** -8 if dtype == torch.bfloat16 else 1e-5) * max(1.0, float(want.abs().max()))
+    d = torch.zeros(n, out, dtype=torch.double, device=cuda)
+    d[:, :classes] = dlogp.double() - logp.double().exp() * dlogp.double().sum(1, keepdim=True)
+    d1 = (d @ Wd[2]) * (a2 > 0)
+    d0 = (d1 @ Wd[1]) * (a1 > 0)
+    for name, got, ref in zip(("dx", "Wa", "Wb", "Wc", "ba", "bb", "bc"), [dx, *grads], [d0 @ Wd[0], d0.T @ a0, d1.T @ a1, d.T @ a2, d0.sum(0), d1.sum(0), d.sum(0)]):
+        top = max(float(ref.abs().max()), 1e-30)
+        # a bias of many rows: n terms of either sign, each rounded; their sum is as large as sqrt(n) of them
+        assert float((got.double() - ref).abs().max()) <= (1e-2 if dtype == torch.bfloat16 else 1e-5) * max(top, 1.0 if name[0] == "b" or n < 3 else 0.0), name
+
+
+def test_readout_refuses_other_widths():
+    L = _lib.lib()
+    assert L.tgt_readout_partial_floats(10, 65, 16, 40) == -1 and L.tgt_readout_partial_floats(10, 32, 0, 40) == -1
+    assert L.tgt_readout_fwd(None, None) != 0 and L.tgt_readout_bwd(None, None) != 0
+    f = _ReadoutFwd(0, 0, 32, 16, 40, 41, None, None, None, None)
+    assert L.tgt_readout_fwd(ctypes.byref(f), None) != 0      # more classes than outputs
+    f.classes = 40
+    assert L.tgt_readout_fwd(ctypes.byref(f), None) == 0      # no rows

@@ -117,6 +117,7 @@ SIGNATURES = {
     "tgt_gen_edge_input": (_i32, [_vp, _vp, _i32, _i32, _vp, _i32, _i32, _i32, _vp, _vp]),
     "tgt_node_frag_bytes": (_i64, [_i32, _i32]),
     "tgt_node_pack": (_i32, [_vp, _vp, _vp, _i32, _vp, _vp, _i32, _i32, _vp, _vp, _vp]),
+    "tgt_node_pack_parts": (_i32, [_vp, _vp, _vp, _vp, _i32, _vp, _vp, _i32, _i32, _vp, _vp, _vp]),
     "tgt_node_fwd": (_i32, [_vp, _vp]),
     "tgt_node_bwd_workers": (_i32, [_i64]),
     "tgt_node_bwd_pre": (_i32, [_vp, _vp]),
@@ -124,6 +125,9 @@ SIGNATURES = {
     "tgt_node_sums": (_i32, [_vp, _i32, _i32, _vp]),
     "tgt_gt_fwd": (_i32, [_vp, _vp]),
     "tgt_gt_bwd": (_i32, [_vp, _vp]),
+    "tgt_readout_fwd": (_i32, [_vp, _vp]),
+    "tgt_readout_partial_floats": (_i64, [_i64, _i32, _i32, _i32]),
+    "tgt_readout_bwd": (_i32, [_vp, _vp]),
     "tgt_sparse_attn_bwd_from_nd": (_i32, [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),
     "tgt_timing_enable": (_i32, [_i32]),
     "tgt_timing_reset": (_i32, []),

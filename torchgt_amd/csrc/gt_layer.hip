@@ -20,17 +20,6 @@ enum { V_BO = 0, V_GAMMA1, V_BETA1, V_B1A, V_B1B, V_B2, V_GAMMA2, V_BETA2, kVecs
 enum { W_O = 0, W_1A, W_1B, W_2A, W_2B };
 
 template <typename T, int R> __device__ __forceinline__ void round_to(TileOf<R>& t) { TGT_EACH(i) t.set(i, stored(t.get(i), (const T*)nullptr)); }
-// relu(u), and (bit i) where u > 0
-template <typename T, int R> __device__ __forceinline__ uint32_t relu(TileOf<R>& u) {
-    uint32_t on = 0;
-    TGT_EACH(i) {
-        const float v = stored(u.get(i), (const T*)nullptr);
-        on |= v > 0.f ? 1u << i : 0u;
-        u.set(i, v > 0.f ? v : 0.f);
-    }
-    return on;
-}
-
 // waves of a workgroup at most
 template <int R> constexpr int gt_fwd_waves() { return R == 32 ? 8 : 16; }
 // float32 takes its packed weights in turns (O and W1, W2, then q, k, v: 72 KB at most next to the row images), bf16 keeps all of them

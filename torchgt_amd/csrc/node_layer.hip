@@ -17,6 +17,7 @@
 // nodes each through the chain and put the bf16 planes of both operands into LDS, four others keep one 32 x 32 block of every
 // weight gradient each and add the products over these 128 nodes beside it (node_roles.h).
 #include "node_roles.h"
+#include "class_rows.h"
 
 namespace tgt {
 namespace {
@@ -25,15 +26,13 @@ namespace {
 constexpr int kPackMats = 96, kPackVecs = 160;
 struct PackArgs {
     const void* mat[kPackMats];
-    int16_t ld[kPackMats], rows[kPackMats];
+    int16_t ld[kPackMats], rows[kPackMats], cols[kPackMats];
     const void* vec[kPackVecs];
     int16_t len[kPackVecs];
     int n_mats, n_vecs, mat0, total_mats, vec0;
     vec16* frags;       // [2][total_mats][kFragVecs]: for y = W x, then for dx = W^T dy
     float* vecs;        // [..][64]
 };
-__device__ __forceinline__ float as_float(float v) { return v; }
-__device__ __forceinline__ float as_float(nbf16 v) { return __uint_as_float((uint32_t)v.x << 16); }
 
 // workgroup = one (weight, direction): 512 operand vectors, one per thread; the workgroups behind the weights copy vectors
 template <typename T> __global__ __launch_bounds__(512) void k_node_pack(const PackArgs a) {
@@ -46,14 +45,14 @@ template <typename T> __global__ __launch_bounds__(512) void k_node_pack(const P
     }
     const int j = b >> 1, back = b & 1;
     const T* W = reinterpret_cast<const T*>(a.mat[j]);
-    const int ld = a.ld[j], rows = a.rows[j];
+    const int ld = a.ld[j], rows = a.rows[j], cols = a.cols[j];
     const int lane = threadIdx.x & 63, sm = threadIdx.x >> 6, s = sm >> 2, m = sm & 3;
     const int out_f = 16 * gray2((lane >> 2) & 3) + 4 * m + (lane & 3), in0 = 16 * (lane >> 4) + 8 * s;
     float v[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const int o = back ? in0 + i : out_f, k = back ? out_f : in0 + i;
-        v[i] = o < rows ? as_float(W[o * ld + k]) : 0.f;
+        v[i] = o < rows && k < cols ? as_float(W[o * ld + k]) : 0.f;
     }
     bf16x8_t p[P];
     to_planes(v, p);
@@ -109,63 +108,6 @@ template <typename T, bool POST, int NEXT> constexpr int fwd_resident_mats() {
 template <typename T, int R, bool POST, int NEXT> constexpr int fwd_lds(int waves) {
     return fwd_resident_mats<T, POST, NEXT>() * kFragVecs<Num<T>::P> * 16 + 10 * kVec * 4 + waves * RowShape<T, R>::kVecs * 16;
 }
-
-// Rows of class values.  A wave's R rows are R C consecutive elements of the [N - tokens, C] array and travel through its
-// row image, in words: for bf16 the image starts one element late where the rows begin in the middle of a word.
-template <typename T, int R> struct ClassRows {
-    static constexpr int kPerWord = 4 / (int)sizeof(T);
-    T* img;
-    int C, lo, hi;            // elements of the wave's rows that exist: [lo, hi)
-    int64_t first, total;     // element of the array the rows start at (negative: token rows), elements of the array
-    int shift;
-    __device__ __forceinline__ ClassRows(vec16* stage, int64_t row0, int64_t N, int tokens, int classes) {
-        C = classes;
-        const int64_t r = row0 - tokens, left = N - row0;
-        first = r * C; total = (N - tokens) * C;
-        lo = r < 0 ? (int)(-r < R ? -r : R) * C : 0;
-        hi = (int)(left < 0 ? 0 : (left < R ? left : R)) * C;
-        shift = kPerWord == 2 ? (int)(first & 1) : 0;
-        img = reinterpret_cast<T*>(stage) + shift;
-    }
-    __device__ __forceinline__ int words() const { return (hi + shift + kPerWord - 1) / kPerWord; }
-    // array -> image; every load is issued before the first is waited for
-    __device__ __forceinline__ void load(const T* __restrict__ src, int lane) {
-        const int n = words();
-        const int64_t w0 = (first - shift) / kPerWord, last = total / kPerWord - 1;
-        const uint32_t* p = reinterpret_cast<const uint32_t*>(src);
-        uint32_t v[R];
-        TGT_EACH(i)
-            if (i * 64 < n && last >= 0) {
-                int64_t w = w0 + i * 64 + lane;
-                w = w < 0 ? 0 : (w > last ? last : w);
-                v[i] = p[w];
-            }
-        wave_sync();
-        uint32_t* d = reinterpret_cast<uint32_t*>(img - shift);
-        TGT_EACH(i)
-            if (i * 64 < n && last >= 0 && i * 64 + lane < n) d[i * 64 + lane] = v[i];
-        wave_sync();
-        if (kPerWord == 2 && (total & 1) && first + hi == total && hi > lo && lane == 0) img[hi - 1] = src[total - 1];      // half a word at the end
-        wave_sync();
-    }
-    __device__ __forceinline__ void store(T* __restrict__ dst, int lane) const {
-        const uint32_t* d = reinterpret_cast<const uint32_t*>(img - shift);
-        T* out = dst + first;
-        const int n = words();
-        for (int w = lane; w < n; w += 64) {
-            const int e = w * kPerWord - shift;
-            if (e >= lo && e + kPerWord <= hi) *reinterpret_cast<uint32_t*>(out + e) = d[w];
-            else {
-#pragma unroll
-                for (int k = 0; k < kPerWord; ++k)
-                    if (e + k >= lo && e + k < hi) out[e + k] = img[e + k];
-            }
-        }
-    }
-};
-template <typename T> __device__ __forceinline__ T to_elem(float v);
-template <> __device__ __forceinline__ float to_elem<float>(float v) { return v; }
-template <> __device__ __forceinline__ nbf16 to_elem<nbf16>(float v) { return nbf16{__builtin_bit_cast(uint16_t, static_cast<__bf16>(v))}; }
 
 template <typename T, int R, bool SAME, bool POST, int NEXT>
 __global__ __launch_bounds__((fwd_waves<T, R, SAME>() * 64)) void k_node_fwd(const tgt_node_fwd_args a) {
@@ -255,46 +197,10 @@ __global__ __launch_bounds__((fwd_waves<T, R, SAME>() * 64)) void k_node_fwd(con
             } else {
                 TileOf<R> y;
                 linear<P, SAME>(y, s, w_next, vn + 2 * kVec, lane);
-                const int C = a.classes;
-                float lse = 0.f;
-                if (!a.linear) {
-                    float top = -INFINITY, sum = 0.f;
-                    TGT_EACH(i) {      // rounded first: log_softmax reads the logits as a T tensor would hold them
-                        y.set(i, stored(y.get(i), (const T*)nullptr));
-                        if (R * g + i < C) top = fmaxf(top, y.get(i));
-                    }
-#pragma unroll
-                    for (int off = R; off < 64; off <<= 1) top = fmaxf(top, __shfl_xor(top, off, 64));
-                    TGT_EACH(i) if (R * g + i < C) sum += expf(y.get(i) - top);
-                    lse = top + logf(node_sum<R>(sum));
-                }
-                const ClassRows<T, R> out(stage, row0, N, a.tokens, C);
-                wave_sync();
-                TGT_EACH(i) if (R * g + i < C) out.img[(lane % R) * C + R * g + i] = to_elem<T>(y.get(i) - lse);
-                wave_sync();
-                out.store(reinterpret_cast<T*>(a.logp), lane);
+                put_classes<T>(reinterpret_cast<T*>(a.logp), y, a.linear, a.classes, a.tokens, row0, N, stage, lane);
             }
         }
     }
-}
-
-// Class gradients of a wave's R rows: d logits = d logp - softmax * sum(d logp) (linear: d logits as they come); zero for tokens and past the end.
-template <typename T, int R> __device__ __forceinline__ void class_grads(TileOf<R>& d, const T* __restrict__ dlogp, const T* __restrict__ logp, bool linear, int C, int tokens, int64_t row0, int64_t N,
-                                                                         vec16* stage, int lane) {
-    const int n = lane % R, g = lane / R;
-    ClassRows<T, R> rows(stage, row0, N, tokens, C);
-    const bool in = n * C >= rows.lo && n * C < rows.hi;
-    const T* mine = rows.img + (in ? n * C + R * g : 0);
-    rows.load(dlogp, lane);
-    float sum = 0.f;
-    TGT_EACH(i) {
-        d.set(i, in && R * g + i < C ? as_float(mine[i]) : 0.f);
-        sum += d.get(i);
-    }
-    if (linear) return;
-    sum = node_sum<R>(sum);
-    rows.load(logp, lane);
-    TGT_EACH(i) if (in && R * g + i < C) d.set(i, d.get(i) - expf(as_float(mine[i])) * sum);
 }
 
 // ---- backward of the part in front of an attention (or of the classes) ------------------------------------------------------
@@ -339,7 +245,7 @@ __global__ __launch_bounds__((Bwd<T, R, CN>::kThreads)) void k_node_bwd_pre(cons
             zero(dy);
 #pragma unroll
             for (int j = 0; j < NM; ++j) {
-                if (CLASSES) class_grads(d, reinterpret_cast<const T*>(a.dlogp), reinterpret_cast<const T*>(a.logp), a.linear, a.classes, a.tokens, (NC * g0 + wave) * R, N, stage, lane);
+                if (CLASSES) ClassGrads<T, R>(reinterpret_cast<const T*>(a.dlogp), reinterpret_cast<const T*>(a.logp), a.linear, a.classes, a.tokens, (NC * g0 + wave) * R, N, stage, lane).settle(d);
                 else {
                     settle<T, true>(d, raw_d, stage, rows, lane);
                     fetch(raw_d, j + 1 < NM ? src[j + 1] : reinterpret_cast<const T*>(a.g_in), rows, lane);
@@ -623,10 +529,16 @@ int64_t tgt_node_frag_bytes(int n_mats, int dtype) {
 
 int tgt_node_pack(const void* const* mats, const int* ld, const int* rows, int n_mats, const void* const* vecs, const int* lens, int n_vecs,
                   int dtype, void* d_frags, float* d_vecs, void* stream) {
+    return tgt_node_pack_parts(mats, ld, rows, nullptr, n_mats, vecs, lens, n_vecs, dtype, d_frags, d_vecs, stream);
+}
+int tgt_node_pack_parts(const void* const* mats, const int* ld, const int* rows, const int* cols, int n_mats, const void* const* vecs, const int* lens, int n_vecs,
+                        int dtype, void* d_frags, float* d_vecs, void* stream) {
     using namespace tgt;
     if (!mats || !ld || !rows || !vecs || !lens || n_mats < 1 || n_vecs < 1 || !d_frags || !d_vecs || !dtype_ok(dtype)) return bad("tgt_node_pack", "null or bad argument");
-    for (int i = 0; i < n_mats; ++i)
-        if (!mats[i] || rows[i] < 1 || rows[i] > 64 || ld[i] < 64 || ld[i] > 32767) return bad("tgt_node_pack", "weights are [1..64, >= 64]");
+    for (int i = 0; i < n_mats; ++i) {
+        const int c = cols ? cols[i] : 64;
+        if (!mats[i] || rows[i] < 1 || rows[i] > 64 || c < 1 || c > 64 || ld[i] < c || ld[i] > 32767) return bad("tgt_node_pack", "weights are [1..64, >= 64]");
+    }
     for (int i = 0; i < n_vecs; ++i)
         if (!vecs[i] || lens[i] < 1 || lens[i] > 64) return bad("tgt_node_pack", "vectors have 1 to 64 elements");
     KernelTimer t(KS_NODE_PACK, (hipStream_t)stream);
@@ -635,7 +547,7 @@ int tgt_node_pack(const void* const* mats, const int* ld, const int* rows, int n
         a.n_mats = std::min(kPackMats, n_mats - m); a.n_vecs = std::min(kPackVecs, n_vecs - v);
         a.mat0 = m; a.vec0 = v; a.total_mats = n_mats;
         a.frags = (vec16*)d_frags; a.vecs = d_vecs;
-        for (int i = 0; i < a.n_mats; ++i) { a.mat[i] = mats[m + i]; a.ld[i] = (int16_t)ld[m + i]; a.rows[i] = (int16_t)rows[m + i]; }
+        for (int i = 0; i < a.n_mats; ++i) { a.mat[i] = mats[m + i]; a.ld[i] = (int16_t)ld[m + i]; a.rows[i] = (int16_t)rows[m + i]; a.cols[i] = (int16_t)(cols ? cols[m + i] : 64); }
         for (int i = 0; i < a.n_vecs; ++i) { a.vec[i] = vecs[v + i]; a.len[i] = (int16_t)lens[v + i]; }
         const int grid = 2 * a.n_mats + (a.n_vecs + 7) / 8;
         if (dtype == TGT_DTYPE_F32) hipLaunchKernelGGL((k_node_pack<float>), dim3(grid), dim3(512), 0, (hipStream_t)stream, a);

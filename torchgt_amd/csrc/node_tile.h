@@ -357,6 +357,17 @@ template <typename T, int R> __device__ __forceinline__ void put_rows(T* __restr
 __device__ __forceinline__ float stored(float v, const float*) { return v; }
 __device__ __forceinline__ float stored(float v, const nbf16*) { return static_cast<float>(static_cast<__bf16>(v)); }
 
+// relu(u), and (bit i) where u > 0
+template <typename T, int R> __device__ __forceinline__ uint32_t relu(TileOf<R>& u) {
+    uint32_t on = 0;
+    TGT_EACH(i) {
+        const float v = stored(u.get(i), (const T*)nullptr);
+        on |= v > 0.f ? 1u << i : 0u;
+        u.set(i, v > 0.f ? v : 0.f);
+    }
+    return on;
+}
+
 // v of this lane plus v of the lane that is 32 further on or back
 __device__ __forceinline__ float both_halves(float v) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);

@@ -1,0 +1,266 @@
+// The readout of the node-level GT (MLPReadout and log_softmax, models/gt_dist_node_level.py:270-286, 337-341) behind layers of 64 features:
+//
+//     forward   logp = log_softmax(Wc relu(Wb relu(Wa x + ba) + bb) + bc)
+//     backward  d logp -> dx and the gradients of the three weights and biases, the activations formed again from x
+//
+// Widths up to 64, 32 and 16 in the model: as a kernel per linear, activation and softmax these are fourteen launches of 3 to 12 us for 64 K nodes
+// that read and write rows of 32 to 128 bytes (33 us forward and 58 backward, and their host time).  Here a wave carries its nodes
+// through all of it (node_tile.h), the narrow weights packed as 64 x 64 with zeros.  Backward: the roles of node_roles.h; bound by the chain of a
+// group's products.  64 K rows in bf16 8.4 us forward, 21 + 5 backward.
+#include "node_roles.h"
+#include "class_rows.h"
+
+namespace tgt {
+namespace {
+
+constexpr int kMats = 3, kRows = 16, kWaves = 16;      // weights; forward: rows of a wave, waves of a workgroup at most
+template <typename T> constexpr int readout_lds(int waves) { return kMats * kFragVecs<Num<T>::P> * 16 + kMats * kVec * 4 + waves * RowShape<T, kRows>::kVecs * 16; }
+
+template <typename T> __global__ __launch_bounds__(kWaves * 64) void k_readout_fwd(const tgt_readout_fwd_args a) {
+    constexpr int P = Num<T>::P, FV = kFragVecs<P>, R = kRows;
+    extern __shared__ __align__(16) unsigned char smem[];
+    vec16* w = reinterpret_cast<vec16*>(smem);
+    float* vec = reinterpret_cast<float*>(w + kMats * FV);
+    const int threads = blockDim.x, NW = threads >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    vec16* stage = reinterpret_cast<vec16*>(vec + kMats * kVec) + wave * RowShape<T, R>::kVecs;
+    const int64_t N = a.rows, tiles = (N + R - 1) / R;
+    copy_params<kMats * kVec>(threads, vec, a.v);
+    copy_vecs_by<kMats * FV>(threads, w, reinterpret_cast<const vec16*>(a.w));
+    __syncthreads();
+    for (int64_t t0 = (int64_t)blockIdx.x * NW + wave; t0 < tiles; t0 += (int64_t)gridDim.x * NW) {
+        const Rows rows(t0, N, R);
+        Raw<T, R> raw;
+        fetch(raw, reinterpret_cast<const T*>(a.x), rows, lane);
+        TileOf<R> x, y;
+        settle<T, false>(x, raw, stage, rows, lane);
+        linear<P, false>(y, x, w, vec, lane);
+        relu<T>(y);
+        linear<P, false>(x, y, w + FV, vec + kVec, lane);
+        relu<T>(x);
+        linear<P, false>(y, x, w + 2 * FV, vec + 2 * kVec, lane);
+        put_classes<T>(reinterpret_cast<T*>(a.logp), y, false, a.classes, 0, t0 * R, N, stage, lane);
+    }
+}
+
+// Where the sums of a worker lie: the three weights as they are, then the biases
+struct Sizes {
+    int m1, m2, out;
+    __host__ __device__ constexpr int rows(int j) const { return j == 0 ? m1 : (j == 1 ? m2 : out); }
+    __host__ __device__ constexpr int cols(int j) const { return j == 0 ? 64 : (j == 1 ? m1 : m2); }
+    __host__ __device__ constexpr int at(int j) const {      // weight j, bias j - 3, behind them all (6)
+        const int w1 = m1 * 64, w2 = w1 + m2 * m1, b0 = w2 + out * m2;
+        return j == 0 ? 0 : (j == 1 ? w1 : (j == 2 ? w2 : (j == 3 ? b0 : (j == 4 ? b0 + m1 : (j == 5 ? b0 + m1 + m2 : b0 + m1 + m2 + out)))));
+    }
+};
+
+// t where the activation was positive, as a T row would hold it
+template <typename T, int R> __device__ __forceinline__ void relu_back(TileOf<R>& t, uint32_t on) {
+    TGT_EACH(i) t.set(i, on >> i & 1u ? stored(t.get(i), (const T*)nullptr) : 0.f);
+}
+
+template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN, kMats>::kThreads)) void k_readout_bwd(const tgt_readout_bwd_args a) {
+    using L = Bwd<T, R, CN, kMats>;
+    constexpr int P = Num<T>::P, FV = kFragVecs<P>, PB = L::kPlane, NC = L::kChain;
+    extern __shared__ __align__(16) unsigned char smem[];
+    unsigned char *p_dy = smem, *p_x = smem + P * PB;
+    vec16* w = reinterpret_cast<vec16*>(smem + L::kW);
+    float* vec = reinterpret_cast<float*>(smem + L::kVecs);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane % R, h = lane / R;
+    const int64_t N = a.rows, groups = (N + CN - 1) / CN;
+    copy_vecs<kMats * kVec / 4, L::kThreads>(reinterpret_cast<vec16*>(vec), reinterpret_cast<const vec16*>(a.v));
+    __syncthreads();
+    float16_t acc[kMats];
+    float col[kMats];
+#pragma unroll
+    for (int j = 0; j < kMats; ++j) {
+        col[j] = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
+    }
+    if (wave < NC) {
+        vec16* stage = reinterpret_cast<vec16*>(smem + L::kStage) + wave * RowShape<T, R>::kVecs;
+        const int row = R * wave + n;
+        Raw<T, R> raw;
+        fetch(raw, reinterpret_cast<const T*>(a.x), Rows(NC * (int64_t)blockIdx.x + wave, N, R), lane);
+        for (int64_t g0 = blockIdx.x; g0 < groups; g0 += gridDim.x) {
+            const int64_t tile = NC * g0 + wave;
+            const Rows rows(tile, N, R);
+            TileOf<R> t, d;
+            Frags<P, R> f, fx, fy;      // x and the first activation, for the weight gradients
+            settle<T, false>(t, raw, stage, rows, lane);
+            make_frags(fx, t);
+            ClassGrads<T, R> classes(reinterpret_cast<const T*>(a.dlogp), reinterpret_cast<const T*>(a.logp), false, a.classes, 0, tile * R, N, stage, lane);
+            if (g0 + gridDim.x < groups) fetch(raw, reinterpret_cast<const T*>(a.x), Rows(tile + NC * (int64_t)gridDim.x, N, R), lane);
+            __syncthreads();                                        // Wa is there; product Wa of the round before is done
+            linear<P, false>(t, fx, w, vec, lane);
+            __syncthreads();                                        // Wa has been used
+            const uint32_t on1 = relu<T>(t);
+            make_frags(fy, t);
+            classes.settle(d);
+            TGT_EACH(i) d.set(i, stored(d.get(i), (const T*)nullptr));
+            col[2] += column_sums(d, lane);
+            make_frags(f, d);
+            __syncthreads();                                        // Wb
+            linear<P, false>(t, fy, w, vec + kVec, lane);
+            __syncthreads();                                        // Wb has been used
+            const uint32_t on2 = relu<T>(t);
+            put_tile_planes<PB, P>(p_x, row, h, t);
+            put_planes<PB>(p_dy, row, h, f);
+            __syncthreads();                                        // planes of Wc; Wc^T
+            zero(t);
+            gemm<P>(t, f, w, lane);                                 // beside product Wc
+            relu_back<T>(t, on2);
+            col[1] += column_sums(t, lane);
+            make_frags(f, t);
+            __syncthreads();                                        // product Wc is done, Wc^T has been used
+            put_planes<PB>(p_dy, row, h, f);
+            put_planes<PB>(p_x, row, h, fy);
+            __syncthreads();                                        // planes of Wb; Wb^T
+            zero(t);
+            gemm<P>(t, f, w, lane);                                 // beside product Wb
+            relu_back<T>(t, on1);
+            col[0] += column_sums(t, lane);
+            make_frags(f, t);
+            __syncthreads();                                        // product Wb is done, Wb^T has been used
+            put_planes<PB>(p_dy, row, h, f);
+            put_planes<PB>(p_x, row, h, fx);
+            __syncthreads();                                        // planes of Wa; Wa^T
+            zero(t);
+            gemm<P>(t, f, w, lane);                                 // dx, beside product Wa
+            __syncthreads();                                        // Wa^T has been used
+            put_rows(reinterpret_cast<T*>(a.dx), t, stage, rows, lane);
+        }
+    } else {
+        const int q = wave - NC, base_dy = operand_base(q >> 1, lane), base_x = operand_base(q & 1, lane);
+        const vec16 *fw = reinterpret_cast<const vec16*>(a.w), *bw = reinterpret_cast<const vec16*>(a.w_back);
+        WeightsAhead<FV> next;
+        next.fetch(fw);
+        for (int64_t g0 = blockIdx.x; g0 < groups; g0 += gridDim.x) {
+            next.hand_over(w, fw + FV);             // Wa, then on to Wb
+            __syncthreads();
+            next.hand_over(w, bw + 2 * FV);         // Wb
+            __syncthreads();
+            next.hand_over(w, bw + FV);             // Wc^T and the planes of Wc
+            node_product<P, PB>(acc[2], p_dy, p_x, base_dy, base_x);
+            __syncthreads();
+            next.hand_over(w, bw);                  // Wb^T and the planes of Wb
+            node_product<P, PB>(acc[1], p_dy, p_x, base_dy, base_x);
+            __syncthreads();
+            next.hand_over(w, fw);                  // Wa^T and the planes of Wa
+            node_product<P, PB>(acc[0], p_dy, p_x, base_dy, base_x);
+            __syncthreads();
+        }
+    }
+    // the worker's sums, in the weights' own sizes
+    __syncthreads();
+    const Sizes z{a.m1, a.m2, a.out};
+    float* mine = a.partial + (int64_t)blockIdx.x * z.at(2 * kMats);
+    float* buf = reinterpret_cast<float*>(smem);
+    if (wave < NC) {
+#pragma unroll
+        for (int c = 0; c < kMats; ++c) buf[(wave * kMats + c) * 64 + lane] = col[c];
+    } else {
+        const int q = wave - NC, c = 32 * (q & 1) + (lane & 31);
+#pragma unroll
+        for (int j = 0; j < kMats; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int i = 32 * (q >> 1) + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                if (i < z.rows(j) && c < z.cols(j)) mine[z.at(j) + i * z.cols(j) + c] = acc[j][r];
+            }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < kMats * 64; i += L::kThreads) {
+        float t = 0.f;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) t += buf[c * kMats * 64 + i];
+        if ((i & 63) < z.rows(i >> 6)) mine[z.at(kMats + (i >> 6)) + (i & 63)] = t;
+    }
+}
+
+// Sums over the workers, 64 elements x 16 slices of them per workgroup: a slice in worker order, then the slices
+struct Outs { void* p[2 * kMats]; };
+__device__ __forceinline__ void put_sum(float* p, float v) { *p = v; }
+__device__ __forceinline__ void put_sum(nbf16* p, float v) { *p = to_elem<nbf16>(v); }
+template <typename T> __global__ __launch_bounds__(1024) void k_readout_sums(const float* __restrict__ partial, int workers, Sizes z, Outs out) {
+    __shared__ float part[16][64];
+    const int total = z.at(2 * kMats), e = blockIdx.x * 64 + (threadIdx.x & 63), sl = threadIdx.x >> 6;
+    const int w0 = workers * sl / 16, w1 = workers * (sl + 1) / 16;
+    const float* __restrict__ src = partial + (e < total ? e : total - 1);
+    float s = 0.f;
+    for (int w = w0; w < w1; w += 16) {
+        float t[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) t[i] = src[(int64_t)(w + i < w1 ? w + i : w0) * total];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s += w + i < w1 ? t[i] : 0.f;
+    }
+    part[sl][threadIdx.x & 63] = s;
+    __syncthreads();
+    if (sl != 0 || e >= total) return;
+    s = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s += part[i][threadIdx.x];
+    int j = 0;
+    while (j + 1 < 2 * kMats && e >= z.at(j + 1)) ++j;
+    if (out.p[j]) put_sum(reinterpret_cast<T*>(out.p[j]) + (e - z.at(j)), s);
+}
+
+template <typename T> int run_fwd(const tgt_readout_fwd_args& a, hipStream_t st) {
+    static std::atomic<uint64_t> done{0};
+    const int waves = fwd_waves_for(a.rows, kRows, kWaves);
+    if (int rc = allow_lds(reinterpret_cast<const void*>(&k_readout_fwd<T>), readout_lds<T>(kWaves), done)) return rc;
+    hipLaunchKernelGGL((k_readout_fwd<T>), dim3(fwd_grid(a.rows, kRows, waves)), dim3(waves * 64), readout_lds<T>(waves), st, a);
+    TGT_HIP_CHECK(hipGetLastError());
+    return TGT_OK;
+}
+template <typename T, int R, int CN> int run_bwd(const tgt_readout_bwd_args& a, hipStream_t st) {
+    using L = Bwd<T, R, CN, kMats>;
+    static std::atomic<uint64_t> done{0};
+    const int workers = bwd_workers(a.rows);
+    if (int rc = launch(&k_readout_bwd<T, R, CN>, done, workers, L::kThreads, L::kBytes, st, a)) return rc;
+    const Sizes z{a.m1, a.m2, a.out};
+    Outs out;
+    for (int j = 0; j < 2 * kMats; ++j) out.p[j] = a.grads[j];
+    hipLaunchKernelGGL((k_readout_sums<T>), dim3((z.at(2 * kMats) + 63) / 64), dim3(1024), 0, st, (const float*)a.partial, workers, z, out);
+    TGT_HIP_CHECK(hipGetLastError());
+    return TGT_OK;
+}
+bool widths_ok(int dtype, int m1, int m2, int out, int classes) {
+    return (dtype == TGT_DTYPE_F32 || dtype == TGT_DTYPE_BF16) && m1 >= 1 && m1 <= 64 && m2 >= 1 && m2 <= 64 && out >= 1 && out <= 64 && classes >= 1 && classes <= out;
+}
+
+}  // namespace
+}  // namespace tgt
+
+extern "C" {
+
+int tgt_readout_fwd(const tgt_readout_fwd_args* a, void* stream) {
+    using namespace tgt;
+    if (!a || a->rows < 0 || !widths_ok(a->dtype, a->m1, a->m2, a->out, a->classes)) return bad("tgt_readout_fwd", "null or bad argument");
+    if (a->rows == 0) return TGT_OK;
+    if (!a->x || !a->w || !a->v || !a->logp) return bad("tgt_readout_fwd", "null pointer");
+    const hipStream_t st = (hipStream_t)stream;
+    KernelTimer t(KS_GT_FWD, st);
+    // sixteen rows per wave, also with many: us with 16 / 32, float32 4 K rows 6.4 / 8.8, 64 K 13.6 / 14.9, 500 K 75.6 / 83.5; bf16 4.6 / 6.8,
+    // 8.4 / 9.5, 47.6 / 46.6
+    return a->dtype == TGT_DTYPE_F32 ? run_fwd<float>(*a, st) : run_fwd<nbf16>(*a, st);
+}
+int64_t tgt_readout_partial_floats(int64_t rows, int m1, int m2, int out) {
+    if (rows < 0 || !tgt::widths_ok(TGT_DTYPE_F32, m1, m2, out, 1)) return -1;
+    return (int64_t)tgt::bwd_workers(rows) * tgt::Sizes{m1, m2, out}.at(2 * tgt::kMats);
+}
+int tgt_readout_bwd(const tgt_readout_bwd_args* a, void* stream) {
+    using namespace tgt;
+    if (!a || a->rows < 1 || !widths_ok(a->dtype, a->m1, a->m2, a->out, a->classes) || !a->x || !a->dlogp || !a->logp || !a->w || !a->w_back || !a->v || !a->dx || !a->partial)
+        return bad("tgt_readout_bwd", "null or bad argument");
+    const hipStream_t st = (hipStream_t)stream;
+    KernelTimer t(KS_GT_BWD, st);
+    // Nodes of a workgroup's group: float32 has registers for the chain with eight waves only (128 nodes put 75 to scratch: 16385 rows 29.9 us with 64
+    // and 33.0, 64000 53 and 66, 500000 356 and 496); bfloat16 as elsewhere (16384 rows 15.9 and 16.2, 16385 21.7 and 16.4, 64000 36 and 26).
+    if (a->dtype == TGT_DTYPE_F32) return run_bwd<float, 16, 64>(*a, st);
+    return groups_of_64(a->rows, false) ? run_bwd<nbf16, 16, 64>(*a, st) : run_bwd<nbf16, 16, 128>(*a, st);
+}
+
+}  // extern "C"

@@ -123,6 +123,8 @@ struct Saved {
     Norm last;
     std::vector<Layer> l;
     const std::vector<double>* eps;
+    void* logp = nullptr;      // fused readout: the log-probabilities [n, classes]
+    int64_t classes = 0;
 };
 
 Norm take_norm(Tape& t, const Dims& D, bool with_sum) { return {with_sum ? t.take(D.N * D.C * D.size) : nullptr, (float*)t.take(4 * D.N), (float*)t.take(4 * D.N)}; }
@@ -140,6 +142,7 @@ void attention_back(Tape& t, const Dims& D, const Layer& l, const tgt_plan_t* pl
 // ---- node-level Graphormer (models/graphormer_dist_node_level.py:316-392) -------------------------------------------------
 // params: Wn, bn, token table; per layer gamma1, beta1, Wq, bq, Wk, bk, Wv, bv, Wo, bo, gamma2, beta2, W1, b1, W2, b2; gamma, beta, Wh, bh
 struct GraphormerModel {
+    static bool fused_readout(const Dims&) { return false; }
     static constexpr int kHead = 3, kTail = 4;
     static constexpr int kQuery = 2, kFfn = 12;
     static void check_shapes(const char* name, const Dims& D, at::TensorList P) {
@@ -228,6 +231,7 @@ struct GraphormerModel {
 // ---- node-level GT (models/gt_dist_node_level.py:218-341) -----------------------------------------------------------------
 // params: Wn, bn; per layer Wq, bq, Wk, bk, Wv, bv, O, bo, gamma1, beta1, W1, b1, W2, b2, gamma2, beta2; readout W, b three times
 struct GtModel {
+    static bool fused_readout(const Dims&) { return false; }
     static constexpr int kHead = 2, kTail = 6;
     static constexpr int kQuery = 0, kFfn = 10;
     static void check_shapes(const char* name, const Dims& D, at::TensorList P) {
@@ -326,18 +330,20 @@ struct GtModel {
 // The same with hidden size 64 and 8, 4 or 2 heads, layers on gt_layer.hip.  Packed per layer: O, W1 (two halves of its rows), W2 (two
 // halves of its columns), Wq, Wk, Wv and bo, gamma1, beta1, b1 (two), b2, gamma2, beta2, bq, bk, bv.
 struct FusedGtModel : GtModel {
-    static constexpr int kMats = 8, kVecs = 11;
+    static constexpr int kMats = 8, kVecs = 11, kOut = 3;      // kOut: weights (and biases) of the readout behind the layers'
     static constexpr int64_t kPre = 3 * 4096 + 5 * 64, kPostA = kPre, kPostB = 2 * 4096 + 4 * 64;      // floats of a worker's partials
     static bool covers(const Dims& D) { return D.C == 64 && D.W == 64 && D.ff == 128 && (D.H == 8 || D.H == 4 || D.H == 2); }
     static int64_t unit(const Dims& D) { return tgt_node_frag_bytes(1, D.code) / 2; }
+    static bool fused_readout(const Dims& D) { return D.M1 <= 64 && D.M2 <= 64 && D.Cp <= 64; }
+    static int64_t mats(const Dims& D) { return kMats * D.L + kOut; }
     static char* weight(const Dims& D, const Saved& s, int64_t l, int i) { return (char*)s.packed + (kMats * l + i) * unit(D); }
-    static char* transposed(const Dims& D, const Saved& s, int64_t l, int i) { return weight(D, s, l + D.L, i); }
-    static float* vec(const Dims& D, const Saved& s, int64_t l, int i) { return (float*)((char*)s.packed + 2 * kMats * D.L * unit(D)) + (kVecs * l + i) * 64; }
+    static char* transposed(const Dims& D, const Saved& s, int64_t l, int i) { return weight(D, s, l, i) + mats(D) * unit(D); }
+    static float* vec(const Dims& D, const Saved& s, int64_t l, int i) { return (float*)((char*)s.packed + 2 * mats(D) * unit(D)) + (kVecs * l + i) * 64; }
     static void pack(Tape& t, const Dims& D, const std::vector<Tensor>& p, Saved& s) {
-        s.packed = t.take(2 * kMats * D.L * unit(D) + kVecs * D.L * 64 * 4);
+        s.packed = t.take(2 * mats(D) * unit(D) + (kVecs * D.L + kOut) * 64 * 4);
         if (t.dry()) return;
         std::vector<const void*> m, v;
-        std::vector<int> ld, rows(kMats * D.L, 64), len(kVecs * D.L, 64);
+        std::vector<int> ld, rows(kMats * D.L, 64), cols(kMats * D.L, 64), len(kVecs * D.L, 64);
         for (int64_t l = 0; l < D.L; ++l) {
             const Tensor* w = &p[kHead + 16 * l];
             auto part = [&](int i, int64_t elements) { return static_cast<char*>(w[i].data_ptr()) + elements * D.size; };
@@ -345,7 +351,15 @@ struct FusedGtModel : GtModel {
             for (int i : {64, 64, 64, 128, 128, 64, 64, 64}) ld.push_back(i);
             for (const void* q : {part(7, 0), part(8, 0), part(9, 0), part(11, 0), part(11, 64), part(13, 0), part(14, 0), part(15, 0), part(1, 0), part(3, 0), part(5, 0)}) v.push_back(q);
         }
-        check(tgt_node_pack(m.data(), ld.data(), rows.data(), (int)m.size(), v.data(), len.data(), (int)v.size(), D.code, s.packed, vec(D, s, 0, 0), D.stream), "tgt_node_pack");
+        // the readout's; where it has a width of its own kernels, the last layer's query weight and bias in its place (not read)
+        const Tensor* out = &p[kHead + 16 * D.L];
+        for (int i = 0; i < kOut; ++i) {
+            const Tensor &W = fused_readout(D) ? out[2 * i] : p[kHead], &b = fused_readout(D) ? out[2 * i + 1] : p[kHead + 1];
+            m.push_back(W.data_ptr()); ld.push_back((int)W.size(1)); rows.push_back((int)W.size(0)); cols.push_back((int)W.size(1));
+            v.push_back(b.data_ptr()); len.push_back((int)b.numel());
+        }
+        check(tgt_node_pack_parts(m.data(), ld.data(), rows.data(), cols.data(), (int)m.size(), v.data(), len.data(), (int)v.size(), D.code, s.packed, vec(D, s, 0, 0), D.stream),
+              "tgt_node_pack_parts");
     }
     static void forward(Tape& t, const Dims& D, const std::vector<Tensor>& p, const void* x, const tgt_plan_t* plan, const Tensor& ws, const std::vector<double>& eps, bool keep,
                         Saved& s) {
@@ -380,8 +394,14 @@ struct FusedGtModel : GtModel {
             }
             if (!t.dry()) check(tgt_gt_fwd(&a, D.stream), "tgt_gt_fwd");
         }
-        readout(t, D, p, s.l[D.L - 1].y1, s);
+        if (!fused_readout(D)) return readout(t, D, p, s.l[D.L - 1].y1, s);
+        s.out = s.l[D.L - 1].y1;
+        tgt_readout_fwd_args a{};
+        a.rows = D.N; a.dtype = D.code; a.m1 = (int)D.M1; a.m2 = (int)D.M2; a.out = (int)D.Cp; a.classes = (int)s.classes;
+        a.x = s.out; a.w = weight(D, s, D.L, 0); a.v = vec(D, s, D.L, 0); a.logp = s.logp;
+        if (!t.dry()) check(tgt_readout_fwd(&a, D.stream), "tgt_readout_fwd");
     }
+    // dlogits: of the log-probabilities where the readout is one kernel
     static void backward(Tape& t, const Dims& D, const std::vector<const void*>& P, const std::vector<void*>& G, const void* x, void* dx, const void* dlogits,
                          const tgt_plan_t* plan, const Tensor& ws, const Saved& s) {
         const int64_t row = D.N * 64 * D.size;
@@ -390,7 +410,15 @@ struct FusedGtModel : GtModel {
         const int workers = tgt_node_bwd_workers(D.N);
         float* partial = (float*)t.take(4 * workers * D.L * (kPre + kPostA + kPostB));
         Sums sums;
-        readout_back(t, D, P, G, dlogits, dm, du, g, s, sums);
+        if (fused_readout(D)) {
+            tgt_readout_bwd_args a{};
+            a.rows = D.N; a.dtype = D.code; a.m1 = (int)D.M1; a.m2 = (int)D.M2; a.out = (int)D.Cp; a.classes = (int)s.classes;
+            a.x = s.out; a.dlogp = dlogits; a.logp = s.logp; a.w = weight(D, s, D.L, 0); a.w_back = transposed(D, s, D.L, 0); a.v = vec(D, s, D.L, 0); a.dx = g;
+            const int order[6] = {0, 2, 4, 1, 3, 5};
+            for (int i = 0; i < 6; ++i) a.grads[i] = G.empty() ? nullptr : G[kHead + 16 * D.L + order[i]];
+            a.partial = (float*)t.take(4 * tgt_readout_partial_floats(D.N, (int)D.M1, (int)D.M2, (int)D.Cp));
+            if (!t.dry()) check(tgt_readout_bwd(&a, D.stream), "tgt_readout_bwd");
+        } else readout_back(t, D, P, G, dlogits, dm, du, g, s, sums);
         std::vector<tgt_node_sum> later;
         auto partial_of = [&](int mats, int ld, std::initializer_list<void*> out) {
             tgt_node_sum d{};
@@ -443,6 +471,15 @@ Tensor log_probabilities(const Saved& s, const Dims& D, int64_t classes, const a
     return at::log_softmax(at::from_blob(s.logits, {D.n, D.Cp}, opt).narrow(1, 0, classes), 1);
 }
 
+// The tensor that a model with a readout of its own writes them to
+template <typename M> Tensor own_log_probabilities(Saved& s, const Dims& D, int64_t classes, const at::TensorOptions& opt) {
+    if (!M::fused_readout(D)) return Tensor();
+    Tensor logp = at::empty({D.n, classes}, opt);
+    s.logp = logp.data_ptr();
+    s.classes = classes;
+    return logp;
+}
+
 template <typename M>
 struct LayeredFn : public torch::autograd::Function<LayeredFn<M>> {
     static Tensor forward(AutogradContext* ctx, Tensor x, at::TensorList P, c10::intrusive_ptr<PlanHolder> holder, Tensor ws, int64_t H, int64_t tokens, int64_t classes,
@@ -454,8 +491,9 @@ struct LayeredFn : public torch::autograd::Function<LayeredFn<M>> {
         for (const Tensor& t : P) save.push_back(t.contiguous());
         Saved s{};
         const auto* plan = reinterpret_cast<const tgt_plan_t*>(holder->h);
+        Tensor logp = own_log_probabilities<M>(s, D, classes, x.options());
         Tensor mem = record(x.options(), [&](Tape& t) { M::forward(t, D, save, x.data_ptr(), plan, ws, eps, true, s); });
-        Tensor logp = log_probabilities(s, D, classes, x.options());
+        if (!s.logp) logp = log_probabilities(s, D, classes, x.options());
         for (const Tensor& t : {x, mem, logp, ws}) save.push_back(t);
         ctx->save_for_backward(save);
         ctx->saved_data["plan"] = holder;
@@ -480,8 +518,14 @@ struct LayeredFn : public torch::autograd::Function<LayeredFn<M>> {
         Tape where;
         where.base = static_cast<char*>(mem.data_ptr());
         M::forward(where, D, sv, x.data_ptr(), plan, ws, eps, true, s);
-        Tensor dlogits = at::_log_softmax_backward_data(grads[0], logp, 1, logp.scalar_type());
-        if (D.Cp != classes) dlogits = at::constant_pad_nd(dlogits, {0, D.Cp - classes});
+        Tensor dlogits = grads[0];
+        if (M::fused_readout(D)) {
+            s.logp = logp.data_ptr();
+            s.classes = classes;
+        } else {
+            dlogits = at::_log_softmax_backward_data(grads[0], logp, 1, logp.scalar_type());
+            if (D.Cp != classes) dlogits = at::constant_pad_nd(dlogits, {0, D.Cp - classes});
+        }
         TORCH_CHECK(dlogits.scalar_type() == x.scalar_type(), "gradient of the logits in another dtype than x");
         dlogits = dlogits.contiguous();
         std::vector<std::vector<int64_t>> shapes;
@@ -527,8 +571,9 @@ Tensor layered(const char* name, const Tensor& x, at::TensorList P, const c10::i
     std::vector<Tensor> p;
     for (const Tensor& t : P) p.push_back(t.contiguous());
     Saved s{};
+    Tensor logp = own_log_probabilities<M>(s, D, classes, x.options());
     Tensor mem = record(x.options(), [&](Tape& t) { M::forward(t, D, p, x.data_ptr(), reinterpret_cast<const tgt_plan_t*>(holder->h), ws, e, false, s); });
-    return log_probabilities(s, D, classes, x.options());
+    return s.logp ? logp : log_probabilities(s, D, classes, x.options());
 }
 Tensor layered_graphormer(const Tensor& x, at::TensorList P, const c10::intrusive_ptr<PlanHolder>& holder, const Tensor& ws, int64_t H, int64_t tokens, int64_t classes,
                           at::ArrayRef<double> eps) {
