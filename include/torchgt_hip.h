@@ -657,6 +657,9 @@ typedef struct {
     float *nd, *partial;
 } tgt_node_bwd_post_args;
 int tgt_node_bwd_post(const tgt_node_bwd_post_args* args, void* stream);
+/* tgt_node_bwd_pre and, on its result, tgt_node_bwd_post of the layer before, in one launch (pre->g_out and post->g_in are not read; LayerNorm in
+ * front, no d_token, no same_bits). */
+int tgt_node_bwd_both(const tgt_node_bwd_pre_args* pre, const tgt_node_bwd_post_args* post, void* stream);
 /* Fixed-order sums of such partials, all of a backward in one launch.  out: mats weights [rows, 64], mats biases [rows],
  * gamma, beta [64] (NULL: not wanted). */
 typedef struct {

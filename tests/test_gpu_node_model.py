@@ -244,3 +244,14 @@ def test_gelu_of_the_fused_layers_is_as_exact_as_the_error_function(cuda, scale)
     (separate,) = _ext.op("linear")(_ext.op("gelu")(u), [one], [zero[0]])
     print(f"gelu, u ~ N(0, {scale}): rms error {rms(fused):.3e}, of the separate kernel {rms(separate):.3e}", flush=True)
     assert rms(fused) <= rms(separate) and float((fused - exact).abs().max()) <= 5e-7
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,classes,layers", [(1, 1, 1), (63, 64, 3), (64, 5, 2), (65, 7, 3), (127, 3, 2), (128, 40, 2), (16384, 9, 2), (16386, 9, 3), (32769, 4, 2)])
+def test_both_sides_of_an_attention_in_one_launch(cuda, dtype, n, classes, layers):
+    """The part in front of an attention and the part behind the one before it as one launch (groups of 64 and 128 nodes that end inside, several
+    groups per workgroup), against the layers one by one"""
+    print(f"both sides: n={n} classes={classes} layers={layers} {dtype}", flush=True)
+    model = scaled(Graphormer(layers, 8, 40, 64, classes, 1, 0.0, 0.0, 0.0, 64, 1), n, dtype, cuda)
+    x = torch.randn(n, 40, generator=torch.Generator().manual_seed(n)).to(cuda, dtype)
+    compare(Graphormer, model, x, GraphPlan(random_edges(n, 1, n + 2, cuda), n + 1), n + 3)

@@ -122,6 +122,7 @@ SIGNATURES = {
     "tgt_node_bwd_workers": (_i32, [_i64]),
     "tgt_node_bwd_pre": (_i32, [_vp, _vp]),
     "tgt_node_bwd_post": (_i32, [_vp, _vp]),
+    "tgt_node_bwd_both": (_i32, [_vp, _vp, _vp]),
     "tgt_node_sums": (_i32, [_vp, _i32, _i32, _vp]),
     "tgt_gt_fwd": (_i32, [_vp, _vp]),
     "tgt_gt_bwd": (_i32, [_vp, _vp]),

@@ -205,236 +205,329 @@ __global__ __launch_bounds__((fwd_waves<T, R, SAME>() * 64)) void k_node_fwd(con
 
 // ---- backward of the part in front of an attention (or of the classes) ------------------------------------------------------
 // NORM false (GT): q, k, v are made of the rows s themselves.
+// What a chain wave has at hand
+template <typename T, int R, int CN> struct Chain {
+    using L = Bwd<T, R, CN>;
+    vec16* stage;
+    const vec16* w;
+    const float* vec;
+    unsigned char *p_dy, *p_x;
+    int lane, wave;
+    // its rows of a group
+    __device__ __forceinline__ int64_t tile(int64_t group) const { return (int64_t)L::kChain * group + wave; }
+    __device__ __forceinline__ Rows rows(int64_t group, int64_t N) const { return Rows(tile(group), N, R); }
+};
+// and a block wave
+template <int P, int PB> struct Blocks {
+    static constexpr int FV = kFragVecs<P>;
+    vec16* w;
+    unsigned char *p_dy, *p_x;
+    int base_dy, base_x;
+    WeightsAhead<FV> next;
+    __device__ __forceinline__ void add(float16_t& acc) const { node_product<P, PB>(acc, p_dy, p_x, base_dy, base_x); }
+};
+
+// One group: d = g_in + what the products and LayerNorm make of dq, dk, dv (or of the classes' gradients).  raw_s and raw_d come with s and
+// the first of the gradients; then_s and then_d say what is asked for when they are free again.
+template <typename T, int R, int CN, bool CLASSES, bool NORM, typename F, typename G>
+__device__ __forceinline__ void pre_chain(const tgt_node_bwd_pre_args& a, const Chain<T, R, CN>& me, int64_t group, Raw<T, R>& raw_s, Raw<T, R>& raw_d, float (&col)[(CLASSES ? 1 : 3) + 2],
+                                          TileOf<R>& d, const F& then_s, const G& then_d) {
+    using L = Bwd<T, R, CN>;
+    constexpr int P = Num<T>::P, NM = CLASSES ? 1 : 3, PB = L::kPlane;
+    const T* src[3] = {reinterpret_cast<const T*>(a.dq), reinterpret_cast<const T*>(a.dk), reinterpret_cast<const T*>(a.dv)};
+    const int64_t N = a.rows;
+    const int lane = me.lane, row = R * me.wave + lane % R, h = lane / R;
+    const Rows rows = me.rows(group, N);
+    TileOf<R> xhat, dy;
+    Frags<P, R> f;
+    settle<T, false>(xhat, raw_s, me.stage, rows, lane);
+    float rstd = 1.f;
+    if constexpr (NORM) rstd = normalise<false>(xhat, a.eps);
+    zero(dy);
+#pragma unroll
+    for (int j = 0; j < NM; ++j) {
+        if (CLASSES) ClassGrads<T, R>(reinterpret_cast<const T*>(a.dlogp), reinterpret_cast<const T*>(a.logp), a.linear, a.classes, a.tokens, me.tile(group) * R, N, me.stage, lane).settle(d);
+        else {
+            settle<T, true>(d, raw_d, me.stage, rows, lane);
+            fetch(raw_d, j + 1 < NM ? src[j + 1] : reinterpret_cast<const T*>(a.g_in), rows, lane);
+        }
+        make_frags(f, d);
+        col[j] += column_sums(d, lane);
+        __syncthreads();                       // weight j is there; j = 0: the planes are free
+        gemm<P>(dy, f, me.w, lane);            // beside product j - 1 of the block waves
+        if (j > 0) __syncthreads();            // product j - 1 is done
+        else {
+            TileOf<R> y;
+            if constexpr (NORM) affine(y, xhat, me.vec, me.vec + kVec, h);
+            else y = xhat;
+            put_tile_planes<PB, P>(me.p_x, row, h, y);
+        }
+        put_planes<PB>(me.p_dy, row, h, f);
+        __syncthreads();                       // planes j are there, weight j has been used
+    }
+    then_s();
+    TGT_EACH(i) dy.set(i, stored(dy.get(i), (const T*)nullptr));
+    if constexpr (NORM) {
+        col[NM + 1] += column_sums(dy, lane);
+        TGT_EACH(i) d.set(i, dy.get(i) * xhat.get(i));
+        col[NM] += column_sums(d, lane);
+    }
+    if (CLASSES) zero(d);
+    else settle<T, true>(d, raw_d, me.stage, rows, lane);
+    then_d();
+    if constexpr (NORM) ln_back(d, dy, xhat, rstd, me.vec, h);
+    else TGT_EACH(i) d.set(i, d.get(i) + dy.get(i));
+}
+// The products beside it.  `after`: the weight that the group's next step begins with.
+template <int NM, int P, int PB> __device__ __forceinline__ void pre_blocks(Blocks<P, PB>& me, const vec16* weights, const vec16* after, float16_t (&acc)[NM]) {
+    constexpr int FV = kFragVecs<P>;
+    me.next.put(me.w);
+    me.next.fetch(NM > 1 ? weights + FV : after);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NM; ++j) {
+        __syncthreads();                       // planes j
+        if (j + 1 < NM) {
+            me.next.put(me.w);
+            me.next.fetch(j + 2 < NM ? weights + (j + 2) * FV : after);
+            __syncthreads();                   // weight j + 1
+        }
+        me.add(acc[j]);
+        if (j + 1 < NM) __syncthreads();       // product j is done
+    }
+}
+
+template <int N> __device__ __forceinline__ void clear(float16_t (&acc)[N]) {
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
+}
+template <int N> __device__ __forceinline__ void clear(float (&col)[N]) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) col[j] = 0.f;
+}
+
+// What the kernels begin with, and the block waves' part of it
+#define TGT_BWD_ROLES()                                                                                                          \
+    using L = Bwd<T, R, CN, NV>;                                                                                                 \
+    constexpr int P = Num<T>::P, FV = kFragVecs<P>, PB = L::kPlane, NC = L::kChain;                                              \
+    extern __shared__ __align__(16) unsigned char smem[];                                                                        \
+    vec16* w = reinterpret_cast<vec16*>(smem + L::kW);                                                                           \
+    float* vec = reinterpret_cast<float*>(smem + L::kVecs);                                                                      \
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);                                 \
+    const Chain<T, R, CN> chain{reinterpret_cast<vec16*>(smem + L::kStage) + wave * RowShape<T, R>::kVecs, w, vec, smem, smem + P * PB, lane, wave}
+#define TGT_BWD_BLOCKS() Blocks<P, PB> blocks{w, smem, smem + P * PB, operand_base((wave - NC) >> 1, lane), operand_base((wave - NC) & 1, lane)}
+
 template <typename T, int R, int CN, bool CLASSES, bool NORM>
 __global__ __launch_bounds__((Bwd<T, R, CN>::kThreads)) void k_node_bwd_pre(const tgt_node_bwd_pre_args a) {
-    using L = Bwd<T, R, CN>;
-    constexpr int P = Num<T>::P, FV = kFragVecs<P>, NM = CLASSES ? 1 : 3, PB = L::kPlane, NC = L::kChain;
-    extern __shared__ __align__(16) unsigned char smem[];
-    unsigned char *p_dy = smem, *p_x = smem + P * PB;
-    vec16* w = reinterpret_cast<vec16*>(smem + L::kW);
-    float* vec = reinterpret_cast<float*>(smem + L::kVecs);
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane / R;
+    constexpr int NV = 5, NM = CLASSES ? 1 : 3;
+    TGT_BWD_ROLES();
     const int64_t N = a.rows, groups = (N + CN - 1) / CN;
     if constexpr (NORM) copy_vecs<2 * kVec / 4, L::kThreads>(reinterpret_cast<vec16*>(vec), reinterpret_cast<const vec16*>(a.v_next));
     __syncthreads();
     float16_t acc[NM];
     float col[NM + 2];
-#pragma unroll
-    for (int j = 0; j < NM; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
-#pragma unroll
-    for (int j = 0; j < NM + 2; ++j) col[j] = 0.f;
+    clear(acc); clear(col);
     if (wave < NC) {
-        vec16* stage = reinterpret_cast<vec16*>(smem + L::kStage) + wave * RowShape<T, R>::kVecs;
-        const T* src[3] = {reinterpret_cast<const T*>(a.dq), reinterpret_cast<const T*>(a.dk), reinterpret_cast<const T*>(a.dv)};
-        const int row = R * wave + lane % R;
         Raw<T, R> raw_s, raw_d;
-        {
-            const Rows rows(NC * (int64_t)blockIdx.x + wave, N, R);
-            fetch(raw_s, reinterpret_cast<const T*>(a.s), rows, lane);
-            if (!CLASSES) fetch(raw_d, src[0], rows, lane);
-        }
+        const auto ask_s = [&](int64_t g) { fetch(raw_s, reinterpret_cast<const T*>(a.s), chain.rows(g, N), lane); };
+        const auto ask_d = [&](int64_t g) { if (!CLASSES) fetch(raw_d, reinterpret_cast<const T*>(a.dq), chain.rows(g, N), lane); };
+        ask_s(blockIdx.x);
+        ask_d(blockIdx.x);
         for (int64_t g0 = blockIdx.x; g0 < groups; g0 += gridDim.x) {
-            const Rows rows(NC * g0 + wave, N, R);
-            TileOf<R> xhat, dy, d;
-            Frags<P, R> f;
-            settle<T, false>(xhat, raw_s, stage, rows, lane);
-            float rstd = 1.f;
-            if constexpr (NORM) rstd = normalise<false>(xhat, a.eps);
-            zero(dy);
-#pragma unroll
-            for (int j = 0; j < NM; ++j) {
-                if (CLASSES) ClassGrads<T, R>(reinterpret_cast<const T*>(a.dlogp), reinterpret_cast<const T*>(a.logp), a.linear, a.classes, a.tokens, (NC * g0 + wave) * R, N, stage, lane).settle(d);
-                else {
-                    settle<T, true>(d, raw_d, stage, rows, lane);
-                    fetch(raw_d, j + 1 < NM ? src[j + 1] : reinterpret_cast<const T*>(a.g_in), rows, lane);
-                }
-                make_frags(f, d);
-                col[j] += column_sums(d, lane);
-                __syncthreads();                       // weight j is there; j = 0: the planes are free
-                gemm<P>(dy, f, w, lane);               // beside product j - 1 of the block waves
-                if (j > 0) __syncthreads();            // product j - 1 is done
-                else {
-                    TileOf<R> y;
-                    if constexpr (NORM) affine(y, xhat, vec, vec + kVec, h);
-                    else y = xhat;
-                    put_tile_planes<PB, P>(p_x, row, h, y);
-                }
-                put_planes<PB>(p_dy, row, h, f);
-                __syncthreads();                       // planes j are there, weight j has been used
-            }
-            if (g0 + gridDim.x < groups) fetch(raw_s, reinterpret_cast<const T*>(a.s), Rows(NC * (g0 + gridDim.x) + wave, N, R), lane);
-            TGT_EACH(i) dy.set(i, stored(dy.get(i), (const T*)nullptr));
-            if constexpr (NORM) {
-                col[NM + 1] += column_sums(dy, lane);
-                TGT_EACH(i) d.set(i, dy.get(i) * xhat.get(i));
-                col[NM] += column_sums(d, lane);
-            }
-            if (CLASSES) zero(d);
-            else {
-                settle<T, true>(d, raw_d, stage, rows, lane);
-                if (g0 + gridDim.x < groups) fetch(raw_d, src[0], Rows(NC * (g0 + gridDim.x) + wave, N, R), lane);
-            }
-            if constexpr (NORM) ln_back(d, dy, xhat, rstd, vec, h);
-            else TGT_EACH(i) d.set(i, d.get(i) + dy.get(i));
-            put_rows(reinterpret_cast<T*>(a.g_out), d, stage, rows, lane);
-            if (a.d_token && NC * g0 + wave < (a.tokens + R - 1) / R) put_rows(reinterpret_cast<T*>(a.d_token), d, stage, Rows(NC * g0 + wave, a.tokens, R), lane);
+            TileOf<R> d;
+            const int64_t ahead = g0 + gridDim.x;
+            pre_chain<T, R, CN, CLASSES, NORM>(a, chain, g0, raw_s, raw_d, col, d, [&]() { if (ahead < groups) ask_s(ahead); }, [&]() { if (ahead < groups) ask_d(ahead); });
+            put_rows(reinterpret_cast<T*>(a.g_out), d, chain.stage, chain.rows(g0, N), lane);
+            if (a.d_token && chain.tile(g0) < (a.tokens + R - 1) / R) put_rows(reinterpret_cast<T*>(a.d_token), d, chain.stage, Rows(chain.tile(g0), a.tokens, R), lane);
         }
     } else {
-        const int q = wave - NC, base_dy = operand_base(q >> 1, lane), base_x = operand_base(q & 1, lane);
+        TGT_BWD_BLOCKS();
         const vec16* weights = reinterpret_cast<const vec16*>(a.w_back);
-        WeightsAhead<FV> next;
-        next.fetch(weights);
-        for (int64_t g0 = blockIdx.x; g0 < groups; g0 += gridDim.x) {
-            next.put(w);
-            next.fetch(weights + (NM > 1 ? FV : 0));
-            __syncthreads();
-#pragma unroll
-            for (int j = 0; j < NM; ++j) {
-                __syncthreads();                       // planes j
-                if (j + 1 < NM) {
-                    next.put(w);
-                    next.fetch(weights + (j + 2 < NM ? j + 2 : 0) * FV);
-                    __syncthreads();                   // weight j + 1
-                }
-                node_product<P, PB>(acc[j], p_dy, p_x, base_dy, base_x);
-                if (j + 1 < NM) __syncthreads();       // product j is done
-            }
-        }
+        blocks.next.fetch(weights);
+        for (int64_t g0 = blockIdx.x; g0 < groups; g0 += gridDim.x) pre_blocks<NM>(blocks, weights, weights, acc);
     }
     write_partial<L, NM, NM + 2>(a.partial + (int64_t)blockIdx.x * (NM * 4096 + (NM + 2) * 64), acc, col, reinterpret_cast<float*>(smem), wave, lane);
 }
 
 // ---- backward of the part behind an attention -------------------------------------------------------------------------------
+// One group: g = ds' in, ds out, and da (d_attn) and the sparse attention's nd to memory.  take_g: hands the group's g over; then: asks for the
+// next group's rows when the registers of these are free.
+template <typename T, int R, int CN, bool SAME, typename F, typename G>
+__device__ __forceinline__ void post_chain(const tgt_node_bwd_post_args& a, const Chain<T, R, CN>& me, const Rows& rows, Raw<T, R>& raw_a, Raw<T, R>& raw_s, float (&col)[5],
+                                           const F& take_g, const G& then) {
+    using L = Bwd<T, R, CN>;
+    constexpr int P = Num<T>::P, PB = L::kPlane;
+    constexpr bool KEEP = P == 1 || CN == 64;      // whether there are registers for the planes of LayerNorm's output
+    const int lane = me.lane, row = R * me.wave + lane % R, h = lane / R;
+    const vec16* w = me.w;
+    const float* vec = me.vec;
+    vec16* stage = me.stage;
+    unsigned char *p_dy = me.p_dy, *p_x = me.p_x;
+    TileOf<R> g, xhat, slope, t;
+    Frags<P, R> f, fy;      // fy: LayerNorm's output, formed again from xhat where it is not kept
+    settle<T, false>(t, raw_a, stage, rows, lane);
+    make_frags(f, t);
+    settle<T, false>(xhat, raw_s, stage, rows, lane);
+    take_g(g);
+    col[2] += column_sums(g, lane);
+    __syncthreads();                                        // Wo is there; product Wo of the round before is done
+    linear<P, SAME>(t, f, w, vec, lane);
+    __syncthreads();                                        // Wo has been used
+    TGT_EACH(i) xhat.set(i, xhat.get(i) + stored(t.get(i), (const T*)nullptr));      // s1
+    t = xhat;
+    const MeanRstd stat = row_stats<SAME>(t, a.eps);
+    TGT_EACH(i) {      // LayerNorm's output is made of s1, its backward reads s1 as the stream holds it
+        t.set(i, (t.get(i) - stat.mean) * stat.rstd);
+        xhat.set(i, (stored(xhat.get(i), (const T*)nullptr) - stat.mean) * stat.rstd);
+    }
+    affine(t, t, vec + kVec, vec + 2 * kVec, h);
+    make_frags(fy, t);
+    __syncthreads();                                        // W1
+    linear<P, SAME>(t, fy, w, vec + 3 * kVec, lane);           // u
+    __syncthreads();                                        // W1 has been used
+    gelu<T, SAME>(t, slope);
+    put_tile_planes<PB, P>(p_x, row, h, t);
+    make_frags(f, g);
+    put_planes<PB>(p_dy, row, h, f);
+    __syncthreads();                                        // planes of W2; W2^T
+    zero(t);
+    gemm<P>(t, f, w, lane);                                 // d gelu, beside product W2
+    TGT_EACH(i) t.set(i, stored(t.get(i) * slope.get(i), (const T*)nullptr));      // du
+    col[1] += column_sums(t, lane);
+    make_frags(f, t);
+    if (!KEEP) {
+        forget(xhat);
+        affine(t, xhat, vec + kVec, vec + 2 * kVec, h);
+    }
+    __syncthreads();                                        // product W2 is done, W2^T has been used
+    put_planes<PB>(p_dy, row, h, f);
+    if constexpr (KEEP) put_planes<PB>(p_x, row, h, fy);
+    else put_tile_planes<PB, P>(p_x, row, h, t);
+    __syncthreads();                                        // planes of W1; W1^T
+    fetch(raw_a, reinterpret_cast<const T*>(a.attn), rows, lane);
+    zero(t);
+    gemm<P>(t, f, w, lane);                                 // d LN, beside product W1
+    TGT_EACH(i) t.set(i, stored(t.get(i), (const T*)nullptr));
+    col[4] += column_sums(t, lane);
+    ln_back(g, t, xhat, stat.rstd, vec + kVec, h);
+    TGT_EACH(i) g.set(i, stored(g.get(i), (const T*)nullptr));
+    TGT_EACH(i) t.set(i, t.get(i) * xhat.get(i));
+    col[3] += column_sums(t, lane);
+    col[0] += column_sums(g, lane);
+    put_rows(reinterpret_cast<T*>(a.g_out), g, stage, rows, lane);
+    make_frags(f, g);
+    settle<T, false>(t, raw_a, stage, rows, lane);
+    __syncthreads();                                        // product W1 is done, W1^T has been used
+    put_planes<PB>(p_dy, row, h, f);
+    put_tile_planes<PB, P>(p_x, row, h, t);
+    __syncthreads();                                        // planes of Wo; Wo^T
+    if (P == 1) then();      // float32 has the registers only after the products
+    zero(g);
+    gemm<P>(g, f, w, lane);                                 // da, beside product Wo
+    __syncthreads();                                        // Wo^T has been used
+    put_rows(reinterpret_cast<T*>(a.d_attn), g, stage, rows, lane);
+    if (a.nd) put_node_side<T>(g, t, a.Z, a.nd, a.heads, rows.first + lane % R, h, lane % R < rows.left);
+    if (P != 1) then();
+}
+template <int P, int PB> __device__ __forceinline__ void post_blocks(Blocks<P, PB>& me, const vec16* fw, const vec16* bw, const vec16* after, float16_t (&acc)[3]) {
+    constexpr int FV = kFragVecs<P>;
+    me.next.hand_over(me.w, fw + FV);             // Wo, then on to W1
+    __syncthreads();
+    me.next.hand_over(me.w, bw + 2 * FV);         // W1
+    __syncthreads();
+    me.next.hand_over(me.w, bw + FV);             // W2^T and the planes of W2
+    me.add(acc[2]);
+    __syncthreads();
+    me.next.hand_over(me.w, bw);                  // W1^T and the planes of W1
+    me.add(acc[1]);
+    __syncthreads();
+    me.next.hand_over(me.w, after);               // Wo^T and the planes of Wo
+    me.add(acc[0]);
+    __syncthreads();
+}
+
 template <typename T, int R, int CN, bool SAME>
 __global__ __launch_bounds__((Bwd<T, R, CN>::kThreads)) void k_node_bwd_post(const tgt_node_bwd_post_args a) {
-    using L = Bwd<T, R, CN>;
-    constexpr int P = Num<T>::P, FV = kFragVecs<P>, PB = L::kPlane, NC = L::kChain;
-    constexpr bool KEEP = P == 1 || CN == 64;      // whether there are registers for the planes of LayerNorm's output
-    extern __shared__ __align__(16) unsigned char smem[];
-    unsigned char *p_dy = smem, *p_x = smem + P * PB;
-    vec16* w = reinterpret_cast<vec16*>(smem + L::kW);
-    float* vec = reinterpret_cast<float*>(smem + L::kVecs);
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane % R, h = lane / R;
+    constexpr int NV = 5;
+    TGT_BWD_ROLES();
     const int64_t N = a.rows, groups = (N + CN - 1) / CN;
     copy_vecs<5 * kVec / 4, L::kThreads>(reinterpret_cast<vec16*>(vec), reinterpret_cast<const vec16*>(a.v_post));
     __syncthreads();
     float16_t acc[3];       // Wo, W1, W2
     float col[5];           // bo, b1, b2, gamma, beta
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
-#pragma unroll
-    for (int j = 0; j < 5; ++j) col[j] = 0.f;
+    clear(acc); clear(col);
     if (wave < NC) {
-        vec16* stage = reinterpret_cast<vec16*>(smem + L::kStage) + wave * RowShape<T, R>::kVecs;
-        const int row = R * wave + n;
         Raw<T, R> raw_a, raw_s, raw_g;
-        {
-            const Rows rows(NC * (int64_t)blockIdx.x + wave, N, R);
+        const auto ask = [&](int64_t g) {
+            const Rows rows = chain.rows(g, N);
             fetch(raw_a, reinterpret_cast<const T*>(a.attn), rows, lane);
             fetch(raw_s, reinterpret_cast<const T*>(a.s), rows, lane);
             fetch(raw_g, reinterpret_cast<const T*>(a.g_in), rows, lane);
-        }
+        };
+        ask(blockIdx.x);
         for (int64_t g0 = blockIdx.x; g0 < groups; g0 += gridDim.x) {
-            const Rows rows(NC * g0 + wave, N, R);
-            const auto fetch_next = [&]() {
-                if (g0 + gridDim.x >= groups) return;
-                const Rows ahead(NC * (g0 + gridDim.x) + wave, N, R);
-                fetch(raw_a, reinterpret_cast<const T*>(a.attn), ahead, lane);
-                fetch(raw_s, reinterpret_cast<const T*>(a.s), ahead, lane);
-                fetch(raw_g, reinterpret_cast<const T*>(a.g_in), ahead, lane);
-            };
-            TileOf<R> g, xhat, slope, t;
-            Frags<P, R> f, fy;      // fy: LayerNorm's output, formed again from xhat where it is not kept
-            settle<T, false>(t, raw_a, stage, rows, lane);
-            make_frags(f, t);
-            settle<T, false>(xhat, raw_s, stage, rows, lane);
-            settle<T, true>(g, raw_g, stage, rows, lane);
-            col[2] += column_sums(g, lane);
-            __syncthreads();                                        // Wo is there; product Wo of the round before is done
-            linear<P, SAME>(t, f, w, vec, lane);
-            __syncthreads();                                        // Wo has been used
-            TGT_EACH(i) xhat.set(i, xhat.get(i) + stored(t.get(i), (const T*)nullptr));      // s1
-            t = xhat;
-            const MeanRstd stat = row_stats<SAME>(t, a.eps);
-            TGT_EACH(i) {      // LayerNorm's output is made of s1, its backward reads s1 as the stream holds it
-                t.set(i, (t.get(i) - stat.mean) * stat.rstd);
-                xhat.set(i, (stored(xhat.get(i), (const T*)nullptr) - stat.mean) * stat.rstd);
-            }
-            affine(t, t, vec + kVec, vec + 2 * kVec, h);
-            make_frags(fy, t);
-            __syncthreads();                                        // W1
-            linear<P, SAME>(t, fy, w, vec + 3 * kVec, lane);           // u
-            __syncthreads();                                        // W1 has been used
-            gelu<T, SAME>(t, slope);
-            put_tile_planes<PB, P>(p_x, row, h, t);
-            make_frags(f, g);
-            put_planes<PB>(p_dy, row, h, f);
-            __syncthreads();                                        // planes of W2; W2^T
-            zero(t);
-            gemm<P>(t, f, w, lane);                                 // d gelu, beside product W2
-            TGT_EACH(i) t.set(i, stored(t.get(i) * slope.get(i), (const T*)nullptr));      // du
-            col[1] += column_sums(t, lane);
-            make_frags(f, t);
-            if (!KEEP) {
-                forget(xhat);
-                affine(t, xhat, vec + kVec, vec + 2 * kVec, h);
-            }
-            __syncthreads();                                        // product W2 is done, W2^T has been used
-            put_planes<PB>(p_dy, row, h, f);
-            if constexpr (KEEP) put_planes<PB>(p_x, row, h, fy);
-            else put_tile_planes<PB, P>(p_x, row, h, t);
-            __syncthreads();                                        // planes of W1; W1^T
-            fetch(raw_a, reinterpret_cast<const T*>(a.attn), rows, lane);
-            zero(t);
-            gemm<P>(t, f, w, lane);                                 // d LN, beside product W1
-            TGT_EACH(i) t.set(i, stored(t.get(i), (const T*)nullptr));
-            col[4] += column_sums(t, lane);
-            ln_back(g, t, xhat, stat.rstd, vec + kVec, h);
-            TGT_EACH(i) g.set(i, stored(g.get(i), (const T*)nullptr));
-            TGT_EACH(i) t.set(i, t.get(i) * xhat.get(i));
-            col[3] += column_sums(t, lane);
-            col[0] += column_sums(g, lane);
-            put_rows(reinterpret_cast<T*>(a.g_out), g, stage, rows, lane);
-            make_frags(f, g);
-            settle<T, false>(t, raw_a, stage, rows, lane);
-            __syncthreads();                                        // product W1 is done, W1^T has been used
-            put_planes<PB>(p_dy, row, h, f);
-            put_tile_planes<PB, P>(p_x, row, h, t);
-            __syncthreads();                                        // planes of Wo; Wo^T
-            if (P == 1) fetch_next();      // float32 has the registers only after the products
-            zero(g);
-            gemm<P>(g, f, w, lane);                                 // da, beside product Wo
-            __syncthreads();                                        // Wo^T has been used
-            put_rows(reinterpret_cast<T*>(a.d_attn), g, stage, rows, lane);
-            if (a.nd) put_node_side<T>(g, t, a.Z, a.nd, a.heads, rows.first + n, h, n < rows.left);
-            if (P != 1) fetch_next();
+            const Rows rows = chain.rows(g0, N);
+            post_chain<T, R, CN, SAME>(a, chain, rows, raw_a, raw_s, col, [&](TileOf<R>& g) { settle<T, true>(g, raw_g, chain.stage, rows, lane); },
+                                       [&]() { if (g0 + gridDim.x < groups) ask(g0 + gridDim.x); });
         }
     } else {
-        const int q = wave - NC, base_dy = operand_base(q >> 1, lane), base_x = operand_base(q & 1, lane);
+        TGT_BWD_BLOCKS();
         const vec16 *fw = reinterpret_cast<const vec16*>(a.w_post), *bw = reinterpret_cast<const vec16*>(a.w_back);
-        WeightsAhead<FV> next;
-        next.fetch(fw);
-        for (int64_t g0 = blockIdx.x; g0 < groups; g0 += gridDim.x) {
-            next.hand_over(w, fw + FV);             // Wo, then on to W1
-            __syncthreads();
-            next.hand_over(w, bw + 2 * FV);         // W1
-            __syncthreads();
-            next.hand_over(w, bw + FV);             // W2^T and the planes of W2
-            node_product<P, PB>(acc[2], p_dy, p_x, base_dy, base_x);
-            __syncthreads();
-            next.hand_over(w, bw);                  // W1^T and the planes of W1
-            node_product<P, PB>(acc[1], p_dy, p_x, base_dy, base_x);
-            __syncthreads();
-            next.hand_over(w, fw);                  // Wo^T and the planes of Wo
-            node_product<P, PB>(acc[0], p_dy, p_x, base_dy, base_x);
-            __syncthreads();
-        }
+        blocks.next.fetch(fw);
+        for (int64_t g0 = blockIdx.x; g0 < groups; g0 += gridDim.x) post_blocks(blocks, fw, bw, fw, acc);
     }
     write_partial<L, 3, 5>(a.partial + (int64_t)blockIdx.x * (3 * 4096 + 5 * 64), acc, col, reinterpret_cast<float*>(smem), wave, lane);
+}
+
+// The part in front of an attention (or the classes) and the part behind the attention before it, one after the other for a group: what
+// passes between them (g_out of the one, g_in of the other) stays in registers, and a launch's first and last microseconds
+// are there once.  A training step of four layers as a replayed graph, us, two launches / one: float32 4 K nodes 330 / 323, 16 K 398 / 389, 64 K
+// 1010 / 1001; bf16 220 / 214, 295 / 283, 567 / 541 (and four launches less of host time).
+constexpr int kBothVecs = 7;
+template <typename T, int R, int CN, bool CLASSES>
+__global__ __launch_bounds__((Bwd<T, R, CN, kBothVecs>::kThreads)) void k_node_bwd_both(const tgt_node_bwd_pre_args a, const tgt_node_bwd_post_args b) {
+    constexpr int NV = kBothVecs, NM = CLASSES ? 1 : 3;
+    TGT_BWD_ROLES();
+    const int64_t N = a.rows, groups = (N + CN - 1) / CN;
+    copy_vecs<2 * kVec / 4, L::kThreads>(reinterpret_cast<vec16*>(vec), reinterpret_cast<const vec16*>(a.v_next));
+    copy_vecs<5 * kVec / 4, L::kThreads>(reinterpret_cast<vec16*>(vec + 2 * kVec), reinterpret_cast<const vec16*>(b.v_post));
+    __syncthreads();
+    float16_t acc[NM], acc_b[3];
+    float col[NM + 2], col_b[5];
+    clear(acc); clear(col); clear(acc_b); clear(col_b);
+    if (wave < NC) {
+        Chain<T, R, CN> behind = chain;
+        behind.vec = vec + 2 * kVec;
+        Raw<T, R> raw_s, raw_d, raw_a;
+        const auto ask = [&](int64_t g) {
+            const Rows rows = chain.rows(g, N);
+            fetch(raw_s, reinterpret_cast<const T*>(a.s), rows, lane);
+            if (!CLASSES) fetch(raw_d, reinterpret_cast<const T*>(a.dq), rows, lane);
+        };
+        ask(blockIdx.x);
+        for (int64_t g0 = blockIdx.x; g0 < groups; g0 += gridDim.x) {
+            TileOf<R> d;
+            const Rows rows = chain.rows(g0, N);
+            pre_chain<T, R, CN, CLASSES, true>(a, chain, g0, raw_s, raw_d, col, d, [&]() { fetch(raw_a, reinterpret_cast<const T*>(b.attn), rows, lane); },
+                                               [&]() { fetch(raw_s, reinterpret_cast<const T*>(b.s), rows, lane); });
+            post_chain<T, R, CN, false>(b, behind, rows, raw_a, raw_s, col_b,
+                                        [&](TileOf<R>& g) { TGT_EACH(i) g.set(i, lane % R < rows.left ? stored(d.get(i), (const T*)nullptr) : 0.f); },
+                                        [&]() { if (g0 + gridDim.x < groups) ask(g0 + gridDim.x); });
+        }
+    } else {
+        TGT_BWD_BLOCKS();
+        const vec16 *weights = reinterpret_cast<const vec16*>(a.w_back), *fw = reinterpret_cast<const vec16*>(b.w_post), *bw = reinterpret_cast<const vec16*>(b.w_back);
+        blocks.next.fetch(weights);
+        for (int64_t g0 = blockIdx.x; g0 < groups; g0 += gridDim.x) {
+            pre_blocks<NM>(blocks, weights, fw, acc);
+            post_blocks(blocks, fw, bw, weights, acc_b);
+        }
+    }
+    write_partial<L, NM, NM + 2>(a.partial + (int64_t)blockIdx.x * (NM * 4096 + (NM + 2) * 64), acc, col, reinterpret_cast<float*>(smem), wave, lane);
+    __syncthreads();
+    write_partial<L, 3, 5>(b.partial + (int64_t)blockIdx.x * (3 * 4096 + 5 * 64), acc_b, col_b, reinterpret_cast<float*>(smem), wave, lane);
 }
 
 // ---- sums of the partials -----------------------------------------------------------------------------------------------
@@ -515,6 +608,12 @@ template <typename T, int R, int CN, bool SAME> int launch_bwd_post(const tgt_no
     static std::atomic<uint64_t> done{0};
     return launch(&k_node_bwd_post<T, R, CN, SAME>, done, bwd_workers(a.rows), L::kThreads, L::kBytes, st, a);
 }
+template <typename T, int R, int CN> int launch_bwd_both(const tgt_node_bwd_pre_args& a, const tgt_node_bwd_post_args& b, hipStream_t st) {
+    using L = Bwd<T, R, CN, kBothVecs>;
+    static std::atomic<uint64_t> done[2];
+    if (a.dlogp) return launch(&k_node_bwd_both<T, R, CN, true>, done[0], bwd_workers(a.rows), L::kThreads, L::kBytes, st, a, b);
+    return launch(&k_node_bwd_both<T, R, CN, false>, done[1], bwd_workers(a.rows), L::kThreads, L::kBytes, st, a, b);
+}
 bool dtype_ok(int dtype) { return dtype == TGT_DTYPE_F32 || dtype == TGT_DTYPE_BF16; }
 
 }  // namespace
@@ -579,11 +678,25 @@ int tgt_node_fwd(const tgt_node_fwd_args* a, void* stream) {
 
 int tgt_node_bwd_workers(int64_t rows) { return rows < 0 ? -1 : tgt::bwd_workers(rows); }
 
-int tgt_node_bwd_pre(const tgt_node_bwd_pre_args* a, void* stream) {
+static int check_pre(const tgt_node_bwd_pre_args* a) {
     using namespace tgt;
-    if (!a || a->rows < 1 || !dtype_ok(a->dtype) || !a->s || !a->g_out || !a->w_back || (a->dlogp && !a->v_next) || !a->partial) return bad("tgt_node_bwd_pre", "null or bad argument");
+    if (!a || a->rows < 1 || !dtype_ok(a->dtype) || !a->s || !a->w_back || (a->dlogp && !a->v_next) || !a->partial) return bad("tgt_node_bwd_pre", "null or bad argument");
     if (a->dlogp ? ((!a->logp && !a->linear) || a->classes < 1 || a->classes > 64 || a->tokens < 0) : (!a->dq || !a->dk || !a->dv || !a->g_in))
         return bad("tgt_node_bwd_pre", "dq, dk, dv, g_in or dlogp, logp and 1 to 64 classes are needed");
+    return TGT_OK;
+}
+static int check_post(const tgt_node_bwd_post_args* a) {
+    using namespace tgt;
+    if (!a || a->rows < 1 || !dtype_ok(a->dtype) || !a->s || !a->attn || !a->g_out || !a->d_attn || !a->w_post || !a->w_back || !a->v_post || !a->partial)
+        return bad("tgt_node_bwd_post", "null or bad argument");
+    if (a->nd && (!a->Z || (a->heads != 8 && a->heads != 4 && a->heads != 2))) return bad("tgt_node_bwd_post", "nd needs Z and 8, 4 or 2 heads");
+    return TGT_OK;
+}
+
+int tgt_node_bwd_pre(const tgt_node_bwd_pre_args* a, void* stream) {
+    using namespace tgt;
+    if (int rc = check_pre(a)) return rc;
+    if (!a->g_out) return bad("tgt_node_bwd_pre", "null or bad argument");
     KernelTimer t(KS_NODE_BWD_PRE, (hipStream_t)stream);
     const hipStream_t st = (hipStream_t)stream;
     if (a->dtype == TGT_DTYPE_F32) return groups_of_64(a->rows, true) ? dispatch_bwd_pre<float, 16, 64>(*a, st) : dispatch_bwd_pre<float, 16, 128>(*a, st);
@@ -592,15 +705,26 @@ int tgt_node_bwd_pre(const tgt_node_bwd_pre_args* a, void* stream) {
 
 int tgt_node_bwd_post(const tgt_node_bwd_post_args* a, void* stream) {
     using namespace tgt;
-    if (!a || a->rows < 1 || !dtype_ok(a->dtype) || !a->s || !a->attn || !a->g_in || !a->g_out || !a->d_attn || !a->w_post || !a->w_back || !a->v_post || !a->partial)
-        return bad("tgt_node_bwd_post", "null or bad argument");
-    if (a->nd && (!a->Z || (a->heads != 8 && a->heads != 4 && a->heads != 2))) return bad("tgt_node_bwd_post", "nd needs Z and 8, 4 or 2 heads");
+    if (int rc = check_post(a)) return rc;
+    if (!a->g_in) return bad("tgt_node_bwd_post", "null or bad argument");
     KernelTimer t(KS_NODE_BWD_POST, (hipStream_t)stream);
     const hipStream_t st = (hipStream_t)stream;
     if (a->dtype == TGT_DTYPE_F32) return groups_of_64(a->rows, true) ? launch_bwd_post<float, 16, 64, false>(*a, st) : launch_bwd_post<float, 16, 128, false>(*a, st);
     const bool small = groups_of_64(a->rows, false);
     if (a->same_bits) return small ? launch_bwd_post<nbf16, 32, 64, true>(*a, st) : launch_bwd_post<nbf16, 32, 128, true>(*a, st);
     return small ? launch_bwd_post<nbf16, 16, 64, false>(*a, st) : launch_bwd_post<nbf16, 16, 128, false>(*a, st);
+}
+
+int tgt_node_bwd_both(const tgt_node_bwd_pre_args* a, const tgt_node_bwd_post_args* b, void* stream) {
+    using namespace tgt;
+    if (int rc = check_pre(a)) return rc;
+    if (int rc = check_post(b)) return rc;
+    if (a->rows != b->rows || a->dtype != b->dtype || !a->v_next || a->d_token || b->same_bits) return bad("tgt_node_bwd_both", "the same rows, LayerNorm in front, no tokens' gradient, no same_bits");
+    KernelTimer t(KS_NODE_BWD_POST, (hipStream_t)stream);
+    const hipStream_t st = (hipStream_t)stream;
+    // float32: groups of 64 whatever the rows (eight waves have 256 registers each; with twelve 209 of a lane's go to scratch: 64 K rows 122 us, 90 with 64)
+    if (a->dtype == TGT_DTYPE_F32) return launch_bwd_both<float, 16, 64>(*a, *b, st);
+    return groups_of_64(a->rows, false) ? launch_bwd_both<nbf16, 16, 64>(*a, *b, st) : launch_bwd_both<nbf16, 16, 128>(*a, *b, st);
 }
 
 int tgt_node_sums(const tgt_node_sum* sums, int count, int dtype, void* stream) {

@@ -172,15 +172,15 @@ struct NodeGraphormerFn : public torch::autograd::Function<NodeGraphormerFn> {
             next_partial += (int64_t)workers * (mats * 4096 + (mats + 2) * 64);
             return s;
         };
+        // the part in front of an attention (or the classes) waits for the part behind the attention before it: one launch for both
+        tgt_node_bwd_pre_args a{};
         {
-            tgt_node_bwd_pre_args a{};
             a.rows = N; a.dtype = code; a.tokens = (int)D.tokens; a.classes = (int)D.C; a.eps = (float)eps[2 * L];
             a.s = at_row(rows, L * N); a.dlogp = dlogp.data_ptr(); a.logp = logp.data_ptr();
             a.w_back = packed.transposed(6 * L); a.v_next = packed.vec(10 * L); a.g_out = g[0]; a.partial = next_partial;
             tgt_node_sum& s = new_sum(1, (int)D.C);
             const Tensor* c = &G.t[3 + 16 * L];
             s.out[0] = c[2].data_ptr(); s.out[1] = c[3].data_ptr(); s.out[2] = c[0].data_ptr(); s.out[3] = c[1].data_ptr();
-            check(tgt_node_bwd_pre(&a, stream), "tgt_node_bwd_pre");
         }
         for (int64_t l = L - 1; l >= 0; --l) {
             const Tensor* w = &G.t[3 + 16 * l];
@@ -194,18 +194,18 @@ struct NodeGraphormerFn : public torch::autograd::Function<NodeGraphormerFn> {
             tgt_node_sum& s = new_sum(3, (int)kWidth);
             static const int post[8] = {8, 12, 14, 9, 13, 15, 10, 11}, pre[8] = {2, 4, 6, 3, 5, 7, 0, 1};
             for (int i = 0; i < 8; ++i) s.out[i] = w[post[i]].data_ptr();
-            check(tgt_node_bwd_post(&b, stream), "tgt_node_bwd_post");
+            check(tgt_node_bwd_both(&a, &b, stream), "tgt_node_bwd_both");
             check(tgt_sparse_attn_bwd_from_nd(plan, q, k, v, (int)H, (int)(kWidth / H), code, da, dq, dk, dvr, ws.data_ptr(), ws.numel(), stream),
                   "tgt_sparse_attn_bwd_from_nd");
-            tgt_node_bwd_pre_args a{};
+            a = tgt_node_bwd_pre_args{};
             a.rows = N; a.dtype = code; a.tokens = (int)D.tokens; a.eps = (float)eps[2 * l];
             a.dq = dq; a.dk = dk; a.dv = dvr; a.g_in = g[1]; a.s = at_row(rows, l * N);
             a.w_back = packed.transposed(6 * l + 3); a.v_next = packed.vec(10 * l + 5); a.g_out = g[0]; a.partial = next_partial;
             a.d_token = l == 0 && D.tokens ? G.t[2].data_ptr() : nullptr;
             tgt_node_sum& s2 = new_sum(3, (int)kWidth);
             for (int i = 0; i < 8; ++i) s2.out[i] = w[pre[i]].data_ptr();
-            check(tgt_node_bwd_pre(&a, stream), "tgt_node_bwd_pre");
         }
+        check(tgt_node_bwd_pre(&a, stream), "tgt_node_bwd_pre");
         check(tgt_node_sums(sums.data(), (int)sums.size(), code, stream), "tgt_node_sums");
         Tensor dx;
         {
