@@ -606,6 +606,20 @@ int tgt_node_pack(const void* const* mats, const int* ld, const int* rows, int n
 /* The same for weights [rows[i] <= 64, cols[i] <= 64] with ld[i] >= cols[i] (columns behind cols[i] count as zero). */
 int tgt_node_pack_parts(const void* const* mats, const int* ld, const int* rows, const int* cols, int n_mats, const void* const* vecs,
                         const int* lens, int n_vecs, int dtype, void* d_frags, float* d_vecs, void* stream);
+/* The same as arguments of tgt_linear_fwd_and_pack: tgt_linear_fwd with one output and, beside it, tgt_node_pack_parts (one launch for 1 to 128 input
+ * features other than 64 and 64 output features, else one after the other; the packed parameters and y may not depend on each other). */
+typedef struct {
+    const void* const* mats;
+    const int *ld, *rows, *cols;
+    int n_mats;
+    const void* const* vecs;
+    const int* lens;
+    int n_vecs;
+    void* d_frags;
+    float* d_vecs;
+} tgt_node_pack_args;
+int tgt_linear_fwd_and_pack(const void* d_x, const void* d_W, const void* d_b, void* d_y, int64_t N, int in_features, int out_features,
+                            const tgt_node_pack_args* pack, int dtype, void* stream);
 /* Forward.  attn: the attention's rows [rows, 64], or NULL for the part in front of the first layer (then s' = s_in, whose
  * first `tokens` rows are taken from `token` and written to s_out; s_in and s_out are the same array).  w_post: packed Wo,
  * W1, W2; v_post: bo, gamma, beta, b1, b2.  q, k, v: rows for the next attention (w_next: packed Wq, Wk, Wv; v_next: gamma,

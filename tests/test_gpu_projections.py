@@ -439,3 +439,39 @@ def test_float32_linears_of_any_width_are_as_exact_as_float32_products(cuda, N, 
         err = rms(got, want)
         print(f"  {name}: {err:.2e} (bound {bound:.2e})", flush=True)
         assert err <= bound, name
+
+
+class _PackArgs(ctypes.Structure):      # tgt_node_pack_args
+    _fields_ = [(k, ctypes.c_void_p) for k in ("mats", "ld", "rows", "cols")] + [("n_mats", ctypes.c_int), ("vecs", ctypes.c_void_p), ("lens", ctypes.c_void_p), ("n_vecs", ctypes.c_int),
+                                                                                ("d_frags", ctypes.c_void_p), ("d_vecs", ctypes.c_void_p)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,features,out,n_mats,n_vecs", [(1, 8, 64, 1, 1), (127, 128, 64, 3, 5), (129, 120, 64, 25, 43), (128, 64, 64, 2, 3), (300, 136, 64, 2, 9), (33, 32, 40, 1, 4), (64, 72, 64, 96, 160),
+                                                          (64, 72, 64, 97, 3), (64, 72, 64, 3, 161), (0, 72, 64, 3, 7)])
+def test_linear_with_the_packing_beside_it(cuda, dtype, n, features, out, n_mats, n_vecs):
+    """tgt_linear_fwd_and_pack gives the bits of tgt_node_pack_parts and of tgt_linear_fwd, in one launch and where it takes two"""
+    print(f"linear and pack: n={n} features={features} out={out} mats={n_mats} vecs={n_vecs} {dtype}", flush=True)
+    L, g, code = _lib.lib(), torch.Generator().manual_seed(n + features + n_mats), (_lib.DTYPE_F32 if dtype == torch.float32 else _lib.DTYPE_BF16)
+    rand = lambda *s: torch.randn(*s, generator=g).to(cuda, dtype)
+    x, W, b = rand(n, features), rand(out, features), rand(out)
+    mats, vecs = [rand(64 - i % 3, 64 - 2 * (i % 5)) for i in range(n_mats)], [rand(64 - i % 7) for i in range(n_vecs)]
+    ints = lambda v: (ctypes.c_int * len(v))(*v)
+    m, ld, rows, cols = (ctypes.c_void_p * n_mats)(*[t.data_ptr() for t in mats]), ints([t.shape[1] for t in mats]), ints([t.shape[0] for t in mats]), ints([t.shape[1] for t in mats])
+    v, lens = (ctypes.c_void_p * n_vecs)(*[t.data_ptr() for t in vecs]), ints([t.numel() for t in vecs])
+    st, at = torch.cuda.current_stream(cuda).cuda_stream, ctypes.addressof
+    got = []
+    for one in (True, False):
+        frags, flat, y = torch.full((L.tgt_node_frag_bytes(n_mats, code),), 7, dtype=torch.uint8, device=cuda), torch.full((n_vecs, 64), 7.0, device=cuda), torch.full((n, out), 7.0, device=cuda).to(dtype)
+        if one:
+            p = _PackArgs(at(m), at(ld), at(rows), at(cols), n_mats, at(v), at(lens), n_vecs, frags.data_ptr(), flat.data_ptr())
+            _lib.check(L.tgt_linear_fwd_and_pack(x.data_ptr(), W.data_ptr(), b.data_ptr(), y.data_ptr(), n, features, out, at(p), code, st))
+        else:
+            _lib.check(L.tgt_node_pack_parts(at(m), at(ld), at(rows), at(cols), n_mats, at(v), at(lens), n_vecs, code, frags.data_ptr(), flat.data_ptr(), st))
+            w1, b1, y1 = ((ctypes.c_void_p * 1)(t.data_ptr()) for t in (W, b, y))
+            _lib.check(L.tgt_linear_fwd(x.data_ptr(), at(w1), at(b1), at(y1), 1, n, features, out, code, st))
+        got.append((frags, flat, y))
+    for a, c in zip(*got):
+        assert torch.equal(a, c)
+    p.n_mats = 0
+    assert L.tgt_linear_fwd_and_pack(x.data_ptr(), W.data_ptr(), b.data_ptr(), y.data_ptr(), n, features, out, at(p), code, st) != 0

@@ -118,6 +118,7 @@ SIGNATURES = {
     "tgt_node_frag_bytes": (_i64, [_i32, _i32]),
     "tgt_node_pack": (_i32, [_vp, _vp, _vp, _i32, _vp, _vp, _i32, _i32, _vp, _vp, _vp]),
     "tgt_node_pack_parts": (_i32, [_vp, _vp, _vp, _vp, _i32, _vp, _vp, _i32, _i32, _vp, _vp, _vp]),
+    "tgt_linear_fwd_and_pack": (_i32, [_vp, _vp, _vp, _vp, _i64, _i32, _i32, _vp, _i32, _vp]),
     "tgt_node_fwd": (_i32, [_vp, _vp]),
     "tgt_node_bwd_workers": (_i32, [_i64]),
     "tgt_node_bwd_pre": (_i32, [_vp, _vp]),

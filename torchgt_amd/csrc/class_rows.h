@@ -6,9 +6,6 @@
 namespace tgt {
 namespace {
 
-__device__ __forceinline__ float as_float(float v) { return v; }
-__device__ __forceinline__ float as_float(nbf16 v) { return __uint_as_float((uint32_t)v.x << 16); }
-
 // Rows of class values.  A wave's R rows are R C consecutive elements of the [N - tokens, C] array and travel through its
 // row image, in words: for bf16 the image starts one element late where the rows begin in the middle of a word.
 template <typename T, int R> struct ClassRows {

@@ -1023,6 +1023,24 @@ int tgt_linear_fwd(const void* d_x, const void* const* d_W, const void* const* d
     return TGT_OK;
 }
 
+int tgt_linear_fwd_and_pack(const void* d_x, const void* d_W, const void* d_b, void* d_y, int64_t N, int in_features, int out_features,
+                            const tgt_node_pack_args* pack, int dtype, void* stream) {
+    using namespace tgt;
+    if (const int rc = check_shape(1, N, in_features, out_features, dtype)) return rc;
+    if (!d_W || (N > 0 && (!d_x || !d_y))) { set_error("linear_fwd_and_pack: null pointer"); return TGT_ERR_INVALID_ARG; }
+    LinArgs a{};
+    a.A[0] = d_x; a.W[0] = d_W; a.bias[0] = d_b; a.out[0] = d_y;
+    a.nw = 1; a.N = N; a.K = in_features; a.M = out_features;
+    bool done;
+    {
+        KernelTimer t(KS_LINEAR_FWD, (hipStream_t)stream);
+        if (const int rc = linear_tiles_and_pack(a, pack, dtype, (hipStream_t)stream, done)) return rc;
+    }
+    if (done) return TGT_OK;
+    if (const int rc = tgt_node_pack_parts(pack->mats, pack->ld, pack->rows, pack->cols, pack->n_mats, pack->vecs, pack->lens, pack->n_vecs, dtype, pack->d_frags, pack->d_vecs, stream)) return rc;
+    return tgt_linear_fwd(d_x, &d_W, &d_b, &d_y, 1, N, in_features, out_features, dtype, stream);
+}
+
 int64_t tgt_linear_bwd_workspace_bytes(int n_out, int in_features, int out_features) {
     using namespace tgt;
     if (n_out < 1 || n_out > 3 || in_features <= 0 || out_features <= 0) return 0;

@@ -18,7 +18,7 @@
 // and smaller than with the float32 instruction at every other shape of eleven (16 to 500 features, 16 to 128 columns, 1 K to 500 K rows).
 // us for 128 -> 64, 64 K rows: y 14.9 / 18.3 / 14.4, dx 15.6 / 19.1 / 18.4, dW with its sum 17.4 / 20.2 / 17.0.
 #include "linear_tiles.h"
-#include "node_tile.h"
+#include "node_pack.h"
 #include <algorithm>
 
 namespace tgt {
@@ -63,9 +63,6 @@ template <typename T> __device__ __forceinline__ void put_cols(T* __restrict__ d
     for (int i = 0; i < RowShape<T>::kAcc; ++i)
         if (r0 + i * PER < rows.left) *reinterpret_cast<vec16*>(p + (int64_t)(r0 + i * PER) * ld) = v[i];
 }
-
-__device__ __forceinline__ float as_float(float v) { return v; }
-__device__ __forceinline__ float as_float(nbf16 v) { return __uint_as_float((uint32_t)v.x << 16); }
 
 // A thread's share of a 64 x 64 piece of the weight on its way to LDS: two operand vectors (outputs o0 .., contraction k0 ..)
 template <typename T> struct Piece { T v[2][8]; };
@@ -142,16 +139,15 @@ template <bool DX> __device__ __forceinline__ void rows_again(const LinArgs& a, 
 // (float32: 80 KB, two workgroups per CU)
 template <typename T> constexpr int lin_lds() { return 2 * kFragVecs<Num<T>::P> * 16 + kWaves * RowShape<T>::kVecs * 16; }
 
-// blockIdx.x: 128 rows; blockIdx.y: `per` of the 64-column pieces of all outputs
-template <typename T, bool DX, bool RESIDENT> __global__ __launch_bounds__(kThreads, 2) void k_linear_tiles(const LinArgs a, const int per) {
+// panel: 128 rows; share: `per` of the 64-column pieces of all outputs
+template <typename T, bool DX, bool RESIDENT> __device__ __forceinline__ void tiles_block(const LinArgs& a, const int per, const int panel, const int share, unsigned char* smem) {
     constexpr int P = Num<T>::P, FV = kFragVecs<P>;
-    extern __shared__ __align__(16) unsigned char smem[];
     vec16* w = reinterpret_cast<vec16*>(smem);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     vec16* stage = w + 2 * FV + wave * RowShape<T>::kVecs;
     const int L = DX ? a.M : a.K, C = DX ? a.K : a.M, nl = (L + 63) / 64, nk = (DX ? a.nw : 1) * nl, nc = (C + 63) / 64;
-    const int first = blockIdx.y * per, all = (DX ? 1 : a.nw) * nc, end = first + per < all ? first + per : all;
-    const Rows rows((int64_t)blockIdx.x * kWaves + wave, a.N);
+    const int first = share * per, all = (DX ? 1 : a.nw) * nc, end = first + per < all ? first + per : all;
+    const Rows rows((int64_t)panel * kWaves + wave, a.N);
     Frags<P> f[RESIDENT ? 2 : 1];
     Raw<T> raw;
     const auto ask_rows = [&](int k) { fetch_cols(raw, reinterpret_cast<const T*>(a.A[k / nl]), L, (k % nl) * 64, rows, lane); };
@@ -209,6 +205,19 @@ template <typename T, bool DX, bool RESIDENT> __global__ __launch_bounds__(kThre
                 rows_again<DX>(a, o, c0, rows, lane);
             }
     }
+}
+
+template <typename T, bool DX, bool RESIDENT> __global__ __launch_bounds__(kThreads, 2) void k_linear_tiles(const LinArgs a, const int per) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    tiles_block<T, DX, RESIDENT>(a, per, blockIdx.x, blockIdx.y, smem);
+}
+// One output of 64 columns, and the packing of a model's parameters, which that output does not depend on: as a launch of its own the packing is
+// 5 to 6 us of a few dozen workgroups with nothing beside them.  128 -> 64 and the parameters of four layers, us, two launches / one: float32 4 K rows
+// 6.0 + 8.9 / 9.6, 37605 5.1 + 14.2 / 13.0, 64 K 5.8 + 16.8 / 19.5, bf16 64 K (GT) 5.6 + 8.3 / 11.4.
+template <typename T> __global__ __launch_bounds__(kThreads, 2) void k_linear_tiles_and_pack(const LinArgs a, const PackArgs p, const int packers) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    if ((int)blockIdx.x < packers) pack_block<T, kThreads>(p, blockIdx.x);
+    else tiles_block<T, false, true>(a, 1, blockIdx.x - packers, 0, smem);
 }
 
 template <typename T, bool DX, bool RESIDENT> int launch(const LinArgs& a, hipStream_t st) {
@@ -356,6 +365,26 @@ int gradw_tiles(const GradWArgs& a, int workers, int dtype, hipStream_t st) {
     // (one piece of x at a time where there is only one)
     if (dtype == TGT_DTYPE_F32) return a.K <= 64 ? launch_gradw<float, 1>(a, workers, st) : launch_gradw<float, 2>(a, workers, st);
     return a.K <= 64 ? launch_gradw<nbf16, 1>(a, workers, st) : launch_gradw<nbf16, 2>(a, workers, st);
+}
+
+// (one column piece of a weight that stays in registers, what one launch can be told; 64 -> 64 has kernels of its own in linear.hip)
+static bool pack_fits(const LinArgs& a, const tgt_node_pack_args& p) { return a.N > 0 && a.M == 64 && a.K != 64 && a.K <= 128 && p.n_mats <= kPackMats && p.n_vecs <= kPackVecs; }
+template <typename T> static int launch_with_pack(const LinArgs& a, const tgt_node_pack_args& p, hipStream_t st) {
+    static std::atomic<uint64_t> done{0};
+    constexpr int lds = lin_lds<T>();
+    if (int rc = allow_lds(reinterpret_cast<const void*>(&k_linear_tiles_and_pack<T>), lds, done)) return rc;
+    const PackArgs args = pack_args(p, 0, 0);
+    const int packers = pack_blocks(args, kThreads);
+    hipLaunchKernelGGL((k_linear_tiles_and_pack<T>), dim3((unsigned)((a.N + 32 * kWaves - 1) / (32 * kWaves) + packers)), dim3(kThreads), lds, st, a, args, packers);
+    TGT_HIP_CHECK(hipGetLastError());
+    return TGT_OK;
+}
+int linear_tiles_and_pack(const LinArgs& a, const tgt_node_pack_args* pack, int dtype, hipStream_t st, bool& done) {
+    done = false;
+    if (int rc = check_pack(pack, dtype)) return rc;
+    if (!pack_fits(a, *pack)) return TGT_OK;
+    done = true;
+    return dtype == TGT_DTYPE_F32 ? launch_with_pack<float>(a, *pack, st) : launch_with_pack<nbf16>(a, *pack, st);
 }
 
 int linear_tiles(const LinArgs& a, bool dx, int dtype, hipStream_t st) {

@@ -18,48 +18,14 @@
 // weight gradient each and add the products over these 128 nodes beside it (node_roles.h).
 #include "node_roles.h"
 #include "class_rows.h"
+#include "node_pack.h"
 
 namespace tgt {
 namespace {
 
-// ---- packing of the parameters ---------------------------------------------------------------------------------------
-constexpr int kPackMats = 96, kPackVecs = 160;
-struct PackArgs {
-    const void* mat[kPackMats];
-    int16_t ld[kPackMats], rows[kPackMats], cols[kPackMats];
-    const void* vec[kPackVecs];
-    int16_t len[kPackVecs];
-    int n_mats, n_vecs, mat0, total_mats, vec0;
-    vec16* frags;       // [2][total_mats][kFragVecs]: for y = W x, then for dx = W^T dy
-    float* vecs;        // [..][64]
-};
-
-// workgroup = one (weight, direction): 512 operand vectors, one per thread; the workgroups behind the weights copy vectors
-template <typename T> __global__ __launch_bounds__(512) void k_node_pack(const PackArgs a) {
-    constexpr int P = Num<T>::P;
-    const int b = blockIdx.x;
-    if (b >= 2 * a.n_mats) {
-        const int i = (b - 2 * a.n_mats) * 8 + threadIdx.x / 64, e = threadIdx.x & 63;
-        if (i < a.n_vecs) a.vecs[(a.vec0 + i) * kVec + e] = e < a.len[i] ? as_float(reinterpret_cast<const T*>(a.vec[i])[e]) : 0.f;
-        return;
-    }
-    const int j = b >> 1, back = b & 1;
-    const T* W = reinterpret_cast<const T*>(a.mat[j]);
-    const int ld = a.ld[j], rows = a.rows[j], cols = a.cols[j];
-    const int lane = threadIdx.x & 63, sm = threadIdx.x >> 6, s = sm >> 2, m = sm & 3;
-    const int out_f = 16 * gray2((lane >> 2) & 3) + 4 * m + (lane & 3), in0 = 16 * (lane >> 4) + 8 * s;
-    float v[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int o = back ? in0 + i : out_f, k = back ? out_f : in0 + i;
-        v[i] = o < rows && k < cols ? as_float(W[o * ld + k]) : 0.f;
-    }
-    bf16x8_t p[P];
-    to_planes(v, p);
-    vec16* dst = a.frags + ((int64_t)(back ? a.total_mats : 0) + a.mat0 + j) * kFragVecs<P>;
-#pragma unroll
-    for (int q = 0; q < P; ++q) dst[(sm * P + q) * 64 + lane] = __builtin_bit_cast(vec16, p[q]);
-}
+// workgroup = one (weight, direction); the workgroups behind the weights copy vectors
+constexpr int kPackThreads = 512;
+template <typename T> __global__ __launch_bounds__(kPackThreads) void k_node_pack(const PackArgs a) { pack_block<T, kPackThreads>(a, blockIdx.x); }
 
 // ---- GELU of a tile of pre-activations (and its slope) ---------------------------------------------------------------------
 // SAME (bf16): every sum and rounding as the separate kernels have it - GELU by the device library's error function, products of
@@ -633,24 +599,14 @@ int tgt_node_pack(const void* const* mats, const int* ld, const int* rows, int n
 int tgt_node_pack_parts(const void* const* mats, const int* ld, const int* rows, const int* cols, int n_mats, const void* const* vecs, const int* lens, int n_vecs,
                         int dtype, void* d_frags, float* d_vecs, void* stream) {
     using namespace tgt;
-    if (!mats || !ld || !rows || !vecs || !lens || n_mats < 1 || n_vecs < 1 || !d_frags || !d_vecs || !dtype_ok(dtype)) return bad("tgt_node_pack", "null or bad argument");
-    for (int i = 0; i < n_mats; ++i) {
-        const int c = cols ? cols[i] : 64;
-        if (!mats[i] || rows[i] < 1 || rows[i] > 64 || c < 1 || c > 64 || ld[i] < c || ld[i] > 32767) return bad("tgt_node_pack", "weights are [1..64, >= 64]");
-    }
-    for (int i = 0; i < n_vecs; ++i)
-        if (!vecs[i] || lens[i] < 1 || lens[i] > 64) return bad("tgt_node_pack", "vectors have 1 to 64 elements");
+    const tgt_node_pack_args p{mats, ld, rows, cols, n_mats, vecs, lens, n_vecs, d_frags, d_vecs};
+    if (int rc = check_pack(&p, dtype)) return rc;
     KernelTimer t(KS_NODE_PACK, (hipStream_t)stream);
     for (int m = 0, v = 0; m < n_mats || v < n_vecs;) {
-        PackArgs a{};
-        a.n_mats = std::min(kPackMats, n_mats - m); a.n_vecs = std::min(kPackVecs, n_vecs - v);
-        a.mat0 = m; a.vec0 = v; a.total_mats = n_mats;
-        a.frags = (vec16*)d_frags; a.vecs = d_vecs;
-        for (int i = 0; i < a.n_mats; ++i) { a.mat[i] = mats[m + i]; a.ld[i] = (int16_t)ld[m + i]; a.rows[i] = (int16_t)rows[m + i]; a.cols[i] = (int16_t)(cols ? cols[m + i] : 64); }
-        for (int i = 0; i < a.n_vecs; ++i) { a.vec[i] = vecs[v + i]; a.len[i] = (int16_t)lens[v + i]; }
-        const int grid = 2 * a.n_mats + (a.n_vecs + 7) / 8;
-        if (dtype == TGT_DTYPE_F32) hipLaunchKernelGGL((k_node_pack<float>), dim3(grid), dim3(512), 0, (hipStream_t)stream, a);
-        else hipLaunchKernelGGL((k_node_pack<nbf16>), dim3(grid), dim3(512), 0, (hipStream_t)stream, a);
+        const PackArgs a = pack_args(p, m, v);
+        const int grid = pack_blocks(a, kPackThreads);
+        if (dtype == TGT_DTYPE_F32) hipLaunchKernelGGL((k_node_pack<float>), dim3(grid), dim3(kPackThreads), 0, (hipStream_t)stream, a);
+        else hipLaunchKernelGGL((k_node_pack<nbf16>), dim3(grid), dim3(kPackThreads), 0, (hipStream_t)stream, a);
         TGT_HIP_CHECK(hipGetLastError());
         m += a.n_mats; v += a.n_vecs;
     }

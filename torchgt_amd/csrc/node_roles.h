@@ -7,7 +7,6 @@
 namespace tgt {
 namespace {
 
-constexpr int kVec = 64;      // floats per parameter vector
 
 // N 16-byte vectors from global memory to LDS by all THREADS threads of a workgroup, every load issued before the first write
 template <int N, int THREADS> __device__ __forceinline__ void copy_vecs(vec16* dst, const vec16* __restrict__ src) {

@@ -32,6 +32,9 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t vec16 __attribute__((ext_vector_type(4)));      // 16 bytes in registers
 struct nbf16 { uint16_t x; };
+__device__ __forceinline__ float as_float(float v) { return v; }
+__device__ __forceinline__ float as_float(nbf16 v) { return __uint_as_float((uint32_t)v.x << 16); }
+constexpr int kVec = 64;      // floats per parameter vector
 
 template <typename T> struct Num;
 template <> struct Num<float> { static constexpr int P = 3; };

@@ -339,8 +339,10 @@ struct FusedGtModel : GtModel {
     static char* weight(const Dims& D, const Saved& s, int64_t l, int i) { return (char*)s.packed + (kMats * l + i) * unit(D); }
     static char* transposed(const Dims& D, const Saved& s, int64_t l, int i) { return weight(D, s, l, i) + mats(D) * unit(D); }
     static float* vec(const Dims& D, const Saved& s, int64_t l, int i) { return (float*)((char*)s.packed + 2 * mats(D) * unit(D)) + (kVecs * l + i) * 64; }
-    static void pack(Tape& t, const Dims& D, const std::vector<Tensor>& p, Saved& s) {
+    // the packed parameters and the first linear's rows
+    static void begin(Tape& t, const Dims& D, const std::vector<Tensor>& p, const void* x, Saved& s) {
         s.packed = t.take(2 * mats(D) * unit(D) + (kVecs * D.L + kOut) * 64 * 4);
+        s.rows_in = t.take(D.N * 64 * D.size);
         if (t.dry()) return;
         std::vector<const void*> m, v;
         std::vector<int> ld, rows(kMats * D.L, 64), cols(kMats * D.L, 64), len(kVecs * D.L, 64);
@@ -358,17 +360,15 @@ struct FusedGtModel : GtModel {
             m.push_back(W.data_ptr()); ld.push_back((int)W.size(1)); rows.push_back((int)W.size(0)); cols.push_back((int)W.size(1));
             v.push_back(b.data_ptr()); len.push_back((int)b.numel());
         }
-        check(tgt_node_pack_parts(m.data(), ld.data(), rows.data(), cols.data(), (int)m.size(), v.data(), len.data(), (int)v.size(), D.code, s.packed, vec(D, s, 0, 0), D.stream),
-              "tgt_node_pack_parts");
+        const tgt_node_pack_args a{m.data(), ld.data(), rows.data(), cols.data(), (int)m.size(), v.data(), len.data(), (int)v.size(), s.packed, vec(D, s, 0, 0)};
+        check(tgt_linear_fwd_and_pack(x, p[0].data_ptr(), p[1].data_ptr(), s.rows_in, D.n, (int)D.F, 64, &a, D.code, D.stream), "tgt_linear_fwd_and_pack");
     }
     static void forward(Tape& t, const Dims& D, const std::vector<Tensor>& p, const void* x, const tgt_plan_t* plan, const Tensor& ws, const std::vector<double>& eps, bool keep,
                         Saved& s) {
         const int64_t row = D.N * 64 * D.size;
         auto P = [&](int64_t i) { return p[i].data_ptr(); };
         s.l.assign(D.L, Layer{});
-        pack(t, D, p, s);
-        s.rows_in = t.take(row);
-        linear(t, D, x, {{P(0), P(1)}}, {s.rows_in}, D.n, D.F, 64);
+        begin(t, D, p, x, s);
         for (int64_t i = 0; i < D.L; ++i) {
             Layer& l = s.l[i];
             if (i > 0 && !keep) l = s.l[0];

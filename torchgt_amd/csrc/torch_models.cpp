@@ -28,8 +28,10 @@ struct Packed {
     int64_t unit = 0;
     int mats = 0;
     Packed() = default;
+    // the linear in front of the layers, which one launch does together with the packing
+    struct First { const void *x, *W, *b; void* y; int64_t rows, features; };
     // layers: first of their 16 L parameters; classes: gamma, beta, Wh, bh or nullptr
-    Packed(const Tensor* layers, int64_t L, const Tensor* classes, int code, const at::TensorOptions& opt, void* stream) {
+    Packed(const Tensor* layers, int64_t L, const Tensor* classes, int code, const at::TensorOptions& opt, void* stream, const First* first = nullptr) {
         std::vector<const void*> m, v;
         std::vector<int> ld, rows, len;
         static const int wi[6] = {8, 12, 14, 2, 4, 6}, vi[10] = {9, 10, 11, 13, 15, 0, 1, 3, 5, 7};
@@ -48,9 +50,11 @@ struct Packed {
         const int64_t bytes = tgt_node_frag_bytes(mats, code), vec_bytes = (int64_t)v.size() * kWidth * 4;
         unit = bytes / (2 * mats);
         frags = at::empty({bytes + vec_bytes}, opt.dtype(at::kByte));
-        check(tgt_node_pack(m.data(), ld.data(), rows.data(), mats, v.data(), len.data(), (int)v.size(), code, frags.data_ptr(),
-                            reinterpret_cast<float*>(static_cast<char*>(frags.data_ptr()) + bytes), stream),
-              "tgt_node_pack");
+        const tgt_node_pack_args a{m.data(), ld.data(), rows.data(), nullptr, mats, v.data(), len.data(), (int)v.size(), frags.data_ptr(),
+                                   reinterpret_cast<float*>(static_cast<char*>(frags.data_ptr()) + bytes)};
+        if (first)
+            check(tgt_linear_fwd_and_pack(first->x, first->W, first->b, first->y, first->rows, (int)first->features, (int)kWidth, &a, code, stream), "tgt_linear_fwd_and_pack");
+        else check(tgt_node_pack(a.mats, a.ld, a.rows, a.n_mats, a.vecs, a.lens, a.n_vecs, code, a.d_frags, a.d_vecs, stream), "tgt_node_pack");
     }
     // for the backward: the buffer and what it was made from
     Packed(const Tensor& buf, int n_mats, int code) : frags(buf), unit(tgt_node_frag_bytes(n_mats, code) / (2 * n_mats)), mats(n_mats) {}
@@ -84,14 +88,10 @@ void graphormer_forward(GraphormerState& st, const GraphormerDims& D, const std:
     st.rows = at::empty({(ns + na) * N, kWidth}, opt);
     st.Z = at::empty({keep ? L * N * D.H : N * D.H}, opt.dtype(at::kFloat));
     st.logp = at::empty({D.n, D.C}, opt);
-    st.packed = Packed(p.data() + 3, L, p.data() + 3 + 16 * L, code, opt, stream);
+    const Packed::First encoder{x.data_ptr(), p[0].data_ptr(), p[1].data_ptr(), at_row(st.rows, D.tokens), D.n, x.size(1)};
+    st.packed = Packed(p.data() + 3, L, p.data() + 3 + 16 * L, code, opt, stream, &encoder);
     auto s_row = [&](int64_t l) { return at_row(st.rows, keep ? l * N : 0); };
     auto a_row = [&](int64_t l, int i) { return at_row(st.rows, (ns + (keep ? 4 * l : 0) + i) * N); };
-    {
-        const void *W[1] = {p[0].data_ptr()}, *B[1] = {p[1].data_ptr()};
-        void* Y[1] = {at_row(st.rows, D.tokens)};
-        check(tgt_linear_fwd(x.data_ptr(), W, B, Y, 1, D.n, (int)x.size(1), (int)kWidth, code, stream), "tgt_linear_fwd");
-    }
     for (int64_t l = 0; l <= L; ++l) {
         tgt_node_fwd_args a{};
         a.rows = N; a.dtype = code; a.tokens = (int)D.tokens;
