@@ -22,7 +22,7 @@ def layer_norm(x, gamma, beta, eps=1e-5):
 
 
 def relu(x):
-    return torch.where(x > 0, x, torch.zeros_like(x))
+    return torch.where(x <= 0, torch.zeros_like(x), x)
 
 
 def _linear(x, p, name):

@@ -41,6 +41,34 @@ def test_relu_forward_backward_is_exact(cuda, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_relu_keeps_nan_as_torch_does(cuda, dtype):
+    """F.relu and its backward: a NaN stays one, its slope is 1; an infinity stays or becomes 0"""
+    u = torch.randn(256, generator=torch.Generator().manual_seed(1)).to(dtype)
+    u[3], u[5], u[70], u[71] = float("nan"), float("inf"), -float("inf"), -0.0
+    dh = torch.randn(256, generator=torch.Generator().manual_seed(2)).to(dtype)
+    ref, uc = u.clone().requires_grad_(True), u.to(cuda).requires_grad_(True)
+    want, got = torch.relu(ref), ReluFunction.apply(uc)
+    for a, b in ((got, want), (torch.autograd.grad(got, uc, dh.to(cuda))[0], torch.autograd.grad(want, ref, dh)[0])):
+        assert torch.equal(a.isnan().cpu(), b.isnan()) and torch.equal(a.nan_to_num(7.).cpu(), b.nan_to_num(7.))
+    # the same in the epilogue of a 64 -> 64 linear, and in the fused layers: a NaN of one feed-forward feature reaches every row
+    L, code = _lib.lib(), _DT[dtype]
+    x, W, b = torch.randn(70, 64, device=cuda).to(dtype), torch.randn(64, 64, device=cuda).to(dtype), torch.zeros(64, device=cuda, dtype=dtype)
+    b[9] = float("nan")
+    v, h = torch.empty_like(x), torch.empty_like(x)
+    _lib.check(L.tgt_linear_act_fwd(x.data_ptr(), W.data_ptr(), b.data_ptr(), 70, 64, 64, code, 2, v.data_ptr(), h.data_ptr(), None))
+    assert h[:, 9].isnan().all() and int(h.isnan().sum()) == 70
+    m = GT(2, 8, 32, 64, 5, 1, 0.0, 0.0, 0.0, 64, 0)
+    with torch.no_grad():
+        m.layers[1].FFN_layer1.bias[17] = float("nan")
+    m = m.to(cuda, dtype)
+    loops = torch.arange(100).repeat(2, 1).to(cuda)
+    for one in (True, False):
+        m.one_operator = one
+        out = m(torch.randn(100, 32, device=cuda).to(dtype), None, loops, attn_type="sparse")
+        assert out.isnan().all(), one
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_gt_forward_backward_matches_oracle(cuda, dtype):
     """GT of the node-level scripts (4 layers, hidden 64, 8 heads, 128-d input, 40 classes) on a 2 000-node power-law
     graph with self-loops: log-probabilities and the gradient of every parameter that takes part."""

@@ -189,16 +189,16 @@ private:
 // nn.GELU() (exact erf form) and F.relu on one value, and dh * d act / du.  One definition for the elementwise kernels
 // and for the epilogues of the projections that apply the activation themselves: both give the same bits.
 //   GELU: h = 0.5 u (1 + erf(u / sqrt 2));  dh/du = 0.5 (1 + erf(u / sqrt 2)) + u exp(-u^2 / 2) / sqrt(2 pi)
-//   RELU: h = max(u, 0);  dh/du = 1 where u > 0
+//   RELU: h = u where not u <= 0, else 0;  dh/du = 1 where not u <= 0 (F.relu keeps a NaN, and its slope there is 1)
 template <bool RELU>
 __device__ __forceinline__ float act_value(float u) {
-    if (RELU) return u > 0.f ? u : 0.f;
+    if (RELU) return u <= 0.f ? 0.f : u;
     const float cdf = 0.5f * (1.f + erff(u * 0.70710678118654752f));
     return u * cdf;
 }
 template <bool RELU>
 __device__ __forceinline__ float act_grad(float u, float dh) {
-    if (RELU) return u > 0.f ? dh : 0.f;
+    if (RELU) return u <= 0.f ? 0.f : dh;
     const float cdf = 0.5f * (1.f + erff(u * 0.70710678118654752f));
     return dh * (cdf + u * __expf(-0.5f * u * u) * 0.39894228040143268f);
 }

@@ -178,7 +178,7 @@ __global__ __launch_bounds__(kEwBlock) void k_layer_norm_bwd(const T* __restrict
 }
 
 // nn.GELU (exact): h = 0.5 u (1 + erf(u / sqrt 2));  dh/du = 0.5 (1 + erf(u / sqrt 2)) + u exp(-u^2 / 2) / sqrt(2 pi)
-// RELU: F.relu instead (the GT layers, models/gt_dist_node_level.py:258,285): h = max(u, 0); dh/du = 1 where u > 0.
+// RELU: F.relu instead (the GT layers, models/gt_dist_node_level.py:258,285): zero (h and slope) where u <= 0; a NaN stays one.
 template <typename T, bool BWD, bool RELU = false>
 __global__ __launch_bounds__(kEwBlock) void k_gelu(const T* __restrict__ u, const T* __restrict__ dh, int64_t nvec,
                                                    T* __restrict__ out) {

@@ -360,13 +360,13 @@ template <typename T, int R> __device__ __forceinline__ void put_rows(T* __restr
 __device__ __forceinline__ float stored(float v, const float*) { return v; }
 __device__ __forceinline__ float stored(float v, const nbf16*) { return static_cast<float>(static_cast<__bf16>(v)); }
 
-// relu(u), and (bit i) where u > 0
+// relu(u), and (bit i) where its slope is 1: as F.relu and its backward, a NaN stays one
 template <typename T, int R> __device__ __forceinline__ uint32_t relu(TileOf<R>& u) {
     uint32_t on = 0;
     TGT_EACH(i) {
         const float v = stored(u.get(i), (const T*)nullptr);
-        on |= v > 0.f ? 1u << i : 0u;
-        u.set(i, v > 0.f ? v : 0.f);
+        on |= v <= 0.f ? 0u : 1u << i;
+        u.set(i, v <= 0.f ? 0.f : v);
     }
     return on;
 }
