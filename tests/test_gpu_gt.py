@@ -220,6 +220,25 @@ class _ReadoutBwd(ctypes.Structure):
                 [(k, ctypes.c_void_p) for k in ("x", "dlogp", "logp", "w", "w_back", "v", "dx")] + [("grads", ctypes.c_void_p * 6), ("partial", ctypes.c_void_p)])
 
 
+def run_readout(x, W, b, dlogp, classes):
+    """log-probabilities, dx and the gradients of W and b from tgt_readout_fwd and tgt_readout_bwd"""
+    L, dtype, code, st = _lib.lib(), x.dtype, _DT[x.dtype], ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    n, (m1, m2, out) = x.shape[0], [t.shape[0] for t in W]
+    ints = lambda *a: (ctypes.c_int * len(a))(*a)
+    ptrs = lambda ts: (ctypes.c_void_p * len(ts))(*[t.data_ptr() for t in ts])
+    unit = L.tgt_node_frag_bytes(3, code)
+    frags, vecs = torch.empty(unit, dtype=torch.uint8, device=x.device), torch.empty(192, device=x.device)
+    _lib.check(L.tgt_node_pack_parts(ptrs(W), ints(64, m1, m2), ints(m1, m2, out), ints(64, m1, m2), 3, ptrs(b), ints(m1, m2, out), 3, code, frags.data_ptr(), vecs.data_ptr(), st))
+    logp, dx, grads = torch.full((n, classes), 7., device=x.device).to(dtype), torch.full_like(x, 7), [torch.full_like(t, 7) for t in W + b]
+    f = _ReadoutFwd(n, code, m1, m2, out, classes, x.data_ptr(), frags.data_ptr(), vecs.data_ptr(), logp.data_ptr())
+    _lib.check(L.tgt_readout_fwd(ctypes.byref(f), st))
+    partial = torch.empty(L.tgt_readout_partial_floats(n, m1, m2, out), device=x.device)
+    r = _ReadoutBwd(n, code, m1, m2, out, classes, x.data_ptr(), dlogp.data_ptr(), logp.data_ptr(), frags.data_ptr(), frags.data_ptr() + unit // 2, vecs.data_ptr(), dx.data_ptr(),
+                    ptrs(grads), partial.data_ptr())
+    _lib.check(L.tgt_readout_bwd(ctypes.byref(r), st))
+    return logp, dx, grads
+
+
 # Weights and rows of -1, 0, 1 (times a power of two): the inputs of both ReLUs and the logits are the same numbers whatever the order of
 # the sums, so no activation changes its side.  What is left: a log-softmax (2^-8 of a bfloat16 result, 1e-5 in float32) and, backward, one rounding of
 # every d logits, du (bfloat16: 2^-9 each of three in a row, and of the results): 1e-2 of the largest; float32 1e-5.
@@ -228,24 +247,12 @@ class _ReadoutBwd(ctypes.Structure):
                                                  (129, 1, 1, 2, 2), (4097, 32, 16, 40, 40), (16385, 64, 32, 16, 13), (70001, 32, 16, 40, 40)])
 def test_readout_in_one_kernel(cuda, dtype, n, m1, m2, out, classes):
     print(f"readout n={n} widths {m1} {m2} {out} classes={classes} {dtype}", flush=True)
-    L, code, st = _lib.lib(), _DT[dtype], ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
     g = torch.Generator(device=cuda).manual_seed(n + out)
     grid = lambda *s: torch.randint(-1, 2, s, generator=g, device=cuda).to(dtype)
     W = [grid(m1, 64) * 0.25, grid(m2, m1) * 0.5, grid(out, m2) * 0.25]
     b = [grid(m1), grid(m2), grid(out)]
     x, dlogp = grid(n, 64), torch.randn(n, classes, generator=g, device=cuda).to(dtype)
-    ints = lambda *a: (ctypes.c_int * len(a))(*a)
-    ptrs = lambda ts: (ctypes.c_void_p * len(ts))(*[t.data_ptr() for t in ts])
-    unit = L.tgt_node_frag_bytes(3, code)
-    frags, vecs = torch.empty(unit, dtype=torch.uint8, device=cuda), torch.empty(192, device=cuda)
-    _lib.check(L.tgt_node_pack_parts(ptrs(W), ints(64, m1, m2), ints(m1, m2, out), ints(64, m1, m2), 3, ptrs(b), ints(m1, m2, out), 3, code, frags.data_ptr(), vecs.data_ptr(), st))
-    logp, dx, grads = torch.full((n, classes), 7., device=cuda).to(dtype), torch.full_like(x, 7), [torch.full_like(t, 7) for t in W + b]
-    f = _ReadoutFwd(n, code, m1, m2, out, classes, x.data_ptr(), frags.data_ptr(), vecs.data_ptr(), logp.data_ptr())
-    _lib.check(L.tgt_readout_fwd(ctypes.byref(f), st))
-    partial = torch.empty(L.tgt_readout_partial_floats(n, m1, m2, out), device=cuda)
-    r = _ReadoutBwd(n, code, m1, m2, out, classes, x.data_ptr(), dlogp.data_ptr(), logp.data_ptr(), frags.data_ptr(), frags.data_ptr() + unit // 2, vecs.data_ptr(), dx.data_ptr(),
-                    ptrs(grads), partial.data_ptr())
-    _lib.check(L.tgt_readout_bwd(ctypes.byref(r), st))
+    logp, dx, grads = run_readout(x, W, b, dlogp, classes)
     held = lambda t: t.to(dtype).double()      # as a row of this type holds it
     Wd, bd, a0 = [t.double() for t in W], [t.double() for t in b], x.double()
     a1 = held(a0 @ Wd[0].T + bd[0]).relu()
@@ -260,6 +267,97 @@ def test_readout_in_one_kernel(cuda, dtype, n, m1, m2, out, classes):
         top = max(float(ref.abs().max()), 1e-30)
         # a bias of many rows: n terms of either sign, each rounded; their sum is as large as sqrt(n) of them
         assert float((got.double() - ref).abs().max()) <= (1e-2 if dtype == torch.bfloat16 else 1e-5) * max(top, 1.0 if name[0] == "b" or n < 3 else 0.0), name
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,m1,m2,out,classes", [(20, 32, 16, 40, 40), (70, 5, 3, 7, 6), (130, 64, 64, 64, 64), (33, 33, 17, 8, 8), (300, 32, 16, 1, 1)])
+@pytest.mark.parametrize("what", ["x", "Wa", "Wb", "Wc", "bias", "killed", "overflow", "dlogp"])
+def test_infinities_go_through_the_readout_as_through_three_linears(cuda, dtype, n, m1, m2, out, classes, what):
+    """Every log-probability and gradient is +-inf, NaN or finite as the products and sums have it, widths of less than 64 and rows past a tile's end
+    included.  `killed`: infinite weights whose pre-activations are all -inf, so that the ReLU ends them; `overflow`: finite operands, infinite products.
+    Weights and rows of -1, 0, 1 times a power of two elsewhere: no ReLU changes its side (see test_readout_in_one_kernel, also for the bars)."""
+    print(f"readout infinities n={n} widths {m1} {m2} {out} classes={classes} {what} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(n + m1)
+    grid = lambda *s: torch.randint(-1, 2, s, generator=g).to(dtype)
+    W, b = [grid(m1, 64) * 0.25, grid(m2, m1) * 0.5, grid(out, m2) * 0.25], [grid(m1), grid(m2), grid(out)]
+    x, dlogp, inf = grid(n, 64), torch.randn(n, classes, generator=g).to(dtype), float("inf")
+    W[0][0, 0] = 0.25
+    if what == "x":
+        x[n // 2, 1], x[n - 1, 63], x[0, 0], x[3, 5], x[3, 6] = inf, -inf, float("nan"), inf, inf
+    elif what in ("Wa", "Wb", "Wc"):
+        w = W["abc".index(what[1])]
+        w[w.shape[0] // 2, w.shape[1] - 1], w[0, 0] = inf, -inf
+    elif what == "bias":
+        b[0][m1 - 1], b[1][0], b[2][out // 2] = -inf, inf, -inf
+    elif what == "killed":
+        x[:, 7] = 1
+        W[0][m1 // 2, 7], W[0][0, 7] = -inf, -inf
+        b[1][m2 - 1] = -inf
+    elif what == "overflow":
+        x[:, 5], x[n - 1], W[0][m1 - 1, 5] = 0, 0, 2.0 ** 100
+        x[n - 1, 5] = 2.0 ** 100
+    else:
+        dlogp[n - 1, classes - 1], dlogp[0, 0] = inf, -inf
+    logp, dx, grads = run_readout(x.to(cuda), [w.to(cuda) for w in W], [t.to(cuda) for t in b], dlogp.to(cuda), classes)
+
+    def product(p, q):      # every product formed and added, in the order and the range of float32
+        s = torch.zeros(p.shape[0], q.shape[1])
+        for k in range(p.shape[1]):
+            s += p[:, k:k + 1].float() * q[k:k + 1].float()
+        return s.double()
+
+    held = lambda t: t.to(dtype).double()
+    Wd, bd = [t.double() for t in W], [t.double() for t in b]
+    a1 = held(product(x, W[0].T) + bd[0]).relu()
+    a2 = held(product(a1, W[1].T) + bd[1]).relu()
+    want = torch.log_softmax(held(product(a2, W[2].T) + bd[2])[:, :classes], 1)
+    back = logp.double().cpu()
+    d = torch.zeros(n, out, dtype=torch.double)
+    d[:, :classes] = dlogp.double() - back.exp() * dlogp.double().sum(1, keepdim=True)
+    d = held(d)
+    d1 = held(torch.where(a2 <= 0, 0.0, product(d, W[2])))
+    d0 = held(torch.where(a1 <= 0, 0.0, product(d1, W[1])))
+    bar, seen = 1e-2 if dtype == torch.bfloat16 else 1e-5, 0
+    refs = [want, product(d0, W[0]), product(d0.T, x), product(d1.T, a1), product(d.T, a2), d0.sum(0), d1.sum(0), d.sum(0)]
+    for name, a, r in zip(("logp", "dx", "Wa", "Wb", "Wc", "ba", "bb", "bc"), [logp, dx, *grads], refs):
+        a = a.double().cpu()
+        assert torch.equal(a.isnan(), r.isnan()) and torch.equal(a.isposinf(), r.isposinf()) and torch.equal(a.isneginf(), r.isneginf()), name
+        fin = r.isfinite()
+        seen += int((~fin).sum())
+        assert not fin.any() or float((a - r)[fin].abs().max()) <= bar * max(1.0, float(r[fin].abs().max())), name
+    assert seen > 0 or what == "killed"
+
+
+@pytest.mark.parametrize("where", ["MLP_layer.FC_layers.0.weight", "MLP_layer.FC_layers.1.weight", "MLP_layer.FC_layers.2.weight", "MLP_layer.FC_layers.1.bias", "x"])
+def test_an_infinity_in_the_model_gives_what_its_modules_give(cuda, where):
+    """float32 GT of hidden size 64 as one operator and module by module: the same infinities and NaN in the log-probabilities, the loss and every gradient"""
+    print(f"gt with an infinity in {where}", flush=True)
+    torch.manual_seed(1)
+    n, model = 300, GT(2, 8, 32, 64, 7, 1, 0.0, 0.0, 0.0, 64, 0)
+    with torch.no_grad():
+        for p in model.parameters():
+            if p.dim() == 2:
+                p.normal_(0, p.shape[1] ** -0.5)
+    x, y = torch.randn(n, 32), torch.randint(0, 7, (n,), device=cuda)
+    if where == "x":
+        x[n // 2, 3] = float("inf")
+    else:
+        with torch.no_grad():
+            p = dict(model.named_parameters())[where]
+            p[(p.shape[0] // 2, p.shape[1] - 1) if p.dim() == 2 else 3] = -float("inf") if p.dim() == 2 else float("inf")
+    model, loops, got = model.to(cuda), torch.arange(n).repeat(2, 1).to(cuda), []
+    for one in (True, False):
+        model.one_operator = one
+        model.zero_grad(set_to_none=True)
+        out = model(x.to(cuda), None, loops, attn_type="sparse")
+        loss = torch.nn.functional.nll_loss(out, y)
+        loss.backward()
+        got.append([("output", out.detach()), ("loss", loss.detach())] + [(k, p.grad) for k, p in model.named_parameters() if p.grad is not None])
+    assert not got[0][0][1].isfinite().all()
+    for (name, a), (_, r) in zip(*got):
+        assert torch.equal(a.isnan(), r.isnan()) and torch.equal(a.isposinf(), r.isposinf()) and torch.equal(a.isneginf(), r.isneginf()), name
+        fin = r.isfinite()
+        assert not fin.any() or float((a - r)[fin].abs().max()) <= 1e-4 * max(1.0, float(r[fin].abs().max())), name
 
 
 def test_readout_refuses_other_widths():

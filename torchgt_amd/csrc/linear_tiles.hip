@@ -108,18 +108,8 @@ template <typename T, int P> __device__ __forceinline__ void put_piece(vec16* ds
     }
 }
 
-// Whether a lane of the wave holds a NaN.  An infinity has no planes (what is left of it behind hi is NaN, and an infinite hi times the
-// mid plane of the other operand has any sign): every output that it touches comes out as NaN and is formed again by plain float32
-// multiply-adds, which give the +-inf or NaN that it has.  The look costs one multiply-add per output (128 -> 64 of 64 K rows: below
-// the runs' difference); the second computation runs for waves with a NaN only.
-template <typename V> __device__ __forceinline__ bool holds_nan(const V& value, int n) {
-    float t = 0.f;
-#pragma unroll
-    for (int i = 0; i < n; ++i) t = fmaf(value(i), 0.f, t);      // (infinities too: they may have become what they are on the way)
-    return __ballot(t != 0.f) != 0;
-}
-
-// the wave's 32 rows of 64 output columns from c0 on, lane = its node's half as in Tile
+// For a wave that `holds_nan`: its 32 rows of 64 output columns from c0 on, lane = its node's half as in Tile.  The look costs one
+// multiply-add per output (128 -> 64 of 64 K rows: below the runs' difference).
 template <bool DX> __device__ __forceinline__ void rows_again(const LinArgs& a, int o, int c0, const Rows& rows, int lane) {
     const int L = DX ? a.M : a.K, C = DX ? a.K : a.M, n = lane & 31;
     if (n >= rows.left) return;

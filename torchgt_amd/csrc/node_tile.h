@@ -227,6 +227,16 @@ template <int P> __device__ __forceinline__ void gemm_apart(Tile& acc, const Fra
     }
 }
 
+// Whether a lane of the wave holds a NaN.  An infinity has no planes (what is left of it behind hi is NaN, and an infinite hi times the
+// mid plane of the other operand has any sign): every output that it touches comes out as NaN and is formed again by plain float32
+// multiply-adds, which give the +-inf or NaN that it has.  That second computation runs for waves with a NaN only.
+template <typename V> __device__ __forceinline__ bool holds_nan(const V& value, int n) {
+    float t = 0.f;
+#pragma unroll
+    for (int i = 0; i < n; ++i) t = fmaf(value(i), 0.f, t);      // (infinities too: they may have become what they are on the way)
+    return __ballot(t != 0.f) != 0;
+}
+
 // LDS exchanges between lanes of one wave: the hardware runs a wave's LDS accesses in order, this keeps the compiler to it
 __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -557,6 +567,13 @@ template <int BYTES, int P, int R> __device__ __forceinline__ void put_tile_plan
 #pragma unroll
         for (int p = 0; p < P; ++p) *reinterpret_cast<bf16x8_t*>(planes + p * BYTES + (base ^ (s << 4))) = f[p];
     }
+}
+// The float whose three planes these are (an infinity and a NaN are their first)
+__device__ __forceinline__ float from_planes(float hi, float mid, float lo) { return fabsf(hi) < INFINITY ? hi + (mid + lo) : hi; }
+// feature c of row r of the planes in LDS
+template <int BYTES> __device__ __forceinline__ float plane_elem(const unsigned char* planes, int r, int c) {
+    const nbf16* e = reinterpret_cast<const nbf16*>(planes + r * 128 + (((c >> 3) ^ (r & 7)) << 4)) + (c & 7);
+    return from_planes(as_float(e[0]), as_float(e[BYTES / 2]), as_float(e[BYTES]));
 }
 // Address of a lane's first piece of the operand that has features 32 block .. + 31 as rows: nodes 8 (lane / 32) ... + 3
 __device__ __forceinline__ int operand_base(int block, int lane) {

@@ -6,7 +6,8 @@
 // Widths up to 64, 32 and 16 in the model: as a kernel per linear, activation and softmax these are fourteen launches of 3 to 12 us for 64 K nodes
 // that read and write rows of 32 to 128 bytes (33 us forward and 58 backward, and their host time).  Here a wave carries its nodes
 // through all of it (node_tile.h), the narrow weights packed as 64 x 64 with zeros.  Backward: the roles of node_roles.h; bound by the chain of a
-// group's products.  64 K rows in bf16 8.4 us forward, 21 + 5 backward.
+// group's products.  64 K rows in bf16 8.4 us forward, 26.4 backward with its sums (5); float32 14.4 and 54.2.  Of these 0.3 and 0.6, 0.6 and 2.7 keep infinities
+// what they are (`mend`, `add_product`).
 #include "node_roles.h"
 #include "class_rows.h"
 
@@ -15,6 +16,72 @@ namespace {
 
 constexpr int kMats = 3, kRows = 16, kWaves = 16;      // weights; forward: rows of a wave, waves of a workgroup at most
 template <typename T> constexpr int readout_lds(int waves) { return kMats * kFragVecs<Num<T>::P> * 16 + kMats * kVec * 4 + waves * RowShape<T, kRows>::kVecs * 16; }
+
+// float32 weight element (o, k) of a packed 64 x 64 weight: o = 16 g + i, i = 0 .. 15, lies `i` further on (node_tile.h)
+struct WeightColumn {
+    const nbf16* e;
+    __device__ __forceinline__ WeightColumn(const vec16* w, int g, int k)
+        : e(reinterpret_cast<const nbf16*>(w + (k >> 3 & 1) * 4 * 3 * 64 + 16 * (k >> 4) + 4 * gray2(g)) + (k & 7)) {}
+    __device__ __forceinline__ float at(int i) const {
+        const nbf16* p = e + ((i >> 2) * 3 * 64 + (i & 3)) * 8;
+        return from_planes(as_float(p[0]), as_float(p[64 * 8]), as_float(p[2 * 64 * 8]));
+    }
+};
+// y = W x + bias (null: without) by plain float32 multiply-adds, x and the weight of `ins` x `outs` that count, zero behind them
+__device__ __forceinline__ void linear_again(TileOf<kRows>& y, const TileOf<kRows>& x, const vec16* w, const float* bias, int outs, int ins, vec16* stage, int lane) {
+    constexpr int R = kRows;
+    const int n = lane % R, g = lane / R;
+    float* row = reinterpret_cast<float*>(stage) + 64 * n;
+    wave_sync();
+    TGT_EACH(i) row[R * g + i] = x.get(i);
+    wave_sync();
+    TGT_EACH(i) y.set(i, bias ? bias[R * g + i] : 0.f);
+#pragma unroll 1
+    for (int k = 0; k < ins; ++k) {
+        const WeightColumn c(w, g, k);
+        const float v = row[k];
+        TGT_EACH(i) {
+            y.set(i, fmaf(c.at(i), v, y.get(i)));
+            if (i % 4 == 3) fence_schedule();
+        }
+    }
+    TGT_EACH(i) if (R * g + i >= outs) y.set(i, 0.f);
+    wave_sync();
+}
+__device__ __forceinline__ void whole(TileOf<kRows>& t, const Frags<3, kRows>& f) {
+#pragma unroll
+    for (int s = 0; s < kRows / 8; ++s) {
+        float v[3][8];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) unpack16(__builtin_bit_cast(vec16, f.p[s][p]), v[p], (const nbf16*)nullptr);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) t.set(8 * s + e, from_planes(v[0][e], v[1][e], v[2][e]));
+    }
+}
+__device__ __forceinline__ void whole(TileOf<kRows>& t, const TileOf<kRows>& f) { t = f; }
+// Behind a product y = W x: what operands that are not finite leave of it where it does not belong.  float32: the product again, without planes
+// (`holds_nan`).  bf16: zeros in the features behind `outs`, where the packing's zeros met an infinity and the next product would read the NaN (the last
+// feature has one if any has).  TAIL: zeros in the rows past the end, whose ReLUs are off then: they must not add to
+// sums over nodes (0 times an infinite weight).
+// The rare part stands apart from the rest: in its place it is a few KB that every wave fetches its way around (bf16, 64 K rows, backward: 25.8 us
+// without `mend`, 28.1 in its place, 26.4 apart; a look of half the instructions, v_maximum3 of two values each, takes as long).
+template <int P, bool TAIL, typename B> __device__ __forceinline__ void mend(TileOf<kRows>& y, const B& x, const vec16* w, const float* bias, int outs, int ins, vec16* stage, const Rows& rows, int lane) {
+    constexpr int R = kRows;
+    const int g = lane / R;
+    bool off;
+    if constexpr (P == 3) off = holds_nan([&](int i) { return y.get(i); }, R);
+    else off = __ballot(g == 3 && outs < 64 && !(y.get(R - 1) == 0.f)) != 0;
+    if (__builtin_expect(off || (TAIL && rows.left < R), 0)) {
+        if constexpr (P == 3) {
+            if (off) {
+                TileOf<R> t;
+                whole(t, x);
+                linear_again(y, t, w, bias, outs, ins, stage, lane);
+            }
+        }
+        TGT_EACH(i) if ((P == 1 && R * g + i >= outs) || (TAIL && lane % R >= rows.left)) y.set(i, 0.f);
+    }
+}
 
 template <typename T> __global__ __launch_bounds__(kWaves * 64) void k_readout_fwd(const tgt_readout_fwd_args a) {
     constexpr int P = Num<T>::P, FV = kFragVecs<P>, R = kRows;
@@ -35,10 +102,13 @@ template <typename T> __global__ __launch_bounds__(kWaves * 64) void k_readout_f
         TileOf<R> x, y;
         settle<T, false>(x, raw, stage, rows, lane);
         linear<P, false>(y, x, w, vec, lane);
+        mend<P, false>(y, x, w, vec, a.m1, 64, stage, rows, lane);
         relu<T>(y);
         linear<P, false>(x, y, w + FV, vec + kVec, lane);
+        mend<P, false>(x, y, w + FV, vec + kVec, a.m2, a.m1, stage, rows, lane);
         relu<T>(x);
         linear<P, false>(y, x, w + 2 * FV, vec + 2 * kVec, lane);
+        if constexpr (P == 3) mend<P, false>(y, x, w + 2 * FV, vec + 2 * kVec, a.out, a.m2, stage, rows, lane);
         put_classes<T>(reinterpret_cast<T*>(a.logp), y, false, a.classes, 0, t0 * R, N, stage, lane);
     }
 }
@@ -54,9 +124,35 @@ struct Sizes {
     }
 };
 
-// t where the activation was positive, as a T row would hold it
+// t where the activation's slope is 1, as a T row would hold it
 template <typename T, int R> __device__ __forceinline__ void relu_back(TileOf<R>& t, uint32_t on) {
     TGT_EACH(i) t.set(i, on >> i & 1u ? stored(t.get(i), (const T*)nullptr) : 0.f);
+}
+
+// acc += dy^T x over a group's nodes, one 32 x 32 block q of it (node_product).  float32: a group's product apart, and again without planes where it
+// `holds_nan`.
+template <int P, int PB> __device__ __forceinline__ void add_product(float16_t& acc, const unsigned char* dy, const unsigned char* x, int base_dy, int base_x, int q, int lane) {
+    if constexpr (P == 1) node_product<P, PB>(acc, dy, x, base_dy, base_x);
+    else {
+        float16_t c;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) c[r] = 0.f;
+        node_product<P, PB>(c, dy, x, base_dy, base_x);
+        if (__builtin_expect(holds_nan([&](int r) { return c[r]; }, 16), 0)) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) c[r] = 0.f;
+#pragma unroll 1
+            for (int n = 0; n < PB / 128; ++n) {
+                const float v = plane_elem<PB>(x, n, 32 * (q & 1) + (lane & 31));
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    c[r] = fmaf(plane_elem<PB>(dy, n, 32 * (q >> 1) + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)), v, c[r]);
+                    if (r % 4 == 3) fence_schedule();
+                }
+            }
+        }
+        acc += c;
+    }
 }
 
 template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN, kMats>::kThreads)) void k_readout_bwd(const tgt_readout_bwd_args a) {
@@ -88,12 +184,13 @@ template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN,
             const Rows rows(tile, N, R);
             TileOf<R> t, d;
             Frags<P, R> f, fx, fy;      // x and the first activation, for the weight gradients
-            settle<T, false>(t, raw, stage, rows, lane);
+            settle<T, true>(t, raw, stage, rows, lane);
             make_frags(fx, t);
             ClassGrads<T, R> classes(reinterpret_cast<const T*>(a.dlogp), reinterpret_cast<const T*>(a.logp), false, a.classes, 0, tile * R, N, stage, lane);
             if (g0 + gridDim.x < groups) fetch(raw, reinterpret_cast<const T*>(a.x), Rows(tile + NC * (int64_t)gridDim.x, N, R), lane);
             __syncthreads();                                        // Wa is there; product Wa of the round before is done
             linear<P, false>(t, fx, w, vec, lane);
+            mend<P, true>(t, fx, w, vec, a.m1, 64, stage, rows, lane);
             __syncthreads();                                        // Wa has been used
             const uint32_t on1 = relu<T>(t);
             make_frags(fy, t);
@@ -103,6 +200,7 @@ template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN,
             make_frags(f, d);
             __syncthreads();                                        // Wb
             linear<P, false>(t, fy, w, vec + kVec, lane);
+            mend<P, true>(t, fy, w, vec + kVec, a.m2, a.m1, stage, rows, lane);
             __syncthreads();                                        // Wb has been used
             const uint32_t on2 = relu<T>(t);
             put_tile_planes<PB, P>(p_x, row, h, t);
@@ -110,6 +208,7 @@ template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN,
             __syncthreads();                                        // planes of Wc; Wc^T
             zero(t);
             gemm<P>(t, f, w, lane);                                 // beside product Wc
+            if constexpr (P == 3) mend<P, false>(t, f, w, nullptr, a.m2, a.out, stage, rows, lane);
             relu_back<T>(t, on2);
             col[1] += column_sums(t, lane);
             make_frags(f, t);
@@ -119,6 +218,7 @@ template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN,
             __syncthreads();                                        // planes of Wb; Wb^T
             zero(t);
             gemm<P>(t, f, w, lane);                                 // beside product Wb
+            if constexpr (P == 3) mend<P, false>(t, f, w, nullptr, a.m1, a.m2, stage, rows, lane);
             relu_back<T>(t, on1);
             col[0] += column_sums(t, lane);
             make_frags(f, t);
@@ -128,6 +228,7 @@ template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN,
             __syncthreads();                                        // planes of Wa; Wa^T
             zero(t);
             gemm<P>(t, f, w, lane);                                 // dx, beside product Wa
+            if constexpr (P == 3) mend<P, false>(t, f, w, nullptr, 64, a.m1, stage, rows, lane);
             __syncthreads();                                        // Wa^T has been used
             put_rows(reinterpret_cast<T*>(a.dx), t, stage, rows, lane);
         }
@@ -142,13 +243,13 @@ template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN,
             next.hand_over(w, bw + 2 * FV);         // Wb
             __syncthreads();
             next.hand_over(w, bw + FV);             // Wc^T and the planes of Wc
-            node_product<P, PB>(acc[2], p_dy, p_x, base_dy, base_x);
+            add_product<P, PB>(acc[2], p_dy, p_x, base_dy, base_x, q, lane);
             __syncthreads();
             next.hand_over(w, bw);                  // Wb^T and the planes of Wb
-            node_product<P, PB>(acc[1], p_dy, p_x, base_dy, base_x);
+            add_product<P, PB>(acc[1], p_dy, p_x, base_dy, base_x, q, lane);
             __syncthreads();
             next.hand_over(w, fw);                  // Wa^T and the planes of Wa
-            node_product<P, PB>(acc[0], p_dy, p_x, base_dy, base_x);
+            add_product<P, PB>(acc[0], p_dy, p_x, base_dy, base_x, q, lane);
             __syncthreads();
         }
     }
