@@ -220,8 +220,8 @@ class _ReadoutBwd(ctypes.Structure):
                 [(k, ctypes.c_void_p) for k in ("x", "dlogp", "logp", "w", "w_back", "v", "dx")] + [("grads", ctypes.c_void_p * 6), ("partial", ctypes.c_void_p)])
 
 
-def run_readout(x, W, b, dlogp, classes):
-    """log-probabilities, dx and the gradients of W and b from tgt_readout_fwd and tgt_readout_bwd"""
+def run_readout(x, W, b, dlogp, classes, logp_back=None):
+    """log-probabilities, dx and the gradients of W and b from tgt_readout_fwd and tgt_readout_bwd (logp_back: the log-probabilities it is told)"""
     L, dtype, code, st = _lib.lib(), x.dtype, _DT[x.dtype], ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
     n, (m1, m2, out) = x.shape[0], [t.shape[0] for t in W]
     ints = lambda *a: (ctypes.c_int * len(a))(*a)
@@ -233,7 +233,7 @@ def run_readout(x, W, b, dlogp, classes):
     f = _ReadoutFwd(n, code, m1, m2, out, classes, x.data_ptr(), frags.data_ptr(), vecs.data_ptr(), logp.data_ptr())
     _lib.check(L.tgt_readout_fwd(ctypes.byref(f), st))
     partial = torch.empty(L.tgt_readout_partial_floats(n, m1, m2, out), device=x.device)
-    r = _ReadoutBwd(n, code, m1, m2, out, classes, x.data_ptr(), dlogp.data_ptr(), logp.data_ptr(), frags.data_ptr(), frags.data_ptr() + unit // 2, vecs.data_ptr(), dx.data_ptr(),
+    r = _ReadoutBwd(n, code, m1, m2, out, classes, x.data_ptr(), dlogp.data_ptr(), (logp if logp_back is None else logp_back).data_ptr(), frags.data_ptr(), frags.data_ptr() + unit // 2, vecs.data_ptr(), dx.data_ptr(),
                     ptrs(grads), partial.data_ptr())
     _lib.check(L.tgt_readout_bwd(ctypes.byref(r), st))
     return logp, dx, grads
@@ -267,6 +267,25 @@ def test_readout_in_one_kernel(cuda, dtype, n, m1, m2, out, classes):
         top = max(float(ref.abs().max()), 1e-30)
         # a bias of many rows: n terms of either sign, each rounded; their sum is as large as sqrt(n) of them
         assert float((got.double() - ref).abs().max()) <= (1e-2 if dtype == torch.bfloat16 else 1e-5) * max(top, 1.0 if name[0] == "b" or n < 3 else 0.0), name
+
+
+@pytest.mark.parametrize("n", [4096, 64000, 300000])
+def test_readout_weight_gradients_are_as_exact_as_float32_products(cuda, n):
+    """rms error of the three weight gradients against 64 bits, of the rms of the result.  Weights of 1, positive rows and log-probabilities of -inf (d logits =
+    dlogp) hand the same two matrices of random float32 numbers to each of the three products, without an error in front of them and with no ReLU near 0.
+    Bound: float32 matrix instructions round the running sum once per two products, which leaves 2^-24 sqrt(1 + k / 12) after the k rows of a worker
+    (test_gpu_projections.py).  Also dx, whose products are exact here."""
+    g = torch.Generator(device=cuda).manual_seed(n)
+    x, dlogp = torch.randn(n, 64, generator=g, device=cuda).abs() + 2.0 ** -20, torch.randn(n, 64, generator=g, device=cuda)
+    one, none = torch.eye(64, device=cuda), torch.zeros(64, device=cuda)
+    _, dx, grads = run_readout(x, [one, one, one], [none, none, none], dlogp, 64, logp_back=torch.full_like(dlogp, -float("inf")))
+    assert torch.equal(dx, dlogp)
+    want = dlogp.double().t().contiguous() @ x.double()
+    errs = [float((a.double() - want).norm() / want.norm()) for a in grads[:3]]
+    k = 64 if n <= 16384 else -(-n // (128 * 256)) * 128      # groups of 64 or 128 rows over 256 CUs
+    bound = 2 ** -24 * (1 + k / 12) ** 0.5
+    print(f"readout exactness n={n}: " + " ".join(f"{e:.2e}" for e in errs) + f" (bound {bound:.2e})", flush=True)
+    assert max(errs) <= bound
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
