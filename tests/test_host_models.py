@@ -70,7 +70,8 @@ def test_models_refuse_cpu_tensors():
         GT(1, 8, 16, 64, 4, 1, 0.0, 0.0, 0.0, 64, 0)(torch.zeros(5, 16), None, torch.zeros(2, 4, dtype=torch.long), attn_type="sparse")
 
 
-@pytest.mark.parametrize("change", ["none", "shared", "none_slot", "own_names", "own_child", "twice", "itself", "extra"])
+@pytest.mark.parametrize("change", ["none", "shared", "none_slot", "own_names", "own_child", "twice", "itself", "extra", "object_names", "object_members",
+                                    "object_modules", "object_child"])
 def test_parameters_are_the_named_parameters_in_their_order(change):
     for m in (Graphormer(2, 8, 16, 64, 5, 1, 0.0, 0.0, 0.0, 64, 1), GT(2, 8, 16, 64, 5, 1, 0.0, 0.0, 0.0, 64, 0),
               GraphLevelGraphormer(2, 8, 64, 0.0, 0.0, 64, "ZINC", "multi_hop", 5, 0.0, 1)):
@@ -91,6 +92,14 @@ def test_parameters_are_the_named_parameters_in_their_order(change):
                 def named_modules(self, *a, **k):
                     return iter(())
             first.hidden = Hidden(4, 4)
+        if change == "object_names":
+            m.named_parameters = lambda *a, of=m, **k: iter(list(torch.nn.Module.named_parameters(of, *a, **k))[:3])
+        if change == "object_members":
+            m._named_members = lambda *a, of=m, **k: iter(list(torch.nn.Module._named_members(of, *a, **k))[2:])
+        if change == "object_modules":
+            m.named_modules = lambda *a, of=m, **k: iter([("", of)])
+        if change == "object_child":
+            m.layers[1].named_modules = lambda *a, **k: iter(())
         if change == "twice":
             m.layers.append(first)
         if change == "itself":

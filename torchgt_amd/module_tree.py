@@ -46,16 +46,22 @@ class OneWalk(nn.Module):
     """``parameters()`` of a model in one walk over its modules.  ``zero_grad``, a gradient clip and a flattening all-reduce each ask for
     them on every step, and ``nn.Module`` spells out the name of every parameter through a generator per module for it: 92 us for
     the 72 parameters of four layers, 38 here (half a step of 4 K nodes is host time).  Names are only left out where nobody could
-    see them: a class that brings its own ``named_parameters`` or ``named_modules`` is asked in the general way."""
+    see them: a class or an object that brings its own ``named_parameters`` or ``named_modules`` is asked in the general way."""
 
     def parameters(self, recurse=True):
-        if not recurse or not _plain_names(type(self)):
+        if not recurse or not _plain_names(type(self)) or not _NAMES.isdisjoint(self.__dict__):
             yield from super().parameters(recurse)
             return
         seen, parents, known, stack = set(), set(), {type(self)}, [self]
         while stack:
             m = stack.pop()
-            own, children = m._parameters, m._modules
+            d = m.__dict__
+            if type(m) not in known or "named_modules" in d:      # (that is all the general way asks a child for)
+                if not _plain_names(type(m)) or "named_modules" in d or "_parameters" not in d or "_modules" not in d:
+                    yield from [q for q in super().parameters() if id(q) not in seen]
+                    return
+                known.add(type(m))
+            own, children = d["_parameters"], d["_modules"]
             if children:
                 if id(m) in parents:      # (a leaf that is there twice has nothing new the second time)
                     continue
@@ -68,12 +74,10 @@ class OneWalk(nn.Module):
             if children:
                 for child in reversed(children.values()):
                     if child is not None:
-                        if type(child) not in known:
-                            if not _plain_names(type(child)):
-                                yield from [q for q in super().parameters() if id(q) not in seen]
-                                return
-                            known.add(type(child))
                         stack.append(child)
+
+
+_NAMES = {"named_parameters", "named_modules", "_named_members"}
 
 
 def _plain_names(cls):
