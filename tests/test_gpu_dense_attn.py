@@ -299,7 +299,7 @@ def test_query_0_backward_forms_the_forwards_score(cuda, dtype, d):
     (3, 25, 2, 8, 1, 0.0), (3, 28, 2, 8, 0, 0.3), (5, 33, 3, 16, 3, 0.0), (300, 34, 4, 8, 0, 0.0), (3, 40, 8, 8, 5, 0.0), (9, 59, 2, 32, 0, 0.0),
     (2, 64, 2, 32, 1, 0.0), (3, 68, 2, 16, 0, 0.4), (3, 90, 2, 8, 7, 0.0), (90, 90, 8, 8, 0, 0.0), (3, 100, 2, 32, 2, 0.0), (9, 111, 8, 16, 0, 0.0),
     (128, 129, 8, 8, 0, 0.0), (3, 129, 8, 8, 1, 0.2), (64, 130, 16, 16, 1, 0.0), (3, 132, 2, 32, 0, 0.0), (2, 161, 2, 8, 0, 0.0), (2, 164, 2, 16, 1, 0.0),
-    (2, 181, 2, 8, 1, 0.0), (2, 182, 2, 32, 0, 0.0), (2, 201, 2, 8, 1, 0.3), (2, 225, 2, 16, 0, 0.0), (2, 249, 2, 8, 1, 0.0), (2, 255, 2, 8, 0, 0.0)])
+    (2, 6, 2, 8, 7, 0.0), (3, 14, 2, 8, 5, 0.0), (2, 50, 2, 16, 6, 0.0), (3, 166, 2, 8, 7, 0.0), (2, 181, 2, 8, 1, 0.0), (2, 182, 2, 32, 0, 0.0), (2, 201, 2, 8, 1, 0.3), (2, 225, 2, 16, 0, 0.0), (2, 249, 2, 8, 1, 0.0), (2, 255, 2, 8, 0, 0.0)])
 def test_plane_in_lds_gives_what_the_general_kernels_give(cuda, b, S, H, d, offset, p_drop):
     print(f"dense plane b={b} S={S} H={H} d={d} offset={offset} p_drop={p_drop}", flush=True)
     g = torch.Generator(device=cuda).manual_seed(S + d)

@@ -64,6 +64,13 @@ struct Plane {
         for (int i = 0; i < W; ++i) out[i] = __builtin_amdgcn_alignbit(w[i + 1], w[i], sh);
     }
 };
+// `words` from the last element on, and the copy's pieces, end inside the LDS of the plane wherever it begins
+constexpr bool plane_fits(int S) {
+    for (int off = 0; off < 16; off += 2)
+        if ((off + 2 * (S * S - 1)) / 4 * 4 + 4 * (kPlaneAhead + 1) > plane_bytes(S) || (off + 2 * S * S + 15) / 16 * 16 > plane_bytes(S)) return false;
+    return S <= 1 || plane_fits(S - 1);
+}
+static_assert(plane_fits(288) && 2 * 288 * 288 > kLdsLimit, "every size that fits the LDS");
 // The first kAhead pieces of a thread are asked for at once (`ask`), in front of everything else; `arrive` puts them into LDS and fetches what is left.
 // (A piece may begin or end outside the tensor, never outside the 16 bytes that one of its elements is in.)
 template <int THREADS> struct PlaneIn {
@@ -234,7 +241,7 @@ __global__ __launch_bounds__(64 * NW, 4) void k_plane_fwd(const dbf16* __restric
     for (int kt = 0; kt < NW; ++kt) {
         const int kb = kt * 32 + 16 * half;      // this lane's keys: kb .. kb + 15
         const bool full = THIN || kt * 32 + 32 <= S;
-        uint32_t b[8];
+        uint32_t b[kPlaneAhead];
         plane.words(qrow + (full ? kb : min(kb, S - 1)), b);
         if (tame && full) {      // (a row's last tile is formed: what lies behind the row's end is another row's)
             uint32_t other = 0;

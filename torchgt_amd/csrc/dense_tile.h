@@ -209,7 +209,8 @@ template <int D> int dense_plane(const DensePlaneCall& c, bool bwd);
 constexpr int plane_tiles(int S) { return S > 32 && S - (S - 1) / 32 * 32 <= 4 ? (S - 1) / 32 : (S + 31) / 32; }
 // Its LDS: images of the heads, and the plane behind the bytes that its address lies above a multiple of 16
 constexpr int kFlagBytes = 64;      // one word per wave
-constexpr int plane_bytes(int S) { return (16 + 2 * S * S + 24 + 15) / 16 * 16; }      // (24: `Plane::words` reads up to 18 bytes past the last element)
+constexpr int kPlaneAhead = 8;      // words that the forward takes from an element on (`Plane::words`), the last of a plane included
+constexpr int plane_bytes(int S) { return (16 + 2 * S * S + 4 * kPlaneAhead + 2 + 15) / 16 * 16; }
 constexpr int plane_fwd_lds(int D, int S) {
     const int rows = (S + 31) / 32 * 32;
     return 2 * D * (2 * rows + 4) + kFlagBytes + plane_bytes(S);
