@@ -569,8 +569,9 @@ __device__ __forceinline__ RecLane load_rec_lane(const WaveRec<LPE>& rec) {
 template <typename T, int MODE> constexpr bool rec_edges_early() { return sizeof(T) == 2 || MODE == MODE_FWD; }
 
 // Whether the walk of a long row keeps its queue of gathers filled (walk_range).  The float32 backward has no registers for it (128 with two
-// rows of its own and two gathered ones per edge) and its gathers are masked.  Beside dense tiles the rows are short and the queue's registers
-// cost a wave per SIMD: 262 K nodes in clusters of 64, forward + backward 158.7 us step by step, 159.8 as a queue.
+// rows of its own and two gathered ones per edge) and its gathers are masked.  Beside dense tiles rows are short as a
+// rule and the queue's registers cost a wave per SIMD: bf16, 262 K nodes in 64 clusters, forward + backward 158.7 us step by step, 159.8 as a queue; rows
+// of 40, 100 and 240 edges beside the tiles 318, 663 and 1500 against 314, 659 and 1495, with a bias 517, 1220 and 2808 against 535, 1235 and 2813.
 template <typename T, int MODE, bool TILES> constexpr bool piped_walk() { return !TILES && (sizeof(T) == 2 || MODE == MODE_FWD); }
 
 // Walks `len` edges starting at sorted position `start` of node `row` with S edge
@@ -589,21 +590,50 @@ __device__ __forceinline__ void walk_range(const Common& c, const SideArgs& s, c
         const int32_t* __restrict__ col = s.col + start;
         const int32_t* __restrict__ eid = ident ? nullptr : s.eid + start;
         const int n = valid ? len : 0;
-#pragma unroll 1
-        for (int e0 = slot; e0 < n; e0 += S * kUnroll) {
-            int nb[kUnroll], ed[kUnroll];
-            bool ok[kUnroll];
+        const auto load_ids = [&](const int e0, int (&nb)[kUnroll], int (&ed)[kUnroll]) {
 #pragma unroll
             for (int u = 0; u < kUnroll; ++u) {
                 const int e = e0 + u * S;
-                ok[u] = e < n;
-                nb[u] = 0; ed[u] = 0;
-                if (ok[u]) {
-                    nb[u] = col[e];
-                    if (HASB) ed[u] = ident ? start + e : eid[e];
+                if constexpr (masked_gathers<T, MODE>()) {
+                    nb[u] = 0; ed[u] = 0;
+                    if (e < n) {
+                        nb[u] = col[e];
+                        if (HASB) ed[u] = ident ? start + e : eid[e];
+                    }
+                } else {      // past the end of the row: its last edge (a line the wave is reading anyway)
+                    const int ec = min(e, n - 1);
+                    nb[u] = col[ec];
+                    ed[u] = HASB ? (ident ? start + ec : eid[ec]) : 0;
                 }
             }
+        };
+        const auto step = [&](const int e0, const int (&nb)[kUnroll], const int (&ed)[kUnroll]) {
+            bool ok[kUnroll];
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u) ok[u] = e0 + u * S < n;
             edge_step<T, LPE, LPH, MODE, HASB>(c, s, rr, nb, ed, ok, el, acc);
+        };
+        if (n <= 0) return;
+        int nb[kUnroll], ed[kUnroll];
+        if constexpr (sizeof(T) == 4) {
+#pragma unroll 1
+            for (int e0 = slot; e0 < n; e0 += S * kUnroll) {
+                load_ids(e0, nb, ed);
+                step(e0, nb, ed);
+            }
+        } else {
+            // the ids of the next step are asked for before this step's gathers: a step waits for one memory round trip, not for two in a
+            // row (2-byte elements leave the registers for it).  65 K nodes, rows of 40, 100 and 240 edges beside tiles, forward + backward: 324, 671 and 1513 us without,
+            // 318, 663 and 1500 with.
+            load_ids(slot, nb, ed);
+#pragma unroll 1
+            for (int e0 = slot; e0 < n; e0 += S * kUnroll) {
+                int nb2[kUnroll], ed2[kUnroll];
+                load_ids(e0 + S * kUnroll, nb2, ed2);
+                step(e0, nb, ed);
+#pragma unroll
+                for (int u = 0; u < kUnroll; ++u) { nb[u] = nb2[u]; ed[u] = ed2[u]; }
+            }
         }
     } else {
         // The edges of a slot are a queue of kUnroll: when one has been used its place is asked for again, with the edge one
