@@ -174,6 +174,20 @@ def test_plan_of_the_remaining_edges_schedules_only_rows_with_edges(cuda, dtype)
         sparse_attention(q, k, v, rest.to(cuda), plan=plan)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,d,bias", [(8, 8, "none"), (8, 8, "edge_head"), (4, 16, "edge"), (2, 8, "none")])
+def test_rows_of_more_than_one_step_beside_tiles(cuda, dtype, H, d, bias):
+    """Remaining rows around the classes (32 edges), the steps (64) and the segments (256, 1024) of the walk, as destinations and as sources"""
+    rng = np.random.default_rng(H + d)
+    N, ends = 1200, []
+    for i, m in enumerate((0, 1, 31, 32, 33, 63, 64, 65, 127, 129, 191, 256, 257, 1023, 1025, 2100)):
+        other = rng.integers(0, N, m)
+        row = np.full(m, 16 * i)
+        ends += [np.stack([other, row]), np.stack([row + 8, other])]
+    rest = torch.from_numpy(rng.permutation(np.concatenate(ends, 1), axis=1))
+    run_case("long rows beside tiles", N, _random_tiles(rng, N, 60), rest, H, d, dtype, bias, H + d, cuda)
+
+
 def test_block_loud_failures(cuda):
     q = torch.randn(100, 8, 8, device=cuda, dtype=torch.bfloat16)
     with pytest.raises(_lib.TorchGTHipError) as exc:
