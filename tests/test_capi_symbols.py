@@ -85,3 +85,13 @@ def test_torch_extension_loads_and_registers_its_operators():
         ops.gelu(torch.zeros(8))
     with pytest.raises(RuntimeError, match="GPU"):
         ops.linear(torch.zeros(4, 8), [torch.zeros(8, 8)], [None])
+
+
+def test_node_feature_sums_take_16_mb_at_most():
+    from torchgt_amd import _lib
+    L = _lib.lib()
+    for rows in (1, 17, 60, 90, 103, 104, 105, 140, 208, 300, 1000, 5000, 200_000):
+        for C in (8, 64, 200):
+            most = max(16 << 20, 4 * C * (3 * rows + 1))      # (a copy at least)
+            assert 0 < L.tgt_graph_node_feature_bwd_workspace_bytes(rows, rows, rows, C) <= most
+            assert 0 < L.tgt_embedding_sum_bwd_workspace_bytes(3 * rows + 1, C) <= most

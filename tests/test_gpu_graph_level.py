@@ -76,11 +76,12 @@ def test_graph_node_feature_matches_oracle(cuda, dtype, C, Fx, num_atoms, num_de
             assert not a[0].any()
 
 
-# Table gradients in LDS (one to four copies, runs of rows that end inside eight, token rows in any place of a run, more channels than lanes)
+# Table gradients in LDS (two to four copies, runs of rows that end inside sixteen, fewer runs than CUs, token rows in any place of a run, more channels than lanes)
 # and beyond it.  Sums of up to n float32 terms in another order: n 2^-24 of the sum of their magnitudes; bf16 results round once more.
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("b,s,C,Fx,atoms,deg", [(1, 1, 64, 1, 64, 64), (5, 7, 64, 1, 64, 64), (3, 8, 40, 2, 9, 5), (40, 9, 64, 1, 64, 64), (7, 128, 64, 3, 64, 64),
-                                                (300, 20, 64, 1, 30, 20), (2, 30, 128, 1, 200, 40), (2, 30, 128, 1, 230, 40), (3, 11, 200, 1, 20, 10)])
+                                                (300, 20, 64, 1, 30, 20), (2, 30, 128, 1, 200, 40), (2, 30, 128, 1, 230, 40), (3, 11, 200, 1, 20, 10),
+                                                (64, 128, 64, 1, 200, 55), (9, 30, 64, 1, 201, 55)])
 def test_node_feature_gradients_at_every_size_of_tables(cuda, b, s, C, Fx, atoms, deg, dtype):
     print(f"node feature gradients b={b} s={s} C={C} Fx={Fx} tables {atoms} / {deg} {dtype}", flush=True)
     g = torch.Generator().manual_seed(b + s)

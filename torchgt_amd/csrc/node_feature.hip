@@ -12,7 +12,7 @@
 //
 // With a few dozen atom types every table row is shared by hundreds of node rows, and atomics on one address serialise
 // (55 us for the 33 K rows of 256 padded graphs into one copy, 43 with the fill into 64, in LDS as slow as in memory).  Tables that
-// fit a workgroup's LDS are summed there without atomics: a wave has a table to itself.  Larger ones are added to
+// fit a workgroup's LDS twice are summed there without atomics: a wave has a table to itself.  Larger ones are added to
 // with vector-memory atomics, neighbouring workgroups into different copies (up to 64, at most 16 MB in all): their results agree to
 // rounding between runs, not bit for bit.
 #include "common.h"
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(256) void k_node_feature_bwd(NodeFeatArgs a, const 
 
 // Tables in LDS.  A workgroup takes a run of rows for all tables: wave w adds the rows of set w / tables to that set's copy of table w % tables,
 // lane = channel, so nobody else writes there and the sums come in row order.  Bound by that chain, one LDS read, add and write per row, and
-// by the loads in front of it, eight rows at a time.  33 K rows of 64 channels, tables of 64 + 64 + 64 + 1 rows: 20 us, and 5
+// by the loads in front of it, sixteen rows at a time.  33 K rows of 64 channels, tables of 64 + 64 + 64 + 1 rows: 20 us, and 5
 // for the sum of 256 copies; with atomics 33, 6 for their fill and 4.
 constexpr int kFeatRows = 16, kFeatSets = 4;
 template <typename T>
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(64 * 3 * kFeatSets) void k_node_feature_bwd_lds(Nod
     if (a.s == 0) F = 0;      // token rows only
     const int rows = a.s + a.has_token, n_rows = a.b * rows, per = (n_rows + gridDim.x - 1) / gridDim.x;
     const int r0 = per * blockIdx.x, r1 = min(r0 + per, n_rows), last = a.b * a.s - 1;
-    // every load of eight rows is asked for before the first is used, also where there is nothing to add (another row's is read then)
+    // every load of sixteen rows is asked for before the first is used, also where there is nothing to add (another row's is read then)
     for (int row = r0 + kFeatRows * set; row < r1; row += kFeatRows * sets) {
         const int g0 = (uint32_t)row / (uint32_t)rows;
         int at = row - g0 * rows, p = g0 * a.s + at - a.has_token;      // the row's place in its graph, the position of its ids
@@ -231,15 +231,20 @@ __global__ __launch_bounds__(256) void k_node_feature_finish(const float* __rest
     else stf(d_tok + (t - n_atom - n_in - n_out), v);
 }
 
-// Copies of the tables that a workgroup's LDS holds (0: none): up to four, at less than a CU's 160 KB
-// (rows are counted in 32 bits there)
-inline int node_feat_sets(int64_t n_acc) { return (int)std::min<int64_t>(kFeatSets, (156 << 10) / (n_acc * (int64_t)sizeof(float))); }
-// Copies of the float sums in memory.  From LDS: one per workgroup, a workgroup per CU at most.  With atomics: as many as stay under 16 MB in
-// all, at most 64.
+// Copies of the tables in a workgroup's LDS (0: none): two to four, at less than a CU's 160 KB.  One alone leaves the chain of a table's rows to one wave:
+// 33 K rows, tables of 321 and 579 rows of 64 channels 50 and 57 us whatever the ids; with atomics 30 and 33 where all rows are used alike, 71 and
+// 71 where four of each table are.  Two, of 257 rows: 33, atomics 30 and 121.
+inline int node_feat_sets(int64_t n_acc) {
+    const int sets = (int)std::min<int64_t>(kFeatSets, (156 << 10) / (n_acc * (int64_t)sizeof(float)));
+    return sets >= 2 ? sets : 0;
+}
+// Copies of the float sums in memory, 16 MB in all at most.  From LDS: one per workgroup, a workgroup per CU at most (rows are counted in 32 bits
+// there).  With atomics: at most 64.
 inline int node_feat_copies(int64_t n_acc) {
-    if (node_feat_sets(n_acc) > 0) return num_cus();
+    const int64_t fit = std::max<int64_t>(1, (16 << 20) / (n_acc * (int64_t)sizeof(float)));
+    if (node_feat_sets(n_acc) > 0) return (int)std::min<int64_t>(num_cus(), fit);
     int copies = 64;
-    while (copies > 1 && n_acc * copies * (int64_t)sizeof(float) > (16 << 20)) copies /= 2;
+    while (copies > fit) copies /= 2;
     return copies;
 }
 
@@ -285,7 +290,7 @@ int node_feature_bwd_impl(NodeFeatArgs a, const void* d_dout, int dtype, void* d
     const int64_t n_rows = (int64_t)a.b * (a.s + a.has_token);
     int copies = node_feat_copies(n_acc);
     if (const int sets = node_feat_sets(n_acc); sets > 0 && n_rows + kFeatRows * kFeatSets <= INT32_MAX) {
-        // a workgroup for every eight rows of each set, at most one per copy
+        // a workgroup for every sixteen rows of each set, at most one per copy
         copies = (int)std::min<int64_t>(copies, (n_rows + kFeatRows * sets - 1) / (kFeatRows * sets));
         if (copies > 0) {
             const int tables = a.has_degree ? 3 : 1, lds = (int)(sets * n_acc * sizeof(float));
