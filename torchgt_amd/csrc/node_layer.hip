@@ -1,5 +1,5 @@
 // The node-local part of a Graphormer encoder layer (models/graphormer_dist_node_level.py:246-314 and
-// models/graphormer_graph_level.py:267-306), hidden and feed-forward width 64, as one forward and two backward kernels.
+// models/graphormer_graph_level.py:267-306), hidden and feed-forward width 64, as one forward and one or two backward kernels.
 //
 //   forward   [attention rows a, residual stream s] -> s1 = s + a Wo^T + bo;  s' = s1 + W2 gelu(W1 LN2(s1) + b1) + b2
 //             and, in the same pass, what the next layer's attention reads: q, k, v = LN1(s') W^T + b - or the class
@@ -8,14 +8,16 @@
 //             classes: one weight, d log_softmax in front)
 //             k_node_bwd_post: ds' -> ds (residual), da, gradients of Wo, W1, W2 and LN2, and (1 / (Z + eps), da . a) per
 //             node and head, which the sparse attention's backward starts from
+//             k_node_bwd_both: the first for a layer and the second for the layer in front of it, as one launch (node level)
 //
 // What bounds them and why this shape.  As one kernel per linear, LayerNorm and activation the part moves 29 rows of 64
 // features per node forward and 47 backward through memory; here it moves 6 and 12 (q, k, v, the residual stream and the
 // attention rows; the intermediate activations are recomputed in the backward from s and a: two products, against two rows
-// written and read).  A wave takes 32 nodes and keeps them in registers through the whole chain (node_tile.h); the waves of
-// a workgroup share the packed weights in LDS.  Weight gradients contract over nodes: in the backward kernels four waves carry 32
-// nodes each through the chain and put the bf16 planes of both operands into LDS, four others keep one 32 x 32 block of every
-// weight gradient each and add the products over these 128 nodes beside it (node_roles.h).
+// written and read).  A wave takes 32 or 16 nodes and keeps them in registers through the whole chain (node_tile.h); the waves of
+// a workgroup share the packed weights in LDS.  Weight gradients contract over nodes: in the backward kernels two to eight waves carry
+// 32 or 16 nodes each through the chain and put the bf16 planes of both operands into LDS, four others keep one 32 x 32 block of every
+// weight gradient each and add the products over these 64 or 128 nodes beside it (node_roles.h).  Which of the sizes a call takes is said with
+// both sides' times at the entry points below and at `groups_of_64`.
 #include "node_roles.h"
 #include "class_rows.h"
 #include "node_pack.h"
@@ -504,8 +506,6 @@ struct SumArgs {
     void* out[kMaxSums][kMaxOut];      // mats x 4096 elements, then vectors of 64 (a null entry is not wanted)
     int16_t mats[kMaxSums], rows[kMaxSums], ld[kMaxSums];   // rows: of the 64 in each matrix and the vectors that follow them (classes)
 };
-__device__ __forceinline__ void put_elem(float* p, float v) { *p = v; }
-__device__ __forceinline__ void put_elem(nbf16* p, float v) { p->x = __builtin_bit_cast(uint16_t, static_cast<__bf16>(v)); }
 
 // 64 consecutive elements x 16 slices of the workers per workgroup: slices in worker order, then the slice sums in order.  Bound by
 // its reads, 50 KB of partials from every worker of every launch of a backward (108 MB for four Graphormer layers): sixteen lanes of a
@@ -543,7 +543,7 @@ template <typename T> __global__ __launch_bounds__(256) void k_node_sums(const S
         const int mats = a.mats[d], rows = a.rows[d];
         const int seg = e < mats * 4096 ? e >> 12 : mats + ((e - mats * 4096) >> 6), at = e < mats * 4096 ? e & 4095 : (e - mats * 4096) & 63;
         const int limit = seg < mats ? rows * 64 : (seg < 2 * mats ? rows : 64);
-        if (a.out[d][seg] && at < limit) put_elem(reinterpret_cast<T*>(a.out[d][seg]) + (seg < mats ? (at >> 6) * a.ld[d] + (at & 63) : at), t);
+        if (a.out[d][seg] && at < limit) reinterpret_cast<T*>(a.out[d][seg])[seg < mats ? (at >> 6) * a.ld[d] + (at & 63) : at] = to_elem<T>(t);
     }
 }
 

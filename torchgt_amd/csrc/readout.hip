@@ -285,8 +285,6 @@ template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN,
 
 // Sums over the workers, 64 elements x 16 slices of them per workgroup: a slice in worker order, then the slices
 struct Outs { void* p[2 * kMats]; };
-__device__ __forceinline__ void put_sum(float* p, float v) { *p = v; }
-__device__ __forceinline__ void put_sum(nbf16* p, float v) { *p = to_elem<nbf16>(v); }
 template <typename T> __global__ __launch_bounds__(1024) void k_readout_sums(const float* __restrict__ partial, int workers, Sizes z, Outs out) {
     __shared__ float part[16][64];
     const int total = z.at(2 * kMats), e = blockIdx.x * 64 + (threadIdx.x & 63), sl = threadIdx.x >> 6;
@@ -308,7 +306,7 @@ template <typename T> __global__ __launch_bounds__(1024) void k_readout_sums(con
     for (int i = 0; i < 16; ++i) s += part[i][threadIdx.x];
     int j = 0;
     while (j + 1 < 2 * kMats && e >= z.at(j + 1)) ++j;
-    if (out.p[j]) put_sum(reinterpret_cast<T*>(out.p[j]) + (e - z.at(j)), s);
+    if (out.p[j]) reinterpret_cast<T*>(out.p[j])[e - z.at(j)] = to_elem<T>(s);
 }
 
 template <typename T> int run_fwd(const tgt_readout_fwd_args& a, hipStream_t st) {

@@ -353,7 +353,7 @@ struct FusedGtModel : GtModel {
             for (int i : {64, 64, 64, 128, 128, 64, 64, 64}) ld.push_back(i);
             for (const void* q : {part(7, 0), part(8, 0), part(9, 0), part(11, 0), part(11, 64), part(13, 0), part(14, 0), part(15, 0), part(1, 0), part(3, 0), part(5, 0)}) v.push_back(q);
         }
-        // the readout's; where it has a width of its own kernels, the last layer's query weight and bias in its place (not read)
+        // the readout's; where it has kernels of its own widths, the first layer's query weight and bias in its place (not read)
         const Tensor* out = &p[kHead + 16 * D.L];
         for (int i = 0; i < kOut; ++i) {
             const Tensor &W = fused_readout(D) ? out[2 * i] : p[kHead], &b = fused_readout(D) ? out[2 * i + 1] : p[kHead + 1];
