@@ -475,3 +475,24 @@ def test_linear_with_the_packing_beside_it(cuda, dtype, n, features, out, n_mats
         assert torch.equal(a, c)
     p.n_mats = 0
     assert L.tgt_linear_fwd_and_pack(x.data_ptr(), W.data_ptr(), b.data_ptr(), y.data_ptr(), n, features, out, at(p), code, st) != 0
+
+
+@pytest.mark.parametrize("n,features,out,n_mats,packs", [(70, 72, 64, 3, 0), (70, 64, 64, 3, 1), (70, 136, 64, 3, 1), (70, 72, 40, 3, 1), (70, 72, 64, 97, 1), (0, 72, 64, 3, 1)])
+def test_linear_with_the_packing_is_timed_once(cuda, n, features, out, n_mats, packs):
+    """One linear and, where the packing is a launch of its own, one packing; no linear without rows"""
+    L, st = _lib.lib(), torch.cuda.current_stream(cuda).cuda_stream
+    x, W, b, y = (torch.zeros(s, device=cuda) for s in ((n, features), (out, features), (out,), (n, out)))
+    w, v = torch.zeros(64, 64, device=cuda), torch.zeros(64, device=cuda)
+    frags, flat = torch.empty(L.tgt_node_frag_bytes(n_mats, _lib.DTYPE_F32), dtype=torch.uint8, device=cuda), torch.empty(64, device=cuda)
+    sizes, mats, vecs, lens = (ctypes.c_int * n_mats)(*[64] * n_mats), (ctypes.c_void_p * n_mats)(*[w.data_ptr()] * n_mats), (ctypes.c_void_p * 1)(v.data_ptr()), (ctypes.c_int * 1)(64)
+    at = ctypes.addressof
+    p = _PackArgs(at(mats), at(sizes), at(sizes), at(sizes), n_mats, at(vecs), at(lens), 1, frags.data_ptr(), flat.data_ptr())
+    L.tgt_timing_enable(1)
+    try:
+        L.tgt_timing_reset()
+        _lib.check(L.tgt_linear_fwd_and_pack(x.data_ptr(), W.data_ptr(), b.data_ptr(), y.data_ptr(), n, features, out, at(p), _lib.DTYPE_F32, st))
+        times = _lib.kernel_timings()
+    finally:
+        L.tgt_timing_reset()
+        L.tgt_timing_enable(0)
+    assert times["linear_fwd"][1] == (n > 0) and times["node_pack"][1] == packs

@@ -1031,12 +1031,12 @@ int tgt_linear_fwd_and_pack(const void* d_x, const void* d_W, const void* d_b, v
     LinArgs a{};
     a.A[0] = d_x; a.W[0] = d_W; a.bias[0] = d_b; a.out[0] = d_y;
     a.nw = 1; a.N = N; a.K = in_features; a.M = out_features;
-    bool done;
-    {
+    bool beside = false;
+    if (const int rc = packs_beside(a, pack, dtype, beside)) return rc;
+    if (beside) {
         KernelTimer t(KS_LINEAR_FWD, (hipStream_t)stream);
-        if (const int rc = linear_tiles_and_pack(a, pack, dtype, (hipStream_t)stream, done)) return rc;
+        return linear_tiles_and_pack(a, *pack, dtype, (hipStream_t)stream);
     }
-    if (done) return TGT_OK;
     if (const int rc = tgt_node_pack_parts(pack->mats, pack->ld, pack->rows, pack->cols, pack->n_mats, pack->vecs, pack->lens, pack->n_vecs, dtype, pack->d_frags, pack->d_vecs, stream)) return rc;
     return tgt_linear_fwd(d_x, &d_W, &d_b, &d_y, 1, N, in_features, out_features, dtype, stream);
 }

@@ -16,8 +16,9 @@ struct LinArgs {
 
 // y_j = x W_j^T + b_j, or (dx) dx = sum_j dy_j W_j
 int linear_tiles(const LinArgs& a, bool dx, int dtype, hipStream_t st);
-// A forward with one output and the packing beside it, where one launch takes both (done: whether it did; else nothing was launched)
-int linear_tiles_and_pack(const LinArgs& a, const tgt_node_pack_args* pack, int dtype, hipStream_t st, bool& done);
+// Whether one launch takes a forward with one output and the packing beside it (an error for a bad packing), and that launch
+int packs_beside(const LinArgs& a, const tgt_node_pack_args* pack, int dtype, bool& fits);
+int linear_tiles_and_pack(const LinArgs& a, const tgt_node_pack_args& pack, int dtype, hipStream_t st);
 
 struct GradWArgs {
     const void* x;         // [N, K]

@@ -357,8 +357,6 @@ int gradw_tiles(const GradWArgs& a, int workers, int dtype, hipStream_t st) {
     return a.K <= 64 ? launch_gradw<nbf16, 1>(a, workers, st) : launch_gradw<nbf16, 2>(a, workers, st);
 }
 
-// (one column piece of a weight that stays in registers, what one launch can be told; 64 -> 64 has kernels of its own in linear.hip)
-static bool pack_fits(const LinArgs& a, const tgt_node_pack_args& p) { return a.N > 0 && a.M == 64 && a.K != 64 && a.K <= 128 && p.n_mats <= kPackMats && p.n_vecs <= kPackVecs; }
 template <typename T> static int launch_with_pack(const LinArgs& a, const tgt_node_pack_args& p, hipStream_t st) {
     static std::atomic<uint64_t> done{0};
     constexpr int lds = lin_lds<T>();
@@ -369,12 +367,14 @@ template <typename T> static int launch_with_pack(const LinArgs& a, const tgt_no
     TGT_HIP_CHECK(hipGetLastError());
     return TGT_OK;
 }
-int linear_tiles_and_pack(const LinArgs& a, const tgt_node_pack_args* pack, int dtype, hipStream_t st, bool& done) {
-    done = false;
+// (one column piece of a weight that stays in registers, what one launch can be told; 64 -> 64 has kernels of its own in linear.hip)
+int packs_beside(const LinArgs& a, const tgt_node_pack_args* pack, int dtype, bool& fits) {
     if (int rc = check_pack(pack, dtype)) return rc;
-    if (!pack_fits(a, *pack)) return TGT_OK;
-    done = true;
-    return dtype == TGT_DTYPE_F32 ? launch_with_pack<float>(a, *pack, st) : launch_with_pack<nbf16>(a, *pack, st);
+    fits = a.N > 0 && a.M == 64 && a.K != 64 && a.K <= 128 && pack->n_mats <= kPackMats && pack->n_vecs <= kPackVecs;
+    return TGT_OK;
+}
+int linear_tiles_and_pack(const LinArgs& a, const tgt_node_pack_args& pack, int dtype, hipStream_t st) {
+    return dtype == TGT_DTYPE_F32 ? launch_with_pack<float>(a, pack, st) : launch_with_pack<nbf16>(a, pack, st);
 }
 
 int linear_tiles(const LinArgs& a, bool dx, int dtype, hipStream_t st) {
