@@ -1334,6 +1334,13 @@ static int ids_bwd_grid(int b, int H) {
     return std::min(total_pairs, std::max(unit, 2 * device_cus() / unit * unit));
 }
 
+// Whether the plane kernels take the backward of every sequence of NT tiles: nothing here would be launched for them
+template <int D, int NT> constexpr bool plane_takes_all() {
+    for (int S = 32 * (NT - 1) + 1; S <= 32 * NT; ++S)
+        if (!dense_plane_pays_bwd(S, D)) return false;
+    return true;
+}
+
 template <typename T, int D, int NT, int BSRC>
 static int launch_dense(const DenseCall& c, bool bwd) {
     constexpr int lds_f0 = fwd_lds_bytes<D, NT>(), lds_b0 = bwd_lds_bytes<D, NT>();
@@ -1351,25 +1358,30 @@ static int launch_dense(const DenseCall& c, bool bwd) {
                       "build the bias tensor instead", c.S, c.ids.ns, c.ids.ne, std::max(lds_f, lds_b), kLdsLimit);
             return TGT_ERR_UNSUPPORTED;
         }
-        if constexpr (BSRC == 0 && std::is_same<T, dbf16>::value)
+        constexpr bool PLANE = BSRC == 0 && std::is_same<T, dbf16>::value, PLANE_BWD = PLANE && plane_takes_all<D, NT>();
+        constexpr bool ONE_WALK = BSRC == 0 && bwd1_fits<D, NT>(), TWO_WALKS = !PLANE_BWD && !ONE_WALK;
+        if constexpr (PLANE)
             if ((c.bias || bwd) && dense_plane_pays((int64_t)c.b * c.H, c.S, D, bwd)) return dense_plane<D>(c, bwd);
         const float scale = sqrtf((float)c.d);     // the reference MULTIPLIES q by sqrt(d)
         const dim3 block(64 * NT);
         const bool thin = c.S - (NT - 1) * 32 <= 4;      // a last tile of at most four rows
         static bool attr_done = false;     // raise the dynamic-LDS cap once per instantiation
         if (!attr_done) {
-            const int cap_f = BSRC == 1 ? kLdsLimit : lds_f0, cap_b = BSRC == 1 ? kLdsLimit : lds_b0;
+            const int cap_f = BSRC == 1 ? kLdsLimit : lds_f0;
             if (cap_f > 48 * 1024) {
                 TGT_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_dense_fwd<T, D, NT, false, BSRC>),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, cap_f));
                 TGT_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_dense_fwd<T, D, NT, true, BSRC>),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, cap_f));
             }
-            if (cap_b > 48 * 1024) {
-                TGT_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_dense_bwd<T, D, NT, false, BSRC>),
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, cap_b));
-                TGT_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_dense_bwd<T, D, NT, true, BSRC>),
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, cap_b));
+            if constexpr (TWO_WALKS) {
+                const int cap_b = BSRC == 1 ? kLdsLimit : lds_b0;
+                if (cap_b > 48 * 1024) {
+                    TGT_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_dense_bwd<T, D, NT, false, BSRC>),
+                                                      hipFuncAttributeMaxDynamicSharedMemorySize, cap_b));
+                    TGT_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_dense_bwd<T, D, NT, true, BSRC>),
+                                                      hipFuncAttributeMaxDynamicSharedMemorySize, cap_b));
+                }
             }
             attr_done = true;
         }
@@ -1391,7 +1403,10 @@ static int launch_dense(const DenseCall& c, bool bwd) {
             else
                 hipLaunchKernelGGL((k_dense_fwd<T, D, NT, false, BSRC>), grid, block, lds_f, c.st, (const T*)c.q, (const T*)c.k,
                                    (const T*)c.v, (const T*)c.bias, (T*)c.o_out, c.o_lse, c.S, c.H, scale, c.b, da, c.ids);
-        } else if constexpr (BSRC == 0 && bwd1_fits<D, NT>()) {
+        } else if constexpr (PLANE_BWD) {
+            set_error("dense attention: no kernel for %d rows of head dim %d", c.S, D);      // (dense_plane has returned)
+            return TGT_ERR_UNSUPPORTED;
+        } else if constexpr (ONE_WALK) {
             // bias tensor (or none) and a shape whose dQ shares fit the LDS: every score tile is formed once
             constexpr int lds1_max = bwd1_lds_bytes<D, NT>();
             const int lds1 = bwd1_lds_bytes<D, NT>(thin ? (NT - 1) * 32 : NT * 32);

@@ -230,13 +230,13 @@ constexpr int plane_bwd_lds(int D, int S) {
 //   graphs 9.7, 14.9, 24.5 against 8.8, 15.6, 28.0.
 // - Backward at head dim 8, up to 24 rows (and one behind 32) are a fraction of a tile either way, and the plane is a phase more:
 //   400 graphs of 12, 20, 28 rows 8.8, 9.7, 11.0 against 8.2, 8.8, 13.7.
+constexpr bool dense_plane_pays_bwd(int S, int D) {
+    return plane_bwd_lds(D, S) <= kLdsLimit && (D == 8 ? S > 24 && S != 33 && S % 16 != 0 : (D == 16 ? S % 64 != 0 : true));
+}
 inline bool dense_plane_pays(int64_t pairs, int S, int D, bool bwd) {
-    if ((bwd ? plane_bwd_lds(D, S) : plane_fwd_lds(D, S)) > kLdsLimit) return false;
-    if (!bwd) {
-        const int thin = S - plane_tiles(S) * 32;
-        return 2 * S * S <= 64 * 1024 && (S % 16 != 0 || (S % 32 == 16 && S < (D == 32 ? 160 : 64))) && (thin < 1 || thin > 2 || pairs >= 4 * device_cus());
-    }
-    return D == 8 ? S > 24 && S != 33 && S % 16 != 0 : (D == 16 ? S % 64 != 0 : true);
+    if (bwd) return dense_plane_pays_bwd(S, D);
+    const int thin = S - plane_tiles(S) * 32;
+    return plane_fwd_lds(D, S) <= kLdsLimit && 2 * S * S <= 64 * 1024 && (S % 16 != 0 || (S % 32 == 16 && S < (D == 32 ? 160 : 64))) && (thin < 1 || thin > 2 || pairs >= 4 * device_cus());
 }
 
 }  // namespace tgt
