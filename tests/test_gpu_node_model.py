@@ -213,19 +213,21 @@ def test_rows_beside_the_lines_between_variants(cuda, n, heads):
                 assert o <= (2e-2 if dtype == torch.bfloat16 else 1e-6 if name == "output" else (2 * n) ** -0.5), f"{name}: {o}"
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n,heads", [(17, 2), (65, 4), (1000, 8), (16383, 8), (16385, 4), (32767, 2), (40000, 4), (65537, 2)])
-def test_gt_gradients_where_no_relu_changes_its_side(cuda, monkeypatch, n, heads):
-    """float32, the rows beside the lines between variants once more: weights in front of a ReLU are small beside its biases of +-2, so its inputs keep their sign
-    (2 against at most 0.2 times ten standard deviations) and the two ways of running the model agree to float32 rounding in every gradient"""
-    print(f"gt without ReLUs near 0: n={n} heads={heads}", flush=True)
-    model = scaled(GT(2, heads, 32, 64, 5, 1, 0.0, 0.0, 0.0, 64, 0), n, torch.float32, cuda)
+def test_gt_gradients_where_no_relu_changes_its_side(cuda, monkeypatch, dtype, n, heads):
+    """The rows beside the lines between variants once more: weights in front of a ReLU are small beside its biases of +-2, so its inputs keep their sign
+    (2 against at most 0.2 times ten standard deviations) and the two ways of running the model agree to rounding in every gradient, and in the output and the
+    input gradient in every element: a row that is lost or another's is off by what a typical element is, a fifth of the largest or more"""
+    print(f"gt without ReLUs near 0: n={n} heads={heads} {dtype}", flush=True)
+    model = scaled(GT(2, heads, 32, 64, 5, 1, 0.0, 0.0, 0.0, 64, 0), n, dtype, cuda)
     relus = [layer.FFN_layer1 for layer in model.layers] + list(model.MLP_layer.FC_layers[:2])
     with torch.no_grad():
         for linear in relus:
             linear.weight.mul_(0.1)
             linear.bias.copy_(torch.where(torch.arange(linear.bias.numel(), device=cuda) % 3 == 2, -2.0, 2.0))
     seen, relu = [], gt.ReluFunction.apply
-    x = torch.randn(n, 32, generator=torch.Generator().manual_seed(n)).to(cuda)
+    x = torch.randn(n, 32, generator=torch.Generator().manual_seed(n)).to(cuda, dtype)
     plan = GraphPlan(random_edges(n, 0, n + 2, cuda), n)
     with monkeypatch.context() as patch:
         patch.setattr(gt.ReluFunction, "apply", staticmethod(lambda u: seen.append(float(u.detach().abs().min())) or relu(u)))
