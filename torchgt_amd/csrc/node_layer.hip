@@ -279,7 +279,7 @@ template <int N> __device__ __forceinline__ void clear(float (&col)[N]) {
 // What the kernels begin with, and the block waves' part of it
 #define TGT_BWD_ROLES()                                                                                                          \
     using L = Bwd<T, R, CN, NV>;                                                                                                 \
-    constexpr int P = Num<T>::P, FV = kFragVecs<P>, PB = L::kPlane, NC = L::kChain;                                              \
+    constexpr int P = Num<T>::P, PB = L::kPlane, NC = L::kChain;                                                                 \
     extern __shared__ __align__(16) unsigned char smem[];                                                                        \
     vec16* w = reinterpret_cast<vec16*>(smem + L::kW);                                                                           \
     float* vec = reinterpret_cast<float*>(smem + L::kVecs);                                                                      \

@@ -45,7 +45,7 @@ def watched_everywhere():
 class OneWalk(nn.Module):
     """``parameters()`` of a model in one walk over its modules.  ``zero_grad``, a gradient clip and a flattening all-reduce each ask for
     them on every step, and ``nn.Module`` spells out the name of every parameter through a generator per module for it: 92 us for
-    the 72 parameters of four layers, 38 here (half a step of 4 K nodes is host time).  Names are only left out where nobody could
+    the 72 parameters of four layers, 43 here (half a step of 4 K nodes is host time).  Names are only left out where nobody could
     see them: a class or an object that brings its own ``named_parameters`` or ``named_modules`` is asked in the general way."""
 
     def parameters(self, recurse=True):
