@@ -225,6 +225,9 @@ constexpr int plane_bwd_lds(int D, int S) {
 //   backward 27, 67, 75 against 22, 43, 55 (head dim 8; with more products per element the conflicts weigh less: 16 with S = 80, 96, 160
 //   43.5, 49, 82 against 58, 56, 99, S = 64, 128 30, 70 against 32, 65, and at 32 all 1.1 to 1.7 times faster; forward at 32, S = 80,
 //   144, 176 29.6, 46, 52 against 54.7, 65, 44).
+// - Forward, few rows: the general kernel's walk takes as long for them as for 32, the plane's loads do not.  400 graphs of 2, 12, 16, 24, 31, 48 rows 4.7, 4.8, 5.0, 5.1,
+//   5.3, 11.2 against 18.7, 13.4, 12.8, 13.7, 15.1, 15.0 (head dim 16 5.0, 5.2, 5.6, 5.7, 6.0, 12.5 against 25.8, 14.1, 13.5, 15.3, 16.9, 18.6); 32 graphs of up
+//   to 31 rows 2.9 (3.1) against 4.1 to 5.3 (4.2 to 6.6), of 48 3.9 (4.2) against 4.5 (4.8).
 // - Forward, a plane of more than 64 KiB leaves one workgroup on a CU: S = 180 30.0 against 29.9, 201 39.3 against 30.6.
 // - Forward, one or two thin rows follow the walk of the first waves, which the other planes of a CU have to cover: S = 129 of 64, 128, 256
 //   graphs 9.7, 14.9, 24.5 against 8.8, 15.6, 28.0.
