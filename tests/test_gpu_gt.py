@@ -12,6 +12,7 @@ import torch
 from oracle import gt as ogt
 from torchgt_amd import _lib, workloads
 from torchgt_amd.gt import _DT, GT, ReluFunction
+from torchgt_amd.multi_head_attention import LinearFunction
 
 pytestmark = pytest.mark.gpu
 
@@ -286,6 +287,37 @@ def test_readout_weight_gradients_are_as_exact_as_float32_products(cuda, n):
     bound = 2 ** -24 * (1 + k / 12) ** 0.5
     print(f"readout exactness n={n}: " + " ".join(f"{e:.2e}" for e in errs) + f" (bound {bound:.2e})", flush=True)
     assert max(errs) <= bound
+
+
+@pytest.mark.parametrize("n,m1,m2,out", [(4096, 32, 16, 40), (4096, 64, 64, 64), (16400, 36, 20, 12)])
+def test_readout_is_as_exact_as_its_linears_and_log_softmax(cuda, n, m1, m2, out):
+    """float32: rms error of log-probabilities and dx against 64 bits, next to that of the separate linears, ReLUs and torch's log_softmax on the same operands: no
+    larger than theirs, 5 % for sums in another order.  (dx of rows without a ReLU input within 1e-5 of 0: those may change their side.)"""
+    def run(dtype, linear, relu):
+        xs = x.to(dtype).requires_grad_(True)
+        y, near = xs, torch.ones(n, dtype=torch.bool, device=cuda)
+        for i in range(3):
+            y = linear(y, W[i].to(dtype), b[i].to(dtype))
+            if i < 2:
+                near &= y.detach().abs().min(1).values > 1e-5
+                y = relu(y)
+        lp = torch.log_softmax(y, 1)
+        return lp.detach(), torch.autograd.grad(lp, xs, dlogp.to(dtype))[0], near
+
+    errs = {"fused": [0.0, 0.0], "separate": [0.0, 0.0]}
+    for seed in range(3):
+        g = torch.Generator(device=cuda).manual_seed(seed + out)
+        rand = lambda *s: torch.randn(*s, generator=g, device=cuda)
+        W, b = [rand(m1, 64) / 8, rand(m2, m1) / m1 ** 0.5, rand(out, m2) / m2 ** 0.5], [rand(m) * 0.1 for m in (m1, m2, out)]
+        x, dlogp = rand(n, 64), rand(n, out)
+        lp, dx, near = run(torch.float64, lambda y, w, c: y @ w.t() + c, torch.relu)
+        fused = run_readout(x, W, b, dlogp, out)
+        for name, (p, d) in (("fused", fused[:2]), ("separate", run(torch.float32, lambda y, w, c: LinearFunction.apply(y, w, c)[0], ReluFunction.apply)[:2])):
+            for i, (a, r) in enumerate(((p, lp), (d[near], dx[near]))):
+                errs[name][i] += float((a.double() - r).norm() / r.norm()) / 3
+    print(f"readout n={n} widths {m1} {m2} {out}: {errs}", flush=True)
+    for a, s in zip(errs["fused"], errs["separate"]):
+        assert a <= 1.05 * s
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

@@ -165,7 +165,7 @@ __global__ __launch_bounds__((fwd_waves<T, R, SAME>() * 64)) void k_node_fwd(con
             } else {
                 TileOf<R> y;
                 linear<P, SAME>(y, s, w_next, vn + 2 * kVec, lane);
-                put_classes<T>(reinterpret_cast<T*>(a.logp), y, a.linear, a.classes, a.tokens, row0, N, stage, lane);
+                put_classes<T, false>(reinterpret_cast<T*>(a.logp), y, a.linear, a.classes, a.tokens, row0, N, stage, lane);
             }
         }
     }

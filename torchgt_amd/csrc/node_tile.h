@@ -227,6 +227,42 @@ template <int P> __device__ __forceinline__ void gemm_apart(Tile& acc, const Fra
     }
 }
 
+// acc += W b for sixteen rows, weights in the layout above, one block of rows after the other: its small terms by themselves, then acc and the
+// main products on top of their sum, which is rounded once per step of 32.  A block's planes are asked for as soon as those of the block before have been used.
+__device__ __forceinline__ void gemm_apart(TileOf<16>& acc, const Frags<3, 16>& b, const vec16* w, int lane) {
+    w += (lane & 0x33) | (gray2((lane >> 2) & 3) << 2);
+    bf16x8_t a[2][3];      // [step][plane]
+    const auto ask = [&](int m, int p) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) a[s][p] = __builtin_bit_cast(bf16x8_t, w[((4 * s + m) * 3 + p) * 64]);
+    };
+    ask(0, 2); ask(0, 1); ask(0, 0);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        float4_t c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            c = mma(a[s][2], b.p[s][0], c);
+            c = mma(a[s][1], b.p[s][1], c);
+            c = mma(a[s][1], b.p[s][0], c);
+        }
+        if (m < 3) { ask(m + 1, 2); ask(m + 1, 1); }
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            c = mma(a[s][0], b.p[s][2], c);
+            c = mma(a[s][0], b.p[s][1], c);
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) c[t] += acc.get(4 * m + t);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) c = mma(a[s][0], b.p[s][0], c);
+        if (m < 3) ask(m + 1, 0);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc.set(4 * m + t, c[t]);
+        fence_schedule();
+    }
+}
+
 // Whether a lane of the wave holds a NaN.  An infinity has no planes (what is left of it behind hi is NaN, and an infinite hi times the
 // mid plane of the other operand has any sign): every output that it touches comes out as NaN and is formed again by plain float32
 // multiply-adds, which give the +-inf or NaN that it has.  That second computation runs for waves with a NaN only.

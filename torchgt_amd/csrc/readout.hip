@@ -6,8 +6,8 @@
 // Widths up to 64, 32 and 16 in the model: as a kernel per linear, activation and softmax these are fourteen launches of 3 to 12 us for 64 K nodes
 // that read and write rows of 32 to 128 bytes (33 us forward and 58 backward, and their host time).  Here a wave carries its nodes
 // through all of it (node_tile.h), the narrow weights packed as 64 x 64 with zeros.  Backward: the roles of node_roles.h; bound by the chain of a
-// group's products.  64 K rows in bf16 8.4 us forward, 26.4 backward with its sums (5); float32 14.4 and 54.2.  Of these 0.3 and 0.6, 0.6 and 2.7 keep infinities
-// what they are (`mend`, `add_product`).
+// group's products.  64 K rows (kernel trace): bf16 10.8 us forward, 24.9 + 4 (the sums) backward; float32 16.5 and 53 + 4.  Of these 0.4 and 0.8, 0.8 and
+// 2.7 keep infinities what they are (`mend`, `add_product`) and the float32 sums as exact as the linears' (`product`).
 #include "node_roles.h"
 #include "class_rows.h"
 
@@ -58,14 +58,13 @@ __device__ __forceinline__ void whole(TileOf<kRows>& t, const Frags<3, kRows>& f
         for (int e = 0; e < 8; ++e) t.set(8 * s + e, from_planes(v[0][e], v[1][e], v[2][e]));
     }
 }
-__device__ __forceinline__ void whole(TileOf<kRows>& t, const TileOf<kRows>& f) { t = f; }
 // Behind a product y = W x: what operands that are not finite leave of it where it does not belong.  float32: the product again, without planes
 // (`holds_nan`).  bf16: zeros in the features behind `outs`, where the packing's zeros met an infinity and the next product would read the NaN (the last
 // feature has one if any has).  TAIL: zeros in the rows past the end, whose ReLUs are off then: they must not add to
 // sums over nodes (0 times an infinite weight).
 // The rare part stands apart from the rest: in its place it is a few KB that every wave fetches its way around (bf16, 64 K rows, backward: 25.8 us
 // without `mend`, 28.1 in its place, 26.4 apart; a look of half the instructions, v_maximum3 of two values each, takes as long).
-template <int P, bool TAIL, typename B> __device__ __forceinline__ void mend(TileOf<kRows>& y, const B& x, const vec16* w, const float* bias, int outs, int ins, vec16* stage, const Rows& rows, int lane) {
+template <int P, bool TAIL> __device__ __forceinline__ void mend(TileOf<kRows>& y, const Frags<P, kRows>& x, const vec16* w, const float* bias, int outs, int ins, vec16* stage, const Rows& rows, int lane) {
     constexpr int R = kRows;
     const int g = lane / R;
     bool off;
@@ -81,6 +80,16 @@ template <int P, bool TAIL, typename B> __device__ __forceinline__ void mend(Til
         }
         TGT_EACH(i) if ((P == 1 && R * g + i >= outs) || (TAIL && lane % R >= rows.left)) y.set(i, 0.f);
     }
+}
+
+// y = W x + bias (null: without).  float32: the small terms of the planes in a sum of their own, as the linears of any width have them.  rms
+// error of the log-probabilities and of dx against 64 bits, widths 32, 16, 40 (64, 64, 64), here / with all six terms in one sum / as separate kernels: 4.5e-8 /
+// 6.9e-8 / 6.2e-8 (4.3e-8 / 7.5e-8 / 6.7e-8) and 1.72e-7 / 1.97e-7 / 1.67e-7 (1.70e-7 / 2.22e-7 / 2.09e-7).  (put_classes has its share in the first.)
+template <int P> __device__ __forceinline__ void product(TileOf<kRows>& y, const Frags<P, kRows>& x, const vec16* w, const float* bias, int lane) {
+    if (bias) load_vec(y, bias, lane / kRows);
+    else zero(y);
+    if constexpr (P == 3) gemm_apart(y, x, w, lane);
+    else gemm<P>(y, x, w, lane);
 }
 
 template <typename T> __global__ __launch_bounds__(kWaves * 64) void k_readout_fwd(const tgt_readout_fwd_args a) {
@@ -99,17 +108,21 @@ template <typename T> __global__ __launch_bounds__(kWaves * 64) void k_readout_f
         const Rows rows(t0, N, R);
         Raw<T, R> raw;
         fetch(raw, reinterpret_cast<const T*>(a.x), rows, lane);
-        TileOf<R> x, y;
-        settle<T, false>(x, raw, stage, rows, lane);
-        linear<P, false>(y, x, w, vec, lane);
+        TileOf<R> y;
+        Frags<P, R> x;
+        settle<T, false>(y, raw, stage, rows, lane);
+        make_frags(x, y);
+        product<P>(y, x, w, vec, lane);
         mend<P, false>(y, x, w, vec, a.m1, 64, stage, rows, lane);
         relu<T>(y);
-        linear<P, false>(x, y, w + FV, vec + kVec, lane);
-        mend<P, false>(x, y, w + FV, vec + kVec, a.m2, a.m1, stage, rows, lane);
-        relu<T>(x);
-        linear<P, false>(y, x, w + 2 * FV, vec + 2 * kVec, lane);
+        make_frags(x, y);
+        product<P>(y, x, w + FV, vec + kVec, lane);
+        mend<P, false>(y, x, w + FV, vec + kVec, a.m2, a.m1, stage, rows, lane);
+        relu<T>(y);
+        make_frags(x, y);
+        product<P>(y, x, w + 2 * FV, vec + 2 * kVec, lane);
         if constexpr (P == 3) mend<P, false>(y, x, w + 2 * FV, vec + 2 * kVec, a.out, a.m2, stage, rows, lane);
-        put_classes<T>(reinterpret_cast<T*>(a.logp), y, false, a.classes, 0, t0 * R, N, stage, lane);
+        put_classes<T, P == 3>(reinterpret_cast<T*>(a.logp), y, false, a.classes, 0, t0 * R, N, stage, lane);
     }
 }
 
@@ -192,7 +205,7 @@ template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN,
             ClassGrads<T, R> classes(reinterpret_cast<const T*>(a.dlogp), reinterpret_cast<const T*>(a.logp), false, a.classes, 0, tile * R, N, stage, lane);
             if (g0 + gridDim.x < groups) fetch(raw, reinterpret_cast<const T*>(a.x), Rows(tile + NC * (int64_t)gridDim.x, N, R), lane);
             __syncthreads();                                        // Wa is there; product Wa of the round before is done
-            linear<P, false>(t, fx, w, vec, lane);
+            product<P>(t, fx, w, vec, lane);
             mend<P, true>(t, fx, w, vec, a.m1, 64, stage, rows, lane);
             __syncthreads();                                        // Wa has been used
             const uint32_t on1 = relu<T>(t);
@@ -202,15 +215,14 @@ template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN,
             col[2] += column_sums(d, lane);
             make_frags(f, d);
             __syncthreads();                                        // Wb
-            linear<P, false>(t, fy, w, vec + kVec, lane);
+            product<P>(t, fy, w, vec + kVec, lane);
             mend<P, true>(t, fy, w, vec + kVec, a.m2, a.m1, stage, rows, lane);
             __syncthreads();                                        // Wb has been used
             const uint32_t on2 = relu<T>(t);
             put_tile_planes<PB, P>(p_x, row, h, t);
             put_planes<PB>(p_dy, row, h, f);
             __syncthreads();                                        // planes of Wc; Wc^T
-            zero(t);
-            gemm<P>(t, f, w, lane);                                 // beside product Wc
+            product<P>(t, f, w, nullptr, lane);                     // beside product Wc
             if constexpr (P == 3) mend<P, false>(t, f, w, nullptr, a.m2, a.out, stage, rows, lane);
             relu_back<T>(t, on2);
             col[1] += column_sums(t, lane);
@@ -219,8 +231,7 @@ template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN,
             put_planes<PB>(p_dy, row, h, f);
             put_planes<PB>(p_x, row, h, fy);
             __syncthreads();                                        // planes of Wb; Wb^T
-            zero(t);
-            gemm<P>(t, f, w, lane);                                 // beside product Wb
+            product<P>(t, f, w, nullptr, lane);                     // beside product Wb
             if constexpr (P == 3) mend<P, false>(t, f, w, nullptr, a.m1, a.m2, stage, rows, lane);
             relu_back<T>(t, on1);
             col[0] += column_sums(t, lane);
@@ -229,8 +240,7 @@ template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN,
             put_planes<PB>(p_dy, row, h, f);
             put_planes<PB>(p_x, row, h, fx);
             __syncthreads();                                        // planes of Wa; Wa^T
-            zero(t);
-            gemm<P>(t, f, w, lane);                                 // dx, beside product Wa
+            product<P>(t, f, w, nullptr, lane);                     // dx, beside product Wa
             if constexpr (P == 3) mend<P, false>(t, f, w, nullptr, 64, a.m1, stage, rows, lane);
             __syncthreads();                                        // Wa^T has been used
             put_rows(reinterpret_cast<T*>(a.dx), t, stage, rows, lane);
