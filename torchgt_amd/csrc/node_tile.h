@@ -227,8 +227,10 @@ template <int P> __device__ __forceinline__ void gemm_apart(Tile& acc, const Fra
     }
 }
 
-// acc += W b for sixteen rows, weights in the layout above, one block of rows after the other: its small terms by themselves, then acc and the
-// main products on top of their sum, which is rounded once per step of 32.  A block's planes are asked for as soon as those of the block before have been used.
+// acc += W b for sixteen rows, weights in the layout above, one block of rows after the other: its small terms in a sum of their own, the main product of each step
+// by itself, and these added up by float adds - a matrix instruction does not round its sum to nearest, and what it leaves adds up over nodes (with both main
+// products on top of the small sum, the gradients of four GT layers behind it are off by 5.7e-7 rms, 5.1e-7 this way).  A block's planes
+// are asked for as soon as those of the block before have been used.
 __device__ __forceinline__ void gemm_apart(TileOf<16>& acc, const Frags<3, 16>& b, const vec16* w, int lane) {
     w += (lane & 0x33) | (gray2((lane >> 2) & 3) << 2);
     bf16x8_t a[2][3];      // [step][plane]
@@ -252,13 +254,12 @@ __device__ __forceinline__ void gemm_apart(TileOf<16>& acc, const Frags<3, 16>& 
             c = mma(a[s][0], b.p[s][2], c);
             c = mma(a[s][0], b.p[s][1], c);
         }
+        float4_t main[2];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) c[t] += acc.get(4 * m + t);
-#pragma unroll
-        for (int s = 0; s < 2; ++s) c = mma(a[s][0], b.p[s][0], c);
+        for (int s = 0; s < 2; ++s) main[s] = mma(a[s][0], b.p[s][0], float4_t{0.f, 0.f, 0.f, 0.f});
         if (m < 3) ask(m + 1, 0);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) acc.set(4 * m + t, c[t]);
+        for (int t = 0; t < 4; ++t) acc.set(4 * m + t, (main[0][t] + main[1][t]) + (c[t] + acc.get(4 * m + t)));
         fence_schedule();
     }
 }

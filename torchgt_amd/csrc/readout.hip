@@ -6,8 +6,8 @@
 // Widths up to 64, 32 and 16 in the model: as a kernel per linear, activation and softmax these are fourteen launches of 3 to 12 us for 64 K nodes
 // that read and write rows of 32 to 128 bytes (33 us forward and 58 backward, and their host time).  Here a wave carries its nodes
 // through all of it (node_tile.h), the narrow weights packed as 64 x 64 with zeros.  Backward: the roles of node_roles.h; bound by the chain of a
-// group's products.  64 K rows (kernel trace): bf16 10.8 us forward, 24.9 + 4 (the sums) backward; float32 16.5 and 53 + 4.  Of these 0.4 and 0.8, 0.8 and
-// 2.7 keep infinities what they are (`mend`, `add_product`) and the float32 sums as exact as the linears' (`product`).
+// group's products.  64 K rows (kernel trace): bf16 10.8 us forward, 24.9 + 4 (the sums) backward; float32 16.6 and 54 + 4.  Of these 0.4 and 0.8, 0.9 and
+// 3.5 keep infinities what they are (`mend`, `add_product`) and the float32 sums as exact as the linears' (`product`).
 #include "node_roles.h"
 #include "class_rows.h"
 
@@ -84,7 +84,7 @@ template <int P, bool TAIL> __device__ __forceinline__ void mend(TileOf<kRows>& 
 
 // y = W x + bias (null: without).  float32: the small terms of the planes in a sum of their own, as the linears of any width have them.  rms
 // error of the log-probabilities and of dx against 64 bits, widths 32, 16, 40 (64, 64, 64), here / with all six terms in one sum / as separate kernels: 4.5e-8 /
-// 6.9e-8 / 6.2e-8 (4.3e-8 / 7.5e-8 / 6.7e-8) and 1.72e-7 / 1.97e-7 / 1.67e-7 (1.70e-7 / 2.22e-7 / 2.09e-7).  (put_classes has its share in the first.)
+// 6.9e-8 / 6.2e-8 (4.3e-8 / 7.5e-8 / 6.7e-8) and 1.70e-7 / 1.97e-7 / 1.67e-7 (1.70e-7 / 2.22e-7 / 2.09e-7).  (put_classes has its share in the first.)
 template <int P> __device__ __forceinline__ void product(TileOf<kRows>& y, const Frags<P, kRows>& x, const vec16* w, const float* bias, int lane) {
     if (bias) load_vec(y, bias, lane / kRows);
     else zero(y);
