@@ -545,25 +545,44 @@ struct RecLane {
     uint32_t code;
     int row, start, len;     // of the row this lane group works on (zeros behind the record's last row)
     int4 cols, eids;         // inline classes: the lane group's four edges (other endpoint, bias row)
-    const int32_t* col_p;    // EDGES == false: where cols and eids are, for a read at the point of use
-    const int32_t* eid_p;
+    const int32_t* rec;      // EDGES == false: the record (a scalar), which rec_cols and rec_eids read where the edges are used
 };
-// EDGES: whether the four edges come along at once.  The 4-byte backward holds two gathered rows per edge in
-// registers and has none to spare for edges that wait through the class dispatch: it reads them where it uses them.
-template <int LPE, bool EDGES>
-__device__ __forceinline__ RecLane load_rec_lane(const WaveRec<LPE>& rec) {
+template <int LPE> __device__ __forceinline__ int4 rec_edges(const int32_t* rec, const int word) {
+    return *reinterpret_cast<const int4*>(rec + word + (threadIdx.x & (kWave - 1)) / LPE * kUnroll);
+}
+template <int LPE> __device__ __forceinline__ int4 rec_cols(const RecLane& r) { return rec_edges<LPE>(r.rec, offsetof(WaveRec<LPE>, col) / 4); }
+template <int LPE> __device__ __forceinline__ int4 rec_eids(const RecLane& r) { return rec_edges<LPE>(r.rec, offsetof(WaveRec<LPE>, eid) / 4); }
+// EDGES: whether the four edges come along at once.  The 4-byte backward holds two gathered rows per edge in registers and has none
+// to spare for edges that wait through the class dispatch: it reads them where it uses them, and here asks for one word of each of
+// their lines, which are near by then.  EIDS: whether there are bias rows to name.
+// Every word is waited for here, in front of the first branch on the code.  The compiler moves a load whose users are behind a branch
+// behind it, and then the code, the row's words and the edges are a memory round trip each (three to five in a row instead of one, of
+// waves that live for three or four).  Forward + backward, before / after: 64 K nodes, 0.53 M edges, float32 with a bias per edge and
+// head 131.2 / 128.5 us; bf16 without a bias 262 K nodes, 5 M edges 412 / 374 us, 870 K nodes, 44 M edges 3275 / 3131 us.
+template <int LPE, bool EDGES, bool EIDS>
+__device__ __forceinline__ RecLane load_rec_lane(const Common& c, const SideArgs& s, const WaveRec<LPE>* recs) {
     const int lg = (threadIdx.x & (kWave - 1)) / LPE;
+    const WaveRec<LPE>& rec = recs[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];
     RecLane r;
+    r.rec = reinterpret_cast<const int32_t*>(&rec);
     r.code = rec.code;
     r.row = rec.row[lg];
     r.start = rec.start[lg];
     r.len = rec.len[lg];
-    r.col_p = rec.col + lg * kUnroll;
-    r.eid_p = rec.eid + lg * kUnroll;
+    int32_t near = 0, near2 = 0;
     if (EDGES) {
-        r.cols = *reinterpret_cast<const int4*>(r.col_p);
-        r.eids = *reinterpret_cast<const int4*>(r.eid_p);
+        r.cols = rec_cols<LPE>(r);
+        if (EIDS) r.eids = rec_eids<LPE>(r);
+    } else {
+        near = rec.col[lg * kUnroll];
+        if (EIDS) near2 = rec.eid[lg * kUnroll];
     }
+    asm volatile("" ::"s"(c.q), "s"(c.k), "s"(c.v), "s"(s.out0), "s"(r.code));
+    asm volatile("" ::"v"(r.row), "v"(r.start), "v"(r.len));
+    if (EDGES) {
+        asm volatile("" ::"v"(r.cols.x), "v"(r.cols.y), "v"(r.cols.z), "v"(r.cols.w));
+        if (EIDS) asm volatile("" ::"v"(r.eids.x), "v"(r.eids.y), "v"(r.eids.z), "v"(r.eids.w));
+    } else asm volatile("" ::"v"(near), "v"(near2));
     return r;
 }
 template <typename T, int MODE> constexpr bool rec_edges_early() { return sizeof(T) == 2 || MODE == MODE_FWD; }
@@ -679,6 +698,8 @@ __device__ __forceinline__ void walk_range(const Common& c, const SideArgs& s, c
         load_row<T, LPE, LPH, MODE>(c, row, el, valid, rr, acc);
         with_offsets<T>(c.narrow, [&](auto zero) {
             using O = decltype(zero);
+            // (the copy for large arrays reads its first ids again: the compiler would keep them through the loop of the other one)
+            if constexpr (std::is_same<O, uint64_t>::value) load_ids(0, nb, ed);
             Gathered<T> g[kUnroll];
 #pragma unroll
             for (int u = 0; u < kUnroll; ++u) ask_edge<T, LPE, LPH, MODE, HASB, O>(c, nb[u], ed[u], el, g[u]);
@@ -711,7 +732,7 @@ template <typename T, int LPE, int LPH, int S, int MODE, int HASB>
 __device__ __forceinline__ void walk_record(const Common& c, const SideArgs& s, const RecLane& rec, const int row,
                                             const int start, const int len, const int slot, const int el,
                                             const bool valid, Acc& acc) {
-    const int4 cols = rec_edges_early<T, MODE>() ? rec.cols : *reinterpret_cast<const int4*>(rec.col_p);
+    const int4 cols = rec_edges_early<T, MODE>() ? rec.cols : rec_cols<LPE>(rec);
     int nb[kUnroll] = {cols.x, cols.y, cols.z, cols.w};
     int ed[kUnroll] = {0, 0, 0, 0};
     bool ok[kUnroll];
@@ -726,7 +747,7 @@ __device__ __forceinline__ void walk_record(const Common& c, const SideArgs& s, 
 #pragma unroll
             for (int u = 0; u < kUnroll; ++u) ed[u] = s.eid[edge_of_slot(start, n, slot + u * S)];
         } else {
-            const int4 e4 = rec_edges_early<T, MODE>() ? rec.eids : *reinterpret_cast<const int4*>(rec.eid_p);
+            const int4 e4 = rec_edges_early<T, MODE>() ? rec.eids : rec_eids<LPE>(rec);
             ed[0] = e4.x; ed[1] = e4.y; ed[2] = e4.z; ed[3] = e4.w;
         }
     }
@@ -1028,7 +1049,7 @@ __device__ __forceinline__ void block_item(const Common& c, const SideArgs& s, c
 }
 
 // Waves per SIMD that the registers of the forward are kept down for: seven without a bias in bf16 rows of 32 and 64 elements, where that
-// costs nothing (72 registers, 76 without the bound, none in scratch; other shapes would spill); four in float32 (128 elements with
+// costs nothing (72 registers, none in scratch; other shapes would spill); four in float32 (128 elements with
 // a bias take 130 registers unbounded: three waves, 38.9 us instead of 37.9 for 20 K nodes and 0.4 M edges)
 template <typename T, int LPE, int HASB, bool TILES> constexpr int fwd_waves() {
     return sizeof(T) == 4 ? 4 : ((LPE == 4 || LPE == 8) && HASB == 0 && !TILES ? 7 : 1);
@@ -1041,13 +1062,13 @@ __global__ __launch_bounds__(kBlock, (fwd_waves<T, LPE, HASB, TILES>())) void k_
                                                      const WaveRec<LPE>* __restrict__ recs) {
     __shared__ BlockLds<LPE> lds;
     const WaveRec<LPE>* r0 = recs + (int64_t)blockIdx.x * (kBlock / kWave);
-    const RecLane rec = load_rec_lane<LPE, true>(r0[threadIdx.x >> 6]);      // in flight while the workgroup's code is looked at
-    const uint32_t code0 = r0->code;
-    if ((code0 & 7u) == kDescBlock) {          // uniform over the workgroup
+    const RecLane rec = load_rec_lane<LPE, true, HASB == 1>(c, s, r0);
+    if ((rec.code & 7u) == kDescBlock) {          // uniform over the workgroup: its four records say so
         block_item<T, LPE, LPH, MODE_FWD, HASB, TILES>(c, s, r0->item, lds);
         return;
     }
-    const uint32_t code = __builtin_amdgcn_readfirstlane(rec.code);
+    uint32_t code = rec.code;
+    asm volatile("" : "+s"(code));      // (one dispatch over all kinds would keep the record's words in registers, or in scratch, through the item's code)
     if ((code & 7u) == kDescNone) return;
     wave_dispatch<T, LPE, LPH, MODE_FWD, HASB, TILES>(c, s, rec, code & 7u);
 }
@@ -1060,14 +1081,14 @@ __global__ __launch_bounds__(kBlock, 4) void k_attn_bwd(const Common c, const Si
     constexpr int HB_D = HASB == 3 ? 2 : HASB;
     constexpr int HB_S = HASB == 3 ? 2 : (HASB ? 1 : 0);
     const WaveRec<LPE>* r0 = recs + (int64_t)blockIdx.x * (kBlock / kWave);
-    const RecLane rec = load_rec_lane<LPE, sizeof(T) == 2>(r0[threadIdx.x >> 6]);      // in flight while the workgroup's code is looked at
-    const uint32_t code0 = r0->code;
-    if ((code0 & 7u) == kDescBlock) {          // uniform over the workgroup
-        if (code0 & kDescSrcSide) block_item<T, LPE, LPH, MODE_BWD_SRC, HB_S, TILES>(c, ss, r0->item, lds);
+    const RecLane rec = load_rec_lane<LPE, sizeof(T) == 2, HB_D == 1 || HB_S == 1>(c, sd, r0);
+    if ((rec.code & 7u) == kDescBlock) {          // uniform over the workgroup: its four records say so
+        if (rec.code & kDescSrcSide) block_item<T, LPE, LPH, MODE_BWD_SRC, HB_S, TILES>(c, ss, r0->item, lds);
         else block_item<T, LPE, LPH, MODE_BWD_DST, HB_D, TILES>(c, sd, r0->item, lds);
         return;
     }
-    const uint32_t code = __builtin_amdgcn_readfirstlane(rec.code);
+    uint32_t code = rec.code;
+    asm volatile("" : "+s"(code));      // (one dispatch over all kinds would keep the record's words in registers, or in scratch, through the item's code)
     if ((code & 7u) == kDescNone) return;
     if (code & kDescSrcSide) wave_dispatch<T, LPE, LPH, MODE_BWD_SRC, HB_S, TILES>(c, ss, rec, code & 7u);
     else wave_dispatch<T, LPE, LPH, MODE_BWD_DST, HB_D, TILES>(c, sd, rec, code & 7u);
