@@ -61,14 +61,17 @@ struct Item { int32_t row, start, len, part; };
 // bits 8.. number of rows.
 //   kind 0..4: wave items of that length class (count <= rows per wave of the shape)
 //   kind 5:    a workgroup item (all four records of the workgroup are equal)
+//   kind 6:    rows of kGroupRowMin .. kGroupRowMax edges (classes 1 to 3), each walked by one lane group
 //   kind 7:    nothing
-constexpr uint32_t kDescBlock = 5, kDescNone = 7, kDescSrcSide = 8;
+constexpr uint32_t kDescBlock = 5, kDescGroup = 6, kDescNone = 7, kDescSrcSide = 8;
+__host__ __device__ constexpr bool desc_is_rows(uint32_t kind) { return kind < (uint32_t)kNumClass || kind == kDescGroup; }
+constexpr int kGroupRowMin = 5, kGroupRowMax = 32, kGroupMinLpe = 8;      // (shapes of fewer lanes per edge have no such list)
 __host__ __device__ constexpr uint32_t desc_code(uint32_t kind, uint32_t src_side, uint32_t count) {
     return kind | (src_side ? kDescSrcSide : 0u) | (count << 8);
 }
 
 // Edge slots of a lane group: natural slot count of the length classes (>32, <=32, <=16, <=8, <=4),
-// capped by the wave (lpe = lanes that cover one edge).
+// capped by the wave (lpe = lanes that cover one edge).  One for kind 6.
 __host__ __device__ constexpr int slots_for_class(int lpe, int cls) {
     const int nat = cls == 0 ? 16 : (cls == 1 ? 8 : (cls == 2 ? 4 : (cls == 3 ? 2 : 1)));
     const int cap = kWave / lpe;
@@ -88,7 +91,8 @@ __host__ __device__ constexpr bool class_inline(int lpe, int cls) {
 //   with edges [start[g], start[g] + len[g]) of the view's sorted arrays (the S groups of a row hold the same
 //   three numbers; zeros behind the wave's last row); col / eid hold for lane group g the four edges s, s + S,
 //   s + 2S, s + 3S of its row at [4g, 4g + 4) (an edge past the end of the row repeats the row's last edge; 0 for
-//   an empty row): all edges of kinds 1..4 (class_inline), the first step of longer rows.
+//   an empty row): all edges of kinds 1..4 (class_inline), the first step of longer rows;
+//   kind 6: the same with S = 1.
 // No address in a record depends on the kind: a lane asks for code, row, start, len and its four edges at once,
 // and one memory round trip gives a wave everything it needs to issue its gathers.  (A workgroup item leaves
 // col / eid unwritten; what a lane reads there is never used.)
@@ -137,12 +141,16 @@ struct Side {
     std::vector<int32_t> homed_off, homed_idx;   // workgroup items by home window: items homed_idx[homed_off[w] .. homed_off[w+1])
 };
 
-// Wave records of one kernel shape (lanes per edge): forward (destination view) and backward
-// (both views, window by window).
+// Wave records of one kernel shape (lanes per edge): forward (destination view) and backward (both views, window by
+// window).  The backward has a second list in plans with `grouped` set, in which the rows of classes 1 to 3 go out as kind 6; the first use of
+// a shape makes one of the two, the other one is made when a call first asks for it.
 struct Schedule {
-    void* fwd = nullptr;    // WaveRec<lpe> [4 * fwd_blocks]
-    void* bwd = nullptr;
-    int32_t fwd_blocks = 0, bwd_blocks = 0;
+    struct List {
+        void* recs = nullptr;    // WaveRec<lpe> [4 * blocks]
+        int32_t blocks = 0;
+        bool ready = false;
+    };
+    List fwd, bwd, bwd_grouped;
     bool ready = false;
 };
 constexpr int kNumLpe = 5;   // lanes per edge 1, 2, 4, 8, 16
@@ -258,15 +266,17 @@ struct tgt_plan {
     // a plan of the edges that remain beside a tile set: rows without edges have no place in its schedules
     // (the tile kernels write them), so the sparse entry points on their own must refuse it
     bool rows_with_edges_only = false;
+    bool grouped = false;    // neighbours are near: the backward has a list with kind 6, the rows of a (window, class) are sorted by length
     tgt::Side dst;   // edges grouped by destination (query) node
     tgt::Side src;   // edges grouped by source (key/value) node
     tgt::Schedule sched[tgt::kNumLpe];   // by log2(lanes per edge); made on first use of a shape
     std::mutex sched_mutex;              // guards that first use
 };
 namespace tgt {
-// Descriptors for kernels with `lpe` lanes per edge; builds them on first use (allocates, copies and
-// synchronises `st` once per plan and shape).  nullptr on error.
-const Schedule* plan_schedule(const tgt_plan* plan, int lpe, hipStream_t st);
+// Descriptors for kernels with `lpe` lanes per edge, of a forward and a backward; builds them on first use (allocates, copies and
+// synchronises `st`, once per plan, shape and list).  nullptr on error.
+enum ScheduleLists { LISTS_ANY = 0, LISTS_BWD = 1, LISTS_BWD_GROUPED = 2 };      // (an `or` of them) which of the backward's lists the caller would like
+const Schedule* plan_schedule(const tgt_plan* plan, int lpe, hipStream_t st, int lists);
 // The same without building anything: nullptr if the shape has not been used or prepared yet.
 const Schedule* plan_schedule_if_ready(const tgt_plan* plan, int lpe);
 }

@@ -99,7 +99,17 @@ __device__ __forceinline__ int sched_category(int len, int wave_row_max, bool sk
 }
 
 // Per side, written by the device and read back once: how many of everything the schedule holds.
-struct SchedHeader { int32_t n_wave, n_long, n_block, n_split, n_parts, n_groups, pad0, pad1; };
+// looked, near: rows whose middle edge was looked at, and those of them whose other endpoint is within kNearRows.
+struct SchedHeader { int32_t n_wave, n_long, n_block, n_split, n_parts, n_groups, looked, near; };
+// Whether the neighbours of most rows are near enough to meet in an XCD's L2: the graph is clustered or reordered, or small.  The rows are
+// then sorted by length, for the backward's list with kind 6 (want_groups in sparse_attn.hip).  Without it the gathers are bound by the
+// traffic behind the L2s and a row's own data, gathered by its self-loop and loaded by both views, should stay close in time: 64 K
+// nodes without clusters, 0.5 M edges, bf16 35.4 us by classes, 38.4 as kind 6; 262 K nodes, 8.6 M edges 550 / 566.  From 16 000 rows on
+// (8000 nodes, 0.26 M edges 17.6 / 18.7), and with ten edges a row unless rows are many (64 K nodes in 64 clusters, 0.5 M edges 32.4 / 33.5, 150 K nodes, 1.2 M edges 68.9 / 67.2).
+constexpr int kNearRows = 8192, kNearWindows = 8;      // (every eighth window is asked)
+constexpr int64_t kManyRows = 128 << 10;
+static bool may_group(int64_t N, int64_t E) { return N >= 16000 && (E >= 10 * N || N >= kManyRows); }
+__host__ __device__ inline bool mostly_near(const SchedHeader& h) { return h.looked > 0 && 2 * (int64_t)h.near >= h.looked; }
 struct BlockMeta;
 // What the schedule kernels read and write, of both views (blockIdx.y)
 struct SchedArgs {
@@ -111,22 +121,33 @@ struct SchedArgs {
     BlockMeta* meta[2];
 };
 
-// counts[window * kSchedCats + cat] = rows of that category among the window's rows (blockDim.x rows)
-__global__ void k_sched_count(const SchedArgs a, int64_t N, int wave_row_max, bool skip_empty) {
+// counts[window * kSchedCats + cat] = rows of that category among the window's rows (blockDim.x rows).  look: whether the edges' distances
+// are asked for (mostly_near)
+__global__ void k_sched_count(const SchedArgs a, int64_t N, int wave_row_max, bool skip_empty, bool look) {
     const int32_t* __restrict__ rowptr = a.rowptr[blockIdx.y];
     uint32_t* __restrict__ counts = a.counts[blockIdx.y];
-    __shared__ uint32_t c[kSchedCats];
+    __shared__ uint32_t c[kSchedCats], near[2];
     if (threadIdx.x < kSchedCats) c[threadIdx.x] = 0;
+    if (threadIdx.x < 2) near[threadIdx.x] = 0;
     __syncthreads();
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int cat = r < N ? sched_category(rowptr[r + 1] - rowptr[r], wave_row_max, skip_empty) : -1;
+    const int start = r < N ? rowptr[r] : 0, len = r < N ? rowptr[r + 1] - start : 0;
+    const int cat = r < N ? sched_category(len, wave_row_max, skip_empty) : -1;
 #pragma unroll
     for (int k = 0; k < kSchedCats; ++k) {
         const uint64_t b = __ballot(cat == k);
         if ((threadIdx.x & 63) == 0 && b) atomicAdd(&c[k], (uint32_t)__popcll(b));   // integer count: order-free
     }
+    look = look && blockIdx.x % kNearWindows == 0;
+    if (look) {
+        const bool asked = len >= kGroupRowMin;
+        const bool is_near = asked && llabs((int64_t)a.col[blockIdx.y][start + (asked ? len / 2 : 0)] - r) <= kNearRows;
+        const uint64_t ba = __ballot(asked), bn = __ballot(is_near);
+        if ((threadIdx.x & 63) == 0 && ba) { atomicAdd(&near[0], (uint32_t)__popcll(ba)); atomicAdd(&near[1], (uint32_t)__popcll(bn)); }
+    }
     __syncthreads();
     if (threadIdx.x < kSchedCats) counts[(int64_t)blockIdx.x * kSchedCats + threadIdx.x] = c[threadIdx.x];
+    if (look && threadIdx.x == 0 && near[0]) { atomicAdd(&a.hdr[blockIdx.y]->looked, (int32_t)near[0]); atomicAdd(&a.hdr[blockIdx.y]->near, (int32_t)near[1]); }
 }
 
 // offs[window, cat]: first position of the window's rows of a category - wave classes count through
@@ -161,10 +182,19 @@ __global__ __launch_bounds__(1024) void k_sched_scan(const SchedArgs a, int nwin
     if (tid == 1023) { hdr->n_wave = (int32_t)sw[1023]; hdr->n_long = (int32_t)sl[1023]; }
 }
 
+// Order of the rows of a category by length, longest first, in steps of the kernels' loops: four edges for rows that one lane group walks,
+// sixteen for those of a whole wave.  Waves of a workgroup, and rows of a wave, then end together.
+constexpr int kLongBin = 16, kLongBins = (kWaveRowMax - kGroupRowMax - 1) / kLongBin + 1, kGroupBin = 4;
+constexpr int kSortBins = kLongBins + 6;
+__device__ __forceinline__ int sort_bin(int len, int cat) {
+    return cat == 0 ? max(kWaveRowMax - len, 0) / kLongBin : (cat == 1 ? kLongBins + (32 - len) / kGroupBin : (cat == 2 ? kLongBins + 4 + (16 - len) / kGroupBin : -1));
+}
+
 // Rows keep their order inside a (window, category): position = offs[window, cat] + rank among the
-// window's rows.  Wave-class rows become wave items at items[position]; long rows are listed (row, first
+// window's rows - behind their order by length where neighbours are near.  Wave-class rows become wave items at items[position]; long rows are listed (row, first
 // edge, length) for the kernels that cut them into workgroup items.
 __global__ void k_sched_fill(const SchedArgs a, int64_t N, int wave_row_max, bool skip_empty, int64_t cap_long) {
+    const bool by_length = mostly_near(*a.hdr[blockIdx.y]);
     const int32_t* __restrict__ rowptr = a.rowptr[blockIdx.y];
     const uint32_t* __restrict__ offs = a.offs[blockIdx.y];
     Item* __restrict__ items = a.items[blockIdx.y];
@@ -186,10 +216,29 @@ __global__ void k_sched_fill(const SchedArgs a, int64_t N, int wave_row_max, boo
         if (cat == k) rank = (uint32_t)__popcll(b & lower);
         if (lane == 0) wave_cnt[wave][k] = (uint32_t)__popcll(b);
     }
+    __shared__ uint32_t wave_bin[kSchedMaxWaves][kSortBins];
+    const int bin = by_length ? sort_bin(len, cat) : -1, bin0 = cat == 0 ? 0 : (cat == 1 ? kLongBins : kLongBins + 4);
+    if (by_length) {
+        if (bin >= 0) rank = 0;
+        for (int k = 0; k < kSortBins; ++k) {
+            const uint64_t b = __ballot(bin == k);
+            if (bin == k) rank += (uint32_t)__popcll(b & lower);
+            else if (bin > k && k >= bin0) rank += (uint32_t)__popcll(b);
+            if (lane == 0) wave_bin[wave][k] = (uint32_t)__popcll(b);
+        }
+    }
     __syncthreads();
     if (cat < 0) return;
     uint32_t pos = offs[(int64_t)blockIdx.x * kSchedCats + cat] + rank;
-    for (int w = 0; w < wave; ++w) pos += wave_cnt[w][cat];
+    if (bin >= 0) {
+        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
+            if (w == wave) continue;
+            for (int k = bin0; k < bin; ++k) pos += wave_bin[w][k];
+            if (w < wave) pos += wave_bin[w][bin];
+        }
+    } else {
+        for (int w = 0; w < wave; ++w) pos += wave_cnt[w][cat];
+    }
     if (cat < kNumClass) {
         items[pos] = Item{(int32_t)r, start, len, -1};
     } else if ((int64_t)pos < cap_long) {
@@ -338,9 +387,10 @@ __global__ void k_emit_items(const SchedArgs a, CutParams cp) {
 //   rows:       the wave items [first, first + n) of one (window, class), rows_per_wave of them per wave
 //   block item: workgroup item `first`; its four waves carry the same record
 //   nothing:    padding to whole workgroups, and behind the end of a list; n waves
-// code: descriptor code (kind, view), the XCD in bits 8 .. 10, bit 11: of the backward's launch.
+// code: descriptor code (kind, view), the XCD in bits 8 .. 10, the list in bits 11 and 12.
 struct Run { int32_t wave0, first, n; uint32_t code; };
-constexpr uint32_t kRunBackward = 1u << 11;
+enum { LIST_FWD = 0, LIST_BWD = 1, LIST_BWD_GROUPED = 2, LIST_COUNT = 3 };
+struct RecordLists { int32_t* recs[LIST_COUNT]; };
 __host__ __device__ inline int32_t run_waves(uint32_t kind, int32_t n, int lpe) {
     if (kind == kDescBlock) return 4;
     if (kind == kDescNone) return n;
@@ -348,7 +398,7 @@ __host__ __device__ inline int32_t run_waves(uint32_t kind, int32_t n, int lpe) 
     return (n + ipw - 1) / ipw;
 }
 
-// One workgroup per run, for the forward's and the backward's launch together; its sixteen waves write the run's wave records
+// One workgroup per run, for all lists that are made together; its sixteen waves write the run's wave records
 // in turn (layout: WaveRec in common.h), the lanes of a wave one edge or bias row each.  Wave lw of
 // XCD x's list is wave lw % 4 of that XCD's (lw / 4)-th workgroup, and workgroup b of the launch runs on XCD b mod 8:
 // record ((lw / 4) * 8 + x) * 4 + lw % 4.  Everything a kernel uses of a record is written: no clearing pass.
@@ -361,7 +411,7 @@ __global__ __launch_bounds__(64 * kRecordWaves) void k_build_records(const Run* 
                                                        const Item* __restrict__ bitems_s, const int32_t* __restrict__ col_d,
                                                        const int32_t* __restrict__ eid_d, const int32_t* __restrict__ col_s,
                                                        const int32_t* __restrict__ eid_s, WaveRecLayout L, int lpe,
-                                                       int32_t* __restrict__ recs_fwd, int32_t* __restrict__ recs_bwd) {
+                                                       const RecordLists lists) {
     const Run run = runs[blockIdx.x];
     const int t = threadIdx.x & 63;
     const uint32_t kind = run.code & 7u, xcd = (run.code >> 8) & 7u;
@@ -369,15 +419,15 @@ __global__ __launch_bounds__(64 * kRecordWaves) void k_build_records(const Run* 
     const Item* items = src ? items_s : items_d;
     const int32_t* col = src ? col_s : col_d;
     const int32_t* eid = src ? eid_s : eid_d;
-    int32_t* const recs = run.code & kRunBackward ? recs_bwd : recs_fwd;
-    const int ipw = kind < (uint32_t)kNumClass ? rows_per_wave(lpe, (int)kind) : 1;
-    const int S = kind < (uint32_t)kNumClass ? slots_for_class(lpe, (int)kind) : 1;
+    int32_t* const recs = lists.recs[(run.code >> 11) & 3u];
+    const int ipw = desc_is_rows(kind) ? rows_per_wave(lpe, (int)kind) : 1;
+    const int S = desc_is_rows(kind) ? slots_for_class(lpe, (int)kind) : 1;
     const int groups = kWave / lpe, waves = run_waves(kind, run.n, lpe);
     const auto record = [&](int w) {
         const int lw = run.wave0 + w;
         return recs + (((int64_t)(lw >> 2) * 8 + xcd) * 4 + (lw & 3)) * L.stride;
     };
-    if (kind >= (uint32_t)kNumClass) {
+    if (!desc_is_rows(kind)) {
         for (int w = threadIdx.x >> 6; w < waves; w += kRecordWaves) {
             int32_t* out = record(w);
             if (t != 0) continue;
@@ -472,8 +522,10 @@ static int env_int(const char* name, int dflt) {
     return x > 0 ? x : dflt;
 }
 
-static int window_rows() {
-    int w = env_int("TGT_WINDOW_ROWS", tgt::kWindowRows);
+// Windows of twice the rows in large graphs: 262 K nodes, 3.9 M edges in 64 clusters, bf16 k_attn_bwd 202 us with 128, 191 with 256; other
+// lists of such graphs take the same time either way (64 K nodes by classes 35.5 and 36.4 us).
+static int window_rows(int64_t N) {
+    int w = env_int("TGT_WINDOW_ROWS", N >= kManyRows ? 2 * tgt::kWindowRows : tgt::kWindowRows);
     w = (w + 63) / 64 * 64;
     return w > 64 * kSchedMaxWaves ? 64 * kSchedMaxWaves : w;
 }
@@ -510,7 +562,7 @@ constexpr int kReportFlag = 16;
 constexpr size_t kOneCopyBytes = 256 << 10;
 
 static int schedule_device(int64_t N, int64_t E, Side* const (&sides)[2], SideScratch (&scr)[2], int32_t* report, BlockMeta* metas, bool skip_empty,
-                           hipStream_t st) {
+                           bool look, int W, hipStream_t st) {
     SchedArgs a{};
     for (int i = 0; i < 2; ++i) {
         Side& side = *sides[i];
@@ -521,7 +573,7 @@ static int schedule_device(int64_t N, int64_t E, Side* const (&sides)[2], SideSc
         sc.cp.spread_seg = env_int("TGT_SPREAD_SEG", tgt::kSpreadSeg);
         sc.cp.spread_segs = kSpreadSegs;
         sc.cp.combine_fan = kCombineFan;
-        sc.W = window_rows();
+        sc.W = W;
         sc.cp.window = sc.W;
         sc.nwin = (int)((N + sc.W - 1) / sc.W);
         sc.cp.near = std::max(1, sc.nwin / 64);
@@ -546,7 +598,7 @@ static int schedule_device(int64_t N, int64_t E, Side* const (&sides)[2], SideSc
         a.meta[i] = metas + i * sc.cap_block;
     }
     const SideScratch& sc = scr[0];      // (sizes and parameters are the same)
-    hipLaunchKernelGGL(k_sched_count, dim3(sc.nwin, 2), dim3(sc.W), 0, st, a, N, sc.wave_row_max, skip_empty);
+    hipLaunchKernelGGL(k_sched_count, dim3(sc.nwin, 2), dim3(sc.W), 0, st, a, N, sc.wave_row_max, skip_empty, look);
     hipLaunchKernelGGL(k_sched_scan, dim3(1, 2), dim3(1024), 0, st, a, sc.nwin);
     hipLaunchKernelGGL(k_sched_fill, dim3(sc.nwin, 2), dim3(sc.W), 0, st, a, N, sc.wave_row_max, skip_empty, sc.cap_long);
     hipLaunchKernelGGL(k_cut_rows, dim3(1, 2), dim3(1024), 0, st, a, sc.cp);
@@ -581,9 +633,10 @@ static void schedule_counts(Side& side, const SideScratch& sc, const int32_t* re
 namespace {
 // Waves of n rows of a class (rows per wave are powers of two)
 struct WaveShift {
-    int sh[kNumClass];
+    int sh[8] = {};      // by kind
     explicit WaveShift(int lpe) {
-        for (int c = 0; c < kNumClass; ++c) { sh[c] = 0; while ((1 << sh[c]) < rows_per_wave(lpe, c)) ++sh[c]; }
+        for (int c = 0; c < 8; ++c)
+            while (desc_is_rows(c) && (1 << sh[c]) < rows_per_wave(lpe, c)) ++sh[c];
     }
     int32_t waves(int c, int64_t n) const { return (int32_t)((n + (1 << sh[c]) - 1) >> sh[c]); }
 };
@@ -593,6 +646,7 @@ struct XcdList {
     int32_t waves = 0;
     const WaveShift* ws = nullptr;
     uint32_t where = 0;      // the list's bits of a run's code
+    bool grouped = false;    // classes 1 to 3 go out together as kind 6
     void add(uint32_t code, int32_t first, int32_t n) {
         if (n <= 0) return;
         runs.push_back(Run{waves, first, n, code | where});
@@ -617,15 +671,21 @@ void append_side(XcdList& xl, const Side& s, int w, int w_items, bool src_side, 
     }
     if (w < 0) return;
     for (int c = (part == 0 ? 0 : 1); c < (part == 0 ? 1 : kNumClass); ++c) {
-        const uint32_t n = s.win_class_cnt[(size_t)w * (kNumClass + 1) + c];
-        xl.add(desc_code((uint32_t)c, src_side, 0), (int32_t)s.win_class_off[(size_t)w * (kNumClass + 1) + c], (int32_t)n);
+        uint32_t n = s.win_class_cnt[(size_t)w * (kNumClass + 1) + c], kind = (uint32_t)c;
+        if (xl.grouped && c >= 1 && c <= 3) {      // (the classes of a window lie behind each other)
+            if (c != 1) continue;
+            kind = kDescGroup;
+            n += s.win_class_cnt[(size_t)w * (kNumClass + 1) + 2] + s.win_class_cnt[(size_t)w * (kNumClass + 1) + 3];
+        }
+        xl.add(desc_code(kind, src_side, 0), (int32_t)s.win_class_off[(size_t)w * (kNumClass + 1) + c], (int32_t)n);
     }
 }
 
 // runs of all windows -> block order.  XCD x gets a contiguous range of windows; it first walks the
 // heavy share of all its windows (long work first keeps the end of the launch short), then window by window.
 // Appends one launch's runs to `all_runs`.
-void place(const std::vector<const Side*>& sides, int lpe, bool backward, int32_t* n_blocks, std::vector<Run>& all_runs) {
+void place(const std::vector<const Side*>& sides, int lpe, int list, int32_t* n_blocks, std::vector<Run>& all_runs) {
+    const bool grouped = list == LIST_BWD_GROUPED;
     const int nwin = sides[0]->n_windows;
     const bool heavy_first = env_int("TGT_HEAVY_FIRST", 1) == 1;
     const WaveShift shift(lpe);
@@ -640,7 +700,7 @@ void place(const std::vector<const Side*>& sides, int lpe, bool backward, int32_
                 const Side* sd = sides[k];
                 for (int32_t q = sd->homed_off[w]; q < sd->homed_off[w + 1]; ++q) c += 1.0 + sd->block_len[sd->homed_idx[q]] / 128.0;
                 for (int kk = 0; kk < kNumClass; ++kk)
-                    c += (kk == 0 ? 0.75 : 0.25) * shift.waves(kk, sd->win_class_cnt[(size_t)w * (kNumClass + 1) + kk]);
+                    c += (kk == 0 ? 0.75 : 0.25) * shift.waves(kk, sd->win_class_cnt[(size_t)w * (kNumClass + 1) + kk]);      // (of grouped rows, too)
             }
             cost[w + 1] = cost[w] + c;
         }
@@ -658,7 +718,8 @@ void place(const std::vector<const Side*>& sides, int lpe, bool backward, int32_
     for (int x = 0; x < 8; ++x) {
         XcdList& wv = xl[x];
         wv.ws = &shift;
-        wv.where = ((uint32_t)x << 8) | (backward ? kRunBackward : 0u);
+        wv.grouped = grouped;
+        wv.where = ((uint32_t)x << 8) | ((uint32_t)list << 11);
         wv.runs.reserve((size_t)(bound[x + 1] - bound[x] + 8) * 8 * sides.size());
         const int w0 = bound[x], w1 = bound[x + 1];
         if (heavy_first) {
@@ -680,7 +741,7 @@ void place(const std::vector<const Side*>& sides, int lpe, bool backward, int32_
                 if (!heavy_first) append_side(wv, *sides[k], w >= w0 ? w : -1, w >= w0 ? w : -1, k == 1, 0);
                 append_side(wv, *sides[k], w >= w0 ? w : -1, wi >= w0 ? wi : -1, k == 1, 1);
             }
-            wv.pad4();
+            if (!grouped) wv.pad4();
         }
     }
     int32_t per = 0;
@@ -692,18 +753,27 @@ void place(const std::vector<const Side*>& sides, int lpe, bool backward, int32_
     }
 }
 
-// The records of both launches.  `runs` feeds an asynchronous copy: it lives until the stream has been synchronised.
-int build_records(const tgt_plan* plan, int lpe, Schedule& sc, const std::vector<Run>& runs, DevBuf& runs_d, hipStream_t st) {
+// The records of the lists that `make` says.  `runs` feeds an asynchronous copy: it lives until the stream has been synchronised.
+int build_records(const tgt_plan* plan, int lpe, Schedule::List* const (&lists)[LIST_COUNT], const bool (&make)[LIST_COUNT], std::vector<Run>& runs,
+                  DevBuf& runs_d, hipStream_t st) {
+    for (int l = 0; l < LIST_COUNT; ++l) {
+        if (!make[l]) continue;
+        if (l == LIST_FWD) place({&plan->dst}, lpe, l, &lists[l]->blocks, runs);
+        else place({&plan->dst, &plan->src}, lpe, l, &lists[l]->blocks, runs);
+    }
     const WaveRecLayout L(lpe);
     const size_t rec = (size_t)L.stride * sizeof(int32_t) * 4;
     if (runs.empty()) return TGT_OK;
     TGT_HIP_CHECK(runs_d.alloc(sizeof(Run) * runs.size(), st));
     TGT_HIP_CHECK(hipMemcpyAsync(runs_d.p, runs.data(), sizeof(Run) * runs.size(), hipMemcpyHostToDevice, st));
-    if (sc.fwd_blocks) TGT_HIP_CHECK(dev_alloc(&sc.fwd, rec * sc.fwd_blocks, st));
-    if (sc.bwd_blocks) TGT_HIP_CHECK(dev_alloc(&sc.bwd, rec * sc.bwd_blocks, st));
+    RecordLists out{};
+    for (int l = 0; l < LIST_COUNT; ++l) {
+        if (make[l] && lists[l]->blocks) TGT_HIP_CHECK(dev_alloc(&lists[l]->recs, rec * lists[l]->blocks, st));
+        out.recs[l] = static_cast<int32_t*>(lists[l]->recs);
+    }
     const Side &d = plan->dst, &s = plan->src;
     hipLaunchKernelGGL(k_build_records, dim3((unsigned)runs.size()), dim3(64 * kRecordWaves), 0, st, runs_d.as<Run>(), d.items, s.items, d.block_items, s.block_items, d.col,
-                       d.eid, s.col, s.eid, L, lpe, static_cast<int32_t*>(sc.fwd), static_cast<int32_t*>(sc.bwd));
+                       d.eid, s.col, s.eid, L, lpe, out);
     TGT_HIP_CHECK(hipGetLastError());
     return TGT_OK;
 }
@@ -715,7 +785,7 @@ const Schedule* plan_schedule_if_ready(const tgt_plan* plan, int lpe) {
     return nullptr;
 }
 
-const Schedule* plan_schedule(const tgt_plan* plan_c, int lpe, hipStream_t st) {
+const Schedule* plan_schedule(const tgt_plan* plan_c, int lpe, hipStream_t st, int want) {
     int idx = 0;
     while (idx < kNumLpe && (1 << idx) != lpe) ++idx;
     if (idx == kNumLpe) { set_error("no schedule for %d lanes per edge", lpe); return nullptr; }
@@ -723,19 +793,30 @@ const Schedule* plan_schedule(const tgt_plan* plan_c, int lpe, hipStream_t st) {
     Schedule& sc = plan->sched[idx];
     // the descriptors of a shape are made once, whichever thread or stream asks first
     std::lock_guard<std::mutex> lock(plan->sched_mutex);
-    if (sc.ready) return &sc;
+    const bool grouped = plan->grouped && lpe >= kGroupMinLpe;
+    if (!grouped) want &= ~LISTS_BWD_GROUPED;
+    // a shape's first use makes the list that 2-byte calls without a bias take, unless the caller names another one
+    if (!sc.ready && !want) want = grouped ? LISTS_BWD_GROUPED : LISTS_BWD;
+    const bool make[LIST_COUNT] = {!sc.ready, (want & LISTS_BWD) && !sc.bwd.ready, (want & LISTS_BWD_GROUPED) && !sc.bwd_grouped.ready};
+    if (!make[LIST_FWD] && !make[LIST_BWD] && !make[LIST_BWD_GROUPED]) return &sc;
+    if (sc.ready) {
+        // The other list is there and says the same: a stream that is being captured, where nothing can be made, goes on with it.
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(st, &capturing) != hipSuccess) { set_error("hipStreamIsCapturing failed"); return nullptr; }
+        if (capturing != hipStreamCaptureStatusNone) return &sc;
+    }
     std::vector<Run> runs;
     DevBuf runs_d;
-    place({&plan->dst}, lpe, false, &sc.fwd_blocks, runs);
-    place({&plan->dst, &plan->src}, lpe, true, &sc.bwd_blocks, runs);
-    int rc = build_records(plan, lpe, sc, runs, runs_d, st);
+    Schedule::List* const lists[LIST_COUNT] = {&sc.fwd, &sc.bwd, &sc.bwd_grouped};
+    int rc = build_records(plan, lpe, lists, make, runs, runs_d, st);
     // the host vector feeds an asynchronous copy: it may go once the stream is idle
     if (hipStreamSynchronize(st) != hipSuccess && rc == TGT_OK) { set_error("hipStreamSynchronize failed"); rc = TGT_ERR_HIP; }
-    if (rc != TGT_OK) {
-        dev_free(sc.fwd); dev_free(sc.bwd);
-        sc = Schedule();
-        return nullptr;
+    for (int l = 0; l < LIST_COUNT; ++l) {
+        if (!make[l]) continue;
+        if (rc == TGT_OK) lists[l]->ready = true;
+        else { dev_free(lists[l]->recs); *lists[l] = Schedule::List(); }
     }
+    if (rc != TGT_OK) return nullptr;
     sc.ready = true;
     return &sc;
 }
@@ -779,7 +860,7 @@ static void free_side(Side& s) {
 
 static void free_schedules(tgt_plan* plan) {
     for (Schedule& sc : plan->sched) {
-        dev_free(sc.fwd); dev_free(sc.bwd);
+        for (Schedule::List* l : {&sc.fwd, &sc.bwd, &sc.bwd_grouped}) dev_free(l->recs);
         sc = Schedule();
     }
 }
@@ -806,7 +887,7 @@ static int create_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, in
     // what comes back to the host, in one copy: the two schedule headers, the range-check flag, per view the
     // per-window row counts and their offsets, and where the workgroup items go if there is room for few of them (else that
     // is a second copy, of the items there are)
-    const int W = window_rows();
+    const int W = window_rows(N);
     const int nwin = (int)((N + W - 1) / W);
     const size_t report_ints = kReportHead + 4 * (size_t)kSchedCats * nwin;
     const size_t cap_meta = (size_t)cap_block_items(N, E), meta_bytes = 2 * sizeof(BlockMeta) * cap_meta;
@@ -826,7 +907,7 @@ static int create_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, in
     SideScratch scr[2];
     Side* const views[2] = {&plan->dst, &plan->src};
     BlockMeta* const metas = reinterpret_cast<BlockMeta*>(report + report_ints);
-    rc = schedule_device(N, E, views, scr, report, metas, plan->rows_with_edges_only, st);
+    rc = schedule_device(N, E, views, scr, report, metas, plan->rows_with_edges_only, may_group(N, E) && !plan->rows_with_edges_only, W, st);
     if (rc) return rc;
     std::vector<int32_t> h_report(report_ints + (one_copy ? meta_bytes / 4 : 0));
     TGT_HIP_CHECK(hipMemcpyAsync(h_report.data(), report, sizeof(int32_t) * h_report.size(), hipMemcpyDeviceToHost, st));
@@ -837,6 +918,8 @@ static int create_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, in
     }
     schedule_counts(plan->dst, scr[0], h_report.data(), 0);
     schedule_counts(plan->src, scr[1], h_report.data(), 1);
+    const SchedHeader* hdr = reinterpret_cast<const SchedHeader*>(h_report.data());
+    plan->grouped = mostly_near(hdr[0]) && mostly_near(hdr[1]);
     // graphs with rows longer than a wave row: where their workgroup items go
     std::vector<BlockMeta> meta[2];
     for (int i = 0; i < 2; ++i) {
@@ -863,7 +946,7 @@ static int create_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, in
         for (size_t i = 0; i < m.size(); ++i) sd.homed_idx[at[sd.block_home[i]]++] = (int32_t)i;
     }
     // the shape of the reference's node-level models (hidden 64: 8 heads of 8, or 4 of 16); other shapes on first use
-    return plan_schedule(plan, 8, st) ? TGT_OK : TGT_ERR_HIP;
+    return plan_schedule(plan, 8, st, LISTS_ANY) ? TGT_OK : TGT_ERR_HIP;
 }
 
 // ---------------------------------------------------------------------------

@@ -604,11 +604,13 @@ __device__ __forceinline__ void walk_range(const Common& c, const SideArgs& s, c
     RowRegs<T> rr;
     // HASB == 2: no edge-id array, the bias rows are in this side's own sorted order (row = sorted position)
     constexpr bool ident = HASB == 2;
+    constexpr bool ONE_ROW = LPE * S == kWave;      // one row per wave: its numbers are scalars
     if constexpr (!piped_walk<T, MODE, TILES>()) {
         load_row<T, LPE, LPH, MODE>(c, row, el, valid, rr, acc);
-        const int32_t* __restrict__ col = s.col + start;
-        const int32_t* __restrict__ eid = ident ? nullptr : s.eid + start;
-        const int n = valid ? len : 0;
+        const int n = ONE_ROW ? __builtin_amdgcn_readfirstlane(valid ? len : 0) : (valid ? len : 0);
+        const int first = ONE_ROW ? __builtin_amdgcn_readfirstlane(start) : start;
+        const int32_t* __restrict__ col = s.col + first;
+        const int32_t* __restrict__ eid = ident ? nullptr : s.eid + first;
         const auto load_ids = [&](const int e0, int (&nb)[kUnroll], int (&ed)[kUnroll]) {
 #pragma unroll
             for (int u = 0; u < kUnroll; ++u) {
@@ -617,12 +619,12 @@ __device__ __forceinline__ void walk_range(const Common& c, const SideArgs& s, c
                     nb[u] = 0; ed[u] = 0;
                     if (e < n) {
                         nb[u] = col[e];
-                        if (HASB) ed[u] = ident ? start + e : eid[e];
+                        if (HASB) ed[u] = ident ? first + e : eid[e];
                     }
                 } else {      // past the end of the row: its last edge (a line the wave is reading anyway)
                     const int ec = min(e, n - 1);
                     nb[u] = col[ec];
-                    ed[u] = HASB ? (ident ? start + ec : eid[ec]) : 0;
+                    ed[u] = HASB ? (ident ? first + ec : eid[ec]) : 0;
                 }
             }
         };
@@ -662,7 +664,6 @@ __device__ __forceinline__ void walk_range(const Common& c, const SideArgs& s, c
         // edges each take 819 + 2292 us in bf16 when all neighbours are within 500 rows, 895 + 2490 us over 64 clusters.  Step by
         // step / as a queue, forward + backward: 870 K nodes in 64 clusters 3386 / 3288 us, 200 K nodes, 8 M edges 717 / 683 us, 262 K
         // nodes, 4.5 M edges, four heads of 16 438 / 419 us; rows of 5 edges have no second step: no difference.
-        constexpr bool ONE_ROW = LPE * S == kWave;      // one row per wave: its numbers are scalars
         const int n = ONE_ROW ? __builtin_amdgcn_readfirstlane(valid ? len : 0) : (valid ? len : 0);
         const int first = ONE_ROW ? __builtin_amdgcn_readfirstlane(start) : start;
         const int32_t* __restrict__ col = s.col + first;
@@ -723,6 +724,92 @@ __device__ __forceinline__ void walk_range(const Common& c, const SideArgs& s, c
             }
         });
     }
+}
+
+// Walks a row of kGroupRowMin edges or more with one lane group, four edges a step, as a queue of gathers like walk_range's: the sums
+// stay in the lanes that write the row, and a wave's prologue is shared by all its rows.  The four ids of a step are one load.
+// The last step starts kUnroll edges in front of the row's end, so that every position read is the row's own, and leaves out the edges
+// that the step before it has added.
+// Where walk_range keeps no queue neither does this: two edges at a time with a bias, which is what the registers allow (calls that
+// prefer the list without kind 6, and find it missing in a capture).
+template <typename T, int LPE, int LPH, int MODE, int HASB, bool TILES>
+__device__ __forceinline__ void walk_group(const Common& c, const SideArgs& s, const RecLane& rec, const int row, const int start,
+                                           const int len, const int el, const bool valid, Acc& acc) {
+    typedef int ids_t __attribute__((ext_vector_type(4), aligned(4)));
+    RowRegs<T> rr;
+    load_row<T, LPE, LPH, MODE>(c, row, el, valid, rr, acc);
+    if (!valid) return;
+    const int last = len - kUnroll;       // where the last step starts
+    with_offsets<T>(c.narrow, [&](auto zero) {
+        using O = decltype(zero);
+        const auto quad = [&](const int32_t* ids, const int from, int (&x)[kUnroll]) {
+            const ids_t v = *reinterpret_cast<const ids_t*>(reinterpret_cast<const char*>(ids) + (O)(uint32_t)(start + from) * 4);
+            x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
+        };
+        const auto bias_rows = [&](const int from, int (&ed)[kUnroll]) {
+            if (HASB == 1) quad(s.eid, from, ed);
+            else {
+#pragma unroll
+                for (int u = 0; u < kUnroll; ++u) ed[u] = HASB == 2 ? start + from + u : 0;
+            }
+        };
+        int nb[kUnroll], ed[kUnroll];
+        if constexpr (!piped_walk<T, MODE, TILES>()) {
+#pragma unroll 1
+            for (int base = 0; base < len; base += kUnroll) {
+                const int from = min(base, last);
+                quad(s.col, from, nb);
+                bias_rows(from, ed);
+                bool ok[kUnroll];
+#pragma unroll
+                for (int u = 0; u < kUnroll; ++u) ok[u] = from + u >= base;
+                if constexpr (HASB == 0) edge_step<T, LPE, LPH, MODE, HASB>(c, s, rr, nb, ed, ok, el, acc);
+                else {
+#pragma unroll 1
+                    for (int h = 0; h < 2; ++h) {
+                        Gathered<T> g[2];
+#pragma unroll
+                        for (int u = 0; u < 2; ++u) ask_edge<T, LPE, LPH, MODE, HASB, O>(c, h ? nb[u + 2] : nb[u], h ? ed[u + 2] : ed[u], el, g[u]);
+#pragma unroll
+                        for (int u = 0; u < 2; ++u)
+                            if (h ? ok[u + 2] : ok[u]) use_edge<T, LPE, LPH, MODE, HASB>(c, s, rr, g[u], h ? ed[u + 2] : ed[u], el, acc);
+                    }
+                }
+            }
+            return;
+        }
+        nb[0] = rec.cols.x; nb[1] = rec.cols.y; nb[2] = rec.cols.z; nb[3] = rec.cols.w;
+        if (std::is_same<O, uint64_t>::value) quad(s.col, 0, nb);      // (see walk_range)
+        if (HASB == 1 && !s.eid_is_map && !std::is_same<O, uint64_t>::value) {
+            ed[0] = rec.eids.x; ed[1] = rec.eids.y; ed[2] = rec.eids.z; ed[3] = rec.eids.w;
+        } else bias_rows(0, ed);
+        int nb2[kUnroll], ed2[kUnroll];
+        quad(s.col, min(kUnroll, last), nb2);
+        bias_rows(min(kUnroll, last), ed2);
+        Gathered<T> g[kUnroll];
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) ask_edge<T, LPE, LPH, MODE, HASB, O>(c, nb[u], ed[u], el, g[u]);
+        int base = 0;
+#pragma unroll 1
+        do {                              // every edge of this step exists, and another step follows: rows have more than kUnroll edges
+            int nb3[kUnroll], ed3[kUnroll];
+            quad(s.col, min(base + 2 * kUnroll, last), nb3);
+            bias_rows(min(base + 2 * kUnroll, last), ed3);
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u) {
+                use_edge<T, LPE, LPH, MODE, HASB>(c, s, rr, g[u], ed[u], el, acc);
+                __builtin_amdgcn_sched_barrier(0);
+                ask_edge<T, LPE, LPH, MODE, HASB, O>(c, nb2[u], ed2[u], el, g[u]);
+                ed[u] = ed2[u]; nb2[u] = nb3[u]; ed2[u] = ed3[u];
+            }
+            base += kUnroll;
+        } while (base < last);
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            arrive_here(g[u].g0); arrive_here(g[u].g1);      // (see edge_step)
+            if (last + u >= base) use_edge<T, LPE, LPH, MODE, HASB>(c, s, rr, g[u], ed[u], el, acc);
+        }
+    });
 }
 
 // The same for a row of at most S * kUnroll edges whose endpoints and bias rows come with the wave's
@@ -801,7 +888,8 @@ __device__ __forceinline__ void write_row(const Common& c, const SideArgs& s, co
 // Rows of one wave: 64 / (LPE*S) rows of one length class, named by the wave's record.  The longest
 // class walks the plan's sorted view step by step; the others find their (at most S * kUnroll) edges
 // in the record itself.
-template <typename T, int LPE, int LPH, int S, int MODE, int HASB, bool TILES, bool INLINE>
+// GROUP: rows that one lane group walks from beginning to end.
+template <typename T, int LPE, int LPH, int S, int MODE, int HASB, bool TILES, bool INLINE, bool GROUP = false>
 __device__ __forceinline__ void wave_rows(const Common& c, const SideArgs& s, const RecLane& rec) {
     constexpr int G = LPE * S;
     const int lane = threadIdx.x & (kWave - 1);
@@ -821,15 +909,20 @@ __device__ __forceinline__ void wave_rows(const Common& c, const SideArgs& s, co
     // pointers); nothing of it is loaded or stored
     if (TILES) valid = valid && !(len == 0 && s.cover[row] != 0);
     Acc acc;
-    if (INLINE) walk_record<T, LPE, LPH, S, MODE, HASB>(c, s, rec, row, start, len, slot, el, valid, acc);
+    if constexpr (GROUP) walk_group<T, LPE, LPH, MODE, HASB, TILES>(c, s, rec, row, start, len, el, valid, acc);
+    else if (INLINE) walk_record<T, LPE, LPH, S, MODE, HASB>(c, s, rec, row, start, len, slot, el, valid, acc);
     else walk_range<T, LPE, LPH, S, MODE, HASB, TILES, true>(c, s, rec, row, start, len, slot, el, valid, acc);
     finish_row<T, LPE, LPH, S, MODE, TILES>(c, s, row, slot, el, valid, acc);
 }
 
 template <typename T, int LPE, int LPH, int MODE, int HASB, bool TILES>
 __device__ __forceinline__ void wave_dispatch(const Common& c, const SideArgs& s, const RecLane& rec, const int kind) {
+    constexpr bool groups = MODE != MODE_FWD && LPE >= kGroupMinLpe;      // (only the backward's launch has kind 6)
     switch (kind) {
         case 0: wave_rows<T, LPE, LPH, slots_for_class(LPE, 0), MODE, HASB, TILES, false>(c, s, rec); break;
+        case (int)kDescGroup:
+            if constexpr (groups) wave_rows<T, LPE, LPH, 1, MODE, HASB, TILES, false, true>(c, s, rec);
+            break;
         case 1: wave_rows<T, LPE, LPH, slots_for_class(LPE, 1), MODE, HASB, TILES, class_inline(LPE, 1)>(c, s, rec); break;
         case 2: wave_rows<T, LPE, LPH, slots_for_class(LPE, 2), MODE, HASB, TILES, class_inline(LPE, 2)>(c, s, rec); break;
         case 3: wave_rows<T, LPE, LPH, slots_for_class(LPE, 3), MODE, HASB, TILES, class_inline(LPE, 3)>(c, s, rec); break;
@@ -1176,6 +1269,19 @@ static bool narrow_offsets(const Call& c) {
     return c.plan->N * row < (1ll << 32) && c.plan->E * edge < (1ll << 32);
 }
 
+// Whether the backward asks for the list in which rows of kGroupRowMin .. kGroupRowMax edges go out as kind 6 (plans whose neighbours are
+// near have it).  bf16: their walks are bound by vector issue, of which a wave of one to four short rows spends a third on its record, the sums over its slots
+// and its row.  k_attn_bwd, rows by classes / as kind 6: 262 K nodes, 5 M edges in 64 clusters, four heads of 16 267 / 229 us, 870 K nodes, 44 M edges
+// 2310 / 2130 us; 100 K nodes, 3.3 M edges in 64 clusters 144 / 124 us, 16 K nodes, 0.5 M edges 30.2 / 28.2; eight heads of 16, 150 K nodes, 3.5 M edges 323 / 267.  With a bias the walk waits for its
+// rows instead, unless there are many edges (eight heads of 8, bias per edge and head, 64 K nodes, 0.6 M edges 48.5 / 50.1, 1.5 M edges 111.7 / 116.2, 150 K nodes, 3.5 M
+// edges 312 / 296; of 16, 64 K nodes, 0.6 M edges 78.1 / 78.0, 1.5 M edges 170 / 157).  float32 waits for memory and keeps no queue: 64 K nodes, 0.6 M edges 53.7 / 61.0, with a
+// bias 150 K nodes, 3.5 M edges 507 / 520.  Beside dense tiles the rows are short.
+template <typename T, int LPE>
+static bool want_groups(const Call& c) {
+    if (sizeof(T) == 4 || LPE < kGroupMinLpe || c.init != nullptr) return false;
+    return c.bias_mode == TGT_BIAS_NONE || LPE > 8 || (c.plan->E >= 16 * c.plan->N && c.plan->E >= (2 << 20));
+}
+
 template <typename T, int LPE, int LPH>
 static int run_fwd(const Call& c) {
     const WsLayout L = ws_layout(c.plan, c.H, c.d);
@@ -1187,7 +1293,7 @@ static int run_fwd(const Call& c) {
     cm.inv_scale = 1.0f / sqrtf((float)c.d);
     SideArgs a{};
     fill_side(a, c.plan->dst);
-    const Schedule* sch = c.no_alloc ? plan_schedule_if_ready(c.plan, LPE) : plan_schedule(c.plan, LPE, c.st);
+    const Schedule* sch = c.no_alloc ? plan_schedule_if_ready(c.plan, LPE) : plan_schedule(c.plan, LPE, c.st, LISTS_ANY);
     if (!sch) {
         if (c.no_alloc) {
             set_error("no launch descriptors for H*d = %d yet: call tgt_plan_prepare(plan, H, d, stream) first", LPE * 8);
@@ -1195,13 +1301,13 @@ static int run_fwd(const Call& c) {
         }
         return TGT_ERR_HIP;
     }
-    const WaveRec<LPE>* desc = static_cast<const WaveRec<LPE>*>(sch->fwd);
+    const WaveRec<LPE>* desc = static_cast<const WaveRec<LPE>*>(sch->fwd.recs);
     if (c.bias_mode & TGT_BIAS_PLAN_ORDER) a.eid = nullptr;             // bias rows in destination-sorted order
     a.out0 = c.o_out; a.out1 = nullptr; a.Z = c.o_Z;
     if (c.init) { a.init0 = c.init->acc; a.initZ = c.init->Z; a.cover = c.init->cover_dst; }
     a.part = c.fwd_part ? c.fwd_part : reinterpret_cast<float*>(c.ws + L.fwd_part);
     a.counters = c.fwd_counters ? c.fwd_counters : reinterpret_cast<int32_t*>(c.ws + L.counters);
-    const int nb = sch->fwd_blocks;
+    const int nb = sch->fwd.blocks;
     if (nb > 0) {
         KernelTimer t(KS_FWD, c.st, !c.no_alloc);       // the entry point that allocates nothing creates no events either
         const bool hb = c.bias_mode != TGT_BIAS_NONE && c.plan->E > 0;       // (a graph without edges has no bias row that a lane could read)
@@ -1257,9 +1363,11 @@ static int run_bwd(const Call& c) {
     int32_t* counters = reinterpret_cast<int32_t*>(c.ws + L.counters);
     SideArgs sd{}, ss{};
     fill_side(sd, c.plan->dst);
-    const Schedule* sch = plan_schedule(c.plan, LPE, c.st);
+    const bool group = want_groups<T, LPE>(c);
+    const Schedule* sch = plan_schedule(c.plan, LPE, c.st, group ? LISTS_BWD_GROUPED : LISTS_BWD);
     if (!sch) return TGT_ERR_HIP;
-    const WaveRec<LPE>* desc = static_cast<const WaveRec<LPE>*>(sch->bwd);
+    const Schedule::List& list = (group ? sch->bwd_grouped : sch->bwd).ready ? (group ? sch->bwd_grouped : sch->bwd) : (group ? sch->bwd : sch->bwd_grouped);
+    const WaveRec<LPE>* desc = static_cast<const WaveRec<LPE>*>(list.recs);
     if (c.bias_mode & TGT_BIAS_PLAN_ORDER) sd.eid = nullptr;
     sd.out0 = c.dq; sd.out1 = c.dbias; sd.Z = nullptr;
     if (c.init) { sd.init0 = c.init->dq; sd.cover = c.init->cover_dst; }
@@ -1272,7 +1380,7 @@ static int run_bwd(const Call& c) {
     if (c.init) { ss.init0 = c.init->dk; ss.init1 = c.init->dv; ss.cover = c.init->cover_src; }
     ss.part = reinterpret_cast<float*>(c.ws + L.dkv_part);
     ss.counters = counters + 2 * (c.plan->dst.n_split + c.plan->dst.n_groups);
-    const int nb = sch->bwd_blocks;
+    const int nb = list.blocks;
     if (nb > 0) {
         KernelTimer t(KS_BWD, c.st);
         const bool hb = c.bias_mode != TGT_BIAS_NONE && c.plan->E > 0;       // (a graph without edges has no bias row that a lane could read)
@@ -1564,7 +1672,7 @@ int tgt_sparse_attn_fwd_noalloc(const tgt_plan_t* plan, const void* d_q, const v
 
 int tgt_plan_prepare(tgt_plan_t* plan, int H, int d, void* stream) {
     if (!plan || H < 1 || d < 1 || (H * d) % 8) { tgt::set_error("tgt_plan_prepare: null plan or H*d not a multiple of 8"); return TGT_ERR_INVALID_ARG; }
-    return tgt::plan_schedule(plan, H * d / 8, static_cast<hipStream_t>(stream)) ? TGT_OK : TGT_ERR_UNSUPPORTED;
+    return tgt::plan_schedule(plan, H * d / 8, static_cast<hipStream_t>(stream), tgt::LISTS_BWD | tgt::LISTS_BWD_GROUPED) ? TGT_OK : TGT_ERR_UNSUPPORTED;
 }
 
 int tgt_sparse_attn_bwd(const tgt_plan_t* plan, const void* d_q, const void* d_k, const void* d_v,
