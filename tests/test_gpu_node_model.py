@@ -213,6 +213,16 @@ def test_rows_beside_the_lines_between_variants(cuda, n, heads):
                 assert o <= (2e-2 if dtype == torch.bfloat16 else 1e-6 if name == "output" else (2 * n) ** -0.5), f"{name}: {o}"
 
 
+@pytest.mark.parametrize("n,heads", [(65536, 8), (65537, 4), (81920, 2), (81921, 8), (131072, 4), (131073, 8), (163841, 2)])
+def test_rows_beside_the_rounds_of_a_forward(cuda, n, heads):
+    """Sixteen or thirty-two rows per wave by the rounds they take: 65536, 81920 and 131072 rows each on 256 CUs"""
+    for dtype in (torch.float32, torch.bfloat16):
+        print(f"rows beside the rounds: n={n} heads={heads} {dtype}", flush=True)
+        model = scaled(Graphormer(1, heads, 32, 64, 5, 1, 0.0, 0.0, 0.0, 64, 1), n, dtype, cuda)
+        x = torch.randn(n - 1, 32, generator=torch.Generator().manual_seed(n)).to(cuda, dtype)      # (one more row: the global token)
+        compare(Graphormer, model, x, GraphPlan(random_edges(n - 1, 1, n + 2, cuda), n), n + 3)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n,heads", [(17, 2), (65, 4), (1000, 8), (16383, 8), (16385, 4), (32767, 2), (40000, 4), (65537, 2)])
 def test_gt_gradients_where_no_relu_changes_its_side(cuda, monkeypatch, dtype, n, heads):

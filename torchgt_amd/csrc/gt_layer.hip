@@ -8,8 +8,8 @@
 // s2, x', q, k, v out; backward: g, x, a (twice), s2 in, two rows out); y, u and relu(u) are recomputed in the backward (three
 // products), s2 is kept, which saves the two products behind them.  The 128 features between the feed-forward linears are two
 // tiles; the backward takes them one after the other, so that no more than one is alive, and keeps of u only its signs.
-// Measured at 65536 nodes (forward with q, k, v / backward, us): float32 50 / 79, bf16 15 / 36; a bf16 training step of four layers
-// 1030 us with the separate kernels behind one operator, 641 with these.
+// Measured at 65536 nodes (forward with q, k, v / backward, us): float32 38 / 79, bf16 15 / 32; a bf16 training step of four layers
+// 1030 us with the separate kernels behind one operator, 557 with these.
 // bf16 forward moves 68 MB in 15 us (4.5 TB/s); float32 is bound by its products (six MFMAs for one and the splitting into planes).
 #include "node_roles.h"
 
@@ -20,16 +20,16 @@ enum { V_BO = 0, V_GAMMA1, V_BETA1, V_B1A, V_B1B, V_B2, V_GAMMA2, V_BETA2, kVecs
 enum { W_O = 0, W_1A, W_1B, W_2A, W_2B };
 
 template <typename T, int R> __device__ __forceinline__ void round_to(TileOf<R>& t) { TGT_EACH(i) t.set(i, stored(t.get(i), (const T*)nullptr)); }
-// waves of a workgroup at most
-template <int R> constexpr int gt_fwd_waves() { return R == 32 ? 8 : 16; }
+// Rows per wave and waves of a workgroup at most.  Four launches of a model, us with sixteen rows / with thirty-two and eight waves: float32 4 K nodes 63 / 82,
+// 64 K 143 / 153, 300 K 606 / 650; bf16 4 K 38 / 46, 64 K 77 / 81, 300 K 216 / 225.
+constexpr int kFwdRows = 16, kFwdWaves = 16;
 // float32 takes its packed weights in turns (O and W1, W2, then q, k, v: 72 KB at most next to the row images), bf16 keeps all of them
 template <typename T> constexpr int gt_fwd_mats() { return sizeof(T) == 4 ? 3 : 8; }
-template <typename T, int R> constexpr int gt_fwd_lds(int waves) { return gt_fwd_mats<T>() * kFragVecs<Num<T>::P> * 16 + (kVecs8 + 3) * kVec * 4 + waves * RowShape<T, R>::kVecs * 16; }
+template <typename T> constexpr int gt_fwd_lds(int waves) { return gt_fwd_mats<T>() * kFragVecs<Num<T>::P> * 16 + (kVecs8 + 3) * kVec * 4 + waves * RowShape<T, kFwdRows>::kVecs * 16; }
 
-template <typename T, int R, bool NEXT> __global__ __launch_bounds__((gt_fwd_waves<R>() * 64)) void k_gt_fwd(const tgt_gt_fwd_args a) {
-    constexpr int P = Num<T>::P, FV = kFragVecs<P>;
-    constexpr bool CUT_AGAIN = P != 1 && R == 32;      // (no registers to keep a tile's planes)
-    const int threads = blockDim.x, kFwdWaves = threads >> 6;
+template <typename T, bool NEXT> __global__ __launch_bounds__(kFwdWaves * 64) void k_gt_fwd(const tgt_gt_fwd_args a) {
+    constexpr int P = Num<T>::P, FV = kFragVecs<P>, R = kFwdRows;
+    const int threads = blockDim.x, NW = threads >> 6;
     constexpr bool RESIDENT = sizeof(T) == 2;
     extern __shared__ __align__(16) unsigned char smem[];
     vec16* w = reinterpret_cast<vec16*>(smem);
@@ -39,27 +39,24 @@ template <typename T, int R, bool NEXT> __global__ __launch_bounds__((gt_fwd_wav
     vec16* stage = reinterpret_cast<vec16*>(vn + 3 * kVec) + wave * RowShape<T, R>::kVecs;
     const vec16 *gw = reinterpret_cast<const vec16*>(a.w), *gn = reinterpret_cast<const vec16*>(a.w_next);
     const int64_t N = a.rows, tiles = (N + R - 1) / R;
-    copy_params<kVecs8 * kVec>(threads, vec, a.vec);
-    if constexpr (NEXT) copy_params<3 * kVec>(threads, vn, a.v_next);
-    if (RESIDENT) {
-        copy_vecs_by<5 * FV>(threads, w, gw);
-        if constexpr (NEXT) copy_vecs_by<3 * FV>(threads, w + 5 * FV, gn);
-        __syncthreads();
-    }
     const vec16 *w2 = RESIDENT ? w + 3 * FV : w, *wn = RESIDENT ? w + 5 * FV : w;
-    for (int64_t t0 = (int64_t)blockIdx.x * kFwdWaves; t0 < tiles; t0 += (int64_t)gridDim.x * kFwdWaves) {
+    Raw<T, R> raw_x, raw_a;
+    const auto ask = [&](int64_t t0) {
+        const Rows rows(t0 + wave, N, R);      // (a wave without rows reads the first one)
+        fetch(raw_a, reinterpret_cast<const T*>(a.attn), rows, lane);
+        fetch(raw_x, reinterpret_cast<const T*>(a.x), rows, lane);
+    };
+    const int64_t first = (int64_t)blockIdx.x * NW;
+    ask(first);
+    copy_direct<(RESIDENT ? 5 : 3) * FV>(threads, w, gw);
+    if constexpr (RESIDENT && NEXT) copy_direct<3 * FV>(threads, w + 5 * FV, gn);
+    copy_direct<kVecs8 * kVec>(threads, vec, a.vec);
+    if constexpr (NEXT) copy_direct<3 * kVec>(threads, vn, a.v_next);
+    landed();
+    __syncthreads();
+    for (int64_t t0 = first;;) {
         const Rows rows(t0 + wave, N, R);
         const bool active = rows.left > 0;
-        Raw<T, R> raw_x, raw_a;
-        if (active) {
-            fetch(raw_a, reinterpret_cast<const T*>(a.attn), rows, lane);
-            fetch(raw_x, reinterpret_cast<const T*>(a.x), rows, lane);
-        }
-        if (!RESIDENT) {
-            __syncthreads();
-            copy_vecs_by<3 * FV>(threads, w, gw);
-            __syncthreads();
-        }
         TileOf<R> s, r[2];
         if (active) {
             TileOf<R> x, y;
@@ -73,16 +70,11 @@ template <typename T, int R, bool NEXT> __global__ __launch_bounds__((gt_fwd_wav
             round_to<T>(s);      // x1
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                if (CUT_AGAIN) forget(y);
                 linear<P, false>(r[j], y, w + (W_1A + j) * FV, vec + (V_B1A + j) * kVec, lane);
                 relu<T>(r[j]);
             }
         }
-        if (!RESIDENT) {
-            __syncthreads();
-            copy_vecs_by<2 * FV>(threads, w, gw + W_2A * FV);
-            __syncthreads();
-        }
+        if (!RESIDENT) replace_weights<2 * FV>(threads, w, gw + W_2A * FV);
         if (active) {
             TileOf<R> y;
             load_vec(y, vec + V_B2 * kVec, lane / R);
@@ -96,21 +88,20 @@ template <typename T, int R, bool NEXT> __global__ __launch_bounds__((gt_fwd_wav
             put_rows(reinterpret_cast<T*>(a.x_out), s, stage, rows, lane);
         }
         if constexpr (NEXT) {
-            if (!RESIDENT) {
-                __syncthreads();
-                copy_vecs_by<3 * FV>(threads, w, gn);
-                __syncthreads();
-            }
+            if (!RESIDENT) replace_weights<3 * FV>(threads, w, gn);
             if (active) {
 #pragma unroll
                 for (int j = 0; j < 3; ++j) {
                     TileOf<R> y;
-                    if (CUT_AGAIN) forget(s);
                     linear<P, false>(y, s, wn + j * FV, vn + j * kVec, lane);
                     put_rows(reinterpret_cast<T*>(j == 0 ? a.q : (j == 1 ? a.k : a.v)), y, stage, rows, lane);
                 }
             }
         }
+        t0 += (int64_t)gridDim.x * NW;
+        if (t0 >= tiles) break;
+        ask(t0);
+        if (!RESIDENT) replace_weights<3 * FV>(threads, w, gw);
     }
 }
 
@@ -252,12 +243,11 @@ template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN,
     write_partial<L, 2, 4>(a.partial_b + (int64_t)blockIdx.x * (2 * 4096 + 4 * 64), acc_b, col_b, buf, wave, lane);
 }
 
-template <typename T, int R, bool NEXT> int run_fwd(const tgt_gt_fwd_args& a, hipStream_t st) {
+template <typename T, bool NEXT> int run_fwd(const tgt_gt_fwd_args& a, hipStream_t st) {
     static std::atomic<uint64_t> done{0};
-    constexpr int most = gt_fwd_waves<R>();
-    const int waves = fwd_waves_for(a.rows, R, most);
-    if (int rc = allow_lds(reinterpret_cast<const void*>(&k_gt_fwd<T, R, NEXT>), gt_fwd_lds<T, R>(most), done)) return rc;
-    hipLaunchKernelGGL((k_gt_fwd<T, R, NEXT>), dim3(fwd_grid(a.rows, R, waves)), dim3(waves * 64), (gt_fwd_lds<T, R>(waves)), st, a);
+    const int waves = fwd_waves_for(a.rows, kFwdRows, kFwdWaves);
+    if (int rc = allow_lds(reinterpret_cast<const void*>(&k_gt_fwd<T, NEXT>), gt_fwd_lds<T>(kFwdWaves), done)) return rc;
+    hipLaunchKernelGGL((k_gt_fwd<T, NEXT>), dim3(fwd_grid(a.rows, kFwdRows, waves)), dim3(waves * 64), (gt_fwd_lds<T>(waves)), st, a);
     TGT_HIP_CHECK(hipGetLastError());
     return TGT_OK;
 }
@@ -280,11 +270,8 @@ int tgt_gt_fwd(const tgt_gt_fwd_args* a, void* stream) {
     if (a->rows == 0) return TGT_OK;
     const hipStream_t st = (hipStream_t)stream;
     KernelTimer t(KS_GT_FWD, st);
-    // rows per wave: 16 in float32 (us with 16 / 32: 4 K nodes 20.5 / 31.1, 64 K 42.7 / 47.1, 200 K 147 / 152), in bf16 while the CUs are
-    // less than three quarters full in one round (4 K 10.7 / 12.2, 37605 14.4 / 14.7, 64 K 17.0 / 16.1, 200 K 43.9 / 43.9)
-    if (a->dtype == TGT_DTYPE_F32) return a->q ? run_fwd<float, 16, true>(*a, st) : run_fwd<float, 16, false>(*a, st);
-    if (4 * a->rows <= 3 * one_round()) return a->q ? run_fwd<nbf16, 16, true>(*a, st) : run_fwd<nbf16, 16, false>(*a, st);
-    return a->q ? run_fwd<nbf16, 32, true>(*a, st) : run_fwd<nbf16, 32, false>(*a, st);
+    if (a->dtype == TGT_DTYPE_F32) return a->q ? run_fwd<float, true>(*a, st) : run_fwd<float, false>(*a, st);
+    return a->q ? run_fwd<nbf16, true>(*a, st) : run_fwd<nbf16, false>(*a, st);
 }
 
 int tgt_gt_bwd(const tgt_gt_bwd_args* a, void* stream) {

@@ -65,8 +65,8 @@ template <typename T, bool SAME, int R> __device__ __forceinline__ void gelu(Til
 // ---- forward ------------------------------------------------------------------------------------------------------------
 enum { NEXT_NONE = 0, NEXT_QKV = 1, NEXT_CLASSES = 2 };
 
-// waves of a workgroup at most
-template <typename T, int R, bool SAME> constexpr int fwd_waves() { return R == 32 && (sizeof(T) == 4 || SAME) ? 8 : 16; }
+// waves of a workgroup at most (float32 of 32 rows: as many as their row images leave room for)
+template <typename T, int R, bool SAME> constexpr int fwd_waves() { return R == 32 && SAME ? 8 : (R == 32 && sizeof(T) == 4 ? 10 : 16); }
 // bf16 keeps all weights of a launch in LDS for the life of the workgroup; float32 planes of six weights (144 KB) do not
 // leave room for the row images, so its two halves take turns (the L2 has them)
 template <typename T, bool POST, int NEXT> constexpr int fwd_resident_mats() {
@@ -92,27 +92,25 @@ __global__ __launch_bounds__((fwd_waves<T, R, SAME>() * 64)) void k_node_fwd(con
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane / R;
     vec16* stage = reinterpret_cast<vec16*>(vec + 10 * kVec) + wave * Shape::kVecs;
     const int64_t N = a.rows, tiles = (N + R - 1) / R;
-    if constexpr (POST) copy_params<5 * kVec>(threads, vec, a.v_post);
-    if constexpr (NEXT != NEXT_NONE) copy_params<(2 + NMP) * kVec>(threads, vn, a.v_next);
-    if (RESIDENT) {
-        if constexpr (POST) copy_vecs_by<3 * FV>(threads, w, reinterpret_cast<const vec16*>(a.w_post));
-        if constexpr (NEXT != NEXT_NONE) copy_vecs_by<NMP * FV>(threads, w_next, reinterpret_cast<const vec16*>(a.w_next));
-        __syncthreads();
-    }
-    for (int64_t t0 = (int64_t)blockIdx.x * NW; t0 < tiles; t0 += (int64_t)gridDim.x * NW) {
+    Raw<T, R> raw_a, raw_s;
+    const auto ask = [&](int64_t t0) {
+        const Rows rows(t0 + wave, N, R);      // (a wave without rows reads the first one)
+        fetch(raw_s, reinterpret_cast<const T*>(a.s_in), rows, lane);
+        if (POST) fetch(raw_a, reinterpret_cast<const T*>(a.attn), rows, lane);
+    };
+    const vec16 *w_post = reinterpret_cast<const vec16*>(a.w_post), *w_after = reinterpret_cast<const vec16*>(a.w_next);
+    const int64_t first = (int64_t)blockIdx.x * NW;
+    ask(first);
+    if constexpr (POST) copy_direct<3 * FV>(threads, w, w_post);
+    if constexpr (NEXT != NEXT_NONE && (RESIDENT || !POST)) copy_direct<NMP * FV>(threads, w_next, w_after);
+    if constexpr (POST) copy_direct<5 * kVec>(threads, vec, a.v_post);
+    if constexpr (NEXT != NEXT_NONE) copy_direct<(2 + NMP) * kVec>(threads, vn, a.v_next);
+    landed();
+    __syncthreads();
+    for (int64_t t0 = first;;) {
         const Rows rows(t0 + wave, N, R);
         const int64_t row0 = (t0 + wave) * R;
         const bool active = rows.left > 0;
-        Raw<T, R> raw_a, raw_s;
-        if (active) {
-            fetch(raw_s, reinterpret_cast<const T*>(a.s_in), rows, lane);
-            if (POST) fetch(raw_a, reinterpret_cast<const T*>(a.attn), rows, lane);
-        }
-        if (!RESIDENT && POST) {
-            __syncthreads();
-            copy_vecs_by<3 * FV>(threads, w, reinterpret_cast<const vec16*>(a.w_post));
-            __syncthreads();
-        }
         TileOf<R> s;
         if (active) {
             if (!POST && row0 < a.tokens) {      // the global tokens in front of the nodes: from their table, and into the stream
@@ -142,11 +140,8 @@ __global__ __launch_bounds__((fwd_waves<T, R, SAME>() * 64)) void k_node_fwd(con
                 put_rows(reinterpret_cast<T*>(a.s_out), s, stage, rows, lane);
             }
         }
-        if constexpr (!RESIDENT && NEXT != NEXT_NONE) {
-            __syncthreads();
-            copy_vecs_by<NMP * FV>(threads, w, reinterpret_cast<const vec16*>(a.w_next));
-            __syncthreads();
-        }
+        constexpr bool SWAP = !RESIDENT && POST && NEXT != NEXT_NONE;
+        if constexpr (SWAP) replace_weights<NMP * FV>(threads, w, w_after);
         if (NEXT && active) {
             normalise<SAME>(s, a.eps_next);
             affine(s, s, vn, vn + kVec, g);
@@ -168,6 +163,10 @@ __global__ __launch_bounds__((fwd_waves<T, R, SAME>() * 64)) void k_node_fwd(con
                 put_classes<T, false>(reinterpret_cast<T*>(a.logp), y, a.linear, a.classes, a.tokens, row0, N, stage, lane);
             }
         }
+        t0 += (int64_t)gridDim.x * NW;
+        if (t0 >= tiles) break;
+        ask(t0);
+        if constexpr (SWAP) replace_weights<3 * FV>(threads, w, w_post);
     }
 }
 
@@ -623,13 +622,15 @@ int tgt_node_fwd(const tgt_node_fwd_args* a, void* stream) {
     if (a->rows == 0) return TGT_OK;
     KernelTimer t(KS_NODE_FWD, (hipStream_t)stream);
     const hipStream_t st = (hipStream_t)stream;
-    // Sixteen rows per wave while that is one round (the chain of a wave is what the launch takes, and more CUs have one), thirty-two
-    // with more rows: us with 16 / 32, float32 4 K nodes 16.6 / 21.8, 37605 23.3 / 26.5, 64 K 31.4 / 30.7, 200 K 107 / 103; bf16
-    // 4 K 10.9 / 18.3, 37605 15.3 / 20.2, 64 K 18.3 / 18.9, 200 K 43.1 / 38.8.  In float32 the weights' way out of LDS is as long as the
-    // products with sixteen rows, so the line lies where the CUs are three quarters full.
-    if (a->dtype == TGT_DTYPE_F32) return 4 * a->rows <= 3 * one_round() ? dispatch_fwd<float, 16, false>(*a, st) : dispatch_fwd<float, 32, false>(*a, st);
+    // Sixteen rows per wave unless thirty-two save rounds: with a round's time next to its number of rows, sixteen rows a wave take float32
+    // 26 + 107 us a round of 64 K rows, thirty-two 25 + 149 us a round of 80 K; bf16 46 + 38 us and, of 128 K, 26 + 78 us.  Five launches of a
+    // model, us with 16 / 32: float32 4 K nodes 62 / 83, 37605 107 / 124, 64 K 133 / 143, 80 K 207 / 174, 100 K 212 / 275, 150 K 328 / 317, 200 K 440 / 461,
+    // 300 K 567 / 621; bf16 4 K 42 / 54, 37605 77 / 89, 64 K 84 / 90, 80 K 118 / 99, 100 K 119 / 114, 150 K 158 / 184, 200 K 194 / 188, 300 K 239 / 262.
+    const auto rounds = [&](int per_cu) { return groups_of(a->rows, per_cu * num_cus()); };
+    if (a->dtype == TGT_DTYPE_F32)
+        return 7 * rounds(32 * fwd_waves<float, 32, false>()) < 5 * rounds(256) ? dispatch_fwd<float, 32, false>(*a, st) : dispatch_fwd<float, 16, false>(*a, st);
     if (a->same_bits) return dispatch_fwd<nbf16, 32, true>(*a, st);
-    return a->rows <= one_round() ? dispatch_fwd<nbf16, 16, false>(*a, st) : dispatch_fwd<nbf16, 32, false>(*a, st);
+    return 2 * rounds(512) <= rounds(256) ? dispatch_fwd<nbf16, 32, false>(*a, st) : dispatch_fwd<nbf16, 16, false>(*a, st);
 }
 
 int tgt_node_bwd_workers(int64_t rows) { return rows < 0 ? -1 : tgt::bwd_workers(rows); }

@@ -24,34 +24,28 @@ template <int N, int THREADS> __device__ __forceinline__ void copy_vecs(vec16* d
     }
 }
 
-// The same for a workgroup of any number of whole waves; N is a number of whole waves' accesses
-template <int K> __device__ __forceinline__ void copy_batch(int threads, vec16* dst, const vec16* __restrict__ src) {
-    vec16 v[K];
-#pragma unroll
-    for (int i = 0; i < K; ++i) v[i] = src[i * threads];
-#pragma unroll
-    for (int i = 0; i < K; ++i) dst[i * threads] = v[i];
+// N 16-byte vectors from global memory straight to LDS, without registers, by a workgroup of any number of whole waves: everything that a kernel begins with
+// is asked for before the first wait.  `landed` waits for what this wave has asked for (its rows, too); the others' follows behind a barrier.
+// With loads to registers and writes to LDS one after the other for vectors and weights, and the rows behind them, a launch began with three
+// or four memory round trips in a row: 37605 nodes in float32 had their first rows settled after 18 800 of 46 700 cycles of k_node_fwd, now after 8700 of
+// 34 900.  Four and five launches of a model, us before / after: float32 4 K nodes 71 / 62, 37605 115 / 107 (GT 125 / 109); bf16 46 / 42, 81 / 77 (GT 72 / 69).
+template <int N> __device__ __forceinline__ void copy_direct(int threads, vec16* dst, const vec16* __restrict__ src) {
+    const int wave0 = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63), lane = threadIdx.x & 63;
+    for (int at = wave0; at < N; at += threads)
+        if (N % 64 == 0 || at + lane < N)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + at + lane), (__attribute__((address_space(3))) void*)(dst + at), 16, 0, 0);
 }
-template <int N> __device__ __forceinline__ void copy_vecs_by(int threads, vec16* dst, const vec16* __restrict__ src) {
-    static_assert(N % 64 == 0, "whole waves");
-    const int wave0 = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63);
-    int k = wave0 < N ? (N - wave0 + threads - 1) / threads : 0, at = threadIdx.x;      // accesses of this wave
-    for (; k > 8; k -= 8, at += 8 * threads) copy_batch<8>(threads, dst + at, src + at);
-    switch (k) {      // the rest in one round trip
-        case 1: copy_batch<1>(threads, dst + at, src + at); break;
-        case 2: copy_batch<2>(threads, dst + at, src + at); break;
-        case 3: copy_batch<3>(threads, dst + at, src + at); break;
-        case 4: copy_batch<4>(threads, dst + at, src + at); break;
-        case 5: copy_batch<5>(threads, dst + at, src + at); break;
-        case 6: copy_batch<6>(threads, dst + at, src + at); break;
-        case 7: copy_batch<7>(threads, dst + at, src + at); break;
-        case 8: copy_batch<8>(threads, dst + at, src + at); break;
-        default: break;
-    }
+template <int N> __device__ __forceinline__ void copy_direct(int threads, float* dst, const float* __restrict__ src) {      // N floats
+    copy_direct<N / 4>(threads, reinterpret_cast<vec16*>(dst), reinterpret_cast<const vec16*>(src));
 }
-// a few parameter vectors
-template <int N> __device__ __forceinline__ void copy_params(int threads, float* dst, const float* __restrict__ src) {
-    for (int at = threadIdx.x; at < N / 4; at += threads) reinterpret_cast<vec16*>(dst)[at] = reinterpret_cast<const vec16*>(src)[at];
+__device__ __forceinline__ void landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// Weights in the place of others that everybody has used, seen by everybody
+template <int N> __device__ __forceinline__ void replace_weights(int threads, vec16* dst, const vec16* __restrict__ src) {
+    __syncthreads();
+    copy_direct<N>(threads, dst, src);
+    landed();
+    __syncthreads();
 }
 
 // A packed weight on its way from memory to LDS through the registers of the four block waves
@@ -158,8 +152,6 @@ int64_t groups_of(int64_t rows, int per) { return std::max<int64_t>(1, (rows + p
 // LDS: with fewer waves the copies are more traffic than the rows)
 int fwd_waves_for(int64_t rows, int per, int most) { return (int)std::min<int64_t>(most, std::max<int64_t>(4, (groups_of(rows, per) + num_cus() - 1) / num_cus())); }
 int fwd_grid(int64_t rows, int per, int waves) { return (int)std::min<int64_t>(num_cus(), groups_of(rows, per * waves)); }
-// Rows that sixteen waves of 16 (or eight of 32) on every CU take in one round
-int64_t one_round(void) { return (int64_t)256 * num_cus(); }
 
 // Backward: nodes of a workgroup's group.  64 while there is a CU for every group of 64 (the chain of a workgroup is what such a launch
 // takes), 128 with more: the products of a group run while its chain goes on, and a barrier costs the same for 64 nodes and for 128.

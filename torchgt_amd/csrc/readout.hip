@@ -101,13 +101,15 @@ template <typename T> __global__ __launch_bounds__(kWaves * 64) void k_readout_f
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     vec16* stage = reinterpret_cast<vec16*>(vec + kMats * kVec) + wave * RowShape<T, R>::kVecs;
     const int64_t N = a.rows, tiles = (N + R - 1) / R;
-    copy_params<kMats * kVec>(threads, vec, a.v);
-    copy_vecs_by<kMats * FV>(threads, w, reinterpret_cast<const vec16*>(a.w));
+    Raw<T, R> raw;
+    const int64_t first = (int64_t)blockIdx.x * NW + wave;
+    fetch(raw, reinterpret_cast<const T*>(a.x), Rows(first, N, R), lane);
+    copy_direct<kMats * FV>(threads, w, reinterpret_cast<const vec16*>(a.w));
+    copy_direct<kMats * kVec>(threads, vec, a.v);
+    landed();
     __syncthreads();
-    for (int64_t t0 = (int64_t)blockIdx.x * NW + wave; t0 < tiles; t0 += (int64_t)gridDim.x * NW) {
+    for (int64_t t0 = first; t0 < tiles;) {
         const Rows rows(t0, N, R);
-        Raw<T, R> raw;
-        fetch(raw, reinterpret_cast<const T*>(a.x), rows, lane);
         TileOf<R> y;
         Frags<P, R> x;
         settle<T, false>(y, raw, stage, rows, lane);
@@ -123,6 +125,8 @@ template <typename T> __global__ __launch_bounds__(kWaves * 64) void k_readout_f
         product<P>(y, x, w + 2 * FV, vec + 2 * kVec, lane);
         if constexpr (P == 3) mend<P, false>(y, x, w + 2 * FV, vec + 2 * kVec, a.out, a.m2, stage, rows, lane);
         put_classes<T, P == 3>(reinterpret_cast<T*>(a.logp), y, false, a.classes, 0, t0 * R, N, stage, lane);
+        t0 += (int64_t)gridDim.x * NW;
+        if (t0 < tiles) fetch(raw, reinterpret_cast<const T*>(a.x), Rows(t0, N, R), lane);
     }
 }
 
