@@ -8,7 +8,7 @@
 // s2, x', q, k, v out; backward: g, x, a (twice), s2 in, two rows out); y, u and relu(u) are recomputed in the backward (three
 // products), s2 is kept, which saves the two products behind them.  The 128 features between the feed-forward linears are two
 // tiles; the backward takes them one after the other, so that no more than one is alive, and keeps of u only its signs.
-// Measured at 65536 nodes (forward with q, k, v / backward, us): float32 38 / 79, bf16 15 / 32; a bf16 training step of four layers
+// Measured at 65536 nodes (forward with q, k, v / backward, us): float32 38 / 79, bf16 15 / 29.5; a bf16 training step of four layers
 // 1030 us with the separate kernels behind one operator, 557 with these.
 // bf16 forward moves 68 MB in 15 us (4.5 TB/s); float32 is bound by its products (six MFMAs for one and the splitting into planes).
 #include "node_roles.h"
@@ -118,8 +118,6 @@ template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN,
     float* vec = reinterpret_cast<float*>(smem + L::kVecs);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane % R, h = lane / R;
     const int64_t N = a.rows, groups = (N + CN - 1) / CN;
-    copy_vecs<kVecs8 * kVec / 4, L::kThreads>(reinterpret_cast<vec16*>(vec), reinterpret_cast<const vec16*>(a.vec));
-    __syncthreads();
     float16_t acc_a[3], acc_b[2];      // O, W1a, W1b; W2a, W2b
     float col_a[5], col_b[4];          // bo, b1a, b1b, gamma1, beta1; b2, -, gamma2, beta2
 #pragma unroll
@@ -135,23 +133,35 @@ template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN,
     if (wave < NC) {
         vec16* stage = reinterpret_cast<vec16*>(smem + L::kStage) + wave * RowShape<T, R>::kVecs;
         const int row = R * wave + n;
+        // bf16 has the registers to ask for a group's rows in the group before it; float32 asks for the attention rows there, for the
+        // others one after the other (64 K nodes in bf16: 32.0 us with every row asked for where it is needed, 29.5)
+        constexpr bool AHEAD = P == 1;
+        Raw<T, R> raw, raw_s2, raw_g, raw_x;
+        const auto ask = [&](Raw<T, R>& r, const void* from, int64_t g) { fetch(r, reinterpret_cast<const T*>(from), Rows(NC * g + wave, N, R), lane); };
+        ask(raw, a.attn, blockIdx.x);
+        if (AHEAD) {
+            ask(raw_s2, a.s2, blockIdx.x);
+            ask(raw_g, a.g_in, blockIdx.x);
+            ask(raw_x, a.x, blockIdx.x);
+        }
         for (int64_t g0 = blockIdx.x; g0 < groups; g0 += gridDim.x) {
             const Rows rows(NC * g0 + wave, N, R);
-            Raw<T, R> raw;
+            const int64_t after = g0 + gridDim.x < groups ? g0 + gridDim.x : g0;
             TileOf<R> y, ds2, dy, t;
-            fetch(raw, reinterpret_cast<const T*>(a.attn), rows, lane);
             settle<T, false>(t, raw, stage, rows, lane);
-            fetch(raw, reinterpret_cast<const T*>(a.s2), rows, lane);
+            if (!AHEAD) ask(raw, a.s2, g0);
             __syncthreads();                                        // O
             linear<P, false>(y, t, w, vec + V_BO * kVec, lane);
             round_to<T>(y);
             __syncthreads();
             {
                 TileOf<R> g;
-                settle<T, false>(t, raw, stage, rows, lane);
-                fetch(raw, reinterpret_cast<const T*>(a.g_in), rows, lane);
+                settle<T, false>(t, AHEAD ? raw_s2 : raw, stage, rows, lane);
+                if (AHEAD) ask(raw_s2, a.s2, after);
+                else ask(raw, a.g_in, g0);
                 const float rstd = normalise<false>(t, a.eps2);
-                settle<T, true>(g, raw, stage, rows, lane);
+                settle<T, true>(g, AHEAD ? raw_g : raw, stage, rows, lane);
+                if (AHEAD) ask(raw_g, a.g_in, after);
                 col_b[3] += column_sums(g, lane);
                 zero(ds2);
                 ln_back(ds2, g, t, rstd, vec + V_GAMMA2 * kVec, h);
@@ -187,9 +197,10 @@ template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN,
                 gemm<P>(dy, f, w, lane);
                 __syncthreads();
             }
-            fetch(raw, reinterpret_cast<const T*>(a.x), rows, lane);
-            settle<T, false>(t, raw, stage, rows, lane);
-            fetch(raw, reinterpret_cast<const T*>(a.attn), rows, lane);
+            if (!AHEAD) ask(raw, a.x, g0);
+            settle<T, false>(t, AHEAD ? raw_x : raw, stage, rows, lane);
+            if (AHEAD) ask(raw_x, a.x, after);
+            else ask(raw, a.attn, g0);
             TGT_EACH(i) t.set(i, t.get(i) + y.get(i));              // s1
             const MeanRstd stat = row_stats<false>(t, a.eps1);
             TGT_EACH(i) t.set(i, (stored(t.get(i), (const T*)nullptr) - stat.mean) * stat.rstd);
@@ -203,6 +214,7 @@ template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN,
             TGT_EACH(i) dy.set(i, stored(stored(dy.get(i), (const T*)nullptr) + y.get(i), (const T*)nullptr));
             col_a[0] += column_sums(dy, lane);
             settle<T, false>(t, raw, stage, rows, lane);
+            ask(raw, a.attn, after);
             Frags<P, R> f;
             put_tile_planes<PB, P>(p_x, row, h, t);
             make_frags(f, dy);
@@ -219,6 +231,8 @@ template <typename T, int R, int CN> __global__ __launch_bounds__((Bwd<T, R, CN,
         const vec16 *fw = reinterpret_cast<const vec16*>(a.w), *bw = reinterpret_cast<const vec16*>(a.w_back);
         WeightsAhead<FV> next;
         next.fetch(fw + W_O * FV);
+        copy_direct<kVecs8 * kVec>(kBlockWaves * 64, vec, a.vec, NC * 64);
+        landed();
         for (int64_t g0 = blockIdx.x; g0 < groups; g0 += gridDim.x) {
             next.hand_over(w, fw + W_1A * FV);          // O
             __syncthreads();

@@ -26,17 +26,18 @@ template <int N, int THREADS> __device__ __forceinline__ void copy_vecs(vec16* d
 
 // N 16-byte vectors from global memory straight to LDS, without registers, by a workgroup of any number of whole waves: everything that a kernel begins with
 // is asked for before the first wait.  `landed` waits for what this wave has asked for (its rows, too); the others' follows behind a barrier.
+// from: the first thread that takes part, of `threads`.
 // With loads to registers and writes to LDS one after the other for vectors and weights, and the rows behind them, a launch began with three
 // or four memory round trips in a row: 37605 nodes in float32 had their first rows settled after 18 800 of 46 700 cycles of k_node_fwd, now after 8700 of
 // 34 900.  Four and five launches of a model, us before / after: float32 4 K nodes 71 / 62, 37605 115 / 107 (GT 125 / 109); bf16 46 / 42, 81 / 77 (GT 72 / 69).
-template <int N> __device__ __forceinline__ void copy_direct(int threads, vec16* dst, const vec16* __restrict__ src) {
-    const int wave0 = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63), lane = threadIdx.x & 63;
+template <int N> __device__ __forceinline__ void copy_direct(int threads, vec16* dst, const vec16* __restrict__ src, int from = 0) {
+    const int wave0 = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63) - from, lane = threadIdx.x & 63;
     for (int at = wave0; at < N; at += threads)
         if (N % 64 == 0 || at + lane < N)
             __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + at + lane), (__attribute__((address_space(3))) void*)(dst + at), 16, 0, 0);
 }
-template <int N> __device__ __forceinline__ void copy_direct(int threads, float* dst, const float* __restrict__ src) {      // N floats
-    copy_direct<N / 4>(threads, reinterpret_cast<vec16*>(dst), reinterpret_cast<const vec16*>(src));
+template <int N> __device__ __forceinline__ void copy_direct(int threads, float* dst, const float* __restrict__ src, int from = 0) {      // N floats
+    copy_direct<N / 4>(threads, reinterpret_cast<vec16*>(dst), reinterpret_cast<const vec16*>(src), from);
 }
 __device__ __forceinline__ void landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
