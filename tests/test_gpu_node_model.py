@@ -289,3 +289,56 @@ def test_both_sides_of_an_attention_in_one_launch(cuda, dtype, n, classes, layer
     model = scaled(Graphormer(layers, 8, 40, 64, classes, 1, 0.0, 0.0, 0.0, 64, 1), n, dtype, cuda)
     x = torch.randn(n, 40, generator=torch.Generator().manual_seed(n)).to(cuda, dtype)
     compare(Graphormer, model, x, GraphPlan(random_edges(n, 1, n + 2, cuda), n + 1), n + 3)
+
+
+class NodeBwdPreArgs(ctypes.Structure):      # tgt_node_bwd_pre_args
+    _fields_ = [("rows", ctypes.c_int64)] + [(k, ctypes.c_int32) for k in ("dtype", "tokens", "classes", "linear")] + [("eps", ctypes.c_float)] + \
+        [(k, ctypes.c_void_p) for k in ("dq", "dk", "dv", "g_in", "s", "dlogp", "logp", "w_back", "v_next", "g_out", "d_token", "partial")]
+
+
+class NodeBwdPostArgs(ctypes.Structure):      # tgt_node_bwd_post_args
+    _fields_ = [("rows", ctypes.c_int64)] + [(k, ctypes.c_int32) for k in ("dtype", "heads", "same_bits")] + [("eps", ctypes.c_float)] + \
+        [(k, ctypes.c_void_p) for k in ("g_in", "s", "attn", "w_post", "w_back", "v_post", "Z", "g_out", "d_attn", "nd", "partial")]
+
+
+@pytest.mark.parametrize("n", [32768, 32769, 33024, 49151, 49152, 49153, 131073, 147456, 147457])
+def test_backward_of_many_rows_is_that_of_its_parts(cuda, n):
+    """bf16 in groups of 192 nodes (32769 to 49152 and 131073 to 147456 rows on 256 CUs) and beside them: every row as in calls of at most 8000 rows (groups of 64), bit
+    for bit, and the partial sums add up to theirs.  Bar of the sums: their float32 rounding, some 2^-24 of a sum's terms; a row that is lost, or counted
+    twice, is 1 / sqrt(n) of a sum or more."""
+    print(f"backward in parts: n={n}", flush=True)
+    L, g, st = _lib.lib(), torch.Generator(device=cuda).manual_seed(n), torch.cuda.current_stream(cuda).cuda_stream
+    rand = lambda *s: torch.randn(s, generator=g, device=cuda)
+    weights, values, vecs = [(rand(64, 64) / 8).bfloat16() for _ in range(3)], (rand(5, 64) / 4).bfloat16(), torch.empty(5, 64, device=cuda)
+    frags = torch.empty(L.tgt_node_frag_bytes(3, _lib.DTYPE_BF16), dtype=torch.uint8, device=cuda)
+    back = frags.data_ptr() + frags.numel() // 2
+    mats, ld = (ctypes.c_void_p * 3)(*[w.data_ptr() for w in weights]), (ctypes.c_int * 3)(64, 64, 64)
+    of_vecs, lens = (ctypes.c_void_p * 5)(*[values[i].data_ptr() for i in range(5)]), (ctypes.c_int * 5)(*[64] * 5)
+    _lib.check(L.tgt_node_pack(ctypes.addressof(mats), ctypes.addressof(ld), ctypes.addressof(ld), 3, ctypes.addressof(of_vecs), ctypes.addressof(lens), 5, _lib.DTYPE_BF16,
+                               frags.data_ptr(), vecs.data_ptr(), st))
+    rows = {k: rand(n, 64).bfloat16() for k in ("dq", "dk", "dv", "g_in", "s", "attn")}
+    Z = rand(n, 8).abs() + 1
+
+    def run(lo, hi):
+        at = {k: t[lo:hi].data_ptr() for k, t in rows.items()}
+        workers = L.tgt_node_bwd_workers(hi - lo)
+        out = {k: torch.empty(hi - lo, 64, dtype=torch.bfloat16, device=cuda) for k in ("pre", "post", "da", "parts", "da_parts")}
+        nd, sums = torch.empty(hi - lo, 8, 2, device=cuda), [torch.full((workers, 3 * 4096 + 5 * 64), float("nan"), device=cuda) for _ in range(3)]
+        pre = NodeBwdPreArgs(rows=hi - lo, dtype=_lib.DTYPE_BF16, eps=1e-5, dq=at["dq"], dk=at["dk"], dv=at["dv"], g_in=at["g_in"], s=at["s"], w_back=back, v_next=vecs.data_ptr(),
+                             g_out=out["pre"].data_ptr(), partial=sums[0].data_ptr())
+        _lib.check(L.tgt_node_bwd_pre(ctypes.addressof(pre), st))
+        for same, g_out, da, s in ((1, "post", "da", sums[1]), (0, "parts", "da_parts", sums[2])):
+            post = NodeBwdPostArgs(rows=hi - lo, dtype=_lib.DTYPE_BF16, heads=8, same_bits=same, eps=1e-5, g_in=at["g_in"], s=at["s"], attn=at["attn"], w_post=frags.data_ptr(),
+                                   w_back=back, v_post=vecs.data_ptr(), Z=Z[lo:hi].data_ptr(), g_out=out[g_out].data_ptr(), d_attn=out[da].data_ptr(), nd=nd.data_ptr(),
+                                   partial=s.data_ptr())
+            _lib.check(L.tgt_node_bwd_post(ctypes.addressof(post), st))
+        return [*out.values(), nd], [s.double().sum(0) for s in sums]
+
+    whole, sums = run(0, n)
+    parts = [run(lo, min(lo + 8000, n)) for lo in range(0, n, 8000)]
+    for i, t in enumerate(whole):
+        assert torch.equal(t, torch.cat([p[0][i] for p in parts])), i
+    for i, t in enumerate(sums):
+        want = sum(p[1][i] for p in parts)
+        for a, b in zip(t.split([4096] * 3 + [64] * 5), want.split([4096] * 3 + [64] * 5)):
+            assert float((a - b).norm()) <= 1e-5 * float(b.norm())

@@ -185,13 +185,21 @@ template <typename T, int R, int CN> struct Chain {
     __device__ __forceinline__ Rows rows(int64_t group, int64_t N) const { return Rows(tile(group), N, R); }
 };
 // and a block wave
-template <int P, int PB> struct Blocks {
-    static constexpr int FV = kFragVecs<P>;
+// (of BW; with two of them a wave has the two blocks of its columns)
+template <int P, int PB, int BW = kBlockWaves> struct Blocks {
+    static constexpr int FV = kFragVecs<P>, EACH = 4 / BW;
     vec16* w;
     unsigned char *p_dy, *p_x;
-    int base_dy, base_x;
-    WeightsAhead<FV> next;
-    __device__ __forceinline__ void add(float16_t& acc) const { node_product<P, PB>(acc, p_dy, p_x, base_dy, base_x); }
+    int base_dy[EACH], base_x;
+    WeightsAhead<FV, BW * 64> next;
+    __device__ __forceinline__ Blocks(vec16* w_, unsigned char* planes, int q, int lane) : w(w_), p_dy(planes), p_x(planes + P * PB), base_x(operand_base(q & 1, lane)) {
+#pragma unroll
+        for (int i = 0; i < EACH; ++i) base_dy[i] = operand_base((q + i * BW) >> 1, lane);
+    }
+    __device__ __forceinline__ void add(float16_t* acc) const {
+#pragma unroll
+        for (int i = 0; i < EACH; ++i) node_product<P, PB>(acc[i], p_dy, p_x, base_dy[i], base_x);
+    }
 };
 
 // One group: d = g_in + what the products and LayerNorm make of dq, dk, dv (or of the classes' gradients).  raw_s and raw_d come with s and
@@ -259,7 +267,7 @@ template <int NM, int P, int PB> __device__ __forceinline__ void pre_blocks(Bloc
             me.next.fetch(j + 2 < NM ? weights + (j + 2) * FV : after);
             __syncthreads();                   // weight j + 1
         }
-        me.add(acc[j]);
+        me.add(acc + j);
         if (j + 1 < NM) __syncthreads();       // product j is done
     }
 }
@@ -276,15 +284,15 @@ template <int N> __device__ __forceinline__ void clear(float (&col)[N]) {
 }
 
 // What the kernels begin with, and the block waves' part of it
-#define TGT_BWD_ROLES()                                                                                                          \
-    using L = Bwd<T, R, CN, NV>;                                                                                                 \
+#define TGT_BWD_ROLES(...)                                                                                                       \
+    using L = Bwd<T, R, CN, NV, ##__VA_ARGS__>;                                                                                                 \
     constexpr int P = Num<T>::P, PB = L::kPlane, NC = L::kChain;                                                                 \
     extern __shared__ __align__(16) unsigned char smem[];                                                                        \
     vec16* w = reinterpret_cast<vec16*>(smem + L::kW);                                                                           \
     float* vec = reinterpret_cast<float*>(smem + L::kVecs);                                                                      \
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);                                 \
     const Chain<T, R, CN> chain{reinterpret_cast<vec16*>(smem + L::kStage) + wave * RowShape<T, R>::kVecs, w, vec, smem, smem + P * PB, lane, wave}
-#define TGT_BWD_BLOCKS() Blocks<P, PB> blocks{w, smem, smem + P * PB, operand_base((wave - NC) >> 1, lane), operand_base((wave - NC) & 1, lane)}
+#define TGT_BWD_BLOCKS() Blocks<P, PB, L::kBlocks> blocks(w, smem, wave - NC, lane)
 
 template <typename T, int R, int CN, bool CLASSES, bool NORM>
 __global__ __launch_bounds__((Bwd<T, R, CN>::kThreads)) void k_node_bwd_pre(const tgt_node_bwd_pre_args a) {
@@ -398,31 +406,32 @@ __device__ __forceinline__ void post_chain(const tgt_node_bwd_post_args& a, cons
     if (a.nd) put_node_side<T>(g, t, a.Z, a.nd, a.heads, rows.first + lane % R, h, lane % R < rows.left);
     if (P != 1) then();
 }
-template <int P, int PB> __device__ __forceinline__ void post_blocks(Blocks<P, PB>& me, const vec16* fw, const vec16* bw, const vec16* after, float16_t (&acc)[3]) {
-    constexpr int FV = kFragVecs<P>;
+template <int P, int PB, int BW> __device__ __forceinline__ void post_blocks(Blocks<P, PB, BW>& me, const vec16* fw, const vec16* bw, const vec16* after, float16_t (&acc)[3 * (4 / BW)]) {
+    constexpr int FV = kFragVecs<P>, EACH = 4 / BW;
     me.next.hand_over(me.w, fw + FV);             // Wo, then on to W1
     __syncthreads();
     me.next.hand_over(me.w, bw + 2 * FV);         // W1
     __syncthreads();
     me.next.hand_over(me.w, bw + FV);             // W2^T and the planes of W2
-    me.add(acc[2]);
+    me.add(acc + 2 * EACH);
     __syncthreads();
     me.next.hand_over(me.w, bw);                  // W1^T and the planes of W1
-    me.add(acc[1]);
+    me.add(acc + 1 * EACH);
     __syncthreads();
     me.next.hand_over(me.w, after);               // Wo^T and the planes of Wo
-    me.add(acc[0]);
+    me.add(acc);
     __syncthreads();
 }
 
+template <typename T, int R, int CN> constexpr int post_block_waves() { return CN / R + kBlockWaves <= 8 || R == 16 ? kBlockWaves : 2; }
 template <typename T, int R, int CN, bool SAME>
-__global__ __launch_bounds__((Bwd<T, R, CN>::kThreads)) void k_node_bwd_post(const tgt_node_bwd_post_args a) {
-    constexpr int NV = 5;
-    TGT_BWD_ROLES();
+__global__ __launch_bounds__((Bwd<T, R, CN, 5, post_block_waves<T, R, CN>()>::kThreads)) void k_node_bwd_post(const tgt_node_bwd_post_args a) {
+    constexpr int NV = 5, BW = post_block_waves<T, R, CN>();
+    TGT_BWD_ROLES(BW);
     const int64_t N = a.rows, groups = (N + CN - 1) / CN;
     copy_vecs<5 * kVec / 4, L::kThreads>(reinterpret_cast<vec16*>(vec), reinterpret_cast<const vec16*>(a.v_post));
     __syncthreads();
-    float16_t acc[3];       // Wo, W1, W2
+    float16_t acc[3 * (4 / BW)];       // Wo, W1, W2
     float col[5];           // bo, b1, b2, gamma, beta
     clear(acc); clear(col);
     if (wave < NC) {
@@ -569,7 +578,7 @@ template <typename T, int R, int CN> int dispatch_bwd_pre(const tgt_node_bwd_pre
     return a.v_next ? launch_bwd_pre<T, R, CN, false, true>(a, st) : launch_bwd_pre<T, R, CN, false, false>(a, st);
 }
 template <typename T, int R, int CN, bool SAME> int launch_bwd_post(const tgt_node_bwd_post_args& a, hipStream_t st) {
-    using L = Bwd<T, R, CN>;
+    using L = Bwd<T, R, CN, 5, post_block_waves<T, R, CN>()>;
     static std::atomic<uint64_t> done{0};
     return launch(&k_node_bwd_post<T, R, CN, SAME>, done, bwd_workers(a.rows), L::kThreads, L::kBytes, st, a);
 }
@@ -657,6 +666,7 @@ int tgt_node_bwd_pre(const tgt_node_bwd_pre_args* a, void* stream) {
     KernelTimer t(KS_NODE_BWD_PRE, (hipStream_t)stream);
     const hipStream_t st = (hipStream_t)stream;
     if (a->dtype == TGT_DTYPE_F32) return groups_of_64(a->rows, true) ? dispatch_bwd_pre<float, 16, 64>(*a, st) : dispatch_bwd_pre<float, 16, 128>(*a, st);
+    if (groups_of_192(a->rows)) return dispatch_bwd_pre<nbf16, 16, 192>(*a, st);
     return groups_of_64(a->rows, false) ? dispatch_bwd_pre<nbf16, 16, 64>(*a, st) : dispatch_bwd_pre<nbf16, 16, 128>(*a, st);
 }
 
@@ -668,6 +678,7 @@ int tgt_node_bwd_post(const tgt_node_bwd_post_args* a, void* stream) {
     const hipStream_t st = (hipStream_t)stream;
     if (a->dtype == TGT_DTYPE_F32) return groups_of_64(a->rows, true) ? launch_bwd_post<float, 16, 64, false>(*a, st) : launch_bwd_post<float, 16, 128, false>(*a, st);
     const bool small = groups_of_64(a->rows, false);
+    if (a->same_bits && groups_of_192(a->rows)) return launch_bwd_post<nbf16, 32, 192, true>(*a, st);
     if (a->same_bits) return small ? launch_bwd_post<nbf16, 32, 64, true>(*a, st) : launch_bwd_post<nbf16, 32, 128, true>(*a, st);
     return small ? launch_bwd_post<nbf16, 16, 64, false>(*a, st) : launch_bwd_post<nbf16, 16, 128, false>(*a, st);
 }

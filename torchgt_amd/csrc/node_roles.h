@@ -49,17 +49,17 @@ template <int N> __device__ __forceinline__ void replace_weights(int threads, ve
     __syncthreads();
 }
 
-// A packed weight on its way from memory to LDS through the registers of the four block waves
-template <int N> struct WeightsAhead {
-    static_assert(N % 256 == 0, "whole vectors per thread");
-    vec16 v[N / 256];
+// A packed weight on its way from memory to LDS through the registers of the block waves (T threads, the last of the workgroup)
+template <int N, int T = 256> struct WeightsAhead {
+    static_assert(N % T == 0 && (T & (T - 1)) == 0, "whole vectors per thread");
+    vec16 v[N / T];
     __device__ __forceinline__ void fetch(const vec16* __restrict__ src) {
 #pragma unroll
-        for (int i = 0; i < N / 256; ++i) v[i] = src[(threadIdx.x & 255) + i * 256];
+        for (int i = 0; i < N / T; ++i) v[i] = src[(threadIdx.x & (T - 1)) + i * T];
     }
     __device__ __forceinline__ void put(vec16* dst) const {
 #pragma unroll
-        for (int i = 0; i < N / 256; ++i) dst[(threadIdx.x & 255) + i * 256] = v[i];
+        for (int i = 0; i < N / T; ++i) dst[(threadIdx.x & (T - 1)) + i * T] = v[i];
     }
     // the weight at hand to LDS, the next one asked for, and the barrier that says so
     __device__ __forceinline__ void hand_over(vec16* dst, const vec16* __restrict__ src) {
@@ -76,10 +76,12 @@ template <int N> struct WeightsAhead {
 // and hand the chain its packed weights one at a time.  So the matrix work of one role runs beside the vector work of the
 // other, and neither has to hold the other's registers (with all waves in both roles, 16 KB of accumulators per wave next to
 // the tiles spilled: 106 us for k_node_bwd_post and 55 us for k_node_bwd_pre at 64 K nodes in float32).
+// With six chain waves of 32 rows there are two block waves of two blocks each: eight waves have 256 registers, nine 168, and
+// the chain of k_node_bwd_post would put 161 of them to scratch.
 constexpr int kBlockWaves = 4;
 
-template <typename T, int R_, int CN_, int NV = 5> struct Bwd {      // NV: parameter vectors
-    static constexpr int R = R_, CN = CN_, P = Num<T>::P, kChain = CN / R, kThreads = (kChain + kBlockWaves) * 64, kPlane = CN * 128;
+template <typename T, int R_, int CN_, int NV = 5, int BW = kBlockWaves> struct Bwd {      // NV: parameter vectors, BW: block waves
+    static constexpr int R = R_, CN = CN_, P = Num<T>::P, kChain = CN / R, kBlocks = BW, kThreads = (kChain + BW) * 64, kPlane = CN * 128;
     static constexpr int kW = 2 * P * kPlane, kStage = kW + kFragVecs<P> * 16, kVecs = kStage + kChain * RowShape<T, R>::kVecs * 16;
     static constexpr int kBytes = kVecs + NV * kVec * 4;
     static_assert(kChain * 5 * 64 * 4 <= kW, "the column sums of the chain waves meet where the planes were");
@@ -87,17 +89,20 @@ template <typename T, int R_, int CN_, int NV = 5> struct Bwd {      // NV: para
 
 // The workgroup's sums to its partial: NM 64 x 64 blocks (registers of the block waves), then NV vectors of 64 (a register
 // of each chain wave; added through LDS).
-template <typename L, int NM, int NV> __device__ __forceinline__ void write_partial(float* __restrict__ mine, const float16_t (&acc)[NM], const float (&col)[NV], float* buf, int wave, int lane) {
+template <typename L, int NM, int NV> __device__ __forceinline__ void write_partial(float* __restrict__ mine, const float16_t (&acc)[NM * (4 / L::kBlocks)], const float (&col)[NV], float* buf, int wave, int lane) {
+    constexpr int EACH = 4 / L::kBlocks;
     __syncthreads();
     if (wave < L::kChain) {
 #pragma unroll
         for (int c = 0; c < NV; ++c) buf[(wave * NV + c) * 64 + lane] = col[c];
     } else {
-        const int q = wave - L::kChain, h = lane >> 5;
+        const int h = lane >> 5;
 #pragma unroll
-        for (int j = 0; j < NM; ++j)
+        for (int j = 0; j < NM * EACH; ++j) {
+            const int q = wave - L::kChain + j % EACH * L::kBlocks;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) mine[j * 4096 + (32 * (q >> 1) + 8 * (r >> 2) + 4 * h + (r & 3)) * 64 + 32 * (q & 1) + (lane & 31)] = acc[j][r];
+            for (int r = 0; r < 16; ++r) mine[j / EACH * 4096 + (32 * (q >> 1) + 8 * (r >> 2) + 4 * h + (r & 3)) * 64 + 32 * (q & 1) + (lane & 31)] = acc[j][r];
+        }
     }
     __syncthreads();
     for (int i = threadIdx.x; i < NV * 64; i += L::kThreads) {
@@ -167,6 +172,15 @@ bool groups_of_64(int64_t rows, bool f32) {
     if (!f32 || rows < 128 * cus) return false;
     const int64_t r64 = (groups_of(rows, 64) + cus - 1) / cus, r128 = (groups_of(rows, 128) + cus - 1) / cus;
     return 4 * r64 <= 7 * r128;
+}
+
+// bf16: 192 nodes where that saves more than a third of the rounds (a round of 192 takes 1.4 times one of 128; from 32769 to 49152 rows
+// there is one instead of two).  128 / 192, us: k_node_bwd_pre 33 K rows 14.3 / 11.5, 48000 15.5 / 14.1, 64000 (two rounds of either) 16.0 / 19.3, 300 K
+// 54.2 / 53.1; k_node_bwd_post of 33 K rows (same_bits) 27.5 / 22.5; k_readout_bwd 48000 26.3 / 20.8.  Not k_node_bwd_both and k_gt_bwd, which put 66 to 133 registers of sixteen waves to scratch (48000: 33.2 / 45.5,
+// 28.0 / 35.0).
+bool groups_of_192(int64_t rows) {
+    const int64_t cus = num_cus();
+    return 3 * ((groups_of(rows, 192) + cus - 1) / cus) < 2 * ((groups_of(rows, 128) + cus - 1) / cus);
 }
 
 template <typename... Args> int launch(void (*kernel)(Args...), std::atomic<uint64_t>& done, int grid, int threads, int lds, hipStream_t st, Args... args) {

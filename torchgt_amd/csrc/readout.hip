@@ -376,6 +376,7 @@ int tgt_readout_bwd(const tgt_readout_bwd_args* a, void* stream) {
     // Nodes of a workgroup's group: float32 has registers for the chain with eight waves only (128 nodes put 75 to scratch: 16385 rows 29.9 us with 64
     // and 33.0, 64000 53 and 66, 500000 356 and 496); bfloat16 as elsewhere (16384 rows 15.9 and 16.2, 16385 21.7 and 16.4, 64000 36 and 26).
     if (a->dtype == TGT_DTYPE_F32) return run_bwd<float, 16, 64>(*a, st);
+    if (groups_of_192(a->rows)) return run_bwd<nbf16, 16, 192>(*a, st);
     return groups_of_64(a->rows, false) ? run_bwd<nbf16, 16, 64>(*a, st) : run_bwd<nbf16, 16, 128>(*a, st);
 }
 
