@@ -357,6 +357,8 @@ int tgt_reformat_create(const int64_t* d_src, const int64_t* d_dst, int64_t E, i
                         void* stream, tgt_reformat_t** out);
 int64_t tgt_reformat_num_edges(const tgt_reformat_t* r);
 int tgt_reformat_export(const tgt_reformat_t* r, int64_t* d_edge_index, int64_t* d_sorted_indices, void* stream);
+/* The edges alone. */
+int tgt_reformat_export_edges(const tgt_reformat_t* r, int64_t* d_edge_index, void* stream);
 int tgt_reformat_destroy(tgt_reformat_t* r);
 /* The rows of a batch in its new order (gt_sp/utils.py:463-472): d_rows[j] = d_idx_batch[old id - tokens] over the new ids,
  * without the global node (old id 0) when tokens is 1; int64 [N - tokens]. */

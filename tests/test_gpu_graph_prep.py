@@ -90,6 +90,29 @@ def test_reformat_hand_computed_compact_counts_and_raw_branch(cuda):
     np.testing.assert_array_equal(got_s.cpu().numpy(), np.arange(7))
 
 
+# Tiles of 1024 nodes, edges and emitted edges that end inside, at and behind one, and of 4096 (more than eight of 1024 per CU); parts of one digit
+# of the sort and of two, pairs of parts that fit the LDS counts (64 x 64) and not; blocks of one edge, and of more than a tile
+@pytest.mark.parametrize("N,E,k,bs", [(1023, 1023, 1, 32), (1024, 1024, 1, 32), (1025, 1025, 1, 33), (1, 3, 1, 1), (40, 0, 2, 16), (1030, 5000, 64, 3), (1030, 5000, 65, 3),
+                                      (2048, 4097, 256, 2), (2049, 4095, 257, 1), (3000, 2500, 3, 7), (2100000, 2200000, 3, 16)])
+def test_reformat_at_the_edges_of_its_tiles(cuda, N, E, k, bs):
+    rng = np.random.default_rng(N + k)
+    part = np.concatenate([np.arange(k), rng.integers(0, k, N - k)])      # (no part is empty)
+    rng.shuffle(part)
+    _check_reformat(rng.integers(0, N, (2, E)), part, k, bs, True, cuda)
+
+
+@pytest.mark.parametrize("blockize", [True, False])
+@pytest.mark.parametrize("where,value", [(0, -1), (1023, 2000), (1024, 1 << 40), (2499, -(1 << 40))])
+def test_reformat_refuses_an_endpoint_out_of_range(cuda, blockize, where, value):
+    rng = np.random.default_rng(where)
+    for end in (0, 1):
+        ei = rng.integers(0, 2000, (2, 2500))
+        ei[end, where] = value
+        with pytest.raises(_lib.TorchGTHipError) as exc:
+            graph_prep.reformat_graph(torch.from_numpy(ei).to(cuda), 4, 16, partition_ids=torch.arange(2000) % 4, blockize=blockize)
+        assert exc.value.code == _lib.ERR_INDEX_RANGE
+
+
 def test_relabel_and_sort_without_blockize(cuda):
     rng = np.random.default_rng(3)
     N, k = 70000, 8

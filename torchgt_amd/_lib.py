@@ -71,6 +71,7 @@ SIGNATURES = {
     "tgt_reformat_create": (_i32, [_vp, _vp, _i64, _i64, _vp, _i32, _i32, _i32, _vp, _c.POINTER(_vp)]),
     "tgt_reformat_num_edges": (_i64, [_vp]),
     "tgt_reformat_export": (_i32, [_vp, _vp, _vp, _vp]),
+    "tgt_reformat_export_edges": (_i32, [_vp, _vp, _vp]),
     "tgt_reformat_destroy": (_i32, [_vp]),
     "tgt_reformat_rows": (_i32, [_vp, _vp, _i32, _vp, _vp]),
     "tgt_sub_edge_index_packed": (_i32, [_vp, _i64, _i64, _vp, _i64, _vp, _i64, _c.POINTER(_i64), _vp]),

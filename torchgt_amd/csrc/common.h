@@ -183,11 +183,17 @@ public:
     // The results live in the sorter's buffers until the next sort() call; copy a
     // result before passing it as input of another sort().
     int sort(const uint32_t* const* keys_in, const uint32_t* const* vals_in, int sorts, int64_t n, int bits, hipStream_t st,
-             const uint32_t** keys_out, const uint32_t** vals_out);
+             const uint32_t** keys_out, const uint32_t** vals_out, bool counted = false);
     int sort(const uint32_t* keys_in, const uint32_t* vals_in, int64_t n, int bits, hipStream_t st, const uint32_t** keys_out,
-             const uint32_t** vals_out) {
-        return sort(&keys_in, vals_in ? &vals_in : nullptr, 1, n, bits, st, keys_out, vals_out);
+             const uint32_t** vals_out, bool counted = false) {
+        return sort(&keys_in, vals_in ? &vals_in : nullptr, 1, n, bits, st, keys_out, vals_out, counted);
     }
+    // Where the kernel that makes the keys puts their first digits' counts (`counted`: it has), tile by tile: workgroup b of `blocks` has the
+    // keys [256 items b, 256 items (b + 1)) and leaves the number of those with digit d in hist[sort][d * blocks + b].
+    struct Counts { uint32_t* hist[2]; int blocks, items; };
+    Counts counts(int64_t n, int sorts) const;
+    static constexpr int kThreads = 256;
+    static constexpr int kFewItems = 4, kManyItems = 16;      // the values of `items`
 private:
     DevBuf buf_;
     int64_t cap_ = 0;

@@ -73,13 +73,51 @@ __global__ void k_fix_edge_index(const int64_t* __restrict__ in, int64_t E0, int
     out[Eo + i] = d;
 }
 
-__global__ void k_check_partition(const int64_t* __restrict__ part, int64_t N, int k, uint32_t* __restrict__ p32,
-                                  unsigned long long* __restrict__ flag) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    int64_t p = part[i];
-    if (p < 0 || p >= k) { flag[0] = 1; p = 0; }
-    p32[i] = (uint32_t)p;
+// The lanes of a wave with the same key (key_bits of it matter) among those that take part
+__device__ __forceinline__ uint64_t lanes_with(uint32_t key, int key_bits, bool in) {
+    uint64_t same = __ballot(in);
+    for (int b = 0; b < key_bits; ++b) {
+        const bool bit = (key >> b) & 1u;
+        const uint64_t bal = __ballot(bit);
+        same &= bit ? bal : ~bal;
+    }
+    return same;
+}
+__device__ __forceinline__ uint64_t lower_lanes() { const int lane = threadIdx.x & 63; return lane == 0 ? 0ull : (~0ull >> (64 - lane)); }
+
+// Range check and 32-bit ids of the parts, the counts of their first digits that the sort by part begins with (RadixSorter::Counts) and, as long
+// as an id is one digit, the nodes of each part (cnt, cleared by the caller; more parts: k_count).  Neighbouring nodes are often in one part:
+// equal digits of a wave are merged first.
+template <int ITEMS>
+__global__ __launch_bounds__(RadixSorter::kThreads) void k_check_partition(const int64_t* __restrict__ part, int64_t N, int k, uint32_t* __restrict__ p32,
+                                                                           unsigned long long* __restrict__ flag, unsigned long long* __restrict__ cnt,
+                                                                           const RadixSorter::Counts c) {
+    constexpr int T = RadixSorter::kThreads;
+    __shared__ uint32_t h[256];
+    const int tid = threadIdx.x;
+    h[tid] = 0;
+    __syncthreads();
+    const int64_t base = (int64_t)blockIdx.x * T * ITEMS + tid;
+    for (int j = 0; j < ITEMS; j += 4) {
+        int64_t p[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) p[u] = part[min(base + (j + u) * T, N - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t i = base + (j + u) * T;
+            const bool in = i < N;
+            if (p[u] < 0 || p[u] >= k) {
+                if (in) flag[0] = 1;
+                p[u] = 0;
+            }
+            if (in) p32[i] = (uint32_t)p[u];
+            const uint64_t same = lanes_with((uint32_t)p[u], 8, in);
+            if (in && (same & lower_lanes()) == 0) atomicAdd(&h[p[u] & 255], (uint32_t)__popcll(same));
+        }
+    }
+    __syncthreads();
+    c.hist[0][(int64_t)tid * c.blocks + blockIdx.x] = h[tid];
+    if (k <= 256 && h[tid]) atomicAdd(&cnt[tid], (unsigned long long)h[tid]);
 }
 
 // mapping[old] = new position; sorted[new] = old (as int64 for the caller)
@@ -95,34 +133,29 @@ __global__ void k_invert(const uint32_t* __restrict__ sorted_old, int64_t N, uin
 // Histogram of keys in [0, nbins).  The bins are few (k or k*k partition pairs) and neighbouring
 // keys are often equal, so equal keys of a wave are first merged with ballots (one LDS add per
 // distinct key and wave), workgroups count in LDS, and only non-empty bins reach global memory.
-// Integer counts: the order of the additions does not matter.
+// Integer counts: the order of the additions does not matter.  keys(i, key, valid): of i, i + blockDim.x, ... (four).
 constexpr int kCountLdsBins = 4096;
-__global__ __launch_bounds__(256) void k_count(const uint32_t* __restrict__ keys, int64_t n, int nbins, int key_bits,
-                                               unsigned long long* __restrict__ cnt) {
+template <typename F> __device__ __forceinline__ void count_keys(const F& keys, int64_t n, int nbins, int key_bits, unsigned long long* __restrict__ cnt) {
     __shared__ uint32_t h[kCountLdsBins];
     const bool lds = nbins <= kCountLdsBins;
     if (lds) {
         for (int b = threadIdx.x; b < nbins; b += blockDim.x) h[b] = 0;
         __syncthreads();
     }
-    const int lane = threadIdx.x & 63;
-    const uint64_t lower = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    const int64_t rounds = (n + stride - 1) / stride;          // the same for every thread: ballots need whole waves
+    const int64_t step = 4ll * gridDim.x * blockDim.x;
+    const int64_t rounds = (n + step - 1) / step;          // the same for every thread: ballots need whole waves
     for (int64_t t = 0; t < rounds; ++t) {
-        const int64_t i = t * stride + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-        const bool valid = i < n;
-        const uint32_t key = valid ? keys[i] : 0u;
-        uint64_t same = __ballot(valid);
-        for (int b = 0; b < key_bits; ++b) {
-            const bool bit = (key >> b) & 1u;
-            const uint64_t bal = __ballot(bit);
-            same &= bit ? bal : ~bal;
-        }
-        if (valid && (same & lower) == 0) {                    // lowest lane of its group of equal keys
-            const uint32_t c = (uint32_t)__popcll(same);
-            if (lds) atomicAdd(&h[key], c);
-            else atomicAdd(&cnt[key], (unsigned long long)c);
+        uint32_t key[4];
+        bool valid[4];
+        keys(t * step + 4ll * blockIdx.x * blockDim.x + threadIdx.x, key, valid);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const uint64_t same = lanes_with(key[u], key_bits, valid[u]);
+            if (valid[u] && (same & lower_lanes()) == 0) {                    // lowest lane of its group of equal keys
+                const uint32_t c = (uint32_t)__popcll(same);
+                if (lds) atomicAdd(&h[key[u]], c);
+                else atomicAdd(&cnt[key[u]], (unsigned long long)c);
+            }
         }
     }
     if (lds) {
@@ -130,6 +163,36 @@ __global__ __launch_bounds__(256) void k_count(const uint32_t* __restrict__ keys
         for (int b = threadIdx.x; b < nbins; b += blockDim.x)
             if (h[b]) atomicAdd(&cnt[b], (unsigned long long)h[b]);
     }
+}
+
+__global__ __launch_bounds__(256) void k_count(const uint32_t* __restrict__ keys, int64_t n, int nbins, int key_bits, unsigned long long* __restrict__ cnt) {
+    count_keys([&](int64_t i, uint32_t (&key)[4], bool (&valid)[4]) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t at = i + (int64_t)u * blockDim.x;
+            valid[u] = at < n;
+            key[u] = keys[min(at, n - 1)];
+        }
+    }, n, nbins, key_bits, cnt);
+}
+// Edges of every pair of parts (part[src] * k + part[dst]) and the range check of the endpoints (flagged, and taken as node 0).  The keys
+// themselves (k_edge_keys) are written where edges are kept only: 0.39 M edges, 8 parts, the two passes 18 us with the gap between them.
+__global__ __launch_bounds__(256) void k_count_pairs(const int64_t* __restrict__ src, const int64_t* __restrict__ dst, int64_t E, int64_t N, const uint32_t* __restrict__ p32,
+                                                     int k, int key_bits, unsigned long long* __restrict__ cnt, unsigned long long* __restrict__ flag) {
+    count_keys([&](int64_t i, uint32_t (&key)[4], bool (&valid)[4]) {
+        int64_t s[4], d[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t at = i + (int64_t)u * blockDim.x;
+            valid[u] = at < E;
+            s[u] = src[min(at, E - 1)]; d[u] = dst[min(at, E - 1)];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if ((s[u] < 0) | (s[u] >= N) | (d[u] < 0) | (d[u] >= N)) { flag[0] = 1; s[u] = 0; d[u] = 0; }
+            key[u] = p32[s[u]] * (uint32_t)k + p32[d[u]];
+        }
+    }, E, k * k, key_bits, cnt);
 }
 
 // per-edge keys: pair = part[src]*k + part[dst], s32 = src, d32 = dst; an endpoint outside [0, N) is flagged and taken as node 0
@@ -177,6 +240,31 @@ __global__ void k_emit_blocks(const Block* __restrict__ blocks, int bs, uint32_t
     }
 }
 
+// The same where nothing but blocks is emitted (block b begins at b bs bs), in the tiles of the sort by new source, with the counts of its
+// first digits (RadixSorter::Counts)
+template <int ITEMS>
+__global__ __launch_bounds__(RadixSorter::kThreads) void k_emit_all_blocks(const Block* __restrict__ blocks, int bs, int64_t n, uint32_t* __restrict__ ns, uint32_t* __restrict__ nd,
+                                                                           const RadixSorter::Counts c) {
+    constexpr int T = RadixSorter::kThreads;
+    __shared__ uint32_t h[256];
+    const int tid = threadIdx.x;
+    h[tid] = 0;
+    __syncthreads();
+    const uint32_t per = (uint32_t)bs * (uint32_t)bs;
+#pragma unroll 4
+    for (int j = 0; j < ITEMS; ++j) {
+        const uint32_t at = blockIdx.x * (uint32_t)(T * ITEMS) + j * T + tid;      // (n is below 2^31)
+        if (at >= n) break;
+        const Block b = blocks[at / per];
+        const uint32_t p = at % per, s = b.r0 + p / (uint32_t)bs;
+        ns[at] = s;
+        nd[at] = b.c0 + p % (uint32_t)bs;
+        atomicAdd(&h[s & 255u], 1u);
+    }
+    __syncthreads();
+    c.hist[0][(int64_t)tid * c.blocks + blockIdx.x] = h[tid];
+}
+
 __global__ void k_write_raw(const uint32_t* __restrict__ ns, const uint32_t* __restrict__ nd, int64_t off,
                             int64_t cnt, int64_t dst_off, int64_t E_raw, int64_t* __restrict__ out) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -222,27 +310,37 @@ static int reformat_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, 
                          const int64_t* d_part, int k, int bs, int blockize, hipStream_t st, tgt_reformat* R) {
     R->N = N;
     DevBuf report, p32, pair, s32, d32;
+    RadixSorter node_sorter;
+    int rc = node_sorter.init(N, st);
+    if (rc) return rc;
     const size_t eb = sizeof(uint32_t) * (size_t)(E ? E : 1);
     // flag, nodes per part, edges per pair of parts: cleared and read back in one go
-    const size_t words = 1 + (size_t)k + (size_t)k * k;
+    const size_t words = (1 + (size_t)k + (size_t)k * k + 1) / 2 * 2;      // (16 bytes at a time: else it takes two launches to clear them)
     TGT_HIP_CHECK(report.alloc(sizeof(unsigned long long) * words, st));
     TGT_HIP_CHECK(p32.alloc(sizeof(uint32_t) * N, st));
     TGT_HIP_CHECK(R->mapping.alloc(sizeof(uint32_t) * N, st));
     TGT_HIP_CHECK(R->sorted_indices.alloc(sizeof(int64_t) * N, st));
-    TGT_HIP_CHECK(pair.alloc(eb, st));
-    TGT_HIP_CHECK(s32.alloc(eb, st));
-    TGT_HIP_CHECK(d32.alloc(eb, st));
     const DevBuf& mapping = R->mapping;
     unsigned long long *const flag = report.as<unsigned long long>(), *const cnt_nodes = flag + 1, *const cnt_pairs = cnt_nodes + k;
     TGT_HIP_CHECK(hipMemsetAsync(report.p, 0, sizeof(unsigned long long) * words, st));
-    hipLaunchKernelGGL(k_check_partition, dim3(nblk(N)), dim3(256), 0, st, d_part, N, k, p32.as<uint32_t>(), flag);
-    const auto count_grid = [](int64_t n) { return dim3((unsigned)std::min<int64_t>(256, (n + 255) / 256)); };
-    hipLaunchKernelGGL(k_count, count_grid(N), dim3(256), 0, st, p32.as<uint32_t>(), N, k, bits_for(k), cnt_nodes);
-    if (E > 0) {
+    const RadixSorter::Counts node_counts = node_sorter.counts(N, 1);
+    hipLaunchKernelGGL(node_counts.items == RadixSorter::kFewItems ? &k_check_partition<RadixSorter::kFewItems> : &k_check_partition<RadixSorter::kManyItems>,
+                       dim3(node_counts.blocks), dim3(RadixSorter::kThreads), 0, st, d_part, N, k, p32.as<uint32_t>(), flag, cnt_nodes, node_counts);
+    const auto count_grid = [](int64_t n) { return dim3((unsigned)std::min<int64_t>(512, (n + 1023) / 1024)); };
+    if (k > 256) hipLaunchKernelGGL(k_count, count_grid(N), dim3(256), 0, st, p32.as<uint32_t>(), N, k, bits_for(k), cnt_nodes);
+    // the edges' keys: for those that are kept as they are
+    const auto edge_keys = [&]() -> int {
+        TGT_HIP_CHECK(pair.alloc(eb, st));
+        TGT_HIP_CHECK(s32.alloc(eb, st));
+        TGT_HIP_CHECK(d32.alloc(eb, st));
         hipLaunchKernelGGL(k_edge_keys, dim3(nblk(E)), dim3(256), 0, st, d_src, d_dst, E, N, p32.as<uint32_t>(), k,
                            pair.as<uint32_t>(), s32.as<uint32_t>(), d32.as<uint32_t>(), flag);
-        hipLaunchKernelGGL(k_count, count_grid(E), dim3(256), 0, st, pair.as<uint32_t>(), E, k * k,
-                           bits_for((int64_t)k * k), cnt_pairs);
+        return TGT_OK;
+    };
+    if (E > 0 && !blockize) {
+        if ((rc = edge_keys()) != TGT_OK) return rc;
+    } else if (E > 0) {
+        hipLaunchKernelGGL(k_count_pairs, count_grid(E), dim3(256), 0, st, d_src, d_dst, E, N, p32.as<uint32_t>(), k, bits_for((int64_t)k * k), cnt_pairs, flag);
     }
     std::vector<unsigned long long> h_report(words);
     TGT_HIP_CHECK(hipMemcpyAsync(h_report.data(), report.p, sizeof(unsigned long long) * words, hipMemcpyDeviceToHost, st));
@@ -253,11 +351,8 @@ static int reformat_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, 
     }
     const unsigned long long *const h_nodes = h_report.data() + 1, *const h_pairs = h_nodes + k;
     // relabel: parts in order, members in ascending old id (gt_sp/utils.py:329-335) = stable sort by part
-    RadixSorter node_sorter;
-    int rc = node_sorter.init(N, st);
-    if (rc) return rc;
     const uint32_t *ks = nullptr, *vs = nullptr;
-    rc = node_sorter.sort(p32.as<uint32_t>(), nullptr, N, bits_for(k), st, &ks, &vs);
+    rc = node_sorter.sort(p32.as<uint32_t>(), nullptr, N, bits_for(k), st, &ks, &vs, true);
     if (rc) return rc;
     hipLaunchKernelGGL(k_invert, dim3(nblk(N)), dim3(256), 0, st, vs, N, R->mapping.as<uint32_t>(),
                        R->sorted_indices.as<int64_t>());
@@ -317,6 +412,7 @@ static int reformat_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, 
     RadixSorter& sorter = R->sorter;
     rc = sorter.init(E_out > E ? E_out : E, st);
     if (rc) return rc;
+    bool counted = false;      // the first digits of the sort by new source
 
     if (!blockize) {
         if (E > 0)
@@ -328,6 +424,7 @@ static int reformat_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, 
             // edges sorted by ((part_src, part_dst), (src, dst)) (gt_sp/utils.py:230-235): LSD over
             // dst, src, pair with the stable sort
             DevBuf tmp, order;
+            if (E > 0 && (rc = edge_keys()) != TGT_OK) return rc;
             TGT_HIP_CHECK(tmp.alloc(eb, st));
             TGT_HIP_CHECK(order.alloc(eb, st));
             const uint32_t *ko = nullptr, *vo = nullptr;
@@ -355,7 +452,13 @@ static int reformat_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, 
             TGT_HIP_CHECK(hipMemcpyAsync(d_blocks.p, blocks.data(), sizeof(Block) * blocks.size(), hipMemcpyHostToDevice, st));
             TGT_HIP_CHECK(hipEventCreateWithFlags(&R->copied, hipEventDisableTiming));
             TGT_HIP_CHECK(hipEventRecord(R->copied, st));
-            hipLaunchKernelGGL(k_emit_blocks, dim3((unsigned)blocks.size()), dim3(256), 0, st, d_blocks.as<Block>(), bs, ns.as<uint32_t>(), nd.as<uint32_t>());
+            counted = raws.empty();
+            const RadixSorter::Counts c = sorter.counts(E_out, 1);
+            if (counted)
+                hipLaunchKernelGGL(c.items == RadixSorter::kFewItems ? &k_emit_all_blocks<RadixSorter::kFewItems> : &k_emit_all_blocks<RadixSorter::kManyItems>, dim3(c.blocks),
+                                   dim3(RadixSorter::kThreads), 0, st, d_blocks.as<Block>(), bs, E_out, ns.as<uint32_t>(), nd.as<uint32_t>(), c);
+            else
+                hipLaunchKernelGGL(k_emit_blocks, dim3((unsigned)blocks.size()), dim3(256), 0, st, d_blocks.as<Block>(), bs, ns.as<uint32_t>(), nd.as<uint32_t>());
         }
     }
     // the blocks as a tile list and the edges kept as they are, for the block attention path
@@ -384,7 +487,7 @@ static int reformat_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, 
     }
     // stable sort by new source (gt_sp/utils.py:354-356)
     if (E_out > 0) {
-        rc = sorter.sort(ns.as<uint32_t>(), nullptr, E_out, bits_for(N), st, &R->keys, &R->order);
+        rc = sorter.sort(ns.as<uint32_t>(), nullptr, E_out, bits_for(N), st, &R->keys, &R->order, counted);
         if (rc) return rc;
     }
     TGT_HIP_CHECK(hipGetLastError());
@@ -674,17 +777,25 @@ int tgt_reformat_create(const int64_t* d_src, const int64_t* d_dst, int64_t E, i
 
 int64_t tgt_reformat_num_edges(const tgt_reformat_t* r) { return r ? r->E_out : -1; }
 
+int tgt_reformat_export_edges(const tgt_reformat_t* r, int64_t* d_edge_index, void* stream) {
+    if (!r || (r->E_out > 0 && !d_edge_index)) {
+        tgt::set_error("tgt_reformat_export_edges: null pointer");
+        return TGT_ERR_INVALID_ARG;
+    }
+    if (r->E_out > 0)
+        hipLaunchKernelGGL(tgt::k_write_sorted, dim3(tgt::nblk(r->E_out)), dim3(256), 0, (hipStream_t)stream, r->keys, r->order, r->nd.as<uint32_t>(), r->E_out, d_edge_index);
+    TGT_HIP_CHECK(hipGetLastError());
+    return TGT_OK;
+}
+
 int tgt_reformat_export(const tgt_reformat_t* r, int64_t* d_edge_index, int64_t* d_sorted_indices, void* stream) {
     if (!r || !d_sorted_indices || (r->E_out > 0 && !d_edge_index)) {
         tgt::set_error("tgt_reformat_export: null pointer");
         return TGT_ERR_INVALID_ARG;
     }
-    hipStream_t st = (hipStream_t)stream;
-    if (r->E_out > 0)
-        hipLaunchKernelGGL(tgt::k_write_sorted, dim3(tgt::nblk(r->E_out)), dim3(256), 0, st, r->keys, r->order, r->nd.as<uint32_t>(), r->E_out, d_edge_index);
-    TGT_HIP_CHECK(hipGetLastError());
+    if (int rc = tgt_reformat_export_edges(r, d_edge_index, stream)) return rc;
     TGT_HIP_CHECK(hipMemcpyAsync(d_sorted_indices, r->sorted_indices.p, sizeof(int64_t) * r->N,
-                                 hipMemcpyDeviceToDevice, st));
+                                 hipMemcpyDeviceToDevice, (hipStream_t)stream));
     return TGT_OK;
 }
 

@@ -33,17 +33,40 @@ const char* last_error() { return g_err; }
 // ---------------------------------------------------------------------------
 // kernels
 // ---------------------------------------------------------------------------
-// int64 endpoints -> uint32, with a range check (flag[0] = 1 on a bad index).
-__global__ void k_convert_validate(const int64_t* __restrict__ src, const int64_t* __restrict__ dst,
-                                   int64_t E, int64_t N, uint32_t* __restrict__ s32,
-                                   uint32_t* __restrict__ d32, int* __restrict__ flag) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= E) return;
-    int64_t s = src[i], d = dst[i];
-    bool bad = (s < 0) | (s >= N) | (d < 0) | (d >= N);
-    if (bad) { flag[0] = 1; s = 0; d = 0; }
-    s32[i] = (uint32_t)s;
-    d32[i] = (uint32_t)d;
+// int64 endpoints -> uint32, with a range check (flag[0] = 1 on a bad index), and the counts of their first digits that both sorts begin
+// with (RadixSorter::Counts: destinations, sources): a launch and a pass over the keys less.
+template <int ITEMS>
+__global__ __launch_bounds__(RadixSorter::kThreads) void k_convert_validate(const int64_t* __restrict__ src, const int64_t* __restrict__ dst, int64_t E, int64_t N,
+                                                                            uint32_t* __restrict__ s32, uint32_t* __restrict__ d32, int* __restrict__ flag,
+                                                                            const RadixSorter::Counts c) {
+    constexpr int T = RadixSorter::kThreads;
+    __shared__ uint32_t h[2][256];
+    const int tid = threadIdx.x;
+    h[0][tid] = h[1][tid] = 0;
+    __syncthreads();
+    const int64_t base = (int64_t)blockIdx.x * T * ITEMS + tid;
+    for (int j = 0; j < ITEMS; j += 4) {
+        int64_t s[4], d[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t i = min(base + (j + u) * T, E - 1);
+            s[u] = src[i]; d[u] = dst[i];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t i = base + (j + u) * T;
+            if (i >= E) continue;
+            const bool bad = (s[u] < 0) | (s[u] >= N) | (d[u] < 0) | (d[u] >= N);
+            if (bad) { flag[0] = 1; s[u] = 0; d[u] = 0; }
+            s32[i] = (uint32_t)s[u];
+            d32[i] = (uint32_t)d[u];
+            atomicAdd(&h[0][d[u] & 255], 1u);      // (integer counts: order-free)
+            atomicAdd(&h[1][s[u] & 255], 1u);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < 2; ++v) c.hist[v][(int64_t)tid * c.blocks + blockIdx.x] = h[v][tid];
 }
 
 // The two views are made by the same launches (blockIdx.y: by destination, by source): a batch's edge list does not fill the
@@ -56,7 +79,17 @@ struct SideArrays {
 // rowptr[r] = first sorted position whose key is >= r (r = 0 .. N): one thread per row, binary
 // search in the sorted keys (a thread per position walking the gap to the next key would leave
 // all the work to one thread when the keys are few or far apart).
-__global__ void k_fill_rowptr(const SideArrays a, int64_t E, int64_t N) {
+// The workgroups behind the first row_blocks: the endpoint and edge id of every sorted position, beside it.
+__global__ __launch_bounds__(256) void k_fill_rowptr_and_col(const SideArrays a, int64_t E, int64_t N, int row_blocks) {
+    if ((int)blockIdx.x >= row_blocks) {
+        const uint32_t *__restrict__ eid = a.order[blockIdx.y], *__restrict__ other = a.other[blockIdx.y];
+        const int64_t pos = (int64_t)(blockIdx.x - row_blocks) * blockDim.x + threadIdx.x;
+        if (pos >= E) return;
+        const uint32_t e = eid[pos];
+        a.col[blockIdx.y][pos] = (int32_t)other[e];
+        a.eid[blockIdx.y][pos] = (int32_t)e;
+        return;
+    }
     const uint32_t* __restrict__ keys = a.keys[blockIdx.y];
     int32_t* __restrict__ rowptr = a.rowptr[blockIdx.y];
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -68,16 +101,6 @@ __global__ void k_fill_rowptr(const SideArrays a, int64_t E, int64_t N) {
         else hi = mid;
     }
     rowptr[r] = (int32_t)lo;
-}
-
-__global__ void k_gather_col(const SideArrays a, int64_t E) {
-    const uint32_t *__restrict__ eid = a.order[blockIdx.y], *__restrict__ other = a.other[blockIdx.y];
-    int32_t *__restrict__ col = a.col[blockIdx.y], *__restrict__ eid_out = a.eid[blockIdx.y];
-    int64_t pos = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (pos >= E) return;
-    uint32_t e = eid[pos];
-    col[pos] = (int32_t)other[e];
-    eid_out[pos] = (int32_t)e;
 }
 
 // ---------------------------------------------------------------------------
@@ -495,7 +518,7 @@ __global__ __launch_bounds__(64 * kRecordWaves) void k_build_records(const Run* 
 // ---------------------------------------------------------------------------
 // host helpers
 // ---------------------------------------------------------------------------
-// Sort edge ids by destination and by source (stable) and fill both views' rowptr / col / eid.
+// Sort edge ids by destination and by source (stable; first digits counted) and fill both views' rowptr / col / eid.
 static int build_sides(const uint32_t* d32, const uint32_t* s32, int64_t E, int64_t N, RadixSorter& sorter, Side& dst, Side& src, hipStream_t st) {
     SideArrays a{};
     a.keys[0] = d32; a.keys[1] = s32;
@@ -505,12 +528,12 @@ static int build_sides(const uint32_t* d32, const uint32_t* s32, int64_t E, int6
     a.eid[0] = dst.eid; a.eid[1] = src.eid;
     if (E > 0) {
         const uint32_t* in[2] = {d32, s32};
-        int rc = sorter.sort(in, nullptr, 2, E, bits_for(N), st, a.keys, a.order);
+        int rc = sorter.sort(in, nullptr, 2, E, bits_for(N), st, a.keys, a.order, true);
         if (rc) return rc;
     }
     const int T = 256;
-    hipLaunchKernelGGL(k_fill_rowptr, dim3((unsigned)((N + 1 + T - 1) / T), 2), dim3(T), 0, st, a, E, N);
-    if (E > 0) hipLaunchKernelGGL(k_gather_col, dim3((unsigned)((E + T - 1) / T), 2), dim3(T), 0, st, a, E);
+    const int row_blocks = (int)((N + 1 + T - 1) / T);
+    hipLaunchKernelGGL(k_fill_rowptr_and_col, dim3((unsigned)(row_blocks + (E + T - 1) / T), 2), dim3(T), 0, st, a, E, N, row_blocks);
     TGT_HIP_CHECK(hipGetLastError());
     return TGT_OK;
 }
@@ -896,9 +919,9 @@ static int create_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, in
     TGT_HIP_CHECK(hipMemsetAsync(report_d.p, 0, sizeof(int32_t) * kReportHead, st));
     int32_t* report = report_d.as<int32_t>();
     if (E > 0) {
-        const int T = 256;
-        hipLaunchKernelGGL(k_convert_validate, dim3((unsigned)((E + T - 1) / T)), dim3(T), 0, st, d_src,
-                           d_dst, E, N, s32.as<uint32_t>(), d32.as<uint32_t>(), report + kReportFlag);
+        const RadixSorter::Counts c = sorter.counts(E, 2);
+        hipLaunchKernelGGL(c.items == RadixSorter::kFewItems ? &k_convert_validate<RadixSorter::kFewItems> : &k_convert_validate<RadixSorter::kManyItems>, dim3(c.blocks),
+                           dim3(RadixSorter::kThreads), 0, st, d_src, d_dst, E, N, s32.as<uint32_t>(), d32.as<uint32_t>(), report + kReportFlag, c);
         TGT_HIP_CHECK(hipGetLastError());
     }
     // out-of-range endpoints were replaced by node 0 (and flagged): everything below runs on valid ids

@@ -12,12 +12,12 @@
 
 namespace tgt {
 
-constexpr int RS_THREADS = 256;
+constexpr int RS_THREADS = RadixSorter::kThreads;
 // Keys per thread (a workgroup's tile is 256 times as many; a wave takes a quarter of it, consecutive keys): 4 as long as every tile of a launch has
 // a place of its own (eight workgroups per CU), 16 with more.  Few keys are bound by the chain of one tile, sixteen rounds of ballots and
 // an LDS counter: 0.53 M keys of two sorts 8.6 us a pass with 4, 12 with 8, 14.5 with 16; 0.2 M of one 6.1, 8.1, 13.9.  Many pay for the
 // digits' counts of every tile: a plan of 2 M edges 584 us and 537 with 16, of 44 M 6.9 ms and 5.5.
-constexpr int kFewItems = 4, kManyItems = 16;
+constexpr int kFewItems = RadixSorter::kFewItems, kManyItems = RadixSorter::kManyItems;
 static int rs_items(int64_t n, int sorts) { return n * sorts <= (int64_t)8 * num_cus() * RS_THREADS * kFewItems ? kFewItems : kManyItems; }
 
 // One or two sorts of the same size in a launch (blockIdx.y): the two views of a plan are sorted side by side - at half a
@@ -229,26 +229,35 @@ int RadixSorter::init(int64_t n, hipStream_t st, int sorts) {
     return TGT_OK;
 }
 
+RadixSorter::Counts RadixSorter::counts(int64_t n, int sorts) const {
+    Counts c{};
+    // items of the capacity: a smaller sort never has more workgroups than there is room for
+    c.items = rs_items(cap_, sorts_);
+    c.blocks = (int)((n + RS_THREADS * c.items - 1) / (RS_THREADS * c.items));
+    for (int i = 0; i < sorts; ++i) c.hist[i] = buf_.as<uint32_t>() + i * (4 * (size_t)cap_ + 256 * (size_t)nblocks_ + 256) + 4 * (size_t)cap_;
+    return c;
+}
+
 int RadixSorter::sort(const uint32_t* const* keys_in, const uint32_t* const* vals_in, int sorts, int64_t n, int bits, hipStream_t st,
-                      const uint32_t** keys_out, const uint32_t** vals_out) {
+                      const uint32_t** keys_out, const uint32_t** vals_out, bool counted) {
     if (n > cap_ || sorts > sorts_) { set_error("RadixSorter: n exceeds capacity"); return TGT_ERR_INVALID_ARG; }
     const int passes = (bits + 7) / 8 > 0 ? (bits + 7) / 8 : 1;
-    // of the capacity: a smaller sort never has more workgroups than there is room for
-    const int items = rs_items(cap_, sorts_), nblocks = (int)((n + RS_THREADS * items - 1) / (RS_THREADS * items));
+    const Counts c = counts(n, sorts);
+    const int items = c.items, nblocks = c.blocks;
     RsArgs a{};
     uint32_t *key[2][2], *val[2][2];      // [sort][ping, pong]
-    uint32_t* at = buf_.as<uint32_t>();
     for (int i = 0; i < sorts; ++i) {
+        uint32_t* at = c.hist[i] - 4 * (size_t)cap_;
         for (int j = 0; j < 2; ++j) { key[i][j] = at; val[i][j] = at + cap_; at += 2 * cap_; }
-        a.hist[i] = at; a.totals[i] = at + 256 * (size_t)nblocks_;
-        at += 256 * (size_t)nblocks_ + 256;
+        a.hist[i] = c.hist[i]; a.totals[i] = c.hist[i] + 256 * (size_t)nblocks_;
         a.keys_in[i] = keys_in[i];
         a.vals_in[i] = vals_in ? vals_in[i] : nullptr;
     }
     for (int p = 0; p < passes && n > 0; ++p) {
         const int shift = 8 * p;
         for (int i = 0; i < sorts; ++i) { a.keys_out[i] = key[i][p & 1]; a.vals_out[i] = val[i][p & 1]; }
-        hipLaunchKernelGGL(items == kFewItems ? &k_rs_hist<kFewItems> : &k_rs_hist<kManyItems>, dim3(nblocks, sorts), dim3(RS_THREADS), 0, st, a, n, shift, nblocks);
+        if (p > 0 || !counted)
+            hipLaunchKernelGGL(items == kFewItems ? &k_rs_hist<kFewItems> : &k_rs_hist<kManyItems>, dim3(nblocks, sorts), dim3(RS_THREADS), 0, st, a, n, shift, nblocks);
         hipLaunchKernelGGL(k_rs_scan_rows, dim3(256, sorts), dim3(256), 0, st, a, nblocks);
         hipLaunchKernelGGL(items == kFewItems ? &k_rs_scatter<kFewItems> : &k_rs_scatter<kManyItems>, dim3(nblocks, sorts), dim3(RS_THREADS), 0, st, a, n, shift, nblocks);
         for (int i = 0; i < sorts; ++i) { a.keys_in[i] = a.keys_out[i]; a.vals_in[i] = a.vals_out[i]; }

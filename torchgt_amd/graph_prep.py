@@ -80,7 +80,7 @@ def reformat_graph(edge_index, k, block_size, beta_coeffi="1", partition_ids=Non
 
 def _reformat(edge_index, k, block_size, partition_ids, blockize, return_tiles, batch=None, tokens=0):
     """``(edges, sorted_indices, tiles, raw edges, rows)``; rows: the nodes of ``batch`` in the new order (without the global
-    node in front of them when ``tokens`` is 1)."""
+    node in front of them when ``tokens`` is 1), in the place of sorted_indices."""
     if partition_ids is None:
         raise ValueError("reformat_graph: partition_ids must be given (METIS is not available)")
     if not edge_index.is_cuda:
@@ -99,9 +99,12 @@ def _reformat(edge_index, k, block_size, partition_ids, blockize, return_tiles, 
         try:
             E_out = L.tgt_reformat_num_edges(handle)
             out = torch.empty((2, E_out), dtype=torch.int64, device=dev)
-            sorted_indices = torch.empty(N, dtype=torch.int64, device=dev)
-            _lib.check(L.tgt_reformat_export(handle, out.data_ptr() if E_out else None,
-                                             sorted_indices.data_ptr(), st))
+            out_ptr, sorted_indices = out.data_ptr() if E_out else None, None
+            if batch is None:
+                sorted_indices = torch.empty(N, dtype=torch.int64, device=dev)
+                _lib.check(L.tgt_reformat_export(handle, out_ptr, sorted_indices.data_ptr(), st))
+            else:
+                _lib.check(L.tgt_reformat_export_edges(handle, out_ptr, st))
             tiles = raw = rows = None
             if return_tiles:
                 import numpy as np
