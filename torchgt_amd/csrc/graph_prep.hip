@@ -25,7 +25,9 @@ namespace tgt {
 // they are first needed, the same numbers as whole blocks of 624 (64 pairs: 180 us of host time with them).
 class LegacyMT {
 public:
-    explicit LegacyMT(uint32_t seed) { mt_[0] = seed; }
+    LegacyMT() = default;
+    explicit LegacyMT(uint32_t s) { seed(s); }
+    void seed(uint32_t s) { mt_[0] = s; }      // (of a new stream)
     uint32_t next() {
         const uint32_t UP = 0x80000000u, LO = 0x7fffffffu, MAG = 0x9908b0dfu;
         const int i = pos_, i1 = i + 1 < 624 ? i + 1 : 0, im = i + 397 < 624 ? i + 397 : i - 227;
@@ -48,6 +50,20 @@ public:
         uint32_t v;
         do { v = next() & (uint32_t)mask; } while (v > rng);
         return (int64_t)v;
+    }
+    // The first state words of up to kTogether streams, side by side: a word is made of the one before it, so one stream waits for the
+    // multiplier with every word (64 pairs of parts, 24 blocks each: 48 us of host time with the draws, 19 together).
+    static constexpr int kTogether = 8;
+    static void seed_together(LegacyMT* g, int n, int words) {
+        uint32_t v[kTogether];
+        for (int l = 0; l < kTogether; ++l) v[l] = l < n ? g[l].mt_[0] : 0u;
+        words = words < 624 ? words : 624;
+        for (int w = 1; w < words; ++w)
+            for (int l = 0; l < kTogether; ++l) {
+                v[l] = 1812433253u * (v[l] ^ (v[l] >> 30)) + (uint32_t)w;
+                g[l].mt_[w] = v[l];
+            }
+        for (int l = 0; l < n; ++l) g[l].seeded_ = words > 1 ? words : 1;
     }
 private:
     void seeded(int upto) {
@@ -359,6 +375,7 @@ static int reformat_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, 
 
     // ---- what to emit, in the reference's order ------------------------------
     struct RawSlice { int64_t lo, cnt, out_off; };
+    struct Stream { size_t block0; int i, j, n; uint32_t seed; };      // the blocks of one pair of parts, drawn from a stream of their own
     std::vector<RawSlice> raws;
     std::vector<Block>& blocks = R->blocks;
     int64_t E_out = 0;
@@ -374,6 +391,8 @@ static int reformat_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, 
         for (size_t pq = 0; pq < (size_t)k * k; ++pq) cum[pq + 1] = cum[pq] + counts[pq];
         for (int i = 1; i < k; ++i) offs[i] = offs[i - 1] + (int64_t)h_nodes[i - 1];
         int64_t keep_cnt = 0;
+        std::vector<Stream> streams;
+        streams.reserve(std::min<size_t>((size_t)k * k, 4096));
         const double per_block = (double)bs * (double)bs;
         for (int i = 0; i < k; ++i) {
             for (int j = 0; j < k; ++j) {
@@ -390,16 +409,32 @@ static int reformat_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, 
                     E_out += c;
                 } else {
                     const int nb = (int)(sparsity * (double)total / per_block) + 1;
-                    LegacyMT rng((uint32_t)keep_cnt);        // np.random.seed(keep_cnt)
                     if (ni >= bs && nj >= bs) {
-                        for (int b = 0; b < nb; ++b) {
-                            const int64_t br = rng.randint(ni / bs);
-                            const int64_t bc = rng.randint(nj / bs);
-                            ++keep_cnt;
-                            blocks.push_back(Block{E_out, (uint32_t)(br * bs + offs[i]), (uint32_t)(bc * bs + offs[j])});
-                            E_out += (int64_t)bs * bs;
-                        }
+                        streams.push_back(Stream{blocks.size(), i, j, nb, (uint32_t)keep_cnt});      // np.random.seed(keep_cnt)
+                        for (int b = 0; b < nb; ++b) blocks.push_back(Block{E_out + (int64_t)b * bs * bs, 0, 0});
+                        keep_cnt += nb;
+                        E_out += (int64_t)nb * bs * bs;
                     }
+                }
+            }
+        }
+        for (size_t s0 = 0; s0 < streams.size(); s0 += LegacyMT::kTogether) {
+            const int n = (int)std::min<size_t>(LegacyMT::kTogether, streams.size() - s0);
+            LegacyMT rng[LegacyMT::kTogether];
+            int most = 0;
+            for (int l = 0; l < n; ++l) {
+                rng[l].seed(streams[s0 + l].seed);
+                most = std::max(most, streams[s0 + l].n);
+            }
+            // draw d reads words d + 1 and d + 397; two draws a block, some of them twice (what is not there yet is made when it is asked for)
+            LegacyMT::seed_together(rng, n, 400 + (int)std::min<int64_t>(3ll * most, 624));
+            for (int l = 0; l < n; ++l) {
+                const Stream& s = streams[s0 + l];
+                const int64_t rows = (int64_t)h_nodes[s.i] / bs, cols = (int64_t)h_nodes[s.j] / bs;
+                for (int b = 0; b < s.n; ++b) {
+                    const int64_t br = rng[l].randint(rows), bc = rng[l].randint(cols);
+                    blocks[s.block0 + b].r0 = (uint32_t)(br * bs + offs[s.i]);
+                    blocks[s.block0 + b].c0 = (uint32_t)(bc * bs + offs[s.j]);
                 }
             }
         }
@@ -462,6 +497,7 @@ static int reformat_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, 
         }
     }
     // the blocks as a tile list and the edges kept as they are, for the block attention path
+    R->tiles.reserve(2 * blocks.size());
     for (const Block& b : blocks) {
         R->tiles.push_back((int32_t)b.r0);
         R->tiles.push_back((int32_t)b.c0);
