@@ -73,8 +73,10 @@ constexpr bool plane_fits(int S) {
 static_assert(plane_fits(288) && 2 * 288 * 288 > kLdsLimit, "every size that fits the LDS");
 // The first kAhead pieces of a thread are asked for at once (`ask`), in front of everything else; `arrive` puts them into LDS and fetches what is left.
 // (A piece may begin or end outside the tensor, never outside the 16 bytes that one of its elements is in.)
-template <int THREADS> struct PlaneIn {
-    static constexpr int kAhead = 8;
+// As many as the largest plane of the variant has, at most eight: eight for every one cost small planes 12 to 22 registers and a wave per SIMD
+// (backward, 8 heads of 8, us with eight / as many: 256 graphs of 41 rows 16.4 / 14.9, 129 54.6 / 54.3, 101 45.2 / 44.7).
+template <int THREADS, int S_MAX> struct PlaneIn {
+    static constexpr int kAhead = std::min(8, (2 * S_MAX * S_MAX + 14 + 15) / 16 / THREADS + 1);
     vec16 v[kAhead];
     const vec16* src;
     int pieces;
@@ -157,7 +159,7 @@ __global__ __launch_bounds__(64 * NW, 4) void k_plane_fwd(const dbf16* __restric
     plane.lds = reinterpret_cast<unsigned char*>(flags) + kFlagBytes;
     plane.off = (int)(reinterpret_cast<uintptr_t>(bias_gh) & 15);
     plane.n = S * S;
-    PlaneIn<THREADS> in;
+    PlaneIn<THREADS, NW * 32 + (THIN ? 4 : 0)> in;
     in.ask(plane, bias_gh);
     const int64_t base = ((int64_t)g * S * H + h) * D;
     const auto row_at = [&](int row) { return base + (int64_t)row * H * D; };
@@ -355,7 +357,7 @@ __global__ __launch_bounds__(64 * NW * W, (D == 32 ? 2 : 4)) void k_plane_bwd(co
     plane.lds = reinterpret_cast<unsigned char*>(thin_part + (THIN ? NW * 8 * D : 0));
     plane.off = (int)(reinterpret_cast<uintptr_t>(dbias ? dbias_gh : bias_gh) & 15);
     plane.n = S * S;
-    PlaneIn<THREADS> in;
+    PlaneIn<THREADS, NW * 32 + (THIN ? 4 : 0)> in;
     if (bias) in.ask(plane, bias_gh);
     // rows of this head: element (row, c) at ((g S + row) H + h) D + c
     const int64_t base = ((int64_t)g * S * H + h) * D;
