@@ -293,3 +293,38 @@ def test_batches_that_are_not_on_the_gpu_are_refused(cuda, edge_type, one_operat
             with pytest.raises(RuntimeError, match="on the GPU|GPU only"):
                 m(types.SimpleNamespace(**{**batch, name: batch[name].cpu()}))
     assert m(types.SimpleNamespace(**batch)).shape == (b, 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("b,s,C,Fx", [(1, 1, 8, 1), (5, 51, 8, 3), (4, 63, 4, 1), (3, 100, 40, 2), (7, 36, 64, 1), (256, 128, 64, 1), (2, 30, 200, 9), (2, 30, 12, 2)])
+def test_node_features_sixteen_bytes_at_a_time(cuda, dtype, b, s, C, Fx):
+    """Rows of whole pieces of 16 bytes against the same call one channel per thread, which a table or an output that begins in the middle of
+    a piece takes: the same bits, also for ids outside the tables (which are clamped) and workgroups that end inside a row."""
+    print(f"node features by pieces: b={b} s={s} C={C} Fx={Fx} {dtype}", flush=True)
+    g, L, st = torch.Generator(device=cuda).manual_seed(b * s + C), _lib.lib(), torch.cuda.current_stream(cuda).cuda_stream
+    code = _lib.DTYPE_F32 if dtype == torch.float32 else _lib.DTYPE_BF16
+    ids = lambda *shape: torch.randint(-3, 24, shape, generator=g, device=cuda)
+    x, ind, outd = ids(b, s, Fx), ids(b, s), ids(b, s)
+    tables = [torch.randn(n, C, generator=g, device=cuda).to(dtype) for n in (20, 15, 12, 1)]
+
+    def shifted(t):
+        room = torch.empty(t.numel() + 1, dtype=dtype, device=cuda)
+        room[1:] = t.reshape(-1)
+        return room[1:].view(t.shape)
+
+    def run(t, out):
+        _lib.check(L.tgt_graph_node_feature_fwd(x.data_ptr(), ind.data_ptr(), outd.data_ptr(), Fx, t[0].data_ptr(), 20, t[1].data_ptr(), 15, t[2].data_ptr(), 12,
+                                                t[3].data_ptr(), b, s, C, code, out.data_ptr(), st))
+        return out
+
+    new = lambda *shape: torch.full(shape, float("nan"), dtype=dtype, device=cuda)
+    want = run(tables, shifted(new(b, s + 1, C)))
+    assert not want.isnan().any()
+    assert torch.equal(run(tables, new(b, s + 1, C)), want)
+    for i in range(4):
+        assert torch.equal(run([shifted(t) if j == i else t for j, t in enumerate(tables)], new(b, s + 1, C)), want), i
+    sums = []
+    for out in (shifted(new(b, s, C)), new(b, s, C)):
+        _lib.check(L.tgt_embedding_sum_fwd(x.data_ptr(), Fx, tables[0].data_ptr(), 20, b, s, C, code, out.data_ptr(), st))
+        sums.append(out)
+    assert torch.equal(sums[1], sums[0]) and not sums[0].isnan().any()

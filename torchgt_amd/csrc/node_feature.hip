@@ -68,6 +68,48 @@ __global__ __launch_bounds__(256) void k_node_feature_fwd(NodeFeatArgs a, const 
     stf(out + t, v);
 }
 
+// The same, 16 bytes of a row per thread: C a multiple of them, every table and `out` 16-byte aligned, fewer than 2^31 threads.  Bound by the two
+// dependent reads of a row's ids and table rows; with a thread per channel every lane divided 64-bit numbers four times and wrote 2 bytes.
+// 33 K rows of 64 channels, bf16: 11.3 / 4.4 us.
+template <typename T> constexpr int kFeatVec = 16 / (int)sizeof(T);
+template <typename T> struct FeatVec { T e[kFeatVec<T>]; };
+template <typename T>
+__global__ __launch_bounds__(256) void k_node_feature_fwd_vec(NodeFeatArgs a, const T* __restrict__ atom, const T* __restrict__ tin, const T* __restrict__ tout,
+                                                              const T* __restrict__ token, T* __restrict__ out) {
+    constexpr int V = kFeatVec<T>;
+    const uint32_t rows = a.s + a.has_token, per = a.C / V, t = blockIdx.x * 256u + threadIdx.x, row = t / per, c = t % per * V;
+    if (row >= (uint32_t)a.b * rows) return;
+    const uint32_t g = row / rows;
+    const int node = (int)(row % rows) + 1 - a.has_token;
+    const auto ask = [&](const T* table, int r) { return *reinterpret_cast<const uint4*>(table + (int64_t)r * a.C + c); };
+    uint4 u;
+    if (node == 0) u = ask(token, 0);
+    else {
+        const int64_t p = (int64_t)g * a.s + (node - 1);
+        float v[V];
+#pragma unroll
+        for (int i = 0; i < V; ++i) v[i] = 0.f;
+        const auto add = [&](const uint4& w) {
+            const FeatVec<T> x = __builtin_bit_cast(FeatVec<T>, w);
+#pragma unroll
+            for (int i = 0; i < V; ++i) v[i] += ldf(x.e + i);
+        };
+        int64_t din = 0, dout = 0;
+        if (a.has_degree) { din = a.in_degree[p]; dout = a.out_degree[p]; }
+        for (int f = 0; f < a.Fx; ++f) add(ask(atom, clamp_id(a.x[p * a.Fx + f], a.num_atoms)));
+        if (a.has_degree) {
+            const uint4 x = ask(tin, clamp_id(din, a.num_in)), y = ask(tout, clamp_id(dout, a.num_out));
+            add(x);
+            add(y);
+        }
+        FeatVec<T> o;
+#pragma unroll
+        for (int i = 0; i < V; ++i) stf(o.e + i, v[i]);
+        u = __builtin_bit_cast(uint4, o);
+    }
+    *reinterpret_cast<uint4*>(out + (int64_t)row * a.C + c) = u;
+}
+
 __global__ __launch_bounds__(256) void k_fill_zero(float* __restrict__ p, int64_t n) {
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (t < n) p[t] = 0.f;
@@ -269,7 +311,18 @@ int node_feature_fwd_impl(NodeFeatArgs a, const void* d_atom_table, const void* 
     if (total == 0) return TGT_OK;
     const dim3 grid((unsigned)((total + 255) / 256));
     hipStream_t st = (hipStream_t)stream;
-    if (dtype == TGT_DTYPE_F32)
+    const int vec = dtype == TGT_DTYPE_F32 ? kFeatVec<float> : kFeatVec<nbf16>;
+    const auto where = [](const void* p) { return reinterpret_cast<uintptr_t>(p); };      // (what is not in use is not read)
+    const uintptr_t ends = where(d_atom_table) | where(d_out) | (a.has_degree ? where(d_in_table) | where(d_out_table) : 0) | (a.has_token ? where(d_graph_token) : 0);
+    if (a.C % vec == 0 && ends % 16 == 0 && total / vec <= INT32_MAX) {
+        const dim3 few((unsigned)((total / vec + 255) / 256));
+        if (dtype == TGT_DTYPE_F32)
+            hipLaunchKernelGGL((k_node_feature_fwd_vec<float>), few, dim3(256), 0, st, a, (const float*)d_atom_table, (const float*)d_in_table, (const float*)d_out_table,
+                               (const float*)d_graph_token, (float*)d_out);
+        else
+            hipLaunchKernelGGL((k_node_feature_fwd_vec<nbf16>), few, dim3(256), 0, st, a, (const nbf16*)d_atom_table, (const nbf16*)d_in_table, (const nbf16*)d_out_table,
+                               (const nbf16*)d_graph_token, (nbf16*)d_out);
+    } else if (dtype == TGT_DTYPE_F32)
         hipLaunchKernelGGL((k_node_feature_fwd<float>), grid, dim3(256), 0, st, a, (const float*)d_atom_table, (const float*)d_in_table,
                            (const float*)d_out_table, (const float*)d_graph_token, (float*)d_out);
     else
