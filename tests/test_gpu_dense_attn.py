@@ -333,3 +333,44 @@ def test_plane_in_lds_gives_what_the_general_kernels_give(cuda, b, S, H, d, offs
             print("  ", name, f"{e:.1e}", flush=True)
             # the backward's dout . out is taken from the stored output: bf16 there, float32 here (2^-9 of it more, twice in dq and dk)
             assert e <= (2 ** -7 if name in ("out", "dv") else 2 ** -6), name
+
+
+# float32 on the matrix instructions: tiles of sixteen rows that end inside, at and behind one, one query or key alone in the last, an odd tile in the
+# last step of 32 keys, the largest sizes of the three head dims (224, 160, 96) and the first of the general kernels
+@pytest.mark.parametrize("b,S,H,d,p_drop", [(3, 1, 2, 8, 0.0), (9, 2, 2, 16, 0.0), (3, 15, 2, 8, 0.4), (3, 16, 8, 32, 0.0), (3, 17, 3, 8, 0.0), (3, 31, 2, 16, 0.3), (3, 32, 2, 8, 0.0),
+                                            (3, 33, 2, 32, 0.2), (17, 48, 8, 8, 0.0), (3, 49, 2, 16, 0.0), (9, 65, 8, 8, 0.1), (3, 96, 2, 32, 0.0), (3, 97, 2, 32, 0.0),
+                                            (2, 128, 2, 8, 0.0), (2, 129, 2, 16, 0.2), (2, 160, 2, 16, 0.0), (2, 161, 2, 16, 0.0), (2, 208, 2, 8, 0.0), (2, 224, 2, 8, 0.1), (2, 225, 2, 8, 0.0)])
+def test_float32_at_the_edges_of_the_tiles(cuda, b, S, H, d, p_drop):
+    # (two rows keep both keys: a row with one has dS = 0, and where the only others' probabilities are nearly 1 the scale of all dS is that of a product p (dP - D)
+    # that cancels: |D| 2^-24 of rounding is 4e-5 of it, in any order of the sums)
+    real = [max(1, S - 7 * i) if S > 2 else S for i in range(b)]
+    for bias in (True, False):
+        run_case("f32-tiles", b, S, H, d, torch.float32, bias, real, S + d, cuda, p_drop=p_drop)
+
+
+@pytest.mark.parametrize("S,d", [(20, 8), (50, 16), (70, 32), (129, 8)])
+def test_float32_infinities_and_masked_rows(cuda, S, d):
+    """Where results are finite, infinite and NaN as a float64 evaluation has it: an infinite value under a mask (0 times inf), a NaN query, a key and a
+    gradient that are infinite, a row without any key and one whose bias is the lowest float."""
+    print(f"dense float32 infinities S={S} d={d}", flush=True)
+    g = torch.Generator().manual_seed(S)
+    q, k, v, dout = (torch.randn(5, S, 2, d, generator=g) for _ in range(4))
+    bias = torch.randn(5, 2, S, S, generator=g)
+    bias[0, :, :, S // 2:] = float("-inf")
+    v[0, S - 1, 0, 3] = float("inf")
+    q[1, S // 2, 1, 2] = float("nan")
+    k[2, 3, 0, d - 1] = float("inf")
+    dout[3, S - 1, 1, 0] = float("-inf")
+    bias[4, 0, S // 3] = float("-inf")
+    bias[4, 1, :, 1:] = torch.finfo(torch.float32).min
+
+    def run(dev, f):
+        ts = [t.to(dev, f).requires_grad_(True) for t in (q, k, v, bias)]
+        o = dense_attention(*ts) if dev != "cpu" else oda.dense_attention(*ts)
+        return (o, *torch.autograd.grad(o, ts, dout.to(dev, f).reshape(o.shape)))
+
+    for name, x, y in zip(("out", "dq", "dk", "dv", "dbias"), run(cuda, torch.float32), run("cpu", torch.float64)):
+        x, y = x.detach().double().cpu(), y.detach()
+        ok = torch.isfinite(y)
+        assert torch.equal(torch.isfinite(x), ok), name
+        assert float((x - y)[ok].abs().max()) <= 1e-5 * float(y[ok].abs().max()), name

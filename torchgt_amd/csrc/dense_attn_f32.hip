@@ -3,9 +3,11 @@
 // The reference's dense CoreAttention.forward (models/graphormer_graph_level.py:186-214, attn_module.py:99-127)
 // computes in float32:  x = (q * sqrt(d)) k^T + attn_bias ; softmax over keys ; dropout ; x v.  The matrix-core
 // kernels of dense_attn.hip round their operands to bf16, which costs 2^-8 on logits that the reference's
-// q * sqrt(d) makes large; a float32 caller who has not asked for that gets these kernels instead: plain fp32
-// multiply-adds on the vector units (head dims of 8 to 32 make the products 8 to 32 deep, far too thin to be
-// bound by them), fp32 softmax with the accurate exponential, 1e-5 against a float64 evaluation.
+// q * sqrt(d) makes large; a float32 caller who has not asked for that gets these kernels instead: float32
+// products and sums, fp32 softmax with the accurate exponential, 1e-5 against a float64 evaluation.
+//
+// Up to 224 rows (160 and 96 with head dims of 16 and 32) the products go to the float32 matrix instructions (k_dense_f32_mm_*, below), a wave per
+// tile of sixteen queries (forward) or keys (backward).  What follows is about the other two kernels, on the vector units.
 //
 // One workgroup per (graph, head).  Forward: K and V of the head sit in LDS, a thread owns one query row and
 // walks the keys with an online softmax; every LDS read of K / V is a broadcast.  A thread that read its own
@@ -17,6 +19,7 @@
 // saved log-sum-exp.
 #include "common.h"
 #include "dense_dropout.h"
+#include <algorithm>
 
 namespace tgt {
 
@@ -246,6 +249,285 @@ __global__ __launch_bounds__(kF32Block) void k_dense_f32_bwd(const float* __rest
     }
 }
 
+// ---- on the matrix instructions ------------------------------------------------------------------------------------------
+// v_mfma_f32_16x16x4_f32: A[i][k] and B[k][j] in lane i (j) + 16 k, C[4 g + t][j] in register t of lane j + 16 g; float32 products, the running sum
+// rounded no more often than by a chain of fmas.  The contractions over queries and keys take their steps in the order in which C leaves
+// them: register t is the B operand of a step over the rows 4 k + t.
+//
+// With a thread per query row 65 rows kept 65 of 256 threads busy, and every element read the row of K (and V) from LDS twice, once for the
+// thread's query and once for its key.  Here a wave has sixteen rows, all of them work, the bias and its gradient go between memory and registers in
+// rows of 64 bytes, and the backward forms a probability once.  us, 8 heads of 8, thread per row / this, forward and backward: 256 graphs of
+// 13 rows 7.6 / 5.3, 13.5 / 6.9; of 41 16.4 / 13.0, 40.8 / 18.9; of 129 120 / 71, 304 / 134 (bias and gradient alone, 136 MB each, 26 and 53 at
+// the rate of a large copy); 64 of 201 101 / 39, 223 / 66; 4 of 129 38 / 13, 87 / 19; heads of 32, 64 of 65 rows 35 / 15, 91 / 35.  Errors against 64 bits
+// a tenth smaller (256 graphs of 41 rows, of the norm: out 1.29e-7 / 1.40e-7 before, dq 2.1e-7 / 2.2e-7, dbias 1.9e-7 / 2.0e-7).
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ f32x4_t mma4(float a, float b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+constexpr int kMmTiles = 16;        // tiles of sixteen rows, a wave each
+template <int D> struct Mm {
+    static constexpr int LD = D + 1, DB = (D + 15) / 16, KS = D / 4;      // row stride in LDS (odd: rows in different banks), blocks of sixteen features, steps over them
+    static int tiles(int S) { return (S + 15) / 16; }
+    static int fwd_lds(int S) { return 2 * 16 * tiles(S) * LD * 4; }
+    static int bwd_lds(int S) {
+        const int n = tiles(S), rows = 16 * n;
+        return (n * rows * D + 2 * rows + 4 * rows * LD + n * 16 * 17) * 4;
+    }
+    static bool fits(int S) { return S > 0 && tiles(S) <= kMmTiles && bwd_lds(S) <= 160 * 1024; }
+    // X[g, :, h, :] -> LDS [rows][LD], rows behind S are zero
+    static __device__ __forceinline__ void stage(const float* __restrict__ X, int g, int h, int S, int H, float f, float* __restrict__ dst, int rows) {
+        for (int c = threadIdx.x; c < rows * KS; c += blockDim.x) {
+            const int row = c / KS, part = c % KS;
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (row < S) v = *reinterpret_cast<const float4*>(X + (((int64_t)g * S + row) * H + h) * D + part * 4);
+            float* to = dst + row * LD + part * 4;
+            to[0] = v.x * f; to[1] = v.y * f; to[2] = v.z * f; to[3] = v.w * f;
+        }
+    }
+};
+
+// Wave w: the queries 16 w ..., a lane's query is its column; 32 keys between two rescalings.
+template <int D, bool DROP>
+__global__ __launch_bounds__(64 * kMmTiles) void k_dense_f32_mm_fwd(const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
+                                                                    const float* __restrict__ bias, float* __restrict__ out, float* __restrict__ lse, int S, int H,
+                                                                    float scale, int nb, const DropArgs da) {
+    using M = Mm<D>;
+    constexpr int LD = M::LD, DB = M::DB, KS = M::KS;
+    extern __shared__ __align__(16) char smem[];
+    const int rows = blockDim.x / 4;
+    float *k_l = reinterpret_cast<float*>(smem), *v_l = k_l + rows * LD;
+    int g, h;
+    if (!pair_of_block(nb, H, g, h)) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, gr = lane >> 4, cd = c % D;
+    const int qi = wave * 16 + c, qrow = min(qi, S - 1);
+    const float* brow = bias ? bias + (((int64_t)g * H + h) * S + qrow) * S : nullptr;
+    // the lane's bias of keys k + 16 u + 4 gr + t
+    const auto ask = [&](int k, float (&b)[8]) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int key = k + 16 * u + 4 * gr;
+            if (!brow) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) b[4 * u + t] = 0.f;
+            } else {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) b[4 * u + t] = brow[min(key + t, S - 1)];
+            }
+        }
+    };
+    float next[8], q[KS];
+    ask(0, next);
+#pragma unroll
+    for (int s = 0; s < KS; ++s) q[s] = Q[(((int64_t)g * S + qrow) * H + h) * D + 4 * s + gr] * scale;      // the reference scales q before the product
+    M::stage(K, g, h, S, H, 1.0f, k_l, rows);
+    M::stage(V, g, h, S, H, 1.0f, v_l, rows);
+    __syncthreads();
+    const uint32_t rh = DROP ? drop_row_hash(da, g * H + h, qi) : 0u;
+    float m = -INFINITY, l = 0.f;
+    f32x4_t o[DB];
+#pragma unroll
+    for (int i = 0; i < DB; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < S; k0 += 32) {
+        float sc[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sc[i] = next[i];
+        if (k0 + 32 < S) ask(k0 + 32, next);
+        float cm = -INFINITY;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int k = k0 + 16 * u;
+            f32x4_t a = {0.f, 0.f, 0.f, 0.f};
+            if (k < S) {
+#pragma unroll
+                for (int s = 0; s < KS; ++s) a = mma4(k_l[(k + c) * LD + 4 * s + gr], q[s], a);
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                sc[4 * u + t] = k + 4 * gr + t < S ? a[t] + sc[4 * u + t] : -INFINITY;
+                cm = fmaxf(cm, sc[4 * u + t]);
+            }
+        }
+        cm = fmaxf(cm, __shfl_xor(cm, 16));
+        cm = fmaxf(cm, __shfl_xor(cm, 32));
+        const float m_new = fmaxf(m, cm), m_use = (m_new == -INFINITY) ? 0.f : m_new;
+        const float alpha = expf(m - m_use);           // m = -inf: 0
+        l *= alpha;
+#pragma unroll
+        for (int i = 0; i < DB; ++i) o[i] *= alpha;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int k = k0 + 16 * u;
+            if (k >= S) break;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const float p = expf(sc[4 * u + t] - m_use);
+                if (k + 4 * gr + t < S) l += p;
+                const float pk = k + 4 * gr + t < S && (!DROP || drop_keep(da, rh, k + 4 * gr + t)) ? p : 0.f;
+#pragma unroll
+                for (int i = 0; i < DB; ++i) o[i] = mma4(v_l[(k + 4 * gr + t) * LD + 16 * i + cd], pk, o[i]);
+            }
+        }
+        m = m_new;
+    }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (qi >= S) return;
+    const float f = (DROP ? da.inv_keep : 1.0f) / l;
+#pragma unroll
+    for (int i = 0; i < DB; ++i)
+        if (D >= 16 || 4 * gr < D)
+            *reinterpret_cast<float4*>(out + (((int64_t)g * S + qi) * H + h) * D + 16 * i + 4 * gr) = make_float4(o[i][0] * f, o[i][1] * f, o[i][2] * f, o[i][3] * f);
+    if (gr == 0) lse[((int64_t)g * H + h) * S + qi] = (m == -INFINITY ? 0.f : m) + logf(l);
+}
+
+// Wave w: the keys 16 w ..., a lane's key is its column, against one tile of queries after the other: dK and dV in registers; dS through a tile in
+// LDS of the wave's own, with rows and columns changed, for its part of dQ, which waits in LDS for the others'.
+template <int D, bool DROP>
+__global__ __launch_bounds__(64 * kMmTiles) void k_dense_f32_mm_bwd(const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
+                                                                    const float* __restrict__ bias, const float* __restrict__ O, const float* __restrict__ lse,
+                                                                    const float* __restrict__ dO, float* __restrict__ dQ, float* __restrict__ dK, float* __restrict__ dV,
+                                                                    float* __restrict__ dbias, int S, int H, float scale, int nb, const DropArgs da) {
+    using M = Mm<D>;
+    constexpr int LD = M::LD, DB = M::DB, KS = M::KS;
+    extern __shared__ __align__(16) char smem[];
+    const int rows = blockDim.x / 4, waves = blockDim.x / 64;
+    float* part = reinterpret_cast<float*>(smem);      // dQ of each wave [rows][D]
+    float* lse_l = part + waves * rows * D;
+    float* dd_l = lse_l + rows;                        // sum_c dout[q, c] out[q, c]
+    float* q_l = dd_l + rows;                          // q * sqrt(d)
+    float* k_l = q_l + rows * LD;
+    float* v_l = k_l + rows * LD;
+    float* g_l = v_l + rows * LD;                      // dout
+    int g, h;
+    if (!pair_of_block(nb, H, g, h)) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, gr = lane >> 4, cd = c % D;
+    float* tile = g_l + rows * LD + wave * 16 * 17;
+    const int ki = wave * 16 + c, kcol = min(ki, S - 1);
+    const bool kok = ki < S;
+    const int64_t plane = ((int64_t)g * H + h) * S * S;
+    const float* bias_gh = bias ? bias + plane : nullptr;
+    float* dbias_gh = dbias ? dbias + plane : nullptr;
+    const auto ask = [&](int q0, float (&b)[4]) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) b[t] = bias_gh ? bias_gh[(int64_t)min(q0 + 4 * gr + t, S - 1) * S + kcol] : 0.f;
+    };
+    float next[4];
+    ask(0, next);
+    M::stage(Q, g, h, S, H, scale, q_l, rows);
+    M::stage(K, g, h, S, H, 1.0f, k_l, rows);
+    M::stage(V, g, h, S, H, 1.0f, v_l, rows);
+    M::stage(dO, g, h, S, H, 1.0f, g_l, rows);
+    {
+        // dout . out by the steps that give dout . v: where one key has all of a row's weight (out = v) the two cancel bit for bit, as they must
+        // (the row's dS is 0).  The wave's rows: the diagonal.
+        const int64_t at = (((int64_t)g * S + kcol) * H + h) * D + gr;
+        float ov[KS], gv[KS];
+#pragma unroll
+        for (int s = 0; s < KS; ++s) { ov[s] = O[at + 4 * s]; gv[s] = dO[at + 4 * s]; }
+        const float L = lse[((int64_t)g * H + h) * S + kcol];
+        f32x4_t dd = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < KS; ++s) dd = mma4(gv[s], ov[s], dd);
+        if (gr == c >> 2) {
+            const float t = (c & 2) ? ((c & 1) ? dd[3] : dd[2]) : ((c & 1) ? dd[1] : dd[0]);
+            dd_l[ki] = kok ? t : 0.f;
+            lse_l[ki] = kok ? L : 0.f;
+        }
+    }
+    __syncthreads();
+    float kb[KS], vb[KS], ka[4][DB];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) { kb[s] = k_l[ki * LD + 4 * s + gr]; vb[s] = v_l[ki * LD + 4 * s + gr]; }
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < DB; ++i) ka[s][i] = k_l[(wave * 16 + 4 * s + gr) * LD + 16 * i + cd];
+    f32x4_t dk[DB], dv[DB];
+#pragma unroll
+    for (int i = 0; i < DB; ++i) dk[i] = dv[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int q0 = 0; q0 < S; q0 += 16) {
+        float b[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) b[t] = next[t];
+        if (q0 + 16 < S) ask(q0 + 16, next);
+        f32x4_t sc = {0.f, 0.f, 0.f, 0.f}, dp = sc;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            sc = mma4(q_l[(q0 + c) * LD + 4 * s + gr], kb[s], sc);
+            dp = mma4(g_l[(q0 + c) * LD + 4 * s + gr], vb[s], dp);
+        }
+        const int r0 = q0 + 4 * gr;
+        const f32x4_t L4 = *reinterpret_cast<const f32x4_t*>(&lse_l[r0]), D4 = *reinterpret_cast<const f32x4_t*>(&dd_l[r0]);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const bool in = kok && r0 + t < S;
+            const float p = expf(sc[t] + b[t] - L4[t]);
+            const float ks = !DROP ? 1.0f : (drop_keep(da, drop_row_hash(da, g * H + h, r0 + t), ki) ? da.inv_keep : 0.f);
+            const float dS = in ? p * (dp[t] * ks - D4[t]) : 0.f, pk = in ? p * ks : 0.f;
+            if (dbias_gh && in) dbias_gh[(int64_t)(r0 + t) * S + ki] = dS;
+            tile[(4 * gr + t) * 17 + c] = dS;
+#pragma unroll
+            for (int i = 0; i < DB; ++i) {
+                dk[i] = mma4(q_l[(r0 + t) * LD + 16 * i + cd], dS, dk[i]);      // q_l holds q * sqrt(d): d s / d k
+                dv[i] = mma4(g_l[(r0 + t) * LD + 16 * i + cd], pk, dv[i]);
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        f32x4_t dq[DB];
+#pragma unroll
+        for (int i = 0; i < DB; ++i) dq[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const float ds = tile[c * 17 + 4 * s + gr];
+#pragma unroll
+            for (int i = 0; i < DB; ++i) dq[i] = mma4(ka[s][i], ds, dq[i]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < DB; ++i)
+            if (D >= 16 || 4 * gr < D) *reinterpret_cast<f32x4_t*>(&part[(wave * rows + q0 + c) * D + 16 * i + 4 * gr]) = dq[i];
+    }
+    if (kok) {
+#pragma unroll
+        for (int i = 0; i < DB; ++i)
+            if (D >= 16 || 4 * gr < D) {
+                const int64_t at = (((int64_t)g * S + ki) * H + h) * D + 16 * i + 4 * gr;
+                *reinterpret_cast<f32x4_t*>(dK + at) = dk[i];
+                *reinterpret_cast<f32x4_t*>(dV + at) = dv[i];
+            }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < S * KS; i += blockDim.x) {      // the waves' shares in order
+        const int row = i / KS, at = i % KS * 4;
+        f32x4_t t = {0.f, 0.f, 0.f, 0.f};
+        for (int w = 0; w < waves; ++w) t += *reinterpret_cast<const f32x4_t*>(&part[(w * rows + row) * D + at]);
+        *reinterpret_cast<f32x4_t*>(dQ + (((int64_t)g * S + row) * H + h) * D + at) = t * scale;
+    }
+}
+
+template <int D>
+static int launch_f32_mm(const DenseF32Call& c, bool bwd) {
+    const float scale = sqrtf((float)D);
+    const bool drop = c.p_drop > 0.f;
+    const DropArgs da = drop_args(c.p_drop, c.seed);
+    const dim3 grid((unsigned)(((c.b + 7) / 8) * 8 * c.H)), block(64 * Mm<D>::tiles(c.S));
+    static std::atomic<uint64_t> done[4];
+    const int lds = bwd ? Mm<D>::bwd_lds(c.S) : Mm<D>::fwd_lds(c.S);
+    KernelTimer t(bwd ? KS_DENSE_BWD : KS_DENSE_FWD, c.st);
+    if (bwd) {
+        const auto kernel = drop ? &k_dense_f32_mm_bwd<D, true> : &k_dense_f32_mm_bwd<D, false>;
+        if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), 160 * 1024, done[2 + drop])) return rc;
+        hipLaunchKernelGGL(kernel, grid, block, lds, c.st, c.q, c.k, c.v, c.bias, c.out, c.lse, c.dout, c.dq, c.dk, c.dv, c.dbias, c.S, c.H, scale, c.b, da);
+    } else {
+        const auto kernel = drop ? &k_dense_f32_mm_fwd<D, true> : &k_dense_f32_mm_fwd<D, false>;
+        if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), 160 * 1024, done[drop])) return rc;
+        hipLaunchKernelGGL(kernel, grid, block, lds, c.st, c.q, c.k, c.v, c.bias, c.o_out, c.o_lse, c.S, c.H, scale, c.b, da);
+    }
+    TGT_HIP_CHECK(hipGetLastError());
+    return TGT_OK;
+}
+
 template <int D>
 static int launch_f32(const DenseF32Call& c, bool bwd) {
     const int lds_bwd = (4 * c.S * D + 2 * c.S) * 4 + c.S * kF32StripLd * 4;
@@ -254,6 +536,8 @@ static int launch_f32(const DenseF32Call& c, bool bwd) {
         set_error("dense attention (float32): S=%d with head dim %d needs %d bytes of LDS (limit %d)", c.S, D, lds_bwd, 160 * 1024);
         return TGT_ERR_UNSUPPORTED;
     }
+    // (the thread-per-row kernels take what is left: more than 224, 160, 96 rows of head dim 8, 16, 32, where a wave's shares of dQ leave the LDS)
+    if (Mm<D>::fits(c.S)) return launch_f32_mm<D>(c, bwd);
     const float scale = sqrtf((float)D);      // the reference MULTIPLIES q by sqrt(d)
     const bool drop = c.p_drop > 0.f;
     const DropArgs da = drop_args(c.p_drop, c.seed);
