@@ -257,10 +257,12 @@ __global__ __launch_bounds__(kF32Block) void k_dense_f32_bwd(const float* __rest
 // With a thread per query row 65 rows kept 65 of 256 threads busy, and every element read the row of K (and V) from LDS twice, once for the
 // thread's query and once for its key.  Here a wave has sixteen rows, all of them work, the bias and its gradient go between memory and registers in
 // rows of 64 bytes, and the backward forms a probability once.  us, 8 heads of 8, thread per row / this, forward and backward: 256 graphs of
-// 13 rows 7.6 / 5.3, 13.5 / 6.9; of 41 16.4 / 13.0, 40.8 / 18.9; of 129 120 / 71, 304 / 134 (bias and gradient alone, 136 MB each, 26 and 53 at
-// the rate of a large copy); 64 of 201 101 / 39, 223 / 66; 4 of 129 38 / 13, 87 / 19; heads of 32, 64 of 65 rows 35 / 15, 91 / 35.  Errors against 64 bits
+// 13 rows 7.6 / 5.3, 13.5 / 6.9; of 41 16.4 / 12.2, 40.8 / 18.7; of 129 120 / 65, 304 / 134 (bias and gradient alone, 136 MB each, 26 and 53 at
+// the rate of a large copy); 64 of 201 101 / 34, 223 / 67; 4 of 129 38 / 12, 87 / 19; heads of 32, 64 of 65 rows 35 / 14, 91 / 35.  (Forward: a lane's four keys
+// of the bias in one load wherever they begin; in four, 71 and 39 where it says 65 and 34.)  Errors against 64 bits
 // a tenth smaller (256 graphs of 41 rows, of the norm: out 1.29e-7 / 1.40e-7 before, dq 2.1e-7 / 2.2e-7, dbias 1.9e-7 / 2.0e-7).
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));      // 16 bytes that begin at any float
 __device__ __forceinline__ f32x4_t mma4(float a, float b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 constexpr int kMmTiles = 16;        // tiles of sixteen rows, a wave each
 template <int D> struct Mm {
@@ -307,6 +309,10 @@ __global__ __launch_bounds__(64 * kMmTiles) void k_dense_f32_mm_fwd(const float*
             if (!brow) {
 #pragma unroll
                 for (int t = 0; t < 4; ++t) b[4 * u + t] = 0.f;
+            } else if (k + 16 * u + 16 <= S) {
+                const f32x4_any v = *reinterpret_cast<const f32x4_any*>(brow + key);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) b[4 * u + t] = v[t];
             } else {
 #pragma unroll
                 for (int t = 0; t < 4; ++t) b[4 * u + t] = brow[min(key + t, S - 1)];
