@@ -684,6 +684,8 @@ typedef struct {
     void* out[8];
 } tgt_node_sum;
 int tgt_node_sums(const tgt_node_sum* sums, int count, int dtype, void* stream);
+/* The same and, in the launch, tgt_reduce_partials of one descriptor (NULL: none) with outputs of the same dtype. */
+int tgt_node_sums_and_reduce(const tgt_node_sum* sums, int count, const tgt_reduce_desc* desc, int dtype, void* stream);
 /* The same for the GT layers (models/gt_dist_node_level.py:218-267), hidden 64, feed-forward 128:
  *     y = a O^T + bo;  x1 = LN1(x + y);  s2 = x1 + W2 relu(W1 y + b1) + b2;  x' = LN2(s2);   q, k, v = x' W^T + b
  * w: packed O, W1 (rows 0 .. 63, 64 .. 127), W2 (columns 0 .. 63, 64 .. 127) with unit frag_bytes(1) / 2; v: bo, gamma1, beta1, b1 (two

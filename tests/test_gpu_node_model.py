@@ -342,3 +342,36 @@ def test_backward_of_many_rows_is_that_of_its_parts(cuda, n):
         want = sum(p[1][i] for p in parts)
         for a, b in zip(t.split([4096] * 3 + [64] * 5), want.split([4096] * 3 + [64] * 5)):
             assert float((a - b).norm()) <= 1e-5 * float(b.norm())
+
+
+class NodeSum(ctypes.Structure):      # tgt_node_sum
+    _fields_ = [("partial", ctypes.c_void_p)] + [(k, ctypes.c_int32) for k in ("workers", "mats", "rows", "ld")] + [("out", ctypes.c_void_p * 8)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("count,features,outputs,workers", [(1, 1, 64, 1), (9, 128, 64, 250), (26, 500, 64, 17), (27, 51, 64, 512), (3, 100, 40, 33)])
+def test_sums_of_a_linear_beside_the_layers(cuda, dtype, count, features, outputs, workers):
+    """The same bits as the two launches: sums of more elements than a layer's and of fewer, more descriptors than a launch takes, and elements that
+    are no multiple of 64 (a launch of their own)"""
+    print(f"sums together: count={count} features={features} outputs={outputs} workers={workers} {dtype}", flush=True)
+    g, L, st = torch.Generator(device=cuda).manual_seed(count), _lib.lib(), torch.cuda.current_stream(cuda).cuda_stream
+    code = _lib.DTYPE_F32 if dtype == torch.float32 else _lib.DTYPE_BF16
+    partials = [torch.randn(max(1, workers // 2), 3 * 4096 + 5 * 64, generator=g, device=cuda) for _ in range(count)]
+    n = outputs * features + outputs
+    of_linear = torch.randn(workers, n, generator=g, device=cuda)
+    outs = []
+    for together in (False, True):
+        layer = [[torch.full((s,), float("nan"), dtype=dtype, device=cuda) for s in (4096, 4096, 4096, 64, 64, 64, 64, 64)] for _ in range(count)]
+        W, b = torch.full((n - outputs,), float("nan"), dtype=dtype, device=cuda), torch.full((outputs,), float("nan"), dtype=dtype, device=cuda)
+        sums = (NodeSum * count)(*[NodeSum(partial=p.data_ptr(), workers=p.shape[0], mats=3, rows=64, ld=0, out=(ctypes.c_void_p * 8)(*[t.data_ptr() for t in o]))
+                                   for p, o in zip(partials, layer)])
+        desc = _lib.ReduceDesc(partial=of_linear.data_ptr(), workers=workers, n=n, n_out=2)
+        desc.out[0], desc.out[1], desc.begin[1] = W.data_ptr(), b.data_ptr(), n - outputs
+        if together:
+            _lib.check(L.tgt_node_sums_and_reduce(ctypes.addressof(sums), count, ctypes.addressof(desc), code, st))
+        else:
+            _lib.check(L.tgt_node_sums(ctypes.addressof(sums), count, code, st))
+            _lib.check(L.tgt_reduce_partials(ctypes.addressof(desc), 1, code, st))
+        outs.append([t for o in layer for t in o] + [W, b])
+    for x, y in zip(*outs):
+        assert torch.equal(x, y) and not x.isnan().any()

@@ -126,6 +126,7 @@ SIGNATURES = {
     "tgt_node_bwd_post": (_i32, [_vp, _vp]),
     "tgt_node_bwd_both": (_i32, [_vp, _vp, _vp]),
     "tgt_node_sums": (_i32, [_vp, _i32, _i32, _vp]),
+    "tgt_node_sums_and_reduce": (_i32, [_vp, _i32, _vp, _i32, _vp]),
     "tgt_gt_fwd": (_i32, [_vp, _vp]),
     "tgt_gt_bwd": (_i32, [_vp, _vp]),
     "tgt_readout_fwd": (_i32, [_vp, _vp]),

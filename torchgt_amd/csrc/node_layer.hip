@@ -513,12 +513,16 @@ struct SumArgs {
     int workers[kMaxSums], n[kMaxSums];
     void* out[kMaxSums][kMaxOut];      // mats x 4096 elements, then vectors of 64 (a null entry is not wanted)
     int16_t mats[kMaxSums], rows[kMaxSums], ld[kMaxSums];   // rows: of the 64 in each matrix and the vectors that follow them (classes)
+    int count;                         // blockIdx.y behind them: the sum of another kernel's partials
+    tgt_reduce_desc other;
 };
 
 // 64 consecutive elements x 16 slices of the workers per workgroup: slices in worker order, then the slice sums in order.  Bound by
 // its reads, 50 KB of partials from every worker of every launch of a backward (108 MB for four Graphormer layers): sixteen lanes of a
 // wave take 16 bytes each of a slice's 64 elements, eight workers in flight.  A lane per element and a wave per slice / this / 256 elements
 // and a wave per slice, us with 64, 250 and 256 workers of four layers: 14.2 / 8.9 / 8.9, 24.3 / 19.8 / 20.0, 27.2 / 26.3 / 25.9 (GT: 34 / 34 / 39).
+// `other` (of the first linear's weight gradient: slices and order are those of k_reduce_partials, so are the bits) as a launch of its own / beside the layers:
+// 4 K nodes 6.5 + 4.0 / 6.7, 64 K 24.4 + 4.8 / 27.1, GT in bf16 32.3 + 4.1 / 32.8.
 constexpr int kSumElems = 64;
 template <int W> __device__ __forceinline__ void add_workers(float4& s, const float* __restrict__ src, int64_t n) {
     float4 t[W];
@@ -529,12 +533,14 @@ template <int W> __device__ __forceinline__ void add_workers(float4& s, const fl
 }
 template <typename T> __global__ __launch_bounds__(256) void k_node_sums(const SumArgs a) {
     __shared__ float part[16][kSumElems];
-    const int d = blockIdx.y, n = a.n[d], e0 = blockIdx.x * kSumElems;      // (n is a multiple of 64)
+    const int d = blockIdx.y, e0 = blockIdx.x * kSumElems;
+    const bool other = d == a.count;
+    const int n = other ? a.other.n : a.n[d], workers = other ? a.other.workers : a.workers[d];      // (n is a multiple of 64)
     if (e0 >= n) return;
     {
         const int sl = threadIdx.x >> 4, el = 4 * (threadIdx.x & 15);
-        const int w0 = a.workers[d] * sl / 16, w1 = a.workers[d] * (sl + 1) / 16;
-        const float* __restrict__ src = a.partial[d] + e0 + el;
+        const int w0 = (int)((int64_t)workers * sl / 16), w1 = (int)((int64_t)workers * (sl + 1) / 16);
+        const float* __restrict__ src = (other ? a.other.partial : a.partial[d]) + e0 + el;
         float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
         int w = w0;
         for (; w + 8 <= w1; w += 8) add_workers<8>(s, src + (int64_t)w * n, n);
@@ -548,6 +554,13 @@ template <typename T> __global__ __launch_bounds__(256) void k_node_sums(const S
         float t = 0.f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) t += part[i][threadIdx.x];
+        if (other) {
+            int seg = 0;
+            for (int i = 1; i < a.other.n_out; ++i)
+                if (e >= a.other.begin[i]) seg = i;
+            if (a.other.out[seg]) reinterpret_cast<T*>(a.other.out[seg])[e - a.other.begin[seg]] = to_elem<T>(t);
+            return;
+        }
         const int mats = a.mats[d], rows = a.rows[d];
         const int seg = e < mats * 4096 ? e >> 12 : mats + ((e - mats * 4096) >> 6), at = e < mats * 4096 ? e & 4095 : (e - mats * 4096) & 63;
         const int limit = seg < mats ? rows * 64 : (seg < 2 * mats ? rows : 64);
@@ -695,9 +708,16 @@ int tgt_node_bwd_both(const tgt_node_bwd_pre_args* a, const tgt_node_bwd_post_ar
     return groups_of_64(a->rows, false) ? launch_bwd_both<nbf16, 16, 64>(*a, *b, st) : launch_bwd_both<nbf16, 16, 128>(*a, *b, st);
 }
 
-int tgt_node_sums(const tgt_node_sum* sums, int count, int dtype, void* stream) {
+int tgt_node_sums(const tgt_node_sum* sums, int count, int dtype, void* stream) { return tgt_node_sums_and_reduce(sums, count, nullptr, dtype, stream); }
+int tgt_node_sums_and_reduce(const tgt_node_sum* sums, int count, const tgt_reduce_desc* desc, int dtype, void* stream) {
     using namespace tgt;
     if (!sums || count < 1 || !dtype_ok(dtype)) return bad("tgt_node_sums", "null or bad argument");
+    if (desc && (!desc->partial || desc->workers < 1 || desc->n < 1 || desc->n_out < 1 || desc->n_out > 6 || desc->begin[0] != 0))
+        return bad("tgt_node_sums_and_reduce", "not a descriptor that a *_deferred call filled in");
+    if (desc && (desc->n % kSumElems != 0 || reinterpret_cast<uintptr_t>(desc->partial) % 16 != 0)) {      // (M K + M elements of a weight: 64 outputs or a multiple)
+        if (int rc = reduce_partials(desc, 1, dtype, (hipStream_t)stream)) return rc;
+        desc = nullptr;
+    }
     KernelTimer t(KS_NODE_SUMS, (hipStream_t)stream);
     for (int c = 0; c < count; c += kMaxSums) {
         SumArgs a{};
@@ -711,7 +731,10 @@ int tgt_node_sums(const tgt_node_sum* sums, int count, int dtype, void* stream) 
             for (int o = 0; o < 2 * s.mats + 2; ++o) a.out[i][o] = s.out[o];
             longest = std::max(longest, a.n[i]);
         }
-        const dim3 grid((unsigned)(longest / kSumElems), (unsigned)m);
+        const bool with_other = desc && c + m == count;
+        a.count = m;
+        if (with_other) { a.other = *desc; longest = std::max(longest, desc->n); }
+        const dim3 grid((unsigned)(longest / kSumElems), (unsigned)(m + with_other));
         if (dtype == TGT_DTYPE_F32) hipLaunchKernelGGL((k_node_sums<float>), grid, dim3(256), 0, (hipStream_t)stream, a);
         else hipLaunchKernelGGL((k_node_sums<nbf16>), grid, dim3(256), 0, (hipStream_t)stream, a);
         TGT_HIP_CHECK(hipGetLastError());

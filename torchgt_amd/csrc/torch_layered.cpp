@@ -449,7 +449,10 @@ struct FusedGtModel : GtModel {
             check(tgt_node_bwd_pre(&b, D.stream), "tgt_node_bwd_pre");
         }
         linear_back(t, D, x, {P[0]}, {g}, dx, {G[0]}, {G[1]}, D.n, D.F, 64, sums);
-        if (!t.dry()) check(tgt_node_sums(later.data(), (int)later.size(), D.code, D.stream), "tgt_node_sums");
+        if (!t.dry()) {
+            check(tgt_node_sums_and_reduce(later.data(), (int)later.size(), &sums.d.back(), D.code, D.stream), "tgt_node_sums_and_reduce");
+            sums.d.pop_back();
+        }
         sums.run(t, D);
     }
 };

@@ -206,17 +206,18 @@ struct NodeGraphormerFn : public torch::autograd::Function<NodeGraphormerFn> {
             for (int i = 0; i < 8; ++i) s2.out[i] = w[pre[i]].data_ptr();
         }
         check(tgt_node_bwd_pre(&a, stream), "tgt_node_bwd_pre");
-        check(tgt_node_sums(sums.data(), (int)sums.size(), code, stream), "tgt_node_sums");
         Tensor dx;
-        {
+        {      // the encoder's weight gradient, whose partials are added up beside the layers'
             if (ctx->needs_input_grad(0)) dx = at::empty_like(x);
             const void *W[1] = {Wn.data_ptr()}, *DY[1] = {g[0] + D.tokens * kWidth * x.element_size()};
             void *DW[1] = {G.t[0].data_ptr()}, *DB[1] = {G.t[1].data_ptr()};
             const int64_t bytes = tgt_linear_bwd_workspace_bytes(1, (int)x.size(1), (int)kWidth);
             Tensor lws = at::empty({bytes}, x.options().dtype(at::kByte));
-            check(tgt_linear_bwd(x.data_ptr(), W, DY, 1, D.n, (int)x.size(1), (int)kWidth, code, dx.defined() ? dx.data_ptr() : nullptr, DW, DB,
-                                 lws.data_ptr(), bytes, stream),
-                  "tgt_linear_bwd");
+            tgt_reduce_desc sum;
+            check(tgt_linear_bwd_deferred(x.data_ptr(), W, DY, 1, D.n, (int)x.size(1), (int)kWidth, code, dx.defined() ? dx.data_ptr() : nullptr, DW, DB,
+                                          lws.data_ptr(), bytes, stream, &sum),
+                  "tgt_linear_bwd_deferred");
+            check(tgt_node_sums_and_reduce(sums.data(), (int)sums.size(), &sum, code, stream), "tgt_node_sums_and_reduce");
         }
         variable_list out;
         out.reserve(G.t.size() + 5);
