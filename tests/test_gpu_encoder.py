@@ -289,3 +289,22 @@ def test_layer_as_one_operator_equals_layer_op_by_op(cuda, dtype):
     assert not m._one_operator(x, None, ei, "sparse")
     m.eval()
     assert m._one_operator(x, None, ei, "sparse")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N,C", [(1, 1), (63, 7), (64, 40), (65, 40), (255, 3), (1025, 47), (3073, 5), (4095, 5), (4096, 40)])
+def test_nll_loss_of_few_rows_has_the_bits_of_many(cuda, dtype, N, C):
+    """Up to 4096 rows go to one workgroup, more to several: rows that do not count, behind the others, change nothing.  Targets outside the classes do not
+    count either, and without any row that does the loss is NaN."""
+    print(f"nll_loss few rows: N={N} C={C} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(N)
+    lp = torch.log_softmax(torch.randn(N, C, generator=g), 1).to(dtype)
+    t = torch.randint(-1, C + 1, (N,), generator=g)
+    t[torch.rand(N, generator=g) < 0.2] = -100
+    t[0] = 0
+    more = 4097 - N
+    losses = [nll_loss(x.to(cuda), y.to(cuda)) for x, y in ((lp, t), (torch.cat([lp, torch.full((more, C), float("nan"), dtype=dtype)]), torch.cat([t, t.new_full((more,), -100)])))]
+    ok = (t >= 0) & (t < C)
+    want = -lp.double()[ok, t[ok]].mean()
+    assert torch.equal(losses[0], losses[1]) and abs(float(losses[0]) - float(want)) <= (2e-6 if dtype == torch.float32 else 2 ** -8) * max(1e-3, abs(float(want)))
+    assert nll_loss(lp.to(cuda), torch.full((N,), -100, device=cuda)).isnan()
