@@ -6,7 +6,7 @@
 // q * sqrt(d) makes large; a float32 caller who has not asked for that gets these kernels instead: float32
 // products and sums, fp32 softmax with the accurate exponential, 1e-5 against a float64 evaluation.
 //
-// Up to 224 rows (160 and 96 with head dims of 16 and 32) the products go to the float32 matrix instructions (k_dense_f32_mm_*, below), a wave per
+// Up to 240 rows (160 and 96 with head dims of 16 and 32) the products go to the float32 matrix instructions (k_dense_f32_mm_*, below), a wave per
 // tile of sixteen queries (forward) or keys (backward).  What follows is about the other two kernels, on the vector units.
 //
 // One workgroup per (graph, head).  Forward: K and V of the head sit in LDS, a thread owns one query row and
@@ -257,8 +257,8 @@ __global__ __launch_bounds__(kF32Block) void k_dense_f32_bwd(const float* __rest
 // With a thread per query row 65 rows kept 65 of 256 threads busy, and every element read the row of K (and V) from LDS twice, once for the
 // thread's query and once for its key.  Here a wave has sixteen rows, all of them work, the bias and its gradient go between memory and registers in
 // rows of 64 bytes, and the backward forms a probability once.  us, 8 heads of 8, thread per row / this, forward and backward: 256 graphs of
-// 13 rows 7.6 / 5.3, 13.5 / 6.9; of 41 16.4 / 12.2, 40.8 / 18.7; of 129 120 / 65, 304 / 134 (bias and gradient alone, 136 MB each, 26 and 53 at
-// the rate of a large copy); 64 of 201 101 / 34, 223 / 67; 4 of 129 38 / 12, 87 / 19; heads of 32, 64 of 65 rows 35 / 14, 91 / 35.  (Forward: a lane's four keys
+// 13 rows 7.6 / 5.3, 13.5 / 6.9; of 41 16.4 / 12.2, 40.8 / 18.7; of 129 120 / 64, 304 / 128 (bias and gradient alone, 136 MB each, 26 and 53 at
+// the rate of a large copy); 64 of 201 101 / 33, 223 / 66; 4 of 129 38 / 12, 87 / 19; heads of 32, 64 of 65 rows 35 / 14, 91 / 35.  (Forward: a lane's four keys
 // of the bias in one load wherever they begin; in four, 71 and 39 where it says 65 and 34.)  Errors against 64 bits
 // a tenth smaller (256 graphs of 41 rows, of the norm: out 1.29e-7 / 1.40e-7 before, dq 2.1e-7 / 2.2e-7, dbias 1.9e-7 / 2.0e-7).
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -266,12 +266,15 @@ typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));      //
 __device__ __forceinline__ f32x4_t mma4(float a, float b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 constexpr int kMmTiles = 16;        // tiles of sixteen rows, a wave each
 template <int D> struct Mm {
-    static constexpr int LD = D + 1, DB = (D + 15) / 16, KS = D / 4;      // row stride in LDS (odd: rows in different banks), blocks of sixteen features, steps over them
+    // row stride in LDS (an odd number of fours: the reads of four features of sixteen rows and of sixteen features of every fourth row both meet every
+    // bank once), blocks of sixteen features, steps over them; row stride of a wave's tile (likewise)
+    static constexpr int LD = D + 4, DB = (D + 15) / 16, KS = D / 4, TD = 20;
     static int tiles(int S) { return (S + 15) / 16; }
     static int fwd_lds(int S) { return 2 * 16 * tiles(S) * LD * 4; }
     static int bwd_lds(int S) {
         const int n = tiles(S), rows = 16 * n;
-        return (n * rows * D + 2 * rows + 4 * rows * LD + n * 16 * 17) * 4;
+        static_assert(16 * TD <= 2 * 16 * LD, "the waves' tiles in the place of K and V");
+        return (n * rows * D + 2 * rows + 4 * rows * LD) * 4;
     }
     static bool fits(int S) { return S > 0 && tiles(S) <= kMmTiles && bwd_lds(S) <= 160 * 1024; }
     // X[g, :, h, :] -> LDS [rows][LD], rows behind S are zero
@@ -280,8 +283,7 @@ template <int D> struct Mm {
             const int row = c / KS, part = c % KS;
             float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
             if (row < S) v = *reinterpret_cast<const float4*>(X + (((int64_t)g * S + row) * H + h) * D + part * 4);
-            float* to = dst + row * LD + part * 4;
-            to[0] = v.x * f; to[1] = v.y * f; to[2] = v.z * f; to[3] = v.w * f;
+            *reinterpret_cast<float4*>(dst + row * LD + part * 4) = make_float4(v.x * f, v.y * f, v.z * f, v.w * f);
         }
     }
 };
@@ -392,28 +394,29 @@ __global__ __launch_bounds__(64 * kMmTiles) void k_dense_f32_mm_bwd(const float*
                                                                     const float* __restrict__ dO, float* __restrict__ dQ, float* __restrict__ dK, float* __restrict__ dV,
                                                                     float* __restrict__ dbias, int S, int H, float scale, int nb, const DropArgs da) {
     using M = Mm<D>;
-    constexpr int LD = M::LD, DB = M::DB, KS = M::KS;
+    constexpr int LD = M::LD, DB = M::DB, KS = M::KS, TD = M::TD;
     extern __shared__ __align__(16) char smem[];
     const int rows = blockDim.x / 4, waves = blockDim.x / 64;
     float* part = reinterpret_cast<float*>(smem);      // dQ of each wave [rows][D]
     float* lse_l = part + waves * rows * D;
     float* dd_l = lse_l + rows;                        // sum_c dout[q, c] out[q, c]
     float* q_l = dd_l + rows;                          // q * sqrt(d)
-    float* k_l = q_l + rows * LD;
+    float* g_l = q_l + rows * LD;                      // dout
+    float* k_l = g_l + rows * LD;
     float* v_l = k_l + rows * LD;
-    float* g_l = v_l + rows * LD;                      // dout
     int g, h;
     if (!pair_of_block(nb, H, g, h)) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, gr = lane >> 4, cd = c % D;
-    float* tile = g_l + rows * LD + wave * 16 * 17;
+    float* tile = k_l + wave * 16 * TD;                // when K and V are in registers
     const int ki = wave * 16 + c, kcol = min(ki, S - 1);
     const bool kok = ki < S;
     const int64_t plane = ((int64_t)g * H + h) * S * S;
     const float* bias_gh = bias ? bias + plane : nullptr;
     float* dbias_gh = dbias ? dbias + plane : nullptr;
+    const int at0 = 4 * gr * S + kcol, last = (S - 1) * S + kcol;      // the lane's elements of the plane: at0 + (q0 + t) S, its last one
     const auto ask = [&](int q0, float (&b)[4]) {
 #pragma unroll
-        for (int t = 0; t < 4; ++t) b[t] = bias_gh ? bias_gh[(int64_t)min(q0 + 4 * gr + t, S - 1) * S + kcol] : 0.f;
+        for (int t = 0; t < 4; ++t) b[t] = bias_gh ? bias_gh[(uint32_t)min(at0 + (q0 + t) * S, last)] : 0.f;
     };
     float next[4];
     ask(0, next);
@@ -449,6 +452,7 @@ __global__ __launch_bounds__(64 * kMmTiles) void k_dense_f32_mm_bwd(const float*
     f32x4_t dk[DB], dv[DB];
 #pragma unroll
     for (int i = 0; i < DB; ++i) dk[i] = dv[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    __syncthreads();      // everybody has its K and V
 #pragma unroll 1
     for (int q0 = 0; q0 < S; q0 += 16) {
         float b[4];
@@ -469,8 +473,8 @@ __global__ __launch_bounds__(64 * kMmTiles) void k_dense_f32_mm_bwd(const float*
             const float p = expf(sc[t] + b[t] - L4[t]);
             const float ks = !DROP ? 1.0f : (drop_keep(da, drop_row_hash(da, g * H + h, r0 + t), ki) ? da.inv_keep : 0.f);
             const float dS = in ? p * (dp[t] * ks - D4[t]) : 0.f, pk = in ? p * ks : 0.f;
-            if (dbias_gh && in) dbias_gh[(int64_t)(r0 + t) * S + ki] = dS;
-            tile[(4 * gr + t) * 17 + c] = dS;
+            if (dbias_gh && in) dbias_gh[(uint32_t)(at0 + (q0 + t) * S)] = dS;
+            tile[(4 * gr + t) * TD + c] = dS;
 #pragma unroll
             for (int i = 0; i < DB; ++i) {
                 dk[i] = mma4(q_l[(r0 + t) * LD + 16 * i + cd], dS, dk[i]);      // q_l holds q * sqrt(d): d s / d k
@@ -484,7 +488,7 @@ __global__ __launch_bounds__(64 * kMmTiles) void k_dense_f32_mm_bwd(const float*
         for (int i = 0; i < DB; ++i) dq[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            const float ds = tile[c * 17 + 4 * s + gr];
+            const float ds = tile[c * TD + 4 * s + gr];
 #pragma unroll
             for (int i = 0; i < DB; ++i) dq[i] = mma4(ka[s][i], ds, dq[i]);
         }
@@ -542,7 +546,7 @@ static int launch_f32(const DenseF32Call& c, bool bwd) {
         set_error("dense attention (float32): S=%d with head dim %d needs %d bytes of LDS (limit %d)", c.S, D, lds_bwd, 160 * 1024);
         return TGT_ERR_UNSUPPORTED;
     }
-    // (the thread-per-row kernels take what is left: more than 224, 160, 96 rows of head dim 8, 16, 32, where a wave's shares of dQ leave the LDS)
+    // (the thread-per-row kernels take what is left: more than 240, 160, 96 rows of head dim 8, 16, 32, where a wave's shares of dQ leave the LDS)
     if (Mm<D>::fits(c.S)) return launch_f32_mm<D>(c, bwd);
     const float scale = sqrtf((float)D);      // the reference MULTIPLIES q by sqrt(d)
     const bool drop = c.p_drop > 0.f;
