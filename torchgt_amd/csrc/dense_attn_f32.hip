@@ -6,7 +6,7 @@
 // q * sqrt(d) makes large; a float32 caller who has not asked for that gets these kernels instead: float32
 // products and sums, fp32 softmax with the accurate exponential, 1e-5 against a float64 evaluation.
 //
-// Up to 240 rows (160 and 96 with head dims of 16 and 32) the products go to the float32 matrix instructions (k_dense_f32_mm_*, below), a wave per
+// Up to 256 rows (192 with a head dim of 32) the products go to the float32 matrix instructions (k_dense_f32_mm_*, below), a wave per
 // tile of sixteen queries (forward) or keys (backward).  What follows is about the other two kernels, on the vector units.
 //
 // One workgroup per (graph, head).  Forward: K and V of the head sit in LDS, a thread owns one query row and
@@ -258,7 +258,7 @@ __global__ __launch_bounds__(kF32Block) void k_dense_f32_bwd(const float* __rest
 // thread's query and once for its key.  Here a wave has sixteen rows, all of them work, the bias and its gradient go between memory and registers in
 // rows of 64 bytes, and the backward forms a probability once.  us, 8 heads of 8, thread per row / this, forward and backward: 256 graphs of
 // 13 rows 7.6 / 5.3, 13.5 / 6.9; of 41 16.4 / 12.2, 40.8 / 18.7; of 129 120 / 64, 304 / 128 (bias and gradient alone, 136 MB each, 26 and 53 at
-// the rate of a large copy); 64 of 201 101 / 33, 223 / 66; 4 of 129 38 / 12, 87 / 19; heads of 32, 64 of 65 rows 35 / 14, 91 / 35.  (Forward: a lane's four keys
+// the rate of a large copy); 64 of 201 101 / 33, 223 / 60; 4 of 129 38 / 12, 87 / 19; heads of 32, 64 of 65 rows 35 / 14, 91 / 27.  (Forward: a lane's four keys
 // of the bias in one load wherever they begin; in four, 71 and 39 where it says 65 and 34.)  Errors against 64 bits
 // a tenth smaller (256 graphs of 41 rows, of the norm: out 1.29e-7 / 1.40e-7 before, dq 2.1e-7 / 2.2e-7, dbias 1.9e-7 / 2.0e-7).
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -271,12 +271,13 @@ template <int D> struct Mm {
     static constexpr int LD = D + 4, DB = (D + 15) / 16, KS = D / 4, TD = 20;
     static int tiles(int S) { return (S + 15) / 16; }
     static int fwd_lds(int S) { return 2 * 16 * tiles(S) * LD * 4; }
-    static int bwd_lds(int S) {
+    // each: the shares of dQ are added up after every step of queries (two steps' shares in LDS), else all of them at the end
+    static int bwd_lds(int S, bool each) {
         const int n = tiles(S), rows = 16 * n;
         static_assert(16 * TD <= 2 * 16 * LD, "the waves' tiles in the place of K and V");
-        return (n * rows * D + 2 * rows + 4 * rows * LD) * 4;
+        return (n * (each ? 32 : rows) * D + 2 * rows + 4 * rows * LD) * 4;
     }
-    static bool fits(int S) { return S > 0 && tiles(S) <= kMmTiles && bwd_lds(S) <= 160 * 1024; }
+    static bool fits(int S) { return S > 0 && tiles(S) <= kMmTiles && bwd_lds(S, true) <= 160 * 1024; }
     // X[g, :, h, :] -> LDS [rows][LD], rows behind S are zero
     static __device__ __forceinline__ void stage(const float* __restrict__ X, int g, int h, int S, int H, float f, float* __restrict__ dst, int rows) {
         for (int c = threadIdx.x; c < rows * KS; c += blockDim.x) {
@@ -387,8 +388,12 @@ __global__ __launch_bounds__(64 * kMmTiles) void k_dense_f32_mm_fwd(const float*
 }
 
 // Wave w: the keys 16 w ..., a lane's key is its column, against one tile of queries after the other: dK and dV in registers; dS through a tile in
-// LDS of the wave's own, with rows and columns changed, for its part of dQ, which waits in LDS for the others'.
-template <int D, bool DROP>
+// LDS of the wave's own, with rows and columns changed, for its share of dQ, which waits in LDS for the others'.  EACH: until the end of the step, behind a
+// barrier, where a wave adds the step's shares up, the next one the next step's; else until the end.  All shares are 4 D S bytes a wave and keep other workgroups
+// off the CU: to the end where three of them fit it all the same (48 KB), or where there is no more than one for a CU.  us, at the end / EACH: 8 heads of 8, 128
+// graphs of 65 rows (27 KB) 21.8 / 23.4, 256 of 129 (70 KB) 128.1 / 128.7, 64 of 201 (129 KB) 65.8 / 59.9, 4 of 129 18.6 / 20.4; heads of 16, 128 of 65 (52 KB)
+// 28.6 / 26.7, 200 of 151 177 / 157; of 32, 64 of 65 (98 KB) 35.4 / 27.2.
+template <int D, bool DROP, bool EACH>
 __global__ __launch_bounds__(64 * kMmTiles) void k_dense_f32_mm_bwd(const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
                                                                     const float* __restrict__ bias, const float* __restrict__ O, const float* __restrict__ lse,
                                                                     const float* __restrict__ dO, float* __restrict__ dQ, float* __restrict__ dK, float* __restrict__ dV,
@@ -397,8 +402,8 @@ __global__ __launch_bounds__(64 * kMmTiles) void k_dense_f32_mm_bwd(const float*
     constexpr int LD = M::LD, DB = M::DB, KS = M::KS, TD = M::TD;
     extern __shared__ __align__(16) char smem[];
     const int rows = blockDim.x / 4, waves = blockDim.x / 64;
-    float* part = reinterpret_cast<float*>(smem);      // dQ of each wave [rows][D]
-    float* lse_l = part + waves * rows * D;
+    float* part = reinterpret_cast<float*>(smem);      // shares of dQ: EACH two steps' [wave][16][D], else [wave][rows][D]
+    float* lse_l = part + waves * (EACH ? 32 : rows) * D;
     float* dd_l = lse_l + rows;                        // sum_c dout[q, c] out[q, c]
     float* q_l = dd_l + rows;                          // q * sqrt(d)
     float* g_l = q_l + rows * LD;                      // dout
@@ -452,6 +457,14 @@ __global__ __launch_bounds__(64 * kMmTiles) void k_dense_f32_mm_bwd(const float*
     f32x4_t dk[DB], dv[DB];
 #pragma unroll
     for (int i = 0; i < DB; ++i) dk[i] = dv[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    // dQ of `n` rows from row0 on: the waves' shares in order
+    const auto add_up = [&](const float* shares, int apart, int row0, int n, int first, int threads) {
+        for (int e = first; e < n * KS; e += threads) {
+            f32x4_t t = {0.f, 0.f, 0.f, 0.f};
+            for (int w = 0; w < waves; ++w) t += *reinterpret_cast<const f32x4_t*>(&shares[w * apart + 4 * e]);
+            *reinterpret_cast<f32x4_t*>(dQ + (((int64_t)g * S + row0 + e / KS) * H + h) * D + e % KS * 4) = t * scale;
+        }
+    };
     __syncthreads();      // everybody has its K and V
 #pragma unroll 1
     for (int q0 = 0; q0 < S; q0 += 16) {
@@ -494,9 +507,20 @@ __global__ __launch_bounds__(64 * kMmTiles) void k_dense_f32_mm_bwd(const float*
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
+        const int step = q0 / 16;
+        float* shares = EACH ? part + (step & 1) * waves * 16 * D : part + q0 * D;
+        const int apart = (EACH ? 16 : rows) * D;      // from a wave's to the next one's
 #pragma unroll
         for (int i = 0; i < DB; ++i)
-            if (D >= 16 || 4 * gr < D) *reinterpret_cast<f32x4_t*>(&part[(wave * rows + q0 + c) * D + 16 * i + 4 * gr]) = dq[i];
+            if (D >= 16 || 4 * gr < D) *reinterpret_cast<f32x4_t*>(&shares[wave * apart + c * D + 16 * i + 4 * gr]) = dq[i];
+        if constexpr (EACH) {
+            __syncthreads();      // (the other step's shares have been read: who adds them up comes here afterwards)
+            if (wave == step % waves) add_up(shares, apart, q0, min(16, S - q0), lane, 64);
+        }
+    }
+    if constexpr (!EACH) {
+        __syncthreads();
+        add_up(part, rows * D, 0, S, threadIdx.x, blockDim.x);
     }
     if (kok) {
 #pragma unroll
@@ -507,13 +531,6 @@ __global__ __launch_bounds__(64 * kMmTiles) void k_dense_f32_mm_bwd(const float*
                 *reinterpret_cast<f32x4_t*>(dV + at) = dv[i];
             }
     }
-    __syncthreads();
-    for (int i = threadIdx.x; i < S * KS; i += blockDim.x) {      // the waves' shares in order
-        const int row = i / KS, at = i % KS * 4;
-        f32x4_t t = {0.f, 0.f, 0.f, 0.f};
-        for (int w = 0; w < waves; ++w) t += *reinterpret_cast<const f32x4_t*>(&part[(w * rows + row) * D + at]);
-        *reinterpret_cast<f32x4_t*>(dQ + (((int64_t)g * S + row) * H + h) * D + at) = t * scale;
-    }
 }
 
 template <int D>
@@ -522,12 +539,15 @@ static int launch_f32_mm(const DenseF32Call& c, bool bwd) {
     const bool drop = c.p_drop > 0.f;
     const DropArgs da = drop_args(c.p_drop, c.seed);
     const dim3 grid((unsigned)(((c.b + 7) / 8) * 8 * c.H)), block(64 * Mm<D>::tiles(c.S));
-    static std::atomic<uint64_t> done[4];
-    const int lds = bwd ? Mm<D>::bwd_lds(c.S) : Mm<D>::fwd_lds(c.S);
+    static std::atomic<uint64_t> done[6];
+    const int whole = Mm<D>::bwd_lds(c.S, false);
+    const bool each = whole > 160 * 1024 || (whole > 48 * 1024 && (int64_t)c.b * c.H > num_cus());
+    const int lds = bwd ? (each ? Mm<D>::bwd_lds(c.S, true) : whole) : Mm<D>::fwd_lds(c.S);
     KernelTimer t(bwd ? KS_DENSE_BWD : KS_DENSE_FWD, c.st);
     if (bwd) {
-        const auto kernel = drop ? &k_dense_f32_mm_bwd<D, true> : &k_dense_f32_mm_bwd<D, false>;
-        if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), 160 * 1024, done[2 + drop])) return rc;
+        const auto kernel = each ? (drop ? &k_dense_f32_mm_bwd<D, true, true> : &k_dense_f32_mm_bwd<D, false, true>)
+                                 : (drop ? &k_dense_f32_mm_bwd<D, true, false> : &k_dense_f32_mm_bwd<D, false, false>);
+        if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), 160 * 1024, done[2 + 2 * each + drop])) return rc;
         hipLaunchKernelGGL(kernel, grid, block, lds, c.st, c.q, c.k, c.v, c.bias, c.out, c.lse, c.dout, c.dq, c.dk, c.dv, c.dbias, c.S, c.H, scale, c.b, da);
     } else {
         const auto kernel = drop ? &k_dense_f32_mm_fwd<D, true> : &k_dense_f32_mm_fwd<D, false>;
@@ -546,7 +566,7 @@ static int launch_f32(const DenseF32Call& c, bool bwd) {
         set_error("dense attention (float32): S=%d with head dim %d needs %d bytes of LDS (limit %d)", c.S, D, lds_bwd, 160 * 1024);
         return TGT_ERR_UNSUPPORTED;
     }
-    // (the thread-per-row kernels take what is left: more than 240, 160, 96 rows of head dim 8, 16, 32, where a wave's shares of dQ leave the LDS)
+    // (the thread-per-row kernels take what is left: more than 256 rows, or 192 of head dim 32, whose images leave the LDS)
     if (Mm<D>::fits(c.S)) return launch_f32_mm<D>(c, bwd);
     const float scale = sqrtf((float)D);      // the reference MULTIPLIES q by sqrt(d)
     const bool drop = c.p_drop > 0.f;
