@@ -68,13 +68,15 @@ def test_many_edges_with_a_bias(cuda):
     close(got, reference(q, k, v, bias, ei, dout, cuda), TOL[torch.bfloat16])
 
 
+@pytest.mark.parametrize("H,d", [(8, 8), (8, 16)])
 @pytest.mark.parametrize("dtype,bias_kind", [(torch.float32, "none"), (torch.float32, "edge_head"), (torch.bfloat16, "edge_head"), (torch.bfloat16, "none")])
-def test_first_backward_inside_a_capture(cuda, dtype, bias_kind):
-    """Nothing can be made while a stream is captured: a call that would take the other list takes the one there is."""
-    n, H, d = 16384, 8, 8
+def test_first_backward_inside_a_capture(cuda, dtype, bias_kind, H, d):
+    """Creating the plan (64 elements a row) and the first call of another shape make every list that a backward of the shape may take: one that is
+    captured before any other backward ran takes the same list as an eager one, and gives its bits."""
+    n = 16384
+    print(f"captured first: {H}x{d} {bias_kind} {dtype}", flush=True)
     ei = near_graph(n, LENGTHS, 5)
     q, k, v, bias, dout = inputs(n, ei.shape[1], H, d, dtype, bias_kind, 6)
-    want = reference(q, k, v, bias, ei, dout)
     L, P = _lib.lib(), lambda x: None if x is None else x.data_ptr()
     plan = GraphPlan(ei.to(cuda), n)
     dev = [None if x is None else x.to(cuda) for x in (q, k, v, bias, dout)]
@@ -83,22 +85,30 @@ def test_first_backward_inside_a_capture(cuda, dtype, bias_kind):
     Z, ws = torch.empty(n, H, device=cuda), plan.workspace(H, d)
     code = _lib.DTYPE_F32 if dtype == torch.float32 else _lib.DTYPE_BF16
     mode = _lib.BIAS_NONE if bias is None else _lib.BIAS_EDGE_HEAD
+    results = [x for x in (out, dq, dk, dv, db) if x is not None]
+
+    def forward(stream):
+        _lib.check(L.tgt_sparse_attn_fwd(plan.handle, P(dev[0]), P(dev[1]), P(dev[2]), P(dev[3]), mode, H, d, code, P(out), P(Z), P(ws), ws.numel(), stream))
 
     def step(stream):
-        _lib.check(L.tgt_sparse_attn_fwd(plan.handle, P(dev[0]), P(dev[1]), P(dev[2]), P(dev[3]), mode, H, d, code, P(out), P(Z), P(ws), ws.numel(), stream))
+        forward(stream)
         _lib.check(L.tgt_sparse_attn_bwd(plan.handle, P(dev[0]), P(dev[1]), P(dev[2]), P(dev[3]), mode, H, d, code, P(out), P(Z), P(dev[4]), P(dq),
                                          P(dk), P(dv), P(db), P(ws), ws.numel(), stream))
 
+    if H * d != 64:
+        forward(torch.cuda.current_stream().cuda_stream)
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         step(torch.cuda.current_stream().cuda_stream)
+    step(torch.cuda.current_stream().cuda_stream)
+    eager = [x.clone() for x in results]
+    close(eager, reference(q, k, v, bias, ei, dout), TOL[dtype])
     for replay in range(3):
-        for x in (out, dq, dk, dv):
+        for x in results:
             x.zero_()
         graph.replay()
         torch.cuda.synchronize()
-        close([x for x in (out, dq, dk, dv, db) if x is not None], want, TOL[dtype])
-        step(torch.cuda.current_stream().cuda_stream)      # eager: makes the list that it prefers
-        torch.cuda.synchronize()
-        close([x for x in (out, dq, dk, dv, db) if x is not None], want, TOL[dtype])
+        for name, x, want in zip(("out", "dq", "dk", "dv", "dbias"), results, eager):
+            assert torch.equal(x, want), f"{name} of replay {replay}"
+        step(torch.cuda.current_stream().cuda_stream)
     plan.close()

@@ -421,7 +421,7 @@ __host__ __device__ inline int32_t run_waves(uint32_t kind, int32_t n, int lpe) 
     return (n + ipw - 1) / ipw;
 }
 
-// One workgroup per run, for all lists that are made together; its sixteen waves write the run's wave records
+// One workgroup per run, for all lists of a shape; its sixteen waves write the run's wave records
 // in turn (layout: WaveRec in common.h), the lanes of a wave one edge or bias row each.  Wave lw of
 // XCD x's list is wave lw % 4 of that XCD's (lw / 4)-th workgroup, and workgroup b of the launch runs on XCD b mod 8:
 // record ((lw / 4) * 8 + x) * 4 + lw % 4.  Everything a kernel uses of a record is written: no clearing pass.
@@ -776,14 +776,12 @@ void place(const std::vector<const Side*>& sides, int lpe, int list, int32_t* n_
     }
 }
 
-// The records of the lists that `make` says.  `runs` feeds an asynchronous copy: it lives until the stream has been synchronised.
-int build_records(const tgt_plan* plan, int lpe, Schedule::List* const (&lists)[LIST_COUNT], const bool (&make)[LIST_COUNT], std::vector<Run>& runs,
-                  DevBuf& runs_d, hipStream_t st) {
-    for (int l = 0; l < LIST_COUNT; ++l) {
-        if (!make[l]) continue;
-        if (l == LIST_FWD) place({&plan->dst}, lpe, l, &lists[l]->blocks, runs);
-        else place({&plan->dst, &plan->src}, lpe, l, &lists[l]->blocks, runs);
-    }
+// The records of all lists.  `runs` feeds an asynchronous copy: it lives until the stream has been synchronised.
+int build_records(const tgt_plan* plan, int lpe, Schedule& sc, std::vector<Run>& runs, DevBuf& runs_d, hipStream_t st) {
+    Schedule::List* const lists[LIST_COUNT] = {&sc.fwd, &sc.bwd, &sc.bwd_grouped};
+    place({&plan->dst}, lpe, LIST_FWD, &sc.fwd.blocks, runs);
+    place({&plan->dst, &plan->src}, lpe, LIST_BWD, &sc.bwd.blocks, runs);
+    if (has_grouped_list(plan, lpe)) place({&plan->dst, &plan->src}, lpe, LIST_BWD_GROUPED, &sc.bwd_grouped.blocks, runs);
     const WaveRecLayout L(lpe);
     const size_t rec = (size_t)L.stride * sizeof(int32_t) * 4;
     if (runs.empty()) return TGT_OK;
@@ -791,7 +789,7 @@ int build_records(const tgt_plan* plan, int lpe, Schedule::List* const (&lists)[
     TGT_HIP_CHECK(hipMemcpyAsync(runs_d.p, runs.data(), sizeof(Run) * runs.size(), hipMemcpyHostToDevice, st));
     RecordLists out{};
     for (int l = 0; l < LIST_COUNT; ++l) {
-        if (make[l] && lists[l]->blocks) TGT_HIP_CHECK(dev_alloc(&lists[l]->recs, rec * lists[l]->blocks, st));
+        if (lists[l]->blocks) TGT_HIP_CHECK(dev_alloc(&lists[l]->recs, rec * lists[l]->blocks, st));
         out.recs[l] = static_cast<int32_t*>(lists[l]->recs);
     }
     const Side &d = plan->dst, &s = plan->src;
@@ -802,13 +800,15 @@ int build_records(const tgt_plan* plan, int lpe, Schedule::List* const (&lists)[
 }
 }  // namespace
 
-const Schedule* plan_schedule_if_ready(const tgt_plan* plan, int lpe) {
+const Schedule* plan_schedule_if_ready(const tgt_plan* plan_c, int lpe) {
+    tgt_plan* plan = const_cast<tgt_plan*>(plan_c);
+    std::lock_guard<std::mutex> lock(plan->sched_mutex);
     for (int idx = 0; idx < kNumLpe; ++idx)
         if ((1 << idx) == lpe) return plan->sched[idx].ready ? &plan->sched[idx] : nullptr;
     return nullptr;
 }
 
-const Schedule* plan_schedule(const tgt_plan* plan_c, int lpe, hipStream_t st, int want) {
+const Schedule* plan_schedule(const tgt_plan* plan_c, int lpe, hipStream_t st) {
     int idx = 0;
     while (idx < kNumLpe && (1 << idx) != lpe) ++idx;
     if (idx == kNumLpe) { set_error("no schedule for %d lanes per edge", lpe); return nullptr; }
@@ -816,30 +816,17 @@ const Schedule* plan_schedule(const tgt_plan* plan_c, int lpe, hipStream_t st, i
     Schedule& sc = plan->sched[idx];
     // the descriptors of a shape are made once, whichever thread or stream asks first
     std::lock_guard<std::mutex> lock(plan->sched_mutex);
-    const bool grouped = plan->grouped && lpe >= kGroupMinLpe;
-    if (!grouped) want &= ~LISTS_BWD_GROUPED;
-    // a shape's first use makes the list that 2-byte calls without a bias take, unless the caller names another one
-    if (!sc.ready && !want) want = grouped ? LISTS_BWD_GROUPED : LISTS_BWD;
-    const bool make[LIST_COUNT] = {!sc.ready, (want & LISTS_BWD) && !sc.bwd.ready, (want & LISTS_BWD_GROUPED) && !sc.bwd_grouped.ready};
-    if (!make[LIST_FWD] && !make[LIST_BWD] && !make[LIST_BWD_GROUPED]) return &sc;
-    if (sc.ready) {
-        // The other list is there and says the same: a stream that is being captured, where nothing can be made, goes on with it.
-        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(st, &capturing) != hipSuccess) { set_error("hipStreamIsCapturing failed"); return nullptr; }
-        if (capturing != hipStreamCaptureStatusNone) return &sc;
-    }
+    if (sc.ready) return &sc;
     std::vector<Run> runs;
     DevBuf runs_d;
-    Schedule::List* const lists[LIST_COUNT] = {&sc.fwd, &sc.bwd, &sc.bwd_grouped};
-    int rc = build_records(plan, lpe, lists, make, runs, runs_d, st);
+    int rc = build_records(plan, lpe, sc, runs, runs_d, st);
     // the host vector feeds an asynchronous copy: it may go once the stream is idle
     if (hipStreamSynchronize(st) != hipSuccess && rc == TGT_OK) { set_error("hipStreamSynchronize failed"); rc = TGT_ERR_HIP; }
-    for (int l = 0; l < LIST_COUNT; ++l) {
-        if (!make[l]) continue;
-        if (rc == TGT_OK) lists[l]->ready = true;
-        else { dev_free(lists[l]->recs); *lists[l] = Schedule::List(); }
+    if (rc != TGT_OK) {
+        for (Schedule::List* l : {&sc.fwd, &sc.bwd, &sc.bwd_grouped}) dev_free(l->recs);
+        sc = Schedule();
+        return nullptr;
     }
-    if (rc != TGT_OK) return nullptr;
     sc.ready = true;
     return &sc;
 }
@@ -969,7 +956,7 @@ static int create_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, in
         for (size_t i = 0; i < m.size(); ++i) sd.homed_idx[at[sd.block_home[i]]++] = (int32_t)i;
     }
     // the shape of the reference's node-level models (hidden 64: 8 heads of 8, or 4 of 16); other shapes on first use
-    return plan_schedule(plan, 8, st, LISTS_ANY) ? TGT_OK : TGT_ERR_HIP;
+    return plan_schedule(plan, 8, st) ? TGT_OK : TGT_ERR_HIP;
 }
 
 // ---------------------------------------------------------------------------

@@ -726,13 +726,14 @@ __device__ __forceinline__ void walk_range(const Common& c, const SideArgs& s, c
     }
 }
 
+// Types and shapes whose backward may take the list with kind 6 (want_groups)
+template <typename T, int LPE> constexpr bool can_group() { return sizeof(T) == 2 && LPE >= kGroupMinLpe; }
+
 // Walks a row of kGroupRowMin edges or more with one lane group, four edges a step, as a queue of gathers like walk_range's: the sums
 // stay in the lanes that write the row, and a wave's prologue is shared by all its rows.  The four ids of a step are one load.
 // The last step starts kUnroll edges in front of the row's end, so that every position read is the row's own, and leaves out the edges
 // that the step before it has added.
-// Where walk_range keeps no queue neither does this: two edges at a time with a bias, which is what the registers allow (calls that
-// prefer the list without kind 6, and find it missing in a capture).
-template <typename T, int LPE, int LPH, int MODE, int HASB, bool TILES>
+template <typename T, int LPE, int LPH, int MODE, int HASB>
 __device__ __forceinline__ void walk_group(const Common& c, const SideArgs& s, const RecLane& rec, const int row, const int start,
                                            const int len, const int el, const bool valid, Acc& acc) {
     typedef int ids_t __attribute__((ext_vector_type(4), aligned(4)));
@@ -754,30 +755,6 @@ __device__ __forceinline__ void walk_group(const Common& c, const SideArgs& s, c
             }
         };
         int nb[kUnroll], ed[kUnroll];
-        if constexpr (!piped_walk<T, MODE, TILES>()) {
-#pragma unroll 1
-            for (int base = 0; base < len; base += kUnroll) {
-                const int from = min(base, last);
-                quad(s.col, from, nb);
-                bias_rows(from, ed);
-                bool ok[kUnroll];
-#pragma unroll
-                for (int u = 0; u < kUnroll; ++u) ok[u] = from + u >= base;
-                if constexpr (HASB == 0) edge_step<T, LPE, LPH, MODE, HASB>(c, s, rr, nb, ed, ok, el, acc);
-                else {
-#pragma unroll 1
-                    for (int h = 0; h < 2; ++h) {
-                        Gathered<T> g[2];
-#pragma unroll
-                        for (int u = 0; u < 2; ++u) ask_edge<T, LPE, LPH, MODE, HASB, O>(c, h ? nb[u + 2] : nb[u], h ? ed[u + 2] : ed[u], el, g[u]);
-#pragma unroll
-                        for (int u = 0; u < 2; ++u)
-                            if (h ? ok[u + 2] : ok[u]) use_edge<T, LPE, LPH, MODE, HASB>(c, s, rr, g[u], h ? ed[u + 2] : ed[u], el, acc);
-                    }
-                }
-            }
-            return;
-        }
         nb[0] = rec.cols.x; nb[1] = rec.cols.y; nb[2] = rec.cols.z; nb[3] = rec.cols.w;
         if (std::is_same<O, uint64_t>::value) quad(s.col, 0, nb);      // (see walk_range)
         if (HASB == 1 && !s.eid_is_map && !std::is_same<O, uint64_t>::value) {
@@ -909,7 +886,7 @@ __device__ __forceinline__ void wave_rows(const Common& c, const SideArgs& s, co
     // pointers); nothing of it is loaded or stored
     if (TILES) valid = valid && !(len == 0 && s.cover[row] != 0);
     Acc acc;
-    if constexpr (GROUP) walk_group<T, LPE, LPH, MODE, HASB, TILES>(c, s, rec, row, start, len, el, valid, acc);
+    if constexpr (GROUP) walk_group<T, LPE, LPH, MODE, HASB>(c, s, rec, row, start, len, el, valid, acc);
     else if (INLINE) walk_record<T, LPE, LPH, S, MODE, HASB>(c, s, rec, row, start, len, slot, el, valid, acc);
     else walk_range<T, LPE, LPH, S, MODE, HASB, TILES, true>(c, s, rec, row, start, len, slot, el, valid, acc);
     finish_row<T, LPE, LPH, S, MODE, TILES>(c, s, row, slot, el, valid, acc);
@@ -917,7 +894,7 @@ __device__ __forceinline__ void wave_rows(const Common& c, const SideArgs& s, co
 
 template <typename T, int LPE, int LPH, int MODE, int HASB, bool TILES>
 __device__ __forceinline__ void wave_dispatch(const Common& c, const SideArgs& s, const RecLane& rec, const int kind) {
-    constexpr bool groups = MODE != MODE_FWD && LPE >= kGroupMinLpe;      // (only the backward's launch has kind 6)
+    constexpr bool groups = MODE != MODE_FWD && can_group<T, LPE>() && !TILES;      // (only the backward's launch has kind 6)
     switch (kind) {
         case 0: wave_rows<T, LPE, LPH, slots_for_class(LPE, 0), MODE, HASB, TILES, false>(c, s, rec); break;
         case (int)kDescGroup:
@@ -1275,10 +1252,10 @@ static bool narrow_offsets(const Call& c) {
 // 2310 / 2130 us; 100 K nodes, 3.3 M edges in 64 clusters 144 / 124 us, 16 K nodes, 0.5 M edges 30.2 / 28.2; eight heads of 16, 150 K nodes, 3.5 M edges 323 / 267.  With a bias the walk waits for its
 // rows instead, unless there are many edges (eight heads of 8, bias per edge and head, 64 K nodes, 0.6 M edges 48.5 / 50.1, 1.5 M edges 111.7 / 116.2, 150 K nodes, 3.5 M
 // edges 312 / 296; of 16, 64 K nodes, 0.6 M edges 78.1 / 78.0, 1.5 M edges 170 / 157).  float32 waits for memory and keeps no queue: 64 K nodes, 0.6 M edges 53.7 / 61.0, with a
-// bias 150 K nodes, 3.5 M edges 507 / 520.  Beside dense tiles the rows are short.
+// bias 150 K nodes, 3.5 M edges 507 / 520 (walked as kind 6 step by step, which no kernel does now).  Beside dense tiles the rows are short.
 template <typename T, int LPE>
 static bool want_groups(const Call& c) {
-    if (sizeof(T) == 4 || LPE < kGroupMinLpe || c.init != nullptr) return false;
+    if (!can_group<T, LPE>() || c.init != nullptr || !has_grouped_list(c.plan, LPE)) return false;
     return c.bias_mode == TGT_BIAS_NONE || LPE > 8 || (c.plan->E >= 16 * c.plan->N && c.plan->E >= (2 << 20));
 }
 
@@ -1293,7 +1270,7 @@ static int run_fwd(const Call& c) {
     cm.inv_scale = 1.0f / sqrtf((float)c.d);
     SideArgs a{};
     fill_side(a, c.plan->dst);
-    const Schedule* sch = c.no_alloc ? plan_schedule_if_ready(c.plan, LPE) : plan_schedule(c.plan, LPE, c.st, LISTS_ANY);
+    const Schedule* sch = c.no_alloc ? plan_schedule_if_ready(c.plan, LPE) : plan_schedule(c.plan, LPE, c.st);
     if (!sch) {
         if (c.no_alloc) {
             set_error("no launch descriptors for H*d = %d yet: call tgt_plan_prepare(plan, H, d, stream) first", LPE * 8);
@@ -1363,10 +1340,9 @@ static int run_bwd(const Call& c) {
     int32_t* counters = reinterpret_cast<int32_t*>(c.ws + L.counters);
     SideArgs sd{}, ss{};
     fill_side(sd, c.plan->dst);
-    const bool group = want_groups<T, LPE>(c);
-    const Schedule* sch = plan_schedule(c.plan, LPE, c.st, group ? LISTS_BWD_GROUPED : LISTS_BWD);
+    const Schedule* sch = plan_schedule(c.plan, LPE, c.st);
     if (!sch) return TGT_ERR_HIP;
-    const Schedule::List& list = (group ? sch->bwd_grouped : sch->bwd).ready ? (group ? sch->bwd_grouped : sch->bwd) : (group ? sch->bwd : sch->bwd_grouped);
+    const Schedule::List& list = want_groups<T, LPE>(c) ? sch->bwd_grouped : sch->bwd;
     const WaveRec<LPE>* desc = static_cast<const WaveRec<LPE>*>(list.recs);
     if (c.bias_mode & TGT_BIAS_PLAN_ORDER) sd.eid = nullptr;
     sd.out0 = c.dq; sd.out1 = c.dbias; sd.Z = nullptr;
@@ -1672,7 +1648,7 @@ int tgt_sparse_attn_fwd_noalloc(const tgt_plan_t* plan, const void* d_q, const v
 
 int tgt_plan_prepare(tgt_plan_t* plan, int H, int d, void* stream) {
     if (!plan || H < 1 || d < 1 || (H * d) % 8) { tgt::set_error("tgt_plan_prepare: null plan or H*d not a multiple of 8"); return TGT_ERR_INVALID_ARG; }
-    return tgt::plan_schedule(plan, H * d / 8, static_cast<hipStream_t>(stream), tgt::LISTS_BWD | tgt::LISTS_BWD_GROUPED) ? TGT_OK : TGT_ERR_UNSUPPORTED;
+    return tgt::plan_schedule(plan, H * d / 8, static_cast<hipStream_t>(stream)) ? TGT_OK : TGT_ERR_UNSUPPORTED;
 }
 
 int tgt_sparse_attn_bwd(const tgt_plan_t* plan, const void* d_q, const void* d_k, const void* d_v,
