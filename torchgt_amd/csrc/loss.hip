@@ -66,10 +66,11 @@ __global__ __launch_bounds__(kLossBlock) void k_nll_finish(const float* __restri
     if (threadIdx.x == 0) { st(loss, -red[0] / (float)cnt[0]); *count = (float)cnt[0]; }
 }
 
-// Both for few rows, by one workgroup: the sums are those of the two kernels, in their order.  A wave has four times 64 rows, their targets
-// and then their values asked for together.  float32, two kernels / one, us: 4096 rows 3.4 + 2.2 / 4.5 and a launch less (8192, eight times 64 rows,
-// 3.6 + 2.2 / 7.1: two kernels).
-constexpr int kLossFew = 4096, kFewBlock = 1024, kFewEach = kLossFew / kFewBlock;
+// Both for few rows, by one workgroup: the sums are those of the two kernels, in their order.  A wave has twice 64 rows, their targets
+// and then their values asked for together.  Bound by those dependent, scattered reads: the values were written on every XCD, and one CU asks for them all.  Behind a
+// log_softmax, caches cleared between passes, two kernels / one, us, float32: 256 rows 2.3 + 2.0 / 2.1, 1024 rows 2.6 + 2.0 / 2.9, 2048 rows 3.0 + 2.0 / 4.2 (bf16 2.9 + 1.8 / 3.7),
+// and a launch less; 4096 rows, four times 64, 3.0 + 2.0 / 7.1 (bf16 3.0 + 1.8 / 5.7): two kernels.
+constexpr int kLossFew = 2048, kFewBlock = 1024, kFewEach = kLossFew / kFewBlock;
 template <typename T>
 __global__ __launch_bounds__(kFewBlock) void k_nll_few(const T* __restrict__ logp, const int64_t* __restrict__ target, int N, int C, int64_t ignore_index,
                                                        T* __restrict__ loss, float* __restrict__ count) {
