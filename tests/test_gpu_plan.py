@@ -102,3 +102,19 @@ def test_plan_is_reproducible(cuda):
     a, b = GraphPlan(ei, 5000), GraphPlan(ei, 5000)
     for which in range(8):
         np.testing.assert_array_equal(a.export(which), b.export(which))
+
+
+@pytest.mark.parametrize("near,lengths,rows", [(True, [1, 12, 6, 30], 256), (False, [1, 5, 2, 6], 256), (False, [1, 12, 6, 30], 128)])
+def test_windows_of_large_graphs(cuda, near, lengths, rows):
+    """From 128 K rows on windows have 256 rows where most neighbours are near or rows are short (below ten edges), else 128: the wave items go window by
+    window, and inside one by length class."""
+    print(f"windows near={near} lengths={lengths}", flush=True)
+    n, g = (1 << 17) + 200, torch.Generator(device=cuda).manual_seed(1)
+    dst = torch.repeat_interleave(torch.arange(n, device=cuda), torch.tensor(lengths, device=cuda).repeat(n // 4))
+    src = (dst + torch.randint(-500, 501, dst.shape, generator=g, device=cuda)).clamp(0, n - 1) if near else torch.randint(0, n, dst.shape, generator=g, device=cuda)
+    plan = GraphPlan(torch.stack([src, dst]), n)
+    items = plan.export(6).reshape(-1, 4)[plan.info()["block_items_dst"]:, 0]
+    for size, in_order in ((rows, True), (rows // 2, False)):
+        assert bool((np.diff(items // size) >= 0).all()) == in_order, size
+    assert np.array_equal(np.sort(items), np.arange(n))
+    plan.close()

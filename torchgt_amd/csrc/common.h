@@ -144,7 +144,7 @@ struct Side {
 // Wave records of one kernel shape (lanes per edge): forward (destination view) and backward (both views, window by
 // window).  The backward has a second list in plans with `grouped` set and shapes of kGroupMinLpe lanes or more, in which the rows of classes
 // 1 to 3 go out as kind 6.  The first use of a shape makes all its lists: which one a later call takes depends on the call alone, and no call
-// finds its list missing in a capture.  (Plan of 262 K nodes in 64 clusters, 4.5 M edges, one backward list / both: 0.80 / 0.85 ms; 870 K nodes, 43 M
+// finds its list missing in a capture.  (Plan of 262 K nodes in 64 clusters, 5 M edges, one backward list / both: 0.80 / 0.85 ms; 870 K nodes, 44 M
 // edges 5.6 / 6.4 ms.  Made when a call first asked for it, the second one took 0.4 and 0.7 ms of that call.)
 struct Schedule {
     struct List {

@@ -130,8 +130,8 @@ struct SchedHeader { int32_t n_wave, n_long, n_block, n_split, n_parts, n_groups
 // nodes without clusters, 0.5 M edges, bf16 35.4 us by classes, 38.4 as kind 6; 262 K nodes, 8.6 M edges 550 / 566.  From 16 000 rows on
 // (8000 nodes, 0.26 M edges 17.6 / 18.7), and with ten edges a row unless rows are many (64 K nodes in 64 clusters, 0.5 M edges 32.4 / 33.5, 150 K nodes, 1.2 M edges 68.9 / 67.2).
 constexpr int kNearRows = 8192, kNearWindows = 8;      // (every eighth window is asked)
-constexpr int64_t kManyRows = 128 << 10;
-static bool may_group(int64_t N, int64_t E) { return N >= 16000 && (E >= 10 * N || N >= kManyRows); }
+constexpr int64_t kManyRows = 128 << 10, kDenseRows = 10;
+static bool may_group(int64_t N, int64_t E) { return N >= 16000 && (E >= kDenseRows * N || N >= kManyRows); }
 __host__ __device__ inline bool mostly_near(const SchedHeader& h) { return h.looked > 0 && 2 * (int64_t)h.near >= h.looked; }
 struct BlockMeta;
 // What the schedule kernels read and write, of both views (blockIdx.y)
@@ -144,33 +144,36 @@ struct SchedArgs {
     BlockMeta* meta[2];
 };
 
-// counts[window * kSchedCats + cat] = rows of that category among the window's rows (blockDim.x rows).  look: whether the edges' distances
-// are asked for (mostly_near)
-__global__ void k_sched_count(const SchedArgs a, int64_t N, int wave_row_max, bool skip_empty, bool look) {
+// How far the edges of every eighth window lead, for mostly_near: a row's middle edge stands for it.
+__global__ __launch_bounds__(kWindowRows) void k_look_near(const SideArrays a, SchedHeader* hdr, int64_t N) {
+    const int64_t r = (int64_t)blockIdx.x * kNearWindows * kWindowRows + threadIdx.x;
+    const int32_t* __restrict__ rowptr = a.rowptr[blockIdx.y];
+    const int start = r < N ? rowptr[r] : 0, len = r < N ? rowptr[r + 1] - start : 0;
+    const bool asked = len >= kGroupRowMin;
+    const bool is_near = asked && llabs((int64_t)a.col[blockIdx.y][start + len / 2] - r) <= kNearRows;
+    const uint64_t ba = __ballot(asked), bn = __ballot(is_near);
+    if ((threadIdx.x & 63) == 0 && ba) {      // (integer counts: order-free)
+        atomicAdd(&hdr[blockIdx.y].looked, (int32_t)__popcll(ba));
+        atomicAdd(&hdr[blockIdx.y].near, (int32_t)__popcll(bn));
+    }
+}
+
+// counts[window * kSchedCats + cat] = rows of that category among the window's rows (blockDim.x rows).
+__global__ void k_sched_count(const SchedArgs a, int64_t N, int wave_row_max, bool skip_empty) {
     const int32_t* __restrict__ rowptr = a.rowptr[blockIdx.y];
     uint32_t* __restrict__ counts = a.counts[blockIdx.y];
-    __shared__ uint32_t c[kSchedCats], near[2];
+    __shared__ uint32_t c[kSchedCats];
     if (threadIdx.x < kSchedCats) c[threadIdx.x] = 0;
-    if (threadIdx.x < 2) near[threadIdx.x] = 0;
     __syncthreads();
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int start = r < N ? rowptr[r] : 0, len = r < N ? rowptr[r + 1] - start : 0;
-    const int cat = r < N ? sched_category(len, wave_row_max, skip_empty) : -1;
+    const int cat = r < N ? sched_category(rowptr[r + 1] - rowptr[r], wave_row_max, skip_empty) : -1;
 #pragma unroll
     for (int k = 0; k < kSchedCats; ++k) {
         const uint64_t b = __ballot(cat == k);
         if ((threadIdx.x & 63) == 0 && b) atomicAdd(&c[k], (uint32_t)__popcll(b));   // integer count: order-free
     }
-    look = look && blockIdx.x % kNearWindows == 0;
-    if (look) {
-        const bool asked = len >= kGroupRowMin;
-        const bool is_near = asked && llabs((int64_t)a.col[blockIdx.y][start + (asked ? len / 2 : 0)] - r) <= kNearRows;
-        const uint64_t ba = __ballot(asked), bn = __ballot(is_near);
-        if ((threadIdx.x & 63) == 0 && ba) { atomicAdd(&near[0], (uint32_t)__popcll(ba)); atomicAdd(&near[1], (uint32_t)__popcll(bn)); }
-    }
     __syncthreads();
     if (threadIdx.x < kSchedCats) counts[(int64_t)blockIdx.x * kSchedCats + threadIdx.x] = c[threadIdx.x];
-    if (look && threadIdx.x == 0 && near[0]) { atomicAdd(&a.hdr[blockIdx.y]->looked, (int32_t)near[0]); atomicAdd(&a.hdr[blockIdx.y]->near, (int32_t)near[1]); }
 }
 
 // offs[window, cat]: first position of the window's rows of a category - wave classes count through
@@ -545,10 +548,14 @@ static int env_int(const char* name, int dflt) {
     return x > 0 ? x : dflt;
 }
 
-// Windows of twice the rows in large graphs: 262 K nodes, 3.9 M edges in 64 clusters, bf16 k_attn_bwd 202 us with 128, 191 with 256; other
-// lists of such graphs take the same time either way (64 K nodes by classes 35.5 and 36.4 us).
-static int window_rows(int64_t N) {
-    int w = env_int("TGT_WINDOW_ROWS", N >= kManyRows ? 2 * tgt::kWindowRows : tgt::kWindowRows);
+// twice: large graphs (kManyRows) whose rows are short (kDenseRows) or whose neighbours are near (mostly_near).  Half as many windows to count and place (plan of
+// 262 K nodes, 5 M edges 1.00 ms with 128 rows, 0.82 with 256), and forward + backward, 128 / 256 rows, us: 64 clusters, bf16 150 K nodes, 2.8 M edges 187 / 175,
+// 262 K, 5 M 345 / 337, 870 K, 44 M 3000 / 2916, with a bias per edge and head 346 / 341, 671 / 664, 7186 / 7117; float32 357 / 356, 707 / 703, 5864 / 5855, with a
+// bias 585 / 580, 1085 / 1083.  No clusters, eight edges a row: float32 228 / 226, 432 / 427, 1540 / 1547, bf16 124 / 124, 223 / 220, 841 / 840, with a bias 183 / 182,
+// 337 / 335, 1233 / 1217; beside tiles 163 / 165, 161 / 161, 528 / 517.  Not where rows have nineteen far neighbours and more, of which a window's rows share few:
+// float32 478 / 491, 882 / 896, 8758 / 8928, eight heads of 16 in bf16 150 K nodes 503 / 521 (eight of 8 246 / 249, 469 / 470, 4736 / 4764).
+static int window_rows(bool twice) {
+    int w = env_int("TGT_WINDOW_ROWS", twice ? 2 * tgt::kWindowRows : tgt::kWindowRows);
     w = (w + 63) / 64 * 64;
     return w > 64 * kSchedMaxWaves ? 64 * kSchedMaxWaves : w;
 }
@@ -585,7 +592,7 @@ constexpr int kReportFlag = 16;
 constexpr size_t kOneCopyBytes = 256 << 10;
 
 static int schedule_device(int64_t N, int64_t E, Side* const (&sides)[2], SideScratch (&scr)[2], int32_t* report, BlockMeta* metas, bool skip_empty,
-                           bool look, int W, hipStream_t st) {
+                           int W, hipStream_t st) {
     SchedArgs a{};
     for (int i = 0; i < 2; ++i) {
         Side& side = *sides[i];
@@ -621,7 +628,7 @@ static int schedule_device(int64_t N, int64_t E, Side* const (&sides)[2], SideSc
         a.meta[i] = metas + i * sc.cap_block;
     }
     const SideScratch& sc = scr[0];      // (sizes and parameters are the same)
-    hipLaunchKernelGGL(k_sched_count, dim3(sc.nwin, 2), dim3(sc.W), 0, st, a, N, sc.wave_row_max, skip_empty, look);
+    hipLaunchKernelGGL(k_sched_count, dim3(sc.nwin, 2), dim3(sc.W), 0, st, a, N, sc.wave_row_max, skip_empty);
     hipLaunchKernelGGL(k_sched_scan, dim3(1, 2), dim3(1024), 0, st, a, sc.nwin);
     hipLaunchKernelGGL(k_sched_fill, dim3(sc.nwin, 2), dim3(sc.W), 0, st, a, N, sc.wave_row_max, skip_empty, sc.cap_long);
     hipLaunchKernelGGL(k_cut_rows, dim3(1, 2), dim3(1024), 0, st, a, sc.cp);
@@ -897,12 +904,10 @@ static int create_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, in
     // what comes back to the host, in one copy: the two schedule headers, the range-check flag, per view the
     // per-window row counts and their offsets, and where the workgroup items go if there is room for few of them (else that
     // is a second copy, of the items there are)
-    const int W = window_rows(N);
-    const int nwin = (int)((N + W - 1) / W);
-    const size_t report_ints = kReportHead + 4 * (size_t)kSchedCats * nwin;
+    const auto report_of = [&](int W) { return kReportHead + 4 * (size_t)kSchedCats * (size_t)((N + W - 1) / W); };      // ints
     const size_t cap_meta = (size_t)cap_block_items(N, E), meta_bytes = 2 * sizeof(BlockMeta) * cap_meta;
     const bool one_copy = meta_bytes <= kOneCopyBytes;
-    TGT_HIP_CHECK(report_d.alloc(sizeof(int32_t) * report_ints + meta_bytes, st));
+    TGT_HIP_CHECK(report_d.alloc(sizeof(int32_t) * report_of(window_rows(false)) + meta_bytes, st));
     TGT_HIP_CHECK(hipMemsetAsync(report_d.p, 0, sizeof(int32_t) * kReportHead, st));
     int32_t* report = report_d.as<int32_t>();
     if (E > 0) {
@@ -916,8 +921,24 @@ static int create_impl(const int64_t* d_src, const int64_t* d_dst, int64_t E, in
     if (rc) return rc;
     SideScratch scr[2];
     Side* const views[2] = {&plan->dst, &plan->src};
+    bool twice = N >= kManyRows && E < kDenseRows * N;
+    if (may_group(N, E) && !plan->rows_with_edges_only) {
+        SideArrays a{};
+        for (int i = 0; i < 2; ++i) { a.rowptr[i] = views[i]->rowptr; a.col[i] = views[i]->col; }
+        constexpr int per = kNearWindows * kWindowRows;
+        hipLaunchKernelGGL(k_look_near, dim3((unsigned)((N + per - 1) / per), 2), dim3(kWindowRows), 0, st, a, reinterpret_cast<SchedHeader*>(report), N);
+        TGT_HIP_CHECK(hipGetLastError());
+        if (N >= kManyRows && !twice) {      // the windows' size follows from it: it comes to the host first
+            SchedHeader h[2];
+            TGT_HIP_CHECK(hipMemcpyAsync(h, report, sizeof(h), hipMemcpyDeviceToHost, st));
+            TGT_HIP_CHECK(hipStreamSynchronize(st));
+            twice = mostly_near(h[0]) && mostly_near(h[1]);
+        }
+    }
+    const int W = window_rows(twice);
+    const size_t report_ints = report_of(W);
     BlockMeta* const metas = reinterpret_cast<BlockMeta*>(report + report_ints);
-    rc = schedule_device(N, E, views, scr, report, metas, plan->rows_with_edges_only, may_group(N, E) && !plan->rows_with_edges_only, W, st);
+    rc = schedule_device(N, E, views, scr, report, metas, plan->rows_with_edges_only, W, st);
     if (rc) return rc;
     std::vector<int32_t> h_report(report_ints + (one_copy ? meta_bytes / 4 : 0));
     TGT_HIP_CHECK(hipMemcpyAsync(h_report.data(), report, sizeof(int32_t) * h_report.size(), hipMemcpyDeviceToHost, st));
