@@ -5,7 +5,7 @@
 //
 // What bounds them and why this shape: as in node_layer.hip, whose roles and register tiles these kernels use.  As separate
 // kernels the part moves 33 rows of 64 features per node forward and 61 backward through memory, here 7 and 7 (forward: x, a in;
-// s2, x', q, k, v out; backward: g, x, a (twice), s2 in, two rows out); y, u and relu(u) are recomputed in the backward (three
+// s2, x', q, k, v out; backward: g, x, a (float32: twice), s2 in, two rows out); y, u and relu(u) are recomputed in the backward (three
 // products), s2 is kept, which saves the two products behind them.  The 128 features between the feed-forward linears are two
 // tiles; the backward takes them one after the other, so that no more than one is alive, and keeps of u only its signs.
 // Measured at 65536 nodes (forward with q, k, v / backward, us): float32 38 / 79, bf16 15 / 29.5; a bf16 training step of four layers
