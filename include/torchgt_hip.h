@@ -125,7 +125,8 @@ int tgt_plan_prepare(tgt_plan_t* plan, int H, int d, void* stream);
 /* info[0]=N, [1]=E, [2]=#schedule items (dst side), [3]=#split rows (dst),
  * [4]=#partial segments (dst), [5..7]= the same for the src side,
  * [8]=segment length limit, [9]=longest row one wave walks, [10],[11]=#workgroup
- * items (dst, src), [12..15] reserved (0). */
+ * items (dst, src), [12] = 1 if neighbours are near, for which the backward has a second list of
+ * wave records, [13..15] reserved (0). */
 int tgt_plan_info(const tgt_plan_t* plan, int64_t info[16]);
 
 #define TGT_PLAN_ROWPTR_DST 0

@@ -6,7 +6,7 @@ import torch
 
 from oracle import graph_prep as gp
 from torchgt_amd import _lib, workloads
-from torchgt_amd.plan import GraphPlan
+from torchgt_amd.plan import GraphPlan, _plan_bytes
 
 pytestmark = pytest.mark.gpu
 
@@ -117,4 +117,23 @@ def test_windows_of_large_graphs(cuda, near, lengths, rows):
     for size, in_order in ((rows, True), (rows // 2, False)):
         assert bool((np.diff(items // size) >= 0).all()) == in_order, size
     assert np.array_equal(np.sort(items), np.arange(n))
+    plan.close()
+
+
+@pytest.mark.parametrize("near", [True, False])
+@pytest.mark.parametrize("n,length", [(20000, 5), (64000, 9), (64000, 17), (64000, 33), (140000, 5), (140000, 17), (140000, 33)])
+def test_bytes_of_a_cached_plan_are_a_bound(cuda, n, length, near):
+    """What the plan cache counts for a plan covers what the plan holds, at the row lengths where a wave record is fullest of rows and emptiest of edges;
+    with near neighbours the backward has two lists of records."""
+    print(f"plan bytes n={n} length={length} near={near}", flush=True)
+    g = torch.Generator(device=cuda).manual_seed(1)
+    dst = torch.arange(n, device=cuda).repeat_interleave(length)
+    src = (dst + torch.randint(-500, 501, dst.shape, generator=g, device=cuda)).clamp(0, n - 1) if near else torch.randint(0, n, dst.shape, generator=g, device=cuda)
+    ei = torch.stack([src, dst])
+    before = torch.cuda.memory_allocated()
+    plan = GraphPlan(ei, n)
+    held = torch.cuda.memory_allocated() - before
+    assert plan.info()["near_neighbours"] == int(near and (length >= 10 or n >= 128 << 10))
+    # (the allocator rounds each of a plan's arrays up to 512 bytes)
+    assert 0 < held <= _plan_bytes(plan) + 32 * 512
     plan.close()

@@ -1134,6 +1134,7 @@ int tgt_plan_info(const tgt_plan_t* plan, int64_t info[16]) {
     info[9] = tgt::kWaveRowMax;
     info[10] = plan->dst.n_block_items;
     info[11] = plan->src.n_block_items;
+    info[12] = plan->grouped;
     return TGT_OK;
 }
 

@@ -72,7 +72,7 @@ class GraphPlan:
         arr = (ctypes.c_int64 * 16)()
         _lib.check(_lib.lib().tgt_plan_info(self.handle, arr))
         keys = ["N", "E", "items_dst", "split_rows_dst", "segments_dst", "items_src", "split_rows_src",
-                "segments_src", "segment_len", "wave_row_max", "block_items_dst", "block_items_src"]
+                "segments_src", "segment_len", "wave_row_max", "block_items_dst", "block_items_src", "near_neighbours"]
         return {k: int(arr[i]) for i, k in enumerate(keys)}
 
     def export(self, which):
@@ -189,8 +189,9 @@ def plan_cache_stats():
 
 
 def _plan_bytes(plan):
-    # two sorted views (rowptr, col, eid), items, wave records of one shape
-    return 56 * plan.num_edges + 450 * plan.num_nodes
+    # two sorted views (rowptr, col, eid), items, wave records of one shape; with near neighbours a second list of the backward's (six
+    # bytes an edge at rows of 17 edges, which take the most for their edges)
+    return (62 if plan.info()["near_neighbours"] else 56) * plan.num_edges + 450 * plan.num_nodes
 
 
 def _evict():
