@@ -245,7 +245,7 @@ def run_readout(x, W, b, dlogp, classes, logp_back=None):
 # every d logits, du (bfloat16: 2^-9 each of three in a row, and of the results): 1e-2 of the largest; float32 1e-5.
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n,m1,m2,out,classes", [(1, 32, 16, 40, 40), (15, 5, 3, 7, 7), (16, 64, 64, 64, 63), (17, 33, 17, 8, 1), (63, 32, 16, 48, 47), (65, 32, 16, 1, 1),
-                                                 (129, 1, 1, 2, 2), (4097, 32, 16, 40, 40), (16385, 64, 32, 16, 13), (70001, 32, 16, 40, 40)])
+                                                 (129, 1, 1, 2, 2), (4097, 32, 16, 40, 40), (16385, 64, 32, 16, 13), (32769, 32, 16, 40, 40), (49152, 64, 64, 64, 63), (70001, 32, 16, 40, 40)])
 def test_readout_in_one_kernel(cuda, dtype, n, m1, m2, out, classes):
     print(f"readout n={n} widths {m1} {m2} {out} classes={classes} {dtype}", flush=True)
     g = torch.Generator(device=cuda).manual_seed(n + out)

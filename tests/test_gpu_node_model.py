@@ -317,17 +317,20 @@ def test_backward_of_many_rows_is_that_of_its_parts(cuda, n):
     _lib.check(L.tgt_node_pack(ctypes.addressof(mats), ctypes.addressof(ld), ctypes.addressof(ld), 3, ctypes.addressof(of_vecs), ctypes.addressof(lens), 5, _lib.DTYPE_BF16,
                                frags.data_ptr(), vecs.data_ptr(), st))
     rows = {k: rand(n, 64).bfloat16() for k in ("dq", "dk", "dv", "g_in", "s", "attn")}
+    rows["logp"], rows["dlogp"] = torch.log_softmax(rand(n, 40), 1).bfloat16(), rand(n, 40).bfloat16()
     Z = rand(n, 8).abs() + 1
 
     def run(lo, hi):
         at = {k: t[lo:hi].data_ptr() for k, t in rows.items()}
         workers = L.tgt_node_bwd_workers(hi - lo)
-        out = {k: torch.empty(hi - lo, 64, dtype=torch.bfloat16, device=cuda) for k in ("pre", "post", "da", "parts", "da_parts")}
-        nd, sums = torch.empty(hi - lo, 8, 2, device=cuda), [torch.full((workers, 3 * 4096 + 5 * 64), float("nan"), device=cuda) for _ in range(3)]
-        pre = NodeBwdPreArgs(rows=hi - lo, dtype=_lib.DTYPE_BF16, eps=1e-5, dq=at["dq"], dk=at["dk"], dv=at["dv"], g_in=at["g_in"], s=at["s"], w_back=back, v_next=vecs.data_ptr(),
-                             g_out=out["pre"].data_ptr(), partial=sums[0].data_ptr())
-        _lib.check(L.tgt_node_bwd_pre(ctypes.addressof(pre), st))
-        for same, g_out, da, s in ((1, "post", "da", sums[1]), (0, "parts", "da_parts", sums[2])):
+        out = {k: torch.empty(hi - lo, 64, dtype=torch.bfloat16, device=cuda) for k in ("pre", "plain", "classes", "post", "da", "parts", "da_parts")}
+        nd, sums = torch.empty(hi - lo, 8, 2, device=cuda), [torch.full((workers, m * 4096 + (m + 2) * 64), float("nan"), device=cuda) for m in (3, 3, 1, 3, 3)]
+        qkv = {k: at[k] for k in ("dq", "dk", "dv", "g_in")}
+        for g_out, s, more in (("pre", sums[0], dict(qkv, v_next=vecs.data_ptr())), ("plain", sums[1], qkv),      # (without LayerNorm: GT)
+                               ("classes", sums[2], dict(dlogp=at["dlogp"], logp=at["logp"], classes=40, v_next=vecs.data_ptr()))):
+            pre = NodeBwdPreArgs(rows=hi - lo, dtype=_lib.DTYPE_BF16, eps=1e-5, s=at["s"], w_back=back, g_out=out[g_out].data_ptr(), partial=s.data_ptr(), **more)
+            _lib.check(L.tgt_node_bwd_pre(ctypes.addressof(pre), st))
+        for same, g_out, da, s in ((1, "post", "da", sums[3]), (0, "parts", "da_parts", sums[4])):
             post = NodeBwdPostArgs(rows=hi - lo, dtype=_lib.DTYPE_BF16, heads=8, same_bits=same, eps=1e-5, g_in=at["g_in"], s=at["s"], attn=at["attn"], w_post=frags.data_ptr(),
                                    w_back=back, v_post=vecs.data_ptr(), Z=Z[lo:hi].data_ptr(), g_out=out[g_out].data_ptr(), d_attn=out[da].data_ptr(), nd=nd.data_ptr(),
                                    partial=s.data_ptr())
@@ -340,7 +343,8 @@ def test_backward_of_many_rows_is_that_of_its_parts(cuda, n):
         assert torch.equal(t, torch.cat([p[0][i] for p in parts])), i
     for i, t in enumerate(sums):
         want = sum(p[1][i] for p in parts)
-        for a, b in zip(t.split([4096] * 3 + [64] * 5), want.split([4096] * 3 + [64] * 5)):
+        sizes = [4096] * (t.numel() // 4096) + [64] * (t.numel() % 4096 // 64)
+        for a, b in zip(t.split(sizes), want.split(sizes)):
             assert float((a - b).norm()) <= 1e-5 * float(b.norm())
 
 
